@@ -72,6 +72,30 @@ def test_mp_f64(cabi, case):
     assert torch.equal(out, cabi.mp_forward(d(X), d(Y), d(R), d(snd), fo, nnodes))
 
 
+@pytest.mark.parametrize("parted", [False, True], ids=["whole", "parts"])
+@pytest.mark.parametrize("C", [32, 64, 96, 224, 256])
+def test_mp_f64_every_edge_count(cabi, C, parted):
+    """Nodes with 0 .. 140 edges each: every remainder of the staged chunks, of the slots and of their trips; with few
+    nodes a node's range is cut into parts, with 2 100 (most of them empty) it is not."""
+    _say("mp f64 edge counts", C, parted)
+    nnodes = 141 if parted else 2100
+    rng = np.random.default_rng(C)
+    deg = np.zeros(nnodes, dtype=np.int64)
+    deg[rng.permutation(nnodes)[:141]] = np.arange(141)
+    rcv = torch.from_numpy(np.repeat(np.arange(nnodes), deg).astype(np.int32))
+    E = rcv.numel()
+    snd = torch.from_numpy(rng.integers(0, nnodes, E).astype(np.int32))
+    X, v, R, G = mp_inputs(nnodes, E, C, 4)
+    Y = O.spherical_harmonics(v).contiguous()
+    d = lambda t: t.to(DEV)
+    fo = cabi.first_occurences(d(rcv), nnodes)
+    perm, off = cabi.stable_key_sort(d(snd), nnodes)
+    close(cabi.mp_forward(d(X), d(Y), d(R), d(snd), fo, nnodes), O.mp_forward(X, Y, R, snd, rcv, nnodes), RTOL, ATOL)
+    for got, want in zip(cabi.mp_backward(d(X), d(Y), d(R), d(G), d(snd), fo, perm, off, nnodes), O.mp_backward(X, Y, R, G, snd, rcv)):
+        close(got, want, RTOL, ATOL)
+
+
+
 def test_mp_f64_agrees_with_f32(cabi):
     """The two precisions of the same op differ by fp32 rounding only."""
     case = (120, 30, 128, "poisson", 0.0, 11)
