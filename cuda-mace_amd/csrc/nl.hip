@@ -1,12 +1,18 @@
 // Neighbour list on the device: all ordered pairs (i, j, S) with |r_j - r_i + S . cell| < cutoff, sorted
 // lexicographically by (i, j, Sx, Sy, Sz) -- the edge list the message-passing kernels consume (row i sorted).
 //
-// Cell list in fractional coordinates of the (possibly triclinic) cell: bins at least one cutoff wide along every
-// axis (measured perpendicular to the other two cell vectors), atoms counting-sorted by bin, one wavefront per
-// atom scanning the neighbouring bins with the lanes spread over a bin's atoms.  Two passes over the candidates
-// (count, then fill after an exclusive scan) give every atom a contiguous segment without atomics; inside a
+// Cell list in fractional coordinates of the (possibly triclinic) cell: bins at least half a cutoff wide along every
+// axis (measured perpendicular to the other two cell vectors; bins of a whole cutoff hold 1.7 times the candidates, and in a
+// cell barely wider than the cutoff six times: a 216-atom crystal with a skin was then one bin and its 27 images), atoms copied bin by bin (in any order inside a bin), one
+// wavefront per atom scanning the neighbouring bins with the lanes spread over the bins' atoms taken together.  Two
+// passes over the candidates (count, then fill after an exclusive scan) give every atom a contiguous segment; inside a
 // segment the hits are placed at their rank under the (j, S) order, so the result is the unique sorted list and
 // is reproducible bit for bit.
+//
+// What bounds it is the chain of dependent memory accesses and the number of launches: a few thousand atoms are a few
+// microseconds of work.  Bin by bin (27 bins of a dozen atoms: offsets, then indices, then positions, each waiting for the
+// one before) a scan took 25 us at 2 000 atoms and 44 us for a 216-atom crystal with 89 neighbours each; now the bins'
+// ranges are looked up side by side and their atoms addressed as one sequence of records.
 //
 // The accept test uses the ORIGINAL fp64 positions and the integer image S only:
 //     v = (r_j - r_i) + (Sx c0 + Sy c1 + Sz c2),   v0 v0 + v1 v1 + v2 v2 < cutoff^2,   (j, S) != (i, 0)
@@ -25,6 +31,7 @@ namespace {
 constexpr int kGridThreads = 1024;
 constexpr int kOffsetsStage = 16 * 1024;  // values staged in LDS at a time by the offsets scan (128 KB)
 constexpr double kBinSlack = 1.0 + 1e-9;
+constexpr double kBinsPerCutoff = 2.0;
 constexpr int kMaxScan = 32;  // most images of the cell scanned on each side of an atom
 
 struct Grid {
@@ -40,13 +47,15 @@ struct Grid {
 
 struct Workspace {
   Grid *grid;
-  int32_t *wrap;          // [N, 3]
-  int32_t *keys;          // [N]
-  int32_t *cell_perm;     // [N]
+  int32_t *wrap;          // [N, 3]  images the atom was wrapped by along periodic axes
+  int32_t *keys;          // [N]     its bin
+  int32_t *slot;          // [N]     its place inside the bin
+  int32_t *cell_count;    // [max_cells]
   int32_t *cell_offsets;  // [max_cells + 1]
   int32_t *degree;        // [N]
-  void *sort_ws;
-  size_t sort_ws_bytes;
+  int32_t *skey;          // [N]     bin, in bin order like the next two
+  double *spos;           // [N, 3]  positions as given
+  int4 *smeta;            // [N]     index of the atom, its wrap
   size_t total;
 };
 
@@ -61,14 +70,17 @@ Workspace carve(void *base, int64_t n, int64_t max_cells) {
     off += align256(bytes);
     return q;
   };
+  auto ints = [&](int64_t count) { return reinterpret_cast<int32_t *>(take(sizeof(int32_t) * static_cast<size_t>(count))); };
   w.grid = reinterpret_cast<Grid *>(take(sizeof(Grid)));
-  w.wrap = reinterpret_cast<int32_t *>(take(sizeof(int32_t) * 3 * n));
-  w.keys = reinterpret_cast<int32_t *>(take(sizeof(int32_t) * n));
-  w.cell_perm = reinterpret_cast<int32_t *>(take(sizeof(int32_t) * n));
-  w.cell_offsets = reinterpret_cast<int32_t *>(take(sizeof(int32_t) * (max_cells + 1)));
-  w.degree = reinterpret_cast<int32_t *>(take(sizeof(int32_t) * n));
-  w.sort_ws_bytes = cm_stable_key_sort_workspace(n, max_cells);
-  w.sort_ws = take(w.sort_ws_bytes);
+  w.wrap = ints(3 * n);
+  w.keys = ints(n);
+  w.slot = ints(n);
+  w.cell_count = ints(max_cells);
+  w.cell_offsets = ints(max_cells + 1);
+  w.degree = ints(n);
+  w.skey = ints(n);
+  w.spos = reinterpret_cast<double *>(take(sizeof(double) * 3 * static_cast<size_t>(n)));
+  w.smeta = reinterpret_cast<int4 *>(take(sizeof(int4) * static_cast<size_t>(n)));
   w.total = off;
   return w;
 }
@@ -79,10 +91,10 @@ __device__ __forceinline__ int floor_div(int a, int b) {
   return q;
 }
 
-// One workgroup: effective cell and its inverse, extent of the atoms along non-periodic axes, bin counts.
-__global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__restrict__ pos, const double *__restrict__ cell,
-                                                               int px, int py, int pz, double cutoff, int nnodes,
-                                                               int max_cells, Grid *__restrict__ grid) {
+// One workgroup: effective cell and its inverse, extent of the atoms along non-periodic axes, bin counts.  Written to
+// *grid (global memory) and *out (LDS; valid for every thread on return).
+__device__ __forceinline__ void make_grid(const double *__restrict__ pos, const double *__restrict__ cell, int px, int py, int pz,
+                                          double cutoff, int nnodes, int max_cells, Grid *__restrict__ grid, Grid *out) {
   __shared__ double inv[9];
   __shared__ double lo[3][kGridThreads / kWave], hi[3][kGridThreads / kWave];
   __shared__ int singular;
@@ -114,7 +126,8 @@ __global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__r
   }
   __syncthreads();
   double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (int i = t; i < nnodes; i += kGridThreads) {
+  // (the range of a fully periodic cell is the cell: the atoms are not looked at)
+  for (int i = t; i < (px && py && pz ? 0 : nnodes); i += kGridThreads) {
     const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -137,7 +150,7 @@ __global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__r
   __syncthreads();
   if (t == 0) {
     const int per[3] = {px, py, pz};
-    Grid g;
+    Grid &g = *out;
     for (int k = 0; k < 9; ++k) {
       g.inv[k] = inv[k];
       g.cellv[k] = cell ? cell[k] : 0.0;
@@ -155,13 +168,13 @@ __global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__r
       if (per[k]) {
         g.fmin[k] = 0.0;
         width[k] = height;
-        const double bins = floor(height / (cutoff * kBinSlack));
+        const double bins = floor(kBinsPerCutoff * height / (cutoff * kBinSlack));
         g.nb[k] = bins >= 1.0 ? static_cast<int>(fmin(bins, 1.0e6)) : 1;
       } else {
         const double ext = (nnodes > 0 && b > a) ? (b - a) : 0.0;
         g.fmin[k] = nnodes > 0 ? a : 0.0;
         width[k] = ext * height;
-        const double bins = floor(width[k] / (cutoff * kBinSlack));
+        const double bins = floor(kBinsPerCutoff * width[k] / (cutoff * kBinSlack));
         g.nb[k] = bins >= 1.0 ? static_cast<int>(fmin(bins, 1.0e6)) : 1;
       }
     }
@@ -192,19 +205,17 @@ __global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__r
     }
     *grid = g;
   }
+  __syncthreads();
 }
 
-__global__ void nl_bin_kernel(const double *__restrict__ pos, const Grid *__restrict__ grid, int nnodes,
-                              int32_t *__restrict__ wrap, int32_t *__restrict__ keys) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nnodes) return;
-  const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
+// Bin of an atom and the images it is wrapped by.
+__device__ __forceinline__ int bin_of(const Grid &g, double x, double y, double z, int (&wrap)[3]) {
   int b[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    double f = x * grid->inv[k] + y * grid->inv[3 + k] + z * grid->inv[6 + k];
+    double f = x * g.inv[k] + y * g.inv[3 + k] + z * g.inv[6 + k];
     int w = 0;
-    if (grid->periodic[k]) {
+    if (g.periodic[k]) {
       const double fl = floor(f);
       f -= fl;
       w = static_cast<int>(fl);
@@ -213,130 +224,315 @@ __global__ void nl_bin_kernel(const double *__restrict__ pos, const Grid *__rest
         w += 1;
       }
     } else {
-      f -= grid->fmin[k];
+      f -= g.fmin[k];
     }
-    int bk = static_cast<int>(f * grid->fscale[k]);
-    bk = bk < 0 ? 0 : (bk > grid->nb[k] - 1 ? grid->nb[k] - 1 : bk);
-    b[k] = bk;
-    wrap[3 * i + k] = w;
+    const int bk = static_cast<int>(f * g.fscale[k]);
+    b[k] = bk < 0 ? 0 : (bk > g.nb[k] - 1 ? g.nb[k] - 1 : bk);
+    wrap[k] = w;
   }
-  keys[i] = (b[0] * grid->nb[1] + b[1]) * grid->nb[2] + b[2];
+  return (b[0] * g.nb[1] + b[1]) * g.nb[2] + b[2];
 }
 
-// The accept test; see the head of this file.  No contraction into fused multiply-adds.
-__device__ __forceinline__ bool within(const double *__restrict__ pi, const double *__restrict__ pj, const int (&S)[3],
-                                       const double *__restrict__ c, double rc2) {
+// Up to kSmallAtoms atoms and bins: the whole cell list by one workgroup, with the bins counted and scanned in LDS, in place
+// of the five launches below.  Beyond that a thread's passes over its atoms cost more than the launches (12 000 atoms: 90
+// against 35 us; 2 000: 17 against 28).
+constexpr int kSmallAtoms = 4 * 1024;
+__global__ __launch_bounds__(kGridThreads) void nl_cells_small_kernel(const double *__restrict__ pos, const double *__restrict__ cell,
+                                                                      int px, int py, int pz, double cutoff, int nnodes, int max_cells,
+                                                                      Workspace w) {
+  extern __shared__ int s_count[];  // [max_cells]
+  __shared__ Grid g;
+  __shared__ int s_wave[kGridThreads / kWave];
+  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+  for (int c = t; c < max_cells; c += kGridThreads) s_count[c] = 0;
+  make_grid(pos, cell, px, py, pz, cutoff, nnodes, max_cells, w.grid, &g);  // ends with a barrier
+  const int ncells = min(g.nb[0] * g.nb[1] * g.nb[2], max_cells);
+  for (int i = t; i < nnodes; i += kGridThreads) {
+    int wr[3];
+    const int key = bin_of(g, pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], wr);
+    w.keys[i] = key;
+    w.slot[i] = atomicAdd(&s_count[key], 1);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w.wrap[3 * i + k] = wr[k];
+  }
+  __syncthreads();
+  // exclusive scan in place: a contiguous run of odd length per thread, then over the threads
+  const int per = ((ncells + kGridThreads - 1) / kGridThreads) | 1;
+  const int lo = min(t * per, ncells), hi = min(lo + per, ncells);
+  int sum = 0;
+  for (int c = lo; c < hi; ++c) sum += s_count[c];
+  int upto = sum;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int v = __shfl_up(upto, d);
+    if (lane >= d) upto += v;
+  }
+  if (lane == kWave - 1) s_wave[wave] = upto;
+  __syncthreads();
+  int run = upto - sum;
+  for (int q = 0; q < wave; ++q) run += s_wave[q];
+  for (int c = lo; c < hi; ++c) {
+    const int v = s_count[c];
+    s_count[c] = run;
+    run += v;
+  }
+  __syncthreads();
+  for (int c = t; c < ncells; c += kGridThreads) w.cell_offsets[c] = s_count[c];
+  if (t == 0) w.cell_offsets[ncells] = nnodes;
+  for (int i = t; i < nnodes; i += kGridThreads) {  // a thread reads back what it wrote itself
+    const int key = w.keys[i];
+    const int at = s_count[key] + w.slot[i];
+    w.skey[at] = key;
+    w.smeta[at] = make_int4(i, w.wrap[3 * i], w.wrap[3 * i + 1], w.wrap[3 * i + 2]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w.spos[3 * static_cast<int64_t>(at) + k] = pos[3 * i + k];
+  }
+}
+
+// The same for more atoms: grid, bins (a counter per bin), a scan, the copy into bin order.
+__global__ __launch_bounds__(kGridThreads) void nl_grid_kernel(const double *__restrict__ pos, const double *__restrict__ cell,
+                                                               int px, int py, int pz, double cutoff, int nnodes,
+                                                               int max_cells, Grid *__restrict__ grid) {
+  __shared__ Grid g;
+  make_grid(pos, cell, px, py, pz, cutoff, nnodes, max_cells, grid, &g);
+}
+
+__global__ void nl_clear_kernel(int32_t *__restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+__global__ void nl_bin_kernel(const double *__restrict__ pos, int nnodes, Workspace w) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nnodes) return;
+  int wr[3];
+  const int key = bin_of(*w.grid, pos[3 * static_cast<int64_t>(i)], pos[3 * static_cast<int64_t>(i) + 1], pos[3 * static_cast<int64_t>(i) + 2], wr);
+  w.keys[i] = key;
+  w.slot[i] = atomicAdd(&w.cell_count[key], 1);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) w.wrap[3 * static_cast<int64_t>(i) + k] = wr[k];
+}
+
+constexpr int kCellStage = 32 * 1024;  // values staged in LDS at a time (128 KB)
+__global__ __launch_bounds__(kGridThreads) void nl_cell_scan_kernel(int max_cells, Workspace w) {
+  __shared__ int part[kGridThreads];
+  __shared__ int stage[kCellStage];
+  const int ncells = min(w.grid->nb[0] * w.grid->nb[1] * w.grid->nb[2], max_cells);
+  const int total = workgroup_exclusive_scan<kGridThreads, kCellStage, int>(
+      ncells, stage, part, [&](int k) { return w.cell_count[k]; }, [&](int k, int before, int) { w.cell_offsets[k] = before; });
+  if (threadIdx.x == 0) w.cell_offsets[ncells] = total;
+}
+
+__global__ void nl_place_kernel(const double *__restrict__ pos, int nnodes, Workspace w) {
+  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (i >= nnodes) return;
+  const int key = w.keys[i];
+  const int64_t at = w.cell_offsets[key] + w.slot[i];
+  w.skey[at] = key;
+  w.smeta[at] = make_int4(static_cast<int>(i), w.wrap[3 * i], w.wrap[3 * i + 1], w.wrap[3 * i + 2]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) w.spos[3 * at + k] = pos[3 * i + k];
+}
+
+// Component k of S . cell, term by term from the left.  No contraction into fused multiply-adds.
+__device__ __forceinline__ double image_shift(const int (&S)[3], const double *c, int k) {
+#pragma clang fp contract(off)
+  return (S[0] * c[k] + S[1] * c[3 + k]) + S[2] * c[6 + k];
+}
+
+// The accept test; see the head of this file.
+__device__ __forceinline__ bool within(const double *pi, const double *pj, const int (&S)[3], const double *c, double rc2) {
 #pragma clang fp contract(off)
   double d2 = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const double shift = (S[0] * c[k] + S[1] * c[3 + k]) + S[2] * c[6 + k];
-    const double v = (pj[k] - pi[k]) + shift;
+    const double v = (pj[k] - pi[k]) + image_shift(S, c, k);
     d2 = k == 0 ? v * v : d2 + v * v;
   }
   return d2 < rc2;
 }
 
-// One wavefront per atom.  FILL = false: degree[i] = number of neighbours.  FILL = true: the neighbours (j, S) are
-// written to scratch[offsets[i] ...] in scan order (j in scratch[0:E], S in scratch[E:4E]).
-template <bool FILL>
-__global__ __launch_bounds__(256) void nl_scan_kernel(const double *__restrict__ pos, const Grid *__restrict__ grid,
-                                                      const int32_t *__restrict__ wrap, const int32_t *__restrict__ keys,
-                                                      const int32_t *__restrict__ cell_perm,
-                                                      const int32_t *__restrict__ cell_offsets, double cutoff, int nnodes,
-                                                      const int32_t *__restrict__ offsets, int64_t nedges,
-                                                      int32_t *__restrict__ degree, int32_t *__restrict__ scratch) {
-  const int lane = threadIdx.x % kWave;
-  const int i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  if (i >= nnodes) return;
-  const int nb0 = grid->nb[0], nb1 = grid->nb[1], nb2 = grid->nb[2];
-  const int key = keys[i];
-  const int bi[3] = {key / (nb1 * nb2), (key / nb2) % nb1, key % nb2};
-  const int wi[3] = {wrap[3 * i], wrap[3 * i + 1], wrap[3 * i + 2]};
-  const double pi[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-  const double rc2 = cutoff * cutoff;
-  const double *c = grid->cellv;
-  const int64_t seg = FILL ? offsets[i] : 0;
-  int count = 0;
-  if (grid->status == 0) {
-    for (int d0 = -grid->nscan[0]; d0 <= grid->nscan[0]; ++d0) {
-      int b0 = bi[0] + d0, B0 = 0;
-      if (grid->periodic[0]) {
-        B0 = floor_div(b0, nb0);
-        b0 -= B0 * nb0;
-      } else if (b0 < 0 || b0 >= nb0) {
-        continue;
-      }
-      for (int d1 = -grid->nscan[1]; d1 <= grid->nscan[1]; ++d1) {
-        int b1 = bi[1] + d1, B1 = 0;
-        if (grid->periodic[1]) {
-          B1 = floor_div(b1, nb1);
-          b1 -= B1 * nb1;
-        } else if (b1 < 0 || b1 >= nb1) {
-          continue;
-        }
-        for (int d2 = -grid->nscan[2]; d2 <= grid->nscan[2]; ++d2) {
-          int b2 = bi[2] + d2, B2 = 0;
-          if (grid->periodic[2]) {
-            B2 = floor_div(b2, nb2);
-            b2 -= B2 * nb2;
-          } else if (b2 < 0 || b2 >= nb2) {
-            continue;
-          }
-          const int cellid = (b0 * nb1 + b1) * nb2 + b2;
-          const int k0 = cell_offsets[cellid], k1 = cell_offsets[cellid + 1];
-          for (int kb = k0; kb < k1; kb += kWave) {
-            const int k = kb + lane;
-            bool hit = false;
-            int j = 0;
-            int S[3] = {0, 0, 0};
-            if (k < k1) {
-              j = cell_perm[k];
-              S[0] = B0 + wi[0] - wrap[3 * j];
-              S[1] = B1 + wi[1] - wrap[3 * j + 1];
-              S[2] = B2 + wi[2] - wrap[3 * j + 2];
-              const double pj[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
-              hit = within(pi, pj, S, c, rc2) && !(j == i && S[0] == 0 && S[1] == 0 && S[2] == 0);
-            }
-            const unsigned long long mask = __ballot(hit);
-            if constexpr (FILL) {
-              if (hit) {
-                const int64_t at = seg + count + __popcll(mask & ((1ull << lane) - 1ull));
-                if (at < nedges) {
-                  scratch[at] = j;
-                  scratch[nedges + 3 * at + 0] = S[0];
-                  scratch[nedges + 3 * at + 1] = S[1];
-                  scratch[nedges + 3 * at + 2] = S[2];
-                }
-              }
-            }
-            count += __popcll(mask);
-          }
-        }
-      }
-    }
-  }
-  if constexpr (!FILL) {
-    if (lane == 0) degree[i] = count;
-  }
-}
-
-// offsets[0 .. n] = exclusive scan of degree[0 .. n-1]; one workgroup, every thread a contiguous run.
-__global__ __launch_bounds__(kGridThreads) void nl_offsets_kernel(const int32_t *__restrict__ degree, int n,
-                                                                  int32_t *__restrict__ offsets) {
-  __shared__ long long part[kGridThreads];
-  __shared__ long long stage[kOffsetsStage];
-  const long long total = workgroup_exclusive_scan<kGridThreads, kOffsetsStage, long long>(
-      n, stage, part, [&](int k) { return degree[k]; },
-      [&](int k, long long before, long long) { offsets[k] = static_cast<int32_t>(before > INT32_MAX ? INT32_MAX : before); });
-  if (threadIdx.x == 0) offsets[n] = static_cast<int32_t>(total > INT32_MAX ? INT32_MAX : total);
-}
+// What the last pass writes when it has a segment's hits in LDS: the list in every form its consumers take.
+struct GraphOut {
+  int32_t *row_i, *row_j;   // [E]
+  int64_t *edge_index;      // [2, E]
+  double *unit_shifts;      // [E, 3]
+  double *shifts;           // [E, 3]
+  int32_t *first_occ;       // [2 N]
+  int64_t *batch, *ptr;     // [N] zeros, {0, N}; may be NULL
+  int32_t *ptr32;           // {0, N}; may be NULL
+};
 
 __device__ __forceinline__ bool key_less(int ja, const int32_t *Sa, int jb, const int32_t *Sb) {
   if (ja != jb) return ja < jb;
   if (Sa[0] != Sb[0]) return Sa[0] < Sb[0];
   if (Sa[1] != Sb[1]) return Sa[1] < Sb[1];
   return Sa[2] < Sb[2];
+}
+
+// One wavefront per atom, atoms in bin order (the waves of a workgroup share their candidates).
+//   COUNT     degree[i] = number of neighbours
+//   SCRATCH   the neighbours (j, S) in scan order to scratch[offsets[i] ...] (j in scratch[0:E], S in scratch[E:4E])
+//   GRAPH     the neighbours collected in LDS (`cap` of them per wave), each written to its rank under the (j, S) order
+enum class Scan { kCount, kScratch, kGraph };
+constexpr int kScanWaves = 4;
+template <Scan MODE>
+__global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w, double cutoff, int nnodes,
+                                                                     const int32_t *__restrict__ offsets, int64_t nedges,
+                                                                     int32_t *__restrict__ scratch, GraphOut out, int cap) {
+  __shared__ int s_before[kScanWaves][kWave], s_first[kScanWaves][kWave], s_image[kScanWaves][kWave];
+  extern __shared__ int s_hits[];  // GRAPH: per wave cap neighbours, then cap images of three
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int at = blockIdx.x * (blockDim.x / kWave) + wave;
+  if (at >= nnodes) return;
+  const Grid *grid = w.grid;
+  const int nb0 = grid->nb[0], nb1 = grid->nb[1], nb2 = grid->nb[2];
+  const int per0 = grid->periodic[0], per1 = grid->periodic[1], per2 = grid->periodic[2];
+  const int r0 = grid->nscan[0], r1 = grid->nscan[1], r2 = grid->nscan[2];
+  const int key = w.skey[at];
+  const int4 me = w.smeta[at];
+  const int i = me.x;
+  const int wi[3] = {me.y, me.z, me.w};
+  const double pi[3] = {w.spos[3 * static_cast<int64_t>(at)], w.spos[3 * static_cast<int64_t>(at) + 1], w.spos[3 * static_cast<int64_t>(at) + 2]};
+  const int bi0 = key / (nb1 * nb2), bi1 = (key / nb2) % nb1, bi2 = key % nb2;
+  const double rc2 = cutoff * cutoff;
+  double c[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) c[k] = grid->cellv[k];
+  const int64_t seg = MODE == Scan::kCount ? 0 : offsets[i];
+  int *hj = s_hits + wave * 4 * cap, *hS = hj + cap;
+  int count = 0;
+  const int m1 = 2 * r1 + 1, m2 = 2 * r2 + 1;
+  const int nscan = grid->status == 0 ? (2 * r0 + 1) * m1 * m2 : 0;
+  for (int first_bin = 0; first_bin < nscan; first_bin += kWave) {
+    // 64 bins side by side: where their atoms begin, how many there are, which image of the cell they belong to
+    const int q = first_bin + lane;
+    int first = 0, cnt = 0, image = 0;
+    if (q < nscan) {
+      int b0 = bi0 + q / (m1 * m2) - r0, b1 = bi1 + (q / m2) % m1 - r1, b2 = bi2 + q % m2 - r2;
+      int B0 = 0, B1 = 0, B2 = 0;
+      if (per0) B0 = floor_div(b0, nb0), b0 -= B0 * nb0;
+      if (per1) B1 = floor_div(b1, nb1), b1 -= B1 * nb1;
+      if (per2) B2 = floor_div(b2, nb2), b2 -= B2 * nb2;
+      if (b0 >= 0 && b0 < nb0 && b1 >= 0 && b1 < nb1 && b2 >= 0 && b2 < nb2) {
+        const int id = (b0 * nb1 + b1) * nb2 + b2;
+        first = w.cell_offsets[id];
+        cnt = w.cell_offsets[id + 1] - first;
+        image = (B0 + 128) | (B1 + 128) << 8 | (B2 + 128) << 16;  // |B| <= kMaxScan
+      }
+    }
+    int upto = cnt;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int v = __shfl_up(upto, d);
+      if (lane >= d) upto += v;
+    }
+    const int total = __shfl(upto, kWave - 1);
+    wave_lds_fence();  // the previous bins' tables have been read
+    s_before[wave][lane] = upto - cnt;
+    s_first[wave][lane] = first;
+    s_image[wave][lane] = image;
+    wave_lds_fence();
+    for (int base = 0; base < total; base += kWave) {
+      const int cand = base + lane;
+      bool hit = false;
+      int j = 0;
+      int S[3] = {0, 0, 0};
+      if (cand < total) {
+        int b = 0;  // the last bin whose atoms begin at or before cand: it is not empty, since cand < total
+#pragma unroll
+        for (int step = kWave / 2; step > 0; step >>= 1)
+          if (s_before[wave][b + step] <= cand) b += step;
+        const int64_t k = s_first[wave][b] + (cand - s_before[wave][b]);
+        const int img = s_image[wave][b];
+        const int4 meta = w.smeta[k];
+        const double pj[3] = {w.spos[3 * k], w.spos[3 * k + 1], w.spos[3 * k + 2]};
+        j = meta.x;
+        S[0] = (img & 255) - 128 + wi[0] - meta.y;
+        S[1] = (img >> 8 & 255) - 128 + wi[1] - meta.z;
+        S[2] = (img >> 16 & 255) - 128 + wi[2] - meta.w;
+        hit = within(pi, pj, S, c, rc2) && !(j == i && S[0] == 0 && S[1] == 0 && S[2] == 0);
+      }
+      const unsigned long long mask = __ballot(hit);
+      const int mine = count + __popcll(mask & ((1ull << lane) - 1ull));
+      if constexpr (MODE == Scan::kScratch) {
+        if (hit && seg + mine < nedges) {
+          scratch[seg + mine] = j;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) scratch[nedges + 3 * (seg + mine) + k] = S[k];
+        }
+      }
+      if constexpr (MODE == Scan::kGraph) {
+        if (hit && mine < cap) {
+          hj[mine] = j;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) hS[3 * mine + k] = S[k];
+        }
+      }
+      count += __popcll(mask);
+    }
+  }
+  if constexpr (MODE == Scan::kCount) {
+    if (lane == 0) w.degree[i] = count;
+  }
+  if constexpr (MODE == Scan::kGraph) {
+    wave_lds_fence();
+    const int d = min(min(count, cap), static_cast<int>(min(static_cast<int64_t>(offsets[i + 1]), nedges) - seg));
+    for (int e = lane; e < d; e += kWave) {
+      const int j = hj[e];
+      const int S[3] = {hS[3 * e], hS[3 * e + 1], hS[3 * e + 2]};
+      int rank = 0;
+      for (int q = 0; q < d; ++q) {
+        const int jq = hj[q];
+        rank += jq < j ? 1 : 0;
+        if (jq == j && q != e) rank += key_less(jq, hS + 3 * q, j, S) ? 1 : 0;
+      }
+      const int64_t to = seg + rank;
+      out.row_i[to] = i;
+      out.row_j[to] = j;
+      out.edge_index[to] = i;
+      out.edge_index[nedges + to] = j;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        out.unit_shifts[3 * to + k] = S[k];
+        out.shifts[3 * to + k] = image_shift(S, c, k);
+      }
+    }
+    if (lane == 0) {
+      out.first_occ[i] = offsets[i];
+      out.first_occ[nnodes + i] = offsets[i + 1];
+      if (out.batch) out.batch[i] = 0;
+      if (at == 0) {
+        if (out.ptr) out.ptr[0] = 0, out.ptr[1] = nnodes;
+        if (out.ptr32) out.ptr32[0] = 0, out.ptr32[1] = nnodes;
+      }
+    }
+  }
+}
+
+// offsets[0 .. n] = exclusive scan of degree[0 .. n-1] and, next to it, the grid's status and the largest degree; one
+// workgroup, every thread a contiguous run.
+__global__ __launch_bounds__(kGridThreads) void nl_offsets_kernel(Workspace w, int n, int32_t *__restrict__ offsets,
+                                                                  int32_t *__restrict__ status, int32_t *__restrict__ max_degree) {
+  __shared__ long long part[kGridThreads];
+  __shared__ long long stage[kOffsetsStage];
+  __shared__ int s_most[kGridThreads / kWave];
+  int most = 0;
+  const long long total = workgroup_exclusive_scan<kGridThreads, kOffsetsStage, long long>(
+      n, stage, part, [&](int k) { return w.degree[k]; },
+      [&](int k, long long before, long long value) {
+        offsets[k] = static_cast<int32_t>(before > INT32_MAX ? INT32_MAX : before);
+        most = max(most, static_cast<int>(value));
+      });
+  for (int d = kWave / 2; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d));
+  if (threadIdx.x % kWave == 0) s_most[threadIdx.x / kWave] = most;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    offsets[n] = static_cast<int32_t>(total > INT32_MAX ? INT32_MAX : total);
+    *status = w.grid->status;
+    for (int q = 1; q < kGridThreads / kWave; ++q) most = max(most, s_most[q]);
+    if (max_degree) *max_degree = most;
+  }
 }
 
 // One wavefront per atom: every hit of its segment goes to its rank under the (j, S) order.
@@ -362,6 +558,48 @@ __global__ __launch_bounds__(256) void nl_rank_kernel(const int32_t *__restrict_
     unit_shifts[3 * at + 1] = S[1];
     unit_shifts[3 * at + 2] = S[2];
   }
+}
+
+// The view of a list sorted by row j, for a list that holds the reverse (j, i, -S) of each of its pairs (i, j, S), as every
+// list of this file does: the pairs sent by s are then the reverses of the pairs of s, in the order of (j, -S), so the view's
+// offsets are the list's own and an entry is found by a binary search in the segment of j.  One launch in place of a
+// counting sort's five.
+__device__ __forceinline__ int compare_pair(int ja, double a0, double a1, double a2, int jb, const double *Sb) {
+  if (ja != jb) return ja < jb ? -1 : 1;
+  if (a0 != Sb[0]) return a0 < Sb[0] ? -1 : 1;
+  if (a1 != Sb[1]) return a1 < Sb[1] ? -1 : 1;
+  if (a2 != Sb[2]) return a2 < Sb[2] ? -1 : 1;
+  return 0;
+}
+__global__ __launch_bounds__(256) void nl_sender_view_kernel(const int32_t *__restrict__ row_i, const int32_t *__restrict__ row_j,
+                                                             const double *__restrict__ unit_shifts,
+                                                             const int32_t *__restrict__ first_occ, int nnodes, int64_t nedges,
+                                                             int32_t *__restrict__ perm) {
+  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (e >= nedges) return;
+  const int i = row_i[e], j = row_j[e];
+  const bool good = static_cast<unsigned>(i) < static_cast<unsigned>(nnodes) && static_cast<unsigned>(j) < static_cast<unsigned>(nnodes);
+  if (!good) {  // not a list of this file: some place, inside the view
+    perm[e] = static_cast<int32_t>(e);
+    return;
+  }
+  const double s0 = -unit_shifts[3 * e], s1 = -unit_shifts[3 * e + 1], s2 = -unit_shifts[3 * e + 2];
+  int lo = first_occ[j], hi = first_occ[nnodes + j];
+  clamp_edge_range(lo, hi, nedges);
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (compare_pair(i, s0, s1, s2, row_j[mid], unit_shifts + 3 * static_cast<int64_t>(mid)) > 0)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  // images of one neighbour come in the opposite order
+  int a0 = first_occ[i], b0 = first_occ[nnodes + i];
+  clamp_edge_range(a0, b0, nedges);
+  int64_t a = e, b = e;
+  while (a > a0 && row_j[a - 1] == j) --a;
+  while (b + 1 < b0 && row_j[b + 1] == j) ++b;
+  perm[a + (b - e)] = static_cast<int32_t>(min(static_cast<int64_t>(lo), nedges - 1));
 }
 
 // ---- the test a Verlet list needs before it is reused: how far has any atom moved since the list was built ----
@@ -411,42 +649,51 @@ extern "C" size_t cm_neighbour_list_workspace(int64_t nnodes, int64_t max_cells)
   return cm::carve(nullptr, nnodes, max_cells).total;
 }
 
+namespace cm {
+namespace {
+
+// Everything up to the offsets of the segments: the cell list and the count of every atom's neighbours.
+int search(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z, double cutoff, int64_t nnodes, int64_t max_cells,
+           void *workspace, size_t workspace_bytes, int32_t *offsets, int32_t *status, int32_t *max_degree, hipStream_t st,
+           const char *what) {
+  CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4, "%s: nnodes out of range", what);
+  CM_REQUIRE(max_cells >= 1 && max_cells < INT32_MAX / 2, "%s: max_cells out of range", what);
+  CM_REQUIRE(cutoff > 0.0 && std::isfinite(cutoff), "%s: cutoff must be positive and finite", what);
+  CM_REQUIRE(offsets != nullptr && status != nullptr, "%s: offsets / status is NULL", what);
+  CM_REQUIRE(nnodes == 0 || positions != nullptr, "%s: positions is NULL", what);
+  CM_REQUIRE(cell != nullptr || !(pbc_x || pbc_y || pbc_z), "%s: a periodic axis needs a cell", what);
+  const Workspace w = carve(workspace, nnodes, max_cells);
+  if (workspace == nullptr || workspace_bytes < w.total) {
+    set_error("%s: workspace of %zu bytes, need %zu", what, workspace_bytes, w.total);
+    return CM_ENOSPC;
+  }
+  const int n = static_cast<int>(nnodes), cells = static_cast<int>(max_cells);
+  if (n <= kSmallAtoms && cells <= kSmallAtoms) {
+    hipLaunchKernelGGL(nl_cells_small_kernel, dim3(1), dim3(kGridThreads), static_cast<unsigned>(cells * sizeof(int)), st, positions, cell,
+                       pbc_x, pbc_y, pbc_z, cutoff, n, cells, w);
+  } else {
+    const dim3 per_atom(static_cast<unsigned>(ceil_div(std::max(n, 1), 256))), block(256);
+    hipLaunchKernelGGL(nl_grid_kernel, dim3(1), dim3(kGridThreads), 0, st, positions, cell, pbc_x, pbc_y, pbc_z, cutoff, n, cells, w.grid);
+    hipLaunchKernelGGL(nl_clear_kernel, dim3(static_cast<unsigned>(ceil_div(cells, 256))), block, 0, st, w.cell_count, cells);
+    hipLaunchKernelGGL(nl_bin_kernel, per_atom, block, 0, st, positions, n, w);
+    hipLaunchKernelGGL(nl_cell_scan_kernel, dim3(1), dim3(kGridThreads), 0, st, cells, w);
+    hipLaunchKernelGGL(nl_place_kernel, per_atom, block, 0, st, positions, n, w);
+  }
+  if (n > 0)
+    hipLaunchKernelGGL(nl_scan_kernel<Scan::kCount>, dim3(static_cast<unsigned>(ceil_div(n, kScanWaves))), dim3(kScanWaves * kWave), 0, st,
+                       w, cutoff, n, static_cast<const int32_t *>(nullptr), int64_t{0}, static_cast<int32_t *>(nullptr), GraphOut{}, 0);
+  hipLaunchKernelGGL(nl_offsets_kernel, dim3(1), dim3(kGridThreads), 0, st, w, n, offsets, status, max_degree);
+  return check_launch(what);
+}
+
+}  // namespace
+}  // namespace cm
+
 extern "C" int cm_neighbour_list_count(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z,
                                        double cutoff, int64_t nnodes, int64_t max_cells, void *workspace,
                                        size_t workspace_bytes, int32_t *offsets, int32_t *status, cm_stream_t stream) {
-  CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4, "cm_neighbour_list_count: nnodes out of range");
-  CM_REQUIRE(max_cells >= 1 && max_cells < INT32_MAX / 2, "cm_neighbour_list_count: max_cells out of range");
-  CM_REQUIRE(cutoff > 0.0 && std::isfinite(cutoff), "cm_neighbour_list_count: cutoff must be positive and finite");
-  CM_REQUIRE(offsets != nullptr && status != nullptr, "cm_neighbour_list_count: offsets / status is NULL");
-  CM_REQUIRE(nnodes == 0 || positions != nullptr, "cm_neighbour_list_count: positions is NULL");
-  CM_REQUIRE(cell != nullptr || !(pbc_x || pbc_y || pbc_z), "cm_neighbour_list_count: a periodic axis needs a cell");
-  const cm::Workspace w = cm::carve(workspace, nnodes, max_cells);
-  if (workspace == nullptr || workspace_bytes < w.total) {
-    cm::set_error("cm_neighbour_list_count: workspace of %zu bytes, need %zu", workspace_bytes, w.total);
-    return CM_ENOSPC;
-  }
-  hipStream_t st = cm::as_stream(stream);
-  const int n = static_cast<int>(nnodes);
-  hipLaunchKernelGGL(cm::nl_grid_kernel, dim3(1), dim3(cm::kGridThreads), 0, st, positions, cell, pbc_x, pbc_y, pbc_z, cutoff, n,
-                     static_cast<int>(max_cells), w.grid);
-  if (n > 0)
-    hipLaunchKernelGGL(cm::nl_bin_kernel, dim3(static_cast<unsigned>(cm::ceil_div(n, 256))), dim3(256), 0, st, positions, w.grid,
-                       n, w.wrap, w.keys);
-  int rc = cm::check_launch("cm_neighbour_list_count (binning)");
-  if (rc != CM_OK) return rc;
-  rc = cm_stable_key_sort(w.keys, nnodes, max_cells, w.cell_perm, w.cell_offsets, w.sort_ws, w.sort_ws_bytes, stream);
-  if (rc != CM_OK) return rc;
-  if (n > 0)
-    hipLaunchKernelGGL(cm::nl_scan_kernel<false>, dim3(static_cast<unsigned>(cm::ceil_div(n, 4))), dim3(256), 0, st, positions,
-                       w.grid, w.wrap, w.keys, w.cell_perm, w.cell_offsets, cutoff, n, static_cast<const int32_t *>(nullptr),
-                       int64_t{0}, w.degree, static_cast<int32_t *>(nullptr));
-  hipLaunchKernelGGL(cm::nl_offsets_kernel, dim3(1), dim3(cm::kGridThreads), 0, st, w.degree, n, offsets);
-  // the status word sits behind the grid header; copy it out with a kernel-free device-to-device copy
-  if (hipMemcpyAsync(status, &w.grid->status, sizeof(int32_t), hipMemcpyDeviceToDevice, st) != hipSuccess) {
-    cm::set_error("cm_neighbour_list_count: status copy failed");
-    return CM_ELAUNCH;
-  }
-  return cm::check_launch("cm_neighbour_list_count");
+  return cm::search(positions, cell, pbc_x, pbc_y, pbc_z, cutoff, nnodes, max_cells, workspace, workspace_bytes, offsets, status, nullptr,
+                    cm::as_stream(stream), "cm_neighbour_list_count");
 }
 
 extern "C" int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnodes, int64_t max_cells,
@@ -462,9 +709,58 @@ extern "C" int cm_neighbour_list_fill(const double *positions, double cutoff, in
   const cm::Workspace w = cm::carve(const_cast<void *>(workspace), nnodes, max_cells);
   hipStream_t st = cm::as_stream(stream);
   const int n = static_cast<int>(nnodes);
-  const dim3 grid(static_cast<unsigned>(cm::ceil_div(n, 4)));
-  hipLaunchKernelGGL(cm::nl_scan_kernel<true>, grid, dim3(256), 0, st, positions, w.grid, w.wrap, w.keys, w.cell_perm,
-                     w.cell_offsets, cutoff, n, offsets, nedges, static_cast<int32_t *>(nullptr), edge_scratch);
-  hipLaunchKernelGGL(cm::nl_rank_kernel, grid, dim3(256), 0, st, offsets, n, nedges, edge_scratch, row_i, row_j, unit_shifts);
+  const dim3 grid(static_cast<unsigned>(cm::ceil_div(n, cm::kScanWaves))), block(cm::kScanWaves * cm::kWave);
+  hipLaunchKernelGGL(cm::nl_scan_kernel<cm::Scan::kScratch>, grid, block, 0, st, w, cutoff, n, offsets, nedges, edge_scratch,
+                     cm::GraphOut{}, 0);
+  hipLaunchKernelGGL(cm::nl_rank_kernel, grid, block, 0, st, offsets, n, nedges, edge_scratch, row_i, row_j, unit_shifts);
   return cm::check_launch("cm_neighbour_list_fill");
+}
+
+extern "C" int cm_neighbour_list_search(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z,
+                                        double cutoff, int64_t nnodes, int64_t max_cells, void *workspace,
+                                        size_t workspace_bytes, int32_t *offsets, int32_t *status, int32_t *max_degree,
+                                        cm_stream_t stream) {
+  CM_REQUIRE(max_degree != nullptr, "cm_neighbour_list_search: max_degree is NULL");
+  return cm::search(positions, cell, pbc_x, pbc_y, pbc_z, cutoff, nnodes, max_cells, workspace, workspace_bytes, offsets, status,
+                    max_degree, cm::as_stream(stream), "cm_neighbour_list_search");
+}
+
+// A wave keeps a segment's hits in LDS, 16 bytes each: four waves per workgroup up to 512 of them, then one.
+static constexpr int kGraphMaxDegree = 8192;
+
+extern "C" int cm_neighbour_list_graph_max_degree(void) { return kGraphMaxDegree; }
+
+extern "C" int cm_neighbour_list_graph(double cutoff, int64_t nnodes, int64_t max_cells, const void *workspace, const int32_t *offsets,
+                                       int64_t nedges, int max_degree, int32_t *row_i, int32_t *row_j, int64_t *edge_index,
+                                       double *unit_shifts, double *shifts, int32_t *first_occ, int64_t *batch, int64_t *ptr,
+                                       int32_t *ptr32, cm_stream_t stream) {
+  CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4, "cm_neighbour_list_graph: nnodes out of range");
+  CM_REQUIRE(max_cells >= 1 && max_cells < INT32_MAX / 2, "cm_neighbour_list_graph: max_cells out of range");
+  CM_REQUIRE(nedges >= 0 && nedges < INT32_MAX / 4, "cm_neighbour_list_graph: nedges out of range");
+  CM_REQUIRE(max_degree >= 0 && max_degree <= kGraphMaxDegree, "cm_neighbour_list_graph: %d neighbours of one atom, at most %d", max_degree,
+             kGraphMaxDegree);
+  CM_REQUIRE(cutoff > 0.0 && std::isfinite(cutoff), "cm_neighbour_list_graph: cutoff must be positive and finite");
+  if (nnodes == 0) return CM_OK;
+  CM_REQUIRE(workspace && offsets && first_occ, "cm_neighbour_list_graph: NULL pointer");
+  CM_REQUIRE(nedges == 0 || (row_i && row_j && edge_index && unit_shifts && shifts), "cm_neighbour_list_graph: NULL edge output");
+  const cm::Workspace w = cm::carve(const_cast<void *>(workspace), nnodes, max_cells);
+  const int n = static_cast<int>(nnodes);
+  const int cap = std::max(kGraphMaxDegree > max_degree ? (max_degree + 63) / 64 * 64 : max_degree, 64);
+  const int waves = cap <= 512 ? cm::kScanWaves : 1;
+  hipLaunchKernelGGL(cm::nl_scan_kernel<cm::Scan::kGraph>, dim3(static_cast<unsigned>(cm::ceil_div(n, waves))), dim3(waves * cm::kWave),
+                     static_cast<unsigned>(waves * cap * 16), cm::as_stream(stream), w, cutoff, n, offsets, nedges,
+                     static_cast<int32_t *>(nullptr), cm::GraphOut{row_i, row_j, edge_index, unit_shifts, shifts, first_occ, batch, ptr, ptr32},
+                     cap);
+  return cm::check_launch("cm_neighbour_list_graph");
+}
+
+extern "C" int cm_symmetric_sender_view(const int32_t *row_i, const int32_t *row_j, const double *unit_shifts,
+                                        const int32_t *first_occ, int64_t nnodes, int64_t nedges, int32_t *sender_perm,
+                                        cm_stream_t stream) {
+  CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4 && nedges >= 0 && nedges < INT32_MAX / 4, "cm_symmetric_sender_view: sizes out of range");
+  if (nedges == 0) return CM_OK;
+  CM_REQUIRE(row_i && row_j && unit_shifts && first_occ && sender_perm, "cm_symmetric_sender_view: NULL pointer");
+  hipLaunchKernelGGL(cm::nl_sender_view_kernel, dim3(static_cast<unsigned>(cm::ceil_div(nedges, 256))), dim3(256), 0,
+                     cm::as_stream(stream), row_i, row_j, unit_shifts, first_occ, static_cast<int>(nnodes), nedges, sender_perm);
+  return cm::check_launch("cm_symmetric_sender_view");
 }

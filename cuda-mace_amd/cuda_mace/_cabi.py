@@ -72,6 +72,10 @@ SIGNATURES = {
     "cm_neighbour_list_workspace": (_sz, [_i64, _i64]),
     "cm_neighbour_list_count": (_i32, [_p, _p, _i32, _i32, _i32, _f64, _i64, _i64, _p, _sz, _p, _p, _p]),
     "cm_neighbour_list_fill": (_i32, [_p, _f64, _i64, _i64, _p, _p, _i64, _p, _p, _p, _p, _p]),
+    "cm_neighbour_list_search": (_i32, [_p, _p, _i32, _i32, _i32, _f64, _i64, _i64, _p, _sz, _p, _p, _p, _p]),
+    "cm_neighbour_list_graph_max_degree": (_i32, []),
+    "cm_neighbour_list_graph": (_i32, [_f64, _i64, _i64, _p, _p, _i64, _i32] + [_p] * 10),
+    "cm_symmetric_sender_view": (_i32, [_p, _p, _p, _p, _i64, _i64, _p, _p]),
     "cm_max_displacement": (_i32, [_p, _p, _i64, _p, _p]),
     # the whole step: (weights struct *, graph struct *, positions, shifts, workspace, bytes, 4 outputs, stream)
     "cm_mace_step_timing": (_i32, [ctypes.c_uint]),
@@ -590,6 +594,15 @@ def symcon_backward(grad, grad_out) -> torch.Tensor:
 # ---- neighbour list -------------------------------------------------------------------------------
 def neighbour_list(positions, cell, pbc, cutoff: float, max_cells: int = 0):
     """(row_i int32 [E], row_j int32 [E], unit_shifts int32 [E, 3]) sorted by (i, j, S); positions fp64 [N, 3] and
+def _list_status(E: int, status: int) -> None:
+    if status == 1:
+        raise CudaMaceError("neighbour list: a periodic axis needs a non-singular cell")
+    if status != 0:
+        raise CudaMaceError("neighbour list: the cell is thinner than cutoff / 32 along a periodic axis")
+    if E >= 2**31 // 4 - 1:
+        raise CudaMaceError("neighbour list: more pairs than int32 indexing holds")
+
+
     cell fp64 [3, 3] (or None) on the device, pbc three booleans.  One host synchronisation (the number of pairs)."""
     N = positions.shape[0]
     dev = positions.device
@@ -604,13 +617,8 @@ def neighbour_list(positions, cell, pbc, cutoff: float, max_cells: int = 0):
             ws.data_ptr(), ws_bytes, head.data_ptr(), head.data_ptr() + 4 * (N + 1), _stream(),
         )
     )
-    E, status = (int(v) for v in head[N:].tolist())
-    if status == 1:
-        raise CudaMaceError("neighbour list: a periodic axis needs a non-singular cell")
-    if status != 0:
-        raise CudaMaceError("neighbour list: the cell is thinner than cutoff / 32 along a periodic axis")
-    if E >= 2**31 // 4 - 1:
-        raise CudaMaceError("neighbour list: more pairs than int32 indexing holds")
+    E, status = head[N:].tolist()
+    _list_status(E, status)
     row_i = torch.empty(E, dtype=I32, device=dev)
     row_j = torch.empty(E, dtype=I32, device=dev)
     S = torch.empty(E, 3, dtype=I32, device=dev)
@@ -627,6 +635,56 @@ def neighbour_list(positions, cell, pbc, cutoff: float, max_cells: int = 0):
 
 def max_displacement(positions, reference, out=None):
     """fp64 [1] on the device: the largest squared distance between the rows of `positions` and `reference` (fp64
+_GRAPH_MAX_DEGREE = lib.cm_neighbour_list_graph_max_degree()
+
+
+def neighbour_graph(positions, cell, pbc, cutoff: float, max_cells: int = 0):
+    """The list of `neighbour_list` in every form the model takes it, as a dict: row_i, row_j int32 [E], edge_index int64
+    [2, E], unit_shifts and shifts fp64 [E, 3], first_occ int32 [2 N] (CSR of row_i), offsets int32 [N + 1] (which is
+    also where the pairs sent by an atom begin in the view sorted by row_j), batch int64 [N] and ptr int64 / int32 [2] of
+    the one graph.  One host synchronisation (the number of pairs)."""
+    N = positions.shape[0]
+    dev = positions.device
+    I64 = torch.int64
+    max_cells = int(max_cells) if max_cells else max(1, min(N, 1 << 22))
+    ws_bytes = lib.cm_neighbour_list_workspace(N, max_cells)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    head = torch.empty(N + 3, dtype=I32, device=dev)  # offsets [N + 1], status, largest degree
+    offsets_ptr = head.data_ptr()
+    px, py, pz = (int(bool(b)) for b in pbc)
+    stream = _stream()
+    _check(lib.cm_neighbour_list_search(_dev(positions, F64, "positions"), _dev(cell, F64, "cell"), px, py, pz, float(cutoff), N, max_cells,
+                                        ws.data_ptr(), ws_bytes, offsets_ptr, offsets_ptr + 4 * (N + 1), offsets_ptr + 4 * (N + 2), stream))
+    E, status, most = head[N:].tolist()
+    _list_status(E, status)
+    if most > _GRAPH_MAX_DEGREE:
+        return None
+    row_i, row_j = torch.empty(E, dtype=I32, device=dev), torch.empty(E, dtype=I32, device=dev)
+    edge_index = torch.empty(2, E, dtype=I64, device=dev)
+    unit_shifts, shifts = torch.empty(E, 3, dtype=F64, device=dev), torch.empty(E, 3, dtype=F64, device=dev)
+    first_occ = torch.empty(2 * N, dtype=I32, device=dev)
+    batch, ptr = torch.empty(N, dtype=I64, device=dev), torch.empty(2, dtype=I64, device=dev)
+    ptr32 = torch.empty(2, dtype=I32, device=dev)
+    if N > 0:
+        at = lambda t: t.data_ptr() if E > 0 else None  # noqa: E731
+        _check(lib.cm_neighbour_list_graph(float(cutoff), N, max_cells, ws.data_ptr(), offsets_ptr, E, most, at(row_i), at(row_j),
+                                           at(edge_index), at(unit_shifts), at(shifts), first_occ.data_ptr(), batch.data_ptr(),
+                                           ptr.data_ptr(), ptr32.data_ptr(), stream))
+    else:
+        ptr.zero_(), ptr32.zero_()
+    return {"row_i": row_i, "row_j": row_j, "edge_index": edge_index, "unit_shifts": unit_shifts, "shifts": shifts,
+            "first_occ": first_occ, "offsets": head[:N + 1], "batch": batch, "ptr": ptr, "ptr32": ptr32}
+
+
+def symmetric_sender_view(row_i, row_j, unit_shifts, first_occ, nnodes: int):
+    """The permutation of stable_key_sort(row_j, nnodes) for a list that holds the reverse of each of its pairs."""
+    E = row_i.numel()
+    perm = torch.empty(E, dtype=I32, device=row_i.device)
+    _check(lib.cm_symmetric_sender_view(_dev(row_i, I32, "row_i"), _dev(row_j, I32, "row_j"), _dev(unit_shifts, F64, "unit_shifts"),
+                                        _dev(first_occ, I32, "first_occ"), nnodes, E, _dev(perm, I32, "sender_perm"), _stream()))
+    return perm
+
+
     [N, 3]); nothing is read back here."""
     N = positions.shape[0]
     if reference.shape != positions.shape:

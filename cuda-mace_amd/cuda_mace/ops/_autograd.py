@@ -111,7 +111,16 @@ def csr_of(receiver: torch.Tensor, nnodes: int) -> torch.Tensor:
 
 
 def sender_view_of(sender: torch.Tensor, nnodes: int):
-    return _cached(sender, "_cm_sender_view", nnodes, lambda: cabi.stable_key_sort(sender, nnodes))
+    def build():
+        # a list of the device search knows that it holds the reverse of each of its pairs: no sort is needed
+        known = sender.__dict__.get("_cm_symmetric_list")
+        if known is not None:
+            row_i, unit_shifts, first_occ, offsets, versions = known
+            if versions == (sender._version, row_i._version, unit_shifts._version) and offsets.numel() == nnodes + 1:
+                return cabi.symmetric_sender_view(row_i, sender, unit_shifts, first_occ, nnodes), offsets
+        return cabi.stable_key_sort(sender, nnodes)
+
+    return _cached(sender, "_cm_sender_view", nnodes, build)
 
 
 def groups_of(atom_types: torch.Tensor, nelements: int):

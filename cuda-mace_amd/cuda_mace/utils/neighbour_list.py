@@ -50,28 +50,46 @@ def get_neighborhood(positions: torch.Tensor, cutoff: float, pbc: Optional[Seque
                      max_cells: int = 0):
     """(edge_index, shifts, unit_shifts, cell) like upstream's helper of the same name, computed on the GPU that
     holds `positions`."""
+    return _search(positions, cutoff, pbc, cell, max_cells)[:4]
+
+
+def _search(positions: torch.Tensor, cutoff: float, pbc, cell, max_cells: int = 0):
+    """(edge_index, shifts, unit_shifts, cell, batch or None, ptr or None)"""
     if not positions.is_cuda:
         raise cabi.CudaMaceError("get_neighborhood: positions must live on the GPU")
     pos = positions.detach().double().contiguous()
     cell_t, pbc = _cell_and_pbc(cell, pbc, pos.device)
-    row_i, row_j, S = cabi.neighbour_list(pos, cell_t, pbc, float(cutoff), max_cells)
-    edge_index = torch.stack([row_i, row_j]).long()
-    # the model derives int32 rows from edge_index once per list; hand it the ones that already exist
+    n = pos.shape[0]
+    batch = ptr = None
+    g = cabi.neighbour_graph(pos, cell_t, pbc, float(cutoff), max_cells)
+    if g is not None:
+        # what the model derives from a list once is already there: leave it where it is looked up
+        edge_index, shifts, unit_shifts, row_i, row_j = g["edge_index"], g["shifts"], g["unit_shifts"], g["row_i"], g["row_j"]
+        batch, ptr, ptr32 = g["batch"], g["ptr"], g["ptr32"]
+        row_i.__dict__["_cm_csr"] = ((row_i._version, row_i.data_ptr(), n), g["first_occ"])
+        row_j.__dict__["_cm_symmetric_list"] = (row_i, unit_shifts, g["first_occ"], g["offsets"],
+                                                (row_j._version, row_i._version, unit_shifts._version))
+        ptr.__dict__["_cm_ptr32"] = ((ptr._version, ptr.data_ptr(), None), ptr32)
+    else:  # an atom with thousands of neighbours
+        row_i, row_j, S = cabi.neighbour_list(pos, cell_t, pbc, float(cutoff), max_cells)
+        edge_index = torch.stack([row_i, row_j]).long()
+        unit_shifts = S.double()
+        shifts = shifts_from_unit_shifts(S, cell_t)
     edge_index.__dict__["_cm_int32_rows"] = ((edge_index._version, edge_index.data_ptr(), None), (row_i, row_j))
-    unit_shifts = S.double()
-    shifts = shifts_from_unit_shifts(S, cell_t)
     if cell_t is None:
         cell_t = torch.zeros(3, 3, dtype=torch.float64, device=pos.device)
-    return edge_index, shifts, unit_shifts, cell_t
+    return edge_index, shifts, unit_shifts, cell_t, batch, ptr
 
 
 def neighbour_data(positions: torch.Tensor, node_attrs: torch.Tensor, cutoff: float, pbc=None, cell=None) -> Dict[str, torch.Tensor]:
     """The `data` dictionary of a single graph for OptimizedInvariantMACE.forward, neighbour list included."""
-    edge_index, shifts, unit_shifts, cell_t = get_neighborhood(positions, cutoff, pbc, cell)
+    edge_index, shifts, unit_shifts, cell_t, batch, ptr = _search(positions, cutoff, pbc, cell)
     n = positions.shape[0]
     dev = positions.device
+    if batch is None:
+        batch = torch.zeros(n, dtype=torch.int64, device=dev)
+        ptr = torch.tensor([0, n], dtype=torch.int64, device=dev)
     return {
-        "positions": positions, "node_attrs": node_attrs, "batch": torch.zeros(n, dtype=torch.int64, device=dev),
-        "ptr": torch.tensor([0, n], dtype=torch.int64, device=dev), "edge_index": edge_index, "unit_shifts": unit_shifts,
-        "shifts": shifts, "cell": cell_t,
+        "positions": positions, "node_attrs": node_attrs, "batch": batch, "ptr": ptr, "edge_index": edge_index,
+        "unit_shifts": unit_shifts, "shifts": shifts, "cell": cell_t,
     }

@@ -382,6 +382,28 @@ int cm_neighbour_list_count(const double *positions, const double *cell, int pbc
 int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnodes, int64_t max_cells,
                            const void *workspace, const int32_t *offsets, int64_t nedges, int32_t *edge_scratch,
                            int32_t *row_i, int32_t *row_j, int32_t *unit_shifts, cm_stream_t stream);
+/* The same list with everything the model reads of it, in two calls that launch three kernels and one (up to 32 768
+ * atoms):
+ *   cm_neighbour_list_search: cm_neighbour_list_count, and max_degree int32 [1] = the most neighbours of one atom.
+ *   cm_neighbour_list_graph: after the caller has read offsets[nnodes] = nedges and max_degree (at most
+ *     cm_neighbour_list_graph_max_degree(); beyond that, cm_neighbour_list_fill), writes row_i, row_j int32 [nedges],
+ *     edge_index int64 [2, nedges] (the same rows), unit_shifts fp64 [nedges, 3], shifts fp64 [nedges, 3] = S . cell (term by
+ *     term from the left, no fused multiply-adds), first_occ int32 [2 nnodes] = cm_first_occurences(row_i) and, where not
+ *     NULL, batch int64 [nnodes] = 0, ptr int64 [2] and ptr32 int32 [2] = {0, nnodes} (one graph).  `workspace` as for
+ *     cm_neighbour_list_fill.
+ *   cm_symmetric_sender_view: sender_perm int32 [nedges] of such a list, the permutation of cm_stable_key_sort(row_j,
+ *     nedges, nnodes): a list that holds the reverse of each of its pairs needs no sort for it, and its sender offsets are
+ *     the list's own offsets. */
+int cm_neighbour_list_search(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z, double cutoff,
+                             int64_t nnodes, int64_t max_cells, void *workspace, size_t workspace_bytes, int32_t *offsets,
+                             int32_t *status, int32_t *max_degree, cm_stream_t stream);
+int cm_neighbour_list_graph_max_degree(void);
+int cm_neighbour_list_graph(double cutoff, int64_t nnodes, int64_t max_cells, const void *workspace, const int32_t *offsets,
+                            int64_t nedges, int max_degree, int32_t *row_i, int32_t *row_j, int64_t *edge_index,
+                            double *unit_shifts, double *shifts, int32_t *first_occ, int64_t *batch, int64_t *ptr, int32_t *ptr32,
+                            cm_stream_t stream);
+int cm_symmetric_sender_view(const int32_t *row_i, const int32_t *row_j, const double *unit_shifts, const int32_t *first_occ,
+                             int64_t nnodes, int64_t nedges, int32_t *sender_perm, cm_stream_t stream);
 
 /*
  * The test a molecular-dynamics driver makes before it reuses a list built out to cutoff + skin: out_sq[0] (fp64,

@@ -89,6 +89,51 @@ def test_degenerate_inputs(cabi):
         _device_list(planar, None, (0, 0, 0), -1.0)
 
 
+GRAPH_CASES = {
+    # atoms, box edge (None: no cell), periodic axes, cutoff
+    "one_atom": (1, None, (0, 0, 0), 5.0),
+    "no_pairs": (5, None, (0, 0, 0), 0.01),
+    "one_atom_images": (1, 3.0, (1, 1, 1), 5.0),
+    "few_atoms_many_images": (7, 3.7, (1, 1, 1), 6.0),
+    "wave_edges": (65, 9.0, (1, 0, 1), 5.0),
+    "box": (1000, 21.5, (1, 1, 1), 5.0),
+    "dense": (900, 9.0, (1, 1, 1), 5.5),          # more than 512 neighbours: one wave per workgroup
+    "denser": (400, 3.0, (0, 0, 0), 6.0),
+    "one_workgroup_most": (32768, 69.0, (1, 1, 1), 4.0),
+    "several_launches": (32769, 69.0, (1, 1, 0), 4.0),
+}
+
+
+@pytest.mark.parametrize("name", list(GRAPH_CASES))
+def test_graph_of_a_list(cabi, name):
+    """cm_neighbour_list_search / _graph: the pairs of cm_neighbour_list_count / _fill (held against the oracle above; against
+    the oracle here too where it is quick), the same in int64 and fp64, shifts, CSR offsets, batch and ptr; and
+    cm_symmetric_sender_view against the stable sort by sender."""
+    from cuda_mace import _cabi as cabi_mod
+    from cuda_mace.utils.neighbour_list import shifts_from_unit_shifts
+
+    n, box, pbc, cutoff = GRAPH_CASES[name]
+    rng = np.random.default_rng(len(name))
+    pos = rng.uniform(-1.0, (box or 6.0) * 1.1, (n, 3))
+    cell = None if box is None else np.eye(3) * box + np.array([[0, 0, 0], [0.3, 0, 0], [0.1, -0.2, 0]])
+    p = torch.tensor(pos, dtype=torch.float64, device=DEV)
+    c = None if cell is None else torch.tensor(cell, dtype=torch.float64, device=DEV)
+    if name in ("one_atom_images", "few_atoms_many_images", "wave_edges"):
+        _check(pos, cell, pbc, cutoff)
+    ri, rj, S = cabi_mod.neighbour_list(p, c, pbc, cutoff)
+    g = cabi_mod.neighbour_graph(p, c, pbc, cutoff)
+    print(name, "pairs", ri.numel(), flush=True)
+    assert torch.equal(g["row_i"], ri) and torch.equal(g["row_j"], rj)
+    assert torch.equal(g["edge_index"], torch.stack([ri, rj]).long())
+    assert torch.equal(g["unit_shifts"], S.double())
+    assert torch.equal(g["shifts"], shifts_from_unit_shifts(S, c))
+    assert torch.equal(g["first_occ"], cabi_mod.first_occurences(ri, n))
+    assert g["batch"].tolist() == [0] * n and g["ptr"].tolist() == [0, n] and g["ptr32"].tolist() == [0, n]
+    perm, off = cabi_mod.stable_key_sort(rj, n)
+    assert torch.equal(g["offsets"], off)
+    assert torch.equal(cabi_mod.symmetric_sender_view(g["row_i"], g["row_j"], g["unit_shifts"], g["first_occ"], n), perm)
+
+
 def test_full_size_box_equals_host_list_and_feeds_the_model(cabi):
     """25 000 atoms: the device list equals the host list of the benchmark generator entry for entry, and the model gives
     bit-identical energy and forces from either."""
