@@ -179,6 +179,7 @@ __global__ __launch_bounds__(kNodes *kHidden) void readout_forward_kernel(
         if (static_cast<unsigned>(row) < static_cast<unsigned>(nnodes)) node_total[row] = en + (node_e0 ? node_e0[node0 + r] : 0.0);
       }
     }
+    if (!d2) continue;  // energies alone: no derivative (a launch argument, the same for every thread)
     __syncthreads();
     // d e / d h2: a thread keeps the 16 weights of its channel in registers and serves a share of the tile's rows
     // (256 / C row groups; the rows' 16 factors are read by all lanes of a group at once)
@@ -222,7 +223,7 @@ int readout_forward_with_totals(const float *h1, const float *h2, const double *
   CM_REQUIRE(hidden >= 1 && hidden <= kHidden, "cm_readout_forward: hidden=%d must be in [1, %d]", hidden, kHidden);
   CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 2, "cm_readout_forward: nnodes out of range");
   if (nnodes == 0) return CM_OK;
-  CM_REQUIRE(h1 && h2 && w1 && W2a && w2b && node_energies && d_h2, "cm_readout_forward: NULL pointer");
+  CM_REQUIRE(h1 && h2 && w1 && W2a && w2b && node_energies, "cm_readout_forward: NULL pointer");
   // at most kMaxGroups workgroups (two per compute unit of a 256-unit device fit by their LDS): each stages the
   // weights once and walks several tiles
   const int64_t tiles = ceil_div(nnodes, kNodes);
@@ -238,6 +239,7 @@ extern "C" int cm_readout_forward(const float *h1, const float *h2, const double
                                   double act_cst, double scale, double shift, int64_t nnodes, int channels, int hidden,
                                   double *node_energies, float *d_h2, double *node_feats64, const int32_t *feats_rows,
                                   cm_stream_t stream) {
+  CM_REQUIRE(nnodes <= 0 || d_h2, "cm_readout_forward: NULL pointer");
   return cm::readout_forward_with_totals(h1, h2, w1, W2a, w2b, act_cst, scale, shift, nnodes, channels, hidden, node_energies, d_h2,
                                          node_feats64, feats_rows, nullptr, nullptr, cm::as_stream(stream));
 }

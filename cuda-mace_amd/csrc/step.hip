@@ -307,6 +307,16 @@ __global__ __launch_bounds__(kSumThreads) void graph_virial_kernel(const double 
   }
 }
 
+// stress = -virial / volume per graph, the volume as the triple product of the cell vectors
+__global__ void stress_kernel(const double *__restrict__ virials, const double *__restrict__ cell, int64_t ngraphs,
+                              double *__restrict__ stress) {
+  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (i >= 9 * ngraphs) return;
+  const double *c = cell + i / 9 * 9;
+  const double volume = fabs(c[0] * (c[4] * c[8] - c[5] * c[7]) + c[1] * (c[5] * c[6] - c[3] * c[8]) + c[2] * (c[3] * c[7] - c[4] * c[6]));
+  stress[i] = -virials[i] / volume;
+}
+
 // A fixed amount of dependent-free fp32 multiply-adds per lane, nothing else: what a box's vector ALUs deliver, for
 // telling boxes apart when the step's VALU-bound kernels differ between runs.
 __global__ __launch_bounds__(256) void probe_fma_kernel(float *out, int iters) {
@@ -363,6 +373,15 @@ extern "C" int cm_probe_fma(float *out, int workgroups, int iters, cm_stream_t s
   return cm::check_launch("cm_probe_fma");
 }
 
+extern "C" int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double *stress, cm_stream_t stream) {
+  CM_REQUIRE(ngraphs >= 0 && ngraphs < INT32_MAX / 16, "cm_stress: number of graphs out of range");
+  if (ngraphs == 0) return CM_OK;
+  CM_REQUIRE(virials && cell && stress, "cm_stress: NULL pointer");
+  hipLaunchKernelGGL(cm::stress_kernel, dim3(static_cast<unsigned>(cm::ceil_div(9 * ngraphs, 256))), dim3(256), 0, cm::as_stream(stream),
+                     virials, cell, ngraphs, stress);
+  return cm::check_launch("cm_stress");
+}
+
 extern "C" size_t cm_mace_step_workspace(int64_t nnodes, int64_t nedges, int channels) {
   if (nnodes < 0 || nedges < 0 || channels <= 0) return 0;
   return cm::Layout(nullptr, nnodes, nedges, channels).bytes;
@@ -405,10 +424,13 @@ extern "C" int cm_mace_step_timing_read(double *total_ms, int64_t *launches, int
   return cm::kStages;
 }
 
-extern "C" int cm_mace_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *positions, const double *shifts,
-                            void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy,
-                            double *forces, double *node_feats, double *virials, double *total_energy, double *total_node_energy,
-                            cm_stream_t stream) {
+namespace {
+
+// The step of cm_mace_step, or, with want_forces false, its forward half alone: no backward chain, and none of what only
+// that chain reads (the contractions' gradient tables, the readouts' derivative) is formed or written.
+int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *positions, const double *shifts, void *workspace,
+             size_t workspace_bytes, double *interaction_energy, double *node_energy, bool want_forces, double *forces,
+             double *node_feats, double *virials, double *total_energy, double *total_node_energy, cm_stream_t stream) {
   CM_REQUIRE(w && g, "cm_mace_step: NULL weights or graph");
   const int64_t N = g->nnodes, E = g->nedges;
   const int C = w->channels, ne = w->nelements;
@@ -435,7 +457,7 @@ extern "C" int cm_mace_step(const cm_mace_weights *w, const cm_mace_graph *g, co
       hipLaunchKernelGGL(cm::copy_or_zero_f64_kernel, dim3(1), dim3(64), 0, st, total_energy, g->graph_e0, static_cast<int64_t>(g->ngraphs));
     return cm::check_launch("cm_mace_step");
   }
-  CM_REQUIRE(positions && node_energy && forces, "cm_mace_step: NULL positions or output");
+  CM_REQUIRE(positions && node_energy && (forces || !want_forces), "cm_mace_step: NULL positions or output");
   CM_REQUIRE(N < INT32_MAX / 4 && E < INT32_MAX, "cm_mace_step: sizes out of range");
   CM_REQUIRE(E == 0 || shifts, "cm_mace_step: NULL shifts");
   CM_REQUIRE(g->first_occ && g->sender_offsets && g->elem_perm && g->elem_offsets && g->onehot_perm && g->onehot_offsets && g->X1,
@@ -485,8 +507,9 @@ extern "C" int cm_mace_step(const cm_mace_weights *w, const cm_mace_graph *g, co
     else
       CM_STAGE(8, cm_linear(bufM[t], w->mix_WT[t], nullptr, nullptr, N, 1, 0, 16, C, C, w->mix_scale[t], none, none, L.bufA, stream));
     // the contraction's gradient table takes the place of the message, which is no longer needed
+    float *table = want_forces ? bufM[t] : nullptr;
     CM_STAGE(t == 0 ? 3 : 9, cm_symcon_forward(L.bufA, el_perm, el_off, w->mono3[t], w->n3[t], w->mono2[t], w->n2[t], w->T3[t], w->T2[t], w->T1[t], N,
-                              ne, C, B[t], bufM[t], stream));
+                              ne, C, B[t], table, stream));
     if (t == 0 && glue)
       CM_STAGE(4, cm_node_glue_forward(L.B1, w->prod_WT[0], w->skip_WT, w->up_WT, oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.h1, L.sc,
                                        L.X2, stream));
@@ -494,12 +517,14 @@ extern "C" int cm_mace_step(const cm_mace_weights *w, const cm_mace_graph *g, co
       CM_STAGE(t == 0 ? 4 : 10, cm_linear(B[t], w->prod_WT[t], nullptr, nullptr, N, 1, 0, 1, C, C, 1.0f, none, t == 1 ? L.sc : none, h[t], stream));
   }
   CM_STAGE(11, cm::readout_forward_with_totals(L.h1, L.h2, w->w1, w->W2a, w->w2b, w->act_cst, w->scale, w->shift, N, C, w->hidden,
-                                               node_energy, L.d_h2, node_feats, g->node_rows, g->node_e0, total_node_energy, st));
-  if (!glue) {  // with the chained kernels the sums ride in the backward chain's launch
+                                               node_energy, want_forces ? L.d_h2 : nullptr, node_feats, g->node_rows, g->node_e0, total_node_energy, st));
+  if (!glue || !want_forces) {  // with the chained kernels the sums ride in the backward chain's launch
     cm::StageTimer timer_(st, 12, timing_mask);
     hipLaunchKernelGGL(cm::segment_sum_f64_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights,
                        g->graph_ptr, interaction_energy, g->graph_e0, total_energy);
   }
+
+  if (!want_forces) return cm::check_launch("cm_mace_energy");
 
   // ---- backward: d(-sum of node energies) / d positions ----
   // The seed is -1 on every node energy (-weight[n] with node weights), so the readouts' backward needs no pass of its
@@ -544,4 +569,22 @@ extern "C" int cm_mace_step(const cm_mace_weights *w, const cm_mace_graph *g, co
     hipLaunchKernelGGL(cm::graph_virial_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, L.node_virial, g->graph_ptr, virials);
   }
   return cm::check_launch("cm_mace_step");
+}
+
+}  // namespace
+
+extern "C" int cm_mace_step(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
+                            void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy,
+                            double *forces, double *node_feats, double *virials, double *total_energy, double *total_node_energy,
+                            cm_stream_t stream) {
+  return run_step(weights, graph, positions, shifts, workspace, workspace_bytes, interaction_energy, node_energy, true, forces,
+                  node_feats, virials, total_energy, total_node_energy, stream);
+}
+
+extern "C" int cm_mace_energy(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions,
+                              const double *shifts, void *workspace, size_t workspace_bytes, double *interaction_energy,
+                              double *node_energy, double *node_feats, double *total_energy, double *total_node_energy,
+                              cm_stream_t stream) {
+  return run_step(weights, graph, positions, shifts, workspace, workspace_bytes, interaction_energy, node_energy, false, nullptr,
+                  node_feats, nullptr, total_energy, total_node_energy, stream);
 }

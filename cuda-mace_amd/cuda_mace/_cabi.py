@@ -82,6 +82,8 @@ SIGNATURES = {
     "cm_probe_fma": (_i32, [_p, _i32, _i32, _p]),
     "cm_mace_step_timing_read": (_i32, [_p, _p, _i32]),
     "cm_mace_step_workspace": (_sz, [_i64, _i64, _i32]),
+    "cm_stress": (_i32, [_p, _p, _i64, _p, _p]),
+    "cm_mace_energy": (_i32, [_p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p]),
     "cm_mace_step": (_i32, [_p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p, _p, _p]),
     # fp64 instantiations: same argument lists, floating-point buffers in double
     "cm_mp_forward_f64": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i32, _p, _p]),
@@ -592,8 +594,6 @@ def symcon_backward(grad, grad_out) -> torch.Tensor:
 
 
 # ---- neighbour list -------------------------------------------------------------------------------
-def neighbour_list(positions, cell, pbc, cutoff: float, max_cells: int = 0):
-    """(row_i int32 [E], row_j int32 [E], unit_shifts int32 [E, 3]) sorted by (i, j, S); positions fp64 [N, 3] and
 def _list_status(E: int, status: int) -> None:
     if status == 1:
         raise CudaMaceError("neighbour list: a periodic axis needs a non-singular cell")
@@ -603,6 +603,8 @@ def _list_status(E: int, status: int) -> None:
         raise CudaMaceError("neighbour list: more pairs than int32 indexing holds")
 
 
+def neighbour_list(positions, cell, pbc, cutoff: float, max_cells: int = 0):
+    """(row_i int32 [E], row_j int32 [E], unit_shifts int32 [E, 3]) sorted by (i, j, S); positions fp64 [N, 3] and
     cell fp64 [3, 3] (or None) on the device, pbc three booleans.  One host synchronisation (the number of pairs)."""
     N = positions.shape[0]
     dev = positions.device
@@ -633,8 +635,6 @@ def _list_status(E: int, status: int) -> None:
     return row_i, row_j, S
 
 
-def max_displacement(positions, reference, out=None):
-    """fp64 [1] on the device: the largest squared distance between the rows of `positions` and `reference` (fp64
 _GRAPH_MAX_DEGREE = lib.cm_neighbour_list_graph_max_degree()
 
 
@@ -685,6 +685,8 @@ def symmetric_sender_view(row_i, row_j, unit_shifts, first_occ, nnodes: int):
     return perm
 
 
+def max_displacement(positions, reference, out=None):
+    """fp64 [1] on the device: the largest squared distance between the rows of `positions` and `reference` (fp64
     [N, 3]); nothing is read back here."""
     N = positions.shape[0]
     if reference.shape != positions.shape:
@@ -693,6 +695,15 @@ def symmetric_sender_view(row_i, row_j, unit_shifts, first_occ, nnodes: int):
         out = torch.empty(1, dtype=F64, device=positions.device)
     _check(lib.cm_max_displacement(_dev(positions, F64, "positions"), _dev(reference, F64, "reference"), N,
                                    _dev(out, F64, "out"), _stream()))
+    return out
+
+
+def stress_of(virials, cell):
+    """-virials / |det cell| per graph; both fp64 [ngraphs, 3, 3]."""
+    if virials.shape != cell.shape:
+        raise CudaMaceError("stress: virials and cell differ in shape")
+    out = torch.empty_like(virials)
+    _check(lib.cm_stress(_dev(virials, F64, "virials"), _dev(cell, F64, "cell"), virials.shape[0], _dev(out, F64, "stress"), _stream()))
     return out
 
 

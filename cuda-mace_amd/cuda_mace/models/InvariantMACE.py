@@ -147,14 +147,15 @@ def get_outputs(energy, positions, displacement, cell, training=False, compute_f
     return forces, virials, stress, None, None
 
 
-def _select_head(per_head: torch.Tensor, node_heads: torch.Tensor) -> torch.Tensor:
-    """per_head[n, node_heads[n]] (the reference's `[arange, node_heads]` indexing, models/InvariantMACE.py:287-289, 336),
+def _select_head(per_head: torch.Tensor, heads_of_nodes) -> torch.Tensor:
+    """per_head[n, heads_of_nodes()[n]] (the reference's `[arange, node_heads]` indexing, models/InvariantMACE.py:287-289,
+    336; the heads are asked for only where there is a choice),
     written as a gather so that its backward is a plain scatter instead of a sort-based index_put."""
     if per_head.dim() == 1:
         return per_head
     if per_head.shape[1] == 1:
         return per_head[:, 0]
-    return torch.gather(per_head, 1, node_heads.view(-1, 1)).squeeze(1)
+    return torch.gather(per_head, 1, heads_of_nodes().view(-1, 1)).squeeze(1)
 
 
 def fused_readout_parameters(readouts, scale_shift):
@@ -443,11 +444,14 @@ class OptimizedInvariantMACE(torch.nn.Module):
             object.__setattr__(self, "_native", NativeStep(self) if NativeStep.supported(self) else False)
         return self._native or None
 
-    def _native_step_for(self, data, training: bool, compute_force: bool, compute_displacement: bool):
+    def _native_step_for(self, data, training: bool, compute_force: bool, compute_displacement: bool, strain: bool = False):
         """The library's one-call step, if this evaluation can run on it: inference with forces (virials and stress come
-        from the same per-edge gradients), one head, positions on the GPU, no strain tensor asked for."""
-        if not (self.native_step and not training and compute_force and not compute_displacement and "head" not in data
-                and data["positions"].is_cuda):
+        from the same per-edge gradients), one head, positions on the GPU, no strain tensor asked for.  Energies alone run
+        on its forward half where the caller cannot differentiate them (gradients switched off) and asks for no virials
+        (`strain`)."""
+        if not (self.native_step and not training and not compute_displacement and "head" not in data and data["positions"].is_cuda):
+            return None
+        if not compute_force and (strain or torch.is_grad_enabled()):
             return None
         return self._native_step_of()
 
@@ -479,9 +483,9 @@ class OptimizedInvariantMACE(torch.nn.Module):
         back to its last pair inside the cutoff, and with this order the pairs that drift inside between two list builds
         are the first of the shell, so the cut stays close to the pairs that count.  One library call on the device
         (cm_graph_prepare), no host synchronisation; it also delivers the CSR offsets and the sender-sorted view of the new
-        list, which are left where the ops look for them.  Returns (perm new -> old [N], inverse [N], edge_perm new -> old
-        [E], relabelled edge_index [2, E], relabelled batch [N]).  Any permutation is valid; this one is cheap and keeps
-        neighbours within a few hundred indices of each other."""
+        list, which are left where the ops look for them.  Returns int32 (perm new -> old [N], inverse [N], edge_perm
+        new -> old [E], relabelled edge_index [2, E]).  Any permutation is valid; this one is cheap and keeps neighbours
+        within a few hundred indices of each other."""
         pos = data["positions"].detach().double().contiguous()
         batch, edge_index = data["batch"], data["edge_index"]
         n, ngraphs = pos.shape[0], int(data["ptr"].numel()) - 1
@@ -494,9 +498,8 @@ class OptimizedInvariantMACE(torch.nn.Module):
             bins -= 1
         g = cabi.graph_prepare(pos, row0, row1, shifts, None if ngraphs == 1 else batch.int().contiguous(), ngraphs,
                                float(self.r_max), bins)
-        perm, inverse, edge_perm = g["node_perm"].long(), g["node_inverse"].long(), g["edge_perm"].long()
         receiver, sender = g["receiver"], g["sender"]
-        new_edges = torch.stack((receiver, sender)).long()
+        new_edges = torch.stack((receiver, sender))
         # what the ops derive from a list is already there: leave it where they look it up
         new_edges.__dict__["_cm_int32_rows"] = ((new_edges._version, new_edges.data_ptr(), None), (receiver, sender))
         receiver.__dict__["_cm_csr"] = ((receiver._version, receiver.data_ptr(), n), g["first_occ"])
@@ -504,7 +507,34 @@ class OptimizedInvariantMACE(torch.nn.Module):
         if data["shifts"].dtype == torch.float64:
             t = data["shifts"]
             edge_index.__dict__["_cm_spatial_shifts"] = (t, (edge_index._version, edge_index.data_ptr(), t._version), g["shifts"])
-        return perm, inverse, edge_perm, new_edges, batch.index_select(0, perm)
+        return g["node_perm"], g["node_inverse"], g["edge_perm"], new_edges
+
+    def _species_of(self, node_attrs: torch.Tensor):
+        """What depends on the species alone, evaluated once per node_attrs tensor and kept while that tensor is unchanged:
+        the atomic reference energies per head, the first layer's linear_up of the node embedding (weights are frozen), the
+        fp32 one-hot matrix and the element index of every node."""
+
+        def species_only():
+            with torch.no_grad():
+                attrs64 = node_attrs.double()
+                return (self.atomic_energies_fn(attrs64),
+                        self.interactions[0].linear_up(self.node_embedding(attrs64).float()))
+
+        e0_per_head, node_feats_up = _cached_for(node_attrs, "_cm_species_only", self._weights_token, species_only)
+        node_attrs32, atom_types = _cached(node_attrs, "_cm_species", None,
+                                           lambda: (node_attrs.detach().float(), node_attrs.detach().argmax(dim=-1).int()))
+        return e0_per_head, node_feats_up, node_attrs32, atom_types
+
+    def _species_in_order(self, node_attrs: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
+        """Rows `perm` of node_attrs, carrying the rows of what `_species_of` knows about it (an MD code keeps its species
+        through many lists: gathered, not evaluated again)."""
+        known = self._species_of(node_attrs)
+        out = node_attrs.detach().index_select(0, perm)
+        e0_per_head, node_feats_up, node_attrs32, atom_types = (t.index_select(0, perm) for t in known)
+        tag = (out._version, out.data_ptr())
+        out.__dict__["_cm_species_only"] = (self._weights_token, tag + (0,), (e0_per_head, node_feats_up))
+        out.__dict__["_cm_species"] = (tag + (None,), (node_attrs32, atom_types))
+        return out
 
     def forward(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,
                 compute_virials: bool = False, compute_stress: bool = False,
@@ -519,38 +549,41 @@ class OptimizedInvariantMACE(torch.nn.Module):
         # Same step on the relabelled graph.  Everything that depends only on the neighbour list or the species is
         # derived once per tensor object; per call the positions are gathered into the new order and forces, node
         # energies and node features gathered back (fixed-order gathers: results stay reproducible bit for bit).
-        perm, inverse, edge_perm, edge_index, batch = _cached(data["edge_index"], "_cm_spatial_order", None,
-                                                              lambda: self._spatial_order(data))
+        perm, inverse, edge_perm, edge_index = _cached(data["edge_index"], "_cm_spatial_order", None,
+                                                       lambda: self._spatial_order(data))
         inner = dict(data)
         # Without strain the positions stay in the caller's order: the geometry kernels read them (and write the forces)
         # through the row map.  The strain path transforms positions per graph and works on a gathered copy; the
         # one-call step needs no strain for virials and stress.
-        direct = (not (compute_virials or compute_stress or compute_displacement)
-                  or self._native_step_for(data, training, compute_force, compute_displacement) is not None)
+        strained = compute_virials or compute_stress or compute_displacement
+        direct = (not strained
+                  or self._native_step_for(data, training, compute_force, compute_displacement, compute_virials or compute_stress) is not None)
         # With compute_force=False the caller differentiates the returned energies itself (a wrapper that sums the
         # energies of some atoms only): the positions then stay attached to the caller's tensor.
         own = data["positions"].detach() if compute_force else data["positions"]
         inner["positions"] = own if direct else own.index_select(0, perm)
-        inner["edge_index"], inner["batch"] = edge_index, batch
+        inner["edge_index"] = edge_index
+        if data["ptr"].numel() > 2:
+            inner["batch"] = _cached_for(data["edge_index"], "_cm_spatial_batch", data["batch"],
+                                         lambda: data["batch"].index_select(0, perm))
         inner["node_attrs"] = _cached_for(data["edge_index"], "_cm_spatial_attrs", data["node_attrs"],
-                                          lambda: data["node_attrs"].index_select(0, perm))
+                                          lambda: self._species_in_order(data["node_attrs"], perm))
         for name in ("shifts", "unit_shifts"):
-            if name in data:
+            if name in data and (name == "shifts" or not direct):  # the integer images serve the strain path alone
                 t = data[name]
                 inner[name] = _cached_for(data["edge_index"], "_cm_spatial_" + name, t, lambda t=t: t.index_select(0, edge_perm))
         if data.get("node_weights") is not None:
             t = data["node_weights"]
             inner["node_weights"] = _cached_for(data["edge_index"], "_cm_spatial_node_weights", t, lambda: t.index_select(0, perm))
-        rows = _cached(data["edge_index"], "_cm_spatial_rows32", None, lambda: (perm.int(), inverse))
         # per-node outputs come back in the caller's order (node_rows)
         return self._forward_ordered(inner, training, compute_force, compute_virials, compute_stress, compute_displacement,
-                                     node_rows=rows, positions_in_caller_order=direct, compute_node_feats=compute_node_feats)
+                                     node_rows=(perm, inverse), positions_in_caller_order=direct, compute_node_feats=compute_node_feats)
 
     def _forward_ordered(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,
                          compute_virials: bool = False, compute_stress: bool = False, compute_displacement: bool = False,
                          node_rows=None, positions_in_caller_order: bool = False,
                          compute_node_feats: bool = True) -> Dict[str, Optional[torch.Tensor]]:
-        """node_rows = (rows int32 [N], inverse int64 [N]): node n of `data` is node rows[n] of the caller, and the
+        """node_rows = (rows int32 [N], inverse int32 [N]): node n of `data` is node rows[n] of the caller, and the
         per-node outputs (forces, node_energy, node_feats) are returned in the caller's order.
         positions_in_caller_order: data["positions"] (and hence the forces) are rows of the caller, read through rows."""
         data["positions"].requires_grad_(True)
@@ -558,31 +591,23 @@ class OptimizedInvariantMACE(torch.nn.Module):
         node_attrs = data["node_attrs"]
         batch = data["batch"]
         node_heads = data["head"][batch] if "head" in data else None  # None: every node reads head 0
-        zero_heads = None if node_heads is not None else _cached(batch, "_cm_zero_heads", None, lambda: torch.zeros_like(batch))
+        heads_of_nodes = lambda: (node_heads if node_heads is not None  # noqa: E731
+                                  else _cached(batch, "_cm_zero_heads", None, lambda: torch.zeros_like(batch)))
         num_graphs = data["ptr"].numel() - 1
         shifts = data["shifts"]
         cell = data.get("cell")
 
         native = None
         if node_rows is None or positions_in_caller_order:
-            native = self._native_step_for(data, training, compute_force, compute_displacement)
+            native = self._native_step_for(data, training, compute_force, compute_displacement, compute_virials or compute_stress)
         displacement = _constant(0.0, (num_graphs, 3, 3), positions.dtype, positions.device)  # replaced below when strained
         if native is None and (compute_virials or compute_stress or compute_displacement):
             positions, shifts, displacement, cell = get_symmetric_displacement(
                 positions=positions, unit_shifts=data["unit_shifts"], cell=cell, edge_index=data["edge_index"],
                 num_graphs=num_graphs, batch=batch)
 
-        # What depends on the species alone -- the atomic reference energies, the node embedding and the first layer's
-        # linear_up of it (weights are frozen) -- is evaluated once per node_attrs tensor and reused while that tensor
-        # is unchanged, like the index structures below.
-        def species_only():
-            with torch.no_grad():
-                attrs64 = node_attrs.double()
-                return (self.atomic_energies_fn(attrs64),
-                        self.interactions[0].linear_up(self.node_embedding(attrs64).float()))
-
-        e0_per_head, node_feats_up = _cached_for(node_attrs, "_cm_species_only", self._weights_token, species_only)
-        node_e0 = _select_head(e0_per_head, zero_heads if node_heads is None else node_heads)
+        e0_per_head, node_feats_up, node_attrs32, atom_types = self._species_of(node_attrs)
+        node_e0 = _select_head(e0_per_head, heads_of_nodes)
         # data["node_weights"] [N] (optional): every node energy enters the graph's energy, and hence the quantity the
         # forces, virials and stress derive from, with this weight (1 for a rank's own atoms, 0 for ghost copies in a
         # domain-decomposed MD code); node_energy itself stays unweighted.
@@ -603,13 +628,10 @@ class OptimizedInvariantMACE(torch.nn.Module):
         node_feats = None
 
         # index structures shared by both layers, cached on the caller's tensors so that they are rebuilt only when
-        # the neighbour list / the species change: int32 edge lists (their CSR offsets and sender-sorted view are in
-        # turn cached on these), the fp32 one-hot matrix and the element index per node
+        # the neighbour list changes: int32 edge lists (their CSR offsets and sender-sorted view are in turn cached on these)
         edge_index = data["edge_index"]
         receiver, sender = _cached(edge_index, "_cm_int32_rows", None,
                                    lambda: (edge_index[0].int().contiguous(), edge_index[1].int().contiguous()))
-        node_attrs32, atom_types = _cached(node_attrs, "_cm_species", None,
-                                           lambda: (node_attrs.detach().float(), node_attrs.detach().argmax(dim=-1).int()))
 
         if native is not None:
             rows32 = None if node_rows is None else node_rows[0]
@@ -623,19 +645,18 @@ class OptimizedInvariantMACE(torch.nn.Module):
                 handle = _cached_per(data["node_weights"], "_cm_native_graphs_weighted", self._weights_token, plain,
                                      lambda: plain.with_node_weights(node_weights, graph_e0()))
             want_virials = compute_virials or compute_stress
-            res = native(handle, positions, shifts, want_feats=compute_node_feats, want_virials=want_virials)
+            res = native(handle, positions, shifts, want_feats=compute_node_feats, want_virials=want_virials, want_forces=compute_force)
             inter_e = res["interaction_energy"]
             virials = res["virials"].to(positions.dtype) if want_virials else None
             stress = None
             if compute_stress and cell is not None:
-                c3 = cell.view(-1, 3, 3).to(virials.dtype)  # the volume as a triple product: a few element-wise launches
-                volume = (c3[:, 0] * torch.linalg.cross(c3[:, 1], c3[:, 2], dim=-1)).sum(dim=-1).abs()
-                stress = -virials / volume.view(-1, 1, 1)
+                c3 = cell.detach().double().reshape(-1, 3, 3).expand_as(res["virials"]).contiguous()
+                stress = cabi.stress_of(res["virials"], c3).to(virials.dtype)
             # energy = e0 + interaction energy and node_energy = node_e0 + its interaction part (already in the caller's
             # order) are written by the step's own kernels: the atomic reference energies ride in the handle
             return {
                 "energy": res["energy"], "node_energy": res["node_energy"], "interaction_energy": inter_e,
-                "forces": res["forces"].to(data["positions"].dtype), "virials": virials, "stress": stress, "hessian": None,
+                "forces": res["forces"].to(data["positions"].dtype) if compute_force else None, "virials": virials, "stress": stress, "hessian": None,
                 "displacement": displacement, "node_feats": res["node_feats"], "edge_forces": None,
             }
 
@@ -670,8 +691,7 @@ class OptimizedInvariantMACE(torch.nn.Module):
                 node_feats = product(node_feats=node_feats, sc=sc, node_attrs=atom_types)  # fp32 [N, C]
             node_feats_list.append(node_feats)
             if not fused_readout:
-                heads = zero_heads if node_heads is None else node_heads
-                node_es_list.append(_select_head(readout(node_feats.double(), heads), heads))
+                node_es_list.append(_select_head(readout(node_feats.double(), heads_of_nodes()), heads_of_nodes))
 
         if fused_readout:
             act_cst, scale, shift = self.readout_constants
@@ -683,7 +703,7 @@ class OptimizedInvariantMACE(torch.nn.Module):
             if node_rows is not None:
                 node_feats_out = node_feats_out.index_select(0, node_rows[1])
             node_inter_es = torch.sum(torch.stack(node_es_list, dim=0), dim=0)
-            node_inter_es = self.scale_shift(node_inter_es, zero_heads if node_heads is None else node_heads)
+            node_inter_es = self.scale_shift(node_inter_es, heads_of_nodes())
         weighted_es = node_inter_es.double() if node_weights is None else node_inter_es.double() * node_weights
         inter_e = scatter_sum(src=weighted_es, index=batch, dim=-1, dim_size=num_graphs, ptr=data["ptr"])
 

@@ -136,7 +136,8 @@ class NativeStep:
                                 graph_e0))
 
     def __call__(self, handle: "_GraphHandle", positions: torch.Tensor, shifts: torch.Tensor, want_feats: bool = True,
-                 want_virials: bool = False) -> Dict[str, torch.Tensor]:
+                 want_virials: bool = False, want_forces: bool = True) -> Dict[str, torch.Tensor]:
+        """want_forces=False: the forward half alone (cm_mace_energy), "forces" and "virials" are None."""
         g = handle.struct
         N, E, C = int(g.nnodes), int(g.nedges), self.channels
         dev = positions.device
@@ -157,17 +158,19 @@ class NativeStep:
                 ws = self._workspace = torch.empty(need, dtype=torch.uint8, device=dev)
         energy = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_energy = torch.empty(N, dtype=F64, device=dev)
-        forces = torch.empty(N, 3, dtype=F64, device=dev)
+        forces = torch.empty(N, 3, dtype=F64, device=dev) if want_forces else None
         feats = torch.empty(N, 2 * C, dtype=F64, device=dev) if want_feats else None
         virials = torch.empty(int(g.ngraphs), 3, 3, dtype=F64, device=dev) if want_virials else None
         total = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_total = torch.empty(N, dtype=F64, device=dev)
-        cabi._check(cabi.lib.cm_mace_step(
-            ctypes.addressof(self.weights), ctypes.addressof(g), _ptr(pos64, F64, "positions"), _ptr(sh64, F64, "shifts"),
-            ws.data_ptr(), ws.numel(), _ptr(energy, F64, "energy"), _ptr(node_energy, F64, "node_energy"),
-            _ptr(forces, F64, "forces"), _ptr(feats, F64, "node_feats") if want_feats else None,
-            _ptr(virials, F64, "virials") if want_virials else None, _ptr(total, F64, "total_energy"),
-            _ptr(node_total, F64, "total_node_energy"), cabi._stream()))
+        head = (ctypes.addressof(self.weights), ctypes.addressof(g), _ptr(pos64, F64, "positions"), _ptr(sh64, F64, "shifts"),
+                ws.data_ptr(), ws.numel(), _ptr(energy, F64, "energy"), _ptr(node_energy, F64, "node_energy"))
+        tail = (_ptr(total, F64, "total_energy"), _ptr(node_total, F64, "total_node_energy"), cabi._stream())
+        if want_forces:
+            cabi._check(cabi.lib.cm_mace_step(*head, _ptr(forces, F64, "forces"), _ptr(feats, F64, "node_feats"),
+                                              _ptr(virials, F64, "virials"), *tail))
+        else:
+            cabi._check(cabi.lib.cm_mace_energy(*head, _ptr(feats, F64, "node_feats"), *tail))
         # energy / node_energy: the interaction part plus the handle's graph_e0 / node_e0, node_energy in the caller's
         # order (rows node_rows of the handle); interaction_node_energy: the interaction part alone, in list order
         return {"interaction_energy": energy, "interaction_node_energy": node_energy, "energy": total, "node_energy": node_total,

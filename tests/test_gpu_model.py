@@ -412,6 +412,30 @@ def test_native_step_equals_autograd_path(cabi, case):
     assert float((a["forces"].cpu() - ref["forces"]).abs().max()) <= F_ATOL
 
 
+@pytest.mark.parametrize("atoms,C,relabel", [(1, 32, False), (60, 64, False), (300, 128, True), (300, 160, True), (2500, 192, False)])
+def test_energy_alone(cabi, atoms, C, relabel):
+    """compute_force=False with gradients switched off runs the forward half of the step (cm_mace_energy): node energies and
+    features of the full step bit for bit, energies up to the order of the final sum, no forces.  With gradients on, the
+    energies stay differentiable."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    data = to_device(make_system(atoms, 4, seed=3, density=None if atoms < 100 else 0.1, cluster_box=12.0 if atoms < 100 else None), "cuda")
+    up = SyntheticInvariantMACE(channels=C, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=30.0, seed=2, shift=0.1)
+    model = OptimizedInvariantMACE(up, device="cuda", spatial_order_min_atoms=0 if relabel else None)
+    full = model(dict(data))
+    with torch.no_grad():
+        only = model(dict(data), compute_force=False)
+        bare = model(dict(data), compute_force=False, compute_node_feats=False)
+    assert only["forces"] is None and only["virials"] is None and only["stress"] is None
+    for key in ("node_energy", "node_feats"):
+        assert torch.equal(only[key], full[key])
+    for key in ("energy", "interaction_energy"):
+        torch.testing.assert_close(only[key], full[key], rtol=1e-12, atol=1e-12)
+        assert torch.equal(bare[key], only[key])
+    assert bare["node_feats"] is None and torch.equal(bare["node_energy"], only["node_energy"])
+    assert model(dict(data), compute_force=False)["energy"].requires_grad
+
+
 @pytest.mark.parametrize("relabel", [True, False], ids=["shell_last", "shell_in_place"])
 def test_native_step_on_a_list_with_a_skin(cabi, relabel):
     """A neighbour list built out to cutoff + skin, at a size where the forward runs the LDS-table kernel: the step walks
