@@ -36,6 +36,7 @@ class MACECalculator:
         self._key = None          # (atomic numbers, cell, pbc, stress wanted) the device calculator was built for
         self._last = None         # positions of the last evaluation
         self._device_calc: Optional[DeviceCalculator] = None
+        self._staged = None       # pinned host buffers
 
     # -- structure -> device ---------------------------------------------------------------------------
     def _node_attrs(self, numbers: np.ndarray) -> torch.Tensor:
@@ -74,12 +75,24 @@ class MACECalculator:
             raise NotImplementedError("properties %s are not implemented (available: %s)" % (unknown, self.implemented_properties))
         want_stress = "stress" in properties
         calc = self._prepare(atoms, want_stress or (self._key is not None and self._key[3]))
-        positions = np.asarray(atoms.get_positions(), dtype=np.float64)
-        out = calc.compute(torch.from_numpy(positions).to(self.device))
-        energy = float(out["energy"].double().sum().cpu())
-        self.results = {"energy": energy, "free_energy": energy, "forces": out["forces"].double().cpu().numpy()}
+        positions = np.asarray(atoms.get_positions(), dtype=np.float64).reshape(-1, 3)
+        n = positions.shape[0]
+        if self._staged is None or self._staged[0].shape[0] != n:
+            # pinned host buffers, kept while the number of atoms stays: positions in; energy, forces and stress out
+            self._staged = (torch.empty(n, 3, dtype=torch.float64, pin_memory=True),
+                            torch.empty(3 * n + 10, dtype=torch.float64, pin_memory=True))
+        sent, received = self._staged
+        sent.numpy()[...] = positions
+        out = calc.compute(sent.to(self.device, non_blocking=True), host_positions=positions)
+        parts = [out["forces"].reshape(-1), out["energy"].reshape(-1)[:1]] + ([out["stress"].reshape(-1)] if calc.compute_stress else [])
+        packed = torch.cat([p.double() for p in parts])  # one copy and one wait instead of three
+        received[:packed.numel()].copy_(packed, non_blocking=True)
+        torch.cuda.current_stream(self.device).synchronize()
+        got = received.numpy()
+        energy = float(got[3 * n])
+        self.results = {"energy": energy, "free_energy": energy, "forces": got[:3 * n].reshape(n, 3).copy()}
         if calc.compute_stress:
-            s = out["stress"].double().reshape(3, 3).cpu().numpy()
+            s = got[3 * n + 1:3 * n + 10].reshape(3, 3)
             self.results["stress"] = np.array([s[0, 0], s[1, 1], s[2, 2], s[1, 2], s[0, 2], s[0, 1]])
         self.atoms = atoms
         self._last = (positions.copy(), self._key)

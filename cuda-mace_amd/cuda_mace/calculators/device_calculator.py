@@ -21,11 +21,12 @@ from __future__ import annotations
 import math
 from typing import Dict, Optional, Sequence
 
+import numpy as np
 import torch
 
 from cuda_mace import _cabi
 from cuda_mace.utils.graph import GraphedStep
-from cuda_mace.utils.neighbour_list import get_neighborhood
+from cuda_mace.utils.neighbour_list import neighbour_data
 
 
 class DeviceCalculator:
@@ -58,6 +59,7 @@ class DeviceCalculator:
         self.steps = 0
         self.dropped = 0  # steps enqueued on a list that turned out stale, and enqueued again
         self._ref_positions: Optional[torch.Tensor] = None
+        self._ref_host: Optional[np.ndarray] = None  # the same on the host, when the caller keeps its atoms there
         self._data: Optional[Dict[str, torch.Tensor]] = None
         self._graph: Optional[GraphedStep] = None
         self._moved_sq = torch.empty(1, dtype=torch.float64, device=node_attrs.device)
@@ -69,15 +71,8 @@ class DeviceCalculator:
     # -- Verlet list ---------------------------------------------------------------------------------------
     def _rebuild(self, positions: torch.Tensor) -> None:
         pos = positions.detach().double().contiguous()
-        edge_index, shifts, unit_shifts, cell = get_neighborhood(pos, self.cutoff + self.skin, self.pbc, self.cell)
-        n = pos.shape[0]
-        dev = pos.device
-        self._data = {
-            "positions": pos.clone(), "node_attrs": self.node_attrs, "edge_index": edge_index, "shifts": shifts,
-            "unit_shifts": unit_shifts, "cell": cell, "batch": torch.zeros(n, dtype=torch.int64, device=dev),
-            "ptr": torch.tensor([0, n], dtype=torch.int64, device=dev),
-        }
         self._ref_positions = pos.clone()
+        self._data = neighbour_data(self._ref_positions, self.node_attrs, self.cutoff + self.skin, self.pbc, self.cell)
         self._graph = None
         if self.use_graph:
             self._graph = GraphedStep(self.model, self._data, warmup=1, compute_virials=self.compute_stress,
@@ -94,25 +89,39 @@ class DeviceCalculator:
         out = self.model(data, compute_virials=self.compute_stress, compute_stress=self.compute_stress, **self._forward_kwargs)
         return {k: v.detach() for k, v in out.items() if isinstance(v, torch.Tensor)}
 
-    def compute(self, positions: torch.Tensor) -> Dict[str, torch.Tensor]:
-        """energy [1], forces [N, 3] (and virials / stress when asked for) at `positions` (fp64, on the GPU)."""
+    def compute(self, positions: torch.Tensor, host_positions: Optional[np.ndarray] = None) -> Dict[str, torch.Tensor]:
+        """energy [1], forces [N, 3] (and virials / stress when asked for) at `positions` (fp64, on the GPU).
+        host_positions (the same values, fp64 [N, 3] in host memory): what a caller whose atoms live on the host has
+        anyway; the displacement test is then made there and nothing waits for the GPU (up to 4 096 atoms, where it costs
+        less than the round trip)."""
         positions = positions.detach().double().contiguous()
         self.steps += 1
+        if host_positions is not None and host_positions.shape[0] > 4096:
+            host_positions = None
         if self._ref_positions is None or self._ref_positions.shape != positions.shape:
-            self._rebuild(positions)
+            return self._on_fresh_list(positions, host_positions)
+        limit = 0.5 * self.skin
+        if host_positions is not None and self._ref_host is not None:
+            d = host_positions - self._ref_host
+            moved = math.sqrt(float(np.einsum("ij,ij->i", d, d).max(initial=0.0)))
+            if not moved <= limit:
+                return self._on_fresh_list(positions, host_positions)
             return self._run(positions)
         _cabi.max_displacement(positions, self._ref_positions, out=self._moved_sq)
         self._moved_sq_host.copy_(self._moved_sq, non_blocking=True)
         self._arrived.record()
-        limit = 0.5 * self.skin
         ahead = self.run_ahead and self._moved + 2.0 * self._growth <= limit
         out = self._run(positions) if ahead else None
         self._arrived.synchronize()  # the scalar, not the step: the step's kernels come after it on the stream
         moved = math.sqrt(float(self._moved_sq_host[0]))
         if not moved <= limit:
             self.dropped += int(ahead)
-            self._rebuild(positions)
-            return self._run(positions)
+            return self._on_fresh_list(positions, host_positions)
         self._growth = max(moved - self._moved, 0.95 * self._growth if math.isfinite(self._growth) else 0.0)
         self._moved = moved
         return out if ahead else self._run(positions)
+
+    def _on_fresh_list(self, positions: torch.Tensor, host_positions: Optional[np.ndarray]) -> Dict[str, torch.Tensor]:
+        self._rebuild(positions)
+        self._ref_host = None if host_positions is None else host_positions.copy()
+        return self._run(positions)
