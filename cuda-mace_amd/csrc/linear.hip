@@ -971,6 +971,260 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
   }
 }
 
+// -----------------------------------------------------------------------------------------------
+// Variant with the weights resident in registers (16 components per node, 160 to 256 columns, K = Nout).
+//
+// Three planes of 160 x 160 weights and more do not fit LDS next to anything else, and the tiled kernels stage the block
+// again for every 128 rows in barrier-separated phases that one or two waves per SIMD cannot overlap: 192 columns ran at
+// 2.8-3.0 TB/s of their bytes, 256 at 2.2.  The register file of a compute unit holds 512 KB: here a workgroup takes a
+// contiguous piece of the list of all 16-row tiles (as the kernel above does), wave w keeps the pieces of its 16 CB weight
+// columns for all of K in its registers (6 CB K / 16 of them) until the weight block changes, and all waves multiply the
+// same tile of X rows, whose piece planes they share through LDS, double-buffered with one barrier per tile.  X goes
+// global -> LDS as raw fp32 by direct loads; a wave splits exactly the pieces it fetched itself, so only the planes are
+// shared.  The waves of a SIMD take turns in the order of their phases: every other one multiplies the current tile before
+// it splits the next.
+//
+// Operands as in the kernel above (weights as the row operand): a lane's accumulators are four consecutive output columns of
+// one row, stored as 16 bytes.  v_mfma_f32_16x16x32_bf16: K steps of 32, piece products in the order of the kernels above.
+//
+// Vector-memory operations of the tile loop are issued from assembly: the loads of tile k + 2 right after the split of tile
+// k + 1, then the stores of a tile; the wait before a split lets exactly those stores stay out.
+//
+// CB: 16 columns per wave give 10, 12 and 14 waves, three or four per SIMD (32 columns per wave: 5, 6 and 7 waves, two on
+// some SIMDs and one on others; 5-8 % slower at 160 and 192); at 256 columns 32 per wave (8 waves) are equal up to 20 000
+// nodes and 1 % faster with row_scale.  32-row tiles: 1-3 % slower.  Two or three tiles requested ahead instead of one: no
+// faster (656 -> 664 us at 100 000 x 192).
+//
+// Measured against the tiled kernels (plain / row_scale): 100 000 x 192 810 / 860 -> 655 / 675 us, 50 000 x 160 326 / 345 ->
+// 285 / 290, 20 000 x 224 255 / 272 -> 180 / 190, 40 000 x 256 595 / 643 -> 415 / 445, 12 000 x 256 183 / 198 -> 122 / 145,
+// equal at 2 048 nodes.  Without its matrix instructions 192 columns take 520 us (4.7 TB/s, the rate of a copy), without
+// loads, stores and split 514 us: what is left is their overlap.
+// -----------------------------------------------------------------------------------------------
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int kWideSegRows = 2048;  // rows whose node numbers a segment keeps in LDS
+
+template <int NT, int CB, bool SCALED>
+__global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void linear_wide_kernel(const float *__restrict__ X, const float *__restrict__ WT,
+                                                                   const int32_t *__restrict__ node_perm,
+                                                                   const int32_t *__restrict__ group_offsets, int nnodes, int ngroups,
+                                                                   int zero_last_group, float scale,
+                                                                   const float *__restrict__ row_scale, float *__restrict__ OUT) {
+  constexpr int K = 32 * NT;                  // = Nout
+  constexpr int TR = 16;                      // rows of a tile
+  constexpr int WAVES = 2 * NT / CB;          // a wave owns CB blocks of 16 output columns
+  constexpr int RB = TR / 16;                 // row blocks
+  constexpr int LD = K + 8;                   // row stride of a plane in elements: an odd number of 16-byte units
+  constexpr int KS = K / 32;
+  constexpr int PIECES = TR * K / 4 / (WAVES * kWave);  // 16-byte pieces of a tile per thread
+  constexpr int STORES = CB * RB;             // per wave and tile
+  constexpr int kSegTiles = kWideSegRows / TR;
+  __shared__ __attribute__((aligned(16))) __bf16 sP[2][3][TR * LD];
+  __shared__ __attribute__((aligned(16))) float sRaw[TR * K];
+  __shared__ __attribute__((aligned(16))) float sScale[SCALED ? TR * K : 4];
+  __shared__ int sId[kWideSegRows];
+  __shared__ int sOff[kResMaxGroups + 1];
+  __shared__ int sCum[kResMaxGroups + 1];
+
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r16 = lane % 16, quarter = lane / 16;
+  const bool late = (wave / 4 & 1) != 0;  // multiplies before it splits
+
+  const int ngw = zero_last_group ? ngroups - 1 : ngroups;
+  if (tid == 0) {
+    int cum = 0;
+    for (int g = 0; g < ngw; ++g) {
+      const int lo = group_offsets ? group_offsets[g] : 0, hi = group_offsets ? group_offsets[g + 1] : nnodes;
+      sOff[g] = lo;
+      sCum[g] = cum;
+      cum += 16 * ((max(hi - lo, 0) + TR - 1) / TR);
+    }
+    sOff[ngw] = group_offsets ? group_offsets[ngw] : nnodes;
+    sCum[ngw] = cum;
+  }
+  if (zero_last_group) {
+    // rows that belong to no weight group: the product is defined as zero
+    const int z0 = group_offsets[ngroups - 1], nz = group_offsets[ngroups] - z0;
+    constexpr int rowq = 16 * K / 4;
+    const int64_t total = static_cast<int64_t>(nz) * rowq;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + tid; i < total; i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+      const int node = node_perm[z0 + static_cast<int>(i / rowq)];
+      if (static_cast<unsigned>(node) < static_cast<unsigned>(nnodes)) st4(OUT + static_cast<int64_t>(node) * 16 * K + 4 * (i % rowq), zero4());
+    }
+  }
+  __syncthreads();
+
+  // this thread's pieces of a tile: row and 16-byte column piece
+  int prow[PIECES], pcol[PIECES];
+#pragma unroll
+  for (int j = 0; j < PIECES; ++j) {
+    const int p = (j * WAVES + wave) * kWave + lane;
+    prow[j] = p / (K / 4);
+    pcol[j] = 4 * (p % (K / 4));
+  }
+  const unsigned raw_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sRaw)) + wave * (kWave * 16);
+  const unsigned scale_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sScale)) + wave * (kWave * 16);
+
+  const int ntiles = sCum[ngw];
+  const int i1 = static_cast<int>(static_cast<int64_t>(ntiles) * (blockIdx.x + 1) / gridDim.x);
+  int i = static_cast<int>(static_cast<int64_t>(ntiles) * blockIdx.x / gridDim.x);
+  int g = 0, held_g = -1, held_l = -1;
+  bf16x8 w[CB][KS][3];  // weight pieces: column block, k step, piece
+
+  while (i < i1) {
+    while (sCum[g + 1] <= i) ++g;
+    const int tg = (sCum[g + 1] - sCum[g]) / 16;  // node tiles of the group
+    const int l = l_of_m((i - sCum[g]) / tg);
+    const int nm = 2 * l + 1;
+    const int blk0 = sCum[g] + tg * l * l;        // first tile of (g, l): tile blk0 + t * nm + (m - l * l)
+    const int t_first = (i - blk0) / nm;
+    const int seg_end = min(min(i1, blk0 + tg * nm), blk0 + (t_first + kSegTiles) * nm);
+    const int t_count = (seg_end - 1 - blk0) / nm - t_first + 1;
+    const int off0 = sOff[g], off1 = sOff[g + 1];
+
+    __syncthreads();  // every wave is done with the previous segment
+    // Row numbers of the segment's node tiles; a row beyond the end of the group stands in for the first row of its tile
+    // (the same values to the same place once more), so that no load or store of the tile loop is conditional.
+    for (int r = tid; r < TR * t_count; r += WAVES * kWave) {
+      const int p0 = off0 + TR * (t_first + r / TR);
+      const int p = p0 + r % TR;
+      int node = node_perm ? node_perm[p < off1 ? p : p0] : (p < off1 ? p : p0);
+      if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) node = node_perm ? node_perm[p0] : p0;
+      if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) node = 0;
+      sId[r] = node;
+    }
+    if (g != held_g || l != held_l) {
+      // a lane feeds 8 consecutive k of one weight column per step
+      const float *Wg = WT + ((static_cast<int64_t>(g) * 4 + l) * K + 16 * CB * wave + r16) * K + 8 * quarter;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          bf16x4 h0, m0, l0, h1, m1, l1;
+          split3(ld4(Wg + 16 * cb * K + 32 * s), h0, m0, l0);
+          split3(ld4(Wg + 16 * cb * K + 32 * s + 4), h1, m1, l1);
+          w[cb][s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+          w[cb][s][1] = __builtin_shufflevector(m0, m1, 0, 1, 2, 3, 4, 5, 6, 7);
+          w[cb][s][2] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      }
+      held_g = g;
+      held_l = l;
+    }
+    __syncthreads();
+
+    const int n = seg_end - i;
+    int t_scales = -1;  // node tile whose row_scale rows are in (or on their way into) sScale
+    auto where = [&](int k, int &m, int &tb) {  // component and first entry of sId of the segment's tile k
+      const int j = i + k - blk0;
+      const int t = j / nm;
+      m = l * l + (j - t * nm);
+      tb = TR * (t - t_first);
+    };
+    auto issue = [&](int k) {
+      int m, tb;
+      where(k, m, tb);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of the raw rows are done
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j)
+        dma16(X + (static_cast<int64_t>(sId[tb + prow[j]]) * 16 + m) * K + pcol[j], raw_lds + j * (WAVES * kWave * 16));
+      if constexpr (SCALED) {
+        if (tb != t_scales) {
+          t_scales = tb;
+#pragma unroll
+          for (int j = 0; j < PIECES; ++j)
+            dma16(row_scale + static_cast<int64_t>(sId[tb + prow[j]]) * K + pcol[j], scale_lds + j * (WAVES * kWave * 16));
+        }
+      }
+    };
+    auto split = [&](int k) {
+      __bf16 *plane = &sP[k & 1][0][0];
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j) {
+        const int p = (j * WAVES + wave) * kWave + lane;
+        f4 v = *reinterpret_cast<const f4 *>(sRaw + 4 * p);
+        if constexpr (SCALED) v *= *reinterpret_cast<const f4 *>(sScale + 4 * p);
+        bf16x4 h, md, lw;
+        split3(v, h, md, lw);
+        const int at = prow[j] * LD + pcol[j];
+        *reinterpret_cast<bf16x4 *>(plane + at) = h;
+        *reinterpret_cast<bf16x4 *>(plane + TR * LD + at) = md;
+        *reinterpret_cast<bf16x4 *>(plane + 2 * TR * LD + at) = lw;
+      }
+    };
+    auto multiply = [&](int k) {
+      int m, tb;
+      where(k, m, tb);
+      const __bf16 *plane = &sP[k & 1][0][0] + r16 * LD + 8 * quarter;
+      v4f acc[RB][CB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        bf16x8 x[RB][3];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) x[rb][q] = *reinterpret_cast<const bf16x8 *>(plane + q * (TR * LD) + 16 * rb * LD + 32 * s);
+        // piece products from small to large; consecutive instructions go to different accumulators
+        constexpr int kW[6] = {0, 2, 1, 0, 1, 0}, kX[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+              acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cb][s][kW[q]], x[rb][kX[q]], acc[rb][cb], 0, 0, 0);
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        float *op = OUT + (static_cast<int64_t>(sId[tb + 16 * rb + r16]) * 16 + m) * K + 16 * CB * wave + 4 * quarter;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const v4f v = acc[rb][cb] * scale;
+          // (the two idle issue slots: see the stores of the kernel above)
+          asm volatile("global_store_dwordx4 %0, %1, off offset:%2\n\ts_nop 1" : : "v"(op), "v"(v), "n"(64 * cb) : "memory");
+        }
+      }
+    };
+
+    issue(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    split(0);
+    if (n > 1) issue(1);
+    // before the first split of the loop only loads are out; the wait below is exact from the second tile on
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int k = 0; k < n; ++k) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // planes of tile k complete, those of tile k - 1 free
+      if (late) multiply(k);
+      if (k + 1 < n) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");  // the loads of tile k + 1; the stores after them may stay out
+        split(k + 1);
+        if (k + 2 < n) issue(k + 2);
+      }
+      if (!late) multiply(k);
+    }
+    i = seg_end;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int NT, int CB>
+int launch_wide(const float *X, const float *WT, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
+                int zero_last_group, float scale, const float *row_scale, float *OUT, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(device_compute_units())), block(2 * NT / CB * kWave);
+  if (row_scale)
+    hipLaunchKernelGGL((linear_wide_kernel<NT, CB, true>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
+                       zero_last_group, scale, row_scale, OUT);
+  else
+    hipLaunchKernelGGL((linear_wide_kernel<NT, CB, false>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
+                       zero_last_group, scale, row_scale, OUT);
+  return check_launch("cm_linear");
+}
+
 template <int K, int NT>
 int launch_resident(const float *X, const float *WT, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
                     int zero_last_group, int Nout, float scale, const float *row_scale, float *OUT, hipStream_t st) {
@@ -1071,12 +1325,17 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
   hipStream_t st = cm::as_stream(stream);
   // 16 components per node, square weights up to 128 and enough rows to give every compute unit a few tiles: the
   // kernel that keeps the weights in LDS (measured against the ring kernel at 25 000 nodes: 87 vs 102-112 us at 128
-  // channels, 58 vs 67-71 at 96, 42 vs 47 at 64; 360 vs 430 us at 100 000 x 128; equal at 2 500 nodes)
+  // channels, 58 vs 67-71 at 96, 42 vs 47 at 64; 360 vs 430 us at 100 000 x 128; equal at 2 500 nodes); at 160 to 256
+  // columns the one that keeps them in registers (equal to the tiled kernels at 2 048 nodes)
   if (ncomp == 16 && K == Nout && !residual && ngroups <= cm::kResMaxGroups && nnodes >= cm::kResMinNodes) {
     switch (K) {
 #define CM_CASE(K_, NT_) \
       case K_: return cm::launch_resident<K_, NT_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, Nout, scale, row_scale, OUT, st);
       CM_CASE(64, 2) CM_CASE(96, 3) CM_CASE(128, 4)
+#undef CM_CASE
+#define CM_CASE(NT_, CB_) \
+      case 32 * NT_: return cm::launch_wide<NT_, CB_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, scale, row_scale, OUT, st);
+      CM_CASE(5, 1) CM_CASE(6, 1) CM_CASE(7, 1) CM_CASE(8, 2)
 #undef CM_CASE
     }
   }
