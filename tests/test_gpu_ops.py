@@ -461,6 +461,23 @@ def test_linear_many_rows_wide(cabi, N, C, ne, seed):
     test_linear_many_rows(cabi, N, C, ne, seed)
 
 
+@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 192), (9007, 224), (12345, 256)])
+def test_scalar_linear_many_rows_wide(cabi, N, C):
+    """One component per node at 160 to 256 columns and 8 192 nodes and more: plain, with row_scale, with a residual that is a
+    tensor of its own, twice for the same bits."""
+    _say("scalar_linear_many_rows_wide", N, C)
+    g = torch.Generator().manual_seed(N)
+    X, S, R = (torch.randn(N, C, generator=g, dtype=torch.float64).float().double() for _ in range(3))
+    W = torch.randn(C, C, generator=g, dtype=torch.float64).float().double()
+    d = lambda t: t.float().to(DEV)
+    WT = W.t().contiguous().float().to(DEV)
+    out = cabi.linear(d(X), WT, scale=1.0)
+    close(out, X @ W, 1e-5, 2e-6)
+    close(cabi.linear(d(X), WT, scale=0.25, row_scale=d(S)), 0.25 * (X * S) @ W, 1e-5, 2e-6)
+    assert torch.equal(cabi.linear(d(X), WT, scale=1.0, residual=d(R)), out + d(R))
+    assert torch.equal(cabi.linear(d(X), WT, scale=1.0), out)
+
+
 @pytest.mark.parametrize("N,C", [(25000, 128), (100000, 192), (5000, 96)])
 def test_linear_at_benchmark_sizes(cabi, N, C):
     """The channel mixing at the node and channel counts of benchmark configurations 4, 5 and 3, per-element weights
