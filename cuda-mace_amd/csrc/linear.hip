@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "mfma_f32.hpp"
 #include "mfma_split.hpp"
 
 namespace cm {
@@ -225,6 +226,61 @@ __global__ __launch_bounds__(kWaves *kWave, ((NT == 5 || NT == 6) ? 2 : 1)) void
 
   // accumulator r of a lane is row 8*(r/4) + 4*(lane/32) + r%4, column lane%32 of the wave's 32x32 block
   store_block<NT>(acc, sNode, wave, half, mrow, ncomp, m, nout_total, col0, scale, residual, OUT);
+}
+
+// -----------------------------------------------------------------------------------------------
+// Few rows: 16 nodes x one component x 16 output columns per wave, operands straight to registers (mfma_f32.hpp).  No LDS,
+// no barrier: a wave waits for the group offsets, for its node's place in the permutation, and once for everything else.
+// In the 21-atom step a launch takes 3.1 us where tiles of 128 rows took 5.7, in the 216-atom, 128-channel step 4.2 and
+// 6.3 - 8.5 us where they took 8.7 and 10.7.
+template <int KQ, bool SCALED, int CB>
+__global__ __launch_bounds__(kWaves *kWave) void linear_few_rows_kernel(const float *__restrict__ X, const float *__restrict__ WT,
+                                                                        const int32_t *__restrict__ node_perm,
+                                                                        const int32_t *__restrict__ group_offsets, int nnodes,
+                                                                        int ngroups, int zero_last_group, int ncomp, float scale,
+                                                                        const float *__restrict__ row_scale, const float *residual,
+                                                                        float *OUT, int nout) {
+  constexpr int K = 16 * KQ;
+  const int lane = threadIdx.x % kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows;
+  const int col0 = few::kRows * CB * (blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);
+  const int m = blockIdx.x % ncomp;
+  const int l = ncomp == 1 ? 0 : l_of_m(m);
+  const int nblocks = ncomp == 1 ? 1 : 4;
+  int g, pos0, gend;
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x / ncomp, few::kRows, g, pos0, gend)) return;
+  int node = -1;
+  if (pos0 + row < gend) node = node_perm ? node_perm[pos0 + row] : pos0 + row;
+  const bool here = static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0;  // a row that is not there computes node 0's and drops it
+  const int64_t at = (in * ncomp + m) * nout + col0 + 4 * part;
+  f4 res[CB], out[CB];
+#pragma unroll
+  for (int c = 0; c < CB; ++c) {
+    res[c] = residual ? ld4(residual + at + few::kRows * c) : zero4();
+    out[c] = zero4();
+  }
+  if (!(zero_last_group && g == ngroups - 1)) {  // (rows of no weight group: the product is defined as zero)
+    const float *wp = WT + ((static_cast<int64_t>(g) * nblocks + l) * nout + col0 + row) * K + 4 * part;
+    few::Rows<KQ> w[CB];
+#pragma unroll
+    for (int c = 0; c < CB; ++c) w[c] = few::load_rows<KQ>(wp + few::kRows * c * K);
+    few::Rows<KQ> x = few::load_rows<KQ>(X + (in * ncomp + m) * K + 4 * part);
+    if constexpr (SCALED) {
+      const few::Rows<KQ> s = few::load_rows<KQ>(row_scale + in * K + 4 * part);
+#pragma unroll
+      for (int q = 0; q < KQ; ++q) x.v[q] *= s.v[q];
+    }
+    few::product<KQ, CB>(x, w, out);
+  }
+  if (!here) return;
+#pragma unroll
+  for (int c = 0; c < CB; ++c) {
+#pragma clang fp contract(off)  // the product is rounded before the residual is added, as everywhere
+    f4 v = out[c] * scale;
+    if (residual) v += res[c];
+    st4(OUT + at + few::kRows * c, v);
+  }
 }
 
 // -----------------------------------------------------------------------------------------------
@@ -1259,6 +1315,22 @@ int launch_resident(const float *X, const float *WT, const int32_t *perm, const 
   return check_launch("cm_linear");
 }
 
+template <int KQ, int CB>
+int launch_few_rows(const float *X, const float *WT, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
+                    int zero_last_group, int ncomp, int Nout, float scale, const float *row_scale, const float *residual, float *OUT,
+                    hipStream_t st) {
+  const int64_t tiles = ceil_div(nnodes, few::kRows) + (offs ? ngroups : 0);
+  const int cols = Nout / (few::kRows * CB), waves = cols % 4 == 0 ? 4 : (cols % 3 == 0 ? 3 : (cols % 2 == 0 ? 2 : 1));
+  const dim3 grid(static_cast<unsigned>(tiles * ncomp), static_cast<unsigned>(cols / waves)), block(waves * kWave);
+  if (row_scale)
+    hipLaunchKernelGGL((linear_few_rows_kernel<KQ, true, CB>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
+                       zero_last_group, ncomp, scale, row_scale, residual, OUT, Nout);
+  else
+    hipLaunchKernelGGL((linear_few_rows_kernel<KQ, false, CB>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
+                       zero_last_group, ncomp, scale, row_scale, residual, OUT, Nout);
+  return check_launch("cm_linear");
+}
+
 template <int NT>
 int launch(const float *X, const float *WT, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
            int zero_last_group, int ncomp, int K, float scale, const float *row_scale, const float *residual, float *OUT,
@@ -1339,6 +1411,16 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
   if (nnodes == 0) return CM_OK;
   CM_REQUIRE(X && W_T && OUT, "cm_linear: NULL pointer");
   hipStream_t st = cm::as_stream(stream);
+  // few rows, any width: the kernel without tiles (the line: mfma_f32.hpp)
+  if (cm::few::applies(nnodes, ncomp, Nout)) {
+    const bool one = cm::few::blocks(nnodes, ncomp, Nout) <= cm::few::kOneColumnBlock;
+    switch (K / 32) {
+#define CM_CASE(KC_) \
+      case KC_: return (one ? cm::launch_few_rows<2 * KC_, 1> : cm::launch_few_rows<2 * KC_, 2>)(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, ncomp, Nout, scale, row_scale, residual, OUT, st);
+      CM_CASE(1) CM_CASE(2) CM_CASE(3) CM_CASE(4) CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8)
+#undef CM_CASE
+    }
+  }
   // 16 components per node, square weights up to 128 and enough rows to give every compute unit a few tiles: the
   // kernel that keeps the weights in LDS (measured against the ring kernel at 25 000 nodes: 87 vs 102-112 us at 128
   // channels, 58 vs 67-71 at 96, 42 vs 47 at 64; 360 vs 430 us at 100 000 x 128; equal at 2 500 nodes); at 160 to 256

@@ -8,9 +8,8 @@
 //   backward   gh1 = gX2 . Wup^T + g1 + skip_e^T(g2)       gB1 = gh1 . Wprod1^T
 //
 // As separate launches of the linear kernel each of them keeps the device busy for a few microseconds and costs a
-// launch; here a workgroup takes a tile of 128 nodes of one element (32 where the node count leaves most compute units
-// without a tile of 128) through the whole chain.  The intermediate rows
-// (h1, gh1) stay in LDS as fp32 and are the X operand of the next product.  Arithmetic, operand split and accumulation
+// launch; in the first kernels below a workgroup takes a tile of 128 nodes of one element (32 where the node count leaves
+// most compute units without a tile of 128) through the whole chain.  The intermediate rows (h1, gh1) stay in LDS as fp32 and are the X operand of the next product.  Arithmetic, operand split and accumulation
 // order are those of the linear kernels (three bf16 pieces per fp32 operand, six piece products on
 // v_mfma_f32_32x32x16_bf16, K in chunks of 32), and every intermediate is rounded to fp32 where the separate launches
 // store it, so the chain returns the bits of the separate launches.
@@ -19,6 +18,7 @@
 // g1[n, c] = -weight[n] scale w1[c] is formed here from the linear readout's weights; g2 = -dE/dh2 arrives as dE/dh2 and
 // its sign goes into the scale of the skip product.
 #include "common.hpp"
+#include "mfma_f32.hpp"
 #include "mfma_split.hpp"
 #include "node_glue.hpp"
 
@@ -229,6 +229,66 @@ __global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_glue_forward_kerne
   });
 }
 
+// ---- few nodes (few::applies): tiles of 16, one wave per 16 output columns, products of mfma_f32.hpp ------------------
+// All weights of the chain and the tile's rows are requested before anything is waited for; between two products stands one
+// trip of the 16 rows through LDS.  Same products and roundings as the few-rows linear kernel, so again the bits of the
+// separate launches.  Measured at 216 nodes and 64 channels against 32-row tiles of the kernels above: forward 9.3 ->
+// 4.4 us, backward 8.7 -> 5.4.
+template <int NT>
+struct FewShared {
+  static constexpr int C = 32 * NT;
+  static constexpr int kThreads = 2 * NT * kWave;
+  static constexpr int kLd = C + 4;  // padded row stride (floats)
+  float tile[few::kRows * kLd];
+};
+
+// The wave's 16 columns of the tile's rows to LDS, and all columns of the lane's row back as an operand.
+template <class S>
+__device__ __forceinline__ void put(S &s, f4 v) {
+  const int lane = threadIdx.x % kWave;
+  *reinterpret_cast<f4 *>(s.tile + (lane % few::kRows) * S::kLd + few::kRows * (threadIdx.x / kWave) + 4 * (lane / few::kRows)) = v;
+}
+template <class S>
+__device__ __forceinline__ few::Rows<S::C / 16> get(const S &s) {
+  const int lane = threadIdx.x % kWave;
+  return few::load_rows<S::C / 16>(s.tile + (lane % few::kRows) * S::kLd + 4 * (lane / few::kRows));
+}
+
+template <int NT>
+__global__ __launch_bounds__(2 * NT *kWave) void node_glue_forward_few_kernel(
+    const float *__restrict__ B1, const float *__restrict__ prod_WT, const float *__restrict__ skip_WT,
+    const float *__restrict__ up_WT, const int32_t *__restrict__ node_perm, const int32_t *__restrict__ group_offsets, int nnodes,
+    int ngroups, float skip_scale, float *__restrict__ h1, float *__restrict__ sc, float *__restrict__ X2) {
+  constexpr int C = 32 * NT, KQ = C / 16;
+  using S = FewShared<NT>;
+  __shared__ __attribute__((aligned(16))) S s;
+  const int lane = threadIdx.x % kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows, col0 = few::kRows * (threadIdx.x / kWave);
+  const int64_t wat = static_cast<int64_t>(col0 + row) * C + 4 * part;
+  few::Rows<KQ> wp[1] = {few::load_rows<KQ>(prod_WT + wat)}, wu[1], ws[1];
+  int g, pos0, gend;
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x, few::kRows, g, pos0, gend)) return;
+  const int node = pos0 + row < gend ? node_perm[pos0 + row] : -1;
+  const bool here = static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0;
+  const bool no_element = g == ngroups - 1;  // nodes of no element: the skip connection is defined as zero there
+  const few::Rows<KQ> x = few::load_rows<KQ>(B1 + in * C + 4 * part);
+  ws[0] = few::load_rows<KQ>(skip_WT + static_cast<int64_t>(no_element ? 0 : g) * C * C + wat);
+  wu[0] = few::load_rows<KQ>(up_WT + wat);
+  __builtin_amdgcn_sched_barrier(0);  // the weights of all three products on their way before the first one waits
+  const int64_t at = in * C + col0 + 4 * part;
+  f4 v[1];
+  few::product<KQ, 1>(x, wp, v);
+  put(s, v[0]);
+  if (here) st4(h1 + at, v[0]);
+  __syncthreads();
+  const few::Rows<KQ> h = get(s);
+  few::product<KQ, 1>(h, wu, v);
+  if (here) st4(X2 + at, v[0]);
+  few::product<KQ, 1>(h, ws, v);
+  if (here) st4(sc + at, no_element ? zero4() : v[0] * skip_scale);
+}
+
 // Energies per graph, riding in the backward launch (its tiles do not depend on them): out[g] = sum over the graph's nodes
 // of weight[n] * node_es[n], strided partial sums of the workgroup's threads (the largest power of two of them) and a tree
 // over them: a fixed order.
@@ -240,22 +300,29 @@ struct EnergySums {
   const double *graph_e0;  // a constant per graph added into `total` (NULL: zero)
   double *total;           // NULL: not asked for
 };
-template <int THREADS>  // a power of two, at most the workgroup's size
+template <int THREADS, int PARTS = 4>  // THREADS: a power of two, at most the workgroup's size
 __device__ __forceinline__ void graph_energy(const EnergySums &q, int graph, double *part) {
   const int tid = threadIdx.x;
   if (tid < THREADS) {
     const int lo = q.graph_ptr[graph], hi = q.graph_ptr[graph + 1];
     auto term = [&](int i) { return q.node_weights ? q.node_weights[i] * q.node_es[i] : q.node_es[i]; };
-    // four strided partial sums per thread, their loads requested together: one sum after the other waits for memory
+    // PARTS strided partial sums per thread, their loads requested together: one sum after the other waits for memory
     // once per node, and this workgroup would outlast the tiles of the launch
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int i = lo + tid;
-    for (; i + 3 * THREADS < hi; i += 4 * THREADS) {
-      const double t0 = term(i), t1 = term(i + THREADS), t2 = term(i + 2 * THREADS), t3 = term(i + 3 * THREADS);
-      s0 += t0, s1 += t1, s2 += t2, s3 += t3;
+    double sum[PARTS];
+#pragma unroll
+    for (int k = 0; k < PARTS; ++k) sum[k] = 0.0;
+    for (int i = lo + tid; i < hi; i += PARTS * THREADS) {
+      double t[PARTS];
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k) t[k] = i + k * THREADS < hi ? term(i + k * THREADS) : 0.0;
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k) sum[k] += t[k];
     }
-    for (; i < hi; i += THREADS) s0 += term(i);
-    part[tid] = (s0 + s1) + (s2 + s3);
+#pragma unroll
+    for (int d = PARTS / 2; d > 0; d /= 2)
+#pragma unroll
+      for (int k = 0; k < d; ++k) sum[k] += sum[k + d];
+    part[tid] = sum[0];
   }
   __syncthreads();
   for (int d = THREADS / 2; d > 0; d >>= 1) {
@@ -324,6 +391,115 @@ __global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_glue_backward_kern
   });
 }
 
+// gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip^T of four columns of a node from the two products
+__device__ __forceinline__ f4 few_gh1(f4 up, f4 skip, const double *w1, double scale, double node_weight, float skip_scale, bool no_element) {
+  const f4 g1{static_cast<float>(-1.0 * scale * w1[0] * node_weight), static_cast<float>(-1.0 * scale * w1[1] * node_weight),
+              static_cast<float>(-1.0 * scale * w1[2] * node_weight), static_cast<float>(-1.0 * scale * w1[3] * node_weight)};
+  const f4 sum = up + g1;
+  return no_element ? sum : sum + skip * -skip_scale;
+}
+
+template <int NT>
+__global__ __launch_bounds__(2 * NT *kWave) void node_glue_backward_few_kernel(
+    const float *__restrict__ gX2, const float *__restrict__ d_h2, const float *__restrict__ up_W, const float *__restrict__ skip_W,
+    const float *__restrict__ prod_W, const double *__restrict__ w1, double scale, const double *__restrict__ node_weights,
+    const int32_t *__restrict__ node_perm, const int32_t *__restrict__ group_offsets, int nnodes, int ngroups, float skip_scale,
+    float *__restrict__ gB1, EnergySums sums, int first_tile) {
+  constexpr int C = 32 * NT, KQ = C / 16;
+  using S = FewShared<NT>;
+  __shared__ __attribute__((aligned(16))) S s;
+  if (static_cast<int>(blockIdx.x) < first_tile) {
+    constexpr int kSum = S::kThreads >= 512 ? 512 : (S::kThreads >= 256 ? 256 : 128);
+    static_assert(sizeof(s.tile) >= kSum * sizeof(double), "the tile holds the partial sums");
+    graph_energy<kSum, 8>(sums, blockIdx.x, reinterpret_cast<double *>(s.tile));
+    return;
+  }
+  const int lane = threadIdx.x % kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows, col0 = few::kRows * (threadIdx.x / kWave);
+  const int64_t wat = static_cast<int64_t>(col0 + row) * C + 4 * part;
+  few::Rows<KQ> wu[1] = {few::load_rows<KQ>(up_W + wat)}, ws[1], wp[1];
+  int g, pos0, gend;
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x - first_tile, few::kRows, g, pos0, gend)) return;
+  const int node = pos0 + row < gend ? node_perm[pos0 + row] : -1;
+  const bool here = static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0;
+  const bool no_element = g == ngroups - 1;
+  const few::Rows<KQ> x = few::load_rows<KQ>(gX2 + in * C + 4 * part), d = few::load_rows<KQ>(d_h2 + in * C + 4 * part);
+  ws[0] = few::load_rows<KQ>(skip_W + static_cast<int64_t>(no_element ? 0 : g) * C * C + wat);
+  wp[0] = few::load_rows<KQ>(prod_W + wat);
+  const double nw = node_weights ? node_weights[in] : 1.0;
+  __builtin_amdgcn_sched_barrier(0);
+  f4 v[1], u[1];
+  few::product<KQ, 1>(x, wu, v);
+  few::product<KQ, 1>(d, ws, u);
+  put(s, few_gh1(v[0], u[0], w1 + col0 + 4 * part, scale, nw, skip_scale, no_element));
+  __syncthreads();
+  few::product<KQ, 1>(get(s), wp, v);
+  if (here) st4(gB1 + in * C + col0 + 4 * part, v[0]);
+}
+
+// From 96 channels on the three products of a tile are too much for one compute unit (its eight waves share four matrix
+// pipes: 3 x 0.9 us at 128 channels, and 3 x 64 KB of weights on their way to it), so the chain is cut at h1 / gh1 and each
+// part spreads its 16-column blocks over the device like any linear.  Measured in the step of 216 nodes and 128 channels
+// (32-row tiles -> both launches): forward 15.4 -> 9.3 us, backward 16.3 -> 11.4 (one launch of the chain above: 10.8, 13.1).
+template <int KQ>
+__global__ __launch_bounds__(4 * kWave) void node_glue_skip_up_kernel(const float *__restrict__ h1, const float *__restrict__ skip_WT,
+                                                                      const float *__restrict__ up_WT, const int32_t *__restrict__ node_perm,
+                                                                      const int32_t *__restrict__ group_offsets, int nnodes, int ngroups,
+                                                                      float skip_scale, float *__restrict__ sc, float *__restrict__ X2) {
+  constexpr int C = 16 * KQ;
+  const int lane = threadIdx.x % kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows;
+  const int block = blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave;  // the first KQ: X2, the others: sc
+  const bool skip = block >= KQ;
+  const int col0 = few::kRows * (skip ? block - KQ : block);
+  int g, pos0, gend;
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x, few::kRows, g, pos0, gend)) return;
+  const int node = pos0 + row < gend ? node_perm[pos0 + row] : -1;
+  const bool here = static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0;
+  f4 v[1] = {zero4()};
+  if (!(skip && g == ngroups - 1)) {
+    const float *W = skip ? skip_WT + static_cast<int64_t>(g) * C * C : up_WT;
+    const few::Rows<KQ> w[1] = {few::load_rows<KQ>(W + static_cast<int64_t>(col0 + row) * C + 4 * part)};
+    few::product<KQ, 1>(few::load_rows<KQ>(h1 + in * C + 4 * part), w, v);
+  }
+  if (here) st4((skip ? sc : X2) + in * C + col0 + 4 * part, skip ? v[0] * skip_scale : v[0]);
+}
+
+template <int KQ>
+__global__ __launch_bounds__(4 * kWave) void node_glue_gh1_kernel(const float *__restrict__ gX2, const float *__restrict__ d_h2,
+                                                                  const float *__restrict__ up_W, const float *__restrict__ skip_W,
+                                                                  const double *__restrict__ w1, double scale,
+                                                                  const double *__restrict__ node_weights, const int32_t *__restrict__ node_perm,
+                                                                  const int32_t *__restrict__ group_offsets, int nnodes, int ngroups,
+                                                                  float skip_scale, float *__restrict__ gh1, EnergySums sums, int first_tile) {
+  constexpr int C = 16 * KQ;
+  constexpr int kSum = 128;
+  if (static_cast<int>(blockIdx.x) < first_tile) {
+    __shared__ double partial[kSum];
+    if (blockIdx.y == 0) graph_energy<kSum, 16>(sums, blockIdx.x, partial);
+    return;
+  }
+  const int lane = threadIdx.x % kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows;
+  const int col0 = few::kRows * (blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);
+  int g, pos0, gend;
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x - first_tile, few::kRows, g, pos0, gend)) return;
+  const int node = pos0 + row < gend ? node_perm[pos0 + row] : -1;
+  const bool here = static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0;
+  const bool no_element = g == ngroups - 1;
+  const int64_t wat = static_cast<int64_t>(col0 + row) * C + 4 * part;
+  const few::Rows<KQ> wu[1] = {few::load_rows<KQ>(up_W + wat)};
+  const few::Rows<KQ> ws[1] = {few::load_rows<KQ>(skip_W + static_cast<int64_t>(no_element ? 0 : g) * C * C + wat)};
+  f4 v[1], u[1];
+  few::product<KQ, 1>(few::load_rows<KQ>(gX2 + in * C + 4 * part), wu, v);
+  few::product<KQ, 1>(few::load_rows<KQ>(d_h2 + in * C + 4 * part), ws, u);
+  if (!here) return;
+  st4(gh1 + in * C + col0 + 4 * part, few_gh1(v[0], u[0], w1 + col0 + 4 * part, scale, node_weights ? node_weights[in] : 1.0, skip_scale, no_element));
+}
+
 // 128-node tiles where they give at least half of the compute units one each, 32-node tiles below that
 inline bool small_tiles(int64_t nnodes) { return ceil_div(nnodes, kGlTile) * 2 < device_compute_units(); }
 
@@ -331,6 +507,19 @@ template <int NT>
 void launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm,
                     const int32_t *offs, int64_t nnodes, int ngroups, float skip_scale, float *h1, float *sc, float *X2,
                     hipStream_t st) {
+  if (few::applies(nnodes, 1, 32 * NT)) {
+    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
+    if constexpr (NT >= 3) {
+      constexpr int kBlocks = 4 * NT, kPerGroup = NT == 3 ? 3 : 4;
+      (void)cm_linear(B1, prod_WT, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, h1, st);
+      hipLaunchKernelGGL((node_glue_skip_up_kernel<2 * NT>), dim3(tiles, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, h1, skip_WT,
+                         up_WT, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, sc, X2);
+    } else {
+      hipLaunchKernelGGL((node_glue_forward_few_kernel<NT>), dim3(tiles), dim3(2 * NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm,
+                         offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
+    }
+    return;
+  }
   if (small_tiles(nnodes)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
     hipLaunchKernelGGL((node_glue_forward_kernel<NT, kGlSmallTile>), dim3(tiles), dim3(NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT,
@@ -345,8 +534,23 @@ void launch_forward(const float *B1, const float *prod_WT, const float *skip_WT,
 template <int NT>
 void launch_backward(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W,
                      const double *w1, double scale, const double *node_weights, const int32_t *perm, const int32_t *offs,
-                     int64_t nnodes, int ngroups, float skip_scale, float *gB1, const EnergySums &sums, hipStream_t st) {
+                     int64_t nnodes, int ngroups, float skip_scale, float *gh1, float *gB1, const EnergySums &sums, hipStream_t st) {
   const unsigned extra = sums.out ? static_cast<unsigned>(sums.ngraphs) : 0u;
+  if (few::applies(nnodes, 1, 32 * NT)) {
+    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
+    if (NT >= 3 && gh1) {
+      constexpr int kBlocks = 2 * NT, kPerGroup = NT % 2 == 0 ? 4 : (NT % 3 == 0 ? 3 : 2);
+      hipLaunchKernelGGL((node_glue_gh1_kernel<2 * NT>), dim3(tiles + extra, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, gX2, d_h2,
+                         up_W, skip_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gh1, sums,
+                         static_cast<int>(extra));
+      (void)cm_linear(gh1, prod_W, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, gB1, st);
+      return;
+    }
+    hipLaunchKernelGGL((node_glue_backward_few_kernel<NT>), dim3(tiles + extra), dim3(2 * NT * kWave), 0, st, gX2, d_h2, up_W, skip_W,
+                       prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
+                       static_cast<int>(extra));
+    return;
+  }
   if (small_tiles(nnodes)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
     hipLaunchKernelGGL((node_glue_backward_kernel<NT, kGlSmallTile>), dim3(tiles + extra), dim3(NT * kWave), 0, st, gX2, d_h2, up_W,
@@ -388,15 +592,15 @@ namespace cm {
 // cm_node_glue_backward whose launch also sums the node energies per graph (operands checked by the caller, cm_mace_step)
 int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W,
                                         const double *w1, double scale, const double *node_weights, const int32_t *node_perm,
-                                        const int32_t *group_offsets, int64_t nnodes, int ngroups, int channels, float skip_scale,
+                                        const int32_t *group_offsets, int64_t nnodes, int ngroups, int channels, float skip_scale, float *gh1,
                                         float *gB1, const double *node_es, const int32_t *graph_ptr, int ngraphs, double *energies,
                                         const double *graph_e0, double *total_energies, hipStream_t st) {
   const EnergySums sums{node_es, node_weights, graph_ptr, energies, ngraphs, graph_e0, total_energies};
   switch (channels / 32) {
-    case 1: launch_backward<1>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gB1, sums, st); break;
-    case 2: launch_backward<2>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gB1, sums, st); break;
-    case 3: launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gB1, sums, st); break;
-    case 4: launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gB1, sums, st); break;
+    case 1: launch_backward<1>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
+    case 2: launch_backward<2>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
+    case 3: launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
+    case 4: launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
     default: set_error("node glue: channels=%d not supported", channels); return CM_EINVAL;
   }
   return check_launch("cm_node_glue_backward");
@@ -414,6 +618,6 @@ extern "C" int cm_node_glue_backward(const float *gX2, const float *d_h2, const 
   if (nnodes == 0) return CM_OK;
   CM_REQUIRE(gX2 && d_h2 && up_W && skip_W && prod_W && w1 && node_perm && group_offsets && gB1, "cm_node_glue_backward: NULL pointer");
   return cm::node_glue_backward_with_energy_sums(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets,
-                                                 nnodes, ngroups, channels, skip_scale, gB1, nullptr, nullptr, 0, nullptr, nullptr,
+                                                 nnodes, ngroups, channels, skip_scale, nullptr, gB1, nullptr, nullptr, 0, nullptr, nullptr,
                                                  nullptr, cm::as_stream(stream));
 }

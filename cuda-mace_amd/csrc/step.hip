@@ -548,7 +548,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // layer 0 (first interaction): its input features depend on the species alone, so no gradient with respect to them
   if (glue) {
     CM_STAGE(17, cm::node_glue_backward_with_energy_sums(L.gX2, L.d_h2, w->up_W, w->skip_W, w->prod_W[0], w->w1, w->scale, g->node_weights,
-                                                         oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.gB, node_energy, g->graph_ptr,
+                                                         oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.gh1, L.gB, node_energy, g->graph_ptr,
                                                          g->ngraphs, interaction_energy, g->graph_e0, total_energy, st));
   } else {
     CM_STAGE(17, cm_linear(L.gX2, w->up_W, nullptr, nullptr, N, 1, 0, 1, C, C, 1.0f, none, L.g1, L.gh1a, stream));

@@ -465,9 +465,9 @@ int cm_graph_prepare(const double *positions, const int32_t *row_i, const int32_
 /* ---------------------------------------------------------------------------------------------
  * The three [nnodes, C] x [C, C] linears between the two interaction layers as one launch per direction: the product's
  * linear and linear_up (the reference's linear_matmul, models/InvariantMACE.py:41-53) and the per-element skip
- * connection between them (element_linear_to_cuda, :56-74; called at :145-150 and :330).  A workgroup takes 128 nodes
- * of one element through the chain with the intermediate rows in LDS; same arithmetic, rounding points and results as
- * the three cm_linear calls it stands for.  channels = 32, 64, 96 or 128 (cm_node_glue_supported).
+ * connection between them (element_linear_to_cuda, :56-74; called at :145-150 and :330).  A workgroup takes a tile of nodes
+ * of one element through the chain with the intermediate rows in LDS (few nodes at 96 and 128 channels: two launches); same
+ * arithmetic, rounding points and results as the three cm_linear calls it stands for.  channels = 32, 64, 96 or 128 (cm_node_glue_supported).
  *   node_perm / group_offsets: nodes grouped by element, ngroups = nelements + 1 with the last group holding the nodes
  *   without an element (their skip connection is zero), as cm_linear takes them with zero_last_group.
  * Forward:  h1 = B1 . prod_W;  sc = skip_scale * h1 . skip_W[element];  X2 = h1 . up_W       (all fp32 [nnodes, C];

@@ -408,6 +408,38 @@ def test_node_glue_chains(cabi, N, C, ne, seed):
                                torch.zeros(3, dtype=torch.int32, device=DEV), 1.0)
 
 
+@pytest.mark.parametrize("N,C,ncomp,ne", [(15, 32, 1, 1), (17, 160, 16, 3), (256, 64, 16, 2), (257, 64, 16, 2), (768, 64, 16, 1), (769, 64, 16, 1),
+                                          (2048, 128, 1, 3), (2049, 128, 1, 3), (3073, 128, 1, 2), (2560, 256, 1, 1), (2561, 256, 1, 70), (193, 96, 16, 1)])
+def test_linear_few_rows(cabi, N, C, ncomp, ne):
+    """Both sides of the lines between one and two column blocks per wave and between this kernel and the tiled ones, with
+    per-element weights, a group without weights, row_scale and (one component) a residual; twice for the same bits."""
+    _say("linear_few_rows", N, C, ncomp, ne)
+    g = torch.Generator().manual_seed(N + C)
+    r32 = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64).float().double()  # noqa: E731
+    nl = 4 if ncomp == 16 else 1
+    X, S, R, W = r32(N, ncomp, C), r32(N, C), r32(N, ncomp, C), r32(ne, nl, C, C)
+    elem = torch.randint(0, ne + 1, (N,), generator=g)  # value ne: the group without weights
+    perm, off = cabi.stable_key_sort(elem.int().to(DEV), ne + 1)
+    shape = (lambda t: t) if ncomp == 16 else (lambda t: t.reshape(N, C))
+    wshape = (lambda t: t) if ncomp == 16 else (lambda t: t.reshape(-1, C, C))
+    d = lambda t: t.float().contiguous().to(DEV)  # noqa: E731
+    WT = wshape(W.transpose(-1, -2).contiguous())
+    ref = torch.zeros(N, ncomp, C, dtype=torch.float64)
+    for e in range(ne):
+        for m in range(ncomp):
+            sel = (elem == e).nonzero()[:, 0]
+            ref[sel, m] = (X[sel, m] * S[sel]) @ W[e, int(math.isqrt(m)) if nl == 4 else 0]
+    out = cabi.linear(d(shape(X)), d(WT), perm, off, scale=1.0, row_scale=d(S), zero_last_group=True)
+    close(out, shape(ref), 1e-5, 2e-6)
+    if ncomp == 1:
+        with_residual = cabi.linear(d(shape(X)), d(WT), perm, off, scale=1.0, row_scale=d(S), zero_last_group=True, residual=d(shape(R)))
+        assert torch.equal(with_residual, out + d(shape(R)))
+    assert torch.equal(cabi.linear(d(shape(X)), d(WT), perm, off, scale=1.0, row_scale=d(S), zero_last_group=True), out)
+    if ncomp == 1 and C == 128:  # the chains of the same products change their form at the same lines
+        test_node_glue_chains(cabi, N, C, ne, N)
+        test_node_glue_chains(cabi, N, 64, ne, N)
+
+
 @pytest.mark.parametrize("N,C,ne,seed", [(2048, 128, 1, 0), (2500, 128, 10, 1), (4099, 96, 5, 2), (3000, 64, 3, 3), (6000, 128, 130, 4)])
 def test_linear_many_rows(cabi, N, C, ne, seed):
     """16-component features with at least 2048 nodes and 64 / 96 / 128 square weights run on the kernel that keeps the
