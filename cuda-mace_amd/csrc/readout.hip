@@ -201,6 +201,120 @@ __global__ __launch_bounds__(kNodes *kHidden) void readout_forward_kernel(
   }
 }
 
+// C a multiple of 16 (every model width): the products on the fp64 matrix instruction, no weights and no rows in LDS.
+//
+// The kernel above is a chain of LDS reads and multiply-adds as long as the channel count, twice, on one workgroup per 16
+// nodes.  Here the four waves of a workgroup share the chain of its 16 nodes: wave w takes the 16-channel pieces w, w + 4, ..
+// of both feature rows, for its share of z (16 hidden units x 16 nodes, v_mfma_f64_16x16x4_f64) and of the first readout;
+// the shares meet once in LDS; then every wave knows all z and forms d2 for its own pieces.  A lane holds row lane % 16
+// of its operands, channels 4 (lane / 16) .. + 3 of a piece; element i of a result is row 4 i + lane / 16 of the 16, which
+// is where the next product wants the hidden unit, and d2 takes the rows of W2a in the order that makes a lane's four
+// results neighbours in memory.
+// Measured (us, the kernel above -> this one): 20 x 64 5.3 -> 3.6, 216 x 128 7.3 -> 5.1, 5 000 x 128 12.4 -> 8.5, 25 000 x 128
+// 32.4 -> 21.7, 12 000 x 256 33.4 -> 19.6 (with the fp64 rows written); few nodes: the latency of its chain, many: memory.
+typedef double d4v __attribute__((ext_vector_type(4)));
+constexpr int kMfmaWaves = 4;
+__global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel(
+    const float *__restrict__ h1, const float *__restrict__ h2, const double *__restrict__ w1, const double *__restrict__ W2a,
+    const double *__restrict__ w2b, double act_cst, double scale, double shift, int nnodes, int C, int H,
+    double *__restrict__ node_es, float *__restrict__ d2, double *__restrict__ feats64, const int32_t *__restrict__ feats_rows,
+    const double *__restrict__ node_e0, double *__restrict__ node_total) {
+  constexpr int kPieces = kMaxC / 16 / kMfmaWaves;  // of a wave, at the widest C
+  __shared__ double sZ[kMfmaWaves][4][kWave];
+  __shared__ double sE[kMfmaWaves][kWave], sE2[kMfmaWaves][kWave], sD[kMfmaWaves][kWave];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int col = lane % 16, part = lane / 16;
+  const int node = blockIdx.x * kNodes + col;
+  const bool here = node < nnodes;
+  const int in = here ? node : nnodes - 1;
+  const int npieces = C / 16;
+  const int unit = 4 * (col % 4) + col / 4;  // hidden unit of operand row col: element i of z is then unit 4 (lane / 16) + i
+  f4 a[kPieces], b[kPieces];
+  double wz[kPieces][4], wd[kPieces][4];
+  d2v wl[kPieces][2];
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int p = wave + kMfmaWaves * u;
+    if (p >= npieces) break;  // the same for the whole wave
+    const int c = 16 * p + 4 * part;
+    a[u] = ld4(h1 + static_cast<int64_t>(in) * C + c);
+    b[u] = ld4(h2 + static_cast<int64_t>(in) * C + c);
+    wl[u][0] = *reinterpret_cast<const d2v *>(w1 + c), wl[u][1] = *reinterpret_cast<const d2v *>(w1 + c + 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      wz[u][i] = unit < H ? W2a[(c + i) * H + unit] : 0.0;
+    }
+    if (d2) {
+      const double *wp = W2a + static_cast<int64_t>(16 * p + 4 * (col % 4) + col / 4) * H + 4 * part;
+      if (H == kHidden) {
+        const d2v lo = reinterpret_cast<const d2v *>(wp)[0], hi = reinterpret_cast<const d2v *>(wp)[1];
+        wd[u][0] = lo.x, wd[u][1] = lo.y, wd[u][2] = hi.x, wd[u][3] = hi.y;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wd[u][i] = 4 * part + i < H ? wp[i] : 0.0;
+      }
+    }
+  }
+  const double gate = 4 * part + wave < H ? w2b[4 * part + wave] * act_cst : 0.0;
+  const int row = feats_rows ? feats_rows[in] : in;
+  const bool row_ok = here && static_cast<unsigned>(row) < static_cast<unsigned>(nnodes);
+
+  d4v z{0.0, 0.0, 0.0, 0.0};
+  double e1 = 0.0;
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int p = wave + kMfmaWaves * u;
+    if (p >= npieces) break;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      z = __builtin_amdgcn_mfma_f64_16x16x4f64(wz[u][i], static_cast<double>(b[u][i]), z, 0, 0, 0);
+      e1 += static_cast<double>(a[u][i]) * wl[u][i / 2][i % 2];
+    }
+    if (feats64 && row_ok) {
+      double *f = feats64 + static_cast<int64_t>(row) * (2 * C) + 16 * p + 4 * part;
+      reinterpret_cast<d2v *>(f)[0] = d2v{a[u].x, a[u].y};
+      reinterpret_cast<d2v *>(f)[1] = d2v{a[u].z, a[u].w};
+      reinterpret_cast<d2v *>(f + C)[0] = d2v{b[u].x, b[u].y};
+      reinterpret_cast<d2v *>(f + C)[1] = d2v{b[u].z, b[u].w};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sZ[wave][i][lane] = z[i];
+  sE[wave][lane] = e1;
+  __syncthreads();
+  // wave i: the gate of element i of z
+  auto total = [&](const auto &v) { return (v(0) + v(1)) + (v(2) + v(3)); };
+  {
+    const double z_i = total([&](int w) { return sZ[w][wave][lane]; });
+    const double sig = 1.0 / (1.0 + exp(-z_i));
+    sE2[wave][lane] = gate * z_i * sig;
+    sD[wave][lane] = gate * (sig + z_i * sig * (1.0 - sig));
+  }
+  __syncthreads();
+  if (wave == 0) {
+    double e = total([&](int w) { return sE[w][lane]; }) + total([&](int w) { return sE2[w][lane]; });
+    e += __shfl_xor(e, 16);
+    e += __shfl_xor(e, 32);
+    if (here && part == 0) {
+      const double en = scale * e + shift;
+      node_es[node] = en;
+      if (node_total && row_ok) node_total[row] = en + (node_e0 ? node_e0[node] : 0.0);
+    }
+  }
+  if (!d2) return;
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int p = wave + kMfmaWaves * u;
+    if (p >= npieces) break;
+    d4v g{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g = __builtin_amdgcn_mfma_f64_16x16x4f64(wd[u][i], sD[i][lane], g, 0, 0, 0);
+    if (here)
+      st4(d2 + static_cast<int64_t>(node) * C + 16 * p + 4 * part,
+          f4{static_cast<float>(scale * g[0]), static_cast<float>(scale * g[1]), static_cast<float>(scale * g[2]), static_cast<float>(scale * g[3])});
+  }
+}
+
 __global__ void readout_backward_kernel(const double *__restrict__ g, const double *__restrict__ w1, const float *__restrict__ d2,
                                         double scale, int64_t total, int C, float *__restrict__ g1, float *__restrict__ g2) {
   const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -224,6 +338,12 @@ int readout_forward_with_totals(const float *h1, const float *h2, const double *
   CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 2, "cm_readout_forward: nnodes out of range");
   if (nnodes == 0) return CM_OK;
   CM_REQUIRE(h1 && h2 && w1 && W2a && w2b && node_energies, "cm_readout_forward: NULL pointer");
+  if (channels % 16 == 0) {
+    hipLaunchKernelGGL(readout_forward_mfma_kernel, dim3(static_cast<unsigned>(ceil_div(nnodes, kNodes))), dim3(kMfmaWaves * kWave), 0, st,
+                       h1, h2, w1, W2a, w2b, act_cst, scale, shift, static_cast<int>(nnodes), channels, hidden, node_energies, d_h2,
+                       node_feats64, rows, node_e0, node_total);
+    return check_launch("cm_readout_forward");
+  }
   // at most kMaxGroups workgroups (two per compute unit of a 256-unit device fit by their LDS): each stages the
   // weights once and walks several tiles
   const int64_t tiles = ceil_div(nnodes, kNodes);
