@@ -144,8 +144,7 @@ __device__ __forceinline__ bool locate_group_tile(const int32_t *__restrict__ gr
     const int lo = lane < ngroups ? group_offsets[lane] : 0, hi = lane < ngroups ? group_offsets[lane + 1] : 0;
     const int tiles = (hi - lo + tile_rows - 1) / tile_rows;
     int upto = tiles;  // inclusive prefix sum over the lanes
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
+    for (int d = 1; d < ngroups; d <<= 1) {
       const int v = __shfl_up(upto, d);
       if (lane >= d) upto += v;
     }
