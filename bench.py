@@ -81,18 +81,24 @@ def traffic_of(table, kernels):
 def forward_kernel_name(C, N):
     """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_spline.hip: cm_mp_edge_forward; the
     benchmark's spline table has 256 knots)."""
-    if 2048 <= N < 2**24 and C % 16 == 0 and N * C < 2**30:
+    share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
+    if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30:
         return "mp_edge_forward_sliced_kernel"
     return "mp_spline_forward_kernel<%d,true>" % C
 
 
 def linear_kernel_name(C, N):
-    """The library runs the [N,16,C] channel-mixing linear on its kernel with LDS-resident weights for 64, 96 and 128
-    columns when there are at least 2 048 nodes, else on the LDS-ring kernel for 64, 96, 128, 224 and 256 columns and on
-    the plain one otherwise."""
+    """The library runs the [N,16,C] channel-mixing linear without tiles for few nodes, from 2 048 nodes on with the weights
+    resident (64, 96 and 128 columns: in LDS, 160 and more: in registers), else on the LDS-ring kernel for 64, 96, 128, 224
+    and 256 columns and on the plain one otherwise."""
     nt = C // 32
+    blocks = (N + 15) // 16 * C
+    if blocks <= 3072:
+        return "linear_few_rows_kernel<%d,false,%d>" % (C // 16, 1 if blocks <= 1024 else 2)
     if nt in (2, 3, 4) and N >= 2048:
         return "linear_resident_kernel<%d,%d,false>" % (C, nt)
+    if nt >= 5 and N >= 2048:
+        return "linear_wide_kernel<%d,%d,16,false>" % (nt, 2 if nt == 8 else 1)
     return ("linear_ring_kernel<%d,false>" if nt in (2, 3, 4, 7, 8) else "linear_kernel<%d,false>") % nt
 
 

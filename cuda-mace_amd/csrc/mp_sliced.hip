@@ -52,7 +52,12 @@ constexpr int kSlThreads = 512;       // two waves per SIMD (three: 168 register
 constexpr int kSlMaxIntervals = 272;  // 136 KB of table (one row of it is the row of zeros)
 constexpr int kSlSub = 4096;          // nodes sorted at a time
 constexpr int kSlBins = 64;           // edge blocks per node that the sort tells apart
-constexpr int kSlMinNodes = 2048;
+// From six rounds of 16 nodes per workgroup on (1 280 nodes at 128 channels, 2 560 at 64); below that some of its waves have none
+// and what the workgroup spends on its slice of the table (4 us) counts.  Measured against one wave per node (us): 1 200 x 192
+// 45.7 -> 32.7, 1 750 x 128 35.4 -> 31.0, 2 000 x 128 38.5 -> 32.1, 3 000 x 64 31.3 -> 28.5, 4 000 x 64 43.0 -> 31.2; four
+// rounds, 2 048 x 64: 22.5 against 25.8.
+constexpr int kSlMinRounds = 6;
+inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)
 
 struct SlicedArgs {
   const float *X, *vec;
@@ -410,8 +415,9 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
 }  // namespace
 
 bool sliced_forward_applies(int64_t nnodes, int channels, int nknots) {
-  return nnodes >= kSlMinNodes && nnodes < (1 << 24) && nnodes * channels < (int64_t{1} << 30) && channels % 16 == 0 && nknots >= 2 &&
-         nknots - 1 < kSlMaxIntervals && device_compute_units() / (2 * (channels / 16)) >= 2;
+  if (channels % 16 != 0 || share_of(channels) < 2) return false;
+  return nnodes > static_cast<int64_t>(share_of(channels)) * (kWave / 4) * (kSlMinRounds - 1) && nnodes < (1 << 24) &&
+         nnodes * channels < (int64_t{1} << 30) && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }
 
 int launch_sliced_forward(const float *X, const float *vec, const float *knots, const float *coeffs, int nknots, float r_width,
@@ -419,7 +425,7 @@ int launch_sliced_forward(const float *X, const float *vec, const float *knots, 
                           int channels, float *out, hipStream_t st) {
   SlicedArgs a{X, vec, sender, first_occ, coeffs, knots, nknots, r_width, r_max, static_cast<int>(nnodes), nedges, channels, out,
                channels / 16, 0};
-  a.share = device_compute_units() / (2 * a.nslices);
+  a.share = share_of(channels);
   hipLaunchKernelGGL(mp_edge_forward_sliced_kernel, dim3(static_cast<unsigned>(a.share * 2 * a.nslices)), dim3(kSlThreads), 0, st, a);
   return check_launch("cm_mp_edge_forward");
 }

@@ -209,6 +209,14 @@ def test_mp_edge_forward_many_nodes(cabi, case):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("case", [(5121, 4, 32, 0.1, 5, 256, 0), (2561, 9, 64, 0.0, 6, 256, 300), (2560, 9, 64, 0.0, 6, 256, 300),
+                                  (1281, 7, 128, 0.1, 7, 272, 0), (1280, 7, 128, 0.1, 7, 272, 0), (641, 11, 256, 0.2, 8, 2, 0)],
+                         ids=lambda c: "N%d_C%d" % (c[0], c[2]))
+def test_mp_edge_forward_on_both_sides_of_the_line(cabi, case):
+    """The smallest node counts at which that kernel is taken, and the largest at which it is not."""
+    test_mp_edge_forward_many_nodes(cabi, case)
+
+
 def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi):
     """40 000 receiver nodes at 256 channels: a workgroup of the LDS-table kernel sorts and serves its nodes in more than
     one batch.  Checked against the kernel that takes harmonics and lengths (same radial table, same per-edge
