@@ -236,3 +236,29 @@ def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi)
     Rv = O.spline_eval(vec[live].norm(dim=1), knots, coeffs, h, 5.0).view(-1, 4, C)
     ref = O.mp_forward(X, O.spherical_harmonics(vec[live]), Rv, snd[live], rcv[live], nnodes)
     close(out[nodes.cuda()], ref[nodes], 2e-5, 2e-6)
+
+
+@pytest.mark.parametrize("case", [(1024, 6, 160, 0.2, 21, 256, 0), (1100, 13, 160, 0.0, 22, 600, 150), (1024, 5, 192, 0.2, 23, 256, 0),
+                                  (1060, 17, 192, 0.0, 24, 2, 129)], ids=lambda c: "N%d_C%d_k%d" % (c[0], c[2], c[5]))
+def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
+    """From 1 024 nodes on at 160 and 192 channels: nodes with every remainder of a group of four edges, one with more than
+    one and more than two chunks of 64, dead edges in between, knots in LDS and in memory, a table of one interval."""
+    nnodes, C = case[0], case[2]
+    snd, rcv, X, vec, knots, coeffs, h = _edge_case(*case)
+    degrees = torch.bincount(rcv.long(), minlength=nnodes)
+    assert set((degrees % 4).tolist()) == {0, 1, 2, 3}
+    G = torch.randn(nnodes, 16, C, generator=torch.Generator().manual_seed(case[4]), dtype=torch.float64)
+    live = (vec.norm(dim=1).float() <= 5.0) & (snd >= 0) & (snd < nnodes)
+    va, Xa = vec[live].clone().requires_grad_(True), X.clone().requires_grad_(True)
+    Rv = O.spline_eval(va.norm(dim=1), knots, coeffs, h, 5.0).view(-1, 4, C)
+    (O.mp_forward(Xa, O.spherical_harmonics(va), Rv, snd[live], rcv[live], nnodes) * G).sum().backward()
+    d = lambda t: t.float().cuda()
+    fo = cabi.first_occurences(rcv.cuda(), nnodes)
+    perm, off = cabi.stable_key_sort(snd.cuda(), nnodes)
+    args = (d(X), d(vec), d(knots), d(coeffs), h, 5.0, d(G), snd.cuda(), fo, perm, off, nnodes)
+    gX, gvec = cabi.mp_edge_backward(*args)
+    close(gX, Xa.grad, 2e-5, 2e-6)
+    close(gvec[live.cuda()], va.grad, 5e-5, 5e-6)
+    assert float(gvec[~live.cuda()].abs().max()) == 0.0
+    assert torch.equal(cabi.mp_edge_backward(*args, need_gvec=False)[0], gX)
+    assert torch.equal(cabi.mp_edge_backward(*args, need_gX=False)[1], gvec)
