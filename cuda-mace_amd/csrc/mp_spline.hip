@@ -749,15 +749,15 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
             if constexpr (WANT_GV) grq += q0 * dr;
           } else {
             const f4 p = x * rl;
+            f4 du = p[0] * d[L][0];  // a sum of its own per degree: one chain over everything loses a little accuracy
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
               if constexpr (WANT_GX) gxe[t] += rl[t] * d[L][t][0];
               if constexpr (!WANT_GV) continue;
               grq[t] += d[L][t][0] * dr[t];
-              ux += p[t] * d[L][t][1];
-              uy += p[t] * d[L][t][2];
-              uz += p[t] * d[L][t][3];
+              if (t > 0) du += p[t] * d[L][t];
             }
+            if constexpr (WANT_GV) ux += du[1], uy += du[2], uz += du[3];
           }
           __builtin_amdgcn_sched_barrier(0);
         };
