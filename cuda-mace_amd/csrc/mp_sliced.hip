@@ -55,8 +55,13 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 // From six rounds of 16 nodes per workgroup on (1 280 nodes at 128 channels, 2 560 at 64); below that some of its waves have none
 // and what the workgroup spends on its slice of the table (4 us) counts.  Measured against one wave per node (us): 1 200 x 192
 // 45.7 -> 32.7, 1 750 x 128 35.4 -> 31.0, 2 000 x 128 38.5 -> 32.1, 3 000 x 64 31.3 -> 28.5, 4 000 x 64 43.0 -> 31.2; four
-// rounds, 2 048 x 64: 22.5 against 25.8.
+// rounds, 2 048 x 64: 22.5 against 25.8.  Up to 2 048 nodes the edges count as well, since the 4 us stay and the rest goes
+// with them (nodes x neighbours x channels): 1 500 x 20 x 128 16.0 -> 17.6, 1 500 x 60 x 128 34.9 -> 30.4, 1 800 x 20 x 96
+// 15.1 -> 17.6; beyond 128 channels, where the other kernel has one edge per wave, the line is lower: 1 100 x 8 x 192
+// 14.4 -> 15.5, 1 300 x 20 x 192 26.0 -> 21.7, 1 500 x 20 x 160 26.0 -> 20.9, 2 000 x 12 x 160 25.9 -> 22.2.
 constexpr int kSlMinRounds = 6;
+constexpr int kSlAnyEdges = 2048;  // nodes
+inline int min_edges_of(int channels) { return channels > 128 ? 12000 : 60000; }
 inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)
 
 struct SlicedArgs {
@@ -414,8 +419,9 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
 
 }  // namespace
 
-bool sliced_forward_applies(int64_t nnodes, int channels, int nknots) {
-  if (channels % 16 != 0 || share_of(channels) < 2) return false;
+bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nknots) {
+  if (channels % 16 != 0 || share_of(channels) < 2 || nedges == 0) return false;
+  if (nnodes < kSlAnyEdges && nedges < min_edges_of(channels)) return false;
   return nnodes > static_cast<int64_t>(share_of(channels)) * (kWave / 4) * (kSlMinRounds - 1) && nnodes < (1 << 24) &&
          nnodes * channels < (int64_t{1} << 30) && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }

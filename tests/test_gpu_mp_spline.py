@@ -210,8 +210,9 @@ def test_mp_edge_forward_many_nodes(cabi, case):
 
 
 @pytest.mark.parametrize("case", [(5121, 4, 32, 0.1, 5, 256, 0), (2561, 9, 64, 0.0, 6, 256, 300), (2560, 9, 64, 0.0, 6, 256, 300),
-                                  (1281, 7, 128, 0.1, 7, 272, 0), (1280, 7, 128, 0.1, 7, 272, 0), (641, 11, 256, 0.2, 8, 2, 0)],
-                         ids=lambda c: "N%d_C%d" % (c[0], c[2]))
+                                  (1281, 7, 128, 0.1, 7, 272, 0), (1280, 7, 128, 0.1, 7, 272, 0), (641, 11, 256, 0.2, 8, 2, 0),
+                                  (1281, 50, 128, 0.0, 7, 272, 0), (641, 20, 256, 0.0, 8, 2, 0)],
+                         ids=lambda c: "N%d_d%d_C%d" % (c[0], c[1], c[2]))
 def test_mp_edge_forward_on_both_sides_of_the_line(cabi, case):
     """The smallest node counts at which that kernel is taken, and the largest at which it is not."""
     test_mp_edge_forward_many_nodes(cabi, case)
