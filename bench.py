@@ -536,7 +536,7 @@ def main():
                                         "duration"})
         others = [entry("mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C, bwd_fb, t_bwd,
                         launches_timed=launches(bwd_name),
-                        note="bounded by VALU issue (~80% of all issue slots), see the counter summary")]
+                        note="bounded by the delivery of the spline table from L2 (8 KB per edge at 128 channels): with a third fewer vector instructions it takes the same time")]
         t_lin = avg_ms("linear")
         if t_lin:
             flops = 32 * N * C * C

@@ -822,8 +822,10 @@ void launch_edge(const float *X, const float *Y, const Spline &sp, const float *
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
   // From 1 024 nodes on, a wave per SIMD: below, a node's chain of staging and first loads is what counts, and this kernel
   // stages more per edge (300 x 192 without / with gX: 19.7 / 28.0 -> 20.7 / 30.3 us; 2 000 x 160: 86.5 / 117 -> 74.1 / 103).
+  // At 192 channels also from 12 edges per node on: 10 000 x 8 without / with gX 75.1 / 100.6 -> 75.1 / 106.0 us, 2 000 x 12
+  // 31.0 / 42.8 -> 27.1 / 39.0; at 160, 10 000 x 8 82.6 / 105.1 -> 78.7 / 102.3.
   if constexpr (FROM_VEC && (C == 160 || C == 192)) {
-    if (nnodes >= kMatrixMinNodes) {
+    if (nnodes >= kMatrixMinNodes && (C == 160 || nedges >= 12 * nnodes)) {
       hipLaunchKernelGGL((mp_edge_backward_matrix_kernel<C, GY, GX>), grid, dim3(kWave), 0, st, X, sp, G, sender, first_occ,
                          static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
       return;

@@ -239,10 +239,10 @@ def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi)
     close(out[nodes.cuda()], ref[nodes], 2e-5, 2e-6)
 
 
-@pytest.mark.parametrize("case", [(1024, 6, 160, 0.2, 21, 256, 0), (1100, 13, 160, 0.0, 22, 600, 150), (1024, 5, 192, 0.2, 23, 256, 0),
-                                  (1060, 17, 192, 0.0, 24, 2, 129)], ids=lambda c: "N%d_C%d_k%d" % (c[0], c[2], c[5]))
+@pytest.mark.parametrize("case", [(1024, 6, 160, 0.2, 21, 256, 0), (1100, 13, 160, 0.0, 22, 600, 150), (1024, 5, 192, 0.2, 23, 256, 0), (1024, 15, 192, 0.2, 25, 256, 0),
+                                  (1060, 17, 192, 0.0, 24, 2, 129)], ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
 def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
-    """From 1 024 nodes on at 160 and 192 channels: nodes with every remainder of a group of four edges, one with more than
+    """From 1 024 nodes on at 160 channels, and with 12 edges per node at 192: nodes with every remainder of a group of four edges, one with more than
     one and more than two chunks of 64, dead edges in between, knots in LDS and in memory, a table of one interval."""
     nnodes, C = case[0], case[2]
     snd, rcv, X, vec, knots, coeffs, h = _edge_case(*case)
