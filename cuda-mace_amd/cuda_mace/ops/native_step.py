@@ -2,8 +2,8 @@
 backward chain are enqueued by the C side, with no interpreter or autograd engine between the launches.
 
 `NativeStep` gathers what that call needs from an `OptimizedInvariantMACE`: the frozen weights as one C struct (built
-once per model), the index structures of a neighbour list and species tensor as another (built once per list), and a
-workspace that is reused from step to step.  Same kernels, same order, same numbers as the autograd path of the model.
+once per model) and the index structures of a neighbour list and species tensor as another (built once per list); outputs
+and scratch memory belong to the call.  Same kernels, same order, same numbers as the autograd path of the model.
 """
 from __future__ import annotations
 
@@ -97,7 +97,6 @@ class NativeStep:
         w.hidden = int(model.readout_W2a.shape[1])
         w.act_cst, w.scale, w.shift = (float(v) for v in model.readout_constants)
         self.weights, self._keep, self.channels, self.nelements = w, keep, C, w.nelements
-        self._workspace = None
 
     def graph(self, edge_index, receiver, sender, node_attrs32, atom_types, ptr, X1, node_rows, node_e0=None,
               graph_e0=None) -> "_GraphHandle":
@@ -146,16 +145,11 @@ class NativeStep:
         sh64 = shifts.detach().to(F64).contiguous()
         if pos64.shape != (N, 3) or sh64.shape != (E, 3):
             raise cabi.CudaMaceError("native step: positions must be [%d, 3] and shifts [%d, 3]" % (N, E))
+        # Scratch memory of this call alone, from torch's allocator: it is handed out again only to later work of this
+        # stream, so calls on other streams or from other threads (ctypes lets go of the interpreter lock) have theirs, and a
+        # captured step has its own for as long as its graph lives.  A steady caller gets the same block every time.
         need = cabi.lib.cm_mace_step_workspace(N, E, C)
-        if torch.cuda.is_current_stream_capturing():
-            # A captured step keeps the address it was recorded with for as long as its graph lives: its workspace comes
-            # from the capture's own memory pool (which the graph owns), never from the buffer eager calls share, which a
-            # later, larger evaluation replaces.
-            ws = torch.empty(need, dtype=torch.uint8, device=dev)
-        else:
-            ws = self._workspace
-            if ws is None or ws.numel() < need or ws.device != dev:
-                ws = self._workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
         energy = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_energy = torch.empty(N, dtype=F64, device=dev)
         forces = torch.empty(N, 3, dtype=F64, device=dev) if want_forces else None

@@ -529,7 +529,9 @@ int cm_node_glue_backward(const float *gX2, const float *d_h2, const float *up_W
  * -dE/d vec_e.  total_energy fp64 [ngraphs] or NULL = interaction_energy + graph_e0; total_node_energy fp64 [nnodes] or NULL
  * = node_energy + node_e0, atom n of the lists written to row node_rows[n] (what the reference returns as "energy" and
  * "node_energy", models/InvariantMACE.py:350-352, without a launch of their own).  workspace: cm_mace_step_workspace(nnodes, nedges, channels) bytes, 256-byte aligned; its
- * contents are scratch.  Nothing is allocated, so the call can be captured into a HIP graph.
+ * contents are scratch.  It belongs to the call until the call's kernels have run: calls on one stream may follow each other
+ * on the same workspace, calls on several streams, or from several threads, need one each (nothing in the library checks
+ * this).  Nothing is allocated, so the call can be captured into a HIP graph.
  */
 typedef struct cm_mace_weights {
   int channels, nelements, nknots, hidden;

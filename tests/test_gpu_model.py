@@ -496,7 +496,7 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
 def test_repeated_evaluations_agree_bit_for_bit_at_every_width(cabi, channels):
     """Every kernel sums in a fixed order and reads nothing it (or an earlier kernel of the same step) has not written:
     the same input gives the same bits again, also after an evaluation of another size has left other values in the
-    shared workspace.  Two sizes per width: with one wave per node and with a node's edges cut into parts (few nodes).
+    memory the next one is given.  Two sizes per width: with one wave per node and with a node's edges cut into parts (few nodes).
     (A kernel whose hand-issued loads were read before they had landed once passed every tolerance test and failed
     only this kind.)"""
     from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
@@ -504,11 +504,11 @@ def test_repeated_evaluations_agree_bit_for_bit_at_every_width(cabi, channels):
     boxes = {"large": to_device(make_system(2100, 4, seed=12, density=0.1), "cuda"),
              "small": to_device(make_system(260, 4, seed=11, density=0.1), "cuda")}
     up = SyntheticInvariantMACE(channels=channels, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=52.0, seed=13)
-    model = OptimizedInvariantMACE(up, device="cuda")  # one model: both boxes share its workspace
+    model = OptimizedInvariantMACE(up, device="cuda")
     first = {k: model(dict(d)) for k, d in boxes.items()}
     assert model._native not in (None, False)
     for _ in range(2):
-        for k, d in boxes.items():  # the other size ran in between: the workspace holds its leftovers
+        for k, d in boxes.items():  # the other size ran in between: the scratch memory holds its leftovers
             again = model(dict(d))
             for key in ("energy", "node_energy", "forces", "node_feats"):
                 assert torch.equal(again[key], first[k][key]), "%s of the %s box differs between evaluations at C=%d" % (key, k, channels)
@@ -610,7 +610,7 @@ def test_a_second_model_on_the_same_tensors_gets_its_own_graph_handle(cabi):
 
 def test_captured_step_survives_a_larger_eager_evaluation(cabi):
     """A step captured as a HIP graph keeps its own workspace: evaluating the same model eagerly on a larger structure
-    afterwards (which replaces the buffer eager calls share) must not disturb the replays."""
+    afterwards must not disturb the replays."""
     from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
     from cuda_mace.utils.graph import GraphedStep
 
@@ -623,7 +623,7 @@ def test_captured_step_survives_a_larger_eager_evaluation(cabi):
     big = model(dict(dev_large))
     torch.cuda.synchronize()
     big2 = model(dict(dev_large))
-    # the eager buffer was replaced and is in use by other work; the replay still reads and writes its own
+    # the memory of the eager calls is in use by other work; the replay still reads and writes its own
     for _ in range(3):
         again = step()
         torch.cuda.synchronize()
@@ -635,3 +635,69 @@ def test_captured_step_survives_a_larger_eager_evaluation(cabi):
     for k, v in first.items():
         assert torch.equal(fresh[k].detach(), v), k
     assert torch.equal(big["forces"], big2["forces"])
+
+
+@pytest.mark.parametrize("channels", [64, 160])
+def test_one_model_on_two_streams(cabi, channels):
+    """Energies and full steps of one model in flight on two streams at once, the first held back so that the second is
+    enqueued before it has run: every result has the bits it has alone."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    up = SyntheticInvariantMACE(channels=channels, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=50.0, seed=2)
+    model = OptimizedInvariantMACE(up, device="cuda")
+    boxes = [to_device(make_system(n, 4, seed=3 + k, density=0.1), "cuda") for k, n in enumerate((700, 430))]
+    keys = ("energy", "node_energy", "node_feats")
+
+    def evaluate(box, forces):
+        if forces:
+            return model(dict(boxes[box]))
+        with torch.no_grad():
+            return model(dict(boxes[box]), compute_force=False)
+
+    alone = {(b, f): evaluate(b, f) for b in range(2) for f in (False, True)}
+    assert model._native not in (None, False)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for first in (False, True):
+        for second in (False, True):
+            for _ in range(3):
+                with torch.cuda.stream(streams[0]):
+                    torch.cuda._sleep(2_000_000)
+                    a = evaluate(0, first)
+                with torch.cuda.stream(streams[1]):
+                    b = evaluate(1, second)
+                    again = evaluate(0, second)
+                torch.cuda.synchronize()
+                for out, want, forces in ((a, alone[0, first], first), (b, alone[1, second], second), (again, alone[0, second], second)):
+                    for k in keys + (("forces",) if forces else ()):
+                        assert torch.equal(out[k], want[k]), (k, first, second)
+
+
+def test_one_model_from_two_threads(cabi):
+    """Two threads, each with a stream of its own, evaluate one model at the same time."""
+    import threading
+
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    up = SyntheticInvariantMACE(channels=96, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=50.0, seed=2)
+    model = OptimizedInvariantMACE(up, device="cuda")
+    boxes = [to_device(make_system(n, 4, seed=5 + k, density=0.1), "cuda") for k, n in enumerate((600, 350))]
+    alone = [{k: model(dict(d))[k] for k in ("energy", "forces", "node_energy")} for d in boxes]
+    torch.cuda.synchronize()
+    differing = []
+
+    def work(box):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                out = model(dict(boxes[box]))
+                stream.synchronize()
+                differing.extend((box, k) for k, v in alone[box].items() if not torch.equal(out[k], v))
+
+    threads = [threading.Thread(target=work, args=(b,)) for b in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not differing
