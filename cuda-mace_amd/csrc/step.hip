@@ -112,8 +112,9 @@ __global__ void weight_rows_kernel(float *__restrict__ x, const double *__restri
 
 // Edge vectors and the edge range of every receiver node cut back to its last edge inside the cutoff, one launch.
 // Thread i forms the vector of edge i (fp64 difference of the positions plus the shift, rounded once to fp32: the
-// arithmetic of cm_edge_geometry_forward) and clears the vector gradients of an edge beyond the cutoff (the backward edge
-// passes skip the edges behind a node's mark, and write the same zeros for those before it).  The thread of a receiver's
+// arithmetic of cm_edge_geometry_forward) and, where a backward chain follows (gv1 and gv2 given), clears the vector
+// gradients of an edge beyond the cutoff (the backward edge passes skip the edges behind a node's mark, and write the same
+// zeros for those before it).  The thread of a receiver's
 // last edge closes the receiver's range: live[n] = first_occ[n], live[nnodes + n] = one past the last edge e of the node
 // with |vec[e]| <= r_max (the node's first edge if there is none).  The message-passing kernels, forward and backward,
 // skip the edges behind that mark, which contribute exact zeros.  A Verlet list holds a third more pairs than the cutoff
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
     vec[3 * i + 1] = v1;
     vec[3 * i + 2] = v2;
     inside = mp::edge_length(v0, v1, v2) <= r_max;
-    if (!inside) {
+    if (!inside && gv1) {
       gv1[3 * i + 0] = gv1[3 * i + 1] = gv1[3 * i + 2] = 0.f;
       gv2[3 * i + 0] = gv2[3 * i + 1] = gv2[3 * i + 2] = 0.f;
     }
@@ -336,7 +337,9 @@ __global__ __launch_bounds__(256) void probe_fma_kernel(float *out, int iters) {
 
 inline size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
-// Carves the workspace; the same walk sizes it (base == nullptr) and lays it out.
+// Carves the workspace; the same walk sizes it (base == nullptr) and lays it out.  Energies alone keep nothing for a backward
+// chain: no gradient rows, no E x C of per-edge gradients, one message for both layers (the first layer's is read before the
+// second's is written, and so is what its contraction leaves).
 struct Layout {
   float *vec, *gv1, *gv2, *bufM1, *bufM2, *bufA, *edge_scratch;
   float *B1, *h1, *sc, *X2, *B2, *h2, *d_h2, *g1, *gB, *gX2, *gh1a, *gh1;
@@ -344,7 +347,7 @@ struct Layout {
   double *node_virial;   // [N, 6]
   size_t bytes;
 
-  Layout(void *base, int64_t N, int64_t E, int C) {
+  Layout(void *base, int64_t N, int64_t E, int C, bool forces) {
     size_t at = 0;
     auto take = [&](size_t n) {
       char *p = base ? static_cast<char *>(base) + at : nullptr;
@@ -352,14 +355,15 @@ struct Layout {
       return p;
     };
     auto f = [&](int64_t n) { return reinterpret_cast<float *>(take(static_cast<size_t>(n) * sizeof(float))); };
+    auto backward = [&](int64_t n) { return forces ? f(n) : nullptr; };
     const int64_t NC = N * C;
-    vec = f(3 * E), gv1 = f(3 * E), gv2 = f(3 * E);
-    bufM1 = f(16 * NC), bufM2 = f(16 * NC), bufA = f(16 * NC);
-    edge_scratch = f(E * C);
-    B1 = f(NC), h1 = f(NC), sc = f(NC), X2 = f(NC), B2 = f(NC), h2 = f(NC), d_h2 = f(NC);
-    g1 = f(NC), gB = f(NC), gX2 = f(NC), gh1a = f(NC), gh1 = f(NC);
+    vec = f(3 * E), gv1 = backward(3 * E), gv2 = backward(3 * E);
+    bufM1 = f(16 * NC), bufM2 = forces ? f(16 * NC) : bufM1, bufA = f(16 * NC);
+    edge_scratch = backward(E * C);
+    B1 = f(NC), h1 = f(NC), sc = f(NC), X2 = f(NC), B2 = forces ? f(NC) : B1, h2 = f(NC), d_h2 = backward(NC);
+    g1 = backward(NC), gB = backward(NC), gX2 = backward(NC), gh1a = backward(NC), gh1 = backward(NC);
     live = reinterpret_cast<int32_t *>(take(static_cast<size_t>(2 * N) * sizeof(int32_t)));
-    node_virial = reinterpret_cast<double *>(take(static_cast<size_t>(6 * N) * sizeof(double)));
+    node_virial = forces ? reinterpret_cast<double *>(take(static_cast<size_t>(6 * N) * sizeof(double))) : nullptr;
     bytes = at;
   }
 };
@@ -384,7 +388,12 @@ extern "C" int cm_stress(const double *virials, const double *cell, int64_t ngra
 
 extern "C" size_t cm_mace_step_workspace(int64_t nnodes, int64_t nedges, int channels) {
   if (nnodes < 0 || nedges < 0 || channels <= 0) return 0;
-  return cm::Layout(nullptr, nnodes, nedges, channels).bytes;
+  return cm::Layout(nullptr, nnodes, nedges, channels, true).bytes;
+}
+
+extern "C" size_t cm_mace_energy_workspace(int64_t nnodes, int64_t nedges, int channels) {
+  if (nnodes < 0 || nedges < 0 || channels <= 0) return 0;
+  return cm::Layout(nullptr, nnodes, nedges, channels, false).bytes;
 }
 
 // Runs one stage; with the stage's timing bit set, between two events recorded on the stream.
@@ -427,7 +436,8 @@ extern "C" int cm_mace_step_timing_read(double *total_ms, int64_t *launches, int
 namespace {
 
 // The step of cm_mace_step, or, with want_forces false, its forward half alone: no backward chain, and none of what only
-// that chain reads (the contractions' gradient tables, the readouts' derivative) is formed or written.
+// that chain reads (the contractions' gradient tables, the readouts' derivative, cleared edge gradients) is formed, written or
+// given room.
 int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *positions, const double *shifts, void *workspace,
              size_t workspace_bytes, double *interaction_energy, double *node_energy, bool want_forces, double *forces,
              double *node_feats, double *virials, double *total_energy, double *total_node_energy, cm_stream_t stream) {
@@ -468,9 +478,9 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
                    (w->mono3[t] == nullptr) == (w->mono2[t] == nullptr),
                "cm_mace_step: NULL weight of layer %d", t);
   CM_REQUIRE(w->r_knots && w->up_WT && w->up_W && w->skip_WT && w->skip_W && w->w1 && w->W2a && w->w2b, "cm_mace_step: NULL weight");
-  const cm::Layout L(workspace, N, E, C);
+  const cm::Layout L(workspace, N, E, C, want_forces);
   if (workspace == nullptr || workspace_bytes < L.bytes) {
-    cm::set_error("cm_mace_step: workspace of %zu bytes, need %zu", workspace_bytes, L.bytes);
+    cm::set_error("cm_mace_step / cm_mace_energy: workspace of %zu bytes, need %zu", workspace_bytes, L.bytes);
     return CM_ENOSPC;
   }
   CM_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "cm_mace_step: workspace must be 256-byte aligned");

@@ -148,7 +148,7 @@ class NativeStep:
         # Scratch memory of this call alone, from torch's allocator: it is handed out again only to later work of this
         # stream, so calls on other streams or from other threads (ctypes lets go of the interpreter lock) have theirs, and a
         # captured step has its own for as long as its graph lives.  A steady caller gets the same block every time.
-        need = cabi.lib.cm_mace_step_workspace(N, E, C)
+        need = (cabi.lib.cm_mace_step_workspace if want_forces else cabi.lib.cm_mace_energy_workspace)(N, E, C)
         ws = torch.empty(need, dtype=torch.uint8, device=dev)
         energy = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_energy = torch.empty(N, dtype=F64, device=dev)

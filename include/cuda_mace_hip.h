@@ -585,9 +585,12 @@ int cm_mace_step(const cm_mace_weights *weights, const cm_mace_graph *graph, con
 /* stress fp64 [ngraphs, 3, 3] = -virials / |det cell|, cell fp64 [ngraphs, 3, 3] row vectors (the reference's get_outputs,
  * models/InvariantMACE.py:354, in one launch). */
 int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double *stress, cm_stream_t stream);
-/* The forward half of cm_mace_step: the same energies and features, bit for bit, without forces.  No backward chain runs and
- * nothing that only it reads is written (12 launches up to 128 channels, 14 beyond).  For callers that compare energies:
- * Monte Carlo moves, screening. */
+/* The forward half of cm_mace_step without forces: node energies and features bit for bit those of the full step; the sums
+ * per graph may differ from its in the last bits (up to 128 channels the full step forms them in another launch, with
+ * another number of partial sums).  No backward chain runs, nothing that only it reads is written, and the workspace,
+ * cm_mace_energy_workspace(nnodes, nedges, channels) bytes, has no room for it (a workspace of cm_mace_step will do as well).
+ * 12 launches up to 128 channels, 14 beyond.  For callers that compare energies: Monte Carlo moves, screening. */
+size_t cm_mace_energy_workspace(int64_t nnodes, int64_t nedges, int channels);
 int cm_mace_energy(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
                    void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy, double *node_feats,
                    double *total_energy, double *total_node_energy, cm_stream_t stream);

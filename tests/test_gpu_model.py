@@ -436,6 +436,36 @@ def test_energy_alone(cabi, atoms, C, relabel):
     assert model(dict(data), compute_force=False)["energy"].requires_grad
 
 
+@pytest.mark.parametrize("atoms,C", [(21, 64), (300, 128), (1400, 192), (9000, 96)])
+def test_energy_stays_inside_its_workspace(cabi, atoms, C):
+    """cm_mace_energy on a list with a skin (pairs beyond the cutoff), its workspace inside a larger buffer of a fixed
+    byte: the bytes behind it are as they were, and node energies and features are those of the full step."""
+    import ctypes
+
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.neighbour_list import neighbour_data
+
+    base = to_device(make_system(atoms, 4, seed=3, density=None if atoms < 100 else 0.1, cluster_box=12.0 if atoms < 100 else None), "cuda")
+    data = neighbour_data(base["positions"], base["node_attrs"], 5.5)
+    up = SyntheticInvariantMACE(channels=C, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=30.0, seed=2)
+    model = OptimizedInvariantMACE(up, device="cuda", spatial_order_min_atoms=None)
+    full = model(dict(data))
+    step, handle = model._native, list(data["edge_index"].__dict__["_cm_native_graphs"].values())[0][2]
+    E = data["edge_index"].shape[1]
+    need = cabi.lib.cm_mace_energy_workspace(atoms, E, C)
+    guard = torch.full((need + (1 << 20),), 0x5A, dtype=torch.uint8, device="cuda")
+    f64 = dict(dtype=torch.float64, device="cuda")
+    energy, node_energy, feats = torch.empty(1, **f64), torch.empty(atoms, **f64), torch.empty(atoms, 2 * C, **f64)
+    args = [ctypes.addressof(step.weights), ctypes.addressof(handle.struct), data["positions"].data_ptr(), data["shifts"].data_ptr(),
+            guard.data_ptr(), need, energy.data_ptr(), node_energy.data_ptr(), feats.data_ptr(), None, None, cabi._stream()]
+    cabi._check(cabi.lib.cm_mace_energy(*args))
+    assert int((guard[need:] != 0x5A).sum()) == 0
+    assert torch.equal(feats, full["node_feats"])
+    torch.testing.assert_close(energy, full["interaction_energy"], rtol=1e-12, atol=1e-12)
+    args[5] = need - 1
+    assert cabi.lib.cm_mace_energy(*args) == -28
+
+
 @pytest.mark.parametrize("relabel", [True, False], ids=["shell_last", "shell_in_place"])
 def test_native_step_on_a_list_with_a_skin(cabi, relabel):
     """A neighbour list built out to cutoff + skin, at a size where the forward runs the LDS-table kernel: the step walks

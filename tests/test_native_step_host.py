@@ -56,3 +56,15 @@ def test_calls_under_way_at_the_same_time_share_no_scratch_memory(monkeypatch):
             evaluate(want_forces=outer)
             (_, a, na), (_, b, nb) = library.calls
             assert a + na <= b or b + nb <= a, "forces %s inside forces %s: both calls write the same memory" % (inner, outer)
+
+
+def test_energies_alone_take_no_memory_of_the_backward_chain(monkeypatch):
+    """Vectors [E, 3] and edge ranges, two [N, 16, C], five [N, C], each rounded up to 256 bytes: nothing of the E x C of
+    per-edge gradients or of the gradient rows."""
+    library, evaluate = _step(monkeypatch)
+    evaluate(want_forces=False)
+    evaluate(want_forces=True)
+    (kind, _, energy), (_, _, step) = library.calls
+    assert kind == "energy"
+    assert energy <= 4 * (3 * E + 2 * N + (2 * 16 + 5) * N * C) + 256 * 9
+    assert step >= energy + 4 * E * C
