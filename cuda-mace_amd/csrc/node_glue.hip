@@ -504,37 +504,39 @@ __global__ __launch_bounds__(4 * kWave) void node_glue_gh1_kernel(const float *_
 inline bool small_tiles(int64_t nnodes) { return ceil_div(nnodes, kGlTile) * 2 < device_compute_units(); }
 
 template <int NT>
-void launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm,
-                    const int32_t *offs, int64_t nnodes, int ngroups, float skip_scale, float *h1, float *sc, float *X2,
-                    hipStream_t st) {
+int launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm,
+                   const int32_t *offs, int64_t nnodes, int ngroups, float skip_scale, float *h1, float *sc, float *X2,
+                   hipStream_t st) {
   if (few::applies(nnodes, 1, 32 * NT)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
     if constexpr (NT >= 3) {
       constexpr int kBlocks = 4 * NT, kPerGroup = NT == 3 ? 3 : 4;
-      (void)cm_linear(B1, prod_WT, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, h1, st);
+      const int rc = cm_linear(B1, prod_WT, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, h1, st);
+      if (rc != CM_OK) return rc;
       hipLaunchKernelGGL((node_glue_skip_up_kernel<2 * NT>), dim3(tiles, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, h1, skip_WT,
                          up_WT, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, sc, X2);
     } else {
       hipLaunchKernelGGL((node_glue_forward_few_kernel<NT>), dim3(tiles), dim3(2 * NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm,
                          offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
     }
-    return;
+    return check_launch("cm_node_glue_forward");
   }
   if (small_tiles(nnodes)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
     hipLaunchKernelGGL((node_glue_forward_kernel<NT, kGlSmallTile>), dim3(tiles), dim3(NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT,
                        perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
-    return;
+    return check_launch("cm_node_glue_forward");
   }
   const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlTile) + ngroups);
   hipLaunchKernelGGL((node_glue_forward_kernel<NT, kGlTile>), dim3(tiles), dim3(4 * NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm,
                      offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
+  return check_launch("cm_node_glue_forward");
 }
 
 template <int NT>
-void launch_backward(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W,
-                     const double *w1, double scale, const double *node_weights, const int32_t *perm, const int32_t *offs,
-                     int64_t nnodes, int ngroups, float skip_scale, float *gh1, float *gB1, const EnergySums &sums, hipStream_t st) {
+int launch_backward(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W,
+                    const double *w1, double scale, const double *node_weights, const int32_t *perm, const int32_t *offs,
+                    int64_t nnodes, int ngroups, float skip_scale, float *gh1, float *gB1, const EnergySums &sums, hipStream_t st) {
   const unsigned extra = sums.out ? static_cast<unsigned>(sums.ngraphs) : 0u;
   if (few::applies(nnodes, 1, 32 * NT)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
@@ -543,25 +545,27 @@ void launch_backward(const float *gX2, const float *d_h2, const float *up_W, con
       hipLaunchKernelGGL((node_glue_gh1_kernel<2 * NT>), dim3(tiles + extra, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, gX2, d_h2,
                          up_W, skip_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gh1, sums,
                          static_cast<int>(extra));
-      (void)cm_linear(gh1, prod_W, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, gB1, st);
-      return;
+      const int rc = check_launch("cm_node_glue_backward");
+      if (rc != CM_OK) return rc;
+      return cm_linear(gh1, prod_W, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, gB1, st);
     }
     hipLaunchKernelGGL((node_glue_backward_few_kernel<NT>), dim3(tiles + extra), dim3(2 * NT * kWave), 0, st, gX2, d_h2, up_W, skip_W,
                        prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
                        static_cast<int>(extra));
-    return;
+    return check_launch("cm_node_glue_backward");
   }
   if (small_tiles(nnodes)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
     hipLaunchKernelGGL((node_glue_backward_kernel<NT, kGlSmallTile>), dim3(tiles + extra), dim3(NT * kWave), 0, st, gX2, d_h2, up_W,
                        skip_W, prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
                        static_cast<int>(extra));
-    return;
+    return check_launch("cm_node_glue_backward");
   }
   const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlTile) + ngroups);
   hipLaunchKernelGGL((node_glue_backward_kernel<NT, kGlTile>), dim3(tiles + extra), dim3(4 * NT * kWave), 0, st, gX2, d_h2, up_W, skip_W,
                      prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
                      static_cast<int>(extra));
+  return check_launch("cm_node_glue_backward");
 }
 
 }  // namespace
@@ -579,12 +583,12 @@ extern "C" int cm_node_glue_forward(const float *B1, const float *prod_WT, const
   CM_REQUIRE(B1 && prod_WT && skip_WT && up_WT && node_perm && group_offsets && h1 && sc && X2, "cm_node_glue_forward: NULL pointer");
   hipStream_t st = cm::as_stream(stream);
   switch (channels / 32) {
-    case 1: cm::launch_forward<1>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st); break;
-    case 2: cm::launch_forward<2>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st); break;
-    case 3: cm::launch_forward<3>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st); break;
-    case 4: cm::launch_forward<4>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st); break;
+    case 1: return cm::launch_forward<1>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st);
+    case 2: return cm::launch_forward<2>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st);
+    case 3: return cm::launch_forward<3>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st);
+    case 4: return cm::launch_forward<4>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st);
   }
-  return cm::check_launch("cm_node_glue_forward");
+  return CM_EINVAL;
 }
 
 namespace cm {
@@ -597,13 +601,12 @@ int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, con
                                         const double *graph_e0, double *total_energies, hipStream_t st) {
   const EnergySums sums{node_es, node_weights, graph_ptr, energies, ngraphs, graph_e0, total_energies};
   switch (channels / 32) {
-    case 1: launch_backward<1>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
-    case 2: launch_backward<2>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
-    case 3: launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
-    case 4: launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st); break;
+    case 1: return launch_backward<1>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
+    case 2: return launch_backward<2>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
+    case 3: return launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
+    case 4: return launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     default: set_error("node glue: channels=%d not supported", channels); return CM_EINVAL;
   }
-  return check_launch("cm_node_glue_backward");
 }
 
 }  // namespace cm
