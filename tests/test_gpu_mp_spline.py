@@ -263,3 +263,27 @@ def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
     assert float(gvec[~live.cuda()].abs().max()) == 0.0
     assert torch.equal(cabi.mp_edge_backward(*args, need_gvec=False)[0], gX)
     assert torch.equal(cabi.mp_edge_backward(*args, need_gX=False)[1], gvec)
+
+
+@pytest.mark.parametrize("nnodes,C", [(1750, 96), (1400, 128), (1000, 160), (900, 192), (700, 256)])
+def test_forward_from_vectors_is_no_less_precise_than_from_harmonics_and_lengths(cabi, nnodes, C):
+    """From vectors these sizes run on the kernel that forms length and direction from one reciprocal square root; given
+    harmonics and lengths they run with one wave per node.  The lengths handed over are those the other kernels form from
+    fp32 vectors: squares added up by fma, a correctly rounded square root.  Over the two million components of the message
+    the relative error against fp64 is a number with three firm digits, so two per cent are allowed."""
+    snd, rcv, X, vec, knots, coeffs, h = _edge_case(nnodes, 52, C, 0.0, 31)
+    X = X.float().double()
+    r2 = torch.zeros(vec.shape[0], dtype=torch.float64)
+    for k in range(3):
+        r2 = (r2 + vec[:, k] ** 2).float().double()  # the product is exact in fp64: one rounding, as in an fma
+    r = r2.sqrt().float()
+    live = (r <= 5.0) & (snd >= 0) & (snd < nnodes)
+    R = O.spline_eval(vec[live].norm(dim=1), knots, coeffs, h, 5.0).view(-1, 4, C)
+    ref = O.mp_forward(X, O.spherical_harmonics(vec[live]), R, snd[live], rcv[live], nnodes)
+    d = lambda t: t.float().cuda()
+    fo = cabi.first_occurences(rcv.cuda(), nnodes)
+    a = cabi.mp_edge_forward(d(X), d(vec), d(knots), d(coeffs), h, 5.0, snd.cuda(), fo, nnodes)
+    b = cabi.mp_spline_forward(d(X), cabi.sh_forward(d(vec)), r.cuda(), d(knots), d(coeffs), h, 5.0, snd.cuda(), fo, nnodes)
+    error_a, error_b = (float((t.double().cpu() - ref).norm() / ref.norm()) for t in (a, b))
+    print("C=%d from vectors %.3e, from harmonics and lengths %.3e" % (C, error_a, error_b), flush=True)
+    assert error_a <= 1.02 * error_b
