@@ -55,16 +55,32 @@ constexpr int kSlThreads = 512;       // two waves per SIMD (three: 168 register
 constexpr int kSlMaxIntervals = 272;  // 136 KB of table (one row of it is the row of zeros)
 constexpr int kSlSub = 4096;          // nodes sorted at a time
 constexpr int kSlBins = 64;           // edge blocks per node that the sort tells apart
-// From six rounds of 16 nodes per workgroup on (1 280 nodes at 128 channels, 2 560 at 64); below that some of its waves have none
-// and what the workgroup spends on its slice of the table (4 us) counts.  Measured against one wave per node (us): 1 200 x 192
-// 45.7 -> 32.7, 1 750 x 128 35.4 -> 31.0, 2 000 x 128 38.5 -> 32.1, 3 000 x 64 31.3 -> 28.5, 4 000 x 64 43.0 -> 31.2; four
-// rounds, 2 048 x 64: 22.5 against 25.8.  Up to 2 048 nodes the edges count as well, since the 4 us stay and the rest goes
-// with them (nodes x neighbours x channels): 1 500 x 20 x 128 16.0 -> 17.6, 1 500 x 60 x 128 34.9 -> 30.4, 1 800 x 20 x 96
-// 15.1 -> 17.6; beyond 128 channels, where the other kernel has one edge per wave, the line is lower: 1 100 x 8 x 192
-// 14.4 -> 15.5, 1 300 x 20 x 192 26.0 -> 21.7, 1 500 x 20 x 160 26.0 -> 20.9, 2 000 x 12 x 160 25.9 -> 22.2.
+// From six rounds of 16 nodes per workgroup on (5 121 nodes at 32 channels, 2 561 at 64, 1 281 at 128, 641 at 256); below
+// that some of its waves have none.  From there on the edges decide: a workgroup spends 4 us on its slice of the table, and
+// nodes with few edges leave it with the fixed part of a round, while the kernel with one wave per node pays per edge.
+// Measured, one wave per node -> this one (us), nodes x neighbours:
+//   32 channels   5 121 x 2 15.9 -> 10.7, 12 000 x 2 30.9 -> 17.4: always
+//   64            2 561 x 20 16.4 -> 17.7, 2 561 x 52 29.8 -> 28.5, 5 000 x 14 22.0 -> 23.2, 5 000 x 20 26.0 -> 25.5, 8 000 x 2 18.6 -> 19.8,
+//                 8 000 x 8 24.9 -> 24.0, 12 000 x 2 25.3 -> 24.3
+//   96, 128       1 681 x 30 x 96 19.2 -> 22.1, 1 681 x 52 31.5 -> 29.9, 3 500 x 14 22.1 -> 23.9, 3 500 x 20 27.0 -> 27.0, 12 000 x 8
+//                 37.7 -> 40.7, 12 000 x 14 54.5 -> 50.2; 1 281 x 52 x 128 28.4 -> 28.9, 2 049 x 8 12.8 -> 17.4, 2 049 x 30
+//                 28.4 -> 26.4, 5 000 x 8 23.9 -> 27.9, 5 000 x 14 33.9 -> 32.8, 12 000 x 8 45.6 -> 49.0, 12 000 x 14 68.0 -> 61.7
+//   160, 224      (there the other kernel fetches five and seven single channels per lane) 961 x 8 x 160 13.7 -> 15.1, 961 x 14
+//                 18.5 -> 17.3, 5 000 x 5 26.7 -> 28.7, 5 000 x 8 33.9 -> 32.3; 721 x 8 x 224 13.9 -> 16.4, 721 x 14 21.6 -> 20.0, 12 000 x 8 87.7 -> 78.5
+//   192, 256      801 x 8 x 192 12.8 -> 14.6, 801 x 14 17.7 -> 16.9, 5 000 x 8 33.6 -> 37.5, 5 000 x 14 50.1 -> 46.2; 641 x 8 x 256
+//                 14.6 -> 17.1, 641 x 14 22.7 -> 20.0, 12 000 x 8 85.9 -> 97.4, 12 000 x 14 137.5 -> 130.8
 constexpr int kSlMinRounds = 6;
-constexpr int kSlAnyEdges = 2048;  // nodes
-inline int min_edges_of(int channels) { return channels > 128 ? 12000 : 60000; }
+inline int64_t min_edges(int64_t nnodes, int channels) {
+  switch (channels) {
+    case 32: return 0;
+    case 64: return 120000 - 10 * nnodes;
+    case 96:
+    case 128: return std::max<int64_t>(60000, 11 * nnodes);
+    case 160:
+    case 224: return std::max<int64_t>(10000, 8 * nnodes);
+    default: return 11 * nnodes;
+  }
+}
 inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)
 
 struct SlicedArgs {
@@ -427,7 +443,7 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
 
 bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nknots) {
   if (channels % 16 != 0 || share_of(channels) < 2 || nedges == 0) return false;
-  if (nnodes < kSlAnyEdges && nedges < min_edges_of(channels)) return false;
+  if (nedges < min_edges(nnodes, channels)) return false;
   return nnodes > static_cast<int64_t>(share_of(channels)) * (kWave / 4) * (kSlMinRounds - 1) && nnodes < (1 << 24) &&
          nnodes * channels < (int64_t{1} << 30) && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }

@@ -218,6 +218,36 @@ def test_mp_edge_forward_on_both_sides_of_the_line(cabi, case):
     test_mp_edge_forward_many_nodes(cabi, case)
 
 
+@pytest.mark.parametrize("case", [(2600, 38, 64, 0.0, 1, 256, 300), (2600, 30, 64, 0.0, 1, 256, 300), (2048, 33, 96, 0.05, 2, 200, 0),
+                                  (2048, 26, 96, 0.05, 2, 200, 0), (1300, 14, 160, 0.3, 3, 256, 0), (1300, 9, 160, 0.3, 3, 256, 0),
+                                  (900, 13, 192, 0.0, 4, 256, 0), (900, 9, 192, 0.0, 4, 256, 0), (1000, 10, 224, 0.0, 5, 256, 0),
+                                  (1000, 7, 224, 0.0, 5, 256, 0), (700, 13, 256, 0.0, 6, 272, 0), (700, 9, 256, 0.0, 6, 272, 0)],
+                         ids=lambda c: "N%d_d%d_C%d" % (c[0], c[1], c[2]))
+def test_mp_edge_forward_on_both_sides_of_the_line_by_edges(cabi, case):
+    """Nodes enough for that kernel, edges just enough and not enough: its heavy node, tables and isolated nodes again."""
+    test_mp_edge_forward_many_nodes(cabi, case)
+
+
+def test_mp_edge_forward_sorts_the_nodes_of_a_workgroup_in_batches(cabi):
+    """40 000 receiver nodes with 13 edges each at 256 channels: 5 000 nodes per workgroup, sorted 4 096 at a time.  Against
+    the kernel that takes harmonics and lengths, and the oracle on a sample of nodes."""
+    nnodes, C = 40000, 256
+    snd, rcv, X, vec, knots, coeffs, h = _edge_case(nnodes, 13, C, 0.1, 9)
+    assert rcv.numel() > 11 * nnodes
+    d = lambda t: t.float().cuda()
+    fo = cabi.first_occurences(rcv.cuda(), nnodes)
+    out = cabi.mp_edge_forward(d(X), d(vec), d(knots), d(coeffs), h, 5.0, snd.cuda(), fo, nnodes)
+    other = cabi.mp_spline_forward(d(X), cabi.sh_forward(d(vec)), d(vec).norm(dim=1), d(knots), d(coeffs), h, 5.0, snd.cuda(), fo, nnodes)
+    # fp32 rounding of length, harmonics and about a dozen terms per sum, against the largest component
+    assert float((out - other).abs().max()) <= 1e-5 * float(other.abs().max())
+    nodes = torch.arange(0, nnodes, 997)
+    pick = torch.isin(rcv.long(), nodes)
+    live = pick & (vec.norm(dim=1).float() <= 5.0) & (snd >= 0) & (snd < nnodes)
+    Rv = O.spline_eval(vec[live].norm(dim=1), knots, coeffs, h, 5.0).view(-1, 4, C)
+    ref = O.mp_forward(X, O.spherical_harmonics(vec[live]), Rv, snd[live], rcv[live], nnodes)
+    close(out[nodes.cuda()], ref[nodes], 2e-5, 2e-6)
+
+
 def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi):
     """40 000 receiver nodes at 256 channels: a workgroup of the LDS-table kernel sorts and serves its nodes in more than
     one batch.  Checked against the kernel that takes harmonics and lengths (same radial table, same per-edge
