@@ -525,15 +525,24 @@ class OptimizedInvariantMACE(torch.nn.Module):
                                            lambda: (node_attrs.detach().float(), node_attrs.detach().argmax(dim=-1).int()))
         return e0_per_head, node_feats_up, node_attrs32, atom_types
 
-    def _species_in_order(self, node_attrs: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
-        """Rows `perm` of node_attrs, carrying the rows of what `_species_of` knows about it (an MD code keeps its species
-        through many lists: gathered, not evaluated again)."""
-        known = self._species_of(node_attrs)
+    def _species_in_order(self, node_attrs: torch.Tensor, perm: torch.Tensor, inverse: torch.Tensor) -> torch.Tensor:
+        """Rows `perm` of node_attrs (`inverse`: where each row went).  The species of an MD code outlive its lists: what
+        `_species_of` knows about the rows in the order of the list before is taken over, not evaluated again.  node_attrs
+        keeps the copy of its latest list alone, so species that come with a list of their own cost one evaluation and
+        no second set of features."""
         out = node_attrs.detach().index_select(0, perm)
-        e0_per_head, node_feats_up, node_attrs32, atom_types = (t.index_select(0, perm) for t in known)
-        tag = (out._version, out.data_ptr())
-        out.__dict__["_cm_species_only"] = (self._weights_token, tag + (0,), (e0_per_head, node_feats_up))
-        out.__dict__["_cm_species"] = (tag + (None,), (node_attrs32, atom_types))
+        tag = (node_attrs._version, node_attrs.data_ptr())
+        before = node_attrs.__dict__.get("_cm_species_ordered")
+        if before is not None and before[0] == tag:
+            _, ordered, its_inverse = before
+            known = ordered.__dict__.get("_cm_species_only")
+            if known is not None and known[0] is self._weights_token:
+                rows = its_inverse.index_select(0, perm)
+                e0_per_head, node_feats_up, node_attrs32, atom_types = (t.index_select(0, rows) for t in self._species_of(ordered))
+                own = (out._version, out.data_ptr())
+                out.__dict__["_cm_species_only"] = (self._weights_token, own + (0,), (e0_per_head, node_feats_up))
+                out.__dict__["_cm_species"] = (own + (None,), (node_attrs32, atom_types))
+        node_attrs.__dict__["_cm_species_ordered"] = (tag, out, inverse)
         return out
 
     def forward(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,
@@ -567,7 +576,7 @@ class OptimizedInvariantMACE(torch.nn.Module):
             inner["batch"] = _cached_for(data["edge_index"], "_cm_spatial_batch", data["batch"],
                                          lambda: data["batch"].index_select(0, perm))
         inner["node_attrs"] = _cached_for(data["edge_index"], "_cm_spatial_attrs", data["node_attrs"],
-                                          lambda: self._species_in_order(data["node_attrs"], perm))
+                                          lambda: self._species_in_order(data["node_attrs"], perm, inverse))
         for name in ("shifts", "unit_shifts"):
             if name in data and (name == "shifts" or not direct):  # the integer images serve the strain path alone
                 t = data[name]

@@ -240,3 +240,44 @@ def test_per_model_cache_survives_a_recycled_token_id():
     loaded = torch.load(buf, weights_only=False)
     assert torch.equal(loaded, owner) and len(loaded.__dict__.get("_slot", {})) == 0
     assert len(copy.deepcopy(owner).__dict__["_slot"]) == 0
+
+
+def test_species_of_a_reordered_list_are_evaluated_once_and_kept_once():
+    """What the model knows about the species (reference energies, first features) in the order of a list: one evaluation
+    for a species tensor, in the order of its first list; later lists of the same tensor take the rows over, and the
+    caller's tensor gets no second copy in its own order."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    model = OptimizedInvariantMACE(SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7), seed=0), device="cpu")
+    evaluations = []
+    up = model.interactions[0].linear_up
+    model.interactions[0].linear_up.register_forward_hook(lambda *a: evaluations.append(1))
+    g = torch.Generator().manual_seed(0)
+
+    def order(n=50):
+        perm = torch.randperm(n, generator=g)
+        inverse = torch.empty_like(perm)
+        inverse[perm] = torch.arange(n)
+        return perm.int(), inverse.int()
+
+    def check(attrs, ordered, perm):
+        assert torch.equal(ordered, attrs[perm.long()])
+        known = model._species_of(ordered)
+        want_up = torch.matmul(model.node_embedding(ordered.double()).float(), up.weights)
+        assert torch.equal(known[0], model.atomic_energies_fn(ordered.double())) and torch.equal(known[1], want_up)
+        assert torch.equal(known[2], ordered.float()) and torch.equal(known[3], ordered.argmax(dim=-1).int())
+
+    attrs = torch.nn.functional.one_hot(torch.randint(0, 3, (50,), generator=g), 3).double()
+    for _ in range(3):  # three lists of one species tensor
+        perm, inverse = order()
+        check(attrs, model._species_in_order(attrs, perm, inverse), perm)
+    assert len(evaluations) == 1 and "_cm_species_only" not in attrs.__dict__
+    attrs[:10] = attrs[10:20].clone()  # another composition in the same tensor
+    perm, inverse = order()
+    check(attrs, model._species_in_order(attrs, perm, inverse), perm)
+    assert len(evaluations) == 2
+    for _ in range(2):  # a tensor of its own for every list
+        own = attrs.clone()
+        perm, inverse = order()
+        check(own, model._species_in_order(own, perm, inverse), perm)
+    assert len(evaluations) == 4
