@@ -1244,7 +1244,11 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
         const int64_t row_at = (static_cast<int64_t>(sId[tb + 16 * rb + r16]) * COMP + m) * K + 16 * CB * wave + 4 * quarter;
         float *op = OUT + row_at;
         f4 res[CB];
-        if constexpr (COMP == 1) {  // may be OUT itself: every element is read and written by the same lane
+        if constexpr (COMP == 1) {
+          // May be OUT itself.  A place that stands in for the first row of its tile reads and writes that row from another
+          // lane of the same wave: all of them have the residual before any of them stores, as long as a tile is one block
+          // of rows (with a single weight group, which is how this form is launched, no row stands in for another tile's).
+          static_assert(RB == 1, "stand-in rows of a later block would read what the first block has stored");
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb) res[cb] = residual ? ld4(residual + row_at + 16 * cb) : zero4();
         }

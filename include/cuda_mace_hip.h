@@ -382,8 +382,8 @@ int cm_neighbour_list_count(const double *positions, const double *cell, int pbc
 int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnodes, int64_t max_cells,
                            const void *workspace, const int32_t *offsets, int64_t nedges, int32_t *edge_scratch,
                            int32_t *row_i, int32_t *row_j, int32_t *unit_shifts, cm_stream_t stream);
-/* The same list with everything the model reads of it, in two calls that launch three kernels and one (up to 32 768
- * atoms):
+/* The same list with everything the model reads of it, in two calls that launch three kernels (up to 4 096 atoms,
+ * seven beyond) and one:
  *   cm_neighbour_list_search: cm_neighbour_list_count, and max_degree int32 [1] = the most neighbours of one atom.
  *   cm_neighbour_list_graph: after the caller has read offsets[nnodes] = nedges and max_degree (at most
  *     cm_neighbour_list_graph_max_degree(); beyond that, cm_neighbour_list_fill), writes row_i, row_j int32 [nedges],

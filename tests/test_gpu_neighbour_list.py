@@ -99,8 +99,10 @@ GRAPH_CASES = {
     "box": (1000, 21.5, (1, 1, 1), 5.0),
     "dense": (900, 9.0, (1, 1, 1), 5.5),          # more than 512 neighbours: one wave per workgroup
     "denser": (400, 3.0, (0, 0, 0), 6.0),
-    "one_workgroup_most": (32768, 69.0, (1, 1, 1), 4.0),
-    "several_launches": (32769, 69.0, (1, 1, 0), 4.0),
+    "one_workgroup_most": (4096, 34.5, (1, 1, 1), 4.0),
+    "several_launches": (4097, 34.5, (1, 1, 0), 4.0),
+    "many_32768": (32768, 69.0, (1, 1, 1), 4.0),
+    "many_32769": (32769, 69.0, (1, 1, 0), 4.0),
 }
 
 
@@ -132,6 +134,36 @@ def test_graph_of_a_list(cabi, name):
     perm, off = cabi_mod.stable_key_sort(rj, n)
     assert torch.equal(g["offsets"], off)
     assert torch.equal(cabi_mod.symmetric_sender_view(g["row_i"], g["row_j"], g["unit_shifts"], g["first_occ"], n), perm)
+
+
+@pytest.mark.parametrize("satellites", [4097, 8191, 8192, 8300])
+def test_atom_with_thousands_of_neighbours(cabi, satellites):
+    """One atom in the middle of a shell of others, all within its cutoff: up to 8 192 neighbours the last pass keeps them in
+    LDS (128 KB), beyond that the list comes from count and fill.  Against the accept test evaluated in numpy."""
+    from cuda_mace import _cabi as cabi_mod
+    from cuda_mace.utils.neighbour_list import _search
+
+    rng = np.random.default_rng(satellites)
+    v = rng.normal(size=(satellites, 3))
+    pos = np.concatenate([v / np.linalg.norm(v, axis=1, keepdims=True) * rng.uniform(4.0, 4.9, (satellites, 1)), np.zeros((1, 3))])
+    n, cutoff = satellites + 1, 5.0
+    rows = []
+    for i in range(n):
+        d = pos - pos[i]
+        near = (d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2] < cutoff * cutoff
+        near[i] = False
+        rows.append(np.nonzero(near)[0])
+    assert len(rows[-1]) == satellites
+    want = np.stack([np.repeat(np.arange(n), [len(r) for r in rows]), np.concatenate(rows)])
+    p = torch.tensor(pos, dtype=torch.float64, device=DEV)
+    g = cabi_mod.neighbour_graph(p, None, (0, 0, 0), cutoff)
+    assert (g is None) == (satellites > 8192)
+    edge_index, shifts, unit_shifts = _search(p, cutoff, None, None)[:3]
+    assert np.array_equal(edge_index.cpu().numpy(), want)
+    assert float(shifts.abs().max()) == 0.0 and float(unit_shifts.abs().max()) == 0.0
+    if g is not None:
+        assert torch.equal(g["edge_index"], edge_index)
+        assert torch.equal(g["first_occ"], cabi_mod.first_occurences(g["row_i"], n))
 
 
 def test_full_size_box_equals_host_list_and_feeds_the_model(cabi):

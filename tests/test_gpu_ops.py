@@ -510,6 +510,22 @@ def test_scalar_linear_many_rows_wide(cabi, N, C):
     assert torch.equal(cabi.linear(d(X), WT, scale=1.0), out)
 
 
+@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 160), (8195, 192), (9007, 224), (12345, 256), (100007, 192)])
+def test_scalar_linear_many_rows_wide_in_place(cabi, N, C):
+    """The residual is the output itself, at node counts that leave the last tile of 16 rows short: the places behind its
+    rows stand in for its first row, which must receive its residual once."""
+    _say("scalar_linear_many_rows_wide_in_place", N, C)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    X, R = (torch.randn(N, C, generator=g, device=DEV) for _ in range(2))
+    W = torch.randn(C, C, generator=g, device=DEV)
+    want = cabi.linear(X, W, scale=1.0) + R
+    for _ in range(3):
+        inout = R.clone()
+        cabi._check(cabi.lib.cm_linear(X.data_ptr(), W.data_ptr(), None, None, N, 1, 0, 1, C, C, 1.0, None, inout.data_ptr(), inout.data_ptr(),
+                                       cabi._stream()))
+        assert torch.equal(inout, want)
+
+
 @pytest.mark.parametrize("N,C", [(25000, 128), (100000, 192), (5000, 96)])
 def test_linear_at_benchmark_sizes(cabi, N, C):
     """The channel mixing at the node and channel counts of benchmark configurations 4, 5 and 3, per-element weights
