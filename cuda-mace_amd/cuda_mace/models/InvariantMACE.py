@@ -360,10 +360,14 @@ class OptimizedInvariantMACE(torch.nn.Module):
         form, or several heads) runs the modules themselves in fp64 as the reference does.  fused_contraction=True runs the
         channel-mixing linear before each symmetric contraction and the contraction as one autograd node whose backward is
         a single kernel; False keeps the reference's separate Linear / ElementalLinear and SymmetricContraction ops.
-        native_step=True (with all three fusions on) hands an inference step without strain -- energy and forces of one
-        head -- to the library as ONE call that enqueues every kernel of the forward and of the backward chain itself
-        (no interpreter or autograd engine between the launches; same kernels, order and numbers as the autograd path,
-        which still serves training, virials / stress and compute_force=False).
+        native_step=True (with all three fusions on) hands an inference step -- energy, forces, virials and stress of one
+        head, or energies alone with gradients switched off -- to the library as ONE call that enqueues every kernel of the
+        forward and of the backward chain itself (no interpreter or autograd engine between the launches; same kernels, order
+        and numbers as the autograd path, which still serves training, compute_displacement and energies that the caller
+        differentiates).  Calls on several streams or from several threads share nothing that a call writes.  What is
+        derived from a list (orders, offsets, species rows) is kept on its tensors and made on the stream of the first
+        evaluation with it: another stream that evaluates the same list waits for that one first, as it would for the
+        list's own tensors.
         spatial_order_min_atoms: from this many atoms on, the model works on a relabelled copy of the graph in which
         atoms that are close in space have close indices (derived once per edge_index tensor), so that the gathers of
         sender rows hit in cache; outputs come back in the caller's order.  None switches the relabelling off."""
@@ -526,23 +530,28 @@ class OptimizedInvariantMACE(torch.nn.Module):
         return e0_per_head, node_feats_up, node_attrs32, atom_types
 
     def _species_in_order(self, node_attrs: torch.Tensor, perm: torch.Tensor, inverse: torch.Tensor) -> torch.Tensor:
-        """Rows `perm` of node_attrs (`inverse`: where each row went).  The species of an MD code outlive its lists: what
-        `_species_of` knows about the rows in the order of the list before is taken over, not evaluated again.  node_attrs
-        keeps the copy of its latest list alone, so species that come with a list of their own cost one evaluation and
-        no second set of features."""
+        """Rows `perm` of node_attrs (`inverse`: where each row went), with what `_species_of` knows about them where it is
+        known.  Species that come with a list of their own are evaluated in that list's order and nothing is kept in the
+        caller's; species that outlive their list, as an MD code's do, are taken back to the caller's order at the second
+        one and gathered from there at every later one."""
+
+        def put(owner, known):
+            tag = (owner._version, owner.data_ptr())
+            owner.__dict__["_cm_species_only"] = (self._weights_token, tag + (0,), known[:2])
+            owner.__dict__["_cm_species"] = (tag + (None,), known[2:])
+
+        def knows(owner):
+            hit = owner.__dict__.get("_cm_species_only")
+            return hit is not None and hit[0] is self._weights_token and hit[1] == (owner._version, owner.data_ptr(), 0)
+
         out = node_attrs.detach().index_select(0, perm)
-        tag = (node_attrs._version, node_attrs.data_ptr())
-        before = node_attrs.__dict__.get("_cm_species_ordered")
-        if before is not None and before[0] == tag:
-            _, ordered, its_inverse = before
-            known = ordered.__dict__.get("_cm_species_only")
-            if known is not None and known[0] is self._weights_token:
-                rows = its_inverse.index_select(0, perm)
-                e0_per_head, node_feats_up, node_attrs32, atom_types = (t.index_select(0, rows) for t in self._species_of(ordered))
-                own = (out._version, out.data_ptr())
-                out.__dict__["_cm_species_only"] = (self._weights_token, own + (0,), (e0_per_head, node_feats_up))
-                out.__dict__["_cm_species"] = (own + (None,), (node_attrs32, atom_types))
-        node_attrs.__dict__["_cm_species_ordered"] = (tag, out, inverse)
+        tag, first, its_inverse = node_attrs.__dict__.pop("_cm_species_first_list", (None, None, None))
+        if not knows(node_attrs) and tag == (node_attrs._version, node_attrs.data_ptr()) and knows(first):
+            put(node_attrs, tuple(t.index_select(0, its_inverse) for t in self._species_of(first)))
+        if knows(node_attrs):
+            put(out, tuple(t.index_select(0, perm) for t in self._species_of(node_attrs)))
+        else:
+            node_attrs.__dict__["_cm_species_first_list"] = ((node_attrs._version, node_attrs.data_ptr()), out, inverse)
         return out
 
     def forward(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,

@@ -242,10 +242,10 @@ def test_per_model_cache_survives_a_recycled_token_id():
     assert len(copy.deepcopy(owner).__dict__["_slot"]) == 0
 
 
-def test_species_of_a_reordered_list_are_evaluated_once_and_kept_once():
+def test_species_of_a_reordered_list_are_evaluated_once():
     """What the model knows about the species (reference energies, first features) in the order of a list: one evaluation
-    for a species tensor, in the order of its first list; later lists of the same tensor take the rows over, and the
-    caller's tensor gets no second copy in its own order."""
+    for a species tensor, in the order of its first list, and no second copy in the caller's order until a second list
+    comes; later lists gather."""
     from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
 
     model = OptimizedInvariantMACE(SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7), seed=0), device="cpu")
@@ -268,10 +268,10 @@ def test_species_of_a_reordered_list_are_evaluated_once_and_kept_once():
         assert torch.equal(known[2], ordered.float()) and torch.equal(known[3], ordered.argmax(dim=-1).int())
 
     attrs = torch.nn.functional.one_hot(torch.randint(0, 3, (50,), generator=g), 3).double()
-    for _ in range(3):  # three lists of one species tensor
+    for k in range(4):  # four lists of one species tensor
         perm, inverse = order()
         check(attrs, model._species_in_order(attrs, perm, inverse), perm)
-    assert len(evaluations) == 1 and "_cm_species_only" not in attrs.__dict__
+        assert len(evaluations) == 1 and ("_cm_species_only" in attrs.__dict__) == (k > 0)
     attrs[:10] = attrs[10:20].clone()  # another composition in the same tensor
     perm, inverse = order()
     check(attrs, model._species_in_order(attrs, perm, inverse), perm)
@@ -280,4 +280,5 @@ def test_species_of_a_reordered_list_are_evaluated_once_and_kept_once():
         own = attrs.clone()
         perm, inverse = order()
         check(own, model._species_in_order(own, perm, inverse), perm)
+        assert "_cm_species_only" not in own.__dict__
     assert len(evaluations) == 4
