@@ -78,13 +78,22 @@ def traffic_of(table, kernels):
     return None if any(p is None for p in parts) else sum(parts)
 
 
-def forward_kernel_name(C, N):
-    """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_spline.hip: cm_mp_edge_forward; the
+def forward_kernel_name(C, N, E):
+    """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_sliced.hip: sliced_forward_applies; the
     benchmark's spline table has 256 knots)."""
     share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
-    if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30:
+    enough = {32: 0, 64: 120000 - 10 * N, 96: max(60000, 11 * N), 128: max(60000, 11 * N), 160: max(10000, 8 * N),
+              224: max(10000, 8 * N)}.get(C, 11 * N)
+    if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
         return "mp_edge_forward_sliced_kernel"
     return "mp_spline_forward_kernel<%d,true>" % C
+
+
+def backward_kernel_name(C, N, E):
+    """Kernel that runs the fused backward edge pass without gX (csrc/mp_spline.hip: launch_edge)."""
+    if N >= 1024 and (C == 160 or (C == 192 and E >= 12 * N)):
+        return "mp_edge_backward_matrix_kernel<%d,true,false>" % C
+    return "mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C
 
 
 def linear_kernel_name(C, N):
@@ -169,9 +178,9 @@ def op_cases(torch, cabi, N, E, C, ne, rcv, snd, with_fused=True, with_node_ops=
         ]
     if with_fused:
         cases += [
-            ("mp_edge_forward (fused harmonics + spline)", forward_kernel_name(C, N), fwd_fb,
+            ("mp_edge_forward (fused harmonics + spline)", forward_kernel_name(C, N, E), fwd_fb,
              lambda: cabi.mp_edge_forward(X, vec, knots, coeffs, float(h), 5.0, snd, fo, N)),
-            ("mp_edge_backward grad_vectors (fused)", "mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C, bwd_fb,
+            ("mp_edge_backward grad_vectors (fused)", backward_kernel_name(C, N, E), bwd_fb,
              lambda: cabi.mp_edge_backward(X, vec, knots, coeffs, float(h), 5.0, G, snd, fo, None, None, N, need_gX=False)),
         ]
     if with_node_ops:
@@ -506,13 +515,14 @@ def main():
         sh_b, spline_b = 88 * E, 4 * (8 * E * C + E)  # harmonics backward, spline backward (each operand once)
         sh_f, spline_f = 76 * E, 4 * (E + 8 * E * C)  # harmonics forward, spline forward (each operand once)
         flops_fwd = 60 * E * C  # per edge and channel: the cubic of 4 degrees (12 FMA), 4 products, 16 accumulations
-        roofline = entry(forward_kernel_name(C, N), fwd_fb, t_fwd, launches_timed=launches(fwd_name),
+        roofline = entry(forward_kernel_name(C, N, E), fwd_fb, t_fwd, launches_timed=launches(fwd_name),
                          note="dominant kernel of the step by total time (two launches per step). Harmonics and radial "
                               "weights are evaluated in-kernel, so its own HBM operands are small; a workgroup keeps its "
                               "part of the spline table (two degrees x 16 channels, 130 KB) in LDS, so the coefficients "
                               "no longer travel through L1 (the kernel it replaces pulled 8 KB per edge from L2 and ran "
-                              "at 0.37-0.46 ms): bounded by vector-instruction issue (counter summary: ~90% of the SIMDs' "
-                              "four-cycle issue slots with two waves per SIMD, LDS half busy), not by HBM; see "
+                              "at 0.37-0.46 ms): bounded by vector-instruction issue (counter summary: 84% of the SIMDs' "
+                              "four-cycle issue slots at 1.8 waves per SIMD; plain multiply-adds issue at one per four "
+                              "cycles with two waves per SIMD and faster only with more; LDS half busy), not by HBM; see "
                               "roofline_other_kernels for the HBM-bound message passing with tabulated R[E,4,C] and for "
                               "the matrix-core linear",
                          binding_resource={
@@ -521,10 +531,10 @@ def main():
                              "flops": flops_fwd, "achieved_TFLOP/s": round(flops_fwd / (t_fwd * 1e-3) / 1e12, 1),
                              "peak_TFLOP/s": 157.3, "frac": round(flops_fwd / (t_fwd * 1e-3) / 1e12 / 157.3, 4),
                              "frac_of_unpacked_rate": round(flops_fwd / (t_fwd * 1e-3) / 1e12 / 78.65, 4),
-                             "meaning": "useful fp32 operations of the formulation against the vector peak (which counts "
-                                        "two-wide packed fp32 instructions; this library is built without them, so one "
-                                        "FMA per lane and four cycles, 78.65 TFLOP/s, is the rate its instructions can "
-                                        "reach: frac_of_unpacked_rate); the kernel issues "
+                             "meaning": "useful fp32 operations of the formulation against the vector peak, and against one "
+                                        "FMA per lane and four cycles, 78.65 TFLOP/s (frac_of_unpacked_rate), which is what "
+                                        "plain multiply-adds reach at the two waves per SIMD that this kernel's registers "
+                                        "allow (75 measured; 125 with eight waves); the kernel issues "
                                         "about 1.8 instructions per useful one (edge set-up per quad of lanes, broadcasts of "
                                         "the edge's values, addresses), and instructions with a cross-lane operand issue at "
                                         "less than half the rate of plain ones on this device"},
@@ -534,9 +544,10 @@ def main():
                              "meaning": "algorithmic HBM bytes of the three separate kernels this launch replaces (message "
                                         "passing with tabulated R, spline evaluation, harmonics) divided by this launch's "
                                         "duration"})
-        others = [entry("mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C, bwd_fb, t_bwd,
+        others = [entry(backward_kernel_name(C, N, E), bwd_fb, t_bwd,
                         launches_timed=launches(bwd_name),
-                        note="bounded by the delivery of the spline table from L2 (8 KB per edge at 128 channels): with a third fewer vector instructions it takes the same time")]
+                        note="bounded by the L1 path (17 loads of 16 bytes per lane and edge, texture-address units 79% busy) next to vector issue "
+                             "(81% of the four-cycle slots at 1.8 waves per SIMD); with all table rows in L1 it takes 15% less")]
         t_lin = avg_ms("linear")
         if t_lin:
             flops = 32 * N * C * C

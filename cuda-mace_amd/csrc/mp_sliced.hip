@@ -3,8 +3,7 @@
 //   out[n, m, c] = sum_{e -> n} X[sender[e], c] * Y_m(vec[e]) * R(|vec[e]|)[l(m), c]
 //
 // The kernels in mp_spline.hip give a wave one receiver node and all 16 components; per edge a lane fetches its 16
-// coefficient pieces of the cubic (8 KB per edge over the wave) from the table in L2, and that delivery is what bounds
-// them.  Here the work is cut the other way: a workgroup owns two degrees, (0, 3) or (1, 2) -- eight components either
+// coefficient pieces of the cubic (8 KB per edge over the wave) through L1, and that path is what bounds them.  Here the work is cut the other way: a workgroup owns two degrees, (0, 3) or (1, 2) -- eight components either
 // way, so every workgroup has the same work per edge -- and one slice of 16 channels, and the part of the table it
 // needs, (nknots - 1) x 4 coefficients x 2 degrees x 16 channels = 130 KB at 256 knots, stays in its LDS for the whole
 // launch.  One workgroup per compute unit; the workgroups of a (pair, slice) split the node range evenly.

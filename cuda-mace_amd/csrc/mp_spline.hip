@@ -575,10 +575,13 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
 // A row of 16 lanes serves one edge, four consecutive channels per lane, 64 channels per step; a group of four edges takes
 // C / 64 steps.  The matrix instructions of degree l + 1 are issued ahead of the arithmetic of degree l, and the pieces
 // of the table for degree l of the next step are requested as soon as this step's are used up (one operand set).
-// What it is bound by, and why not at every width: both edge passes fetch 17 pieces of 16 bytes per edge and four channels
-// from L2, and that delivery sets their pace.  This one issues a third fewer vector instructions (390 against 590 per four
-// edges at 128 channels), which changes little where the other one's lanes are full; it wins where they are not, at 160
-// channels (40 of 64 lanes) and at 192 (pieces of 12 bytes, which cost the path what 16 do).  12 000 nodes x 52 edges,
+// What it is bound by, and why not at every width: both edge passes load 17 pieces of 16 bytes per edge and four channels
+// through L1, and that path sets their pace (texture-address units busy 78 to 84 % of the time in either; with every edge on
+// one table interval and its own sender's row, so that all pieces hit in L1, 25 000 x 52 x 128 takes 385 us instead of 450
+// on the other kernel and 25 000 x 52 x 192 622 instead of 664 on this one: the way from L2 to L1 costs 6 to 15 %).  This one
+// issues a third fewer vector instructions (390 against 590 per four edges at 128 channels; 53 % of the four-cycle issue
+// slots at 192 against 80 % for the other at 128), which changes little where the other one's lanes are full; it wins where
+// they are not, at 160 channels (40 of 64 lanes) and at 192 (pieces of 12 bytes, which cost the path what 16 do).  12 000 nodes x 52 edges,
 // both kernels without / with gX and its sender pass, us: 64 channels 139 / 190 -> 137 / 194, 96 200 / 284 -> 228 / 321,
 // 128 238 / 323 -> 228 / 330, 160 387 / 527 -> 321 / 471, 192 369 / 509 -> 329 / 486, 224 427 / 595 -> 425 / 618, 256
 // 440 / 630 -> 442 / 650; 60 000 x 128 1 034 -> 1 055.
