@@ -366,8 +366,8 @@ class OptimizedInvariantMACE(torch.nn.Module):
         and numbers as the autograd path, which still serves training, compute_displacement and energies that the caller
         differentiates).  Calls on several streams or from several threads share nothing that a call writes.  What is
         derived from a list (orders, offsets, species rows) is kept on its tensors and made on the stream of the first
-        evaluation with it: another stream that evaluates the same list waits for that one first, as it would for the
-        list's own tensors.
+        evaluation with it (as the model's own tables are made at its first one): another stream that evaluates the same
+        list waits for that one first, as it would for the list's own tensors.
         spatial_order_min_atoms: from this many atoms on, the model works on a relabelled copy of the graph in which
         atoms that are close in space have close indices (derived once per edge_index tensor), so that the gathers of
         sender rows hit in cache; outputs come back in the caller's order.  None switches the relabelling off."""
