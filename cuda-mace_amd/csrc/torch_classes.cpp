@@ -10,6 +10,7 @@
 // valid only while the tensors they were derived from are alive and unmodified, so that they are built once per
 // neighbour list / model and never outlive their source.
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/custom_class.h>
 #include <torch/script.h>
 
@@ -94,6 +95,7 @@ struct Dep {
 struct Entry {
   std::vector<Dep> deps;
   std::vector<Tensor> value;
+  std::vector<c10::hip::HIPStream> streams;  // those that may use the value, the one that made it first
   bool valid() const {
     for (const Dep &d : deps) {
       if (d.impl.expired()) return false;
@@ -118,11 +120,15 @@ class DerivedCache {
         bool same = true;
         for (size_t i = 0; i < owners.size(); ++i)
           same = same && it->second.deps[i].impl.lock().get() == owners[i].unsafeGetTensorImpl();
-        if (same) return it->second.value;
+        if (same) {
+          share(it->second, owners[0]);
+          return it->second.value;
+        }
       }
     }
     Entry e;
     e.value = build();
+    if (owners[0].is_cuda()) e.streams.push_back(c10::hip::getCurrentHIPStream(owners[0].device().index()));
     for (const Tensor &t : owners)
       e.deps.push_back(Dep{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), t._version()});
     std::lock_guard<std::mutex> lock(mutex_);
@@ -135,6 +141,26 @@ class DerivedCache {
   }
 
  private:
+  // A value found on another stream than the one that made it: that stream waits for the maker, and the allocator is told
+  // that it reads the value.  Not while it is capturing: torch synchronises before a capture begins.
+  static void share(Entry &e, const Tensor &owner) {
+    if (e.streams.empty()) return;
+    const c10::hip::HIPStream here = c10::hip::getCurrentHIPStream(owner.device().index());
+    if (std::find(e.streams.begin(), e.streams.end(), here) != e.streams.end()) return;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(here.stream(), &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return;
+    hipEvent_t made = nullptr;
+    TORCH_CHECK(hipEventCreateWithFlags(&made, hipEventDisableTiming) == hipSuccess, "derived tensors: no event");
+    const bool ok = hipEventRecord(made, e.streams[0].stream()) == hipSuccess && hipStreamWaitEvent(here.stream(), made, 0) == hipSuccess;
+    (void)hipEventDestroy(made);
+    TORCH_CHECK(ok, "derived tensors: waiting for the stream that made them failed");
+    // the stream under the device type that this build of torch gives its tensors
+    const c10::Stream reader(c10::Stream::UNSAFE, owner.device(), here.id());
+    for (const Tensor &t : e.value)
+      if (t.is_cuda()) t.record_stream(reader);
+    e.streams.push_back(here);
+  }
+
   std::mutex mutex_;
   std::map<Key, Entry> map_;
 };

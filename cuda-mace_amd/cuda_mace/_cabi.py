@@ -141,6 +141,12 @@ def _stream() -> int:
 F32, F64, I32 = torch.float32, torch.float64, torch.int32
 
 
+def as_f64(t: torch.Tensor) -> torch.Tensor:
+    """The tensor's values as a contiguous fp64 tensor without a graph: itself where it is one."""
+    t = t.detach()
+    return t if t.dtype is F64 and t.is_contiguous() else t.to(F64).contiguous()
+
+
 def _typed(name: str, like: torch.Tensor):
     """(entry point, dtype) for the precision of `like`: `name` for fp32 tensors, `name`_f64 for fp64 ones (message
     passing, harmonics, spline and contraction exist in both, as in the reference)."""

@@ -23,7 +23,8 @@ from cuda_mace.ops.spherical_harmonics import SphericalHarmonics
 from cuda_mace.ops.symmetric_contraction import SymmetricContraction as CUDAContraction
 from cuda_mace import _cabi as cabi
 from cuda_mace.ops._autograd import (EdgeGeometryAutograd, LinearContractionAutograd, ReadoutEnergyAutograd, ScalarLinearAutograd,
-                                     _cached, _cached_for, _cached_per, groups_of, groups_of_one_hot, monomials_from_packed)
+                                     _cached, _cached_for, _cached_per, _found, _here, _leave, _leave_for, groups_of, groups_of_one_hot,
+                                     monomials_from_packed)
 from cuda_mace.utils.irreps import Instruction
 
 
@@ -110,7 +111,7 @@ def get_symmetric_displacement(positions, unit_shifts, cell, edge_index, num_gra
     return positions, shifts, displacement, cell
 
 
-_CONSTANTS: Dict[tuple, torch.Tensor] = {}
+_CONSTANTS: Dict[tuple, tuple] = {}
 
 
 def _constant(value: float, shape, dtype, device) -> torch.Tensor:
@@ -119,8 +120,9 @@ def _constant(value: float, shape, dtype, device) -> torch.Tensor:
     key = (float(value), tuple(shape), dtype, device)
     hit = _CONSTANTS.get(key)
     if hit is None:
-        hit = _CONSTANTS[key] = torch.full(tuple(shape), float(value), dtype=dtype, device=device)
-    return hit
+        made = torch.full(tuple(shape), float(value), dtype=dtype, device=device)
+        hit = _CONSTANTS[key] = (made, [_here(made)])
+    return _found(hit[0], *hit)
 
 
 def get_outputs(energy, positions, displacement, cell, training=False, compute_force=True, compute_virials=False,
@@ -364,10 +366,9 @@ class OptimizedInvariantMACE(torch.nn.Module):
         head, or energies alone with gradients switched off -- to the library as ONE call that enqueues every kernel of the
         forward and of the backward chain itself (no interpreter or autograd engine between the launches; same kernels, order
         and numbers as the autograd path, which still serves training, compute_displacement and energies that the caller
-        differentiates).  Calls on several streams or from several threads share nothing that a call writes.  What is
-        derived from a list (orders, offsets, species rows) is kept on its tensors and made on the stream of the first
-        evaluation with it (as the model's own tables are made at its first one): another stream that evaluates the same
-        list waits for that one first, as it would for the list's own tensors.
+        differentiates).  Calls on several streams or from several threads share nothing that a call writes; what is
+        derived from a list once (orders, offsets, species rows) is kept on its tensors, and a stream that finds it made by
+        another one waits for that stream.
         spatial_order_min_atoms: from this many atoms on, the model works on a relabelled copy of the graph in which
         atoms that are close in space have close indices (derived once per edge_index tensor), so that the gathers of
         sender rows hit in cache; outputs come back in the caller's order.  None switches the relabelling off."""
@@ -505,12 +506,11 @@ class OptimizedInvariantMACE(torch.nn.Module):
         receiver, sender = g["receiver"], g["sender"]
         new_edges = torch.stack((receiver, sender))
         # what the ops derive from a list is already there: leave it where they look it up
-        new_edges.__dict__["_cm_int32_rows"] = ((new_edges._version, new_edges.data_ptr(), None), (receiver, sender))
-        receiver.__dict__["_cm_csr"] = ((receiver._version, receiver.data_ptr(), n), g["first_occ"])
-        sender.__dict__["_cm_sender_view"] = ((sender._version, sender.data_ptr(), n), (g["sender_perm"], g["sender_offsets"]))
+        _leave(new_edges, "_cm_int32_rows", None, (receiver, sender))
+        _leave(receiver, "_cm_csr", n, g["first_occ"])
+        _leave(sender, "_cm_sender_view", n, (g["sender_perm"], g["sender_offsets"]))
         if data["shifts"].dtype == torch.float64:
-            t = data["shifts"]
-            edge_index.__dict__["_cm_spatial_shifts"] = (t, (edge_index._version, edge_index.data_ptr(), t._version), g["shifts"])
+            _leave_for(edge_index, "_cm_spatial_shifts", data["shifts"], g["shifts"])
         return g["node_perm"], g["node_inverse"], g["edge_perm"], new_edges
 
     def _species_of(self, node_attrs: torch.Tensor):
@@ -536,22 +536,22 @@ class OptimizedInvariantMACE(torch.nn.Module):
         one and gathered from there at every later one."""
 
         def put(owner, known):
-            tag = (owner._version, owner.data_ptr())
-            owner.__dict__["_cm_species_only"] = (self._weights_token, tag + (0,), known[:2])
-            owner.__dict__["_cm_species"] = (tag + (None,), known[2:])
+            _leave_for(owner, "_cm_species_only", self._weights_token, known[:2])
+            _leave(owner, "_cm_species", None, known[2:])
 
         def knows(owner):
             hit = owner.__dict__.get("_cm_species_only")
             return hit is not None and hit[0] is self._weights_token and hit[1] == (owner._version, owner.data_ptr(), 0)
 
         out = node_attrs.detach().index_select(0, perm)
-        tag, first, its_inverse = node_attrs.__dict__.pop("_cm_species_first_list", (None, None, None))
-        if not knows(node_attrs) and tag == (node_attrs._version, node_attrs.data_ptr()) and knows(first):
+        tag, before, streams = node_attrs.__dict__.pop("_cm_species_first_list", (None, None, None))
+        if not knows(node_attrs) and tag == (node_attrs._version, node_attrs.data_ptr()) and knows(before[0]):
+            first, its_inverse = _found(node_attrs, before, streams)
             put(node_attrs, tuple(t.index_select(0, its_inverse) for t in self._species_of(first)))
         if knows(node_attrs):
             put(out, tuple(t.index_select(0, perm) for t in self._species_of(node_attrs)))
         else:
-            node_attrs.__dict__["_cm_species_first_list"] = ((node_attrs._version, node_attrs.data_ptr()), out, inverse)
+            node_attrs.__dict__["_cm_species_first_list"] = ((node_attrs._version, node_attrs.data_ptr()), (out, inverse), [_here(out)])
         return out
 
     def forward(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,

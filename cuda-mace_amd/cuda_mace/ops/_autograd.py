@@ -52,14 +52,65 @@ def _traced(name: str):
     return decorate
 
 
+# A derived value is made on the stream of the call that first asks for it, and calls on other streams find it too: every
+# entry ends with the handles of the streams that may use its value, the one that made it first.
+def _here(owner: torch.Tensor, _raw=cabi._raw_stream or (lambda device: torch.cuda.current_stream(device).cuda_stream)) -> int:
+    device = owner.get_device()  # -1 on the host; this runs at every lookup
+    return _raw(device) if device >= 0 else 0
+
+
+def _tensors_of(val):
+    if isinstance(val, torch.Tensor):
+        yield val
+    elif isinstance(val, (tuple, list)):
+        for v in val:
+            yield from _tensors_of(v)
+    elif hasattr(val, "_keep"):
+        yield from _tensors_of(val._keep)
+
+
+def _share(val, streams, here: int) -> None:
+    """Lets the current stream (`here`) use `val`: it waits for the stream that made it, and the memory is not handed out
+    again while it still reads."""
+    if torch.cuda.is_current_stream_capturing():
+        return  # torch synchronises before a capture begins, and what a graph reads is kept by whoever keeps the graph
+    stream = torch.cuda.current_stream()
+    stream.wait_stream(torch.cuda.ExternalStream(streams[0]) if streams[0] else torch.cuda.default_stream())
+    for t in _tensors_of(val):
+        if t.is_cuda:
+            t.record_stream(stream)
+    streams.append(here)
+
+
+def _found(owner: torch.Tensor, val, streams):
+    """`val`, for a call on the current stream."""
+    here = _here(owner)
+    if here not in streams:
+        _share(val, streams, here)
+    return val
+
+
+def _leave(owner: torch.Tensor, slot: str, key, val) -> None:
+    """Puts a value that is known already where `_cached` looks it up."""
+    owner.__dict__[slot] = ((owner._version, owner.data_ptr(), key), val, [_here(owner)])
+
+
+def _leave_for(owner: torch.Tensor, slot: str, other, val) -> None:
+    """The same for `_cached_for`."""
+    owner.__dict__[slot] = (other, (owner._version, owner.data_ptr(), getattr(other, "_version", 0)), val, [_here(owner)])
+
+
 def _cached(owner: torch.Tensor, slot: str, key, build):
     """Value derived from `owner`, rebuilt when owner was modified in place or `key` differs."""
     tag = (owner._version, owner.data_ptr(), key)
     hit = owner.__dict__.get(slot)
     if hit is not None and hit[0] == tag:
+        here = _here(owner)
+        if here not in hit[2]:
+            _share(hit[1], hit[2], here)
         return hit[1]
     val = build()
-    owner.__dict__[slot] = (tag, val)
+    owner.__dict__[slot] = (tag, val, [_here(owner)])
     return val
 
 
@@ -70,9 +121,12 @@ def _cached_for(owner: torch.Tensor, slot: str, other, build):
     hit = owner.__dict__.get(slot)
     tag = (owner._version, owner.data_ptr(), getattr(other, "_version", 0))
     if hit is not None and hit[0] is other and hit[1] == tag:
+        here = _here(owner)
+        if here not in hit[3]:
+            _share(hit[2], hit[3], here)
         return hit[2]
     val = build()
-    owner.__dict__[slot] = (other, tag, val)
+    owner.__dict__[slot] = (other, tag, val, [_here(owner)])
     return val
 
 
@@ -100,9 +154,12 @@ def _cached_per(owner: torch.Tensor, slot: str, token, other, build):
     tag = (owner._version, owner.data_ptr(), getattr(other, "_version", 0))
     hit = table.get(token)
     if hit is not None and hit[0] is other and hit[1] == tag:
+        here = _here(owner)
+        if here not in hit[3]:
+            _share(hit[2], hit[3], here)
         return hit[2]
     val = build()
-    table[token] = (other, tag, val)
+    table[token] = (other, tag, val, [_here(owner)])
     return val
 
 

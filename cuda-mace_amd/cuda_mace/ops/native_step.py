@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from .. import _cabi as cabi
-from ._autograd import _cached, csr_of, groups_of, groups_of_one_hot, sender_view_of
+from ._autograd import _cached, _found, _here, csr_of, groups_of, groups_of_one_hot, sender_view_of
 
 _fp = ctypes.c_void_p
 
@@ -97,6 +97,7 @@ class NativeStep:
         w.hidden = int(model.readout_W2a.shape[1])
         w.act_cst, w.scale, w.shift = (float(v) for v in model.readout_constants)
         self.weights, self._keep, self.channels, self.nelements = w, keep, C, w.nelements
+        self._streams = [_here(keep[0])]
 
     def graph(self, edge_index, receiver, sender, node_attrs32, atom_types, ptr, X1, node_rows, node_e0=None,
               graph_e0=None) -> "_GraphHandle":
@@ -122,11 +123,11 @@ class NativeStep:
         g.node_weights = None
         F64 = torch.float64
         if node_e0 is not None:
-            node_e0 = node_e0.detach().to(F64).contiguous()
+            node_e0 = cabi.as_f64(node_e0)
             if node_e0.shape != (N,):
                 raise cabi.CudaMaceError("native step: node_e0 must be [%d]" % N)
         if graph_e0 is not None:
-            graph_e0 = graph_e0.detach().to(F64).contiguous()
+            graph_e0 = cabi.as_f64(graph_e0)
             if graph_e0.shape != (int(g.ngraphs),):
                 raise cabi.CudaMaceError("native step: graph_e0 must be [%d]" % int(g.ngraphs))
         g.node_e0 = _ptr(node_e0, F64, "node_e0") if node_e0 is not None else None
@@ -137,19 +138,18 @@ class NativeStep:
     def __call__(self, handle: "_GraphHandle", positions: torch.Tensor, shifts: torch.Tensor, want_feats: bool = True,
                  want_virials: bool = False, want_forces: bool = True) -> Dict[str, torch.Tensor]:
         """want_forces=False: the forward half alone (cm_mace_energy), "forces" and "virials" are None."""
+        _found(positions, self, self._streams)
         g = handle.struct
         N, E, C = int(g.nnodes), int(g.nedges), self.channels
         dev = positions.device
         F64 = torch.float64
-        pos64 = positions.detach().to(F64).contiguous()
-        sh64 = shifts.detach().to(F64).contiguous()
+        pos64, sh64 = cabi.as_f64(positions), cabi.as_f64(shifts)
         if pos64.shape != (N, 3) or sh64.shape != (E, 3):
             raise cabi.CudaMaceError("native step: positions must be [%d, 3] and shifts [%d, 3]" % (N, E))
         # Scratch memory of this call alone, from torch's allocator: it is handed out again only to later work of this
         # stream, so calls on other streams or from other threads (ctypes lets go of the interpreter lock) have theirs, and a
         # captured step has its own for as long as its graph lives.  A steady caller gets the same block every time.
-        need = (cabi.lib.cm_mace_step_workspace if want_forces else cabi.lib.cm_mace_energy_workspace)(N, E, C)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        ws = torch.empty(handle.workspace(want_forces, C), dtype=torch.uint8, device=dev)
         energy = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_energy = torch.empty(N, dtype=F64, device=dev)
         forces = torch.empty(N, 3, dtype=F64, device=dev) if want_forces else None
@@ -157,14 +157,14 @@ class NativeStep:
         virials = torch.empty(int(g.ngraphs), 3, 3, dtype=F64, device=dev) if want_virials else None
         total = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
         node_total = torch.empty(N, dtype=F64, device=dev)
+        feats_at, virials_at = (None if t is None else t.data_ptr() for t in (feats, virials))
         head = (ctypes.addressof(self.weights), ctypes.addressof(g), _ptr(pos64, F64, "positions"), _ptr(sh64, F64, "shifts"),
-                ws.data_ptr(), ws.numel(), _ptr(energy, F64, "energy"), _ptr(node_energy, F64, "node_energy"))
-        tail = (_ptr(total, F64, "total_energy"), _ptr(node_total, F64, "total_node_energy"), cabi._stream())
+                ws.data_ptr(), ws.numel(), energy.data_ptr(), node_energy.data_ptr())
+        tail = (total.data_ptr(), node_total.data_ptr(), cabi._stream())
         if want_forces:
-            cabi._check(cabi.lib.cm_mace_step(*head, _ptr(forces, F64, "forces"), _ptr(feats, F64, "node_feats"),
-                                              _ptr(virials, F64, "virials"), *tail))
+            cabi._check(cabi.lib.cm_mace_step(*head, forces.data_ptr(), feats_at, virials_at, *tail))
         else:
-            cabi._check(cabi.lib.cm_mace_energy(*head, _ptr(feats, F64, "node_feats"), *tail))
+            cabi._check(cabi.lib.cm_mace_energy(*head, feats_at, *tail))
         # energy / node_energy: the interaction part plus the handle's graph_e0 / node_e0, node_energy in the caller's
         # order (rows node_rows of the handle); interaction_node_energy: the interaction part alone, in list order
         return {"interaction_energy": energy, "interaction_node_energy": node_energy, "energy": total, "node_energy": node_total,
@@ -173,7 +173,15 @@ class NativeStep:
 
 class _GraphHandle:
     def __init__(self, struct, keep):
-        self.struct, self._keep = struct, keep
+        self.struct, self._keep, self._bytes = struct, keep, {}
+
+    def workspace(self, forces: bool, channels: int) -> int:
+        """Bytes of scratch memory of a call on this handle."""
+        nbytes = self._bytes.get((forces, channels))
+        if nbytes is None:
+            size = cabi.lib.cm_mace_step_workspace if forces else cabi.lib.cm_mace_energy_workspace
+            nbytes = self._bytes[forces, channels] = size(int(self.struct.nnodes), int(self.struct.nedges), channels)
+        return nbytes
 
     def with_node_weights(self, weights: torch.Tensor, graph_e0: Optional[torch.Tensor] = None) -> "_GraphHandle":
         """The same index structures with a weight per node energy (fp64 [nnodes], in the order of the lists): the step
@@ -183,10 +191,10 @@ class _GraphHandle:
             raise cabi.CudaMaceError("node weights must be [%d]" % int(self.struct.nnodes))
         g = _Graph()
         ctypes.memmove(ctypes.addressof(g), ctypes.addressof(self.struct), ctypes.sizeof(_Graph))
-        w = weights.detach().to(torch.float64).contiguous()
+        w = cabi.as_f64(weights)
         g.node_weights = _ptr(w, torch.float64, "node_weights")
         if graph_e0 is not None:
-            graph_e0 = graph_e0.detach().to(torch.float64).contiguous()
+            graph_e0 = cabi.as_f64(graph_e0)
             if graph_e0.shape != (int(g.ngraphs),):
                 raise cabi.CudaMaceError("graph_e0 must be [%d]" % int(g.ngraphs))
             g.graph_e0 = _ptr(graph_e0, torch.float64, "graph_e0")

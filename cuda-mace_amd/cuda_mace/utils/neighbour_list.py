@@ -19,6 +19,7 @@ from typing import Dict, Optional, Sequence, Tuple
 import torch
 
 from cuda_mace import _cabi as cabi
+from cuda_mace.ops._autograd import _leave
 
 
 def _cell_and_pbc(cell, pbc, device) -> Tuple[Optional[torch.Tensor], Tuple[bool, bool, bool]]:
@@ -57,7 +58,7 @@ def _search(positions: torch.Tensor, cutoff: float, pbc, cell, max_cells: int = 
     """(edge_index, shifts, unit_shifts, cell, batch or None, ptr or None)"""
     if not positions.is_cuda:
         raise cabi.CudaMaceError("get_neighborhood: positions must live on the GPU")
-    pos = positions.detach().double().contiguous()
+    pos = cabi.as_f64(positions)
     cell_t, pbc = _cell_and_pbc(cell, pbc, pos.device)
     n = pos.shape[0]
     batch = ptr = None
@@ -66,16 +67,16 @@ def _search(positions: torch.Tensor, cutoff: float, pbc, cell, max_cells: int = 
         # what the model derives from a list once is already there: leave it where it is looked up
         edge_index, shifts, unit_shifts, row_i, row_j = g["edge_index"], g["shifts"], g["unit_shifts"], g["row_i"], g["row_j"]
         batch, ptr, ptr32 = g["batch"], g["ptr"], g["ptr32"]
-        row_i.__dict__["_cm_csr"] = ((row_i._version, row_i.data_ptr(), n), g["first_occ"])
+        _leave(row_i, "_cm_csr", n, g["first_occ"])
         row_j.__dict__["_cm_symmetric_list"] = (row_i, unit_shifts, g["first_occ"], g["offsets"],
                                                 (row_j._version, row_i._version, unit_shifts._version))
-        ptr.__dict__["_cm_ptr32"] = ((ptr._version, ptr.data_ptr(), None), ptr32)
+        _leave(ptr, "_cm_ptr32", None, ptr32)
     else:  # an atom with thousands of neighbours
         row_i, row_j, S = cabi.neighbour_list(pos, cell_t, pbc, float(cutoff), max_cells)
         edge_index = torch.stack([row_i, row_j]).long()
         unit_shifts = S.double()
         shifts = shifts_from_unit_shifts(S, cell_t)
-    edge_index.__dict__["_cm_int32_rows"] = ((edge_index._version, edge_index.data_ptr(), None), (row_i, row_j))
+    _leave(edge_index, "_cm_int32_rows", None, (row_i, row_j))
     if cell_t is None:
         cell_t = torch.zeros(3, 3, dtype=torch.float64, device=pos.device)
     return edge_index, shifts, unit_shifts, cell_t, batch, ptr

@@ -731,3 +731,29 @@ def test_one_model_from_two_threads(cabi):
         t.join()
     torch.cuda.synchronize()
     assert not differing
+
+
+@pytest.mark.parametrize("atoms,relabel,native", [(300, False, True), (300, False, False), (900, True, True)])
+def test_a_list_first_seen_on_another_stream(cabi, atoms, relabel, native):
+    """A list evaluated for the first time on a stream that is held back, and right after on another one: the second
+    evaluation finds what the first derives from the list and waits for it.  Also a second model on the same list."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    kwargs = dict(spatial_order_min_atoms=0 if relabel else None, native_step=native)
+    models = [OptimizedInvariantMACE(SyntheticInvariantMACE(channels=64, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=50.0, seed=s),
+                                     device="cuda", **kwargs) for s in (2, 3)]
+    host = make_system(atoms, 4, seed=7, density=0.1)
+    want = [{k: m(to_device(host, "cuda"))[k].detach() for k in ("energy", "forces", "node_energy")} for m in models]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for _ in range(3):
+        data = to_device(host, "cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            torch.cuda._sleep(4_000_000)
+            a = models[0](dict(data))
+        with torch.cuda.stream(streams[1]):
+            b = models[0](dict(data))
+            c = models[1](dict(data))
+        torch.cuda.synchronize()
+        for k in want[0]:
+            assert torch.equal(a[k].detach(), want[0][k]) and torch.equal(b[k].detach(), want[0][k]) and torch.equal(c[k].detach(), want[1][k]), k

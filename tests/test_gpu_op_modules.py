@@ -186,3 +186,35 @@ def test_model_surgery_tool_against_a_callable_source_model(cabi, tmp_path, caps
     assert errs["energy"][1] <= 1e-5 * abs(energy), printed
     assert errs["forces"][1] <= 1e-4, printed
     assert torch.load(out_path, weights_only=False).orig_model is not None
+
+
+def test_index_structures_made_on_another_stream():
+    """Message passing and a contraction on index tensors that a held-back stream has seen first: the second stream waits for
+    what the first derives from them."""
+    from cuda_mace.ops import InvariantMessagePassingTP
+
+    g = torch.Generator(device="cuda").manual_seed(0)
+    N, E, C = 500, 9000, 64
+    tp = InvariantMessagePassingTP()
+    X, Y, R = (torch.randn(*s, device="cuda", generator=g) for s in ((N, C), (16, E), (E, 4, C)))
+    receiver = torch.randint(0, N, (E,), device="cuda", generator=g).sort().values.int()
+    sender = torch.randint(0, N, (E,), device="cuda", generator=g).int()
+
+    def run(rcv, snd):
+        x = X.clone().requires_grad_(True)
+        out = tp(x, Y, R, snd, rcv, N)
+        (gx,) = torch.autograd.grad([out], [x], [torch.ones_like(out)])
+        return out.detach(), gx
+
+    want = run(receiver, sender)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for _ in range(3):
+        rcv, snd = receiver.clone(), sender.clone()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            torch.cuda._sleep(4_000_000)
+            a = run(rcv, snd)
+        with torch.cuda.stream(streams[1]):
+            b = run(rcv, snd)
+        torch.cuda.synchronize()
+        assert all(torch.equal(p, w) and torch.equal(q, w) for p, q, w in zip(a, b, want))

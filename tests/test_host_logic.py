@@ -282,3 +282,42 @@ def test_species_of_a_reordered_list_are_evaluated_once():
         check(own, model._species_in_order(own, perm, inverse), perm)
         assert "_cm_species_only" not in own.__dict__
     assert len(evaluations) == 4
+
+
+def test_derived_values_are_shared_between_streams(monkeypatch):
+    """A value found on another stream than the one that made it: that stream joins once, with the value in hand, and the
+    maker never; a value made anew belongs to the stream that made it."""
+    from cuda_mace.ops import _autograd as A
+
+    stream, joined = [11], []
+    monkeypatch.setattr(A, "_here", lambda owner: stream[0])
+
+    def share(val, streams, here):
+        joined.append((val, streams[0], here))
+        streams.append(here)
+
+    monkeypatch.setattr(A, "_share", share)
+    class Token:
+        pass
+
+    owner, other, token = torch.arange(4), torch.zeros(2), Token()
+    lookups = (lambda: A._cached(owner, "_a", 1, lambda: "a"), lambda: A._cached_for(owner, "_b", other, lambda: "b"),
+               lambda: A._cached_per(owner, "_c", token, other, lambda: "c"))
+    for lookup, name in zip(lookups, "abc"):
+        stream[0] = 11
+        assert lookup() == name and lookup() == name and not joined
+        stream[0] = 22
+        assert lookup() == name and lookup() == name and joined == [(name, 11, 22)]
+        stream[0] = 11
+        assert lookup() == name and len(joined) == 1
+        joined.clear()
+    stream[0] = 33
+    owner.add_(1)  # every value is made again, here
+    for lookup in lookups:
+        lookup()
+    assert not joined
+    A._leave(owner, "_d", None, "d")
+    A._leave_for(owner, "_e", other, "e")
+    stream[0] = 44
+    assert A._cached(owner, "_d", None, lambda: "never built") == "d" and A._cached_for(owner, "_e", other, lambda: "never built") == "e"
+    assert joined == [("d", 33, 44), ("e", 33, 44)]

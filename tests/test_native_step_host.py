@@ -39,7 +39,7 @@ def _step(monkeypatch):
     monkeypatch.setattr(_cabi, "_stream", lambda: 0)
     monkeypatch.setattr(native_step, "_ptr", lambda t, dtype, name: None if t is None else t.data_ptr())
     step = native_step.NativeStep.__new__(native_step.NativeStep)
-    step.weights, step._keep, step.channels, step.nelements = native_step._Weights(), [], C, 4
+    step.weights, step._keep, step.channels, step.nelements, step._streams = native_step._Weights(), [], C, 4, [0]
     graph = native_step._Graph()
     graph.nnodes, graph.nedges, graph.ngraphs = N, E, 1
     handle = native_step._GraphHandle(graph, ())
