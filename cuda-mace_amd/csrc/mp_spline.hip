@@ -341,6 +341,12 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
     float *__restrict__ gY, float *__restrict__ g_r, float *__restrict__ gXe, int parts) {
   using K = Cfg<C>;
   using vec = typename K::vec;
+  // From edge vectors, the harmonic m = 0 is the constant 1: q_0 is the gradient row itself, and nothing needs the gradient
+  // of that harmonic, so its place in the reduction over the slot carries the radial sum (which had a reduction, a lane
+  // exchange through LDS and an array of its own next to the unused sixteenth dot product).  us, without / with gX and its
+  // sender pass: 25 000 x 52 x 128 445 / 635 -> 414 / 632, 12 000 x 52 x 96 196 / 268 -> 181 / 264, 12 000 x 52 x 256
+  // 430 / 596 -> 388 / 581, 11 000 x 10 x 64 42 / 55 -> 39 / 53.
+  constexpr bool kRadialInFirst = FROM_VEC && WANT_GY && WANT_GR;
   __shared__ __attribute__((aligned(16))) float sY[kChunk * 16];
   __shared__ int sS[kChunk];
   __shared__ int sIdx[kChunk];
@@ -479,9 +485,13 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
         const vec a = o.ca[L], b = o.cb[L], c = o.cc[L], d = o.cd[L];
         const vec rl = a + xr * (b + xr * (c + xr * d));
         vec q = zerov<vec>();
+        if constexpr (FROM_VEC && L == 0) {
+          q = g[0];
+        } else {
 #pragma unroll
-        for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) q += y[m] * g[m];
-        if constexpr (WANT_GY) {
+          for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) q += y[m] * g[m];
+        }
+        if constexpr (WANT_GY && !(kRadialInFirst && L == 0)) {
           const vec t = o.x * rl;
 #pragma unroll
           for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) p[m] = dotv(g[m], t);
@@ -494,7 +504,8 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
       per_l(std::integral_constant<int, 2>{});
       per_l(std::integral_constant<int, 3>{});
       float grv = 0.f;
-      if constexpr (WANT_GR) grv = hsumv(o.x * grq);
+      if constexpr (kRadialInFirst) p[0] = dotv(o.x, grq);
+      else if constexpr (WANT_GR) grv = hsumv(o.x * grq);
 
       if constexpr (WANT_GX) {
         // streamed out: 666 MB at the headline size, read once by the sender pass (measured 2 % on the whole step).
@@ -506,7 +517,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
       // Unconditional (the last edge of a slot fetches itself again): loads under a branch would make every later wait
       // assume that they were not issued, i.e. wait for all but the oldest few of them.
       fetch(next, j + K::EPW < nlive ? j + K::EPW : j);
-      if constexpr (WANT_GR) {
+      if constexpr (WANT_GR && !kRadialInFirst) {
         const float tot = slot_sum<K::SW>(grv);
         if (cl == 0) sGr[j] = tot;
       }
@@ -536,7 +547,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
 #pragma unroll
           for (int m = 0; m < 16; ++m) gy[m] = sGY[m * kChunk + lane];
           sh::vjp(d, gy, gin);
-          const float gr = sGr[lane];
+          const float gr = gy[0];  // kRadialInFirst
           float o0 = gin[0] + gr * d.y, o1 = gin[1] + gr * d.z, o2 = gin[2] + gr * d.x;
           if (g_r) {
             // g_r doubles as an optional [E, 3] addend in this variant (another layer's gradient of the same vectors);
