@@ -116,42 +116,81 @@ __device__ __forceinline__ float dpp_move(float v) {
 // lane bit 0 goes through a quad permutation with selects, and lane bit 1 (and bit 5 for 64-lane slots) is a plain
 // sum.  Every lane ends with the total for m = reduced_index16(cl) in p[0].
 //
-// SW == 16 / 8: the stages over lane bits 0 and 1 stay inside a quad and go through DPP; the rest through
-// ds_bpermute.  Result: m = bitrev4(cl) in p[0] (SW == 16), or the two totals m = bitrev3(cl) * 2 + {0, 1} in p[0], p[1].
+// SW == 16: the same two stages over lane bits 3 and 2, then lane bits 1 and 0 through quad permutations with selects: m = cl in
+// p[0].  SW == 8: lane bit 2 by masked DPP adds, then the quad; the two totals m = reduced_pair8(cl) + {0, 1} in p[0], p[1].
+// The stages over lane bits 3 and 2: four values from sixteen.
+__device__ __forceinline__ void halve_lane_bits_3_2(float (&p)[16]) {
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      // lane bit 2: lanes of banks 0 and 2 read four lanes up (rotate right by 12), banks 1 and 3 four lanes down
+      "v_add_f32_dpp %0, %0, %0 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %1, %1, %1 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %3, %3, %3 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %4, %4 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %1, %5, %5 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %6, %6 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %3, %7, %7 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "s_nop 0"  // with the wait state the compiler adds after the block: two before a lane-crossing read of %3
+      : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
+      : "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+}
+// The stage over lane bit 2 alone, eight values from sixteen: lanes of banks 0 and 2 read four lanes up (rotate right by 12), banks 1
+// and 3 four lanes down.
+__device__ __forceinline__ void halve_lane_bit2(float (&p)[16]) {
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %1, %1, %1 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %3, %3, %3 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %4, %4, %4 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %5, %5, %5 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %6, %6, %6 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %7, %7, %7 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %8, %8 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %1, %9, %9 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %10, %10 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %3, %11, %11 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %4, %12, %12 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %5, %13, %13 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %6, %14, %14 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %7, %15, %15 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
+      "s_nop 0"
+      : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
+      : "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+}
+// One halving stage inside a quad: lanes with `hi` keep p[N + k], the others p[k], plus the partner's.
+template <int CTRL, int N>
+__device__ __forceinline__ void halve_in_quad(float (&p)[16], bool hi) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float keep = hi ? p[N + k] : p[k];
+    const float send = hi ? p[k] : p[N + k];
+    p[k] = keep + dpp_move<CTRL>(send);
+  }
+}
 template <int SW>
 __device__ __forceinline__ void slot_reduce16(float (&p)[16], int cl) {
   static_assert(SW >= 8, "slot width");
   if constexpr (SW >= 32) {
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        // lane bit 2: lanes of banks 0 and 2 read four lanes up (rotate right by 12), banks 1 and 3 four lanes down
-        "v_add_f32_dpp %0, %0, %0 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %1, %1, %1 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %2, %2, %2 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %3, %3, %3 row_ror:12 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %0, %4, %4 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %1, %5, %5 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %2, %6, %6 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %3, %7, %7 row_ror:4 row_mask:0xf bank_mask:0xa\n\t"
-        "s_nop 0"  // with the wait state the compiler adds after the block: two before a lane-crossing read of %3
-        : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
-        : "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+    halve_lane_bits_3_2(p);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       // first result: row 0 of p[k] over row 0 of p[2+k]; second: row 1 of p[k] over row 1 of p[2+k]
@@ -169,41 +208,18 @@ __device__ __forceinline__ void slot_reduce16(float (&p)[16], int cl) {
     p[0] += dpp_move<0x4E>(p[0]);
     if constexpr (SW >= 64) p[0] += __shfl_xor(p[0], 32);
     return;
-  }
-  {
-    const bool hi = cl & 1;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float keep = hi ? p[8 + k] : p[k];
-      const float send = hi ? p[k] : p[8 + k];
-      p[k] = keep + dpp_move<0xB1>(send);
-    }
-  }
-  {
-    const bool hi = cl & 2;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float keep = hi ? p[4 + k] : p[k];
-      const float send = hi ? p[k] : p[4 + k];
-      p[k] = keep + dpp_move<0x4E>(send);
-    }
-  }
-  {
-    const bool hi = cl & 4;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const float keep = hi ? p[2 + k] : p[k];
-      const float send = hi ? p[k] : p[2 + k];
-      p[k] = keep + __shfl_xor(send, 4);
-    }
-  }
-  if constexpr (SW >= 16) {
-    const bool hi = cl & 8;
-    const float keep = hi ? p[1] : p[0];
-    const float send = hi ? p[0] : p[1];
-    p[0] = keep + __shfl_xor(send, 8);
+  } else if constexpr (SW == 16) {
+    halve_lane_bits_3_2(p);
+    halve_in_quad<0x4E, 2>(p, cl & 2);
+    halve_in_quad<0xB1, 1>(p, cl & 1);
+  } else {
+    halve_lane_bit2(p);
+    halve_in_quad<0x4E, 4>(p, cl & 2);
+    halve_in_quad<0xB1, 2>(p, cl & 1);
   }
 }
+// first of the two totals a lane of an eight-lane slot holds: lane bits 2, 1, 0 are bits 3, 2, 1 of m
+__device__ __forceinline__ int reduced_pair8(int cl) { return 2 * (cl & 7); }
 
 // Plain sum of one value over the SW lanes of a slot; every lane gets the total.  Inside a row of 16 lanes: quad sums,
 // then rotations by 4 and 8 (all DPP); across rows: ds_bpermute.
@@ -227,7 +243,7 @@ __device__ __forceinline__ float slot_sum(float v) {
 template <int SW>
 __device__ __forceinline__ int reduced_index16(int cl) {
   if constexpr (SW >= 32) return (cl & 12) | ((cl >> 3) & 2) | (cl & 1);  // lane bits 3, 2, 4, 0
-  return ((cl & 1) << 3) | ((cl & 2) << 1) | ((cl & 4) >> 1) | ((cl & 8) >> 3);
+  return cl & 15;
 }
 
 // Writes the reduced gY values of edge j into the LDS tile sGY[m][kChunk].
@@ -238,7 +254,7 @@ __device__ __forceinline__ void store_reduced16(const float (&p)[16], int cl, in
   } else if constexpr (SW == 16) {
     sGY[reduced_index16<SW>(cl) * kChunk + j] = p[0];
   } else {
-    const int m0 = (((cl & 1) << 2) | (cl & 2) | ((cl & 4) >> 2)) * 2;
+    const int m0 = reduced_pair8(cl);
     sGY[m0 * kChunk + j] = p[0];
     sGY[(m0 + 1) * kChunk + j] = p[1];
   }

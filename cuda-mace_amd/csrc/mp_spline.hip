@@ -156,7 +156,31 @@ __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const in
 }
 
 constexpr int kMatrixMinNodes = 1024;  // see launch_edge
-constexpr int kKnotsInLds = 512;  // knots the backward edge pass keeps in LDS (more are read from memory)
+constexpr int kKnotsInLds = 512;  // knots the backward edge pass keeps in LDS (more, or fewer than four, are read from memory)
+
+// A wave's copy of the knots on its way to LDS, four per lane and load (a load instruction occupies the L1 path for 16 cycles
+// whatever its width; one dword per lane took eight of them, as many as half an edge does).
+struct KnotCopy {
+  static constexpr int kLoads = kKnotsInLds / (4 * kWave);
+  typedef float Four __attribute__((ext_vector_type(4), aligned(4)));  // the caller's array may start at any float
+  Four v[kLoads];
+  __device__ __forceinline__ static bool applies(const Spline &sp) { return sp.nknots >= 4 && sp.nknots <= kKnotsInLds; }
+  __device__ __forceinline__ static int at(const Spline &sp, int lane, int q) { return min(4 * (lane + kWave * q), sp.nknots - 4); }
+  __device__ __forceinline__ void request(const Spline &sp, int lane) {
+    if (!applies(sp)) return;
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q)
+      if (q == 0 || sp.nknots > 4 * kWave * q) v[q] = *reinterpret_cast<const Four *>(sp.knots + at(sp, lane, q));
+  }
+  __device__ __forceinline__ void store(const Spline &sp, int lane, float *lds) const {
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q)
+      if (q == 0 || sp.nknots > 4 * kWave * q) {
+        float *to = lds + at(sp, lane, q);
+        to[0] = v[q].x, to[1] = v[q].y, to[2] = v[q].z, to[3] = v[q].w;
+      }
+  }
+};
 
 // LDS of one wave's staged chunk: Y [kChunk][16], sender, knot interval, offset in it, position (floats / ints)
 constexpr int kStageBytes = kChunk * 64 + 4 * kChunk * 4;
@@ -334,8 +358,104 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::
 // -----------------------------------------------------------------------------------------------
 // backward, edge pass: gY, g_r and the per-edge contribution to gX
 // -----------------------------------------------------------------------------------------------
+// what an edge brings in: the sender's row piece and the 16 pieces of its knot interval
+template <class K>
+struct Operands {
+  typename K::vec x, ca[4], cb[4], cc[4], cd[4];
+  float xr;
+};
+
+template <int C, class K>
+__device__ __forceinline__ void fetch_operands(Operands<K> &o, const float *__restrict__ X, const float *__restrict__ tab, int s, int idx,
+                                               float xr, unsigned cla) {
+  o.xr = xr;
+  o.x = K::ld(X + (static_cast<unsigned>(s) * C + unsigned(K::off(cla))));
+  const unsigned co = static_cast<unsigned>(idx) * (16u * C) + unsigned(K::off(cla));
+#pragma unroll
+  for (int L = 0; L < 4; ++L) {
+    // addressed from the middle of the interval's 16C-float row (offsets within +-8C floats: one address and
+    // immediate offsets, up to C = 128)
+    const float *mid = tab + (co + 8 * C);
+    o.ca[L] = K::ld(mid + (L * C - 8 * C));
+    o.cb[L] = K::ld(mid + (L * C - 4 * C));
+    o.cc[L] = K::ld(mid + L * C);
+    o.cd[L] = K::ld(mid + (L * C + 4 * C));
+  }
+}
+
+// A lane's part of one edge: p[m] = sum over its channels of X R_l(m) g_m, gxe = sum_l R_l q_l and grq = sum_l q_l dR_l/dr.
+// kConstantFirst: the harmonic m = 0 is the constant 1 and its gradient is not wanted (p[0] is left alone).
+template <class K, bool kConstantFirst, bool WANT_GY, bool WANT_GR, bool WANT_GX>
+__device__ __forceinline__ void edge_products(const Operands<K> &o, const float (&y)[16], const typename K::vec (&g)[16], float (&p)[16],
+                                              typename K::vec &gxe, typename K::vec &grq) {
+  using vec = typename K::vec;
+  const float xr = o.xr;
+  const float xr2 = 2.f * xr, xr3 = 3.f * xr * xr;
+  auto per_l = [&](auto lc) {
+    constexpr int L = decltype(lc)::value;
+    const vec a = o.ca[L], b = o.cb[L], c = o.cc[L], d = o.cd[L];
+    const vec rl = a + xr * (b + xr * (c + xr * d));
+    vec q = zerov<vec>();
+    if constexpr (kConstantFirst && L == 0) {
+      q = g[0];
+    } else {
+#pragma unroll
+      for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) q += y[m] * g[m];
+    }
+    if constexpr (WANT_GY && !(kConstantFirst && L == 0)) {
+      const vec t = o.x * rl;
+#pragma unroll
+      for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) p[m] = dotv(g[m], t);
+    }
+    if constexpr (WANT_GX) gxe += rl * q;
+    if constexpr (WANT_GR) grq += q * (b + xr2 * c + xr3 * d);  // q_l * dR_l/dr
+  };
+  per_l(std::integral_constant<int, 0>{});
+  per_l(std::integral_constant<int, 1>{});
+  per_l(std::integral_constant<int, 2>{});
+  per_l(std::integral_constant<int, 3>{});
+}
+
+// the 16 staged harmonics of edge j
+__device__ __forceinline__ void staged_harmonics(const float *sY, int j, float (&y)[16]) {
+  const f4 *yp = reinterpret_cast<const f4 *>(sY + j * 16);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f4 v = yp[q];
+    y[4 * q] = v.x, y[4 * q + 1] = v.y, y[4 * q + 2] = v.z, y[4 * q + 3] = v.w;
+  }
+}
+
+// Gradient with respect to the vector of edge e: harmonics Jacobian applied to the reduced sums sGY[m][k], plus the radial sum
+// (in the place of m = 0) along the direction.  addend: an optional [E, 3] array (another layer's gradient of the same
+// vectors) to write the sum with; formed from the rounded value, as a separate addition pass would form it.
+__device__ __forceinline__ void finish_vector_gradient(const float *vec, int64_t e, const float *sGY, int k, const float *addend, float *gvec) {
+  const float v0 = vec[3 * e + 0], v1 = vec[3 * e + 1], v2 = vec[3 * e + 2];
+  const sh::Direction d = sh::direction(v0, v1, v2);
+  float gy[16], gin[3];
+#pragma unroll
+  for (int m = 0; m < 16; ++m) gy[m] = sGY[m * kChunk + k];
+  sh::vjp(d, gy, gin);
+  const float gr = gy[0];
+  float o0 = gin[0] + gr * d.y, o1 = gin[1] + gr * d.z, o2 = gin[2] + gr * d.x;
+  if (addend) {
+    o0 = __fadd_rn(o0, addend[3 * e + 0]);
+    o1 = __fadd_rn(o1, addend[3 * e + 1]);
+    o2 = __fadd_rn(o2, addend[3 * e + 2]);
+  }
+  gvec[3 * e + 0] = o0;
+  gvec[3 * e + 1] = o1;
+  gvec[3 * e + 2] = o2;
+}
+
+// Up to 64 channels three waves per SIMD on one operand set (168 registers): a trip's chain of lane exchanges is as long there as
+// at 128 channels for half or a quarter of the arithmetic, and a third wave fills it (11 000 x 52 x 64 100.6 -> 95.8 us, 3 000 x
+// 52 x 64 31.2 -> 27.6, 11 000 x 10 x 32 27.8 -> 24.4).  From 96 on the L1 path is the limit (25 000 x 52 x 128 389 against 394).
+template <int C, bool FROM_VEC>
+constexpr bool kOneOperandSet = FROM_VEC && C <= 64;
+
 template <int C, bool FROM_VEC, bool WANT_GY, bool WANT_GR, bool WANT_GX>
-__global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_edge_kernel(
+__global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_BWD_WAVES)) void mp_spline_backward_edge_kernel(
     const float *__restrict__ X, const float *__restrict__ Y, Spline sp, const float *__restrict__ G,
     const int32_t *__restrict__ sender, const int32_t *__restrict__ first_occ, int nnodes, int64_t nedges,
     float *__restrict__ gY, float *__restrict__ g_r, float *__restrict__ gXe, int parts) {
@@ -347,12 +467,18 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
   // sender pass: 25 000 x 52 x 128 445 / 635 -> 414 / 632, 12 000 x 52 x 96 196 / 268 -> 181 / 264, 12 000 x 52 x 256
   // 430 / 596 -> 388 / 581, 11 000 x 10 x 64 42 / 55 -> 39 / 53.
   constexpr bool kRadialInFirst = FROM_VEC && WANT_GY && WANT_GR;
+  // Every slot needs all of the node's 16 rows: loaded row by row, each of the two, four or eight slots fetches them for itself,
+  // and 16 load instructions are as many as an edge per slot takes.  The rows are one piece of memory: fetched once, 16 bytes
+  // per lane, and handed out through LDS, they are C / 16 instructions.
+  constexpr bool kRowsThroughLds = FROM_VEC && K::EPW > 1;
   __shared__ __attribute__((aligned(16))) float sY[kChunk * 16];
   __shared__ int sS[kChunk];
   __shared__ int sIdx[kChunk];
   __shared__ float sXr[kChunk];
   __shared__ int sOrig[kChunk];
-  __shared__ float sGY[16 * kChunk];  // [m][edge]
+  // The node's gradient rows on their way into registers, then the reduced gY, [m][edge].
+  __shared__ __attribute__((aligned(16))) float sRows[kRowsThroughLds && 16 * C > 16 * kChunk ? 16 * C : 16 * kChunk];
+  float *const sGY = sRows;
   __shared__ float sGr[kChunk];
   // The knots, where there are at most kKnotsInLds of them: the staging looks one up per edge, and a lookup in memory is
   // waited for behind everything the wave has in flight (the gradient rows from HBM first of all).
@@ -366,10 +492,9 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
   const int cl = lane % K::SW;
   const bool active = cl < K::LPE;
   const unsigned cla = active ? cl : 0;  // lanes beyond the channel count read lane 0's addresses; their g is zero
-  const bool knots_in_lds = sp.nknots <= kKnotsInLds;
-  float knot[kKnotsInLds / kWave];
-#pragma unroll
-  for (int q = 0; q < kKnotsInLds / kWave; ++q) knot[q] = sp.knots[min(lane + kWave * q, sp.nknots - 1)];
+  const bool knots_in_lds = KnotCopy::applies(sp);
+  KnotCopy knots;
+  knots.request(sp, lane);
   __builtin_amdgcn_sched_barrier(0);
   int e0 = first_occ[node];
   int e1 = first_occ[nnodes + node];
@@ -394,16 +519,18 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
     __builtin_amdgcn_sched_barrier(0);
   }
   vec g[16];
-  {
+  f4 rows[kRowsThroughLds ? C / 16 : 1];
+  if constexpr (kRowsThroughLds) {
+    const float *gp = G + static_cast<int64_t>(node) * (16 * C) + 4 * lane;
+#pragma unroll
+    for (int q = 0; q < C / 16; ++q) rows[q] = ld4_stream(gp + 256 * q);
+  } else {
     const float *gp = G + static_cast<int64_t>(node) * (16 * C) + K::off(cl);
 #pragma unroll
     for (int m = 0; m < 16; ++m) g[m] = active ? K::ld_stream(gp + m * C) : zerov<vec>();  // read once
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (knots_in_lds) {
-#pragma unroll
-    for (int q = 0; q < kKnotsInLds / kWave; ++q) sKnots[lane + kWave * q] = knot[q];
-  }
+  if (knots_in_lds) knots.store(sp, lane, sKnots);
 
   // The first chunk is written out ahead of the loop over the others (most nodes have no others): at a loop's head the
   // compiler has to assume that the loads a previous iteration left in flight (a slot's last, unused look-ahead) are still
@@ -436,73 +563,30 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
     };
     const int nlive = stage_edges<FROM_VEC, FROM_VEC && decltype(first_chunk)::value>(
         Y, sender, sp, nnodes, nedges, cursor, e1, lane, sY, sS, sIdx, sXr, sOrig, dead, ahead, sKnots, knots_in_lds);
+    if constexpr (kRowsThroughLds && decltype(first_chunk)::value) {
+#pragma unroll
+      for (int q = 0; q < C / 16; ++q) st4(sRows + 4 * lane + 256 * q, rows[q]);
+    }
     wave_lds_fence();
+    if constexpr (kRowsThroughLds && decltype(first_chunk)::value) {
+#pragma unroll
+      for (int m = 0; m < 16; ++m) g[m] = active ? K::ld(sRows + m * C + K::off(cla)) : zerov<vec>();
+      wave_lds_fence();  // the rows' place is the reduced sums' from here on
+    }
     // Every lane of a slot takes part in the reductions, so the loop bound is slot-uniform; only live edges are staged.
     // The loop is rotated: the sender row and the 16 coefficient pieces of the NEXT edge are requested right after the
     // arithmetic of the current one, so they travel while the cross-lane reductions (a chain of dependent lane
     // exchanges) run.
     // Two operand sets used in turn (the loop body is written out twice), so that the set being loaded is never copied
-    // into the set being consumed.
-    struct Operands {
-      vec x, ca[4], cb[4], cc[4], cd[4];
-      float xr;
-    };
-    auto fetch = [&](Operands &o, int j) {
-      const int s = sS[j];
-      const int idx = sIdx[j];
-      o.xr = sXr[j];
-      o.x = K::ld(X + (static_cast<unsigned>(s) * C + unsigned(K::off(cla))));
-      const unsigned co = static_cast<unsigned>(idx) * (16u * C) + unsigned(K::off(cla));
-      const float *__restrict__ tab = sp.coeffs;
-#pragma unroll
-      for (int L = 0; L < 4; ++L) {
-        // addressed from the middle of the interval's 16C-float row (offsets within +-8C floats: one address and
-        // immediate offsets, up to C = 128)
-        const float *mid = tab + (co + 8 * C);
-        o.ca[L] = K::ld(mid + (L * C - 8 * C));
-        o.cb[L] = K::ld(mid + (L * C - 4 * C));
-        o.cc[L] = K::ld(mid + L * C);
-        o.cd[L] = K::ld(mid + (L * C + 4 * C));
-      }
-    };
-    auto edge = [&](const Operands &o, int j, Operands &next) {
+    // into the set being consumed; or one set (kOneOperandSet), whose values are used up when the next edge's are requested.
+    auto fetch = [&](Operands<K> &o, int j) { fetch_operands<C>(o, X, sp.coeffs, sS[j], sIdx[j], sXr[j], cla); };
+    auto edge = [&](Operands<K> &o, int j, Operands<K> &next) {
       float y[16];
-      {
-        const f4 *yp = reinterpret_cast<const f4 *>(sY + j * 16);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f4 v = yp[q];
-          y[4 * q] = v.x, y[4 * q + 1] = v.y, y[4 * q + 2] = v.z, y[4 * q + 3] = v.w;
-        }
-      }
-      const float xr = o.xr;
-      const float xr2 = 2.f * xr, xr3 = 3.f * xr * xr;
+      staged_harmonics(sY, j, y);
       float p[16];
       vec gxe = zerov<vec>();
       vec grq = zerov<vec>();
-      auto per_l = [&](auto lc) {
-        constexpr int L = decltype(lc)::value;
-        const vec a = o.ca[L], b = o.cb[L], c = o.cc[L], d = o.cd[L];
-        const vec rl = a + xr * (b + xr * (c + xr * d));
-        vec q = zerov<vec>();
-        if constexpr (FROM_VEC && L == 0) {
-          q = g[0];
-        } else {
-#pragma unroll
-          for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) q += y[m] * g[m];
-        }
-        if constexpr (WANT_GY && !(kRadialInFirst && L == 0)) {
-          const vec t = o.x * rl;
-#pragma unroll
-          for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) p[m] = dotv(g[m], t);
-        }
-        if constexpr (WANT_GX) gxe += rl * q;
-        if constexpr (WANT_GR) grq += q * (b + xr2 * c + xr3 * d);  // q_l * dR_l/dr
-      };
-      per_l(std::integral_constant<int, 0>{});
-      per_l(std::integral_constant<int, 1>{});
-      per_l(std::integral_constant<int, 2>{});
-      per_l(std::integral_constant<int, 3>{});
+      edge_products<K, FROM_VEC, WANT_GY, WANT_GR, WANT_GX>(o, y, g, p, gxe, grq);
       float grv = 0.f;
       if constexpr (kRadialInFirst) p[0] = dotv(o.x, grq);
       else if constexpr (WANT_GR) grv = hsumv(o.x * grq);
@@ -514,6 +598,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
         if (active) K::st_stream(gXe + static_cast<int64_t>(base + sOrig[j]) * C + K::off(cl), gxe);
         __builtin_amdgcn_sched_barrier(0);  // keeps the instruction scheduler from sinking the store below the loads
       }
+      if constexpr (kOneOperandSet<C, FROM_VEC>) __builtin_amdgcn_sched_barrier(0);  // no request before its landing registers are free
       // Unconditional (the last edge of a slot fetches itself again): loads under a branch would make every later wait
       // assume that they were not issued, i.e. wait for all but the oldest few of them.
       fetch(next, j + K::EPW < nlive ? j + K::EPW : j);
@@ -526,45 +611,34 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_spline_backward_
         store_reduced16<K::SW>(p, cl, j, sGY);
       }
     };
-    Operands opa, opb;
+    Operands<K> opa;
     if (slot < nlive) fetch(opa, slot);
-    for (int j = slot; j < nlive; j += 2 * K::EPW) {
-      edge(opa, j, opb);
-      if (j + K::EPW >= nlive) break;
-      edge(opb, j + K::EPW, opa);
+    if constexpr (kOneOperandSet<C, FROM_VEC>) {
+#pragma unroll 1
+      for (int j = slot; j < nlive; j += K::EPW) edge(opa, j, opa);
+    } else {
+      Operands<K> opb;
+      for (int j = slot; j < nlive; j += 2 * K::EPW) {
+        edge(opa, j, opb);
+        if (j + K::EPW >= nlive) break;
+        edge(opb, j + K::EPW, opa);
+      }
     }
     if constexpr (WANT_GY || WANT_GR) {
       wave_lds_fence();
       // lane k < nlive finishes the k-th staged edge
-      if (lane < nlive) {
-        const int64_t e = base + sOrig[lane];
+      int k = lane;
+      asm volatile("; addresses formed from here, not carried through the loops" : "+v"(k));
+      if (k < nlive) {
+        const int64_t e = base + sOrig[k];
         if constexpr (FROM_VEC) {
-          // gradient with respect to the edge vector: harmonics Jacobian applied to gY, plus g_r along the direction
-          // (gY doubles as the output pointer of the [E, 3] vector gradient in this variant)
-          const float v0 = sp.vec[3 * e + 0], v1 = sp.vec[3 * e + 1], v2 = sp.vec[3 * e + 2];
-          const sh::Direction d = sh::direction(v0, v1, v2);
-          float gy[16], gin[3];
-#pragma unroll
-          for (int m = 0; m < 16; ++m) gy[m] = sGY[m * kChunk + lane];
-          sh::vjp(d, gy, gin);
-          const float gr = gy[0];  // kRadialInFirst
-          float o0 = gin[0] + gr * d.y, o1 = gin[1] + gr * d.z, o2 = gin[2] + gr * d.x;
-          if (g_r) {
-            // g_r doubles as an optional [E, 3] addend in this variant (another layer's gradient of the same vectors);
-            // the sum is formed from the rounded value, as a separate addition pass would form it
-            o0 = __fadd_rn(o0, g_r[3 * e + 0]);
-            o1 = __fadd_rn(o1, g_r[3 * e + 1]);
-            o2 = __fadd_rn(o2, g_r[3 * e + 2]);
-          }
-          gY[3 * e + 0] = o0;
-          gY[3 * e + 1] = o1;
-          gY[3 * e + 2] = o2;
+          finish_vector_gradient(sp.vec, e, sGY, k, g_r, gY);  // gY is the [E, 3] output in this variant, g_r its addend
         } else {
           if constexpr (WANT_GY) {
 #pragma unroll
-            for (int m = 0; m < 16; ++m) gY[m * nedges + e] = sGY[m * kChunk + lane];
+            for (int m = 0; m < 16; ++m) gY[m * nedges + e] = sGY[m * kChunk + k];
           }
-          if constexpr (WANT_GR) g_r[e] = sGr[lane];
+          if constexpr (WANT_GR) g_r[e] = sGr[k];
         }
       }
     }
@@ -627,10 +701,9 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
   constexpr bool kHalf = C % 64 != 0;
   const bool twin = kHalf && cl >= 8;
   const auto step_offset = [&](int h) { return 64 * h - (twin && h == H - 1 ? 32 : 0); };
-  const bool knots_in_lds = sp.nknots <= kKnotsInLds;
-  float knot[kKnotsInLds / kWave];
-#pragma unroll
-  for (int q = 0; q < kKnotsInLds / kWave; ++q) knot[q] = sp.knots[min(lane + kWave * q, sp.nknots - 1)];
+  const bool knots_in_lds = KnotCopy::applies(sp);
+  KnotCopy knots;
+  knots.request(sp, lane);
   __builtin_amdgcn_sched_barrier(0);
   int e0 = first_occ[node];
   int e1 = first_occ[nnodes + node];
@@ -664,10 +737,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (knots_in_lds) {
-#pragma unroll
-    for (int q = 0; q < kKnotsInLds / kWave; ++q) sKnots[lane + kWave * q] = knot[q];
-  }
+  if (knots_in_lds) knots.store(sp, lane, sKnots);
 
   int cursor = e0;
   auto chunk = [&](auto first_chunk) {
