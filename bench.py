@@ -91,8 +91,8 @@ def forward_kernel_name(C, N, E):
 
 def backward_kernel_name(C, N, E):
     """Kernel that runs the fused backward edge pass without gX (csrc/mp_spline.hip: launch_edge)."""
-    if N >= 1024 and (C == 160 or (C == 192 and E >= 12 * N)):
-        return "mp_edge_backward_matrix_kernel<%d,true,false>" % C
+    if C in (160, 192, 224):
+        return "mp_edge_backward_steps_kernel<%d,true,false>" % C
     return "mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C
 
 

@@ -81,16 +81,13 @@ struct RawEdge {
   int s;
   float v0, v1, v2;
 };
-// GRADS (FROM_VEC only): instead of the 16 harmonics, sY receives kGradRow floats per edge, for every m >= 1 the harmonic
-// and its derivatives with respect to the three components of the direction.
-constexpr int kGradRow = 15 * 4;
-template <bool FROM_VEC, bool AHEAD = false, bool GRADS = false, class DeadFn>
+template <bool FROM_VEC, bool AHEAD = false, class DeadFn>
 __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const int32_t *__restrict__ sender, const Spline &sp,
                                            int nnodes, int64_t nedges, int &base, int e1, int lane, float *sY, int *sS,
                                            int *sIdx, float *sXr, int *sOrig, DeadFn dead,
                                            RawEdge ahead = RawEdge{-1, 0.f, 0.f, 0.f}, const float *lds_knots = nullptr,
                                            bool use_lds_knots = false) {
-  static_assert(FROM_VEC || (!AHEAD && !GRADS), "raw edges are handed in, and gradients staged, for the edge-vector variant only");
+  static_assert(FROM_VEC || !AHEAD, "raw edges are handed in for the edge-vector variant only");
   const int first = base;
   int nlive = 0;
   // one pass over up to kChunk raw edges; the first one is written out on its own where its raw edges are handed in, so
@@ -102,7 +99,6 @@ __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const in
     float y[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) y[m] = 0.f;
-    sh::Direction d{0.f, 0.f, 0.f, 0.f};
     if (lane < cnt) {
       const int64_t e = base + lane;
       if constexpr (FROM_VEC) {
@@ -113,8 +109,7 @@ __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const in
           s = sender[e], v0 = sp.vec[3 * e + 0], v1 = sp.vec[3 * e + 1], v2 = sp.vec[3 * e + 2];
         }
         locate(sp, edge_length(v0, v1, v2), idx, x, lds_knots, use_lds_knots);
-        d = sh::direction(v0, v1, v2);
-        if constexpr (!GRADS) sh::eval(d, y);
+        sh::eval(sh::direction(v0, v1, v2), y);
       } else {
         s = sender[e];
         locate(sp, sp.r[e], idx, x, lds_knots, use_lds_knots);
@@ -134,15 +129,9 @@ __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const in
       sIdx[pos] = idx;
       sXr[pos] = x;
       sOrig[pos] = base - first + lane;
-      if constexpr (GRADS) {
-        sh::each_with_gradient(d, [&](int m, float v, float dx, float dy, float dz) {
-          *reinterpret_cast<f4 *>(sY + pos * kGradRow + 4 * (m - 1)) = f4{v, dx, dy, dz};
-        });
-      } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<f4 *>(sY + pos * 16 + 4 * q) = f4{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
-      }
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f4 *>(sY + pos * 16 + 4 * q) = f4{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
     }
     dead(base, consumed, live_mask, lane < consumed && !live);
     nlive = min(kChunk, nlive + nlive_pass);
@@ -155,16 +144,16 @@ __device__ __forceinline__ int stage_edges(const float *__restrict__ Y, const in
   return nlive;
 }
 
-constexpr int kMatrixMinNodes = 1024;  // see launch_edge
 constexpr int kKnotsInLds = 512;  // knots the backward edge pass keeps in LDS (more, or fewer than four, are read from memory)
 
 // A wave's copy of the knots on its way to LDS, four per lane and load (a load instruction occupies the L1 path for 16 cycles
 // whatever its width; one dword per lane took eight of them, as many as half an edge does).
+template <int kMost = kKnotsInLds>
 struct KnotCopy {
-  static constexpr int kLoads = kKnotsInLds / (4 * kWave);
+  static constexpr int kLoads = kMost / (4 * kWave);
   typedef float Four __attribute__((ext_vector_type(4), aligned(4)));  // the caller's array may start at any float
   Four v[kLoads];
-  __device__ __forceinline__ static bool applies(const Spline &sp) { return sp.nknots >= 4 && sp.nknots <= kKnotsInLds; }
+  __device__ __forceinline__ static bool applies(const Spline &sp) { return sp.nknots >= 4 && sp.nknots <= kMost; }
   __device__ __forceinline__ static int at(const Spline &sp, int lane, int q) { return min(4 * (lane + kWave * q), sp.nknots - 4); }
   __device__ __forceinline__ void request(const Spline &sp, int lane) {
     if (!applies(sp)) return;
@@ -426,15 +415,13 @@ __device__ __forceinline__ void staged_harmonics(const float *sY, int j, float (
   }
 }
 
-// Gradient with respect to the vector of edge e: harmonics Jacobian applied to the reduced sums sGY[m][k], plus the radial sum
-// (in the place of m = 0) along the direction.  addend: an optional [E, 3] array (another layer's gradient of the same
+// Gradient with respect to the vector of edge e: harmonics Jacobian applied to the reduced sums gy, plus the radial sum (in the
+// place of m = 0) along the direction.  addend: an optional [E, 3] array (another layer's gradient of the same
 // vectors) to write the sum with; formed from the rounded value, as a separate addition pass would form it.
-__device__ __forceinline__ void finish_vector_gradient(const float *vec, int64_t e, const float *sGY, int k, const float *addend, float *gvec) {
+__device__ __forceinline__ void finish_vector_gradient(const float *vec, int64_t e, const float (&gy)[16], const float *addend, float *gvec) {
   const float v0 = vec[3 * e + 0], v1 = vec[3 * e + 1], v2 = vec[3 * e + 2];
   const sh::Direction d = sh::direction(v0, v1, v2);
-  float gy[16], gin[3];
-#pragma unroll
-  for (int m = 0; m < 16; ++m) gy[m] = sGY[m * kChunk + k];
+  float gin[3];
   sh::vjp(d, gy, gin);
   const float gr = gy[0];
   float o0 = gin[0] + gr * d.y, o1 = gin[1] + gr * d.z, o2 = gin[2] + gr * d.x;
@@ -492,8 +479,8 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
   const int cl = lane % K::SW;
   const bool active = cl < K::LPE;
   const unsigned cla = active ? cl : 0;  // lanes beyond the channel count read lane 0's addresses; their g is zero
-  const bool knots_in_lds = KnotCopy::applies(sp);
-  KnotCopy knots;
+  const bool knots_in_lds = KnotCopy<>::applies(sp);
+  KnotCopy<> knots;
   knots.request(sp, lane);
   __builtin_amdgcn_sched_barrier(0);
   int e0 = first_occ[node];
@@ -632,7 +619,10 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
       if (k < nlive) {
         const int64_t e = base + sOrig[k];
         if constexpr (FROM_VEC) {
-          finish_vector_gradient(sp.vec, e, sGY, k, g_r, gY);  // gY is the [E, 3] output in this variant, g_r its addend
+          float sums[16];
+#pragma unroll
+          for (int m = 0; m < 16; ++m) sums[m] = sGY[m * kChunk + k];
+          finish_vector_gradient(sp.vec, e, sums, g_r, gY);  // gY is the [E, 3] output in this variant, g_r its addend
         } else {
           if constexpr (WANT_GY) {
 #pragma unroll
@@ -648,61 +638,52 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
 }
 
 // -----------------------------------------------------------------------------------------------
-// backward, edge pass from edge vectors at 160 and 192 channels: the contractions over m on the matrix cores
+// backward, edge pass from edge vectors at 160, 192 and 224 channels: four edges side by side, the channels in steps of 64
 // -----------------------------------------------------------------------------------------------
-// With u the edge's direction, P_l = X R_l and q_l = sum_{m in l} Y_m g_m as above, the gradient with respect to u is
-//   dE/du_k = sum_{l, c} P_l[c] D_lk[c],   D_lk[c] = sum_{m in l} (dY_m/du_k) g_m[c],
-// so that q_l and the three D_lk are four sums over the same rows of g with coefficients that belong to the edge alone: a
-// product [4 outputs of each of 4 edges, m] x [m, channels] for v_mfma_f32_16x16x4_f32.  A lane receives the four outputs
-// of one edge and channel (rows 4 (lane / 16) .. + 3 of a column), which is what the sums over channels need next: four
-// numbers per edge to reduce instead of seventeen, and no multiply-add with g on the vector ALU.
+// In the kernel above an edge of 160, 192 or 224 channels takes a whole wave, and its 17 load instructions move 40 or 56 lanes of
+// 16 bytes or 64 of 12 where 64 of 16 cost the L1 path the same (16 cycles for any load of 8 to 16 bytes per lane).  Here a row of 16 lanes serves an edge, four channels per lane, a group
+// of four edges takes C / 64 steps of 17 full-width loads, and the sixteen sums of an edge go through one reduction
+// over 16 lanes instead of 64.  The node's gradient rows of a step would be 64 registers for each of the steps: they stay in
+// LDS, from where a degree's rows are read as the degree is worked on (all rows of lanes read the same 256 bytes, at a
+// quarter of what the same bytes cost through L1).  The table's pieces for degree l of the next step are requested as soon as
+// this step's are used up (one operand set).
 //
-// A row of 16 lanes serves one edge, four consecutive channels per lane, 64 channels per step; a group of four edges takes
-// C / 64 steps.  The matrix instructions of degree l + 1 are issued ahead of the arithmetic of degree l, and the pieces
-// of the table for degree l of the next step are requested as soon as this step's are used up (one operand set).
-// What it is bound by, and why not at every width: both edge passes load 17 pieces of 16 bytes per edge and four channels
-// through L1, and that path sets their pace (texture-address units busy 78 to 84 % of the time in either; with every edge on
-// one table interval and its own sender's row, so that all pieces hit in L1, 25 000 x 52 x 128 takes 385 us instead of 450
-// on the other kernel and 25 000 x 52 x 192 622 instead of 664 on this one: the way from L2 to L1 costs 6 to 15 %).  This one
-// issues a third fewer vector instructions (390 against 590 per four edges at 128 channels; 53 % of the four-cycle issue
-// slots at 192 against 80 % for the other at 128), which changes little where the other one's lanes are full; it wins where
-// they are not, at 160 channels (40 of 64 lanes) and at 192 (pieces of 12 bytes, which cost the path what 16 do).  12 000 nodes x 52 edges,
-// both kernels without / with gX and its sender pass, us: 64 channels 139 / 190 -> 137 / 194, 96 200 / 284 -> 228 / 321,
-// 128 238 / 323 -> 228 / 330, 160 387 / 527 -> 321 / 471, 192 369 / 509 -> 329 / 486, 224 427 / 595 -> 425 / 618, 256
-// 440 / 630 -> 442 / 650; 60 000 x 128 1 034 -> 1 055.
-// The rows m >= 1 fall into four blocks of four, 1-3 and 8, 4-7, 9-12, 13-15 and an empty place: the first one serves
-// degrees 1 and 2, with zeros in the other degree's places of A; the empty place holds zeros in B.
-__device__ __forceinline__ int row_of_block(int block, int place) {
-  return block == 0 ? (place == 3 ? 8 : 1 + place) : block == 1 ? 4 + place : block == 2 ? 9 + place : place == 3 ? 15 : 13 + place;
-}
-
+// The contractions over m stay on the vector ALU: the fp32 matrix instruction computes no faster than plain multiply-adds (32
+// cycles for 1 024 of them, 2.3 to 2.8 per 64) and takes the SIMD's time from them, and the kernel that had
+// q_l and the gradient with respect to the direction on it, with every product padded to four m, spent 640 cycles per four
+// edges and step there against the 370 of the sums here.  Against that kernel and, where it did not run, the one above, us
+// without / with gX and its sender pass: 192 channels 100 nodes x 52 11.8 / 19.6 -> 11.1 / 18.3, 1 100 56 / 80 -> 39 / 64,
+// 11 000 314 / 442 -> 276 / 414, 40 000 1 089 / 1 598 -> 1 003 / 1 522, 4 000 x 4 22.1 / 30.3 -> 22.3 / 30.5; 160 channels 100
+// 15.5 / 23.9 -> 11.1 / 18.5, 11 000 319 / 428 -> 262 / 381, 4 000 x 4 24.6 -> 20.4; 224 channels 1 000 40.5 / 53.6 -> 41.4 / 55.7,
+// 3 000 127 / 161 -> 112 / 147, 30 000 913 / 1 366 -> 909 / 1 358, 11 000 x 4 61.6 -> 61.2.  Not at the widths that fill the lanes
+// of the kernel above: 256 357 / 524 -> 359 / 535, 96 170 / 242 -> 176 / 247, 128 (25 000) 406 / 616 -> 399 / 612.
 template <int C, bool WANT_GV, bool WANT_GX>
-__global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_matrix_kernel(
+__global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_steps_kernel(
     const float *__restrict__ X, Spline sp, const float *__restrict__ G, const int32_t *__restrict__ sender,
     const int32_t *__restrict__ first_occ, int nnodes, int64_t nedges, float *__restrict__ gvec,
     const float *__restrict__ addend, float *__restrict__ gXe, int parts) {
   static_assert(C % 32 == 0, "channel count");
   constexpr int H = (C + 63) / 64;
-  __shared__ __attribute__((aligned(16))) float sA[kChunk * kGradRow];
-  __shared__ __attribute__((aligned(16))) float sG[kChunk * 4];  // per edge: g_r and the gradient with respect to u
-  __shared__ __attribute__((aligned(16))) float sG0[C];          // the node's gradient row m = 0
+  __shared__ __attribute__((aligned(16))) float sY[kChunk * 16];  // harmonics of an edge, then its reduced sums
+  __shared__ __attribute__((aligned(16))) float sRows[16 * C];    // the node's gradient rows
   __shared__ int sS[kChunk];
   __shared__ int sIdx[kChunk];
   __shared__ float sXr[kChunk];
   __shared__ int sOrig[kChunk];
-  __shared__ float sKnots[kKnotsInLds];
+  constexpr int kKnots = C == 224 ? 256 : kKnotsInLds;  // 160 KB hold eight waves' arrays at every width
+  __shared__ float sKnots[kKnots];
 
   const int node = parts == 1 ? blockIdx.x : blockIdx.x / parts;
   const int lane = threadIdx.x;
-  const int row = lane / 16;  // which edge of a group, and which of a block's four m
+  const int row = lane / 16;  // which edge of a group
   const int cl = lane % 16;
   // The last step of a channel count that is an odd multiple of 32 has work for half of a row's lanes; the others repeat
   // it with the sender's row taken as zero, which leaves them out of the sums over channels.
   constexpr bool kHalf = C % 64 != 0;
   const bool twin = kHalf && cl >= 8;
   const auto step_offset = [&](int h) { return 64 * h - (twin && h == H - 1 ? 32 : 0); };
-  const bool knots_in_lds = KnotCopy::applies(sp);
-  KnotCopy knots;
+  const bool knots_in_lds = KnotCopy<kKnots>::applies(sp);
+  KnotCopy<kKnots> knots;
   knots.request(sp, lane);
   __builtin_amdgcn_sched_barrier(0);
   int e0 = first_occ[node];
@@ -725,16 +706,11 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
     ahead.v0 = sp.vec[3 * e + 0], ahead.v1 = sp.vec[3 * e + 1], ahead.v2 = sp.vec[3 * e + 2];
     __builtin_amdgcn_sched_barrier(0);
   }
-  f4 g0 = zero4(), gb[H][4];
+  f4 rows[C / 16];
   {
-    const float *gp = G + static_cast<int64_t>(node) * (16 * C);
-    if (4 * lane < C) g0 = ld4_stream(gp + 4 * lane);
+    const float *gp = G + static_cast<int64_t>(node) * (16 * C) + 4 * lane;
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        gb[h][b] = b == 3 && row == 3 ? zero4() : ld4_stream(gp + row_of_block(b, row) * C + step_offset(h) + 4 * cl);
-    }
+    for (int q = 0; q < C / 16; ++q) rows[q] = ld4_stream(gp + 256 * q);
   }
   __builtin_amdgcn_sched_barrier(0);
   if (knots_in_lds) knots.store(sp, lane, sKnots);
@@ -750,14 +726,17 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
         for (int k = 0; k < 3; ++k) gvec[3 * e + k] = addend ? addend[3 * e + k] : 0.f;
       }
     };
-    const int nlive = stage_edges<true, decltype(first_chunk)::value, true>(nullptr, sender, sp, nnodes, nedges, cursor, e1, lane, sA, sS,
-                                                                           sIdx, sXr, sOrig, dead, ahead, sKnots, knots_in_lds);
-    if (decltype(first_chunk)::value && 4 * lane < C) *reinterpret_cast<f4 *>(sG0 + 4 * lane) = g0;
+    const int nlive = stage_edges<true, decltype(first_chunk)::value>(nullptr, sender, sp, nnodes, nedges, cursor, e1, lane, sY, sS, sIdx,
+                                                                     sXr, sOrig, dead, ahead, sKnots, knots_in_lds);
+    if constexpr (decltype(first_chunk)::value) {
+#pragma unroll
+      for (int q = 0; q < C / 16; ++q) st4(sRows + 4 * lane + 256 * q, rows[q]);
+    }
     wave_lds_fence();
     if (nlive == 0) return;
 
     f4 ca[4], cb[4], cc[4], cd[4], x, xnext;
-    float a[5], xr;
+    float xr;
     unsigned co, xo;  // element offsets of the lane's pieces of the edge's table row and of its sender's row
     const auto locate_group = [&](int s, unsigned &o_tab, unsigned &o_x, float &o_xr) {
       const int j = min(4 * s + row, nlive - 1);
@@ -772,15 +751,6 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
       cc[L] = ld4(mid + L * C);
       cd[L] = ld4(mid + (L * C + 4 * C));
     };
-    const auto coefficients = [&](int s) {
-      const float *ap = sA + min(4 * s + cl / 4, nlive - 1) * kGradRow + (cl & 3);
-      const float first = ap[4 * (row_of_block(0, row) - 1)];
-      a[0] = row < 3 ? first : 0.f;
-      a[1] = ap[4 * (row_of_block(1, row) - 1)];
-      a[2] = row < 3 ? 0.f : first;
-      a[3] = ap[4 * (row_of_block(2, row) - 1)];
-      a[4] = ap[4 * (row_of_block(3, row) - 1)];
-    };
     locate_group(0, co, xo, xr);
     // in the loop's order: the waits in the loop count from the end of whichever way leads into it
     x = ld4(X + (xo + step_offset(0)));
@@ -790,15 +760,18 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
       request(L, co + step_offset(0));
       __builtin_amdgcn_sched_barrier(0);
     }
-    coefficients(0);
 
     const int ngroups = (nlive + 3) / 4;
     for (int s = 0; s < ngroups; ++s) {
-      float gr = 0.f, ux = 0.f, uy = 0.f, uz = 0.f;
       unsigned co_next, xo_next;
       float xr_next;
       locate_group(min(s + 1, ngroups - 1), co_next, xo_next, xr_next);
-      const int orig = sOrig[min(4 * s + row, nlive - 1)];
+      const int j = min(4 * s + row, nlive - 1);
+      const int orig = sOrig[j];
+      float y[16], p[16];
+      staged_harmonics(sY, j, y);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) p[m] = 0.f;
       const float xr2 = 2.f * xr, xr3 = 3.f * xr * xr;
 #pragma unroll
       for (int h = 0; h < H; ++h) {
@@ -807,77 +780,55 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_ma
         const unsigned next_tab = (last ? co_next : co) + next_step;
         xnext = ld4(X + ((last ? xo_next : xo) + next_step));
         if (kHalf && last && twin) x = zero4();
-        f4 d[4][4];  // [degree][channel]: q, then the three D
-        const auto products = [&](auto lc) {
-          constexpr int L = decltype(lc)::value;
-          constexpr int a0 = L == 1 ? 0 : L == 2 ? 1 : 3, b0 = L == 1 ? 0 : L == 2 ? 1 : 2, b1 = L == 2 ? 0 : 3;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) d[L][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[a0], gb[h][b0][t], zero4(), 0, 0, 0);
-          if constexpr (L > 1) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) d[L][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[a0 + 1], gb[h][b1][t], d[L][t], 0, 0, 0);
-          }
-        };
+        const float *rows_of_step = sRows + step_offset(h) + 4 * cl;
         f4 gxe = zero4(), grq = zero4();
         const auto degree = [&](auto lc) {
           constexpr int L = decltype(lc)::value;
-          if constexpr (L < 3) products(std::integral_constant<int, L + 1>{});
+          f4 g[2 * L + 1];
+#pragma unroll
+          for (int m = 0; m < 2 * L + 1; ++m) g[m] = ld4(rows_of_step + (L * L + m) * C);
           const f4 ra = ca[L], rb = cb[L], rc = cc[L], rd = cd[L];
           const f4 rl = ra + xr * (rb + xr * (rc + xr * rd));
           const f4 dr = rb + xr2 * rc + xr3 * rd;
-          __builtin_amdgcn_sched_barrier(0);  // keeps the scheduler from collecting loads or matrix instructions
+          __builtin_amdgcn_sched_barrier(0);  // keeps the scheduler from collecting loads
           request(L, next_tab);
-          if constexpr (L == 0) {
-            const f4 q0 = *reinterpret_cast<const f4 *>(sG0 + step_offset(h) + 4 * cl);
-            if constexpr (WANT_GX) gxe += rl * q0;
-            if constexpr (WANT_GV) grq += q0 * dr;
-          } else {
-            const f4 p = x * rl;
-            f4 du = p[0] * d[L][0];  // a sum of its own per degree: one chain over everything loses a little accuracy
+          f4 q = g[0];
+          if constexpr (L > 0) {
+            q = y[L * L] * g[0];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              if constexpr (WANT_GX) gxe[t] += rl[t] * d[L][t][0];
-              if constexpr (!WANT_GV) continue;
-              grq[t] += d[L][t][0] * dr[t];
-              if (t > 0) du += p[t] * d[L][t];
+            for (int m = 1; m < 2 * L + 1; ++m) q += y[L * L + m] * g[m];
+            if constexpr (WANT_GV) {
+              const f4 t = x * rl;
+#pragma unroll
+              for (int m = 0; m < 2 * L + 1; ++m)
+                p[L * L + m] = fmaf(g[m].w, t.w, fmaf(g[m].z, t.z, fmaf(g[m].y, t.y, fmaf(g[m].x, t.x, p[L * L + m]))));
             }
-            if constexpr (WANT_GV) ux += du[1], uy += du[2], uz += du[3];
           }
+          if constexpr (WANT_GX) gxe += rl * q;
+          if constexpr (WANT_GV) grq += q * dr;
           __builtin_amdgcn_sched_barrier(0);
         };
         degree(std::integral_constant<int, 0>{});
         degree(std::integral_constant<int, 1>{});
         degree(std::integral_constant<int, 2>{});
         degree(std::integral_constant<int, 3>{});
-        if constexpr (WANT_GV) gr += hsum4(x * grq);
+        if constexpr (WANT_GV) p[0] += dot4(x, grq);  // the radial sum in the place of m = 0, as above
         // unconditional: rows of lanes beyond the last edge have worked on the last edge and store its values again
         if constexpr (WANT_GX) st4_stream(gXe + static_cast<int64_t>(base + orig) * C + step_offset(h) + 4 * cl, gxe);
         x = xnext;
       }
-      coefficients(min(s + 1, ngroups - 1));
       co = co_next, xo = xo_next, xr = xr_next;
       if constexpr (WANT_GV) {
-        gr = slot_sum<16>(gr), ux = slot_sum<16>(ux), uy = slot_sum<16>(uy), uz = slot_sum<16>(uz);
-        if (cl == 0) *reinterpret_cast<f4 *>(sG + 4 * (4 * s + row)) = f4{gr, ux, uy, uz};
+        slot_reduce16<16>(p, cl);
+        sY[j * 16 + reduced_index16<16>(cl)] = p[0];  // (a row beyond the last edge: the last edge's value again)
       }
     }
     if constexpr (!WANT_GV) return;
     wave_lds_fence();
     if (lane < nlive) {
-      const int64_t e = base + sOrig[lane];
-      const f4 sums = *reinterpret_cast<const f4 *>(sG + 4 * lane);
-      const sh::Direction u = sh::direction(sp.vec[3 * e + 0], sp.vec[3 * e + 1], sp.vec[3 * e + 2]);
-      float gin[3];
-      sh::project(u, sums.y, sums.z, sums.w, gin);
-      float o0 = gin[0] + sums.x * u.y, o1 = gin[1] + sums.x * u.z, o2 = gin[2] + sums.x * u.x;
-      if (addend) {
-        o0 = __fadd_rn(o0, addend[3 * e + 0]);
-        o1 = __fadd_rn(o1, addend[3 * e + 1]);
-        o2 = __fadd_rn(o2, addend[3 * e + 2]);
-      }
-      gvec[3 * e + 0] = o0;
-      gvec[3 * e + 1] = o1;
-      gvec[3 * e + 2] = o2;
+      float sums[16];
+      staged_harmonics(sY, lane, sums);
+      finish_vector_gradient(sp.vec, base + sOrig[lane], sums, addend, gvec);
     }
   };
   chunk(std::true_type{});
@@ -904,19 +855,13 @@ void launch_edge(const float *X, const float *Y, const Spline &sp, const float *
                  hipStream_t st) {
   const int parts = parts_for(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
-  // From 1 024 nodes on, a wave per SIMD: below, a node's chain of staging and first loads is what counts, and this kernel
-  // stages more per edge (300 x 192 without / with gX: 19.7 / 28.0 -> 20.7 / 30.3 us; 2 000 x 160: 86.5 / 117 -> 74.1 / 103).
-  // At 192 channels also from 12 edges per node on: 10 000 x 8 without / with gX 75.1 / 100.6 -> 75.1 / 106.0 us, 2 000 x 12
-  // 31.0 / 42.8 -> 27.1 / 39.0; at 160, 10 000 x 8 82.6 / 105.1 -> 78.7 / 102.3.
-  if constexpr (FROM_VEC && (C == 160 || C == 192)) {
-    if (nnodes >= kMatrixMinNodes && (C == 160 || nedges >= 12 * nnodes)) {
-      hipLaunchKernelGGL((mp_edge_backward_matrix_kernel<C, GY, GX>), grid, dim3(kWave), 0, st, X, sp, G, sender, first_occ,
-                         static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
-      return;
-    }
+  if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {  // at every size: see the kernel
+    hipLaunchKernelGGL((mp_edge_backward_steps_kernel<C, GY, GX>), grid, dim3(kWave), 0, st, X, sp, G, sender, first_occ,
+                       static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
+  } else {
+    hipLaunchKernelGGL((mp_spline_backward_edge_kernel<C, FROM_VEC, GY, GR, GX>), grid, dim3(kWave), 0, st, X, Y, sp, G, sender,
+                       first_occ, static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
   }
-  hipLaunchKernelGGL((mp_spline_backward_edge_kernel<C, FROM_VEC, GY, GR, GX>), grid, dim3(kWave), 0, st, X, Y, sp, G, sender,
-                     first_occ, static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
 }
 
 // gY / g_r: outputs of the Y-and-r variant; in the FROM_VEC variant gY is the [E, 3] vector gradient and g_r, when given,

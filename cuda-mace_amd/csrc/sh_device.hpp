@@ -77,32 +77,6 @@ __device__ __forceinline__ void eval(const DirectionT<T> &d, T (&Y)[16]) {
   Y[15] = kA * x * (x2 - T(3) * y2);
 }
 
-// For every m >= 1 in turn: store(m, Y_m, dY_m/dx, dY_m/dy, dY_m/dz), the derivatives with respect to the components of the
-// unit vector treated as free (what vjp sums up before the chain rule through the normalisation, `project`).
-template <typename T, class Store>
-__device__ __forceinline__ void each_with_gradient(const DirectionT<T> &d, Store store) {
-  using K = Const<T>;
-  constexpr T kS3 = K::kS3, kS5 = K::kS5, kS7 = K::kS7, kS15 = K::kS15, kS105 = K::kS105, kA = K::kA, kB = K::kB;
-  const T x = d.x, y = d.y, z = d.z;
-  const T x2 = x * x, y2 = y * y, z2 = z * z;
-  const T xy = x * y, yz = y * z, xz = x * z, x2my2 = x2 - y2, f = T(4) * z2 - x2 - y2, h = T(2) * z2 - x2 - y2;
-  store(1, kS3 * y, T(0), kS3, T(0));
-  store(2, kS3 * z, T(0), T(0), kS3);
-  store(3, kS3 * x, kS3, T(0), T(0));
-  store(4, kS15 * xy, kS15 * y, kS15 * x, T(0));
-  store(5, kS15 * yz, T(0), kS15 * z, kS15 * y);
-  store(6, T(0.5) * kS5 * h, -kS5 * x, -kS5 * y, T(2) * kS5 * z);
-  store(7, kS15 * xz, kS15 * z, T(0), kS15 * x);
-  store(8, T(0.5) * kS15 * x2my2, kS15 * x, -kS15 * y, T(0));
-  store(9, kA * y * (T(3) * x2 - y2), T(6) * kA * xy, T(3) * kA * x2my2, T(0));
-  store(10, kS105 * xy * z, kS105 * yz, kS105 * xz, kS105 * xy);
-  store(11, kB * y * f, T(-2) * kB * xy, kB * (f - T(2) * y2), T(8) * kB * yz);
-  store(12, T(0.5) * kS7 * z * (T(2) * z2 - T(3) * x2 - T(3) * y2), T(-3) * kS7 * xz, T(-3) * kS7 * yz, T(1.5) * kS7 * h);
-  store(13, kB * x * f, kB * (f - T(2) * x2), T(-2) * kB * xy, T(8) * kB * xz);
-  store(14, T(0.5) * kS105 * z * x2my2, kS105 * xz, -kS105 * yz, T(0.5) * kS105 * x2my2);
-  store(15, kA * x * (x2 - T(3) * y2), T(3) * kA * x2my2, T(-6) * kA * xy, T(0));
-}
-
 // Gradient with respect to the un-normalised input, in input axis order, from the gradient (sx, sy, sz) with respect to
 // the components of the unit vector treated as free: (I - v v^T) / |in|.
 template <typename T>
