@@ -5,7 +5,7 @@
 // The kernels in mp_spline.hip give a wave one receiver node and all 16 components; per edge a lane fetches its 16
 // coefficient pieces of the cubic (8 KB per edge over the wave) through L1, and that path is what bounds them.  Here the work is cut the other way: a workgroup owns two degrees, (0, 3) or (1, 2) -- eight components either
 // way, so every workgroup has the same work per edge -- and one slice of 16 channels, and the part of the table it
-// needs, (nknots - 1) x 4 coefficients x 2 degrees x 16 channels = 130 KB at 256 knots, stays in its LDS for the whole
+// needs, (nknots - 1) x 4 coefficients x 2 degrees x 16 channels = 130 KB at 256 knots (147 KB as it is laid out), stays in its LDS for the whole
 // launch.  One workgroup per compute unit; the workgroups of a (pair, slice) split the node range evenly.
 //
 // Inside a workgroup a quad of four lanes serves one receiver node, four channels per lane, so a wave works on 16 nodes
@@ -17,14 +17,15 @@
 // byte offsets of an edge (table row, X row) come from lane j through a quad permutation of the DPP operand of the
 // address addition, once per step.
 //
-// LDS layout of the table slice: interval idx at 512 idx bytes; inside it the (a, b, c, d) of degree li (0 / 1: first /
-// second of the pair), channel 4 k + 2 p + b of the slice at 256 li + 64 (p + 2 b) + 16 k: the four lanes of a quad read
-// 64 contiguous bytes.  A 16-byte LDS read is served 16 lanes, i.e. four quads with unrelated intervals, at a time, and
-// the row stride is a multiple of the bank span, so quads that read the same piece position collide.  Which channel a
-// register stands for is a matter of addresses only (which 8 bytes of the X row land in it, which pieces are read for
-// it, where its sums are stored), so the quads at odd places take their two channel pairs in the other order: an odd
-// and an even quad never touch the same banks, two even (or two odd) ones do (a two-way conflict; avoiding it as well
-// would need X loads of four bytes).
+// LDS layout of the table slice: interval idx at 576 idx bytes; inside it the (a, b, c, d) of degree li (0 / 1: first / second of
+// the pair), channel 4 k + d of the slice at 256 li + 64 d + 16 k: the four lanes of a quad read 64 contiguous bytes.  A 16-byte
+// LDS read is served 16 lanes, i.e. four quads with unrelated intervals, at a time, and takes as many cycles as quads meet
+// in a quarter of the banks.  With rows a multiple of the bank span apart all four meet; at 576 bytes the quarter is (d +
+// idx) mod 4, and 2.1 meet on average.  Two orders of the channels for quads at odd and even places hold it to two, with X
+// rows in two 8-byte loads (which cost the L1 path twice what one of 16 bytes does) or with exchanges in registers, and four
+// orders to one: 25 000 x 52 x 128 257 us with two loads, 247 with exchanges, 236 with the rows 576 bytes apart (and the
+// table's pieces at constant offsets from one address); 96 channels 202 / 198 / 187, 192 (40 000) 618 / 600 / 582, 64 channels
+// with ten neighbours 29.3 / 28.4 / 26.3; four orders by exchanges 256 at 128 channels.
 //
 // Everything a step needs from memory is requested ahead, with registers that rotate in three sets so that nothing that
 // a load is still on its way into ever has to be copied (a copy would wait for the load): the sender and vector of a
@@ -34,10 +35,10 @@
 // shortens the life of the landing registers); scheduling barriers keep every request in its step.
 //
 // Receiver nodes differ in their edge counts and the 16 nodes of a wave advance together, so a workgroup sorts its nodes
-// (4 096 at a time) by their number of edge blocks and its waves draw 16 neighbours of that order at a time from a
+// (2 816 at a time) by their number of edge blocks and its waves draw 16 neighbours of that order at a time from a
 // counter in LDS.  Which wave serves a node does not change the node's result: a node's edges are summed in list order, in
 // two chains (even and odd places) that are added up at the end.  The second set of sums takes the last of the register
-// file (254 of 256) and no time; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
+// file (252 of 256) and no time; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
 // with one wave per node: 96 channels 2.68e-7 -> 2.54e-7 (2.70e-7), 128 2.73 -> 2.59 (2.74), 192 2.67 -> 2.52 (2.69), 256
 // 2.81 -> 2.67 (2.83).
 #include <algorithm>
@@ -51,8 +52,9 @@ namespace mp {
 namespace {
 
 constexpr int kSlThreads = 512;       // two waves per SIMD (three: 168 registers, equal at 25 000 nodes, 8 % slower at 50 000)
-constexpr int kSlMaxIntervals = 272;  // 136 KB of table (one row of it is the row of zeros)
-constexpr int kSlSub = 4096;          // nodes sorted at a time
+constexpr unsigned kSlRowBytes = 576;  // of a knot interval: 512 and a quarter of the bank span
+constexpr int kSlMaxIntervals = 272;   // 153 KB of table (one row of it is the row of zeros)
+constexpr int kSlSub = 2816;          // nodes sorted at a time: what LDS holds next to the largest table
 constexpr int kSlBins = 64;           // edge blocks per node that the sort tells apart
 // From six rounds of 16 nodes per workgroup on (5 121 nodes at 32 channels, 2 561 at 64, 1 281 at 128, 641 at 256); below
 // that some of its waves have none.  From there on the edges decide: a workgroup spends 4 us on its slice of the table, and
@@ -95,8 +97,6 @@ struct SlicedArgs {
   int nslices;  // C / 16
   int share;    // workgroups per (pair, slice)
 };
-
-typedef float f2 __attribute__((ext_vector_type(2)));
 
 // value of `v` in lane J of the reader's quad of four lanes (quad permutation of the DPP operand)
 template <int J>
@@ -158,42 +158,27 @@ struct Raw {  // what a lane loads for its edge of a block
   float v0, v1, v2;
 };
 
-// per-lane constants of the channel order (see the head of the file)
-struct LaneMap {
-  unsigned x[2];    // byte offset inside an X / out row of the lane's two channel pairs, in ITS order
-  unsigned lds[2];  // byte offset inside a table row of the piece (first degree, first channel) of each pair
-};
-
-// q[4 li + 2 p + b]: (a, b, c, d) of degree li, channel b of the lane's pair p
+// q[4 li + d]: (a, b, c, d) of degree li, channel d of the lane's four; `at`: the lane's place in the first row of the table
 template <int J>
-__device__ __forceinline__ void read_pieces(const char *tab, unsigned io, const LaneMap &m, f4 (&q)[8]) {
-  const unsigned row = quadu<J>(io);
+__device__ __forceinline__ void read_pieces(const char *at, unsigned io, f4 (&q)[8]) {
+  const char *row = at + quadu<J>(io);
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const char *at = tab + (row + m.lds[p]);
-    q[0 + 2 * p + 0] = *reinterpret_cast<const f4 *>(at);
-    q[0 + 2 * p + 1] = *reinterpret_cast<const f4 *>(at + 128);
-    q[4 + 2 * p + 0] = *reinterpret_cast<const f4 *>(at + 256);
-    q[4 + 2 * p + 1] = *reinterpret_cast<const f4 *>(at + 384);
-  }
+  for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const f4 *>(row + 64 * i);
 }
 
 template <int J>
-__device__ __forceinline__ void request_row(const float *__restrict__ X, unsigned xo, const LaneMap &m, f2 (&x)[2]) {
-  const unsigned row = quadu<J>(xo);
-  const char *base = reinterpret_cast<const char *>(X);
-  x[0] = *reinterpret_cast<const f2 *>(base + (row + m.x[0]));
-  x[1] = *reinterpret_cast<const f2 *>(base + (row + m.x[1]));
+__device__ __forceinline__ void request_row(const float *__restrict__ X, unsigned xo, unsigned place, f4 &x) {
+  x = *reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(X) + (quadu<J>(xo) + place));
 }
 
 // Steps J .. 3 of a block: `cur` is the block, xin[j] the X values of the edge of step j; as soon as step j has taken
 // them, the values of step j of the block after next (`fut`) are requested into xout[j].
 template <int P, int J>
 __device__ __forceinline__ void edge_step(const float *__restrict__ X, const char *tab, const Prepared &cur, const Gathered &all,
-                                          const Prepared &fut, const LaneMap &m, const f2 (&xin)[4][2], f2 (&xout)[4][2],
+                                          const Prepared &fut, unsigned place, const f4 (&xin)[4], f4 (&xout)[4],
                                           f4 (&q)[8], float (&acc)[2][8][4]) {
-  const float xs[4] = {xin[J][0].x, xin[J][0].y, xin[J][1].x, xin[J][1].y};
-  request_row<J>(X, fut.xo, m, xout[J]);
+  const f4 xs = xin[J];
+  request_row<J>(X, fut.xo, place, xout[J]);
   const float xr = all.xr[J];
   float y[8];
 #pragma unroll
@@ -207,13 +192,13 @@ __device__ __forceinline__ void edge_step(const float *__restrict__ X, const cha
       t[li][d] = xs[d] * fmaf(xr, fmaf(xr, fmaf(xr, c.w, c.z), c.y), c.x);
     }
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J + 1 < 4) read_pieces<J + 1>(tab, cur.io, m, q);
+  if constexpr (J + 1 < 4) read_pieces<J + 1>(tab, cur.io, q);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int d = 0; d < 4; ++d) acc[J & 1][i][d] = fmaf(y[i], t[i < Pair<P>::M0 ? 0 : 1][d], acc[J & 1][i][d]);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J + 1 < 4) edge_step<P, J + 1>(X, tab, cur, all, fut, m, xin, xout, q, acc);
+  if constexpr (J + 1 < 4) edge_step<P, J + 1>(X, tab, cur, all, fut, place, xin, xout, q, acc);
 }
 
 // the rounds of one sorted sub-range: nodes lo + order[0 .. cnt)
@@ -222,18 +207,12 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
                                            const unsigned short *sOrder, int *sNext, int lo, int cnt, int slice) {
   const int lane = threadIdx.x % kWave;
   const int k = lane & 3;         // place in the quad: channels 4 k .. 4 k + 3 of the slice
-  const int u = (lane >> 2) & 1;  // parity of the quad's place among the four that an LDS access serves together
   const int gw = lane >> 2;       // node of the wave's round
-  LaneMap m;
-#pragma unroll
-  for (int pr = 0; pr < 2; ++pr) {
-    m.x[pr] = static_cast<unsigned>(4 * (slice * 16 + 4 * k + 2 * (pr ^ u)));
-    m.lds[pr] = static_cast<unsigned>(64 * (pr ^ u) + 16 * k);
-  }
-  const char *tab = reinterpret_cast<const char *>(sTab);
+  const unsigned place = static_cast<unsigned>(4 * (slice * 16 + 4 * k));  // byte offset of the lane's channels in an X / out row
+  const char *tab = reinterpret_cast<const char *>(sTab) + 16 * k;
   const int C = p.C;
   const int last_edge = static_cast<int>(p.nedges) - 1;  // the launcher does not come here without edges
-  const unsigned zero_row = static_cast<unsigned>(p.nknots - 1) * 512u;
+  const unsigned zero_row = static_cast<unsigned>(p.nknots - 1) * kSlRowBytes;
   const float inv_width = 1.0f / p.r_width;
 
   for (;;) {
@@ -250,6 +229,7 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
       clamp_edge_range(e0, e1, p.nedges);
     }
     const int nblk = (e1 - e0 + 3) >> 2;
+    const int first_mine = e0 + k;
     const unsigned own_row = static_cast<unsigned>(node >= 0 ? node : 0) * static_cast<unsigned>(4 * C);
     float acc[2][8][4];
 #pragma unroll
@@ -260,12 +240,13 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
     // Unconditional (an edge index beyond the list reads the last edge, and prepare() discards it): loads under a
     // branch would make the later waits cover everything in flight.
     auto request = [&](int blk) {
-      const int64_t e = min(e0 + 4 * blk + k, last_edge);
-      return Raw{p.sender[e], p.vec[3 * e + 0], p.vec[3 * e + 1], p.vec[3 * e + 2]};
+      const unsigned e = static_cast<unsigned>(min(first_mine + 4 * blk, last_edge));
+      const float *v = reinterpret_cast<const float *>(reinterpret_cast<const char *>(p.vec) + 12u * e);
+      return Raw{*reinterpret_cast<const int *>(reinterpret_cast<const char *>(p.sender) + 4u * e), v[0], v[1], v[2]};
     };
     auto prepare = [&](const Raw &r, int blk) {
       Prepared o;
-      const bool valid = e0 + 4 * blk + k < e1;
+      const bool valid = first_mine + 4 * blk < e1;
       // Direction from one reciprocal square root (the hardware's, one Newton step: within an ulp), the length from it by
       // one more Newton step, whose residual r2 - len^2 is exact in an fma (without it the length is off by 1.4 times the
       // rounding of a square root, and the message by 3 to 8 % more than the other forward kernels' on the same edges), the
@@ -291,21 +272,21 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
       for (int i = 0; i < 8; ++i) o.y[i] = live ? o.y[i] : 0.f;
       o.xr = live ? len - knot : 0.f;
       o.xo = live ? __umul24(static_cast<unsigned>(r.s), static_cast<unsigned>(4 * C)) : own_row;  // both below 2^24
-      o.io = live ? static_cast<unsigned>(idx) * 512u : zero_row;
+      o.io = live ? __umul24(static_cast<unsigned>(idx), kSlRowBytes) : zero_row;
       return o;
     };
-    auto rows = [&](const Prepared &o, f2 (&x)[4][2]) {
-      request_row<0>(p.X, o.xo, m, x[0]);
-      request_row<1>(p.X, o.xo, m, x[1]);
-      request_row<2>(p.X, o.xo, m, x[2]);
-      request_row<3>(p.X, o.xo, m, x[3]);
+    auto rows = [&](const Prepared &o, f4 (&x)[4]) {
+      request_row<0>(p.X, o.xo, place, x[0]);
+      request_row<1>(p.X, o.xo, place, x[1]);
+      request_row<2>(p.X, o.xo, place, x[2]);
+      request_row<3>(p.X, o.xo, place, x[3]);
     };
 
     // three sets that rotate: block b computes from set b % 3 while the rows of block b + 2 are requested into set
     // (b + 2) % 3 and the raw values of block b + 3 into raw set b % 3
     Raw r0 = request(0), r1 = request(1), r2 = request(2);
     Prepared p0 = prepare(r0, 0), p1 = prepare(r1, 1), p2;
-    f2 x0[4][2], x1[4][2], x2[4][2];
+    f4 x0[4], x1[4], x2[4];
     f4 q[8];
     Gathered all;
     rows(p0, x0);
@@ -314,26 +295,26 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
       r0 = request(blk + 3);
       __builtin_amdgcn_sched_barrier(0);
       p2 = prepare(r2, blk + 2);
-      read_pieces<0>(tab, p0.io, m, q);
+      read_pieces<0>(tab, p0.io, q);
       all = gather(p0);
       __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p0, all, p2, m, x0, x2, q, acc);
+      edge_step<P, 0>(p.X, tab, p0, all, p2, place, x0, x2, q, acc);
       if (!__any(blk + 1 < nblk)) break;
       r1 = request(blk + 4);
       __builtin_amdgcn_sched_barrier(0);
       p0 = prepare(r0, blk + 3);
-      read_pieces<0>(tab, p1.io, m, q);
+      read_pieces<0>(tab, p1.io, q);
       all = gather(p1);
       __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p1, all, p0, m, x1, x0, q, acc);
+      edge_step<P, 0>(p.X, tab, p1, all, p0, place, x1, x0, q, acc);
       if (!__any(blk + 2 < nblk)) break;
       r2 = request(blk + 5);
       __builtin_amdgcn_sched_barrier(0);
       p1 = prepare(r1, blk + 4);
-      read_pieces<0>(tab, p2.io, m, q);
+      read_pieces<0>(tab, p2.io, q);
       all = gather(p2);
       __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p2, all, p1, m, x2, x1, q, acc);
+      edge_step<P, 0>(p.X, tab, p2, all, p1, place, x2, x1, q, acc);
       if (!__any(blk + 3 < nblk)) break;
     }
 
@@ -341,16 +322,14 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
       char *op = reinterpret_cast<char *>(p.out + static_cast<int64_t>(node) * 16 * C);
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int pr = 0; pr < 2; ++pr)
-          *reinterpret_cast<f2 *>(op + static_cast<int64_t>(Pair<P>::row(i)) * (4 * C) + m.x[pr]) =
-              f2{acc[0][i][2 * pr] + acc[1][i][2 * pr], acc[0][i][2 * pr + 1] + acc[1][i][2 * pr + 1]};
+        *reinterpret_cast<f4 *>(op + static_cast<int64_t>(Pair<P>::row(i)) * (4 * C) + place) =
+            f4{acc[0][i][0] + acc[1][i][0], acc[0][i][1] + acc[1][i][1], acc[0][i][2] + acc[1][i][2], acc[0][i][3] + acc[1][i][3]};
     }
   }
 }
 
 __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(const SlicedArgs p) {
-  __shared__ __attribute__((aligned(16))) float sTab[kSlMaxIntervals * 128];
+  __shared__ __attribute__((aligned(16))) float sTab[kSlMaxIntervals * (kSlRowBytes / 4)];
   __shared__ float sKnots[kSlMaxIntervals + 1];
   __shared__ unsigned short sOrder[kSlSub];
   __shared__ int sHist[kSlBins];
@@ -381,20 +360,21 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
   const int lo = static_cast<int>(static_cast<int64_t>(p.nnodes) * j / p.share);
   const int hi = static_cast<int>(static_cast<int64_t>(p.nnodes) * (j + 1) / p.share);
 
-  // the slice of the table: coeffs[idx][coef][l C + 16 slice + 4 k + 2 pr + b] -> byte 512 idx + 256 li + 64 (pr + 2 b)
-  // + 16 k of sTab, (a, b, c, d) together
+  // the slice of the table: coeffs[idx][coef][l C + 16 slice + 4 k + d] -> byte kSlRowBytes idx + 256 li + 64 d + 16 k of sTab,
+  // (a, b, c, d) together
+  constexpr int kRow = kSlRowBytes / 4;
   const int intervals = p.nknots - 1;
   for (int i = tid; i < intervals * 32; i += kSlThreads) {
     const int idx = i >> 5, coef = (i >> 3) & 3, li = (i >> 2) & 1, k = i & 3;
     const int l = pair == 0 ? (li == 0 ? 0 : 3) : (li == 0 ? 1 : 2);
     const f4 v = ld4(p.coeffs + (static_cast<int64_t>(idx * 4 + coef) * 4 + l) * p.C + slice * 16 + 4 * k);
-    float *dst = sTab + idx * 128 + 64 * li + 4 * k + coef;
-    dst[0] = v.x;   // pr 0, b 0
-    dst[32] = v.y;  // pr 0, b 1
-    dst[16] = v.z;  // pr 1, b 0
-    dst[48] = v.w;  // pr 1, b 1
+    float *dst = sTab + idx * kRow + 64 * li + 4 * k + coef;
+    dst[0] = v.x;
+    dst[16] = v.y;
+    dst[32] = v.z;
+    dst[48] = v.w;
   }
-  for (int i = tid; i < 128; i += kSlThreads) sTab[intervals * 128 + i] = 0.f;  // the row of edges that do not count
+  for (int i = tid; i < 128; i += kSlThreads) sTab[intervals * kRow + i] = 0.f;  // the row of edges that do not count
   for (int i = tid; i < p.nknots; i += kSlThreads) sKnots[i] = p.knots[i];
 
   for (int sub = lo; sub < hi; sub += kSlSub) {
@@ -444,7 +424,7 @@ bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nk
   if (channels % 16 != 0 || share_of(channels) < 2 || nedges == 0) return false;
   if (nedges < min_edges(nnodes, channels)) return false;
   return nnodes > static_cast<int64_t>(share_of(channels)) * (kWave / 4) * (kSlMinRounds - 1) && nnodes < (1 << 24) &&
-         nnodes * channels < (int64_t{1} << 30) && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
+         nnodes * channels < (int64_t{1} << 30) && nedges <= UINT32_MAX / 12 && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }
 
 int launch_sliced_forward(const float *X, const float *vec, const float *knots, const float *coeffs, int nknots, float r_width,

@@ -229,7 +229,7 @@ def test_mp_edge_forward_on_both_sides_of_the_line_by_edges(cabi, case):
 
 
 def test_mp_edge_forward_sorts_the_nodes_of_a_workgroup_in_batches(cabi):
-    """40 000 receiver nodes with 13 edges each at 256 channels: 5 000 nodes per workgroup, sorted 4 096 at a time.  Against
+    """40 000 receiver nodes with 13 edges each at 256 channels: 5 000 nodes per workgroup, sorted 2 816 at a time.  Against
     the kernel that takes harmonics and lengths, and the oracle on a sample of nodes."""
     nnodes, C = 40000, 256
     snd, rcv, X, vec, knots, coeffs, h = _edge_case(nnodes, 13, C, 0.1, 9)
