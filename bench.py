@@ -82,8 +82,8 @@ def forward_kernel_name(C, N, E):
     """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_sliced.hip: sliced_forward_applies; the
     benchmark's spline table has 256 knots)."""
     share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
-    enough = {32: 0, 64: 120000 - 10 * N, 96: max(60000, 11 * N), 128: max(60000, 11 * N), 160: max(10000, 8 * N),
-              224: max(10000, 8 * N)}.get(C, 11 * N)
+    enough = {32: 0, 64: 120000 - 10 * N, 96: 65000 + 2 * N, 128: 50000 + 5 * N // 2, 160: 17000 + 5 * N // 2,
+              192: 14000 + 11 * N // 2, 224: 8000 + 3 * N}.get(C, 8000 + 5 * N)
     if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
         return "mp_edge_forward_sliced_kernel"
     return "mp_spline_forward_kernel<%d,true>" % C

@@ -41,7 +41,6 @@
 // file (252 of 256) and no time; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
 // with one wave per node: 96 channels 2.68e-7 -> 2.54e-7 (2.70e-7), 128 2.73 -> 2.59 (2.74), 192 2.67 -> 2.52 (2.69), 256
 // 2.81 -> 2.67 (2.83).
-#include <algorithm>
 #include <type_traits>
 
 #include "mp_common.hpp"
@@ -61,25 +60,28 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 // nodes with few edges leave it with the fixed part of a round, while the kernel with one wave per node pays per edge.
 // Measured, one wave per node -> this one (us), nodes x neighbours:
 //   32 channels   5 121 x 2 15.9 -> 10.7, 12 000 x 2 30.9 -> 17.4: always
-//   64            2 561 x 20 16.4 -> 17.7, 2 561 x 52 29.8 -> 28.5, 5 000 x 14 22.0 -> 23.2, 5 000 x 20 26.0 -> 25.5, 8 000 x 2 18.6 -> 19.8,
-//                 8 000 x 8 24.9 -> 24.0, 12 000 x 2 25.3 -> 24.3
-//   96, 128       1 681 x 30 x 96 19.2 -> 22.1, 1 681 x 52 31.5 -> 29.9, 3 500 x 14 22.1 -> 23.9, 3 500 x 20 27.0 -> 27.0, 12 000 x 8
-//                 37.7 -> 40.7, 12 000 x 14 54.5 -> 50.2; 1 281 x 52 x 128 28.4 -> 28.9, 2 049 x 8 12.8 -> 17.4, 2 049 x 30
-//                 28.4 -> 26.4, 5 000 x 8 23.9 -> 27.9, 5 000 x 14 33.9 -> 32.8, 12 000 x 8 45.6 -> 49.0, 12 000 x 14 68.0 -> 61.7
-//   160, 224      (there the other kernel fetches five and seven single channels per lane) 961 x 8 x 160 13.7 -> 15.1, 961 x 14
-//                 18.5 -> 17.3, 5 000 x 5 26.7 -> 28.7, 5 000 x 8 33.9 -> 32.3; 721 x 8 x 224 13.9 -> 16.4, 721 x 14 21.6 -> 20.0, 12 000 x 8 87.7 -> 78.5
-//   192, 256      801 x 8 x 192 12.8 -> 14.6, 801 x 14 17.7 -> 16.9, 5 000 x 8 33.6 -> 37.5, 5 000 x 14 50.1 -> 46.2; 641 x 8 x 256
-//                 14.6 -> 17.1, 641 x 14 22.7 -> 20.0, 12 000 x 8 85.9 -> 97.4, 12 000 x 14 137.5 -> 130.8
+//   64            2 561 x 20 16.4 -> 17.7, 2 500 x 52 27.6 -> 25.4, 5 000 x 15 21.8 -> 20.9, 8 000 x 4 20.2 -> 18.4
+//   96            1 000 x 52 19.1 -> 23.0, 1 700 x 52 26.5 -> 26.9, 3 000 x 20 21.9 -> 23.7, 8 000 x 10 29.7 -> 28.8, 12 000 x 5.7 30.8 ->
+//                 32.1, 12 000 x 7.5 35.6 -> 33.6, 25 000 x 4.1 50.7 -> 49.5
+//   128           1 000 x 52 22.3 -> 24.0, 1 300 x 52 28.1 -> 25.9, 2 500 x 15 20.1 -> 21.2, 3 500 x 15 26.1 -> 25.3, 6 000 x 10 29.2 ->
+//                 28.6, 12 000 x 5.7 36.3 -> 36.8, 12 000 x 7.5 43.2 -> 41.8, 25 000 x 4.1 60.1 -> 59.4, 25 000 x 7.6 85.3 -> 69.9
+//   160           1 200 x 15 17.3 -> 17.1, 2 000 x 10 18.0 -> 19.8, 5 000 x 4.2 23.3 -> 24.3, 5 000 x 8 33.9 -> 32.3, 12 000 x 4 43.7 -> 42.9
+//   192           1 200 x 15 18.0 -> 17.6, 2 000 x 10 18.5 -> 21.1, 5 000 x 7.7 30.6 -> 31.4, 5 000 x 10 37.2 -> 34.5, 12 000 x 5.7 51.8 ->
+//                 54.4
+//   224           721 x 8 13.9 -> 16.4, 600 x 15 16.0 -> 15.9, 2 000 x 10 22.5 -> 22.2, 12 000 x 4 57.0 -> 53.4
+//   256           1 200 x 10 18.6 -> 19.9, 2 000 x 10 23.5 -> 23.2, 5 000 x 7.7 38.4 -> 36.6, 12 000 x 5.7 63.6 -> 65.0, 12 000 x 7.5 78.6 ->
+//                 69.6, 12 000 x 10 96.1 -> 80.6
 constexpr int kSlMinRounds = 6;
 inline int64_t min_edges(int64_t nnodes, int channels) {
   switch (channels) {
     case 32: return 0;
     case 64: return 120000 - 10 * nnodes;
-    case 96:
-    case 128: return std::max<int64_t>(60000, 11 * nnodes);
-    case 160:
-    case 224: return std::max<int64_t>(10000, 8 * nnodes);
-    default: return 11 * nnodes;
+    case 96: return 65000 + 2 * nnodes;
+    case 128: return 50000 + 5 * nnodes / 2;
+    case 160: return 17000 + 5 * nnodes / 2;
+    case 192: return 14000 + 11 * nnodes / 2;
+    case 224: return 8000 + 3 * nnodes;
+    default: return 8000 + 5 * nnodes;
   }
 }
 inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)

@@ -228,6 +228,14 @@ def test_mp_edge_forward_on_both_sides_of_the_line_by_edges(cabi, case):
     test_mp_edge_forward_many_nodes(cabi, case)
 
 
+@pytest.mark.parametrize("case", [(2048, 36, 96, 0.05, 2, 200, 0), (1300, 25, 160, 0.3, 3, 256, 0), (900, 22, 192, 0.0, 4, 256, 0),
+                                  (1000, 12, 224, 0.0, 5, 256, 0), (700, 17, 256, 0.0, 6, 272, 0), (9000, 9, 128, 0.1, 7, 128, 300)],
+                         ids=lambda c: "N%d_d%d_C%d" % (c[0], c[1], c[2]))
+def test_mp_edge_forward_just_above_the_line_by_edges(cabi, case):
+    """As above, with the edges that the line asks for at these widths, and many nodes with few edges."""
+    test_mp_edge_forward_many_nodes(cabi, case)
+
+
 def test_mp_edge_forward_sorts_the_nodes_of_a_workgroup_in_batches(cabi):
     """40 000 receiver nodes with 13 edges each at 256 channels: 5 000 nodes per workgroup, sorted 2 816 at a time.  Against
     the kernel that takes harmonics and lengths, and the oracle on a sample of nodes."""
@@ -272,8 +280,8 @@ def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi)
 @pytest.mark.parametrize("case", [(1024, 6, 160, 0.2, 21, 256, 0), (1100, 13, 160, 0.0, 22, 600, 150), (1024, 5, 192, 0.2, 23, 256, 0), (1024, 15, 192, 0.2, 25, 256, 0),
                                   (1060, 17, 192, 0.0, 24, 2, 129)], ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
 def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
-    """From 1 024 nodes on at 160 channels, and with 12 edges per node at 192: nodes with every remainder of a group of four edges, one with more than
-    one and more than two chunks of 64, dead edges in between, knots in LDS and in memory, a table of one interval."""
+    """Widths on both sides of the kernel with a row of 16 lanes per edge: nodes with every remainder of a group of four edges, one
+    with more than one and more than two chunks of 64, dead edges in between, knots in LDS and in memory, a table of one interval."""
     nnodes, C = case[0], case[2]
     snd, rcv, X, vec, knots, coeffs, h = _edge_case(*case)
     degrees = torch.bincount(rcv.long(), minlength=nnodes)
@@ -293,6 +301,16 @@ def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
     assert float(gvec[~live.cuda()].abs().max()) == 0.0
     assert torch.equal(cabi.mp_edge_backward(*args, need_gvec=False)[0], gX)
     assert torch.equal(cabi.mp_edge_backward(*args, need_gX=False)[1], gvec)
+
+
+@pytest.mark.parametrize("case", [(40, 9, 160, 0.0, 31, 3, 0), (90, 21, 192, 0.0, 32, 257, 150), (300, 19, 224, 0.1, 33, 600, 150),
+                                  (1100, 13, 224, 0.0, 34, 256, 129), (40, 7, 64, 0.0, 35, 4, 0), (300, 13, 64, 0.1, 36, 512, 150),
+                                  (1100, 9, 32, 0.1, 37, 5, 150), (2100, 6, 128, 0.1, 38, 513, 70), (300, 17, 96, 0.0, 39, 256, 130)],
+                         ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
+def test_mp_edge_backward_few_and_many_nodes(cabi, case):
+    """Few nodes (an edge range cut into parts) and many, every width class, partly filled groups, trips and chunks, and tables on
+    both sides of what the copy of the knots takes (four knots at a time, up to 256 or 512)."""
+    test_mp_edge_backward_on_the_matrix_cores(cabi, case)
 
 
 @pytest.mark.parametrize("nnodes,C", [(1750, 96), (1400, 128), (1000, 160), (900, 192), (700, 256)])
