@@ -14,6 +14,8 @@
 // v_mfma_f32_32x32x16_bf16, K in chunks of 32), and every intermediate is rounded to fp32 where the separate launches
 // store it, so the chain returns the bits of the separate launches.
 //
+// A third launch has the product linear of the second layer, the readouts and the product of their derivative (node_head below).
+//
 // g1 and g2 are the gradients of minus the (weighted) sum of node energies with respect to the two layers' features:
 // g1[n, c] = -weight[n] scale w1[c] is formed here from the linear readout's weights; g2 = -dE/dh2 arrives as dE/dh2 and
 // its sign goes into the scale of the skip product.
@@ -21,6 +23,7 @@
 #include "mfma_f32.hpp"
 #include "mfma_split.hpp"
 #include "node_glue.hpp"
+#include "readout_device.hpp"
 
 // Products and the additions that follow them stay separate roundings, as they are where separate launches store the
 // product before the next one adds to it.
@@ -500,6 +503,272 @@ __global__ __launch_bounds__(4 * kWave) void node_glue_gh1_kernel(const float *_
   st4(gh1 + in * C + col0 + 4 * part, few_gh1(v[0], u[0], w1 + col0 + 4 * part, scale, node_weights ? node_weights[in] : 1.0, skip_scale, no_element));
 }
 
+// ---- head: h2 = B2 . Wprod + sc, readouts of h1 and h2, gB2 = -w dE/dh2 . Wprod^T (w: the node's weight) --------------
+// Between the second layer's contraction and the backward chain every step is per node: a product with a residual, the
+// readouts (readout.hip has their arithmetic and the meaning of the operands), and the product of their derivative.  h2 stays
+// in LDS: of the [N, C] rows only dE/dh2 is written besides gB2, for the skip connection's gradient.  The readouts are
+// bound by nothing but the fp64 matrix rate and the chain of a tile, 0.9 us each way at 128 x 128 on four matrix pipes.
+// Measured inside the step, three launches -> one (us): 21 x 64 9.0 -> 5.2, 216 x 128 14.8 -> 12.4, 2 000 x 128 15.4 -> 12.5 (tiles
+// of 16 nodes), 5 000 x 96 24.0 -> 15.6, 10 752 x 64 23.9 -> 13.5 (tiles of 32), 25 000 x 128 66.6 -> 40 (128; with tiles of 64, two
+// rounds of workgroups by their registers, 48; its 112 MB, half of them the fp64 feature rows, take 21).
+// Without d_h2 (energies alone) the kernel ends with the energies.  Bits of the separate launches, as above.
+// A wave takes tiles of 16 nodes, all classes of pieces of each (in the separate kernel four waves share the classes of a
+// tile; where there are two waves per tile they share them); the weights of the readouts wait in LDS.
+template <int NT, int ROWS>
+__global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_head_kernel(
+    const float *__restrict__ B2, const float *__restrict__ sc, const float *__restrict__ h1, const float *__restrict__ prod_WT,
+    const float *__restrict__ prod_W, readout::Weights w, readout::Outputs out, const double *__restrict__ node_weights, int nnodes,
+    float *__restrict__ d_h2, float *__restrict__ gB2) {
+  constexpr int C = 32 * NT, kPieces = C / 16, kHidden = readout::kHidden;
+  using S = GlueShared<NT, ROWS>;
+  constexpr int kWaves = S::kThreads / kWave, kTiles = ROWS / 16;
+  constexpr int kLdW = kHidden + 2;  // row stride of W2a in LDS (doubles): the four lane groups of a read start 64 bytes apart in bank space
+  __shared__ __attribute__((aligned(16))) S s;
+  __shared__ __attribute__((aligned(16))) double sW[C * kLdW], sw1[C];
+  const int tid = threadIdx.x;
+  const int node0 = blockIdx.x * ROWS, nrows = min(ROWS, nnodes - node0);  // consecutive nodes
+  sc += static_cast<int64_t>(node0) * C, h1 += static_cast<int64_t>(node0) * C;
+  if (d_h2) d_h2 += static_cast<int64_t>(node0) * C, gB2 += static_cast<int64_t>(node0) * C;
+  stage_nodes(s, nullptr, node0, nnodes, nnodes);
+
+  WeightPieces<S> wa;
+  RowPieces<S> a0;
+  fetch_weights<S>(prod_WT, wa);
+  fetch_rows(s, B2, a0);
+  constexpr int kWPer = (C * kHidden + S::kThreads - 1) / S::kThreads;
+  double w2a[kWPer];
+#pragma unroll
+  for (int i = 0; i < kWPer; ++i) {
+    const int q = tid + i * S::kThreads, c = q / kHidden, j = q % kHidden;
+    w2a[i] = c < C && j < w.hidden ? w.W2a[c * w.hidden + j] : 0.0;
+  }
+  const double w1v = tid < C ? w.w1[tid] : 0.0;
+  // the residual rows go to the tile, as the readouts' weights go to LDS: during the product no registers are left for them
+  constexpr int kTilePer = ROWS * C / 4 / S::kThreads;
+  static_assert(kTilePer * S::kThreads == ROWS * C / 4, "the tile's pieces divide evenly among the threads");
+  f4 res[kTilePer];
+#pragma unroll
+  for (int i = 0; i < kTilePer; ++i) {
+    const int q = tid + i * S::kThreads;
+    res[i] = ld4(sc + min(4 * q / C, nrows - 1) * C + 4 * q % C);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < kTilePer; ++i) {
+    const int q = tid + i * S::kThreads;
+    *reinterpret_cast<f4 *>(s.tile + 4 * q / C * S::kLdT + 4 * q % C) = res[i];
+  }
+#pragma unroll
+  for (int i = 0; i < kWPer; ++i) {
+    const int q = tid + i * S::kThreads;
+    if (q < C * kHidden) sW[q / kHidden * kLdW + q % kHidden] = w2a[i];
+  }
+  if (tid < C) sw1[tid] = w1v;
+
+  v16f acc;
+  product<S, false>(s, &a0, wa, acc);
+  if (d_h2) fetch_weights<S>(prod_W, wa);
+  for_each_output<S>(acc, [&](int row, int col, float v) {
+    float &h2 = s.tile[row * S::kLdT + col];
+    h2 = v * 1.0f + h2;
+  });
+  __syncthreads();
+
+  // a wave has half of the classes, of the hidden units and of the pieces of its tile where there are two per tile
+  constexpr int kShare = kWaves >= 2 * kTiles ? 2 : 1, kMine = readout::kClasses / kShare;
+  static_assert(kShare == 1 || kWaves == kShare * kTiles, "every wave has a tile: they all meet at the barriers");
+  static_assert(kShare == 1 || sizeof(s.a) >= kWaves * kWave * 3 * sizeof(double), "two values per lane and an energy to exchange");
+  double(*swap)[3][kWave] = reinterpret_cast<double(*)[3][kWave]>(s.a);
+  const int lane = tid % kWave, col = lane % 16, part = lane / 16;
+  const int half = tid / kWave % kShare, other = tid / kWave ^ (kShare - 1);
+  for (int t = tid / kWave / kShare; t < kTiles; t += kWaves / kShare) {
+    float *mine = s.tile + (16 * t + col) * S::kLdT + 4 * part;  // the lane's node of the tile, its channels of piece 0
+    const bool here = 16 * t + col < nrows;
+    const int node = node0 + 16 * t + col;
+    const int row = here && out.rows ? out.rows[node] : node;
+    const bool row_ok = here && static_cast<unsigned>(row) < static_cast<unsigned>(nnodes);
+    const int at = (here ? 16 * t + col : 0) * C + 4 * part;
+    // classes kMine half .. : piece u of the wave is class kMine half + u % kMine
+    constexpr int kOwn = kPieces / kShare;
+    static_assert(kShare == 1 || kPieces % readout::kClasses == 0, "the halves have the same number of pieces");
+    auto piece = [&](int u) { return readout::kClasses * (u / kMine) + kMine * half + u % kMine; };
+    readout::d4v z[kMine];
+    double e1[kMine];
+#pragma unroll
+    for (int k = 0; k < kMine; ++k) z[k] = readout::d4v{0.0, 0.0, 0.0, 0.0}, e1[k] = 0.0;
+    f4 a[kOwn];
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) a[u] = ld4(h1 + at + 16 * piece(u));
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) {
+      const f4 b = *reinterpret_cast<const f4 *>(mine + 16 * piece(u));
+      const int c = 16 * piece(u) + 4 * part;
+      double wz[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wz[i] = sW[(c + i) * kLdW + readout::operand_row(col)];
+      readout::add_z(z[u % kMine], wz, b);
+      readout::add_linear(e1[u % kMine], *reinterpret_cast<const readout::d2v *>(sw1 + c), *reinterpret_cast<const readout::d2v *>(sw1 + c + 2), a[u]);
+      if (out.feats64 && row_ok) readout::store_feats(out.feats64 + static_cast<int64_t>(row) * (2 * C) + c, C, a[u], b);
+    }
+    // sums in pairs, (0 + 1) + (2 + 3), of classes and of hidden units, whoever has them
+    readout::d4v zsum = z[0] + z[1];
+    double esum = e1[0] + e1[1], e2[4], d[4];
+    auto gate = [&](int i) { return 4 * part + i < w.hidden ? w.w2b[4 * part + i] * w.act_cst : 0.0; };
+    if constexpr (kShare == 1) {
+      zsum = zsum + (z[2] + z[3]);
+      esum = esum + (e1[2] + e1[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) readout::activate(gate(i), zsum[i], e2[i], d[i]);
+      esum = esum + ((e2[0] + e2[1]) + (e2[2] + e2[3]));
+    } else {
+      // unit 2 half + j of the lane's four: from the other wave its share of z, to it (in the second exchange) the derivative
+      double(&out1)[3][kWave] = swap[tid / kWave], (&in1)[3][kWave] = swap[other];
+      out1[0][lane] = half == 0 ? zsum[2] : zsum[0];
+      out1[1][lane] = half == 0 ? zsum[3] : zsum[1];
+      out1[2][lane] = esum;
+      __syncthreads();
+      const double z0 = (half == 0 ? zsum[0] : zsum[2]) + in1[0][lane], z1 = (half == 0 ? zsum[1] : zsum[3]) + in1[1][lane];
+      esum = esum + in1[2][lane];
+      double d0, d1;
+      readout::activate(gate(2 * half), z0, e2[0], d0);
+      readout::activate(gate(2 * half + 1), z1, e2[1], d1);
+      __syncthreads();
+      out1[0][lane] = d0, out1[1][lane] = d1, out1[2][lane] = e2[0] + e2[1];
+      __syncthreads();
+      esum = esum + ((e2[0] + e2[1]) + in1[2][lane]);
+      const double d2 = in1[0][lane], d3 = in1[1][lane];
+      d[0] = half == 0 ? d0 : d2, d[1] = half == 0 ? d1 : d3, d[2] = half == 0 ? d2 : d0, d[3] = half == 0 ? d3 : d1;
+    }
+    const double en = readout::node_energy(esum, w.scale, w.shift);
+    if (here && part == 0 && half == 0) readout::store_energy(out, node, row, row_ok, en);
+    if (!d_h2) continue;
+#pragma unroll 2
+    for (int u = 0; u < kOwn; ++u) {
+      const int p = piece(u);
+      const double *wp = sW + (16 * p + readout::operand_row(col)) * kLdW + 4 * part;
+      const double wd[4] = {wp[0], wp[1], wp[2], wp[3]};
+      f4 g = readout::derivative(wd, d, w.scale);
+      if (node_weights) {
+        const double nw = here ? node_weights[node] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g[i] = static_cast<float>(static_cast<double>(g[i]) * nw);
+      }
+      if (here) st4(d_h2 + at + 16 * p, g);
+      *reinterpret_cast<f4 *>(mine + 16 * p) = g;  // read above by the lane itself
+    }
+  }
+  if (!d_h2) return;
+  product<S, true>(s, nullptr, wa, acc);
+  for_each_output<S>(acc, [&](int row, int col, float v) {
+    if (row < nrows) gB2[row * C + col] = v * -1.0f;
+  });
+}
+
+// Few nodes: tiles of 16, a wave per 16 columns, the readouts' sums shared by the waves as in the separate kernel.
+template <int NT>
+__global__ __launch_bounds__(2 * NT *kWave) void node_head_few_kernel(
+    const float *__restrict__ B2, const float *__restrict__ sc, const float *__restrict__ h1, const float *__restrict__ prod_WT,
+    const float *__restrict__ prod_W, readout::Weights w, readout::Outputs out, const double *__restrict__ node_weights, int nnodes,
+    float *__restrict__ d_h2, float *__restrict__ gB2) {
+  constexpr int C = 32 * NT, KQ = C / 16, kWaves = 2 * NT;
+  constexpr int kClasses = readout::kClasses, kUsed = KQ < kClasses ? KQ : kClasses;  // classes that have a piece
+  constexpr int kPer = (KQ + kClasses - 1) / kClasses;                                // pieces of a class
+  using S = FewShared<NT>;
+  __shared__ __attribute__((aligned(16))) S s;
+  __shared__ double sZ[kUsed][4][kWave], sE[kUsed][kWave], sE2[4][kWave], sD[4][kWave];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int row = lane % few::kRows, part = lane / few::kRows, col0 = few::kRows * wave;
+  const int64_t wat = static_cast<int64_t>(col0 + row) * C + 4 * part;
+  const int node = blockIdx.x * few::kRows + row;
+  const bool here = node < nnodes;
+  const int64_t in = here ? node : 0;
+  few::Rows<KQ> wp[1] = {few::load_rows<KQ>(prod_WT + wat)}, wq[1];
+  const few::Rows<KQ> x = few::load_rows<KQ>(B2 + in * C + 4 * part);
+  __builtin_amdgcn_sched_barrier(0);  // the first product's operands first: the loads of a compute unit return one after the other
+  const int64_t at = in * C + col0 + 4 * part;
+  const f4 residual = ld4(sc + at);
+  // what this wave needs for the readouts: class `wave` of the pieces, element `wave` of z, piece `wave` of the derivative
+  f4 a[kPer];
+  double wz[kPer][4], wd[4];
+  readout::d2v wl[kPer][2];
+  if (wave < kUsed) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int c = 16 * (wave + kClasses * u) + 4 * part;
+      if (c >= C) break;  // the same for the whole wave
+      a[u] = ld4(h1 + in * C + c);
+      wl[u][0] = *reinterpret_cast<const readout::d2v *>(w.w1 + c), wl[u][1] = *reinterpret_cast<const readout::d2v *>(w.w1 + c + 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wz[u][i] = readout::operand_row(row) < w.hidden ? w.W2a[(c + i) * w.hidden + readout::operand_row(row)] : 0.0;
+    }
+  }
+  const double *wd_at = w.W2a + static_cast<int64_t>(16 * wave + readout::operand_row(row)) * w.hidden + 4 * part;
+  if (w.hidden == readout::kHidden) {
+    const readout::d2v lo = reinterpret_cast<const readout::d2v *>(wd_at)[0], hi = reinterpret_cast<const readout::d2v *>(wd_at)[1];
+    wd[0] = lo.x, wd[1] = lo.y, wd[2] = hi.x, wd[3] = hi.y;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wd[i] = 4 * part + i < w.hidden ? wd_at[i] : 0.0;
+  }
+  auto gate_of = [&](int i) { return 4 * part + i < w.hidden ? w.w2b[4 * part + i] * w.act_cst : 0.0; };
+  const double gate = gate_of(wave % 4);
+  const int to = here && out.rows ? out.rows[in] : node;
+  const bool to_ok = here && static_cast<unsigned>(to) < static_cast<unsigned>(nnodes);
+  const double nw = node_weights ? node_weights[in] : 1.0;
+  if (d_h2) wq[0] = few::load_rows<KQ>(prod_W + wat);
+  __builtin_amdgcn_sched_barrier(0);  // all operands on their way before the first product waits
+
+  f4 v[1];
+  few::product<KQ, 1>(x, wp, v);
+  put(s, v[0] + residual);
+  __syncthreads();
+  if (wave < kUsed) {
+    readout::d4v z{0.0, 0.0, 0.0, 0.0};
+    double e1 = 0.0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int c = 16 * (wave + kClasses * u) + 4 * part;
+      if (c >= C) break;
+      const f4 b = *reinterpret_cast<const f4 *>(s.tile + row * S::kLd + c);
+      readout::add_z(z, wz[u], b);
+      readout::add_linear(e1, wl[u][0], wl[u][1], a[u]);
+      if (out.feats64 && to_ok) readout::store_feats(out.feats64 + static_cast<int64_t>(to) * (2 * C) + c, C, a[u], b);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sZ[wave][i][lane] = z[i];
+    sE[wave][lane] = e1;
+  }
+  __syncthreads();
+  auto total = [&](const auto &get_class) {
+    double q[kClasses];
+#pragma unroll
+    for (int k = 0; k < kClasses; ++k) q[k] = k < kUsed ? get_class(k < kUsed ? k : 0) : 0.0;
+    return (q[0] + q[1]) + (q[2] + q[3]);
+  };
+  for (int i = wave; i < 4; i += kWaves) {
+    const double z_i = total([&](int k) { return sZ[k][i][lane]; });
+    readout::activate(i == wave ? gate : gate_of(i), z_i, sE2[i][lane], sD[i][lane]);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const double e = total([&](int k) { return sE[k][lane]; }) + ((sE2[0][lane] + sE2[1][lane]) + (sE2[2][lane] + sE2[3][lane]));
+    const double en = readout::node_energy(e, w.scale, w.shift);
+    if (here && part == 0) readout::store_energy(out, node, to, to_ok, en);
+  }
+  if (!d_h2) return;
+  const double d[4] = {sD[0][lane], sD[1][lane], sD[2][lane], sD[3][lane]};
+  f4 g = readout::derivative(wd, d, w.scale);
+  if (node_weights) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = static_cast<float>(static_cast<double>(g[i]) * nw);
+  }
+  if (here) st4(d_h2 + at, g);
+  put(s, g);  // the rows of h2 have been read
+  __syncthreads();
+  few::product<KQ, 1>(get(s), wq, v);
+  if (here) st4(gB2 + at, v[0] * -1.0f);
+}
+
 // 128-node tiles where they give at least half of the compute units one each, 32-node tiles below that
 inline bool small_tiles(int64_t nnodes) { return ceil_div(nnodes, kGlTile) * 2 < device_compute_units(); }
 
@@ -568,6 +837,22 @@ int launch_backward(const float *gX2, const float *d_h2, const float *up_W, cons
   return check_launch("cm_node_glue_backward");
 }
 
+template <int NT>
+int launch_head(const float *B2, const float *sc, const float *h1, const float *prod_WT, const float *prod_W, const readout::Weights &w,
+                const readout::Outputs &out, const double *node_weights, int64_t nnodes, float *d_h2, float *gB2, hipStream_t st) {
+  const int n = static_cast<int>(nnodes);
+  if (few::applies(nnodes, 1, 32 * NT))
+    hipLaunchKernelGGL((node_head_few_kernel<NT>), dim3(static_cast<unsigned>(ceil_div(nnodes, few::kRows))), dim3(2 * NT * kWave), 0, st, B2, sc, h1,
+                       prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
+  else if (small_tiles(nnodes))
+    hipLaunchKernelGGL((node_head_kernel<NT, kGlSmallTile>), dim3(static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile))), dim3(NT * kWave), 0, st, B2,
+                       sc, h1, prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
+  else
+    hipLaunchKernelGGL((node_head_kernel<NT, kGlTile>), dim3(static_cast<unsigned>(ceil_div(nnodes, kGlTile))), dim3(4 * NT * kWave), 0, st, B2, sc,
+                       h1, prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
+  return check_launch("cm_mace_step");
+}
+
 }  // namespace
 }  // namespace cm
 
@@ -606,6 +891,18 @@ int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, con
     case 3: return launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     case 4: return launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     default: set_error("node glue: channels=%d not supported", channels); return CM_EINVAL;
+  }
+}
+
+int node_head(const float *B2, const float *sc, const float *h1, const float *prod_WT, const float *prod_W, const readout::Weights &w,
+              const readout::Outputs &out, const double *node_weights, int64_t nnodes, int channels, float *d_h2, float *gB2, hipStream_t st) {
+  CM_REQUIRE(w.hidden >= 1 && w.hidden <= readout::kHidden, "cm_mace_step: hidden=%d must be in [1, %d]", w.hidden, readout::kHidden);
+  switch (channels / 32) {
+    case 1: return launch_head<1>(B2, sc, h1, prod_WT, prod_W, w, out, node_weights, nnodes, d_h2, gB2, st);
+    case 2: return launch_head<2>(B2, sc, h1, prod_WT, prod_W, w, out, node_weights, nnodes, d_h2, gB2, st);
+    case 3: return launch_head<3>(B2, sc, h1, prod_WT, prod_W, w, out, node_weights, nnodes, d_h2, gB2, st);
+    case 4: return launch_head<4>(B2, sc, h1, prod_WT, prod_W, w, out, node_weights, nnodes, d_h2, gB2, st);
+    default: set_error("node head: channels=%d not supported", channels); return CM_EINVAL;
   }
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "readout_device.hpp"
 
 namespace cm {
 
@@ -14,5 +15,10 @@ int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, con
                                         const int32_t *group_offsets, int64_t nnodes, int ngroups, int channels, float skip_scale, float *gh1,
                                         float *gB1, const double *node_es, const int32_t *graph_ptr, int ngraphs, double *energies,
                                         const double *graph_e0, double *total_energies, hipStream_t st);
+
+// h2 = B2 . Wprod + sc (kept on chip), the readouts of h1 and h2 with everything cm_readout_forward writes, and, with d_h2
+// given, d_h2 = weight dE/dh2 (node_weights NULL: one) and gB2 = -d_h2 . Wprod^T.  32 to 128 channels (cm_node_glue_supported).
+int node_head(const float *B2, const float *sc, const float *h1, const float *prod_WT, const float *prod_W, const readout::Weights &w,
+              const readout::Outputs &out, const double *node_weights, int64_t nnodes, int channels, float *d_h2, float *gB2, hipStream_t st);
 
 }  // namespace cm

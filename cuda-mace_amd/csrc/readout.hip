@@ -21,18 +21,20 @@
 
 #include "common.hpp"
 #include "readout.hpp"
+#include "readout_device.hpp"
 
 namespace cm {
 namespace {
 
 constexpr int kNodes = 16;    // nodes per workgroup
-constexpr int kHidden = 16;   // threads per node = largest hidden width handled
+using readout::kHidden;       // threads per node = largest hidden width handled
+using readout::d2v;
+using readout::d4v;
 constexpr int kMaxC = 256;
 constexpr int kLdW = kMaxC + 2;   // row stride (doubles) of W2a transposed, [hidden][channel]: rows j and j + 1 start 4 banks apart,
                                   // so the 16 hidden units of a node read their 16-byte pieces without conflicts
 constexpr int kMaxGroups = 512;   // workgroups of a forward launch
 constexpr int kLdS = kMaxC + 4;   // row stride (floats) of a feature tile: 16-byte aligned rows, the four nodes of a wave 4 banks apart
-typedef double d2v __attribute__((ext_vector_type(2)));
 
 __global__ __launch_bounds__(kNodes *kHidden) void readout_forward_kernel(
     const float *__restrict__ h1, const float *__restrict__ h2, const double *__restrict__ w1, const double *__restrict__ W2a,
@@ -212,7 +214,6 @@ __global__ __launch_bounds__(kNodes *kHidden) void readout_forward_kernel(
 // results neighbours in memory.
 // Measured (us, the kernel above -> this one): 20 x 64 5.3 -> 3.6, 216 x 128 7.3 -> 5.1, 5 000 x 128 12.4 -> 8.5, 25 000 x 128
 // 32.4 -> 21.7, 12 000 x 256 33.4 -> 19.6 (with the fp64 rows written); few nodes: the latency of its chain, many: memory.
-typedef double d4v __attribute__((ext_vector_type(4)));
 constexpr int kMfmaWaves = 4;
 __global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel(
     const float *__restrict__ h1, const float *__restrict__ h2, const double *__restrict__ w1, const double *__restrict__ W2a,
@@ -228,7 +229,7 @@ __global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel
   const bool here = node < nnodes;
   const int in = here ? node : nnodes - 1;
   const int npieces = C / 16;
-  const int unit = 4 * (col % 4) + col / 4;  // hidden unit of operand row col: element i of z is then unit 4 (lane / 16) + i
+  const int unit = readout::operand_row(col);
   f4 a[kPieces], b[kPieces];
   double wz[kPieces][4], wd[kPieces][4];
   d2v wl[kPieces][2];
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel
       wz[u][i] = unit < H ? W2a[(c + i) * H + unit] : 0.0;
     }
     if (d2) {
-      const double *wp = W2a + static_cast<int64_t>(16 * p + 4 * (col % 4) + col / 4) * H + 4 * part;
+      const double *wp = W2a + static_cast<int64_t>(16 * p + readout::operand_row(col)) * H + 4 * part;
       if (H == kHidden) {
         const d2v lo = reinterpret_cast<const d2v *>(wp)[0], hi = reinterpret_cast<const d2v *>(wp)[1];
         wd[u][0] = lo.x, wd[u][1] = lo.y, wd[u][2] = hi.x, wd[u][3] = hi.y;
@@ -265,18 +266,9 @@ __global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel
   for (int u = 0; u < kPieces; ++u) {
     const int p = wave + kMfmaWaves * u;
     if (p >= npieces) break;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      z = __builtin_amdgcn_mfma_f64_16x16x4f64(wz[u][i], static_cast<double>(b[u][i]), z, 0, 0, 0);
-      e1 += static_cast<double>(a[u][i]) * wl[u][i / 2][i % 2];
-    }
-    if (feats64 && row_ok) {
-      double *f = feats64 + static_cast<int64_t>(row) * (2 * C) + 16 * p + 4 * part;
-      reinterpret_cast<d2v *>(f)[0] = d2v{a[u].x, a[u].y};
-      reinterpret_cast<d2v *>(f)[1] = d2v{a[u].z, a[u].w};
-      reinterpret_cast<d2v *>(f + C)[0] = d2v{b[u].x, b[u].y};
-      reinterpret_cast<d2v *>(f + C)[1] = d2v{b[u].z, b[u].w};
-    }
+    readout::add_z(z, wz[u], b[u]);
+    readout::add_linear(e1, wl[u][0], wl[u][1], a[u]);
+    if (feats64 && row_ok) readout::store_feats(feats64 + static_cast<int64_t>(row) * (2 * C) + 16 * p + 4 * part, C, a[u], b[u]);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) sZ[wave][i][lane] = z[i];
@@ -286,32 +278,22 @@ __global__ __launch_bounds__(kMfmaWaves *kWave) void readout_forward_mfma_kernel
   auto total = [&](const auto &v) { return (v(0) + v(1)) + (v(2) + v(3)); };
   {
     const double z_i = total([&](int w) { return sZ[w][wave][lane]; });
-    const double sig = 1.0 / (1.0 + exp(-z_i));
-    sE2[wave][lane] = gate * z_i * sig;
-    sD[wave][lane] = gate * (sig + z_i * sig * (1.0 - sig));
+    readout::activate(gate, z_i, sE2[wave][lane], sD[wave][lane]);
   }
   __syncthreads();
   if (wave == 0) {
-    double e = total([&](int w) { return sE[w][lane]; }) + total([&](int w) { return sE2[w][lane]; });
-    e += __shfl_xor(e, 16);
-    e += __shfl_xor(e, 32);
-    if (here && part == 0) {
-      const double en = scale * e + shift;
-      node_es[node] = en;
-      if (node_total && row_ok) node_total[row] = en + (node_e0 ? node_e0[node] : 0.0);
-    }
+    const double e = total([&](int w) { return sE[w][lane]; }) + total([&](int w) { return sE2[w][lane]; });
+    const double en = readout::node_energy(e, scale, shift);
+    if (here && part == 0) readout::store_energy(readout::Outputs{node_es, feats64, feats_rows, node_e0, node_total}, node, row, row_ok, en);
   }
   if (!d2) return;
+  const double d[4] = {sD[0][lane], sD[1][lane], sD[2][lane], sD[3][lane]};
 #pragma unroll
   for (int u = 0; u < kPieces; ++u) {
     const int p = wave + kMfmaWaves * u;
     if (p >= npieces) break;
-    d4v g{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) g = __builtin_amdgcn_mfma_f64_16x16x4f64(wd[u][i], sD[i][lane], g, 0, 0, 0);
-    if (here)
-      st4(d2 + static_cast<int64_t>(node) * C + 16 * p + 4 * part,
-          f4{static_cast<float>(scale * g[0]), static_cast<float>(scale * g[1]), static_cast<float>(scale * g[2]), static_cast<float>(scale * g[3])});
+    const f4 g = readout::derivative(wd[u], d, scale);
+    if (here) st4(d2 + static_cast<int64_t>(node) * C + 16 * p + 4 * part, g);
   }
 }
 

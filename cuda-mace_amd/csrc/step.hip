@@ -523,11 +523,17 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
     if (t == 0 && glue)
       CM_STAGE(4, cm_node_glue_forward(L.B1, w->prod_WT[0], w->skip_WT, w->up_WT, oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.h1, L.sc,
                                        L.X2, stream));
-    else
+    else if (t == 0 || !glue)
       CM_STAGE(t == 0 ? 4 : 10, cm_linear(B[t], w->prod_WT[t], nullptr, nullptr, N, 1, 0, 1, C, C, 1.0f, none, t == 1 ? L.sc : none, h[t], stream));
   }
-  CM_STAGE(11, cm::readout_forward_with_totals(L.h1, L.h2, w->w1, w->W2a, w->w2b, w->act_cst, w->scale, w->shift, N, C, w->hidden,
-                                               node_energy, want_forces ? L.d_h2 : nullptr, node_feats, g->node_rows, g->node_e0, total_node_energy, st));
+  if (glue)  // with the product linear before the readouts and, for forces, the one behind their derivative
+    CM_STAGE(11, cm::node_head(L.B2, L.sc, L.h1, w->prod_WT[1], w->prod_W[1],
+                               cm::readout::Weights{w->w1, w->W2a, w->w2b, w->act_cst, w->scale, w->shift, w->hidden},
+                               cm::readout::Outputs{node_energy, node_feats, g->node_rows, g->node_e0, total_node_energy}, g->node_weights, N, C,
+                               want_forces ? L.d_h2 : nullptr, L.gB, st));
+  else
+    CM_STAGE(11, cm::readout_forward_with_totals(L.h1, L.h2, w->w1, w->W2a, w->w2b, w->act_cst, w->scale, w->shift, N, C, w->hidden,
+                                                 node_energy, want_forces ? L.d_h2 : nullptr, node_feats, g->node_rows, g->node_e0, total_node_energy, st));
   if (!glue || !want_forces) {  // with the chained kernels the sums ride in the backward chain's launch
     cm::StageTimer timer_(st, 12, timing_mask);
     hipLaunchKernelGGL(cm::segment_sum_f64_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights,
@@ -541,17 +547,17 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // own: the gradient with respect to the second layer's features is -d_h2 (the sign goes into the scale of the two
   // linears that consume it, which is exact; node weights scale its rows first), the one with respect to the first
   // layer's is a constant row (times the node's weight).
-  if (!glue || g->node_weights) {  // the chained kernel forms the constant rows itself
+  if (!glue) {  // the chained kernels form the constant rows themselves and weight the others
     cm::StageTimer timer_(st, 13, timing_mask);
     const dim3 grid(static_cast<unsigned>(std::min<int64_t>(cm::ceil_div(N * C, 256), 2048)));
-    if (!glue)
-      hipLaunchKernelGGL(cm::seed_linear_readout_kernel, grid, dim3(256), 0, st, L.g1, w->w1, w->scale, g->node_weights,
-                         static_cast<int64_t>(N) * C, C);
+    hipLaunchKernelGGL(cm::seed_linear_readout_kernel, grid, dim3(256), 0, st, L.g1, w->w1, w->scale, g->node_weights,
+                       static_cast<int64_t>(N) * C, C);
     if (g->node_weights)
       hipLaunchKernelGGL(cm::weight_rows_kernel, grid, dim3(256), 0, st, L.d_h2, g->node_weights, static_cast<int64_t>(N) * C, C);
   }
   // layer 1 (second interaction)
-  CM_STAGE(14, cm_linear(L.d_h2, w->prod_W[1], nullptr, nullptr, N, 1, 0, 1, C, C, -1.0f, none, none, L.gB, stream));
+  if (!glue)
+    CM_STAGE(14, cm_linear(L.d_h2, w->prod_W[1], nullptr, nullptr, N, 1, 0, 1, C, C, -1.0f, none, none, L.gB, stream));
   CM_STAGE(15, cm_linear(L.bufM2, w->mix_W[1], nullptr, nullptr, N, 1, 0, 16, C, C, w->mix_scale[1], L.gB, none, L.bufA, stream));
   CM_STAGE(16, cm_mp_edge_backward(L.X2, L.vec, w->r_knots, w->spline[1], w->nknots, w->r_width, w->r_max, L.bufA, g->sender,
                               fo_live, g->sender_perm, g->sender_offsets, N, E, C, L.gX2, L.gv2, L.edge_scratch, stream));

@@ -522,6 +522,28 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
     torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
+@pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32)])
+def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
+    """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 32
+    and 64 nodes with a partly filled last one, against the separate launches: bit for bit, for forces and for energies alone,
+    with weights on the node energies and without."""
+    data = make_system(natoms, 4, seed=7, density=None, cluster_box=12.0) if natoms < 130 else make_system(natoms, 4, seed=7, density=0.015)
+    _, model = _build(channels, (1, 6, 7, 8), data, seed=8)
+    dev = to_device(data, "cuda")
+    weighted = dict(dev, node_weights=torch.rand(natoms, generator=torch.Generator().manual_seed(9), dtype=torch.float64).cuda())
+    for inputs, keys in ((dev, {}), (weighted, {}), (dev, {"compute_force": False})):
+        monkeypatch.delenv("CM_STEP_GLUE", raising=False)
+        with torch.set_grad_enabled(not keys):  # energies alone take the library's call with gradients off
+            a = model(dict(inputs), **keys)
+            monkeypatch.setenv("CM_STEP_GLUE", "-1")
+            b = model(dict(inputs), **keys)
+        monkeypatch.delenv("CM_STEP_GLUE")
+        assert model._native not in (None, False)
+        for key in ("node_energy", "node_feats") + (() if keys else ("forces",)):
+            assert torch.equal(a[key], b[key]), key
+        torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
+
+
 @pytest.mark.parametrize("channels", [32, 64, 96, 128, 160, 192, 224, 256])
 def test_repeated_evaluations_agree_bit_for_bit_at_every_width(cabi, channels):
     """Every kernel sums in a fixed order and reads nothing it (or an earlier kernel of the same step) has not written:
