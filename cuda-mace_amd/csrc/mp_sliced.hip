@@ -27,18 +27,22 @@
 // table's pieces at constant offsets from one address); 96 channels 202 / 198 / 187, 192 (40 000) 618 / 600 / 582, 64 channels
 // with ten neighbours 29.3 / 28.4 / 26.3; four orders by exchanges 256 at 128 channels.
 //
-// Everything a step needs from memory is requested ahead, with registers that rotate in three sets so that nothing that
-// a load is still on its way into ever has to be copied (a copy would wait for the load): the sender and vector of a
-// lane's edge three blocks ahead, the X pieces two blocks ahead (what is in flight per compute unit, against the
-// latency of L2 under this load, sets the rate of the X gather), the table pieces of the next step while the current
-// one accumulates.  The instruction scheduler, left to itself, moves each request down to the end of the block (it
-// shortens the life of the landing registers); scheduling barriers keep every request in its step.
+// Everything is requested ahead into registers that the step before has just used up, so that none that a load is still on
+// its way into has to be copied (a copy would wait for the load): the sender and vector of a lane's edge one block ahead, the X
+// piece of an edge when the edge at its place of the block before is done, the table pieces of a channel (both degrees, 32
+// bytes) two channels ahead, as soon as those in their place have been multiplied with X.  That is 168 registers, three
+// waves per SIMD.  With X rows two blocks ahead, prepared edges and vectors in three rotating sets and all pieces of a step
+// together it was 250, and two waves do not cover each other's waits: 25 000 x 52 x 128 246 -> 238 us, 5 000 x 96 50.4 -> 45.9,
+// 10 007 x 160 135 -> 128, 40 000 x 192 610 -> 600, 10 752 x 10 x 64 26.1 -> 21.3 (of which 1.5 by the pieces of the table that a
+// thread stages being requested four at a time), 2 000 x 52 x 128 28.3 -> 26.0, 12 000 x 256 even; with six neighbours 12 000 x 256
+// 63 -> 66.  Of the 238 us 128 channels take 217 with every X row in L1, 231 with edges of one length (no bank conflicts), 188
+// with both.  The instruction scheduler, left to itself, moves each request down to the end of the block (it shortens the life
+// of the landing registers); scheduling barriers keep every request in its place.
 //
 // Receiver nodes differ in their edge counts and the 16 nodes of a wave advance together, so a workgroup sorts its nodes
 // (2 816 at a time) by their number of edge blocks and its waves draw 16 neighbours of that order at a time from a
 // counter in LDS.  Which wave serves a node does not change the node's result: a node's edges are summed in list order, in
-// two chains (even and odd places) that are added up at the end.  The second set of sums takes the last of the register
-// file (252 of 256) and no time; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
+// two chains (even and odd places) that are added up at the end; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
 // with one wave per node: 96 channels 2.68e-7 -> 2.54e-7 (2.70e-7), 128 2.73 -> 2.59 (2.74), 192 2.67 -> 2.52 (2.69), 256
 // 2.81 -> 2.67 (2.83).
 #include <type_traits>
@@ -50,7 +54,7 @@ namespace cm {
 namespace mp {
 namespace {
 
-constexpr int kSlThreads = 512;       // two waves per SIMD (three: 168 registers, equal at 25 000 nodes, 8 % slower at 50 000)
+constexpr int kSlThreads = 768;       // three waves per SIMD, which 168 registers allow
 constexpr unsigned kSlRowBytes = 576;  // of a knot interval: 512 and a quarter of the bank span
 constexpr int kSlMaxIntervals = 272;   // 153 KB of table (one row of it is the row of zeros)
 constexpr int kSlSub = 2816;          // nodes sorted at a time: what LDS holds next to the largest table
@@ -160,65 +164,65 @@ struct Raw {  // what a lane loads for its edge of a block
   float v0, v1, v2;
 };
 
-// q[4 li + d]: (a, b, c, d) of degree li, channel d of the lane's four; `at`: the lane's place in the first row of the table
-template <int J>
-__device__ __forceinline__ void read_pieces(const char *at, unsigned io, f4 (&q)[8]) {
-  const char *row = at + quadu<J>(io);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const f4 *>(row + 64 * i);
-}
-
 template <int J>
 __device__ __forceinline__ void request_row(const float *__restrict__ X, unsigned xo, unsigned place, f4 &x) {
   x = *reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(X) + (quadu<J>(xo) + place));
 }
 
-// Steps J .. 3 of a block: `cur` is the block, xin[j] the X values of the edge of step j; as soon as step j has taken
-// them, the values of step j of the block after next (`fut`) are requested into xout[j].
+// the pieces (a, b, c, d) of channel D of both degrees from the edge's row of the table
+template <int D>
+__device__ __forceinline__ void request_pieces(const char *row, f4 (&q)[2]) {
+  q[0] = *reinterpret_cast<const f4 *>(row + 64 * D);
+  q[1] = *reinterpret_cast<const f4 *>(row + 256 + 64 * D);
+}
+
+// channel D of step J
+template <int P, int J, int D>
+__device__ __forceinline__ void channel(const char *ahead, float xr, float xs, const Gathered &all, f4 (&q)[2], float (&acc)[2][8][4]) {
+  float t[2];
+#pragma unroll
+  for (int li = 0; li < 2; ++li) t[li] = xs * fmaf(xr, fmaf(xr, fmaf(xr, q[li].w, q[li].z), q[li].y), q[li].x);
+  __builtin_amdgcn_sched_barrier(0);
+  request_pieces<(D + 2) % 4>(ahead, q);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[J & 1][i][D] = fmaf(all.y[i][J], t[i < Pair<P>::M0 ? 0 : 1], acc[J & 1][i][D]);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Steps J .. 3 of a block whose first table row starts at `row`; behind step j the X values of the next block's edge at
+// that place are requested into x[j], and from the third channel on the pieces are those of the step after.
 template <int P, int J>
-__device__ __forceinline__ void edge_step(const float *__restrict__ X, const char *tab, const Prepared &cur, const Gathered &all,
-                                          const Prepared &fut, unsigned place, const f4 (&xin)[4], f4 (&xout)[4],
-                                          f4 (&q)[8], float (&acc)[2][8][4]) {
-  const f4 xs = xin[J];
-  request_row<J>(X, fut.xo, place, xout[J]);
-  const float xr = all.xr[J];
-  float y[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) y[i] = all.y[i][J];
-  float t[2][4];
-#pragma unroll
-  for (int li = 0; li < 2; ++li)
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const f4 c = q[4 * li + d];
-      t[li][d] = xs[d] * fmaf(xr, fmaf(xr, fmaf(xr, c.w, c.z), c.y), c.x);
-    }
+__device__ __forceinline__ void edge_step(const float *__restrict__ X, const char *tab, unsigned io, const Gathered &all, const Prepared &nxt,
+                                          unsigned place, const char *row, f4 (&x)[4], f4 (&q)[2][2], float (&acc)[2][8][4]) {
+  const char *next_row = tab + (quadu<(J + 1) % 4>(J < 3 ? io : nxt.io) + place);
+  channel<P, J, 0>(row, all.xr[J], x[J].x, all, q[0], acc);
+  channel<P, J, 1>(row, all.xr[J], x[J].y, all, q[1], acc);
+  channel<P, J, 2>(next_row, all.xr[J], x[J].z, all, q[0], acc);
+  channel<P, J, 3>(next_row, all.xr[J], x[J].w, all, q[1], acc);
+  request_row<J>(X, nxt.xo, place, x[J]);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J + 1 < 4) read_pieces<J + 1>(tab, cur.io, q);
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int d = 0; d < 4; ++d) acc[J & 1][i][d] = fmaf(y[i], t[i < Pair<P>::M0 ? 0 : 1][d], acc[J & 1][i][d]);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J + 1 < 4) edge_step<P, J + 1>(X, tab, cur, all, fut, place, xin, xout, q, acc);
+  if constexpr (J + 1 < 4) edge_step<P, J + 1>(X, tab, io, all, nxt, place, next_row, x, q, acc);
 }
 
 // the rounds of one sorted sub-range: nodes lo + order[0 .. cnt)
 template <int P>
 __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTab, const float *sKnots,
                                            const unsigned short *sOrder, int *sNext, int lo, int cnt, int slice) {
-  const int lane = threadIdx.x % kWave;
-  const int k = lane & 3;         // place in the quad: channels 4 k .. 4 k + 3 of the slice
-  const int gw = lane >> 2;       // node of the wave's round
-  const unsigned place = static_cast<unsigned>(4 * (slice * 16 + 4 * k));  // byte offset of the lane's channels in an X / out row
-  const char *tab = reinterpret_cast<const char *>(sTab) + 16 * k;
+  const int k = threadIdx.x & 3;  // place in the quad: channels 4 k .. 4 k + 3 of the slice
+  const unsigned place = 16u * static_cast<unsigned>(k);  // byte offset of the lane's channels in its slice of an X / out row, and of its pieces in a row of the table
+  const char *tab = reinterpret_cast<const char *>(sTab);
+  const float *X = p.X + 16 * slice;
+  float *out = p.out + 16 * slice;
   const int C = p.C;
   const int last_edge = static_cast<int>(p.nedges) - 1;  // the launcher does not come here without edges
   const unsigned zero_row = static_cast<unsigned>(p.nknots - 1) * kSlRowBytes;
-  const float inv_width = 1.0f / p.r_width;
+  const float inv_width = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, 1.0f / p.r_width)));
 
   for (;;) {
     int base = 0;
+    int lane = threadIdx.x % kWave;
+    asm volatile("" : "+v"(lane));  // as above: formed anew for every round
+    const int gw = lane >> 2;       // node of the wave's round
     if (lane == 0) base = atomicAdd(sNext, kWave / 4);
     base = __builtin_amdgcn_readfirstlane(base);
     if (base >= cnt) break;
@@ -230,9 +234,7 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
       e1 = p.first_occ[p.nnodes + node];
       clamp_edge_range(e0, e1, p.nedges);
     }
-    const int nblk = (e1 - e0 + 3) >> 2;
     const int first_mine = e0 + k;
-    const unsigned own_row = static_cast<unsigned>(node >= 0 ? node : 0) * static_cast<unsigned>(4 * C);
     float acc[2][8][4];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -273,58 +275,39 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
 #pragma unroll
       for (int i = 0; i < 8; ++i) o.y[i] = live ? o.y[i] : 0.f;
       o.xr = live ? len - knot : 0.f;
-      o.xo = live ? __umul24(static_cast<unsigned>(r.s), static_cast<unsigned>(4 * C)) : own_row;  // both below 2^24
+      o.xo = __umul24(static_cast<unsigned>(live ? r.s : max(node, 0)), static_cast<unsigned>(4 * C));  // both below 2^24
       o.io = live ? __umul24(static_cast<unsigned>(idx), kSlRowBytes) : zero_row;
       return o;
     };
-    auto rows = [&](const Prepared &o, f4 (&x)[4]) {
-      request_row<0>(p.X, o.xo, place, x[0]);
-      request_row<1>(p.X, o.xo, place, x[1]);
-      request_row<2>(p.X, o.xo, place, x[2]);
-      request_row<3>(p.X, o.xo, place, x[3]);
-    };
-
-    // three sets that rotate: block b computes from set b % 3 while the rows of block b + 2 are requested into set
-    // (b + 2) % 3 and the raw values of block b + 3 into raw set b % 3
-    Raw r0 = request(0), r1 = request(1), r2 = request(2);
-    Prepared p0 = prepare(r0, 0), p1 = prepare(r1, 1), p2;
-    f4 x0[4], x1[4], x2[4];
-    f4 q[8];
-    Gathered all;
-    rows(p0, x0);
-    rows(p1, x1);
-    for (int blk = 0;; blk += 3) {
-      r0 = request(blk + 3);
+    Raw raw = request(0);
+    Prepared nxt = prepare(raw, 0);
+    raw = request(1);
+    f4 x[4], q[2][2];
+    request_row<0>(X, nxt.xo, place, x[0]);
+    request_row<1>(X, nxt.xo, place, x[1]);
+    request_row<2>(X, nxt.xo, place, x[2]);
+    request_row<3>(X, nxt.xo, place, x[3]);
+    const char *row = tab + (quadu<0>(nxt.io) + place);
+    request_pieces<0>(row, q[0]);
+    request_pieces<1>(row, q[1]);
+    for (int blk = 0;; ++blk) {
+      const Prepared cur = nxt;
+      nxt = prepare(raw, blk + 1);  // before the gathering: fewer values live at a time
       __builtin_amdgcn_sched_barrier(0);
-      p2 = prepare(r2, blk + 2);
-      read_pieces<0>(tab, p0.io, q);
-      all = gather(p0);
+      raw = request(blk + 2);
+      const Gathered all = gather(cur);
       __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p0, all, p2, place, x0, x2, q, acc);
-      if (!__any(blk + 1 < nblk)) break;
-      r1 = request(blk + 4);
-      __builtin_amdgcn_sched_barrier(0);
-      p0 = prepare(r0, blk + 3);
-      read_pieces<0>(tab, p1.io, q);
-      all = gather(p1);
-      __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p1, all, p0, place, x1, x0, q, acc);
-      if (!__any(blk + 2 < nblk)) break;
-      r2 = request(blk + 5);
-      __builtin_amdgcn_sched_barrier(0);
-      p1 = prepare(r1, blk + 4);
-      read_pieces<0>(tab, p2.io, q);
-      all = gather(p2);
-      __builtin_amdgcn_sched_barrier(0);
-      edge_step<P, 0>(p.X, tab, p2, all, p1, place, x2, x1, q, acc);
-      if (!__any(blk + 3 < nblk)) break;
+      edge_step<P, 0>(X, tab, cur.io, all, nxt, place, tab + (quadu<0>(cur.io) + place), x, q, acc);
+      if (!__any(first_mine + 4 * (blk + 1) < e1)) break;  // the first lane of a quad tells for all four
     }
 
     if (node >= 0) {
-      char *op = reinterpret_cast<char *>(p.out + static_cast<int64_t>(node) * 16 * C);
+      unsigned at = place;
+      asm volatile("" : "+v"(at));  // keeps the address out of the registers of the edge loop
+      char *op = reinterpret_cast<char *>(out + static_cast<int64_t>(node) * 16 * C) + at;
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        *reinterpret_cast<f4 *>(op + static_cast<int64_t>(Pair<P>::row(i)) * (4 * C) + place) =
+        *reinterpret_cast<f4 *>(op + static_cast<int64_t>(Pair<P>::row(i)) * (4 * C)) =
             f4{acc[0][i][0] + acc[1][i][0], acc[0][i][1] + acc[1][i][1], acc[0][i][2] + acc[1][i][2], acc[0][i][3] + acc[1][i][3]};
     }
   }
@@ -366,31 +349,44 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
   // (a, b, c, d) together
   constexpr int kRow = kSlRowBytes / 4;
   const int intervals = p.nknots - 1;
-  for (int i = tid; i < intervals * 32; i += kSlThreads) {
-    const int idx = i >> 5, coef = (i >> 3) & 3, li = (i >> 2) & 1, k = i & 3;
-    const int l = pair == 0 ? (li == 0 ? 0 : 3) : (li == 0 ? 1 : 2);
-    const f4 v = ld4(p.coeffs + (static_cast<int64_t>(idx * 4 + coef) * 4 + l) * p.C + slice * 16 + 4 * k);
-    float *dst = sTab + idx * kRow + 64 * li + 4 * k + coef;
-    dst[0] = v.x;
-    dst[16] = v.y;
-    dst[32] = v.z;
-    dst[48] = v.w;
+  constexpr int kAhead = 4;  // pieces of a thread requested together
+  for (int i0 = tid; i0 < intervals * 32; i0 += kAhead * kSlThreads) {
+    f4 v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = min(i0 + u * kSlThreads, intervals * 32 - 1);
+      const int idx = i >> 5, coef = (i >> 3) & 3, li = (i >> 2) & 1, k = i & 3;
+      const int l = pair == 0 ? (li == 0 ? 0 : 3) : (li == 0 ? 1 : 2);
+      v[u] = ld4(p.coeffs + (static_cast<int64_t>(idx * 4 + coef) * 4 + l) * p.C + slice * 16 + 4 * k);
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = min(i0 + u * kSlThreads, intervals * 32 - 1);  // beyond the table: the last piece once more
+      const int idx = i >> 5, coef = (i >> 3) & 3, li = (i >> 2) & 1, k = i & 3;
+      float *dst = sTab + idx * kRow + 64 * li + 4 * k + coef;
+      dst[0] = v[u].x;
+      dst[16] = v[u].y;
+      dst[32] = v[u].z;
+      dst[48] = v[u].w;
+    }
   }
   for (int i = tid; i < 128; i += kSlThreads) sTab[intervals * kRow + i] = 0.f;  // the row of edges that do not count
   for (int i = tid; i < p.nknots; i += kSlThreads) sKnots[i] = p.knots[i];
 
   for (int sub = lo; sub < hi; sub += kSlSub) {
     const int cnt = min(kSlSub, hi - sub);
+    int here = tid;  // opaque: what the sort derives from it is formed anew for every sub-range, not kept through the rounds
+    asm volatile("" : "+v"(here));
     __syncthreads();  // every wave has left the previous sub-range (and the table is staged)
-    if (tid < kSlBins) sHist[tid] = 0;
-    if (tid == 0) sNext = 0;
+    if (here < kSlBins) sHist[here] = 0;
+    if (here == 0) sNext = 0;
     __syncthreads();
     // counting sort by the number of edge blocks, most blocks first
     constexpr int kPerThread = (kSlSub + kSlThreads - 1) / kSlThreads;
     int bin[kPerThread];
 #pragma unroll
     for (int q = 0; q < kPerThread; ++q) {
-      const int i = tid + q * kSlThreads;
+      const int i = here + q * kSlThreads;
       bin[q] = -1;
       if (i < cnt) {
         int e0 = p.first_occ[sub + i], e1 = p.first_occ[p.nnodes + sub + i];
@@ -400,7 +396,7 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
       }
     }
     __syncthreads();
-    if (tid == 0) {
+    if (here == 0) {
       int run = 0;
       for (int b = 0; b < kSlBins; ++b) {
         const int n = sHist[b];
@@ -411,7 +407,7 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kPerThread; ++q)
-      if (bin[q] >= 0) sOrder[atomicAdd(&sHist[bin[q]], 1)] = static_cast<unsigned short>(tid + q * kSlThreads);
+      if (bin[q] >= 0) sOrder[atomicAdd(&sHist[bin[q]], 1)] = static_cast<unsigned short>(here + q * kSlThreads);
     __syncthreads();
     if (pair == 0)
       run_rounds<0>(p, sTab, sKnots, sOrder, &sNext, sub, cnt, slice);
