@@ -78,14 +78,14 @@ def traffic_of(table, kernels):
     return None if any(p is None for p in parts) else sum(parts)
 
 
-def forward_kernel_name(C, N, E):
+def forward_kernel_name(C, N, E, in_step=False):
     """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_sliced.hip: sliced_forward_applies; the
-    benchmark's spline table has 256 knots)."""
+    benchmark's spline table has 256 knots; the one-call step hands it an edge's vector and sender as one record)."""
     share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
     enough = {32: 0, 64: 120000 - 10 * N, 96: 65000 + 2 * N, 128: 50000 + 5 * N // 2, 160: 17000 + 5 * N // 2,
               192: 14000 + 11 * N // 2, 224: 8000 + 3 * N}.get(C, 8000 + 5 * N)
     if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
-        return "mp_edge_forward_sliced_kernel"
+        return "mp_edge_forward_sliced_kernel<%s>" % ("true" if in_step else "false")
     return "mp_spline_forward_kernel<%d,true>" % C
 
 
@@ -515,7 +515,7 @@ def main():
         sh_b, spline_b = 88 * E, 4 * (8 * E * C + E)  # harmonics backward, spline backward (each operand once)
         sh_f, spline_f = 76 * E, 4 * (E + 8 * E * C)  # harmonics forward, spline forward (each operand once)
         flops_fwd = 60 * E * C  # per edge and channel: the cubic of 4 degrees (12 FMA), 4 products, 16 accumulations
-        roofline = entry(forward_kernel_name(C, N, E), fwd_fb, t_fwd, launches_timed=launches(fwd_name),
+        roofline = entry(forward_kernel_name(C, N, E, native), fwd_fb, t_fwd, launches_timed=launches(fwd_name),
                          note="dominant kernel of the step by total time (two launches per step). Harmonics and radial "
                               "weights are evaluated in-kernel, so its own HBM operands are small; a workgroup keeps its "
                               "part of the spline table (two degrees x 16 channels, 130 KB) in LDS, so the coefficients "

@@ -284,12 +284,18 @@ int launch_sender_pass(int channels, const float *gXe, const int32_t *perm, cons
                        int64_t nedges, float *gX, hipStream_t st, const float *live_vec = nullptr,
                        const float *live_r = nullptr, float r_max = 0.f);
 
-// Forward from edge vectors with the radial table in LDS, one degree and one 32-channel slice per workgroup (defined in
-// mp_sliced.hip): whether it takes a launch of this shape, and the launch.
+// Forward from edge vectors with the radial table in LDS, two degrees and one 16-channel slice per workgroup (defined in
+// mp_sliced.hip): whether it takes a launch of this shape, and the launch.  records: NULL, or per edge 16 bytes, the vector and
+// the sender (at most kMaxRecords edges), from which it reads instead of from vec and sender.
+constexpr int64_t kMaxRecords = UINT32_MAX / 16;  // 32-bit byte offsets
 bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nknots);
-int launch_sliced_forward(const float *X, const float *vec, const float *knots, const float *coeffs, int nknots, float r_width,
-                          float r_max, const int32_t *sender, const int32_t *first_occ, int64_t nnodes, int64_t nedges,
+int launch_sliced_forward(const float *X, const float *vec, const void *records, const float *knots, const float *coeffs, int nknots,
+                          float r_width, float r_max, const int32_t *sender, const int32_t *first_occ, int64_t nnodes, int64_t nedges,
                           int channels, float *out, hipStream_t st);
+
+// cm_mp_edge_forward of a caller that has written records (defined in mp_spline.hip; operands already checked by the caller).
+int edge_forward_from_records(const float *X, const void *records, const float *r_knots, const float *coeffs, int nknots, float r_width,
+                              float r_max, const int32_t *first_occ, int64_t nnodes, int64_t nedges, int channels, float *out, hipStream_t st);
 
 // The spline-fused backward edge pass from edge vectors without gX, writing (this layer's vector gradient + addend[e])
 // (defined in mp_spline.hip; operands as cm_mp_edge_backward, already checked by the caller).

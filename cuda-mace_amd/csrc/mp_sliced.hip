@@ -90,8 +90,11 @@ inline int64_t min_edges(int64_t nnodes, int channels) {
 }
 inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)
 
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+
 struct SlicedArgs {
   const float *X, *vec;
+  const u4 *records;  // per edge the vector and, as bits, the sender (then vec and sender are not read), or NULL
   const int32_t *sender, *first_occ;
   const float *coeffs, *knots;
   int nknots;
@@ -205,7 +208,7 @@ __device__ __forceinline__ void edge_step(const float *__restrict__ X, const cha
 }
 
 // the rounds of one sorted sub-range: nodes lo + order[0 .. cnt)
-template <int P>
+template <int P, bool RECORDS>
 __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTab, const float *sKnots,
                                            const unsigned short *sOrder, int *sNext, int lo, int cnt, int slice) {
   const int k = threadIdx.x & 3;  // place in the quad: channels 4 k .. 4 k + 3 of the slice
@@ -245,6 +248,10 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
     // branch would make the later waits cover everything in flight.
     auto request = [&](int blk) {
       const unsigned e = static_cast<unsigned>(min(first_mine + 4 * blk, last_edge));
+      if constexpr (RECORDS) {
+        const u4 v = *reinterpret_cast<const u4 *>(reinterpret_cast<const char *>(p.records) + 16u * e);
+        return Raw{static_cast<int>(v[3]), __uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2])};
+      }
       const float *v = reinterpret_cast<const float *>(reinterpret_cast<const char *>(p.vec) + 12u * e);
       return Raw{*reinterpret_cast<const int *>(reinterpret_cast<const char *>(p.sender) + 4u * e), v[0], v[1], v[2]};
     };
@@ -313,6 +320,7 @@ __device__ __forceinline__ void run_rounds(const SlicedArgs &p, const float *sTa
   }
 }
 
+template <bool RECORDS>
 __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(const SlicedArgs p) {
   __shared__ __attribute__((aligned(16))) float sTab[kSlMaxIntervals * (kSlRowBytes / 4)];
   __shared__ float sKnots[kSlMaxIntervals + 1];
@@ -410,9 +418,9 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
       if (bin[q] >= 0) sOrder[atomicAdd(&sHist[bin[q]], 1)] = static_cast<unsigned short>(here + q * kSlThreads);
     __syncthreads();
     if (pair == 0)
-      run_rounds<0>(p, sTab, sKnots, sOrder, &sNext, sub, cnt, slice);
+      run_rounds<0, RECORDS>(p, sTab, sKnots, sOrder, &sNext, sub, cnt, slice);
     else
-      run_rounds<1>(p, sTab, sKnots, sOrder, &sNext, sub, cnt, slice);
+      run_rounds<1, RECORDS>(p, sTab, sKnots, sOrder, &sNext, sub, cnt, slice);
   }
 }
 
@@ -425,13 +433,17 @@ bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nk
          nnodes * channels < (int64_t{1} << 30) && nedges <= UINT32_MAX / 12 && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }
 
-int launch_sliced_forward(const float *X, const float *vec, const float *knots, const float *coeffs, int nknots, float r_width,
-                          float r_max, const int32_t *sender, const int32_t *first_occ, int64_t nnodes, int64_t nedges,
+int launch_sliced_forward(const float *X, const float *vec, const void *records, const float *knots, const float *coeffs, int nknots,
+                          float r_width, float r_max, const int32_t *sender, const int32_t *first_occ, int64_t nnodes, int64_t nedges,
                           int channels, float *out, hipStream_t st) {
-  SlicedArgs a{X, vec, sender, first_occ, coeffs, knots, nknots, r_width, r_max, static_cast<int>(nnodes), nedges, channels, out,
-               channels / 16, 0};
+  SlicedArgs a{X, vec, static_cast<const u4 *>(records), sender, first_occ, coeffs, knots, nknots, r_width, r_max, static_cast<int>(nnodes), nedges,
+               channels, out, channels / 16, 0};
   a.share = share_of(channels);
-  hipLaunchKernelGGL(mp_edge_forward_sliced_kernel, dim3(static_cast<unsigned>(a.share * 2 * a.nslices)), dim3(kSlThreads), 0, st, a);
+  const dim3 grid(static_cast<unsigned>(a.share * 2 * a.nslices));
+  if (records)
+    hipLaunchKernelGGL(mp_edge_forward_sliced_kernel<true>, grid, dim3(kSlThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(mp_edge_forward_sliced_kernel<false>, grid, dim3(kSlThreads), 0, st, a);
   return check_launch("cm_mp_edge_forward");
 }
 

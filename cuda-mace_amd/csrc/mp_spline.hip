@@ -961,7 +961,7 @@ extern "C" int cm_mp_edge_forward(const float *X, const float *vectors, const fl
   int rc = cm::check_spline("cm_mp_edge_forward", vectors, r_knots, coeffs, nknots, r_width, nedges, nnodes, channels);
   if (rc != CM_OK) return rc;
   if (cm::mp::sliced_forward_applies(nnodes, nedges, channels, nknots))
-    return cm::mp::launch_sliced_forward(X, vectors, r_knots, coeffs, nknots, r_width, r_max, sender, first_occ, nnodes, nedges,
+    return cm::mp::launch_sliced_forward(X, vectors, nullptr, r_knots, coeffs, nknots, r_width, r_max, sender, first_occ, nnodes, nedges,
                                          channels, out, cm::as_stream(stream));
   const cm::Spline sp{vectors, nullptr, r_knots, coeffs, nknots, r_width, r_max};
   rc = CM_EINVAL;
@@ -971,6 +971,13 @@ extern "C" int cm_mp_edge_forward(const float *X, const float *vectors, const fl
 
 namespace cm {
 namespace mp {
+
+int edge_forward_from_records(const float *X, const void *records, const float *r_knots, const float *coeffs, int nknots, float r_width,
+                              float r_max, const int32_t *first_occ, int64_t nnodes, int64_t nedges, int channels, float *out, hipStream_t st) {
+  const int rc = check_spline("cm_mace_step", static_cast<const float *>(records), r_knots, coeffs, nknots, r_width, nedges, nnodes, channels);
+  if (rc != CM_OK) return rc;
+  return launch_sliced_forward(X, nullptr, records, r_knots, coeffs, nknots, r_width, r_max, nullptr, first_occ, nnodes, nedges, channels, out, st);
+}
 
 // cm_mp_edge_backward without gX whose vector gradient is written as (this layer's gradient + addend[e]): saves the pass
 // that adds two layers' gradients of the same edge vectors.  Arguments as checked by the caller (cm_mace_step).

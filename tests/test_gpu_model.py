@@ -466,6 +466,14 @@ def test_energy_stays_inside_its_workspace(cabi, atoms, C):
     assert cabi.lib.cm_mace_energy(*args) == -28
 
 
+@pytest.mark.parametrize("atoms,C", [(5200, 32), (2700, 64)])
+def test_energy_with_and_without_room_for_edge_records(cabi, atoms, C):
+    """The forward with the table in LDS reads 16-byte records; for energies alone they lie where vectors and h2 are, which takes
+    no more neighbours than channels: 70 on 32 channels (vectors and senders are read instead) and on 64, inside the workspace
+    and with the bits of the full step, which always has room for them."""
+    test_energy_stays_inside_its_workspace(cabi, atoms, C)
+
+
 @pytest.mark.parametrize("relabel", [True, False], ids=["shell_last", "shell_in_place"])
 def test_native_step_on_a_list_with_a_skin(cabi, relabel):
     """A neighbour list built out to cutoff + skin, at a size where the forward runs the LDS-table kernel: the step walks
