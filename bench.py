@@ -206,7 +206,8 @@ def op_cases(torch, cabi, N, E, C, ne, rcv, snd, with_fused=True, with_node_ops=
             ("spline forward (R only)", "spline_forward_sliced_kernel" if E >= 1 << 15 else "spline_forward_kernel<false>",
              4 * (E + 4 * E * C),
              lambda: cabi.spline_forward(r, knots, coeffs, float(h), 5.0)),
-            ("spline backward", "spline_backward_sliced_kernel" if E >= 1 << 15 else "spline_backward_kernel",
+            ("spline backward", "spline_backward_sliced_kernel" if E >= 1 << 19 else
+             ("spline_backward_sorted_kernel<%d>" % min(-(-C // 32), 4) if E >= 1 << 15 else "spline_backward_kernel"),
              4 * (4 * E * C + 2 * E),
              lambda: cabi.spline_backward(r, knots, coeffs, R.view(E, 4 * C), float(h), 5.0)),
             ("symmetric contraction forward + gradient", "symcon_lmax3_kernel<float,true>", 4 * (33 * N * C + N),

@@ -149,9 +149,142 @@ __global__ __launch_bounds__(256) void spline_backward_kernel(
   if (lane == 0) gr[e] = sum;
 }
 
-// ---- LDS-table variant of the backward for long edge lists -------------------------------------------------------
-// As in the forward, the kernel above reads 48 bytes of coefficients through L1 for every 16 bytes of the gradient
-// stream.  Here a workgroup owns a chunk of consecutive edges and sums them slice by slice: for each slice of 32
+// ---- backward from 32 768 edges on: edges in the order of their knot intervals --------------------------------------
+// The kernel above reads 48 bytes of coefficients for every 16 bytes of the gradient stream, from L2, and that traffic is what
+// bounds it.  Here a workgroup of 16 waves, one per compute unit, takes a
+// chunk of consecutive edges and serves them in the order of their intervals (a counting sort in LDS): the edges it works
+// on at a time share a few rows of the table, which stay in L1.  Half a wave serves an edge, ITER 16-byte pieces of the row
+// per lane, all of them requested before the first is used (up to 512 outputs: beyond, 512 at a time; two edges at a time
+// where a row is one piece per lane: 122 880 x 128 29.7 -> 18.9 us).  An edge's sum does not depend on its place in the order.
+// Measured (edges x outputs, us), one wave per edge / the LDS-table kernel below / this one: 33 000 x 256 13.8 / 41.5 / 11.7, 33 000 x
+// 512 20.5 / 80.7 / 20.3, 122 880 x 128 40.5 / 26.0 / 18.9, 122 880 x 384 62.0 / 72.3 / 46.4 (its stream alone 35.6), 122 880 x 1 024 133 /
+// 235 / 120, 300 000 x 512 165 / 170 / 137, 400 000 x 128 133 / 55 / 53, 600 000 x 128 199 / 73 / 78, 600 000 x 1 024 642 / 611 / 554, 900 000 x
+// 512 493 / 390 / 411, 1 300 000 x 512 707 / 526 / 590.  Error against fp64 8.0e-8 to 9.8e-8, the LDS-table kernel's 7.9e-8 to 1.3e-7.
+constexpr int kSpSortThreads = 1024;
+constexpr int kSpSortChunk = 4096;  // edges of a chunk: their place in it takes 12 bits
+constexpr int kSpSortBins = 256;
+constexpr int kSpSortMaxKnots = 1 << 20;  // the interval takes the other 20 bits of a word
+
+template <int ITER>
+__global__ __launch_bounds__(kSpSortThreads) void spline_backward_sorted_kernel(
+    const float *__restrict__ r, const float *__restrict__ r_knots, const float *__restrict__ coeffs,
+    const float *__restrict__ gR, int64_t nedges, int nknots, int J, float r_width, float r_max, float *__restrict__ gr, int chunk) {
+  __shared__ float sX[kSpSortChunk];
+  __shared__ unsigned sEdge[kSpSortChunk];  // interval << 12 | place in the chunk
+  __shared__ __attribute__((aligned(16))) int sHist[kSpSortBins];
+  __shared__ int sCount;
+  constexpr int kPer = kSpSortChunk / kSpSortThreads;
+  const int tid = threadIdx.x;
+  const int lane = tid % 32, slot = tid / 32;  // an edge's lanes
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * chunk;
+  const int n = static_cast<int>(min(static_cast<int64_t>(chunk), nedges - c0));
+  if (tid < kSpSortBins) sHist[tid] = 0;
+  __syncthreads();
+  int bin[kPer];
+  unsigned word[kPer];
+  float x[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int i = tid + q * kSpSortThreads;
+    bin[q] = -1;
+    if (i >= n) continue;
+    const float re = r[c0 + i];
+    if (re <= r_max) {
+      const int idx = knot_index(re, r_width, nknots);
+      x[q] = re - r_knots[idx];
+      word[q] = static_cast<unsigned>(idx) << 12 | static_cast<unsigned>(i);
+      bin[q] = idx * kSpSortBins / (nknots - 1);
+      atomicAdd(&sHist[bin[q]], 1);
+    } else {
+      gr[c0 + i] = 0.f;
+    }
+  }
+  __syncthreads();
+  if (tid < kWave) {  // places of the bins, four per lane
+    int4 c = reinterpret_cast<int4 *>(sHist)[tid];
+    const int mine = c.x + c.y + c.z + c.w;
+    int upto = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int below = __shfl_up(upto, d);
+      upto += tid >= d ? below : 0;
+    }
+    const int first = upto - mine;
+    reinterpret_cast<int4 *>(sHist)[tid] = make_int4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
+    if (tid == kWave - 1) sCount = upto;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    if (bin[q] < 0) continue;
+    const int at = atomicAdd(&sHist[bin[q]], 1);
+    sX[at] = x[q];
+    sEdge[at] = word[q];
+  }
+  __syncthreads();
+
+  constexpr int kEdges = ITER == 1 ? 2 : 1;  // of a slot at a time
+  const int count = sCount;
+  for (int p = kEdges * slot; p < count; p += kEdges * (kSpSortThreads / 32)) {
+    unsigned w[kEdges];
+    float xs[kEdges];
+    int64_t e[kEdges];
+    f4 acc[kEdges];
+#pragma unroll
+    for (int u = 0; u < kEdges; ++u) {
+      const int at = min(p + u, count - 1);  // beyond the last edge: the last one once more
+      w[u] = sEdge[at], xs[u] = sX[at];
+      e[u] = c0 + (w[u] & (kSpSortChunk - 1));
+      acc[u] = zero4();
+    }
+    for (int j0 = 0; j0 < J; j0 += 128 * ITER) {
+      f4 g[kEdges][ITER], b[kEdges][ITER], c[kEdges][ITER], d[kEdges][ITER];
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u) {
+        const float *cp = coeffs + (static_cast<int64_t>(w[u] >> 12) * 4 + 1) * J, *gp = gR + e[u] * J;
+#pragma unroll
+        for (int i = 0; i < ITER; ++i) {
+          const int j = j0 + 128 * i + 4 * lane, at = j < J ? j : 0;
+          g[u][i] = ld4_stream(gp + at), b[u][i] = ld4(cp + at), c[u][i] = ld4(cp + J + at), d[u][i] = ld4(cp + 2 * J + at);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u)
+#pragma unroll
+        for (int i = 0; i < ITER; ++i) {
+          const f4 v = g[u][i] * (b[u][i] + xs[u] * (2.f * c[u][i] + (3.f * xs[u]) * d[u][i]));
+          acc[u] += j0 + 128 * i + 4 * lane < J ? v : zero4();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kEdges; ++u) {
+      float sum = hsum4(acc[u]);
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+      if (lane == 0) gr[e[u]] = sum;
+    }
+  }
+}
+
+void launch_spline_backward_sorted(const float *r, const float *r_knots, const float *coeffs, const float *gR, int64_t nedges,
+                                   int nknots, int J, float r_width, float r_max, float *gr, hipStream_t st) {
+  const int64_t cus = device_compute_units();
+  const int64_t rounds = ceil_div(nedges, cus * kSpSortChunk);  // chunks per compute unit
+  const int chunk = static_cast<int>(ceil_div(nedges, cus * rounds));
+  const dim3 grid(static_cast<unsigned>(ceil_div(nedges, chunk))), block(kSpSortThreads);
+#define CM_SORTED(ITER_) \
+  hipLaunchKernelGGL(spline_backward_sorted_kernel<ITER_>, grid, block, 0, st, r, r_knots, coeffs, gR, nedges, nknots, J, r_width, r_max, gr, chunk)
+  switch (std::min<int64_t>(ceil_div(J, 128), 4)) {
+    case 1: CM_SORTED(1); break;
+    case 2: CM_SORTED(2); break;
+    case 3: CM_SORTED(3); break;
+    default: CM_SORTED(4); break;
+  }
+#undef CM_SORTED
+}
+
+// ---- LDS-table variant of the backward for the longest edge lists --------------------------------------------------
+// Even in the order of the intervals the coefficients pass through L1, 48 bytes for every 16 of the gradient stream.  Here a workgroup owns a chunk of consecutive edges and sums them slice by slice: for each slice of 32
 // outputs it loads the derivative's coefficients (b, 2c, 3d per interval: 384 bytes, 104 KB at most) into LDS, streams
 // that slice of its edges' gradient rows (one 128-byte line per edge) and adds each edge's partial sum to the edge's
 // cell in LDS; after the last slice the cells go to grad_r.  One lane group adds to a cell per slice, and the slices
@@ -160,6 +293,7 @@ __global__ __launch_bounds__(256) void spline_backward_kernel(
 // the bytes of the gradient stream at 5 000 edges per chunk.
 constexpr int kSpBwdRow = 3 * kSpSlice;  // floats per interval
 constexpr int kSpBwdChunk = 8192;        // edges per chunk at most (their sums: 32 KB of LDS)
+constexpr int64_t kSpBwdMinEdges = 1 << 19;  // below, loading the slices costs more than it saves: see the kernel above
 
 __global__ __launch_bounds__(kSpThreads) void spline_backward_sliced_kernel(
     const float *__restrict__ r, const float *__restrict__ r_knots, const float *__restrict__ coeffs,
@@ -331,8 +465,13 @@ extern "C" int cm_spline_backward(const float *r, const float *r_knots, const fl
   CM_REQUIRE(r_width > 0.f, "cm_spline_backward: r_width must be positive");
   if (nedges == 0) return CM_OK;
   CM_REQUIRE(r && r_knots && coeffs && grad_R && grad_r, "cm_spline_backward: NULL pointer");
-  if (cm::spline_sliced_applies(nedges, nknots, noutputs)) {
+  if (nedges >= cm::kSpBwdMinEdges && cm::spline_sliced_applies(nedges, nknots, noutputs)) {
     cm::launch_spline_backward_sliced(r, r_knots, coeffs, grad_R, nedges, nknots, noutputs, r_width, r_max, grad_r,
+                                      cm::as_stream(stream));
+    return cm::check_launch("cm_spline_backward");
+  }
+  if (nedges >= cm::kSpMinEdges && nknots <= cm::kSpSortMaxKnots) {
+    cm::launch_spline_backward_sorted(r, r_knots, coeffs, grad_R, nedges, nknots, noutputs, r_width, r_max, grad_r,
                                       cm::as_stream(stream));
     return cm::check_launch("cm_spline_backward");
   }

@@ -271,8 +271,8 @@ def test_sh_forward_backward(cabi, E, seed):
 # ------------------------------------------------------------------------------------------------
 # spline
 # ------------------------------------------------------------------------------------------------
-# from 32 768 edges on the forward without derivative and the backward run on their LDS-table kernels: full rows of
-# slices, a last slice of 8 of 32 outputs, and more edges than one pass of chunks holds (256 workgroups x 8 192)
+# from 32 768 edges on the forward without derivative, from 524 288 on the backward run on their LDS-table kernels: full rows
+# of slices, a last slice of 8 of 32 outputs, and more edges than one pass of chunks holds (256 workgroups x 8 192)
 @pytest.mark.parametrize("E,J,seed", [(1, 128, 0), (777, 384, 1), (5000, 512, 2), (300, 768, 3), (40_000, 512, 4),
                                       (70_001, 72, 5), (2_200_003, 8, 6)])
 def test_spline_forward_backward(cabi, E, J, seed):
@@ -304,6 +304,39 @@ def test_spline_forward_backward(cabi, E, J, seed):
     bound = 5e-6 * (gR.abs() * der_ref.abs()).sum(-1) + 1e-30
     assert bool(((gr.double().cpu() - gr_ref).abs() <= bound).all())
     assert float(val[(r32 > r_max).to(DEV)].abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("E,J,nknots", [(32_768, 128, 256), (33_001, 132, 256), (40_000, 4, 2), (50_003, 260, 3), (34_567, 516, 2000),
+                                        (32_769, 1028, 300), (524_287, 8, 256), (1_100_003, 4, 300)])
+def test_spline_backward_in_the_order_of_the_intervals(cabi, E, J, nknots):
+    """Rows of one to nine groups of 128 outputs with a partly filled last one, tables of one interval, of more than there are bins
+    and of more than the LDS-table kernel takes (two chunks per compute unit then); edges beyond the cutoff give zero whatever
+    their gradient.  fp32 against fp64: per term four roundings of the cubic's derivative, one of the product and, with a lane's
+    chain of up to nine and a tree, at most 18 of the sum, 2^-24 each; 5e-6 (84 of them) of the sum of the magnitudes of b, 2 c x and
+    3 d x^2 times the gradient, which the cancellation inside the derivative is measured against."""
+    _say("spline backward sorted", E, J, nknots)
+    g = torch.Generator().manual_seed(E + J)
+    r_max = 5.0
+    knots = torch.linspace(0.0, 6.0, nknots, dtype=torch.float64)
+    h = 6.0 / (nknots - 1)
+    coeffs = torch.randn(nknots - 1, 4, J, generator=g, dtype=torch.float64) / torch.tensor([1.0, h, h ** 2, h ** 3], dtype=torch.float64)[None, :, None]
+    coeffs = coeffs.float().double()
+    r32 = (torch.rand(E, generator=g, dtype=torch.float64) * 5.6 + 0.2).float()
+    gR = torch.randn(E, J, generator=g).double()
+    gR[r32 > r_max] = float("nan")
+    gr = cabi.spline_backward(r32.to(DEV), knots.float().to(DEV), coeffs.float().to(DEV), gR.float().to(DEV), h, r_max).double().cpu()
+    idx = (r32 / torch.tensor(h, dtype=torch.float32)).long().clamp(0, nknots - 2)  # the kernels' lookup, in fp32
+    x = (r32 - knots.float()[idx]).double()[:, None]
+    live = r32 <= r_max
+    for lo in range(0, E, 100_000):
+        s = slice(lo, min(lo + 100_000, E))
+        c = coeffs[idx[s]]
+        terms = [c[:, 1], 2 * c[:, 2] * x[s], 3 * c[:, 3] * x[s] ** 2]
+        ref = (gR[s] * (terms[0] + terms[1] + terms[2])).sum(-1)
+        bound = 5e-6 * (gR[s].abs() * sum(t.abs() for t in terms)).sum(-1)
+        ok = live[s]
+        assert bool(((gr[s] - ref).abs()[ok] <= bound[ok]).all())
+        assert float(gr[s][~ok].abs().sum()) == 0.0
 
 
 # ------------------------------------------------------------------------------------------------
