@@ -158,6 +158,23 @@ def test_spline_f64(cabi, E, J, seed):
     assert float(val[(r > r_max).to(DEV)].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("E,J,seed", [(2047, 130, 11), (2048, 130, 12), (2049, 2, 13), (5001, 256, 14), (3001, 33, 15), (4000, 640, 16)])
+def test_spline_f64_one_and_two_outputs_per_lane(cabi, E, J, seed):
+    """As above on both sides of the two rules (2 048 edges, odd rows); rows that start between 16-byte boundaries give the values
+    that aligned ones do."""
+    test_spline_f64(cabi, E, J, seed)
+    g = torch.Generator().manual_seed(seed)
+    knots = torch.linspace(0.0, 6.0, 64, dtype=F64, device=DEV)
+    h, r = float(knots[1]), (torch.rand(E, generator=g, dtype=F64) * 5.6).to(DEV)
+    odd = lambda n, *shape: torch.randn(n + 1, generator=g, dtype=F64).to(DEV)[1:].view(*shape)
+    coeffs, gR = odd(63 * 4 * J, 63, 4, J), odd(E * J, E, J)
+    assert coeffs.data_ptr() % 16 == 8 and gR.data_ptr() % 16 == 8
+    assert torch.equal(cabi.spline_forward(r, knots, coeffs, h, 5.0), cabi.spline_forward(r, knots, coeffs.clone(), h, 5.0))
+    mine, aligned = cabi.spline_backward(r, knots, coeffs, gR, h, 5.0), cabi.spline_backward(r, knots, coeffs.clone(), gR.clone(), h, 5.0)
+    scale = torch.linalg.vector_norm(gR, dim=1) * 40.0 * J ** 0.5  # of the terms: |b + 2 c x + 3 d x^2| below 10, the sum of J of them
+    assert bool(((mine - aligned).abs() <= 1e-15 * scale + 1e-300).all())  # sums of J terms in two orders
+
+
 def _symcon_module(ne, C, seed):
     from cuda_mace.models.upstream_like import _SymmetricContraction
     from cuda_mace.ops.symmetric_contraction import SymmetricContraction
