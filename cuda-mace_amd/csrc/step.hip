@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "geometry.hpp"
 #include "mp_common.hpp"
 #include "node_glue.hpp"
 #include "readout.hpp"
@@ -252,36 +253,8 @@ __global__ __launch_bounds__(kSumThreads) void segment_sum_f64_kernel(const doub
 
 // Virials from the per-edge gradients the backward chain ends with: under a symmetric strain every edge vector becomes
 // vec + vec . strain, so -dE/d strain = 1/2 sum_e (vec_e (x) gv_e + gv_e (x) vec_e) with gv_e = -dE/d vec_e, which is what
-// the chain delivers.  Two levels, both in a fixed order: per receiver node (eight lanes share a node's edges), then per
-// graph.  node_virial [nnodes, 6]: xx, yy, zz, yz, xz, xy.
-__global__ __launch_bounds__(256) void node_virial_kernel(const float *__restrict__ vec, const float *__restrict__ gv,
-                                                          const int32_t *__restrict__ first_occ, int nnodes, int64_t nedges,
-                                                          double *__restrict__ node_virial) {
-  const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  const int n = static_cast<int>(t >> 3), sub = static_cast<int>(t & 7);
-  double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  if (n < nnodes) {
-    int e0 = first_occ[n], e1 = first_occ[nnodes + n];
-    clamp_edge_range(e0, e1, nedges);
-    for (int64_t e = e0 + sub; e < e1; e += 8) {
-      const double v0 = vec[3 * e + 0], v1 = vec[3 * e + 1], v2 = vec[3 * e + 2];
-      const double g0 = gv[3 * e + 0], g1 = gv[3 * e + 1], g2 = gv[3 * e + 2];
-      acc[0] += v0 * g0, acc[1] += v1 * g1, acc[2] += v2 * g2;
-      acc[3] += 0.5 * (v1 * g2 + v2 * g1), acc[4] += 0.5 * (v0 * g2 + v2 * g0), acc[5] += 0.5 * (v0 * g1 + v1 * g0);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    acc[k] += __shfl_xor(acc[k], 1);
-    acc[k] += __shfl_xor(acc[k], 2);
-    acc[k] += __shfl_xor(acc[k], 4);
-  }
-  if (n < nnodes && sub == 0) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) node_virial[6 * static_cast<int64_t>(n) + k] = acc[k];
-  }
-}
-
+// the chain delivers.  Two levels, both in a fixed order: per receiver node (with the forces, geometry.hip), then per graph.
+// node_virial [nnodes, 6]: xx, yy, zz, yz, xz, xy.
 // virials[g] (3 x 3, symmetric) = sum of node_virial over the graph's nodes; one workgroup per graph, strided partial sums
 // and a tree over them
 __global__ __launch_bounds__(kSumThreads) void graph_virial_kernel(const double *__restrict__ node_virial,
@@ -592,14 +565,13 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // its vector gradient is written onto the second layer's: gv1 = (this layer's) + gv2
   CM_STAGE(21, cm::mp::edge_backward_onto(g->X1, L.vec, w->r_knots, w->spline[0], w->nknots, w->r_width, w->r_max, L.bufA, g->sender,
                                          fo_live, N, E, C, L.gv1, L.gv2, st));
-  CM_STAGE(23, cm_edge_geometry_backward(positions, g->receiver, g->sender, shifts, g->node_rows, g->first_occ, g->sender_perm,
-                                    g->sender_offsets, L.gv1, nullptr, N, E, forces, nullptr, stream));
   if (virials) {
+    CM_STAGE(23, cm::forces_and_node_virials(L.gv1, L.vec, g->node_rows, g->first_occ, g->sender_perm, g->sender_offsets, N, E, forces, L.node_virial, st));
     cm::StageTimer timer_(st, 24, timing_mask);
-    if (N > 0)
-      hipLaunchKernelGGL(cm::node_virial_kernel, dim3(static_cast<unsigned>(cm::ceil_div(8 * N, 256))), dim3(256), 0, st, L.vec, L.gv1,
-                       g->first_occ, static_cast<int>(N), E, L.node_virial);
     hipLaunchKernelGGL(cm::graph_virial_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, L.node_virial, g->graph_ptr, virials);
+  } else {
+    CM_STAGE(23, cm_edge_geometry_backward(positions, g->receiver, g->sender, shifts, g->node_rows, g->first_occ, g->sender_perm,
+                                           g->sender_offsets, L.gv1, nullptr, N, E, forces, nullptr, stream));
   }
   return cm::check_launch("cm_mace_step");
 }

@@ -589,7 +589,7 @@ int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double
  * per graph may differ from its in the last bits (up to 128 channels the full step forms them in another launch, with
  * another number of partial sums).  No backward chain runs, nothing that only it reads is written, and the workspace,
  * cm_mace_energy_workspace(nnodes, nedges, channels) bytes, has no room for it (a workspace of cm_mace_step will do as well).
- * 11 launches up to 128 channels (12 with few nodes at 96 and 128), 13 beyond.  For callers that compare energies: Monte Carlo moves, screening. */
+ * 10 launches up to 128 channels (11 with few nodes at 96 and 128), 13 beyond.  For callers that compare energies: Monte Carlo moves, screening. */
 size_t cm_mace_energy_workspace(int64_t nnodes, int64_t nedges, int channels);
 int cm_mace_energy(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
                    void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy, double *node_feats,

@@ -466,6 +466,22 @@ def test_energy_stays_inside_its_workspace(cabi, atoms, C):
     assert cabi.lib.cm_mace_energy(*args) == -28
 
 
+@pytest.mark.parametrize("atoms", [2000, 2100])
+def test_virials_on_both_sides_of_a_quarter_wave_per_atom(cabi, atoms):
+    """The virials that come with the forces of the one-call step, per node from a wave or a quarter of one, against the strain
+    derivative (bounds as for the smaller systems above); the forces have the bits of the call without them."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    data = to_device(make_system(atoms, 4, seed=12, density=0.05), "cuda")
+    up = SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=26.0, seed=4)
+    native, eager = (OptimizedInvariantMACE(up, device="cuda", native_step=on) for on in (True, False))
+    a, c = native(dict(data)), native(dict(data), compute_virials=True, compute_stress=True)
+    d = eager(dict(data), compute_virials=True, compute_stress=True)
+    assert torch.equal(c["forces"], a["forces"])
+    for key in ("virials", "stress"):
+        torch.testing.assert_close(c[key], d[key].detach(), rtol=0, atol=2e-6 * float(d[key].abs().max()))
+
+
 @pytest.mark.parametrize("atoms,C", [(5200, 32), (2700, 64)])
 def test_energy_with_and_without_room_for_edge_records(cabi, atoms, C):
     """The forward with the table in LDS reads 16-byte records; for energies alone they lie where vectors and h2 are, which takes

@@ -708,6 +708,12 @@ def test_edge_geometry(cabi, nnodes, avg, iso, seed):
     assert torch.equal(gpos_m[d(rows).long()], gpos)
 
 
+@pytest.mark.parametrize("nnodes,avg,iso,seed", [(2048, 70, 0.1, 4), (2049, 70, 0.1, 5), (2051, 3, 0.4, 6), (2500, 16, 0.0, 7)])
+def test_edge_geometry_with_a_wave_or_a_quarter_per_atom(cabi, nnodes, avg, iso, seed):
+    """Both sides of the atom count that decides it: atoms without edges, with fewer than a trip holds and with more."""
+    test_edge_geometry(cabi, nnodes, avg, iso, seed)
+
+
 # ---- readouts ---------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("N,C,H,seed", [(1, 32, 16, 0), (1000, 128, 16, 1), (37, 96, 5, 2), (515, 256, 1, 3), (16, 64, 16, 4), (50, 30, 7, 5), (20000, 128, 16, 6)])
 def test_readout_forward_backward(cabi, N, C, H, seed):
