@@ -82,9 +82,9 @@ def forward_kernel_name(C, N, E, in_step=False):
     """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_sliced.hip: sliced_forward_applies; the
     benchmark's spline table has 256 knots; the one-call step hands it an edge's vector and sender as one record)."""
     share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
-    enough = {32: 0, 64: 120000 - 10 * N, 96: 65000 + 2 * N, 128: 50000 + 5 * N // 2, 160: 17000 + 5 * N // 2,
-              192: 14000 + 11 * N // 2, 224: 8000 + 3 * N}.get(C, 8000 + 5 * N)
-    if 80 * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
+    enough = {32: 0, 64: 26000, 96: 34000 + 6 * N // 5, 128: 24000 + 2 * N, 160: 3500 + 7 * N // 2,
+              192: 4000 + 11 * N // 2, 224: 8000 + 3 * N}.get(C, 8000 + 5 * N)
+    if {32: 60, 160: 64}.get(C, 76) * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
         return "mp_edge_forward_sliced_kernel<%s>" % ("true" if in_step else "false")
     return "mp_spline_forward_kernel<%d,true>" % C
 

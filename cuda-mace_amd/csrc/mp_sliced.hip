@@ -59,31 +59,31 @@ constexpr unsigned kSlRowBytes = 576;  // of a knot interval: 512 and a quarter 
 constexpr int kSlMaxIntervals = 272;   // 153 KB of table (one row of it is the row of zeros)
 constexpr int kSlSub = 2816;          // nodes sorted at a time: what LDS holds next to the largest table
 constexpr int kSlBins = 64;           // edge blocks per node that the sort tells apart
-// From six rounds of 16 nodes per workgroup on (5 121 nodes at 32 channels, 2 561 at 64, 1 281 at 128, 641 at 256); below
-// that some of its waves have none.  From there on the edges decide: a workgroup spends 4 us on its slice of the table, and
+// From nearly five rounds of 16 nodes per workgroup on (2 432 nodes at 64 channels, 1 216 at 128; 3 840 and 768 at 32 and 160); below
+// that most of its waves have none.  From there on the edges decide: a workgroup spends 3 us on its slice of the table, and
 // nodes with few edges leave it with the fixed part of a round, while the kernel with one wave per node pays per edge.
 // Measured, one wave per node -> this one (us), nodes x neighbours:
-//   32 channels   5 121 x 2 15.9 -> 10.7, 12 000 x 2 30.9 -> 17.4: always
-//   64            2 561 x 20 16.4 -> 17.7, 2 500 x 52 27.6 -> 25.4, 5 000 x 15 21.8 -> 20.9, 8 000 x 4 20.2 -> 18.4
-//   96            1 000 x 52 19.1 -> 23.0, 1 700 x 52 26.5 -> 26.9, 3 000 x 20 21.9 -> 23.7, 8 000 x 10 29.7 -> 28.8, 12 000 x 5.7 30.8 ->
-//                 32.1, 12 000 x 7.5 35.6 -> 33.6, 25 000 x 4.1 50.7 -> 49.5
-//   128           1 000 x 52 22.3 -> 24.0, 1 300 x 52 28.1 -> 25.9, 2 500 x 15 20.1 -> 21.2, 3 500 x 15 26.1 -> 25.3, 6 000 x 10 29.2 ->
-//                 28.6, 12 000 x 5.7 36.3 -> 36.8, 12 000 x 7.5 43.2 -> 41.8, 25 000 x 4.1 60.1 -> 59.4, 25 000 x 7.6 85.3 -> 69.9
-//   160           1 200 x 15 17.3 -> 17.1, 2 000 x 10 18.0 -> 19.8, 5 000 x 4.2 23.3 -> 24.3, 5 000 x 8 33.9 -> 32.3, 12 000 x 4 43.7 -> 42.9
-//   192           1 200 x 15 18.0 -> 17.6, 2 000 x 10 18.5 -> 21.1, 5 000 x 7.7 30.6 -> 31.4, 5 000 x 10 37.2 -> 34.5, 12 000 x 5.7 51.8 ->
-//                 54.4
-//   224           721 x 8 13.9 -> 16.4, 600 x 15 16.0 -> 15.9, 2 000 x 10 22.5 -> 22.2, 12 000 x 4 57.0 -> 53.4
-//   256           1 200 x 10 18.6 -> 19.9, 2 000 x 10 23.5 -> 23.2, 5 000 x 7.7 38.4 -> 36.6, 12 000 x 5.7 63.6 -> 65.0, 12 000 x 7.5 78.6 ->
-//                 69.6, 12 000 x 10 96.1 -> 80.6
-constexpr int kSlMinRounds = 6;
+//   32 channels   2 600 x 52 19.2 -> 22.8, 4 000 x 10 14.7 -> 11.5, 4 000 x 52 25.1 -> 22.7, 12 000 x 2 30.9 -> 17.4: always
+//   64            2 000 x 52 22.8 -> 23.3, 2 560 x 10 12.0 -> 12.2, 2 560 x 25 18.2 -> 16.9, 2 560 x 52 29.2 -> 24.9, 4 000 x 10 15.7 -> 13.5
+//   96            1 700 x 15 12.1 -> 13.5, 1 700 x 52 27.4 -> 24.9, 3 000 x 4 10.5 -> 12.4, 3 000 x 15 18.8 -> 17.9, 8 000 x 4 19.9 -> 20.4, 8 000
+//                 x 15 40.4 -> 30.6
+//   128           1 000 x 52 22.6 -> 22.3, 1 300 x 15 12.5 -> 13.9, 1 300 x 25 16.9 -> 16.4, 1 700 x 15 14.4 -> 14.6, 3 000 x 5 13.4 -> 14.7,
+//                 3 000 x 10 17.6 -> 17.0, 6 000 x 5 21.2 -> 20.7, 12 000 x 2.8 27.0 -> 29.9, 12 000 x 5 34.9 -> 33.4
+//   160           500 x 52 23.0 -> 22.0, 800 x 7 11.7 -> 11.8, 800 x 15 16.0 -> 13.8, 800 x 52 31.5 -> 24.2, 1 200 x 7 12.7 -> 12.0, 3 000 x 7 20.5 -> 18.4
+//   192           500 x 52 19.5 -> 22.7, 800 x 7 11.4 -> 12.2, 800 x 15 16.3 -> 14.3, 1 200 x 7 12.2 -> 13.2, 3 000 x 7 20.6 -> 20.4
+//   224           721 x 8 13.9 -> 16.4, 600 x 15 16.0 -> 15.9, 2 000 x 10 22.5 -> 22.2, 12 000 x 4 57.0 -> 53.4 (an earlier form, a few per
+//                 cent slower)
+//   256           500 x 52 23.8 -> 25.4, 700 x 10 14.6 -> 14.5, 700 x 25 18.7 -> 19.0, 1 000 x 10 16.8 -> 16.3, 2 000 x 4 15.1 -> 18.4, 2 000 x 10
+//                 23.8 -> 22.3, 5 000 x 4 27.6 -> 30.8, 12 000 x 4 51.5 -> 61.5, 12 000 x 10 96.9 -> 81.5
+inline int64_t min_nodes_per_workgroup(int channels) { return channels == 32 ? 60 : (channels == 160 ? 64 : 76); }
 inline int64_t min_edges(int64_t nnodes, int channels) {
   switch (channels) {
     case 32: return 0;
-    case 64: return 120000 - 10 * nnodes;
-    case 96: return 65000 + 2 * nnodes;
-    case 128: return 50000 + 5 * nnodes / 2;
-    case 160: return 17000 + 5 * nnodes / 2;
-    case 192: return 14000 + 11 * nnodes / 2;
+    case 64: return 26000;
+    case 96: return 34000 + 6 * nnodes / 5;
+    case 128: return 24000 + 2 * nnodes;
+    case 160: return 3500 + 7 * nnodes / 2;
+    case 192: return 4000 + 11 * nnodes / 2;
     case 224: return 8000 + 3 * nnodes;
     default: return 8000 + 5 * nnodes;
   }
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
 bool sliced_forward_applies(int64_t nnodes, int64_t nedges, int channels, int nknots) {
   if (channels % 16 != 0 || share_of(channels) < 2 || nedges == 0) return false;
   if (nedges < min_edges(nnodes, channels)) return false;
-  return nnodes > static_cast<int64_t>(share_of(channels)) * (kWave / 4) * (kSlMinRounds - 1) && nnodes < (1 << 24) &&
+  return nnodes > share_of(channels) * min_nodes_per_workgroup(channels) && nnodes < (1 << 24) &&
          nnodes * channels < (int64_t{1} << 30) && nedges <= UINT32_MAX / 12 && nknots >= 2 && nknots - 1 < kSlMaxIntervals;
 }
 

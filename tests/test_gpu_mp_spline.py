@@ -229,7 +229,9 @@ def test_mp_edge_forward_on_both_sides_of_the_line_by_edges(cabi, case):
 
 
 @pytest.mark.parametrize("case", [(2048, 36, 96, 0.05, 2, 200, 0), (1300, 25, 160, 0.3, 3, 256, 0), (900, 22, 192, 0.0, 4, 256, 0),
-                                  (1000, 12, 224, 0.0, 5, 256, 0), (700, 17, 256, 0.0, 6, 272, 0), (9000, 9, 128, 0.1, 7, 128, 300)],
+                                  (1000, 12, 224, 0.0, 5, 256, 0), (700, 17, 256, 0.0, 6, 272, 0), (9000, 9, 128, 0.1, 7, 128, 300),
+                                  (3841, 3, 32, 0.3, 8, 256, 0), (2433, 11, 64, 0.0, 9, 256, 70), (1217, 23, 128, 0.0, 10, 256, 0), (769, 9, 160, 0.0, 11, 256, 0),
+                                  (609, 53, 256, 0.0, 12, 256, 0)],
                          ids=lambda c: "N%d_d%d_C%d" % (c[0], c[1], c[2]))
 def test_mp_edge_forward_just_above_the_line_by_edges(cabi, case):
     """As above, with the edges that the line asks for at these widths, and many nodes with few edges."""
