@@ -116,8 +116,7 @@ __device__ __forceinline__ unsigned quadu(unsigned v) {
 // The value of `v` in each of the four lanes of the reader's quad: element i is lane i's.  One matrix instruction: the
 // 4x4x1 form works on 16 independent blocks of four lanes, D_b[i][j] = A_b[i] B_b[j] + C_b[i][j], with A_b[i] taken from
 // lane i of the block and row i of D in register i of every lane; B = 1 and C = 0 make it a copy (exact for every
-// normal number).  It runs on the matrix pipe, which this kernel does not use otherwise, in place of four moves with a
-// DPP operand on the vector pipe, which is the one that bounds the kernel.
+// normal number), 8 cycles of the SIMD instead of the four moves with a DPP operand at 4.4 each.
 __device__ __forceinline__ f4 quad_gather(float v) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(v, 1.0f, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 }
