@@ -521,9 +521,9 @@ def main():
                               "weights are evaluated in-kernel, so its own HBM operands are small; a workgroup keeps its "
                               "part of the spline table (two degrees x 16 channels, 130 KB) in LDS, so the coefficients "
                               "no longer travel through L1 (the kernel it replaces pulled 8 KB per edge from L2 and ran "
-                              "at 0.37-0.46 ms): bounded by vector-instruction issue (counter summary: 84% of the SIMDs' "
-                              "four-cycle issue slots at 1.8 waves per SIMD; plain multiply-adds issue at one per four "
-                              "cycles with two waves per SIMD and faster only with more; LDS half busy), not by HBM; see "
+                              "at 0.37-0.46 ms): bounded inside the compute units, by L1 misses of the sender rows, LDS "
+                              "(74% busy) and vector issue (one instruction per 3.9 cycles and SIMD, 2.6 waves) "
+                              "together, not by HBM; see "
                               "roofline_other_kernels for the HBM-bound message passing with tabulated R[E,4,C] and for "
                               "the matrix-core linear",
                          binding_resource={
@@ -533,10 +533,10 @@ def main():
                              "peak_TFLOP/s": 157.3, "frac": round(flops_fwd / (t_fwd * 1e-3) / 1e12 / 157.3, 4),
                              "frac_of_unpacked_rate": round(flops_fwd / (t_fwd * 1e-3) / 1e12 / 78.65, 4),
                              "meaning": "useful fp32 operations of the formulation against the vector peak, and against one "
-                                        "FMA per lane and four cycles, 78.65 TFLOP/s (frac_of_unpacked_rate), which is what "
-                                        "plain multiply-adds reach at the two waves per SIMD that this kernel's registers "
-                                        "allow (75 measured; 125 with eight waves); the kernel issues "
-                                        "about 1.8 instructions per useful one (edge set-up per quad of lanes, broadcasts of "
+                                        "FMA per lane and four cycles, 78.65 TFLOP/s (frac_of_unpacked_rate), which multiply-adds "
+                                        "with a scalar operand reach with two waves per SIMD (75 measured; 125 with eight; "
+                                        "with register operands alone one issues per 2.2 to 2.8 cycles); the kernel issues "
+                                        "about 1.5 instructions per useful one (edge set-up per quad of lanes, broadcasts of "
                                         "the edge's values, addresses), and instructions with a cross-lane operand issue at "
                                         "less than half the rate of plain ones on this device"},
                          unfused_equivalent={
@@ -547,8 +547,8 @@ def main():
                                         "duration"})
         others = [entry(backward_kernel_name(C, N, E), bwd_fb, t_bwd,
                         launches_timed=launches(bwd_name),
-                        note="bounded by the L1 path (17 loads of 16 bytes per lane and edge, texture-address units 79% busy) next to vector issue "
-                             "(81% of the four-cycle slots at 1.8 waves per SIMD); with all table rows in L1 it takes 15% less")]
+                        note="bounded by the L1 path (17 loads of 16 bytes per lane and edge at 16 cycles each: 85% of the pass) next to vector "
+                             "issue, which two waves per SIMD do not overlap; with all table rows in L1 it takes 15% less")]
         t_lin = avg_ms("linear")
         if t_lin:
             flops = 32 * N * C * C
