@@ -95,22 +95,6 @@ __global__ void copy_or_zero_f64_kernel(double *p, const double *src, int64_t n)
     p[i] = src ? src[i] : 0.0;
 }
 
-// g1[n, c] = -weight[n] * scale * w1[c]: the gradient of -sum(weight * node energies) with respect to the first layer's
-// features (the linear readout); without weights the same row for every node
-__global__ void seed_linear_readout_kernel(float *__restrict__ g1, const double *__restrict__ w1, double scale,
-                                           const double *__restrict__ node_weights, int64_t total, int C) {
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    g1[i] = static_cast<float>(-1.0 * scale * w1[i % C] * (node_weights ? node_weights[i / C] : 1.0));
-}
-
-// rows of x [nnodes, C] times the node's weight (the second readout's derivative, when node energies carry weights)
-__global__ void weight_rows_kernel(float *__restrict__ x, const double *__restrict__ node_weights, int64_t total, int C) {
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    x[i] = static_cast<float>(static_cast<double>(x[i]) * node_weights[i / C]);
-}
-
 // Edge vectors and the edge range of every receiver node cut back to its last edge inside the cutoff, one launch.
 // Thread i forms the vector of edge i (fp64 difference of the positions plus the shift, rounded once to fp32: the
 // arithmetic of cm_edge_geometry_forward), writes it as the row of `vec` the backward chain reads and, for the forward kernel with
@@ -225,11 +209,10 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
 // out[g] = sum of x over the nodes ptr[g] .. ptr[g + 1]: one workgroup per graph, every thread a strided partial sum, a
 // tree over the partials: the same order on every run.
 constexpr int kSumThreads = 1024;
-__global__ __launch_bounds__(kSumThreads) void segment_sum_f64_kernel(const double *__restrict__ x, const double *__restrict__ weights,
-                                                                     const int32_t *__restrict__ ptr, double *__restrict__ out,
-                                                                     const double *__restrict__ graph_e0, double *__restrict__ total) {
+__device__ __forceinline__ void segment_sum(const double *__restrict__ x, const double *__restrict__ weights, const int32_t *__restrict__ ptr,
+                                            double *__restrict__ out, const double *__restrict__ graph_e0, double *__restrict__ total, int graph) {
   __shared__ double part[kSumThreads];
-  const int lo = ptr[blockIdx.x], hi = ptr[blockIdx.x + 1];
+  const int lo = ptr[graph], hi = ptr[graph + 1];
   auto term = [&](int i) { return weights ? weights[i] * x[i] : x[i]; };
   // four strided partial sums per thread, their loads requested together (one sum waits for memory once per element)
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
@@ -246,8 +229,51 @@ __global__ __launch_bounds__(kSumThreads) void segment_sum_f64_kernel(const doub
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[blockIdx.x] = part[0];
-    if (total) total[blockIdx.x] = part[0] + (graph_e0 ? graph_e0[blockIdx.x] : 0.0);
+    out[graph] = part[0];
+    if (total) total[graph] = part[0] + (graph_e0 ? graph_e0[graph] : 0.0);
+  }
+}
+
+__global__ __launch_bounds__(kSumThreads) void segment_sum_f64_kernel(const double *__restrict__ x, const double *__restrict__ weights,
+                                                                     const int32_t *__restrict__ ptr, double *__restrict__ out,
+                                                                     const double *__restrict__ graph_e0, double *__restrict__ total) {
+  segment_sum(x, weights, ptr, out, graph_e0, total, blockIdx.x);
+}
+
+// Between the readouts and the backward chain of the separate launches (beyond 128 channels): the graph energies, a workgroup each,
+// and in the others the seeds of the chain, a wave per node: g1[n, c] = -weight[n] * scale * w1[c], the gradient of
+// -sum(weight * node energies) with respect to the first layer's features (the linear readout), without weights the same row
+// for every node; with weights d_h2's rows (the second readout's derivative) times the node's weight.  One launch instead of two or,
+// with weights, three, each of them a latency for a small system, with the sum of a large graph alongside the rows.  In the step (us):
+// 60 x 192 7 -> 3.2, 12 000 x 256 with weights 23.5 -> 11.6, 100 000 x 192 41 -> 32 (the rows, 16 bytes per lane, and the sum alike).
+__global__ __launch_bounds__(kSumThreads) void energies_and_seeds_kernel(const double *__restrict__ node_es, const double *__restrict__ node_weights,
+                                                                        const int32_t *__restrict__ ptr, double *__restrict__ energies,
+                                                                        const double *__restrict__ graph_e0, double *__restrict__ total, int ngraphs,
+                                                                        float *__restrict__ g1, float *__restrict__ d_h2,
+                                                                        const double *__restrict__ w1, double scale, int nnodes, int C) {
+  if (static_cast<int>(blockIdx.x) < ngraphs) {
+    segment_sum(node_es, node_weights, ptr, energies, graph_e0, total, blockIdx.x);
+    return;
+  }
+  constexpr int kWaves = kSumThreads / kWave;
+  const int c = 4 * (threadIdx.x % kWave);
+  if (c >= C) return;
+  double w[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) w[k] = w1[c + k];
+  for (int n = (blockIdx.x - ngraphs) * kWaves + threadIdx.x / kWave; n < nnodes; n += (gridDim.x - ngraphs) * kWaves) {
+    const int64_t at = static_cast<int64_t>(n) * C + c;
+    const double nw = node_weights ? node_weights[n] : 1.0;
+    f4 g;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) g[k] = static_cast<float>(-1.0 * scale * w[k] * nw);
+    st4(g1 + at, g);
+    if (node_weights) {
+      f4 d = ld4(d_h2 + at);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = static_cast<float>(static_cast<double>(d[k]) * nw);
+      st4(d_h2 + at, d);
+    }
   }
 }
 
@@ -524,7 +550,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   else
     CM_STAGE(11, cm::readout_forward_with_totals(L.h1, L.h2, w->w1, w->W2a, w->w2b, w->act_cst, w->scale, w->shift, N, C, w->hidden,
                                                  node_energy, want_forces ? L.d_h2 : nullptr, node_feats, g->node_rows, g->node_e0, total_node_energy, st));
-  if (!glue || !want_forces) {  // with the chained kernels the sums ride in the backward chain's launch
+  if (!want_forces) {
     cm::StageTimer timer_(st, 12, timing_mask);
     hipLaunchKernelGGL(cm::segment_sum_f64_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights,
                        g->graph_ptr, interaction_energy, g->graph_e0, total_energy);
@@ -537,13 +563,11 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // own: the gradient with respect to the second layer's features is -d_h2 (the sign goes into the scale of the two
   // linears that consume it, which is exact; node weights scale its rows first), the one with respect to the first
   // layer's is a constant row (times the node's weight).
-  if (!glue) {  // the chained kernels form the constant rows themselves and weight the others
+  if (!glue) {  // the chained kernels form the constant rows themselves, weight the others, and take the energy sums along
     cm::StageTimer timer_(st, 13, timing_mask);
-    const dim3 grid(static_cast<unsigned>(std::min<int64_t>(cm::ceil_div(N * C, 256), 2048)));
-    hipLaunchKernelGGL(cm::seed_linear_readout_kernel, grid, dim3(256), 0, st, L.g1, w->w1, w->scale, g->node_weights,
-                       static_cast<int64_t>(N) * C, C);
-    if (g->node_weights)
-      hipLaunchKernelGGL(cm::weight_rows_kernel, grid, dim3(256), 0, st, L.d_h2, g->node_weights, static_cast<int64_t>(N) * C, C);
+    const unsigned rows = static_cast<unsigned>(std::min<int64_t>(cm::ceil_div(N, cm::kSumThreads / cm::kWave), 1024));
+    hipLaunchKernelGGL(cm::energies_and_seeds_kernel, dim3(g->ngraphs + rows), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights, g->graph_ptr,
+                       interaction_energy, g->graph_e0, total_energy, g->ngraphs, L.g1, L.d_h2, w->w1, w->scale, static_cast<int>(N), C);
   }
   // layer 1 (second interaction)
   if (!glue)

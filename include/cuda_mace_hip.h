@@ -567,8 +567,8 @@ typedef struct cm_mace_graph {
  * returns, per stage, the accumulated milliseconds and the number of timed launches since the mask was set (arrays of
  * at least 25 entries; the return value is the number of stages).  Setting a mask resets the accumulators.  A step
  * enqueued while its stream is capturing is not timed (events recorded into a capture cannot be read back).  Stages: 0 edge geometry and live edge ranges; 1 / 7 message passing forward of layer
- * 0 / 1; 2 / 8 channel mixing; 3 / 9 contraction; 4 / 10 linear after it; 5 skip connection; 6 linear_up; 11 readouts (up to 128 channels with 10 and 14 in their launch); 12 energy sums per graph;
- * 13 seeds of the backward chain; 14 / 19 linear after the contraction, backward; 15 / 20 channel mixing backward (contraction
+ * 0 / 1; 2 / 8 channel mixing; 3 / 9 contraction; 4 / 10 linear after it; 5 skip connection; 6 linear_up; 11 readouts (up to 128 channels with 10 and 14 in their launch); 12 energy sums per graph (energies alone);
+ * 13 seeds of the backward chain, with 12 in their launch; 14 / 19 linear after the contraction, backward; 15 / 20 channel mixing backward (contraction
  * backward folded in); 16 message passing backward of layer 1 (edge pass + sender pass); 21 of layer 0 (edge pass
  * only); 17 linear_up backward; 18 skip backward; 22 sum of the two layers' per-edge gradients; 23 edge geometry backward
  * (forces); 24 virials. */

@@ -482,6 +482,28 @@ def test_virials_on_both_sides_of_a_quarter_wave_per_atom(cabi, atoms):
         torch.testing.assert_close(c[key], d[key].detach(), rtol=0, atol=2e-6 * float(d[key].abs().max()))
 
 
+@pytest.mark.parametrize("sizes,C,weighted", [((1,), 160, False), ((17, 40, 3), 224, True), ((150, 230, 120), 256, False), ((16390,), 160, True)])
+def test_energies_and_seeds_of_the_separate_launches(cabi, sizes, C, weighted):
+    """Beyond 128 channels the graph energies and the rows that start the backward chain come from one launch: several graphs, rows of
+    40 to 64 lanes, a last workgroup partly filled and, from 16 384 atoms on, more than one trip, with and without weights on the
+    node energies, against the path through autograd (bounds as for the systems above)."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.synthetic import collate
+
+    one = lambda n, k: make_system(n, 4, seed=40 + k, density=None if n < 130 else 0.02, cluster_box=12.0 if n < 130 else None)
+    data = one(sizes[0], 0) if len(sizes) == 1 else collate([one(n, k) for k, n in enumerate(sizes)])
+    data = to_device(data, "cuda")
+    if weighted:
+        data["node_weights"] = torch.rand(sum(sizes), generator=torch.Generator().manual_seed(3), dtype=torch.float64).cuda()
+    up = SyntheticInvariantMACE(channels=C, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=12.0, seed=4, shift=0.1)
+    native, eager = (OptimizedInvariantMACE(up, device="cuda", native_step=on) for on in (True, False))
+    a, b = native(dict(data)), eager(dict(data))
+    assert native._native not in (None, False)
+    torch.testing.assert_close(a["energy"], b["energy"].detach(), rtol=1e-12, atol=1e-12)
+    assert torch.equal(a["node_energy"], b["node_energy"].detach())
+    torch.testing.assert_close(a["forces"], b["forces"].detach(), rtol=0, atol=5e-7 * float(b["forces"].abs().max()) + 1e-30)
+
+
 @pytest.mark.parametrize("atoms,C", [(5200, 32), (2700, 64)])
 def test_energy_with_and_without_room_for_edge_records(cabi, atoms, C):
     """The forward with the table in LDS reads 16-byte records; for energies alone they lie where vectors and h2 are, which takes
