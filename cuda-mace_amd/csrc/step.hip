@@ -363,10 +363,13 @@ struct Layout {
     vec = f(3 * E), h2 = f(NC);
     // Energies alone read no vectors but the records', and write h2 when the last record has been read: there the records lie
     // across both, where they fit (with more neighbours than channels they do not, and the forward reads vectors and senders)
-    records = forces ? f(4 * E) : (E <= NC ? vec : nullptr);
+    // With forces they lie where the backward pass, which begins after the last forward has read them, puts its per-edge
+    // gradients: E C floats, of which C >= 32 are an edge's, and they take four.
+    records = forces ? nullptr : (E <= NC ? vec : nullptr);
     gv1 = backward(3 * E), gv2 = backward(3 * E);
     bufM1 = f(16 * NC), bufM2 = forces ? f(16 * NC) : bufM1, bufA = f(16 * NC);
     edge_scratch = backward(E * C);
+    if (forces) records = edge_scratch;
     B1 = f(NC), h1 = f(NC), sc = f(NC), X2 = f(NC), B2 = forces ? f(NC) : B1, d_h2 = backward(NC);
     g1 = backward(NC), gB = backward(NC), gX2 = backward(NC), gh1a = backward(NC), gh1 = backward(NC);
     live = reinterpret_cast<int32_t *>(take(static_cast<size_t>(2 * N) * sizeof(int32_t)));

@@ -68,3 +68,14 @@ def test_energies_alone_take_no_memory_of_the_backward_chain(monkeypatch):
     assert kind == "energy"
     assert energy <= 4 * (3 * E + 2 * N + (2 * 16 + 5) * N * C) + 256 * 9
     assert step >= energy + 4 * E * C
+
+
+def test_forces_take_no_memory_for_edge_records():
+    """Edge vectors and their gradients of both layers (9 E floats), the per-edge gradients (E C) and what the nodes need, each
+    piece rounded up to 256 bytes: the 16-byte records of the forward lie where the per-edge gradients go afterwards."""
+    from cuda_mace import _cabi
+
+    up = lambda nbytes: -(-nbytes // 256) * 256
+    for n, e, c in ((N, E, C), (21, 170, 32), (5000, 260574, 96), (1, 70000, 256), (7, 0, 64)):
+        pieces = 3 * [12 * e] + [4 * e * c] + 3 * [64 * n * c] + 12 * [4 * n * c] + [8 * n, 48 * n]
+        assert _cabi.lib.cm_mace_step_workspace(n, e, c) == sum(up(p) for p in pieces), (n, e, c)
