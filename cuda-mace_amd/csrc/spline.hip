@@ -387,6 +387,10 @@ __device__ __forceinline__ int knot_index(double r, double r_width, int nknots) 
 // forward's bound, and 16-byte loads and stores halve the L1 path's instructions.  30 000 edges x 256 outputs forward 28.9 ->
 // 13.3 us, backward 18.7 -> 13.8 (its stream 11.6), 30 000 x 512 52.5 -> 23.8 and 31.5 -> 24.8, 100 000 x 256 86 -> 39 and 53 -> 43; below some
 // two thousand edges the backward with pairs is half a microsecond behind (1 000 x 256 4.5 -> 5.0), so they take one at a time.
+// In the forward the edge's number is a scalar: all edges inside the cutoff / half of them, when every lane had formed the edge's
+// part and rows were read beyond the cutoff too -> now (us), 30 000 x 256 13.2 / 12.7 -> 12.2 / 11.0, 300 000 x 64 59 / 58 -> 45 / 35,
+// 300 000 x 128 68 / 67 -> 57 / 44, 300 000 x 256 124 / 113 -> 114 / 107, 100 000 x 512 78 / 73 -> 77 / 75; with the derivative as a second output, where two streams of
+// stores set the pace, 100 000 x 512 143 / 144 -> 142 / 147, 300 000 x 128 91 / 89 -> 92 / 103.
 template <int VEC>
 struct Doubles {
   typedef double type __attribute__((ext_vector_type(VEC)));
@@ -407,22 +411,26 @@ __global__ __launch_bounds__(256) void spline_forward_f64_kernel(const double *_
                                                                  double *__restrict__ R_deriv) {
   typedef typename Doubles<VEC>::type dv;
   const int lane = threadIdx.x % kWave;
-  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x / kWave) + threadIdx.x / kWave;
+  // one edge for the whole wave, which the compiler is told: its length comes by a scalar load, the cutoff is a scalar branch
+  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (e >= nedges) return;
   const double re = r[e];
-  const bool live = re <= r_max;
-  const int idx = live ? knot_index(re, r_width, nknots) : 0;
+  if (!(re <= r_max)) {  // beyond the cutoff (or no number): zeros, and no row of the table is read
+#pragma unroll 1
+    for (int j = VEC * lane; j < J; j += VEC * kWave) {
+      std_stream<VEC>(R_out + e * J + j, dv{});
+      if (R_deriv) std_stream<VEC>(R_deriv + e * J + j, dv{});
+    }
+    return;
+  }
+  const int idx = knot_index(re, r_width, nknots);
   const double x = re - r_knots[idx];
   const double *cp = coeffs + static_cast<int64_t>(idx) * 4 * J;
 #pragma unroll 1
   for (int j = VEC * lane; j < J; j += VEC * kWave) {
     const dv a = ldd<VEC>(cp + j), b = ldd<VEC>(cp + J + j), c = ldd<VEC>(cp + 2 * J + j), d = ldd<VEC>(cp + 3 * J + j);
-    const dv val = a + x * (b + x * (c + x * d));
-    std_stream<VEC>(R_out + e * J + j, live ? val : dv{});
-    if (R_deriv) {
-      const dv der = b + x * (2.0 * c + (3.0 * x) * d);
-      std_stream<VEC>(R_deriv + e * J + j, live ? der : dv{});
-    }
+    std_stream<VEC>(R_out + e * J + j, a + x * (b + x * (c + x * d)));
+    if (R_deriv) std_stream<VEC>(R_deriv + e * J + j, b + x * (2.0 * c + (3.0 * x) * d));
   }
 }
 

@@ -175,6 +175,25 @@ def test_spline_f64_one_and_two_outputs_per_lane(cabi, E, J, seed):
     assert bool(((mine - aligned).abs() <= 1e-15 * scale + 1e-300).all())  # sums of J terms in two orders
 
 
+@pytest.mark.parametrize("E,J", [(300, 4), (3001, 33), (20_000, 64), (20_000, 65), (2049, 640)])
+def test_spline_f64_reads_nothing_of_the_table_beyond_the_cutoff(cabi, E, J):
+    """Lengths beyond the cutoff and lengths that are no numbers give zeros, value and derivative, in every kernel of the forward,
+    whatever the table's rows hold that no length points at."""
+    g = torch.Generator().manual_seed(E + J)
+    knots = torch.linspace(0.0, 6.0, 64, dtype=F64)
+    h = float(knots[1])
+    coeffs = torch.randn(63, 4, J, generator=g, dtype=F64)
+    r = torch.rand(E, generator=g, dtype=F64) * 2.0 + 1.0
+    dead = torch.rand(E, generator=g) < 0.4
+    r[dead] = torch.tensor([5.0000001, 7.0, float("inf"), float("nan")], dtype=F64)[torch.randint(0, 4, (int(dead.sum()),), generator=g)]
+    coeffs[0], coeffs[40:] = float("nan"), float("inf")  # rows 10 to 31 hold the lengths inside
+    val, der = cabi.spline_forward(r.to(DEV), knots.to(DEV), coeffs.to(DEV), h, 5.0, want_deriv=True)
+    val_ref, der_ref = O.spline_eval(r[~dead], knots, coeffs, h, 5.0, deriv=True)
+    for out, ref in ((val, val_ref), (der, der_ref)):
+        close(out[~dead.to(DEV)], ref, RTOL, ATOL)
+        assert float(out[dead.to(DEV)].abs().sum()) == 0.0
+
+
 def _symcon_module(ne, C, seed):
     from cuda_mace.models.upstream_like import _SymmetricContraction
     from cuda_mace.ops.symmetric_contraction import SymmetricContraction
