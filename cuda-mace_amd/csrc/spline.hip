@@ -382,6 +382,30 @@ __device__ __forceinline__ int knot_index(double r, double r_width, int nknots) 
   return idx < 0 ? 0 : (idx > nknots - 2 ? nknots - 2 : idx);
 }
 
+// One thread per output: for short rows and few of them.
+template <bool DERIV>
+__global__ void spline_forward_f64_kernel(const double *__restrict__ r, const double *__restrict__ r_knots,
+                                          const double *__restrict__ coeffs, int64_t nedges, int nknots, int J,
+                                          double r_width, double r_max, double *__restrict__ R_out,
+                                          double *__restrict__ R_deriv) {
+  const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (t >= nedges * J) return;
+  const int64_t e = t / J;
+  const int j = static_cast<int>(t - e * J);
+  const double re = r[e];
+  double val = 0.0, der = 0.0;
+  if (re <= r_max) {
+    const int idx = knot_index(re, r_width, nknots);
+    const double x = re - r_knots[idx];
+    const double *cp = coeffs + static_cast<int64_t>(idx) * 4 * J + j;
+    const double a = cp[0], b = cp[J], c = cp[2 * J], d = cp[3 * J];
+    val = a + x * (b + x * (c + x * d));
+    if (DERIV) der = b + x * (2.0 * c + (3.0 * x) * d);
+  }
+  R_out[t] = val;
+  if (DERIV) R_deriv[t] = der;
+}
+
 // A wave per edge, VEC consecutive outputs per lane and trip: what depends on the edge alone (the interval, a division in fp64)
 // is formed once per edge instead of once per output, which with the split of a flat index into edge and output had been the
 // forward's bound, and 16-byte loads and stores halve the L1 path's instructions.  30 000 edges x 256 outputs forward 28.9 ->
@@ -405,10 +429,10 @@ __device__ __forceinline__ void std_stream(double *p, typename Doubles<VEC>::typ
 }
 
 template <int VEC>
-__global__ __launch_bounds__(256) void spline_forward_f64_kernel(const double *__restrict__ r, const double *__restrict__ r_knots,
-                                                                 const double *__restrict__ coeffs, int64_t nedges, int nknots, int J,
-                                                                 double r_width, double r_max, double *__restrict__ R_out,
-                                                                 double *__restrict__ R_deriv) {
+__global__ __launch_bounds__(256) void spline_forward_f64_wave_kernel(const double *__restrict__ r, const double *__restrict__ r_knots,
+                                                                      const double *__restrict__ coeffs, int64_t nedges, int nknots, int J,
+                                                                      double r_width, double r_max, double *__restrict__ R_out,
+                                                                      double *__restrict__ R_deriv) {
   typedef typename Doubles<VEC>::type dv;
   const int lane = threadIdx.x % kWave;
   // one edge for the whole wave, which the compiler is told: its length comes by a scalar load, the cutoff is a scalar branch
@@ -469,6 +493,17 @@ inline bool pairs_of_doubles(int64_t nedges, int J, std::initializer_list<const 
   for (const void *p : pointers)
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
   return true;
+}
+
+// Whether the forward gives an edge a wave.  A trip of the wave, 64 or 128 outputs, costs what some 45 threads with an output each
+// do, and below some 700 000 outputs there are too few waves for their trips, one after the other, to cover each other.  Measured,
+// a thread per output -> a wave per edge (us): pairs, one trip, 300 000 x 4 6.6 -> 45, x 24 28 -> 45, x 40 43.5 -> 44.7, x 48 51 -> 45,
+// 30 000 x 40 6.6 -> 7.0, x 48 7.8 -> 7.3; single outputs, two trips, 300 000 x 81 84 -> 84, x 97 99 -> 85, 30 000 x 81 11.0 -> 12.0, x 97
+// 12.5 -> 12.3; three, 30 000 x 129 15.7 -> 15.9, x 161 19.0 -> 16.2; few rows, 1 000 x 512 4.3 -> 5.4, 2 000 x 225 4.8 -> 5.4, 10 000 x 64
+// 4.8 -> 5.3, 10 000 x 97 5.9 -> 6.1, 10 000 x 128 7.0 -> 4.6.  The launch counts its threads in 32 bits: 64 per edge here.
+inline bool wave_per_edge_f64(int64_t nedges, int J, bool pairs) {
+  const int64_t trips = ceil_div(J, pairs ? 2 * kWave : kWave);
+  return J >= 48 * trips - 4 && nedges * J >= 700000 && nedges < (int64_t{1} << 32) / kWave - kWave;
 }
 
 }  // namespace
@@ -538,15 +573,19 @@ extern "C" int cm_spline_forward_f64(const double *r, const double *r_knots, con
   if (nedges == 0) return CM_OK;
   CM_REQUIRE(r && r_knots && coeffs && R_out, "cm_spline_forward_f64: NULL pointer");
   const int block = 256;
-  const int per = block / cm::kWave;
-  CM_REQUIRE(cm::ceil_div(nedges * noutputs, block) < INT32_MAX, "cm_spline_forward_f64: problem too large for one launch");
-  const dim3 grid(static_cast<unsigned>(cm::ceil_div(nedges, per)));
-  if (cm::pairs_of_doubles(nedges, noutputs, {coeffs, R_out, R_deriv}))
-    hipLaunchKernelGGL(cm::spline_forward_f64_kernel<2>, grid, dim3(block), 0, cm::as_stream(stream), r, r_knots, coeffs,
-                       nedges, nknots, noutputs, r_width, r_max, R_out, R_deriv);
-  else
-    hipLaunchKernelGGL(cm::spline_forward_f64_kernel<1>, grid, dim3(block), 0, cm::as_stream(stream), r, r_knots, coeffs,
-                       nedges, nknots, noutputs, r_width, r_max, R_out, R_deriv);
+  const int64_t threads = nedges * noutputs;
+  CM_REQUIRE(cm::ceil_div(threads, block) < INT32_MAX, "cm_spline_forward_f64: problem too large for one launch");
+  const bool pairs = cm::pairs_of_doubles(nedges, noutputs, {coeffs, R_out, R_deriv});
+  const bool waves = cm::wave_per_edge_f64(nedges, noutputs, pairs);
+  const dim3 grid(static_cast<unsigned>(cm::ceil_div(waves ? nedges * cm::kWave : threads, block)));
+#define CM_FORWARD_F64(KERNEL)                                                                                               \
+  hipLaunchKernelGGL(KERNEL, grid, dim3(block), 0, cm::as_stream(stream), r, r_knots, coeffs, nedges, nknots, noutputs, r_width, \
+                     r_max, R_out, R_deriv)
+  if (waves && pairs) CM_FORWARD_F64(cm::spline_forward_f64_wave_kernel<2>);
+  else if (waves) CM_FORWARD_F64(cm::spline_forward_f64_wave_kernel<1>);
+  else if (R_deriv) CM_FORWARD_F64(cm::spline_forward_f64_kernel<true>);
+  else CM_FORWARD_F64(cm::spline_forward_f64_kernel<false>);
+#undef CM_FORWARD_F64
   return cm::check_launch("cm_spline_forward_f64");
 }
 

@@ -175,6 +175,25 @@ def test_spline_f64_one_and_two_outputs_per_lane(cabi, E, J, seed):
     assert bool(((mine - aligned).abs() <= 1e-15 * scale + 1e-300).all())  # sums of J terms in two orders
 
 
+@pytest.mark.parametrize("E,J,seed", [(30_001, 43, 17), (30_001, 44, 18), (29_999, 91, 19), (29_999, 93, 20), (5468, 128, 21), (5469, 128, 22),
+                                      (20_001, 3, 23)])
+def test_spline_f64_a_thread_per_output_and_a_wave_per_edge(cabi, E, J, seed):
+    """On both sides of the rule between the forward's two kernels: row length, for one trip of the wave and for two, and outputs."""
+    test_spline_f64(cabi, E, J, seed)
+
+
+def test_spline_f64_more_edges_than_waves_in_a_launch(cabi):
+    """2^26 edges with one output each: a launch with a wave per edge would have 2^32 threads, one with a thread per output has 2^26."""
+    E = (1 << 26) + 5
+    knots = torch.linspace(0.0, 6.0, 64, dtype=F64, device=DEV)
+    coeffs = torch.randn(63, 4, 1, generator=torch.Generator().manual_seed(3), dtype=F64).to(DEV)
+    r = torch.rand(E, device=DEV, dtype=F64) * 5.6
+    out = cabi.spline_forward(r, knots, coeffs, float(knots[1]), 5.0)
+    for part in (slice(0, 1000), slice(E // 2, E // 2 + 1000), slice(E - 1000, E)):
+        assert torch.equal(out[part], cabi.spline_forward(r[part].contiguous(), knots, coeffs, float(knots[1]), 5.0))
+    assert float(out[(r > 5.0)].abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("E,J", [(300, 4), (3001, 33), (20_000, 64), (20_000, 65), (2049, 640)])
 def test_spline_f64_reads_nothing_of_the_table_beyond_the_cutoff(cabi, E, J):
     """Lengths beyond the cutoff and lengths that are no numbers give zeros, value and derivative, in every kernel of the forward,
