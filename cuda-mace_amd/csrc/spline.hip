@@ -157,10 +157,7 @@ __global__ __launch_bounds__(256) void spline_backward_kernel(
 // on at a time share a few rows of the table, which stay in L1.  Half a wave serves an edge, ITER 16-byte pieces of the row
 // per lane, all of them requested before the first is used (up to 512 outputs: beyond, 512 at a time; two edges at a time
 // where a row is one piece per lane: 122 880 x 128 29.7 -> 18.9 us).  An edge's sum does not depend on its place in the order.
-// Measured (edges x outputs, us), one wave per edge / the LDS-table kernel below / this one: 33 000 x 256 13.8 / 41.5 / 11.7, 33 000 x
-// 512 20.5 / 80.7 / 20.3, 122 880 x 128 40.5 / 26.0 / 18.9, 122 880 x 384 62.0 / 72.3 / 46.4 (its stream alone 35.6), 122 880 x 1 024 133 /
-// 235 / 120, 300 000 x 512 165 / 170 / 137, 400 000 x 128 133 / 55 / 53, 600 000 x 128 199 / 73 / 78, 600 000 x 1 024 642 / 611 / 554, 900 000 x
-// 512 493 / 390 / 411, 1 300 000 x 512 707 / 526 / 590.  Error against fp64 8.0e-8 to 9.8e-8, the LDS-table kernel's 7.9e-8 to 1.3e-7.
+// Which of the two it is from 32 768 edges on: see spline_backward_sliced_from.
 constexpr int kSpSortThreads = 1024;
 constexpr int kSpSortChunk = 4096;  // edges of a chunk: their place in it takes 12 bits
 constexpr int kSpSortBins = 256;
@@ -284,7 +281,7 @@ void launch_spline_backward_sorted(const float *r, const float *r_knots, const f
 #undef CM_SORTED
 }
 
-// ---- LDS-table variant of the backward for the longest edge lists --------------------------------------------------
+// ---- LDS-table variant of the backward for the longest lists and for short rows --------------------------------------------------
 // Even in the order of the intervals the coefficients pass through L1, 48 bytes for every 16 of the gradient stream.  Here a workgroup owns a chunk of consecutive edges and sums them slice by slice: for each slice of 32
 // outputs it loads the derivative's coefficients (b, 2c, 3d per interval: 384 bytes, 104 KB at most) into LDS, streams
 // that slice of its edges' gradient rows (one 128-byte line per edge) and adds each edge's partial sum to the edge's
@@ -294,7 +291,6 @@ void launch_spline_backward_sorted(const float *r, const float *r_knots, const f
 // the bytes of the gradient stream at 5 000 edges per chunk.
 constexpr int kSpBwdRow = 3 * kSpSlice;  // floats per interval
 constexpr int kSpBwdChunk = 8192;        // edges per chunk at most (their sums: 32 KB of LDS)
-constexpr int64_t kSpBwdMinEdges = 1 << 19;  // below, loading the slices costs more than it saves: see the kernel above
 
 __global__ __launch_bounds__(kSpThreads) void spline_backward_sliced_kernel(
     const float *__restrict__ r, const float *__restrict__ r_knots, const float *__restrict__ coeffs,
@@ -373,6 +369,26 @@ void launch_spline_backward_sliced(const float *r, const float *r_knots, const f
   const int groups = static_cast<int>(std::min<int64_t>(cus, ceil_div(nedges, chunk)));
   hipLaunchKernelGGL(spline_backward_sliced_kernel, dim3(static_cast<unsigned>(groups)), dim3(kSpThreads), 0, st, r, r_knots,
                      coeffs, gR, nedges, nknots, J, r_width, r_max, gr, static_cast<int>(ceil_div(J, kSpSlice)), chunk);
+}
+
+// Edges from which the LDS-table kernel is the faster one.  It pays a fixed 3 to 6 us per slice of 32 outputs (staging, less with
+// fewer knots) and then for the outputs there are; the kernel in the order of the intervals pays for what its lanes span, 128
+// outputs or a multiple, beyond 512 a multiple of 512, and half a wave per edge however short the row.  So the line falls with the
+// square of the part of the span that a row fills; but not below 2^19 edges where its sums are the longer chains (error against fp64,
+// in the order of the intervals / LDS table: 32 outputs 6.89e-8 / 6.64e-8, 128 8.06 / 7.84, 192 8.46 / 8.35, 256 8.54 / 8.89, 512 8.88 /
+// 10.2, 1 024 9.62 / 12.6).  Measured, in the order of the intervals / LDS table (us), 256 knots:
+//   4 outputs  33 000 5.5 / 6.7, 60 000 7.2 / 6.9, 300 000 29.7 / 11.4      32 40 000 6.9 / 6.8, 300 000 35 / 13    64 90 000 12.9 / 13.5, 110 000 15.3 / 14.0
+//   96   200 000 27.6 / 28.7, 250 000 33.2 / 30.1         128 400 000 52.9 / 54.6, 500 000 65.5 / 61.1
+//   160  200 000 44.5 / 45.9, 250 000 54 / 48             192 250 000 55.5 / 56.7, 350 000 76 / 73       256 700 000 160 / 162, 800 000 181 / 176
+//   320  400 000 126 / 134, 500 000 155 / 152             448 400 000 170 / 184, 500 000 213 / 209       512 700 000 315 / 330, 800 000 362 / 351
+//   640  250 000 186 / 191, 350 000 258 / 245             768 400 000 316 / 344, 600 000 476 / 457       1 024 800 000 728 / 748, 900 000 828 / 808
+// and with 32 knots 128 200 000 28.5 / 29.5, 400 000 53 / 47; 512 300 000 128 / 141, 600 000 256 / 248; 1 024 600 000 500 / 492.
+inline int64_t spline_backward_sliced_from(int nknots, int J) {
+  const int span = J <= 512 ? static_cast<int>(ceil_div(J, 128) * 128) : static_cast<int>(ceil_div(J, 512) * 512);
+  const double part = 32.0 * static_cast<double>(ceil_div(J, 32)) / span;
+  const double most = span == 128 ? 430e3 : (span > 512 ? 850e3 : (part == 1.0 ? 720e3 : 600e3));
+  const int64_t line = static_cast<int64_t>(most * part * part * (290 + nknots) / 546.0);
+  return std::max<int64_t>(line, span > 256 ? 1 << 19 : 40000);
 }
 
 // fp64 variants (the reference dispatches the spline on float and double, jit_wrappers/src/cubic_spline_wrapper.cpp:50,
@@ -546,7 +562,7 @@ extern "C" int cm_spline_backward(const float *r, const float *r_knots, const fl
   CM_REQUIRE(r_width > 0.f, "cm_spline_backward: r_width must be positive");
   if (nedges == 0) return CM_OK;
   CM_REQUIRE(r && r_knots && coeffs && grad_R && grad_r, "cm_spline_backward: NULL pointer");
-  if (nedges >= cm::kSpBwdMinEdges && cm::spline_sliced_applies(nedges, nknots, noutputs)) {
+  if (cm::spline_sliced_applies(nedges, nknots, noutputs) && nedges >= cm::spline_backward_sliced_from(nknots, noutputs)) {
     cm::launch_spline_backward_sliced(r, r_knots, coeffs, grad_R, nedges, nknots, noutputs, r_width, r_max, grad_r,
                                       cm::as_stream(stream));
     return cm::check_launch("cm_spline_backward");

@@ -271,8 +271,8 @@ def test_sh_forward_backward(cabi, E, seed):
 # ------------------------------------------------------------------------------------------------
 # spline
 # ------------------------------------------------------------------------------------------------
-# from 32 768 edges on the forward without derivative, from 524 288 on the backward run on their LDS-table kernels: full rows
-# of slices, a last slice of 8 of 32 outputs, and more edges than one pass of chunks holds (256 workgroups x 8 192)
+# from 32 768 edges on the forward without derivative, and the backward from a number of edges on that depends on the row, run on
+# their LDS-table kernels: full rows of slices, a last slice of 8 of 32 outputs, and more edges than one pass of chunks holds (256 workgroups x 8 192)
 @pytest.mark.parametrize("E,J,seed", [(1, 128, 0), (777, 384, 1), (5000, 512, 2), (300, 768, 3), (40_000, 512, 4),
                                       (70_001, 72, 5), (2_200_003, 8, 6)])
 def test_spline_forward_backward(cabi, E, J, seed):
@@ -337,6 +337,15 @@ def test_spline_backward_in_the_order_of_the_intervals(cabi, E, J, nknots):
         ok = live[s]
         assert bool(((gr[s] - ref).abs()[ok] <= bound[ok]).all())
         assert float(gr[s][~ok].abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("E,J,nknots", [(39_999, 32, 256), (40_000, 32, 256), (60_001, 8, 256), (107_499, 64, 256), (107_500, 64, 256), (63_396, 64, 32), (63_397, 64, 32),
+                                        (125_771, 160, 3), (125_772, 160, 3), (524_288, 260, 2)])
+def test_spline_backward_on_both_sides_of_the_line_of_its_row(cabi, E, J, nknots):
+    """Short rows on the LDS-table kernel, and the last and first lists on either side of the line that a row's length and the
+    number of knots draw (107 500 edges at 64 outputs and 256 knots, 63 397 with 32 knots; at least 40 000, and 2^19 beyond 256
+    outputs)."""
+    test_spline_backward_in_the_order_of_the_intervals(cabi, E, J, nknots)
 
 
 # ------------------------------------------------------------------------------------------------
