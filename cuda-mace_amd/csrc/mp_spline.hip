@@ -638,7 +638,7 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
 }
 
 // -----------------------------------------------------------------------------------------------
-// backward, edge pass from edge vectors at 160, 192 and 224 channels: four edges side by side, the channels in steps of 64
+// backward, edge pass from edge vectors at 160, 192 and 224 channels (most sizes: steps_of_four_edges): four edges side by side, the channels in steps of 64
 // -----------------------------------------------------------------------------------------------
 // In the kernel above an edge of 160, 192 or 224 channels takes a whole wave, and its 17 load instructions move 40 or 56 lanes of
 // 16 bytes or 64 of 12 where 64 of 16 cost the L1 path the same (16 cycles for any load of 8 to 16 bytes per lane).  Here a row of 16 lanes serves an edge, four channels per lane, a group
@@ -653,10 +653,10 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
 // q_l and the gradient with respect to the direction on it, with every product padded to four m, spent 640 cycles per four
 // edges and step there against the 370 of the sums here.  Against that kernel and, where it did not run, the one above, us
 // without / with gX and its sender pass: 192 channels 100 nodes x 52 11.8 / 19.6 -> 11.1 / 18.3, 1 100 56 / 80 -> 39 / 64,
-// 11 000 314 / 442 -> 276 / 414, 40 000 1 089 / 1 598 -> 1 003 / 1 522, 4 000 x 4 22.1 / 30.3 -> 22.3 / 30.5; 160 channels 100
-// 15.5 / 23.9 -> 11.1 / 18.5, 11 000 319 / 428 -> 262 / 381, 4 000 x 4 24.6 -> 20.4; 224 channels 1 000 40.5 / 53.6 -> 41.4 / 55.7,
-// 3 000 127 / 161 -> 112 / 147, 30 000 913 / 1 366 -> 909 / 1 358, 11 000 x 4 61.6 -> 61.2.  Not at the widths that fill the lanes
-// of the kernel above: 256 357 / 524 -> 359 / 535, 96 170 / 242 -> 176 / 247, 128 (25 000) 406 / 616 -> 399 / 612.
+// 11 000 314 / 442 -> 276 / 414, 40 000 1 089 / 1 598 -> 1 003 / 1 522; 160 channels 100 15.5 / 23.9 -> 11.1 / 18.5,
+// 11 000 319 / 428 -> 262 / 381, 4 000 x 4 24.6 -> 20.4; 224 channels 3 000 127 / 161 -> 112 / 147, 30 000 913 / 1 366 -> 909 / 1 358.
+// Not at the widths that fill the lanes of the kernel above: 256 357 / 524 -> 359 / 535, 96 170 / 242 -> 176 / 247, 128 (25 000)
+// 406 / 616 -> 399 / 612; and not everywhere at 192 and 224: see steps_of_four_edges.
 template <int C, bool WANT_GV, bool WANT_GX>
 __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_steps_kernel(
     const float *__restrict__ X, Spline sp, const float *__restrict__ G, const int32_t *__restrict__ sender,
@@ -670,7 +670,10 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
   __shared__ int sIdx[kChunk];
   __shared__ float sXr[kChunk];
   __shared__ int sOrig[kChunk];
-  constexpr int kKnots = C == 224 ? 256 : kKnotsInLds;  // 160 KB hold eight waves' arrays at every width
+  // 160 KB hold eight waves' arrays at every width.  At 224 channels that leaves room for 256 knots; more are read from memory, which
+  // costs less than a place for 512 and seven waves (400 knots, us without / with gX: 1 000 x 52 49.8 / 68.0 -> 39.4 / 56.3, 3 000 x 52
+  // 112 / 158 -> 105 / 148, 6 000 x 12 62.2 / 87.8 -> 61.4 / 86.4, 216 x 52 14.4 / 22.9 -> 15.2 / 23.7).
+  constexpr int kKnots = C == 224 ? 256 : kKnotsInLds;
   __shared__ float sKnots[kKnots];
 
   const int node = parts == 1 ? blockIdx.x : blockIdx.x / parts;
@@ -768,9 +771,10 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
       locate_group(min(s + 1, ngroups - 1), co_next, xo_next, xr_next);
       const int j = min(4 * s + row, nlive - 1);
       const int orig = sOrig[j];
-      // Two chains per sum, a lane's first and last two channels: in one chain of up to 16 the error of the vector gradient against
-      // fp64 is 2.515e-7 at 192 channels and 2.562e-7 at 224, in two 2.503e-7 and 2.550e-7 (one edge per wave or matrix products:
-      // 2.500e-7 and 2.545e-7, three parts in a thousand being the scatter of the figure), in the same time.
+      // Two chains per sum over m >= 1, a lane's first and last two channels (the radial sum has one, of a product per step: its
+      // four channels are added up first).  Error of the vector gradient against fp64, mean of four graphs, one edge per wave or
+      // matrix products / one chain / two: 160 channels 2.504e-7 / - / 2.500e-7, 192 2.514 / 2.52 / 2.513, 224 2.560 / 2.57 / 2.563 (the
+      // graphs differ by 0.04e-7; a second chain for the radial sum: 2.498, 2.511, 2.565).
       float y[16], p[16], r[16];
       staged_harmonics(sY, j, y);
 #pragma unroll
@@ -856,19 +860,45 @@ int launch_forward(const float *X, const float *Y, const Spline &sp, const int32
   return check_launch(FROM_VEC ? "cm_mp_edge_forward" : "cm_mp_spline_forward");
 }
 
+// Whether the edge pass from edge vectors takes a group of four edges per step (mp_edge_backward_steps_kernel) or an edge per wave.
+// At 160 channels always.  At 192 and 224 a receiver with few edges leaves most of its last group empty, and the rows of its
+// gradient pass through LDS for nothing; at 224 the two are level as long as every SIMD has both its waves (the kernel with an
+// edge per wave keeps the gradient rows in registers, the other reads them from LDS, which eight waves share), and the steps gain
+// where a chip is partly filled.  us without / with gX, steps -> an edge per wave:
+//   192  60 x 2.6 6.4 / 10.6 -> 5.6 / 10.1, 60 x 5 6.6 / 10.8 -> 7.1 / 11.6, 500 x 4.9 8.3 / 13.1 -> 7.9 / 12.7, 500 x 7 8.8 / 14.5 -> 9.2 / 15.0, 3 000 x 0.9 11.8 / 16.4 -> 9.6 / 14.3,
+//        3 000 x 5 20.3 / 28.4 -> 19.7 / 27.8, 3 000 x 9.5 26.9 / 38.2 -> 28.1 / 39.7, 20 000 x 0.9 49 / 66 -> 42 / 58, 20 000 x 7 116 / 163 -> 118 / 164
+//   224  500 x 1.7 7.8 / 12.4 -> 7.2 / 11.5, 1 000 x 2.6 8.7 / 13.5 -> 9.5 / 13.6, 500 x 3.8 8.2 / 12.8 -> 8.7 / 13.4, 3 000 x 5 24.0 / 33.7 -> 22.9 / 31.8, 3 000 x 9.5 32 / 45 -> 32.5 / 45,
+//        20 000 x 1.7 77 / 99 -> 74 / 95, 20 000 x 2.7 87 / 114 -> 89 / 116, 20 000 x 3.8 99 / 132 -> 102 / 136; one round of waves: 500 x 52 (four parts) 23.5 / 34.4 -> 22.7 / 32.8,
+//        1 000 x 52 (two) 38.4 / 55.1 -> 36.8 / 53.3, 2 048 x 12 24.9 / 35.9 -> 23.7 / 34.2; part of one: 216 x 52 13.8 / 22.2 -> 18.2 / 23.6,
+//        1 200 x 52 50 / 77 -> 58 / 83
+template <int C>
+bool steps_of_four_edges(int64_t nnodes, int64_t nedges, int parts) {
+  if constexpr (C == 160) return true;
+  if constexpr (C == 192) return nedges >= 5 * nnodes;
+  if constexpr (C == 224) {
+    const int64_t waves = nnodes * parts;
+    if (waves > 1536 && waves <= 2048) return false;
+    return 2 * nedges >= (waves > 2048 && waves <= 8192 ? 10 : 5) * nnodes;
+  }
+  return false;
+}
+
 template <int C, bool FROM_VEC, bool GY, bool GR, bool GX>
 void launch_edge(const float *X, const float *Y, const Spline &sp, const float *G, const int32_t *sender,
                  const int32_t *first_occ, int64_t nnodes, int64_t nedges, float *gY, float *g_r, float *gXe,
                  hipStream_t st) {
   const int parts = parts_for(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
-  if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {  // at every size: see the kernel
-    hipLaunchKernelGGL((mp_edge_backward_steps_kernel<C, GY, GX>), grid, dim3(kWave), 0, st, X, sp, G, sender, first_occ,
-                       static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
-  } else {
+  if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {
+    if (steps_of_four_edges<C>(nnodes, nedges, parts)) {
+      hipLaunchKernelGGL((mp_edge_backward_steps_kernel<C, GY, GX>), grid, dim3(kWave), 0, st, X, sp, G, sender, first_occ,
+                         static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
+      return;
+    }
+  }
+  if constexpr (!FROM_VEC || C != 160)
     hipLaunchKernelGGL((mp_spline_backward_edge_kernel<C, FROM_VEC, GY, GR, GX>), grid, dim3(kWave), 0, st, X, Y, sp, G, sender,
                        first_occ, static_cast<int>(nnodes), nedges, gY, g_r, gXe, parts);
-  }
 }
 
 // gY / g_r: outputs of the Y-and-r variant; in the FROM_VEC variant gY is the [E, 3] vector gradient and g_r, when given,

@@ -315,6 +315,20 @@ def test_mp_edge_backward_few_and_many_nodes(cabi, case):
     test_mp_edge_backward_on_the_matrix_cores(cabi, case)
 
 
+@pytest.mark.parametrize("case", [(600, 4, 192, 0.0, 41, 256, 70), (600, 6, 192, 0.0, 42, 256, 70), (700, 2, 224, 0.0, 43, 256, 66),
+                                  (700, 4, 224, 0.0, 44, 300, 66), (1537, 9, 224, 0.0, 45, 256, 0), (1536, 9, 224, 0.0, 46, 256, 0),
+                                  (2048, 6, 224, 0.1, 47, 512, 130), (2049, 4, 224, 0.0, 48, 256, 0), (2049, 6, 224, 0.0, 49, 256, 0),
+                                  (500, 51, 224, 0.0, 50, 256, 0)],
+                         ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
+def test_mp_edge_backward_on_both_sides_of_the_line(cabi, case):
+    """The sizes between which 192 and 224 channels change from groups of four edges to an edge per wave: edges per node, and at 224
+    a round of waves, whole or in parts."""
+    nnodes, C, E = case[0], case[2], _edge_case(*case)[0].numel()
+    per_node = {(600, 4): 5, (600, 6): 5, (700, 2): 2.5, (700, 4): 2.5, (2049, 4): 5, (2049, 6): 5}.get(case[:2])
+    assert per_node is None or (E < per_node * nnodes) == (case[1] < per_node)
+    test_mp_edge_backward_on_the_matrix_cores(cabi, case)
+
+
 @pytest.mark.parametrize("nnodes,C", [(1750, 96), (1400, 128), (1000, 160), (900, 192), (700, 256)])
 def test_forward_from_vectors_is_no_less_precise_than_from_harmonics_and_lengths(cabi, nnodes, C):
     """From vectors these sizes run on the kernel that forms length and direction from one reciprocal square root; given
