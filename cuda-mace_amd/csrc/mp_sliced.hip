@@ -45,6 +45,8 @@
 // two chains (even and odd places) that are added up at the end; error of the message against fp64 at 52 neighbours, one chain -> two, and of the kernels
 // with one wave per node: 96 channels 2.68e-7 -> 2.54e-7 (2.70e-7), 128 2.73 -> 2.59 (2.74), 192 2.67 -> 2.52 (2.69), 256
 // 2.81 -> 2.67 (2.83).
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "mp_common.hpp"
@@ -68,25 +70,47 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 //   96            1 700 x 15 12.1 -> 13.5, 1 700 x 52 27.4 -> 24.9, 3 000 x 4 10.5 -> 12.4, 3 000 x 15 18.8 -> 17.9, 8 000 x 4 19.9 -> 20.4, 8 000
 //                 x 15 40.4 -> 30.6
 //   128           1 000 x 52 22.6 -> 22.3, 1 300 x 15 12.5 -> 13.9, 1 300 x 25 16.9 -> 16.4, 1 700 x 15 14.4 -> 14.6, 3 000 x 5 13.4 -> 14.7,
-//                 3 000 x 10 17.6 -> 17.0, 6 000 x 5 21.2 -> 20.7, 12 000 x 2.8 27.0 -> 29.9, 12 000 x 5 34.9 -> 33.4
+//                 3 000 x 10 17.6 -> 17.0, 6 000 x 5 21.2 -> 20.7, 12 000 x 2.8 27.0 -> 29.9, 12 000 x 5 34.9 -> 33.4, 16 000 x 3.8 35.1 -> 37.4
 //   160           500 x 52 23.0 -> 22.0, 800 x 7 11.7 -> 11.8, 800 x 15 16.0 -> 13.8, 800 x 52 31.5 -> 24.2, 1 200 x 7 12.7 -> 12.0, 3 000 x 7 20.5 -> 18.4
 //   192           500 x 52 19.5 -> 22.7, 800 x 7 11.4 -> 12.2, 800 x 15 16.3 -> 14.3, 1 200 x 7 12.2 -> 13.2, 3 000 x 7 20.6 -> 20.4
 //   224           721 x 8 13.9 -> 16.4, 600 x 15 16.0 -> 15.9, 2 000 x 10 22.5 -> 22.2, 12 000 x 4 57.0 -> 53.4 (an earlier form, a few per
 //                 cent slower)
-//   256           500 x 52 23.8 -> 25.4, 700 x 10 14.6 -> 14.5, 700 x 25 18.7 -> 19.0, 1 000 x 10 16.8 -> 16.3, 2 000 x 4 15.1 -> 18.4, 2 000 x 10
-//                 23.8 -> 22.3, 5 000 x 4 27.6 -> 30.8, 12 000 x 4 51.5 -> 61.5, 12 000 x 10 96.9 -> 81.5
+//   256           650 x 9.5 13.0 -> 13.7, 650 x 14 16.8 -> 15.2, 700 x 24 23.2 -> 17.6, 700 x 28 (in two parts) 17.6 -> 18.1, 1 000 x 9.3 15.5 -> 15.4, 1 700 x 8
+//                 18.2 -> 19.1, 2 500 x 7.3 21.0 -> 21.4, 4 000 x 6 26.2 -> 26.8, 4 000 x 7 29.9 -> 28.1, 8 000 x 6 42.9 -> 44.7, 8 000 x 7 47.4 -> 46.6,
+//                 12 000 x 6 60.6 -> 62.8, 12 000 x 7 67.8 -> 66.9
+// Beyond 256 MB of output, what the last-level cache holds, its writes reach memory as the 64-byte pieces of rows that a workgroup's
+// 16 channels are, and what that costs per node has to be won back by edges: the line is then a number of neighbours that grows
+// with the logarithm of the output and with the channels (up to 64 channels it does not come to that).  One wave per node -> this
+// one (reading vectors / the step's records), us:
+//   96            40 000 x 5 78 -> 79 / 77, 60 000 x 7 193 -> 193 / 192, 100 000 x 5 291 -> 328 / 321, x 9.3 369 -> 374 / 365, 200 000 x 14 881 -> 805 / 787
+//   128           25 000 x 3.8 51 -> 54 / 54, x 5 60 -> 57 / 56, 60 000 x 9.4 278 -> 292 / 281, x 12 309 -> 301 / 281, 100 000 x 7 416 -> 467 / 457, 400 000 x 14
+//                 2 194 -> 2 392 / 2 326, x 19 2 750 -> 2 641 / 2 590
+//   160           30 000 x 5 124 -> 125 / 125, 60 000 x 7 327 -> 359 / 346, x 12 403 -> 385 / 369, 100 000 x 9.3 605 -> 652 / 634, x 15 756 -> 721 / 695
+//   192           30 000 x 7 170 -> 188 / 174, 60 000 x 9.4 398 -> 460 / 444, x 15 505 -> 498 / 468, 100 000 x 9.3 659 -> 787 / 765, x 17 927 -> 915 / 882
+//   224           30 000 x 7 222 -> 232 / 230, 60 000 x 9.4 490 -> 522 / 506, x 15 616 -> 579 / 553, 100 000 x 9.3 797 -> 891 / 865, x 17 1 132 -> 1 049 / 1 012
+//   256           30 000 x 9.4 261 -> 317 / 300, x 15 333 -> 315 / 280, 60 000 x 15 651 -> 747 / 718, x 25 980 -> 850 / 816, 100 000 x 9.3 839 -> 1 141 / 1 118,
+//                 x 25 1 610 -> 1 557 / 1 494
 inline int64_t min_nodes_per_workgroup(int channels) { return channels == 32 ? 60 : (channels == 160 ? 64 : 76); }
 inline int64_t min_edges(int64_t nnodes, int channels) {
-  switch (channels) {
-    case 32: return 0;
-    case 64: return 26000;
-    case 96: return 34000 + 6 * nnodes / 5;
-    case 128: return 24000 + 2 * nnodes;
-    case 160: return 3500 + 7 * nnodes / 2;
-    case 192: return 4000 + 11 * nnodes / 2;
-    case 224: return 8000 + 3 * nnodes;
-    default: return 8000 + 5 * nnodes;
-  }
+  struct Line {
+    int64_t cached;             // edges, while the output fits the last-level cache
+    double per_node, doubling;  // beyond: neighbours, and how many more for twice the output
+  };
+  const Line line = [&]() -> Line {
+    switch (channels) {
+      case 32: return {0, 0.0, 0.0};
+      case 64: return {26000, 0.0, 0.0};
+      case 96: return {std::max(34000 + 6 * nnodes / 5, 4 * nnodes), 6.5, 1.1};
+      case 128: return {std::max(24000 + 2 * nnodes, 17 * nnodes / 4), 6.7, 3.0};
+      case 160: return {3500 + 7 * nnodes / 2, 5.0, 3.9};
+      case 192: return {4000 + 11 * nnodes / 2, 6.5, 4.6};
+      case 224: return {8000 + 3 * nnodes, 5.3, 3.8};
+      default: return {5000 + 23 * nnodes / 4, 5.0, 7.5};
+    }
+  }();
+  const double caches = 64.0 * static_cast<double>(nnodes) * channels / (1 << 28);  // 16 components of 4 bytes in 256 MB
+  if (caches <= 1.0) return line.cached;
+  return std::max(line.cached, static_cast<int64_t>((line.per_node + line.doubling * std::log2(caches)) * static_cast<double>(nnodes)));
 }
 inline int share_of(int channels) { return device_compute_units() / (2 * (channels / 16)); }  // workgroups per (pair, slice)
 
