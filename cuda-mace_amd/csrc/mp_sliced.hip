@@ -64,7 +64,7 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 // From nearly five rounds of 16 nodes per workgroup on (2 432 nodes at 64 channels, 1 216 at 128; 3 840 and 768 at 32 and 160); below
 // that most of its waves have none.  From there on the edges decide: a workgroup spends 3 us on its slice of the table, and
 // nodes with few edges leave it with the fixed part of a round, while the kernel with one wave per node pays per edge.
-// Measured, one wave per node -> this one (us), nodes x neighbours:
+// Measured, the launch alone, one wave per node -> this one (us), nodes x neighbours:
 //   32 channels   2 600 x 52 19.2 -> 22.8, 4 000 x 10 14.7 -> 11.5, 4 000 x 52 25.1 -> 22.7, 12 000 x 2 30.9 -> 17.4: always
 //   64            2 000 x 52 22.8 -> 23.3, 2 560 x 10 12.0 -> 12.2, 2 560 x 25 18.2 -> 16.9, 2 560 x 52 29.2 -> 24.9, 4 000 x 10 15.7 -> 13.5
 //   96            1 700 x 15 12.1 -> 13.5, 1 700 x 52 27.4 -> 24.9, 3 000 x 4 10.5 -> 12.4, 3 000 x 15 18.8 -> 17.9, 8 000 x 4 19.9 -> 20.4, 8 000
@@ -78,18 +78,25 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 //   256           650 x 9.5 13.0 -> 13.7, 650 x 14 16.8 -> 15.2, 700 x 24 23.2 -> 17.6, 700 x 28 (in two parts) 17.6 -> 18.1, 1 000 x 9.3 15.5 -> 15.4, 1 700 x 8
 //                 18.2 -> 19.1, 2 500 x 7.3 21.0 -> 21.4, 4 000 x 6 26.2 -> 26.8, 4 000 x 7 29.9 -> 28.1, 8 000 x 6 42.9 -> 44.7, 8 000 x 7 47.4 -> 46.6,
 //                 12 000 x 6 60.6 -> 62.8, 12 000 x 7 67.8 -> 66.9
-// Beyond 256 MB of output, what the last-level cache holds, its writes reach memory as the 64-byte pieces of rows that a workgroup's
-// 16 channels are, and what that costs per node has to be won back by edges: the line is then a number of neighbours that grows
-// with the logarithm of the output and with the channels (up to 64 channels it does not come to that).  One wave per node -> this
-// one (reading vectors / the step's records), us:
-//   96            40 000 x 5 78 -> 79 / 77, 60 000 x 7 193 -> 193 / 192, 100 000 x 5 291 -> 328 / 321, x 9.3 369 -> 374 / 365, 200 000 x 14 881 -> 805 / 787
-//   128           25 000 x 3.8 51 -> 54 / 54, x 5 60 -> 57 / 56, 60 000 x 9.4 278 -> 292 / 281, x 12 309 -> 301 / 281, 100 000 x 7 416 -> 467 / 457, 400 000 x 14
-//                 2 194 -> 2 392 / 2 326, x 19 2 750 -> 2 641 / 2 590
-//   160           30 000 x 5 124 -> 125 / 125, 60 000 x 7 327 -> 359 / 346, x 12 403 -> 385 / 369, 100 000 x 9.3 605 -> 652 / 634, x 15 756 -> 721 / 695
-//   192           30 000 x 7 170 -> 188 / 174, 60 000 x 9.4 398 -> 460 / 444, x 15 505 -> 498 / 468, 100 000 x 9.3 659 -> 787 / 765, x 17 927 -> 915 / 882
-//   224           30 000 x 7 222 -> 232 / 230, 60 000 x 9.4 490 -> 522 / 506, x 15 616 -> 579 / 553, 100 000 x 9.3 797 -> 891 / 865, x 17 1 132 -> 1 049 / 1 012
-//   256           30 000 x 9.4 261 -> 317 / 300, x 15 333 -> 315 / 280, 60 000 x 15 651 -> 747 / 718, x 25 980 -> 850 / 816, 100 000 x 9.3 839 -> 1 141 / 1 118,
-//                 x 25 1 610 -> 1 557 / 1 494
+// Launched over and over by itself it finds its output in the last-level cache.  Inside a step it does not, and writes that reach
+// memory as the 64-byte pieces of rows that a workgroup's 16 channels are cost more per node than few neighbours win back: from
+// several thousand nodes on the line is a number of neighbours, and beyond 256 MB of output, what that cache holds, one that grows
+// with the logarithm of the output (up to 64 channels it does not come to that).  Energies alone, the whole call, one wave per node
+// -> this one, us:
+//   96   25 000 x 4.9 408 -> 409, x 7 425 -> 419, 45 000 x 4.8 712 -> 715, x 7 742 -> 734
+//   128  6 000 x 5 169 -> 170, 20 000 x 4.9 416 -> 415, 30 000 x 5 615 -> 623, x 7 646 -> 638, 50 000 x 9.3 1 132 -> 1 187, x 13 1 214 -> 1 205
+//   160  12 000 x 2.6 377 -> 382, x 4.8 392 -> 385, 25 000 x 4.9 772 -> 776, 40 000 x 7 1 187 -> 1 228, x 13 1 329 -> 1 278
+//   192  6 000 x 6 260 -> 263, x 8.4 272 -> 270, 20 000 x 6 715 -> 750, x 8.3 745 -> 746, 35 000 x 10 1 257 -> 1 297, x 14 1 336 -> 1 323
+//   224  6 000 x 2.8 305 -> 311, x 5 316 -> 310, 12 000 x 4.8 528 -> 528, 20 000 x 7 878 -> 881, 35 000 x 7 1 500 -> 1 545, x 13 1 661 -> 1 586
+//   256  3 000 x 7 236 -> 240, x 9.5 244 -> 243, 12 000 x 9.3 629 -> 636, x 15 700 -> 677, 20 000 x 7 981 -> 1 031, x 15 1 121 -> 1 100, 35 000 x 11.5 1 825 ->
+//        1 889, x 15 1 931 -> 1 902
+// With forces:
+//   128  35 000 x 6 1 548 -> 1 545, 60 000 x 8.3 2 696 -> 2 752, x 10.5 2 880 -> 2 881, 100 000 x 10.4 4 904 -> 4 990, x 13 5 154 -> 5 133
+//   192  20 000 x 8.3 1 509 -> 1 510, 35 000 x 8.2 2 516 -> 2 543, x 10.4 2 670 -> 2 670, 60 000 x 8.3 4 270 -> 4 328, x 13 4 793 -> 4 743, 100 000 x 10.4 7 572 -> 7 700,
+//        x 16 8 652 -> 8 485
+//   224  35 000 x 6 3 000 -> 3 012, x 8.2 3 206 -> 3 164, 60 000 x 6 5 115 -> 5 130, x 8.3 5 454 -> 5 368
+//   256  6 000 x 8.4 765 -> 778, x 16 882 -> 880, 12 000 x 8.2 1 279 -> 1 318, x 13 1 408 -> 1 393, 20 000 x 8.3 2 055 -> 2 076, x 13 2 272 -> 2 249, 60 000 x 10.5 6 442 ->
+//        6 559, x 16 7 247 -> 7 153, 80 000 x 13 9 053 -> 9 270, x 19 10 491 -> 10 346
 inline int64_t min_nodes_per_workgroup(int channels) { return channels == 32 ? 60 : (channels == 160 ? 64 : 76); }
 inline int64_t min_edges(int64_t nnodes, int channels) {
   struct Line {
@@ -100,12 +107,12 @@ inline int64_t min_edges(int64_t nnodes, int channels) {
     switch (channels) {
       case 32: return {0, 0.0, 0.0};
       case 64: return {26000, 0.0, 0.0};
-      case 96: return {std::max(34000 + 6 * nnodes / 5, 4 * nnodes), 6.5, 1.1};
-      case 128: return {std::max(24000 + 2 * nnodes, 17 * nnodes / 4), 6.7, 3.0};
-      case 160: return {3500 + 7 * nnodes / 2, 5.0, 3.9};
-      case 192: return {4000 + 11 * nnodes / 2, 6.5, 4.6};
-      case 224: return {8000 + 3 * nnodes, 5.3, 3.8};
-      default: return {5000 + 23 * nnodes / 4, 5.0, 7.5};
+      case 96: return {std::max(34000 + 6 * nnodes / 5, 5 * nnodes), 5.5, 2.0};
+      case 128: return {std::max(24000 + 2 * nnodes, 9 * nnodes / 2), 7.0, 3.2};
+      case 160: return {std::max(3500 + 7 * nnodes / 2, 21 * nnodes / 5), 6.5, 2.5};
+      case 192: return {std::max(4000 + 11 * nnodes / 2, 15 * nnodes / 2), 9.0, 1.9};
+      case 224: return {std::max(8000 + 3 * nnodes, 9 * nnodes / 2), 6.0, 1.5};
+      default: return {std::max(5000 + 23 * nnodes / 4, 21 * nnodes / 2), 11.0, 2.0};
     }
   }();
   const double caches = 64.0 * static_cast<double>(nnodes) * channels / (1 << 28);  // 16 components of 4 bytes in 256 MB
