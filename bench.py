@@ -79,21 +79,30 @@ def traffic_of(table, kernels):
 
 
 def forward_kernel_name(C, N, E, in_step=False):
-    """Kernel that runs the fused forward from edge vectors at this shape (csrc/mp_sliced.hip: sliced_forward_applies; the
-    benchmark's spline table has 256 knots; the one-call step hands it an edge's vector and sender as one record)."""
-    share = 256 // (2 * (C // 16))  # workgroups per pair of degrees and 16-channel slice on 256 compute units
-    enough = {32: 0, 64: 26000, 96: 34000 + 6 * N // 5, 128: 24000 + 2 * N, 160: 3500 + 7 * N // 2,
-              192: 4000 + 11 * N // 2, 224: 8000 + 3 * N}.get(C, 8000 + 5 * N)
-    if {32: 60, 160: 64}.get(C, 76) * share < N < 2**24 and C % 16 == 0 and N * C < 2**30 and E >= max(enough, 1):
+    """Kernel that runs the fused forward from edge vectors at this shape, as the library says (the benchmark's spline table has
+    256 knots; the one-call step hands it an edge's vector and sender as one record)."""
+    from cuda_mace import _cabi
+
+    if _cabi.lib.cm_mp_edge_forward_kernel(N, E, C, 256) == 1:
         return "mp_edge_forward_sliced_kernel<%s>" % ("true" if in_step else "false")
     return "mp_spline_forward_kernel<%d,true>" % C
 
 
 def backward_kernel_name(C, N, E):
-    """Kernel that runs the fused backward edge pass without gX (csrc/mp_spline.hip: launch_edge)."""
-    if C in (160, 192, 224):
+    """Kernel that runs the fused backward edge pass without gX, as the library says."""
+    from cuda_mace import _cabi
+
+    if _cabi.lib.cm_mp_edge_backward_kernel(N, E, C) == 1:
         return "mp_edge_backward_steps_kernel<%d,true,false>" % C
     return "mp_spline_backward_edge_kernel<%d,true,true,true,false>" % C
+
+
+def spline_backward_kernel_name(C, E):
+    """Kernel that runs the spline's backward to the four degrees of C channels, as the library says."""
+    from cuda_mace import _cabi
+
+    return ("spline_backward_kernel", "spline_backward_sorted_kernel<%d>" % min(-(-C // 32), 4),
+            "spline_backward_sliced_kernel")[_cabi.lib.cm_spline_backward_kernel(E, 256, 4 * C)]
 
 
 def linear_kernel_name(C, N):
@@ -206,8 +215,7 @@ def op_cases(torch, cabi, N, E, C, ne, rcv, snd, with_fused=True, with_node_ops=
             ("spline forward (R only)", "spline_forward_sliced_kernel" if E >= 1 << 15 else "spline_forward_kernel<false>",
              4 * (E + 4 * E * C),
              lambda: cabi.spline_forward(r, knots, coeffs, float(h), 5.0)),
-            ("spline backward", "spline_backward_sliced_kernel" if E >= 1 << 19 else
-             ("spline_backward_sorted_kernel<%d>" % min(-(-C // 32), 4) if E >= 1 << 15 else "spline_backward_kernel"),
+            ("spline backward", spline_backward_kernel_name(C, E),
              4 * (4 * E * C + 2 * E),
              lambda: cabi.spline_backward(r, knots, coeffs, R.view(E, 4 * C), float(h), 5.0)),
             ("symmetric contraction forward + gradient", "symcon_lmax3_kernel<float,true>", 4 * (33 * N * C + N),

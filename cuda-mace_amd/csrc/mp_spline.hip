@@ -986,6 +986,17 @@ extern "C" int cm_mp_spline_backward(const float *X, const float *Y, const float
   return rc;
 }
 
+extern "C" int cm_mp_edge_forward_kernel(int64_t nnodes, int64_t nedges, int channels, int nknots) {
+  return cm_channels_supported(channels) && nnodes > 0 && cm::mp::sliced_forward_applies(nnodes, nedges, channels, nknots) ? 1 : 0;
+}
+
+extern "C" int cm_mp_edge_backward_kernel(int64_t nnodes, int64_t nedges, int channels) {
+  if (nnodes <= 0) return 0;
+  bool steps = false;
+  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, cm::mp::parts_for(nnodes, nedges)));
+  return steps ? 1 : 0;
+}
+
 extern "C" int cm_mp_edge_forward(const float *X, const float *vectors, const float *r_knots, const float *coeffs, int nknots,
                                   float r_width, float r_max, const int32_t *sender, const int32_t *first_occ,
                                   int64_t nnodes, int64_t nedges, int channels, float *out, cm_stream_t stream) {

@@ -553,6 +553,12 @@ extern "C" int cm_spline_forward(const float *r, const float *r_knots, const flo
   return cm::check_launch("cm_spline_forward");
 }
 
+extern "C" int cm_spline_backward_kernel(int64_t nedges, int nknots, int noutputs) {
+  if (nknots < 2 || noutputs < 1) return 0;
+  if (cm::spline_sliced_applies(nedges, nknots, noutputs) && nedges >= cm::spline_backward_sliced_from(nknots, noutputs)) return 2;
+  return nedges >= cm::kSpMinEdges && nknots <= cm::kSpSortMaxKnots ? 1 : 0;
+}
+
 extern "C" int cm_spline_backward(const float *r, const float *r_knots, const float *coeffs, const float *grad_R,
                                   int64_t nedges, int nknots, int noutputs, float r_width, float r_max,
                                   float *grad_r, cm_stream_t stream) {
@@ -562,12 +568,13 @@ extern "C" int cm_spline_backward(const float *r, const float *r_knots, const fl
   CM_REQUIRE(r_width > 0.f, "cm_spline_backward: r_width must be positive");
   if (nedges == 0) return CM_OK;
   CM_REQUIRE(r && r_knots && coeffs && grad_R && grad_r, "cm_spline_backward: NULL pointer");
-  if (cm::spline_sliced_applies(nedges, nknots, noutputs) && nedges >= cm::spline_backward_sliced_from(nknots, noutputs)) {
+  const int kernel = cm_spline_backward_kernel(nedges, nknots, noutputs);
+  if (kernel == 2) {
     cm::launch_spline_backward_sliced(r, r_knots, coeffs, grad_R, nedges, nknots, noutputs, r_width, r_max, grad_r,
                                       cm::as_stream(stream));
     return cm::check_launch("cm_spline_backward");
   }
-  if (nedges >= cm::kSpMinEdges && nknots <= cm::kSpSortMaxKnots) {
+  if (kernel == 1) {
     cm::launch_spline_backward_sorted(r, r_knots, coeffs, grad_R, nedges, nknots, noutputs, r_width, r_max, grad_r,
                                       cm::as_stream(stream));
     return cm::check_launch("cm_spline_backward");

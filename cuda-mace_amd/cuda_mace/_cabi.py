@@ -49,6 +49,8 @@ SIGNATURES = {
     "cm_mp_backward_per_m": (_i32, [_p] * 8 + [_i64, _i64, _i32] + [_p] * 5),
     "cm_mp_spline_forward": (_i32, [_p] * 5 + [_i32, _f32, _f32, _p, _p, _i64, _i64, _i32, _p, _p]),
     "cm_mp_spline_backward": (_i32, [_p] * 5 + [_i32, _f32, _f32] + [_p] * 5 + [_i64, _i64, _i32] + [_p] * 5),
+    "cm_mp_edge_forward_kernel": (_i32, [_i64, _i64, _i32, _i32]),
+    "cm_mp_edge_backward_kernel": (_i32, [_i64, _i64, _i32]),
     "cm_mp_edge_forward": (_i32, [_p] * 4 + [_i32, _f32, _f32, _p, _p, _i64, _i64, _i32, _p, _p]),
     "cm_mp_edge_backward": (_i32, [_p] * 4 + [_i32, _f32, _f32] + [_p] * 5 + [_i64, _i64, _i32] + [_p] * 4),
     "cm_edge_geometry_forward": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _p, _p, _p]),
@@ -56,6 +58,7 @@ SIGNATURES = {
     "cm_sh_forward": (_i32, [_p, _i64, _p, _p]),
     "cm_sh_backward": (_i32, [_p, _p, _i64, _p, _p]),
     "cm_spline_forward": (_i32, [_p, _p, _p, _i64, _i32, _i32, _f32, _f32, _p, _p, _p]),
+    "cm_spline_backward_kernel": (_i32, [_i64, _i32, _i32]),
     "cm_spline_backward": (_i32, [_p, _p, _p, _p, _i64, _i32, _i32, _f32, _f32, _p, _p]),
     "cm_linear": (_i32, [_p, _p, _p, _p, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _p, _p, _p, _p]),
     "cm_symcon_tables": (_i32, [_p, _p, _p, _i32, _p, _p, _p, _i32, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _p, _p, _p, _p]),

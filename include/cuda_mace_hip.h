@@ -178,7 +178,12 @@ int cm_mp_spline_backward(const float *X, const float *Y, const float *r, const 
  * (models/InvariantMACE.py:306, 320, 105-112); Y[16, nedges], grad_Y and grad_r never exist.
  *   vectors fp32 [nedges, 3].  Backward: grad_vectors fp32 [nedges, 3] (may be NULL) is the full gradient with respect
  *   to the edge vector, harmonics Jacobian and radial part included; gX as in cm_mp_backward.
+ * cm_mp_edge_forward_kernel / cm_mp_edge_backward_kernel say which kernel a launch of these sizes takes, so that whoever names
+ *   it in a profile or a benchmark need not repeat the rule: 0 is the kernel with one wave per receiver node (backward: an edge
+ *   per wave or part of one), 1 the forward with the radial table in LDS or the backward in steps of four edges.
  */
+int cm_mp_edge_forward_kernel(int64_t nnodes, int64_t nedges, int channels, int nknots);
+int cm_mp_edge_backward_kernel(int64_t nnodes, int64_t nedges, int channels);
 int cm_mp_edge_forward(const float *X, const float *vectors, const float *r_knots, const float *coeffs,
                        int nknots, float r_width, float r_max, const int32_t *sender,
                        const int32_t *first_occ, int64_t nnodes, int64_t nedges, int channels,
@@ -236,7 +241,10 @@ int cm_edge_geometry_backward(const double *positions, const int32_t *row_a, con
  *   r [nedges]; r_knots [nknots]; coeffs [nknots - 1, 4, noutputs]; R_out [nedges, noutputs];
  *   R_deriv [nedges, noutputs] or NULL.  noutputs must be a multiple of 4.
  * Backward: grad_r[e] = sum_j grad_R[e, j] * dR/dr[e, j], with dR/dr recomputed from the table.
+ * cm_spline_backward_kernel: which kernel a backward of these sizes takes (0 one wave per edge, 1 edges in the order of their knot
+ *   intervals, 2 the table in LDS).
  */
+int cm_spline_backward_kernel(int64_t nedges, int nknots, int noutputs);
 int cm_spline_forward(const float *r, const float *r_knots, const float *coeffs, int64_t nedges,
                       int nknots, int noutputs, float r_width, float r_max, float *R_out,
                       float *R_deriv, cm_stream_t stream);

@@ -45,6 +45,29 @@ def test_host_side_validation_needs_no_gpu():
     assert lib.cm_stable_key_sort_workspace(100, 10) >= 4 * 120
 
 
+def test_the_library_names_the_kernels_it_takes():
+    """Which kernel a launch takes, at sizes far from the lines between them and just on their two sides, on 256 compute units."""
+    lib = ctypes.CDLL(LIB)
+    i64 = ctypes.c_int64
+    forward = lambda n, e, c, k=256: lib.cm_mp_edge_forward_kernel(i64(n), i64(e), c, k)
+    assert forward(25000, 1301200, 128) == 1 and forward(100000, 5206338, 192) == 1 and forward(60000, 200000, 64) == 1
+    assert forward(25000, 1301200, 128, 300) == 0  # the table does not fit LDS
+    assert forward(500, 50000, 128) == 0 and forward(25000, 0, 128) == 0 and forward(0, 0, 128) == 0 and forward(25000, 1301200, 48) == 0
+    assert forward(20000, 89999, 128) == 0 and forward(20000, 90000, 128) == 1
+    # output of twice the last-level cache and more: 11 neighbours, and two more for every doubling
+    n = 1 << 15
+    assert forward(n, 13 * n - 1, 256) == 0 and forward(n, 13 * n, 256) == 1 and forward(2 * n, 15 * 2 * n - 1, 256) == 0
+    assert forward(2 * n, 15 * 2 * n, 256) == 1
+    backward = lambda n, e, c: lib.cm_mp_edge_backward_kernel(i64(n), i64(e), c)
+    assert [backward(3000, 150000, c) for c in (32, 64, 96, 128, 160, 192, 224, 256)] == [0, 0, 0, 0, 1, 1, 1, 0]
+    assert backward(3000, 14999, 192) == 0 and backward(3000, 15000, 192) == 1 and backward(3000, 14999, 224) == 0
+    assert backward(2048, 100000, 224) == 0 and backward(1536, 36000, 224) == 1 and backward(0, 0, 192) == 0
+    spline = lambda e, j, k=256: lib.cm_spline_backward_kernel(i64(e), k, j)
+    assert [spline(e, 512) for e in (1000, 32767, 32768, 719999, 720000)] == [0, 0, 1, 1, 2]
+    assert [spline(e, 4) for e in (39999, 40000)] == [1, 2] and [spline(e, 260) for e in (524287, 524288)] == [1, 2]
+    assert spline(2000000, 512, 300) == 1 and spline(2000000, 512, (1 << 20) + 1) == 0
+
+
 def test_binding_rejects_host_tensors():
     import pytest
     import torch
