@@ -499,7 +499,7 @@ int cm_node_glue_backward(const float *gX2, const float *d_h2, const float *up_W
  * Python forward over its TorchScript classes followed by an autograd backward (models/InvariantMACE.py:246-379:
  * interactions :76-160, products :330, readouts :336, scale/shift :344, forces through get_outputs :354): same kernels,
  * same order, same numbers as that sequence, without a Python interpreter or an autograd engine between the launches
- * (18 launches up to 128 channels, 20 with few nodes at 96 and 128, 24 beyond; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
+ * (16 launches up to 128 channels, 18 with few nodes at 96 and 128, 23 beyond; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
  *
  * cm_mace_weights: the model's frozen weights in the layouts the op modules hold them (device pointers).
  *   spline[t]      [nknots - 1, 4, 4C]   radial spline table of layer t (cm_spline_forward's coeffs)

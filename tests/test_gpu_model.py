@@ -571,7 +571,7 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
 @pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32)])
 def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
     """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 32
-    and 64 nodes with a partly filled last one, against the separate launches: bit for bit, for forces and for energies alone,
+    and 128 nodes with a partly filled last one, against the separate launches: bit for bit, for forces and for energies alone,
     with weights on the node energies and without."""
     data = make_system(natoms, 4, seed=7, density=None, cluster_box=12.0) if natoms < 130 else make_system(natoms, 4, seed=7, density=0.015)
     _, model = _build(channels, (1, 6, 7, 8), data, seed=8)

@@ -282,9 +282,10 @@ def test_mp_edge_forward_many_nodes_agrees_with_harmonics_and_lengths_path(cabi)
 
 @pytest.mark.parametrize("case", [(1024, 6, 160, 0.2, 21, 256, 0), (1100, 13, 160, 0.0, 22, 600, 150), (1024, 5, 192, 0.2, 23, 256, 0), (1024, 15, 192, 0.2, 25, 256, 0),
                                   (1060, 17, 192, 0.0, 24, 2, 129)], ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
-def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
-    """Widths on both sides of the kernel with a row of 16 lanes per edge: nodes with every remainder of a group of four edges, one
-    with more than one and more than two chunks of 64, dead edges in between, knots in LDS and in memory, a table of one interval."""
+def test_mp_edge_backward_of_four_edges_per_step(cabi, case):
+    """The kernel with a row of 16 lanes per edge (and, at five edges per node and 192 channels, the one with an edge per wave):
+    nodes with every remainder of a group of four edges, one with more than one and more than two chunks of 64, dead edges in
+    between, knots in LDS and in memory, a table of one interval."""
     nnodes, C = case[0], case[2]
     snd, rcv, X, vec, knots, coeffs, h = _edge_case(*case)
     degrees = torch.bincount(rcv.long(), minlength=nnodes)
@@ -313,7 +314,7 @@ def test_mp_edge_backward_on_the_matrix_cores(cabi, case):
 def test_mp_edge_backward_few_and_many_nodes(cabi, case):
     """Few nodes (an edge range cut into parts) and many, every width class, partly filled groups, trips and chunks, and tables on
     both sides of what the copy of the knots takes (four knots at a time, up to 256 or 512)."""
-    test_mp_edge_backward_on_the_matrix_cores(cabi, case)
+    test_mp_edge_backward_of_four_edges_per_step(cabi, case)
 
 
 @pytest.mark.parametrize("case", [(600, 4, 192, 0.0, 41, 256, 70), (600, 6, 192, 0.0, 42, 256, 70), (700, 2, 224, 0.0, 43, 256, 66),
@@ -327,7 +328,7 @@ def test_mp_edge_backward_on_both_sides_of_the_line(cabi, case):
     nnodes, C, E = case[0], case[2], _edge_case(*case)[0].numel()
     per_node = {(600, 4): 5, (600, 6): 5, (700, 2): 2.5, (700, 4): 2.5, (2049, 4): 5, (2049, 6): 5}.get(case[:2])
     assert per_node is None or (E < per_node * nnodes) == (case[1] < per_node)
-    test_mp_edge_backward_on_the_matrix_cores(cabi, case)
+    test_mp_edge_backward_of_four_edges_per_step(cabi, case)
 
 
 @pytest.mark.parametrize("nnodes,C", [(1750, 96), (1400, 128), (1000, 160), (900, 192), (700, 256)])
