@@ -562,12 +562,13 @@ def main():
             flops = 32 * N * C * C
             tf = flops / (t_lin * 1e-3) / 1e12
             lin_bytes = 4 * (32 * N * C + 4 * C * C)
+            # resident weights: two fp16 pieces per operand, three products; the others: three bf16 pieces, six
+            pieces = 3 if linear_kernel_name(C, N).startswith(("linear_resident", "linear_wide")) else 6
             others.append(entry(linear_kernel_name(C, N), lin_bytes, t_lin, launches_timed=launches("linear"),
-                                matrix_cores={"fp32_equivalent_TFLOP/s": round(tf, 1), "instruction_TFLOP/s_bf16": round(6 * tf, 1),
-                                              "frac_of_bf16_peak": round(6 * tf / 2500.0, 4)},
+                                matrix_cores={"fp32_equivalent_TFLOP/s": round(tf, 1), "instruction_TFLOP/s_16_bit": round(pieces * tf, 1),
+                                              "frac_of_16_bit_peak": round(pieces * tf / 2500.0, 4)},
                                 note="[N,16,C] x [C,C] channel mixing: bound by its memory traffic, not by the matrix cores "
-                                     "(every fp32 product is six bf16 piece products on v_mfma_f32_32x32x16_bf16, which "
-                                     "keeps the pipes about a third busy)"))
+                                     "(every fp32 product is %d products of 16-bit pieces on the matrix cores)" % pieces))
             others[-1]["traffic"] = traffic_of(traffic["standalone"], linear_kernel_name(C, N)) if default_workload else None
     else:
         # The model drives the tabulated ops through the TorchScript classes, which the Python-side brackets above do not

@@ -14,7 +14,7 @@
 // a single launch; per-element weights are selected through a node permutation that lists the nodes group
 // by group, without any host synchronisation.
 //
-// Arithmetic: every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
+// Arithmetic (the two kernels with resident weights at the end of this file have their own): every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
 // in all), and the product is accumulated in fp32 from the six piece products that matter (hi.hi, hi.mid, mid.hi, hi.lo,
 // lo.hi, mid.mid; the dropped ones are below 2^-24 of the product) on v_mfma_f32_32x32x16_bf16, whose rate is 16x that of
 // the fp32 matrix instruction.  The result matches an fp32 GEMM to rounding (measured rms error 1.7e-7 against fp64 on
@@ -703,9 +703,17 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 // The kernels above stage the K x Nout weight block again for every tile of 128 rows (as many bytes from L2 as the tile
 // has from HBM) and walk K in barrier-separated phases.  Here a launch has one workgroup per compute unit, and a
 // workgroup takes a contiguous piece of the list of all 32-row tiles, ordered by (weight group, l, node tile, m within
-// l), so that it needs one or two weight blocks in its whole life: it splits a block once into three bf16 planes that
-// cover all of K (102 KB at 128 x 128) and then its four waves run independently of each other, one 32-row tile at a
+// l), so that it needs one or two weight blocks in its whole life: it splits a block once into two fp16 planes that
+// cover all of K (70 KB at 128 x 128) and then its four waves run independently of each other, one 32-row tile at a
 // time, with no barrier until the weight block changes.
+//
+// Two fp16 pieces per operand and three piece products on v_mfma_f32_32x32x16_f16 (mfma_split.hpp), rows of X and columns of W
+// scaled by powers of two that the output takes back: half the matrix instructions of three bf16 pieces and six products,
+// four vector instructions per value instead of five and a half, two thirds of the fragment reads.  The products with a low piece
+// have an accumulator of their own, so a sum of K terms is rounded K / 16 times.  us and rms error against fp64 (normal
+// values), bf16 -> fp16: 25 000 x 128 90.4 -> 80.3, 1.65e-7 -> 1.13e-7, with a weight block per element 93.4 -> 85.0, with row_scale 97.9 ->
+// 90.9, 1.68e-7 -> 1.15e-7; 96 columns 1.41e-7 -> 1.07e-7, 64 1.12e-7 -> 1.02e-7, equal times at 5 000 and 10 752 nodes (one
+// accumulator: 1.45e-7 at 128, 1.32e-7 at 96, 1.16e-7 at 64).
 //
 // What a wave has in flight lives in registers, not in LDS: the loads of tile i + 1 (16 x 16 bytes per lane at 128
 // columns, whole 128-byte lines of 8 rows per instruction) are issued before tile i is multiplied and land in
@@ -715,7 +723,7 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 // long as both operands agree; it is chosen such that a lane reads two aligned 16-byte pieces.  The operands are swapped
 // with respect to the kernels above (weights as the row operand, X rows as the column operand): a lane's accumulators
 // are then 4 consecutive output columns of one row; a block of 32 columns goes back through the same corner of LDS and
-// leaves as whole lines.  The piece products and their order are those of the kernels above.
+// leaves as whole lines.
 //
 // Contract of the hand-issued memory operations of the tile loop (the loads and the stores): a load names its landing
 // registers at issue time although the data arrives by the explicit wait that precedes their first use, which is
@@ -741,6 +749,18 @@ constexpr int kResMinNodes = 2048;
 constexpr int kOutLd = 36;            // floats per row of a wave's output staging block (32 columns + 16 bytes)
 constexpr int kResSegNodeTiles = 64;  // node tiles whose row numbers a segment keeps in LDS
 
+__device__ __forceinline__ float largest4(f4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
+// largest value over eight neighbouring lanes, in all of them
+__device__ __forceinline__ float max_over_8(float v) {
+  auto with = [&](auto ctrl) {
+    constexpr int kCtrl = decltype(ctrl)::value;
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false)));
+  };
+  v = with(std::integral_constant<int, 0xB1>{});   // lane ^ 1
+  v = with(std::integral_constant<int, 0x4E>{});   // lane ^ 2
+  return with(std::integral_constant<int, 0x141>{});  // the eight lanes in reverse
+}
+
 template <int K, int NT, bool SCALED>
 __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
     const float *__restrict__ X, const float *__restrict__ WT, const int32_t *__restrict__ node_perm,
@@ -749,7 +769,9 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
   constexpr int NOUT = 32 * NT;  // columns of this workgroup: blockIdx.y * NOUT onwards of the ldo columns of OUT
   constexpr int LD = K + 8;      // row stride of a plane in elements: an odd number of 16-byte units
   constexpr int KS = K / 16;
-  __shared__ __attribute__((aligned(16))) __bf16 sW[3 * NOUT * LD];
+  __shared__ __attribute__((aligned(16))) _Float16 sW[2 * NOUT * LD];
+  __shared__ __attribute__((aligned(16))) float sColumn[NOUT];  // largest magnitude of a weight column, then what takes its scale back
+  __shared__ float sRowMax[kResWaves * 32];
   __shared__ int sId[kResSegNodeTiles * 32];
   constexpr int kChunk = K <= 96 ? K : 64;  // columns of X per trip through LDS
   constexpr int kTLd = kChunk + 4;          // floats per row of the transposition block: an odd number of 16-byte units
@@ -819,7 +841,7 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       sId[r] = node;
     }
     if (g != staged_g || l != staged_l) {
-      // W^T[c0 + j, :] of block (g, l) -> three planes; inside every 16 k the two middle groups of four trade places, so
+      // W^T[c0 + j, :] of block (g, l) -> two planes; inside every 16 k the two middle groups of four trade places, so
       // that the 8 values a lane reads at 16 s + 8 half are k = 16 s + 4 half + {0..3, 8..11}
       const float *Wg = WT + ((static_cast<int64_t>(g) * 4 + l) * ldo + c0) * K;
       // all loads of a thread first (16 at 128 x 128), then the splits: one trip through L2 instead of one per piece
@@ -831,18 +853,28 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
         const int q = it * (kResWaves * kWave) + tid;
         wv[it] = ld4(Wg + static_cast<int64_t>(q / (K / 4)) * K + 4 * (q % (K / 4)));
       }
+      if (tid < NOUT) sColumn[tid] = 0.f;
+      __syncthreads();
+      // eight neighbouring threads hold pieces of one column (K / 4 is a multiple of eight)
+#pragma unroll
+      for (int it = 0; it < kPieces; ++it) {
+        const float big = max_over_8(largest4(wv[it]));
+        if (tid % 8 == 0) atomicMax(reinterpret_cast<unsigned *>(sColumn) + (it * (kResWaves * kWave) + tid) / (K / 4), __float_as_uint(big));
+      }
+      __syncthreads();
 #pragma unroll
       for (int it = 0; it < kPieces; ++it) {
         const int q = it * (kResWaves * kWave) + tid;
         const int j = q / (K / 4), kq = q % (K / 4);
-        bf16x4 h, md, lw;
-        split3(wv[it], h, md, lw);
+        f16x4 h, lw;
+        split2(wv[it], piece_scale(sColumn[j], kLeastColumnExponent).s, h, lw);
         const int sub = kq & 3;
         const int at = j * LD + 16 * (kq >> 2) + 4 * (sub == 1 ? 2 : (sub == 2 ? 1 : sub));
-        *reinterpret_cast<bf16x4 *>(sW + at) = h;
-        *reinterpret_cast<bf16x4 *>(sW + NOUT * LD + at) = md;
-        *reinterpret_cast<bf16x4 *>(sW + 2 * NOUT * LD + at) = lw;
+        *reinterpret_cast<f16x4 *>(sW + at) = h;
+        *reinterpret_cast<f16x4 *>(sW + NOUT * LD + at) = lw;
       }
+      __syncthreads();
+      if (tid < NOUT) sColumn[tid] = ldexpf(scale, piece_scale(sColumn[tid], kLeastColumnExponent).exponent);
       staged_g = g;
       staged_l = l;
     }
@@ -906,7 +938,7 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
         }
       }
     };
-    const __bf16 *wl = sW + mrow * LD + 8 * half;
+    const _Float16 *wl = sW + mrow * LD + 8 * half;
     int m_next, tb_next;
     issue(wb, m_next, tb_next);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -914,11 +946,12 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NT) : "memory");
       const int m_cur = m_next, tb_cur = tb_next;
       f4 cur[2 * KS];
+      float big[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < kChunks; ++c) {
         wave_lds_fence();
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg)
+        for (int rg = 0; rg < 4; ++rg) {
 #pragma unroll
           for (int ln = 0; ln < kLines; ++ln) {
             const int j = (c * 4 + rg) * kLines + ln;
@@ -928,8 +961,14 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
               asm volatile("; landed %0" : "+a"(sland[j]));
               v *= sland[j];
             }
+            big[rg] = fmaxf(big[rg], largest4(v));
             *reinterpret_cast<f4 *>(stg + (8 * rg + orow) * kTLd + 32 * ln + 4 * opiece) = v;
           }
+          if (c == kChunks - 1) {  // the eight lanes of a row have all of it
+            const float row = max_over_8(big[rg]);
+            if (opiece == 0) sRowMax[32 * wave + 8 * rg + orow] = row;
+          }
+        }
         wave_lds_fence();
         // k step s of the chunk: the lane's values are columns 16 s + 4 half + {0..3} and 16 s + 8 + 4 half + {0..3}
 #pragma unroll
@@ -941,52 +980,46 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       }
 #pragma unroll
       for (int j = 0; j < 2 * KS; ++j) asm volatile("" : "+v"(cur[j]));
+      const PieceScale row = piece_scale(sRowMax[32 * wave + mrow], kLeastRowExponent);
       if (idx + 1 < we) issue(idx + 1, m_next, tb_next);
 
-      v16f acc[NT];
+      v16f acc[NT], acs[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[t][r] = acs[t][r] = 0.f;
       // One wave per SIMD: nothing but this wave's own instruction stream can fill the issue slots between two matrix
       // instructions (32 cycles apart), so the k loop is pipelined in the source: the pieces of X and the weight fragments of
       // step s + 1 are prepared while the 6 NT matrix instructions of step s run, and the scheduler is told to weave them
       // (per matrix instruction: three vector instructions, and an LDS read for the first 3 NT of them).
-      constexpr int kSplitOps = (64 + 6 * NT - 1) / (6 * NT);  // the split of a step is about 60 vector instructions
-      bf16x8 xq[2][3], wq[2][NT][3];
+      constexpr int kSplitOps = (32 + 3 * NT - 1) / (3 * NT);  // the split of a step is about 24 vector instructions
+      f16x8 xq[2][2], wq[2][NT][2];
       auto prepare = [&](int s, auto par) {
         constexpr int P = decltype(par)::value;
-        bf16x4 h0, m0, l0, h1, m1, l1;
-        split3(cur[2 * s], h0, m0, l0);
-        split3(cur[2 * s + 1], h1, m1, l1);
+        f16x4 h0, l0, h1, l1;
+        split2(cur[2 * s], row.s, h0, l0);
+        split2(cur[2 * s + 1], row.s, h1, l1);
         xq[P][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-        xq[P][1] = __builtin_shufflevector(m0, m1, 0, 1, 2, 3, 4, 5, 6, 7);
-        xq[P][2] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        xq[P][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int p = 0; p < 3; ++p) wq[P][t][p] = *reinterpret_cast<const bf16x8 *>(wl + p * NOUT * LD + 32 * t * LD + 16 * s);
+          for (int p = 0; p < 2; ++p) wq[P][t][p] = *reinterpret_cast<const f16x8 *>(wl + p * NOUT * LD + 32 * t * LD + 16 * s);
       };
       auto step = [&](int s, auto par) {
         constexpr int P = decltype(par)::value;
         if (s + 1 < KS) prepare(s + 1, std::integral_constant<int, 1 - P>{});
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][0], xq[P][2], acc[t], 0, 0, 0);
+        for (int t = 0; t < NT; ++t) acs[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][0], xq[P][1], acs[t], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][2], xq[P][0], acc[t], 0, 0, 0);
+        for (int t = 0; t < NT; ++t) acs[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][1], xq[P][0], acs[t], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][1], xq[P][1], acc[t], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][0], xq[P][1], acc[t], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][1], xq[P][0], acc[t], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wq[P][t][0], xq[P][0], acc[t], 0, 0, 0);
+        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][0], xq[P][0], acc[t], 0, 0, 0);
         if (s + 1 < KS) {
 #pragma unroll
-          for (int i = 0; i < 6 * NT; ++i) {
+          for (int i = 0; i < 3 * NT; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // one matrix instruction
-            if (i < 3 * NT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+            if (i < 2 * NT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
             __builtin_amdgcn_sched_group_barrier(0x002, kSplitOps, 0);          // a share of the split arithmetic
           }
         }
@@ -1000,6 +1033,8 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
         step(s, std::integral_constant<int, 0>{});
         if (s + 1 < KS) step(s + 1, std::integral_constant<int, 1>{});
       }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] += acs[t];
       // accumulator r of a lane: output column 32 t + 8 (r / 4) + 4 half + r % 4 of row mrow of the tile.  Stored from
       // here a row would leave in 32-byte pieces; a block of 32 columns goes through the wave's own corner of LDS instead
       // (rows padded to 9 x 16 bytes: conflict-free both ways) and leaves as whole 128-byte lines, 8 rows per store.
@@ -1011,8 +1046,12 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       for (int t = 0; t < NT; ++t) {
         wave_lds_fence();
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<f4 *>(stg + mrow * kOutLd + 8 * q + 4 * half) = f4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]} * scale;
+        for (int q = 0; q < 4; ++q) {
+          f4 v = f4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]} * ld4(sColumn + 32 * t + 8 * q + 4 * half);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] = __builtin_ldexpf(v[k], row.exponent);
+          st4(stg + mrow * kOutLd + 8 * q + 4 * half, v);
+        }
         wave_lds_fence();
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1034,17 +1073,19 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
 // again for every 128 rows in barrier-separated phases that one or two waves per SIMD cannot overlap: 192 columns ran at
 // 2.8-3.0 TB/s of their bytes, 256 at 2.2.  The register file of a compute unit holds 512 KB: here a workgroup takes a
 // contiguous piece of the list of all 16-row tiles (as the kernel above does), wave w keeps the pieces of its 16 CB weight
-// columns for all of K in its registers (6 CB K / 16 of them) until the weight block changes, and all waves multiply the
+// columns for all of K in its registers (CB K / 4 of them) until the weight block changes, and all waves multiply the
 // same tile of X rows, whose piece planes they share through LDS, double-buffered with one barrier per tile.  X goes
 // global -> LDS as raw fp32 by direct loads; a wave splits exactly the pieces it fetched itself, so only the planes are
 // shared.  The waves of a SIMD take turns in the order of their phases: every other one multiplies the current tile before
 // it splits the next.
 //
 // Operands as in the kernel above (weights as the row operand): a lane's accumulators are four consecutive output columns of
-// one row, stored as 16 bytes.  v_mfma_f32_16x16x32_bf16: K steps of 32, piece products in the order of the kernels above.
+// one row, stored as 16 bytes.  Two fp16 pieces per operand as above, v_mfma_f32_16x16x32_f16: K steps of 32.  A row is
+// fetched by several waves, and its scale needs its largest value: a wave takes its pieces of tile k + 2 from LDS into registers
+// and adds them to the maxima of the rows (LDS atomics) while tile k is multiplied, and splits them a barrier later.
 //
-// Vector-memory operations of the tile loop are issued from assembly: the loads of tile k + 2 right after the split of tile
-// k + 1, then the stores of a tile; the wait before a split lets exactly those stores stay out.
+// Vector-memory operations of the tile loop are issued from assembly: the loads of tile k + 3 right after tile k + 2 has been
+// taken, then the stores of a tile; the wait before a tile is taken lets exactly those stores stay out.
 //
 // CB: 16 columns per wave give 10, 12 and 14 waves, three or four per SIMD (32 columns per wave: 5, 6 and 7 waves, two on
 // some SIMDs and one on others; 5-8 % slower at 160 and 192); at 256 columns 32 per wave (8 waves) are equal up to 20 000
@@ -1053,8 +1094,9 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
 //
 // Measured against the tiled kernels (plain / row_scale): 100 000 x 192 810 / 860 -> 655 / 675 us, 50 000 x 160 326 / 345 ->
 // 285 / 290, 20 000 x 224 255 / 272 -> 180 / 190, 40 000 x 256 595 / 643 -> 415 / 445, 12 000 x 256 183 / 198 -> 122 / 145,
-// equal at 2 048 nodes.  Without its matrix instructions 192 columns take 520 us (4.7 TB/s, the rate of a copy), without
-// loads, stores and split 514 us: what is left is their overlap.
+// equal at 2 048 nodes.  That was with three bf16 pieces and six products, whose matrix instructions alone took 514 of the 655
+// us at 192 columns; with two fp16 pieces, us and rms error against fp64: 100 000 x 192 647 -> 557, 1.96e-7 -> 1.24e-7, 20 000 x 224
+// 184 -> 134, 2.14e-7 -> 1.29e-7, 12 000 x 256 137 -> 110, 2.31e-7 -> 1.34e-7, 10 007 x 160 64.8 -> 61.1, 1.77e-7 -> 1.18e-7.
 // -----------------------------------------------------------------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kWideMinScalarNodes = 8192;
@@ -1075,7 +1117,9 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
   constexpr int PIECES = TR * K / 4 / (WAVES * kWave);  // 16-byte pieces of a tile per thread
   constexpr int STORES = CB * RB;             // per wave and tile
   constexpr int kSegTiles = kWideSegRows / TR;
-  __shared__ __attribute__((aligned(16))) __bf16 sP[2][3][TR * LD];
+  __shared__ __attribute__((aligned(16))) _Float16 sP[2][2][TR * LD];
+  __shared__ unsigned sRowMax[4][TR];  // largest magnitude of a row (its bits): of the tile multiplied, the next two, and one being cleared
+  __shared__ __attribute__((aligned(16))) float sColumn[K];
   __shared__ __attribute__((aligned(16))) float sRaw[TR * K];
   __shared__ __attribute__((aligned(16))) float sScale[SCALED ? TR * K : 4];
   __shared__ int sId[kWideSegRows];
@@ -1130,7 +1174,8 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
   const int i1 = static_cast<int>(static_cast<int64_t>(ntiles) * (blockIdx.x + 1) / gridDim.x);
   int i = static_cast<int>(static_cast<int64_t>(ntiles) * blockIdx.x / gridDim.x);
   int g = 0, held_g = -1, held_l = -1;
-  bf16x8 w[CB][KS][3];  // weight pieces: column block, k step, piece
+  f16x8 w[CB][KS][2];  // weight pieces: column block, k step, piece
+  f4 column[CB];       // what takes the weight columns' scales back, of the four columns whose sums a lane gets
 
   while (i < i1) {
     while (sCum[g + 1] <= i) ++g;
@@ -1159,19 +1204,33 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
       const float *Wg = WT + ((static_cast<int64_t>(g) * (COMP == 1 ? 1 : 4) + l) * K + 16 * CB * wave + r16) * K + 8 * quarter;
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
+        f4 v[2 * KS];
+        float big = 0.f;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          bf16x4 h0, m0, l0, h1, m1, l1;
-          split3(ld4(Wg + 16 * cb * K + 32 * s), h0, m0, l0);
-          split3(ld4(Wg + 16 * cb * K + 32 * s + 4), h1, m1, l1);
+          v[2 * s] = ld4(Wg + 16 * cb * K + 32 * s), v[2 * s + 1] = ld4(Wg + 16 * cb * K + 32 * s + 4);
+          big = fmaxf(big, fmaxf(largest4(v[2 * s]), largest4(v[2 * s + 1])));
+        }
+        big = fmaxf(big, __shfl_xor(big, 16));
+        big = fmaxf(big, __shfl_xor(big, 32));  // the four lanes of a column
+        const PieceScale of = piece_scale(big, kLeastColumnExponent);
+        if (quarter == 0) sColumn[16 * CB * wave + 16 * cb + r16] = ldexpf(scale, of.exponent);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          f16x4 h0, l0, h1, l1;
+          split2(v[2 * s], of.s, h0, l0);
+          split2(v[2 * s + 1], of.s, h1, l1);
           w[cb][s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-          w[cb][s][1] = __builtin_shufflevector(m0, m1, 0, 1, 2, 3, 4, 5, 6, 7);
-          w[cb][s][2] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+          w[cb][s][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
       }
+      wave_lds_fence();  // a wave reads back its own columns
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) column[cb] = ld4(sColumn + 16 * CB * wave + 16 * cb + 4 * quarter);
       held_g = g;
       held_l = l;
     }
+    for (int r = tid; r < 4 * TR; r += WAVES * kWave) sRowMax[r / TR][r % TR] = 0;
     __syncthreads();
 
     const int n = seg_end - i;
@@ -1198,46 +1257,49 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
         }
       }
     };
-    auto split = [&](int k) {
-      __bf16 *plane = &sP[k & 1][0][0];
+    // This wave's pieces of tile k, once they are there, from LDS into registers, and their part in the rows' largest magnitudes.
+    f4 piece[PIECES];
+    auto take = [&](int k) {
 #pragma unroll
       for (int j = 0; j < PIECES; ++j) {
         const int p = (j * WAVES + wave) * kWave + lane;
-        f4 v = *reinterpret_cast<const f4 *>(sRaw + 4 * p);
-        if constexpr (SCALED) v *= *reinterpret_cast<const f4 *>(sScale + 4 * p);
-        bf16x4 h, md, lw;
-        split3(v, h, md, lw);
+        piece[j] = *reinterpret_cast<const f4 *>(sRaw + 4 * p);
+        if constexpr (SCALED) piece[j] *= *reinterpret_cast<const f4 *>(sScale + 4 * p);
+        const float big = max_over_8(largest4(piece[j]));  // eight neighbouring lanes hold pieces of one row
+        if (lane % 8 == 0) atomicMax(&sRowMax[k & 3][prow[j]], __float_as_uint(big));
+      }
+    };
+    auto split = [&](int k) {
+      _Float16 *plane = &sP[k & 1][0][0];
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j) {
+        f16x4 h, lw;
+        split2(piece[j], piece_scale(__uint_as_float(sRowMax[k & 3][prow[j]]), kLeastRowExponent).s, h, lw);
         const int at = prow[j] * LD + pcol[j];
-        *reinterpret_cast<bf16x4 *>(plane + at) = h;
-        *reinterpret_cast<bf16x4 *>(plane + TR * LD + at) = md;
-        *reinterpret_cast<bf16x4 *>(plane + 2 * TR * LD + at) = lw;
+        *reinterpret_cast<f16x4 *>(plane + at) = h;
+        *reinterpret_cast<f16x4 *>(plane + TR * LD + at) = lw;
       }
     };
     auto multiply = [&](int k) {
       int m, tb;
       where(k, m, tb);
-      const __bf16 *plane = &sP[k & 1][0][0] + r16 * LD + 8 * quarter;
-      v4f acc[RB][CB];
+      const _Float16 *plane = &sP[k & 1][0][0] + r16 * LD + 8 * quarter;
+      static_assert(RB == 1, "a lane's sums belong to one row");
+      const int exponent = piece_scale(__uint_as_float(sRowMax[k & 3][r16]), kLeastRowExponent).exponent;
+      v4f acc[CB], small[CB];  // products of high pieces, and those with a low one
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int cb = 0; cb < CB; ++cb) acc[cb] = small[cb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        bf16x8 x[RB][3];
+        f16x8 x[2];
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int q = 0; q < 2; ++q) x[q] = *reinterpret_cast<const f16x8 *>(plane + q * (TR * LD) + 32 * s);
 #pragma unroll
-          for (int q = 0; q < 3; ++q) x[rb][q] = *reinterpret_cast<const bf16x8 *>(plane + q * (TR * LD) + 16 * rb * LD + 32 * s);
-        // piece products from small to large; consecutive instructions go to different accumulators
-        constexpr int kW[6] = {0, 2, 1, 0, 1, 0}, kX[6] = {2, 0, 1, 1, 0, 0};
+        for (int cb = 0; cb < CB; ++cb) small[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][0], x[1], small[cb], 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
+        for (int cb = 0; cb < CB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][0], x[0], acc[cb], 0, 0, 0);
 #pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-              acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cb][s][kW[q]], x[rb][kX[q]], acc[rb][cb], 0, 0, 0);
+        for (int cb = 0; cb < CB; ++cb) small[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][1], x[0], small[cb], 0, 0, 0);
       }
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
@@ -1257,7 +1319,9 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
           v4f v;
           {
 #pragma clang fp contract(off)  // the product is rounded before the residual is added, as everywhere
-            v = acc[rb][cb] * scale;
+            v = (acc[cb] + small[cb]) * column[cb];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = __builtin_ldexpf(v[i], exponent);
             if (COMP == 1 && residual) v = v + res[cb];
           }
           // (the two idle issue slots: see the stores of the kernel above)
@@ -1268,17 +1332,26 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
 
     issue(0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    split(0);
+    take(0);
     if (n > 1) issue(1);
-    // before the first split of the loop only loads are out; the wait below is exact from the second tile on
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // largest magnitudes of tile 0 complete
+    split(0);
+    if (n > 1) take(1);
+    if (n > 2) issue(2);
+    // before the first wait of the loop only loads are out; it is exact from the second tile on
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     for (int k = 0; k < n; ++k) {
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // planes of tile k complete, those of tile k - 1 free
+      // planes of tile k and largest magnitudes of tile k + 1 complete, the planes of tile k - 1 free
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       if (late) multiply(k);
       if (k + 1 < n) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");  // the loads of tile k + 1; the stores after them may stay out
         split(k + 1);
-        if (k + 2 < n) issue(k + 2);
+        if (tid < TR) sRowMax[(k + 3) & 3][tid] = 0;  // last read when tile k - 1 was multiplied
+        if (k + 2 < n) {
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");  // the loads of tile k + 2; the stores after them may stay out
+          take(k + 2);
+          if (k + 3 < n) issue(k + 3);
+        }
       }
       if (!late) multiply(k);
     }

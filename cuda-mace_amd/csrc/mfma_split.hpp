@@ -1,5 +1,5 @@
-// Operand types of v_mfma_f32_32x32x16_bf16 and the split of an fp32 value into three bf16 pieces, shared by the kernels
-// that run fp32 products on the bf16 matrix instruction (linear.hip, node_glue.hip).
+// Operand types of the 16-bit matrix instructions and the splits of an fp32 value into three bf16 or two fp16 pieces, shared by
+// the kernels that run fp32 products on them (linear.hip, node_glue.hip).
 #pragma once
 
 #include "common.hpp"
@@ -32,5 +32,37 @@ __device__ __forceinline__ void split3(f4 v, bf16x4 &hi, bf16x4 &mid, bf16x4 &lo
   mid = __builtin_bit_cast(bf16x4, u2{m0, m1});
   lo = __builtin_bit_cast(bf16x4, u2{l0, l1});
 }
+
+// The split into two fp16 pieces, for v_mfma_f32_32x32x16_f16 and its like: s v = hi + lo with s a power of two that brings
+// the largest value of the row (of X) or column (of W) that v belongs to to [2^14, 2^15).  Both pieces are rounded to nearest, so hi
+// + lo is within 2^-24 of s v wherever |s v| >= 2^-1, i.e. down to 2^-15 of the row's largest value, and below that within 2^-25, 2^-39
+// of the row's largest value.  Three piece products (hi hi, hi lo, lo hi) make the product; the dropped one, lo lo, is below 2^-24 of it.
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split2_pair(float v0, float v1, float s, f16x2 &hi, f16x2 &lo) {
+  const float a = v0 * s, b = v1 * s;
+  hi = __builtin_convertvector(f2{a, b}, f16x2);
+  lo = __builtin_convertvector(f2{a - static_cast<float>(hi.x), b - static_cast<float>(hi.y)}, f16x2);
+}
+__device__ __forceinline__ void split2(f4 v, float s, f16x4 &hi, f16x4 &lo) {
+  f16x2 h0, l0, h1, l1;
+  split2_pair(v.x, v.y, s, h0, l0);
+  split2_pair(v.z, v.w, s, h1, l1);
+  hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3);
+  lo = __builtin_shufflevector(l0, l1, 0, 1, 2, 3);
+}
+// Scale of a row or column from its largest magnitude, and what takes it back: s = 2^-exponent.  `least`: the smallest biased
+// exponent told apart (a smaller largest value, zero among them, is scaled as that one); infinities and NaN take the largest scale down.
+struct PieceScale {
+  float s;
+  int exponent;
+};
+__device__ __forceinline__ PieceScale piece_scale(float largest, int least) {
+  const int e = min(max(static_cast<int>(__float_as_uint(largest) >> 23), least), 254);
+  return {__uint_as_float(static_cast<unsigned>(268 - e) << 23), e - 141};
+}
+constexpr int kLeastRowExponent = 14;     // s up to 2^127
+constexpr int kLeastColumnExponent = 24;  // s up to 2^117: its inverse times the call's scale stays a normal number
 
 }  // namespace cm

@@ -535,6 +535,39 @@ def test_linear_many_rows_wide(cabi, N, C, ne, seed):
     test_linear_many_rows(cabi, N, C, ne, seed)
 
 
+@pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256)])
+def test_linear_scales_of_rows_and_columns(cabi, N, C):
+    """The kernels with resident weights scale rows of X and columns of W by powers of two: rows and columns multiplied by powers of
+    two give the same bits, multiplied alike (as long as nothing leaves the normal range), also next to rows of zeros, in one tile
+    with huge ones.  Errors stay within the bound of the split, element by element: |x w| times 3 * 2^-24 for the two roundings and
+    the dropped product, 2^-39 of the row's and the column's largest values for what falls below the pieces' range, and K fp32 sums
+    (at most K 2^-24 of the sum of magnitudes), on rows whose values spread over 30 powers of two."""
+    _say("linear_scales", N, C)
+    g = torch.Generator().manual_seed(C)
+    X, W = torch.randn(N, 16, C, generator=g), torch.randn(4, C, C, generator=g)
+    S = torch.randn(N, C, generator=g)
+    rows = torch.randint(-50, 51, (N, 16, 1), generator=g)
+    columns = torch.randint(-30, 31, (4, C, 1), generator=g)
+    d = lambda t: t.float().contiguous().to(DEV)  # noqa: E731
+    lm = torch.tensor([0] + [1] * 3 + [2] * 5 + [3] * 7)
+    grown = torch.ldexp(X, rows)
+    grown[5], grown[7] = 0.0, torch.ldexp(X[7], torch.tensor(60))
+    factor = torch.ldexp(torch.ones(N, 16, C), rows + columns[lm, :, 0])
+    factor[5], factor[7] = 0.0, torch.ldexp(torch.ones(16, C), 60 + columns[lm, :, 0])
+    for scale in (None, S):
+        more = {} if scale is None else {"row_scale": d(scale)}
+        base = cabi.linear(d(X), d(W), scale=0.7, **more)
+        out = cabi.linear(d(grown), d(torch.ldexp(W, columns)), scale=0.7, **more)
+        assert torch.equal(out, base * d(factor))
+    spread = torch.ldexp(X, torch.randint(-30, 1, X.shape, generator=g))
+    out = cabi.linear(d(spread), d(W), scale=1.0).double().cpu()
+    xd, wd = spread.double(), W.double()[lm]                      # [16, C, C], W^T rows are output columns
+    ref = torch.einsum("nmk,mjk->nmj", xd, wd)
+    size = torch.einsum("nmk,mjk->nmj", xd.abs(), wd.abs())
+    floor = 2.0 ** -39 * (xd.abs().amax(-1, keepdim=True) * wd.abs().sum(-1) + xd.abs().sum(-1, keepdim=True) * wd.abs().amax(-1))
+    assert bool(((out - ref).abs() <= (3.0 + C) * 2.0 ** -24 * size + floor).all())
+
+
 @pytest.mark.parametrize("N,C", [(8192, 160), (8193, 192), (9007, 224), (12345, 256)])
 def test_scalar_linear_many_rows_wide(cabi, N, C):
     """One component per node at 160 to 256 columns and 8 192 nodes and more: plain, with row_scale, with a residual that is a
