@@ -698,32 +698,37 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 }
 
 // -----------------------------------------------------------------------------------------------
-// Variant with the weights resident in LDS (16 components per node, K = Nout up to 128).
+// Variant with the weights resident in LDS (16 components per node, K = Nout = 64, 96 or 128).
 //
 // The kernels above stage the K x Nout weight block again for every tile of 128 rows (as many bytes from L2 as the tile
 // has from HBM) and walk K in barrier-separated phases.  Here a launch has one workgroup per compute unit, and a
-// workgroup takes a contiguous piece of the list of all 32-row tiles, ordered by (weight group, l, node tile, m within
+// workgroup takes a contiguous piece of the list of all 16-row tiles, ordered by (weight group, l, node tile, m within
 // l), so that it needs one or two weight blocks in its whole life: it splits a block once into two fp16 planes that
-// cover all of K (70 KB at 128 x 128) and then its four waves run independently of each other, one 32-row tile at a
+// cover all of K (70 KB at 128 x 128) and then its eight waves run independently of each other, one 16-row tile at a
 // time, with no barrier until the weight block changes.
 //
-// Two fp16 pieces per operand and three piece products on v_mfma_f32_32x32x16_f16 (mfma_split.hpp), rows of X and columns of W
+// Two fp16 pieces per operand and three piece products on v_mfma_f32_16x16x32_f16 (mfma_split.hpp), rows of X and columns of W
 // scaled by powers of two that the output takes back: half the matrix instructions of three bf16 pieces and six products,
 // four vector instructions per value instead of five and a half, two thirds of the fragment reads.  The products with a low piece
-// have an accumulator of their own, so a sum of K terms is rounded K / 16 times.  us and rms error against fp64 (normal
+// have an accumulator of their own, so a sum of K terms is rounded K / 32 times.  us and rms error against fp64 (normal
 // values), bf16 -> fp16: 25 000 x 128 90.4 -> 80.3, 1.65e-7 -> 1.13e-7, with a weight block per element 93.4 -> 85.0, with row_scale 97.9 ->
 // 90.9, 1.68e-7 -> 1.15e-7; 96 columns 1.41e-7 -> 1.07e-7, 64 1.12e-7 -> 1.02e-7, equal times at 5 000 and 10 752 nodes (one
 // accumulator: 1.45e-7 at 128, 1.32e-7 at 96, 1.16e-7 at 64).
 //
-// What a wave has in flight lives in registers, not in LDS: the loads of tile i + 1 (16 x 16 bytes per lane at 128
+// Two waves per SIMD on 16-row tiles: four waves on 32-row tiles (32x32x16 instructions, half the weight fragments per row, what the
+// figures above were taken with) spent 6 500 cycles on a tile of 96 columns whose matrix instructions take 1 700, because a
+// wave alone on its SIMD issues an instruction every six cycles.  Now 25 000 x 128 80 -> 72, with a weight block per element 82 -> 78, with
+// row_scale 96 (the row_scale rows come again for each l); 10 752 x 64 24.9 -> 21.3, 5 000 x 96 x 10 elements 24.9 -> 20.8, 2 500 x 128 x
+// 10 with row_scale 27.3 -> 21.3, 50 000 x 64 74 -> 70.  Twelve waves are equal at 64 and 96 columns and spill at 128.
+//
+// What a wave has in flight lives in registers, not in LDS: the loads of tile i + 1 (8 x 16 bytes per lane at 128
 // columns, whole 128-byte lines of 8 rows per instruction) are issued before tile i is multiplied and land in
 // accumulator-file registers; 64 KB per compute unit are on their way at any time.  When its turn comes a tile changes
 // from that row-major layout to the operand layout of the matrix instruction (a lane holds 8 values of one row per
-// 16-wide k step) through the wave's own corner of LDS, 64 columns at a time.  The order of k inside a step is free as
-// long as both operands agree; it is chosen such that a lane reads two aligned 16-byte pieces.  The operands are swapped
-// with respect to the kernels above (weights as the row operand, X rows as the column operand): a lane's accumulators
-// are then 4 consecutive output columns of one row; a block of 32 columns goes back through the same corner of LDS and
-// leaves as whole lines.
+// 32-wide k step) through the wave's own corner of LDS, up to 96 columns at a time; the rows' largest values are found on the way.
+// The operands are swapped with respect to the kernels above (weights as the row operand, X rows as the column operand): a lane's
+// accumulators are then 4 consecutive output columns of one row; a block of 32 columns goes back through the same corner of LDS
+// and leaves as whole lines.
 //
 // Contract of the hand-issued memory operations of the tile loop (the loads and the stores): a load names its landing
 // registers at issue time although the data arrives by the explicit wait that precedes their first use, which is
@@ -733,21 +738,17 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 // stored registers may be overwritten (the compiler inserts them for the stores it knows; without them the last lanes of
 // the following block were stored instead).
 //
-// What was measured on the way (25 000 x 128, one box each): loads of 32 bytes per lane and row, which is what a lane
-// feeds per k step, request every line four times, and the kernel then ran at the rate of the compute unit's queue of
-// outstanding misses (118 us; whole lines: 99 us); stores under a branch make the compiler wait for everything in
-// flight at the top of the loop (hence no conditional rows, see the row numbers below); weaving the operand split of
-// the next k step between the matrix instructions took it to 87 us.  Without its matrix instructions the kernel takes
-// 62 us and without its loads and stores 72 us: what remains is that one wave per SIMD does its memory waits, its LDS
-// round trips and its matrix instructions one after the other.  Two waves per SIMD (eight waves, a tile landing in
-// chunks of 32 columns, no weaving) came out equal at this size and 7 % slower at 100 000 nodes; two tiles ahead
-// instead of one changes nothing (and 64 outstanding instructions per wave is where the counter ends).
+// Loads of 32 bytes per lane and row, which is what a lane feeds per k step, request every line four times, and the kernel then
+// ran at the rate of the compute unit's queue of outstanding misses (25 000 x 128 118 us; whole lines: 99 us); stores under a
+// branch make the compiler wait for everything in flight at the top of the loop (hence no conditional rows, see the row numbers below).
 // -----------------------------------------------------------------------------------------------
-constexpr int kResWaves = 4;
+constexpr int kResWaves = 8;
+constexpr int kResRows = 16;   // rows of a tile
+constexpr int kResSegRows = 2048;  // rows whose numbers a segment keeps in LDS
+typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kResMaxGroups = 128;
 constexpr int kResMinNodes = 2048;
 constexpr int kOutLd = 36;            // floats per row of a wave's output staging block (32 columns + 16 bytes)
-constexpr int kResSegNodeTiles = 64;  // node tiles whose row numbers a segment keeps in LDS
 
 __device__ __forceinline__ float largest4(f4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
 // largest value over eight neighbouring lanes, in all of them
@@ -762,20 +763,21 @@ __device__ __forceinline__ float max_over_8(float v) {
 }
 
 template <int K, int NT, bool SCALED>
-__global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
+__global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_resident_kernel(
     const float *__restrict__ X, const float *__restrict__ WT, const int32_t *__restrict__ node_perm,
-    const int32_t *__restrict__ group_offsets, int nnodes, int ngroups, int zero_last_group, int ldo, float scale,
+    const int32_t *__restrict__ group_offsets, int nnodes, int ngroups, int zero_last_group, float scale,
     const float *__restrict__ row_scale, float *__restrict__ OUT) {
-  constexpr int NOUT = 32 * NT;  // columns of this workgroup: blockIdx.y * NOUT onwards of the ldo columns of OUT
+  constexpr int NOUT = 32 * NT;
+  static_assert(K == NOUT, "square weights");
   constexpr int LD = K + 8;      // row stride of a plane in elements: an odd number of 16-byte units
-  constexpr int KS = K / 16;
+  constexpr int KS = K / 32;
   __shared__ __attribute__((aligned(16))) _Float16 sW[2 * NOUT * LD];
   __shared__ __attribute__((aligned(16))) float sColumn[NOUT];  // largest magnitude of a weight column, then what takes its scale back
-  __shared__ float sRowMax[kResWaves * 32];
-  __shared__ int sId[kResSegNodeTiles * 32];
+  __shared__ float sRowMax[kResWaves * kResRows];
+  __shared__ int sId[kResSegRows];
   constexpr int kChunk = K <= 96 ? K : 64;  // columns of X per trip through LDS
   constexpr int kTLd = kChunk + 4;          // floats per row of the transposition block: an odd number of 16-byte units
-  constexpr int kStageFloats = 32 * (kTLd > kOutLd ? kTLd : kOutLd);  // a wave's own corner of LDS
+  constexpr int kStageFloats = kResRows * (kTLd > kOutLd ? kTLd : kOutLd);  // a wave's own corner of LDS
   __shared__ __attribute__((aligned(16))) float sStage[kResWaves * kStageFloats];
   __shared__ int sOff[kResMaxGroups + 1];
   __shared__ int sCum[kResMaxGroups + 1];
@@ -783,9 +785,7 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int mrow = lane % 32;
-  const int half = lane / 32;
-  const int c0 = blockIdx.y * NOUT;
+  const int r16 = lane % 16, quarter = lane / 16;
 
   // groups that have weights, their row ranges in the grouped node order and their first tile in the tile list
   const int ngw = zero_last_group ? ngroups - 1 : ngroups;
@@ -795,19 +795,19 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       const int lo = group_offsets ? group_offsets[g] : 0, hi = group_offsets ? group_offsets[g + 1] : nnodes;
       sOff[g] = lo;
       sCum[g] = cum;
-      cum += 16 * ((max(hi - lo, 0) + 31) / 32);
+      cum += 16 * ((max(hi - lo, 0) + kResRows - 1) / kResRows);
     }
     sOff[ngw] = group_offsets ? group_offsets[ngw] : nnodes;
     sCum[ngw] = cum;
   }
-  if (zero_last_group && blockIdx.y == 0) {
+  if (zero_last_group) {
     // rows that belong to no weight group: the product is defined as zero (a residual still passes through)
     const int z0 = group_offsets[ngroups - 1], nz = group_offsets[ngroups] - z0;
-    const int rowq = 16 * ldo / 4;
+    constexpr int rowq = 16 * NOUT / 4;
     const int64_t total = static_cast<int64_t>(nz) * rowq;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + tid; i < total; i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
       const int node = node_perm[z0 + static_cast<int>(i / rowq)];
-      if (static_cast<unsigned>(node) < static_cast<unsigned>(nnodes)) st4(OUT + static_cast<int64_t>(node) * 16 * ldo + 4 * (i % rowq), zero4());
+      if (static_cast<unsigned>(node) < static_cast<unsigned>(nnodes)) st4(OUT + static_cast<int64_t>(node) * 16 * NOUT + 4 * (i % rowq), zero4());
     }
   }
   __syncthreads();
@@ -824,54 +824,53 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
     const int nm = 2 * l + 1;
     const int blk0 = sCum[g] + tg * l * l;        // first tile of (g, l): tile blk0 + t * nm + (m - l * l)
     const int t_first = (i - blk0) / nm;
-    const int seg_end = min(min(i1, blk0 + tg * nm), blk0 + (t_first + kResSegNodeTiles) * nm);
+    const int seg_end = min(min(i1, blk0 + tg * nm), blk0 + (t_first + kResSegRows / kResRows) * nm);
     const int t_count = (seg_end - 1 - blk0) / nm - t_first + 1;
     const int off0 = sOff[g], off1 = sOff[g + 1];
+    const bool new_weights = g != staged_g || l != staged_l;
 
+    // W^T[j, :] of block (g, l) -> two planes.  All loads of a thread first, ahead of the row numbers: one trip through L2.
+    const float *Wg = WT + (static_cast<int64_t>(g) * 4 + l) * NOUT * K;
+    constexpr int kPieces = (NOUT * (K / 4) + kResWaves * kWave - 1) / (kResWaves * kWave);
+    const auto piece_of = [&](int it) { return min(it * (kResWaves * kWave) + tid, NOUT * (K / 4) - 1); };  // beyond the block: its last piece once more
+    f4 wv[kPieces];
+    if (new_weights) {
+#pragma unroll
+      for (int it = 0; it < kPieces; ++it) {
+        const int q = piece_of(it);
+        wv[it] = ld4(Wg + static_cast<int64_t>(q / (K / 4)) * K + 4 * (q % (K / 4)));
+      }
+    }
     __syncthreads();  // every wave is done with the previous segment
     // Row numbers of the segment's node tiles.  A row beyond the end of the group (or an index outside the node range)
     // stands in for the first row of its tile: it then computes that row's values once more and stores the same bits
     // to the same place, so that no load or store of the tile loop is conditional.
-    for (int r = tid; r < 32 * t_count; r += kResWaves * kWave) {
-      const int p0 = off0 + 32 * (t_first + r / 32);
-      const int p = p0 + r % 32;
+    for (int r = tid; r < kResRows * t_count; r += kResWaves * kWave) {
+      const int p0 = off0 + kResRows * (t_first + r / kResRows);
+      const int p = p0 + r % kResRows;
       int node = node_perm ? node_perm[p < off1 ? p : p0] : (p < off1 ? p : p0);
       if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) node = node_perm ? node_perm[p0] : p0;
       if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) node = 0;
       sId[r] = node;
     }
-    if (g != staged_g || l != staged_l) {
-      // W^T[c0 + j, :] of block (g, l) -> two planes; inside every 16 k the two middle groups of four trade places, so
-      // that the 8 values a lane reads at 16 s + 8 half are k = 16 s + 4 half + {0..3, 8..11}
-      const float *Wg = WT + ((static_cast<int64_t>(g) * 4 + l) * ldo + c0) * K;
-      // all loads of a thread first (16 at 128 x 128), then the splits: one trip through L2 instead of one per piece
-      constexpr int kPieces = NOUT * (K / 4) / (kResWaves * kWave);
-      static_assert(NOUT * (K / 4) % (kResWaves * kWave) == 0, "weight staging map");
-      f4 wv[kPieces];
-#pragma unroll
-      for (int it = 0; it < kPieces; ++it) {
-        const int q = it * (kResWaves * kWave) + tid;
-        wv[it] = ld4(Wg + static_cast<int64_t>(q / (K / 4)) * K + 4 * (q % (K / 4)));
-      }
+    if (new_weights) {
       if (tid < NOUT) sColumn[tid] = 0.f;
       __syncthreads();
       // eight neighbouring threads hold pieces of one column (K / 4 is a multiple of eight)
 #pragma unroll
       for (int it = 0; it < kPieces; ++it) {
         const float big = max_over_8(largest4(wv[it]));
-        if (tid % 8 == 0) atomicMax(reinterpret_cast<unsigned *>(sColumn) + (it * (kResWaves * kWave) + tid) / (K / 4), __float_as_uint(big));
+        if (tid % 8 == 0) atomicMax(reinterpret_cast<unsigned *>(sColumn) + piece_of(it) / (K / 4), __float_as_uint(big));
       }
       __syncthreads();
 #pragma unroll
       for (int it = 0; it < kPieces; ++it) {
-        const int q = it * (kResWaves * kWave) + tid;
+        const int q = piece_of(it);
         const int j = q / (K / 4), kq = q % (K / 4);
         f16x4 h, lw;
         split2(wv[it], piece_scale(sColumn[j], kLeastColumnExponent).s, h, lw);
-        const int sub = kq & 3;
-        const int at = j * LD + 16 * (kq >> 2) + 4 * (sub == 1 ? 2 : (sub == 2 ? 1 : sub));
-        *reinterpret_cast<f16x4 *>(sW + at) = h;
-        *reinterpret_cast<f16x4 *>(sW + NOUT * LD + at) = lw;
+        *reinterpret_cast<f16x4 *>(sW + j * LD + 4 * kq) = h;
+        *reinterpret_cast<f16x4 *>(sW + NOUT * LD + j * LD + 4 * kq) = lw;
       }
       __syncthreads();
       if (tid < NOUT) sColumn[tid] = ldexpf(scale, piece_scale(sColumn[tid], kLeastColumnExponent).exponent);
@@ -889,20 +888,18 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
     // Tile loop.  Every global access in it is issued from assembly in a fixed order and waited for by an explicit count
     // (the compiler would sink part of a prefetch down to its use and then wait for everything that is in flight, the
     // stores of the previous tile included):
-    //     tile i:  wait: all but the stores of tile i - 1 | landing registers -> working registers (times row_scale)
+    //     tile i:  wait: all but the stores of tile i - 1 | landing registers (times row_scale) -> LDS -> pieces
     //              | issue the loads of tile i + 1 | multiply | output block by block through LDS, issue the stores
-    // The landing registers are accumulator-file registers (a load may write them directly; nothing else competes for
-    // them, so the compiler has no reason to move them while a load is in flight), the working set lives in ordinary
-    // registers.
     // Loads are whole lines: one instruction fetches 128 bytes of each of 8 rows (lane = 16-byte piece opiece of row
     // 8 rg + orow; in 32-byte pieces, which is what a lane feeds per k step, every line would be requested four times and
     // the compute unit's queue of outstanding misses would hold a quarter of the bytes).  The landed values change to the
     // operand layout through the wave's own corner of LDS, kChunk columns at a time.
+    constexpr int kRg = kResRows / 8;
     constexpr int kLines = kChunk / 32;  // 128-byte lines of a row per chunk
     constexpr int kChunks = K / kChunk;
     static_assert(K % kChunk == 0 && kChunk % 32 == 0, "chunks of whole lines");
-    f4 land[2 * KS];                           // index (chunk * 4 + rg) * kLines + line
-    f4 sland[SCALED ? 2 * KS : 1];
+    f4 land[kRg * K / 32];                     // index (chunk * kRg + rg) * kLines + line
+    f4 sland[SCALED ? kRg * K / 32 : 1];
     float *stg = sStage + wave * kStageFloats;
     const int orow = lane / 8, opiece = lane % 8;
     int t_scales = -1;  // node tile whose row_scale rows are in (or on their way into) sland
@@ -910,16 +907,16 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
       const int j = idx - blk0;
       const int t = j / nm;
       m_of = l * l + (j - t * nm);
-      tb_of = 32 * (t - t_first);
+      tb_of = kResRows * (t - t_first);
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
+      for (int rg = 0; rg < kRg; ++rg) {
         const int nd = sId[tb_of + 8 * rg + orow];
         const float *xp = X + (static_cast<int64_t>(nd) * 16 + m_of) * K + 4 * opiece;
 #pragma unroll
         for (int c = 0; c < kChunks; ++c)
 #pragma unroll
           for (int ln = 0; ln < kLines; ++ln)
-            asm volatile("global_load_dwordx4 %0, %1, off offset:%2 nt" : "=a"(land[(c * 4 + rg) * kLines + ln]) : "v"(xp), "n"(4 * (c * kChunk + 32 * ln)) : "memory");
+            asm volatile("global_load_dwordx4 %0, %1, off offset:%2 nt" : "=a"(land[(c * kRg + rg) * kLines + ln]) : "v"(xp), "n"(4 * (c * kChunk + 32 * ln)) : "memory");
       }
       if constexpr (SCALED) {
         // the 2 l + 1 tiles of a node tile follow each other and share their row_scale rows: fetched once (these loads
@@ -927,34 +924,36 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
         if (t != t_scales) {
           t_scales = t;
 #pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
+          for (int rg = 0; rg < kRg; ++rg) {
             const float *sp = row_scale + static_cast<int64_t>(sId[tb_of + 8 * rg + orow]) * K + 4 * opiece;
 #pragma unroll
             for (int c = 0; c < kChunks; ++c)
 #pragma unroll
               for (int ln = 0; ln < kLines; ++ln)
-                asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=a"(sland[(c * 4 + rg) * kLines + ln]) : "v"(sp), "n"(4 * (c * kChunk + 32 * ln)) : "memory");
+                asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=a"(sland[(c * kRg + rg) * kLines + ln]) : "v"(sp), "n"(4 * (c * kChunk + 32 * ln)) : "memory");
           }
         }
       }
     };
-    const _Float16 *wl = sW + mrow * LD + 8 * half;
+    const _Float16 *wl = sW + r16 * LD + 8 * quarter;
     int m_next, tb_next;
     issue(wb, m_next, tb_next);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     for (int idx = wb; idx < we; ++idx) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NT) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRg * NT) : "memory");
       const int m_cur = m_next, tb_cur = tb_next;
+      float big[kRg];
+#pragma unroll
+      for (int rg = 0; rg < kRg; ++rg) big[rg] = 0.f;
       f4 cur[2 * KS];
-      float big[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < kChunks; ++c) {
         wave_lds_fence();
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
+        for (int rg = 0; rg < kRg; ++rg) {
 #pragma unroll
           for (int ln = 0; ln < kLines; ++ln) {
-            const int j = (c * 4 + rg) * kLines + ln;
+            const int j = (c * kRg + rg) * kLines + ln;
             asm volatile("; landed %0" : "+a"(land[j]));
             f4 v = land[j];
             if constexpr (SCALED) {
@@ -966,100 +965,80 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
           }
           if (c == kChunks - 1) {  // the eight lanes of a row have all of it
             const float row = max_over_8(big[rg]);
-            if (opiece == 0) sRowMax[32 * wave + 8 * rg + orow] = row;
+            if (opiece == 0) sRowMax[kResRows * wave + 8 * rg + orow] = row;
           }
         }
         wave_lds_fence();
-        // k step s of the chunk: the lane's values are columns 16 s + 4 half + {0..3} and 16 s + 8 + 4 half + {0..3}
+        // k step s of the chunk: the lane's values are columns 32 s + 8 quarter + {0..7}
 #pragma unroll
-        for (int sc = 0; sc < kChunk / 16; ++sc) {
-          const int s = c * (kChunk / 16) + sc;
-          cur[2 * s] = *reinterpret_cast<const f4 *>(stg + mrow * kTLd + 16 * sc + 4 * half);
-          cur[2 * s + 1] = *reinterpret_cast<const f4 *>(stg + mrow * kTLd + 16 * sc + 8 + 4 * half);
+        for (int sc = 0; sc < kChunk / 32; ++sc) {
+          const int s = c * (kChunk / 32) + sc;
+          cur[2 * s] = *reinterpret_cast<const f4 *>(stg + r16 * kTLd + 32 * sc + 8 * quarter);
+          cur[2 * s + 1] = *reinterpret_cast<const f4 *>(stg + r16 * kTLd + 32 * sc + 8 * quarter + 4);
         }
       }
-#pragma unroll
-      for (int j = 0; j < 2 * KS; ++j) asm volatile("" : "+v"(cur[j]));
-      const PieceScale row = piece_scale(sRowMax[32 * wave + mrow], kLeastRowExponent);
+      const PieceScale row = piece_scale(sRowMax[kResRows * wave + r16], kLeastRowExponent);
       if (idx + 1 < we) issue(idx + 1, m_next, tb_next);
-
-      v16f acc[NT], acs[NT];
+      f16x8 x[KS][2];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][r] = acs[t][r] = 0.f;
-      // One wave per SIMD: nothing but this wave's own instruction stream can fill the issue slots between two matrix
-      // instructions (32 cycles apart), so the k loop is pipelined in the source: the pieces of X and the weight fragments of
-      // step s + 1 are prepared while the 6 NT matrix instructions of step s run, and the scheduler is told to weave them
-      // (per matrix instruction: three vector instructions, and an LDS read for the first 3 NT of them).
-      constexpr int kSplitOps = (32 + 3 * NT - 1) / (3 * NT);  // the split of a step is about 24 vector instructions
-      f16x8 xq[2][2], wq[2][NT][2];
-      auto prepare = [&](int s, auto par) {
-        constexpr int P = decltype(par)::value;
+      for (int s = 0; s < KS; ++s) {
         f16x4 h0, l0, h1, l1;
         split2(cur[2 * s], row.s, h0, l0);
         split2(cur[2 * s + 1], row.s, h1, l1);
-        xq[P][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-        xq[P][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        x[s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+        x[s][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float *orows[kRg];
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+      for (int r = 0; r < kRg; ++r)
+        orows[r] = OUT + (static_cast<int64_t>(sId[tb_cur + 8 * r + orow]) * 16 + m_cur) * NOUT + 4 * opiece;
+
+      constexpr int GB = NT % 2 == 0 ? 4 : 2;  // column blocks of 16 at a time
 #pragma unroll
-          for (int p = 0; p < 2; ++p) wq[P][t][p] = *reinterpret_cast<const f16x8 *>(wl + p * NOUT * LD + 32 * t * LD + 16 * s);
-      };
-      auto step = [&](int s, auto par) {
-        constexpr int P = decltype(par)::value;
-        if (s + 1 < KS) prepare(s + 1, std::integral_constant<int, 1 - P>{});
+      for (int t0 = 0; t0 < 2 * NT; t0 += GB) {
+        v4f acc[GB], small[GB];  // products of high pieces, and those with a low one
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acs[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][0], xq[P][1], acs[t], 0, 0, 0);
+        for (int t = 0; t < GB; ++t) acc[t] = small[t] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acs[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][1], xq[P][0], acs[t], 0, 0, 0);
+        for (int s = 0; s < KS; ++s) {
+          f16x8 wh[GB], wo[GB];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[P][t][0], xq[P][0], acc[t], 0, 0, 0);
-        if (s + 1 < KS) {
+          for (int t = 0; t < GB; ++t) {
+            wh[t] = *reinterpret_cast<const f16x8 *>(wl + 16 * (t0 + t) * LD + 32 * s);
+            wo[t] = *reinterpret_cast<const f16x8 *>(wl + NOUT * LD + 16 * (t0 + t) * LD + 32 * s);
+          }
 #pragma unroll
-          for (int i = 0; i < 3 * NT; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // one matrix instruction
-            if (i < 2 * NT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-            __builtin_amdgcn_sched_group_barrier(0x002, kSplitOps, 0);          // a share of the split arithmetic
+          for (int t = 0; t < GB; ++t) small[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[t], x[s][1], small[t], 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < GB; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[t], x[s][0], acc[t], 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < GB; ++t) small[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wo[t], x[s][0], small[t], 0, 0, 0);
+          if (K == 128) __builtin_amdgcn_sched_barrier(0);  // fragment reads of later steps hoisted further would not fit the register file
+        }
+        // accumulator r of a lane: output column 16 t + 4 quarter + r of row r16 of the tile.  A block of 32 columns goes
+        // through the wave's own corner of LDS (rows padded to 9 x 16 bytes: conflict-free both ways) and leaves as whole
+        // 128-byte lines, 8 rows per store.
+#pragma unroll
+        for (int t = 0; t < GB; t += 2) {
+          wave_lds_fence();
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            f4 v = (acc[t + q] + small[t + q]) * ld4(sColumn + 16 * (t0 + t + q) + 4 * quarter);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = __builtin_ldexpf(v[k], row.exponent);
+            st4(stg + r16 * kOutLd + 16 * q + 4 * quarter, v);
+          }
+          wave_lds_fence();
+#pragma unroll
+          for (int r = 0; r < kRg; ++r) {
+            const f4 v = *reinterpret_cast<const f4 *>(stg + (8 * r + orow) * kOutLd + 4 * opiece);
+            // the two idle issue slots are what the compiler puts between a 16-byte store and an instruction that
+            // overwrites the registers it stores from; it does not see this store
+            asm volatile("global_store_dwordx4 %0, %1, off offset:%2\n\ts_nop 1" : : "v"(orows[r]), "v"(v), "n"(64 * (t0 + t)) : "memory");
           }
         }
-        // nothing else moves across k steps: fragment reads of later steps hoisted further would not fit the register file
         __builtin_amdgcn_sched_barrier(0);
-      };
-      prepare(0, std::integral_constant<int, 0>{});
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < KS; s += 2) {
-        step(s, std::integral_constant<int, 0>{});
-        if (s + 1 < KS) step(s + 1, std::integral_constant<int, 1>{});
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] += acs[t];
-      // accumulator r of a lane: output column 32 t + 8 (r / 4) + 4 half + r % 4 of row mrow of the tile.  Stored from
-      // here a row would leave in 32-byte pieces; a block of 32 columns goes through the wave's own corner of LDS instead
-      // (rows padded to 9 x 16 bytes: conflict-free both ways) and leaves as whole 128-byte lines, 8 rows per store.
-      float *orows[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        orows[r] = OUT + (static_cast<int64_t>(sId[tb_cur + 8 * r + orow]) * 16 + m_cur) * ldo + c0 + 4 * opiece;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        wave_lds_fence();
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          f4 v = f4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]} * ld4(sColumn + 32 * t + 8 * q + 4 * half);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) v[k] = __builtin_ldexpf(v[k], row.exponent);
-          st4(stg + mrow * kOutLd + 8 * q + 4 * half, v);
-        }
-        wave_lds_fence();
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const f4 v = *reinterpret_cast<const f4 *>(stg + (8 * r + orow) * kOutLd + 4 * opiece);
-          // the two idle issue slots are what the compiler puts between a 16-byte store and an instruction that
-          // overwrites the registers it stores from; it does not see this store
-          asm volatile("global_store_dwordx4 %0, %1, off offset:%2\n\ts_nop 1" : : "v"(orows[r]), "v"(v), "n"(128 * t) : "memory");
-        }
       }
     }
     // every landing register has been consumed: nothing this wave issued can still write a register
@@ -1098,7 +1077,6 @@ __global__ __launch_bounds__(kResWaves *kWave, 1) void linear_resident_kernel(
 // us at 192 columns; with two fp16 pieces, us and rms error against fp64: 100 000 x 192 647 -> 557, 1.96e-7 -> 1.24e-7, 20 000 x 224
 // 184 -> 134, 2.14e-7 -> 1.29e-7, 12 000 x 256 137 -> 110, 2.31e-7 -> 1.34e-7, 10 007 x 160 64.8 -> 61.1, 1.77e-7 -> 1.18e-7.
 // -----------------------------------------------------------------------------------------------
-typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kWideMinScalarNodes = 8192;
 constexpr int kWideSegRows = 2048;  // rows whose node numbers a segment keeps in LDS
 
@@ -1376,19 +1354,14 @@ int launch_wide(const float *X, const float *WT, const int32_t *perm, const int3
 
 template <int K, int NT>
 int launch_resident(const float *X, const float *WT, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
-                    int zero_last_group, int Nout, float scale, const float *row_scale, float *OUT, hipStream_t st) {
-  // one workgroup per compute unit.  (The kernel can also split the columns over grid.y, 32 NT per workgroup: the
-  // workgroups that share X rows are then a multiple of 8 apart in launch order, i.e. on one XCD and its L2.  Measured at
-  // 192 = 2 x 96 and 256 = 4 x 64 columns it only equals the kernels above, because every column block splits the X rows
-  // again, so those widths are not routed here.)
-  const int ycount = Nout / (32 * NT);
-  const dim3 grid(static_cast<unsigned>(std::max(8, device_compute_units() / ycount / 8 * 8)), static_cast<unsigned>(ycount)), block(kResWaves * kWave);
+                    int zero_last_group, float scale, const float *row_scale, float *OUT, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(device_compute_units())), block(kResWaves * kWave);
   if (row_scale)
     hipLaunchKernelGGL((linear_resident_kernel<K, NT, true>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
-                       zero_last_group, Nout, scale, row_scale, OUT);
+                       zero_last_group, scale, row_scale, OUT);
   else
     hipLaunchKernelGGL((linear_resident_kernel<K, NT, false>), grid, block, 0, st, X, WT, perm, offs, static_cast<int>(nnodes), ngroups,
-                       zero_last_group, Nout, scale, row_scale, OUT);
+                       zero_last_group, scale, row_scale, OUT);
   return check_launch("cm_linear");
 }
 
@@ -1505,7 +1478,7 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
   if (ncomp == 16 && K == Nout && !residual && ngroups <= cm::kResMaxGroups && nnodes >= cm::kResMinNodes) {
     switch (K) {
 #define CM_CASE(K_, NT_) \
-      case K_: return cm::launch_resident<K_, NT_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, Nout, scale, row_scale, OUT, st);
+      case K_: return cm::launch_resident<K_, NT_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, scale, row_scale, OUT, st);
       CM_CASE(64, 2) CM_CASE(96, 3) CM_CASE(128, 4)
 #undef CM_CASE
 #define CM_CASE(NT_, CB_) \
