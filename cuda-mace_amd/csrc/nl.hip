@@ -21,6 +21,7 @@
 // rounding in the fractional coordinates cannot lose a pair.  Atoms may lie outside the cell (unwrapped
 // trajectories): the wrap count of each atom enters S.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 
 #include "common.hpp"
@@ -511,9 +512,12 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
 }
 
 // offsets[0 .. n] = exclusive scan of degree[0 .. n-1] and, next to it, the grid's status and the largest degree; one
-// workgroup, every thread a contiguous run.
+// workgroup, every thread a contiguous run.  `counts` (two words of host memory, may be NULL): offsets[n] in the upper half
+// of the first, the largest degree and the status above bit 0 in the second, and bit 0 of each set, so that a host that
+// polls them needs no order between the two stores (a release to the host would write back the whole L2 first).
 __global__ __launch_bounds__(kGridThreads) void nl_offsets_kernel(Workspace w, int n, int32_t *__restrict__ offsets,
-                                                                  int32_t *__restrict__ status, int32_t *__restrict__ max_degree) {
+                                                                  int32_t *__restrict__ status, int32_t *__restrict__ max_degree,
+                                                                  unsigned long long *__restrict__ counts) {
   __shared__ long long part[kGridThreads];
   __shared__ long long stage[kOffsetsStage];
   __shared__ int s_most[kGridThreads / kWave];
@@ -528,10 +532,18 @@ __global__ __launch_bounds__(kGridThreads) void nl_offsets_kernel(Workspace w, i
   if (threadIdx.x % kWave == 0) s_most[threadIdx.x / kWave] = most;
   __syncthreads();
   if (threadIdx.x == 0) {
-    offsets[n] = static_cast<int32_t>(total > INT32_MAX ? INT32_MAX : total);
-    *status = w.grid->status;
+    const int32_t pairs = static_cast<int32_t>(total > INT32_MAX ? INT32_MAX : total), state = w.grid->status;
+    offsets[n] = pairs;
+    if (status) *status = state;
     for (int q = 1; q < kGridThreads / kWave; ++q) most = max(most, s_most[q]);
     if (max_degree) *max_degree = most;
+    if (counts) {
+      const auto word = [](int32_t high, int32_t low) {
+        return static_cast<unsigned long long>(static_cast<uint32_t>(high)) << 32 | static_cast<unsigned long long>(low) << 1 | 1ull;
+      };
+      __hip_atomic_store(counts, word(pairs, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(counts + 1, word(most, state), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -654,12 +666,12 @@ namespace {
 
 // Everything up to the offsets of the segments: the cell list and the count of every atom's neighbours.
 int search(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z, double cutoff, int64_t nnodes, int64_t max_cells,
-           void *workspace, size_t workspace_bytes, int32_t *offsets, int32_t *status, int32_t *max_degree, hipStream_t st,
-           const char *what) {
+           void *workspace, size_t workspace_bytes, int32_t *offsets, int32_t *status, int32_t *max_degree,
+           unsigned long long *counts, hipStream_t st, const char *what) {
   CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4, "%s: nnodes out of range", what);
   CM_REQUIRE(max_cells >= 1 && max_cells < INT32_MAX / 2, "%s: max_cells out of range", what);
   CM_REQUIRE(cutoff > 0.0 && std::isfinite(cutoff), "%s: cutoff must be positive and finite", what);
-  CM_REQUIRE(offsets != nullptr && status != nullptr, "%s: offsets / status is NULL", what);
+  CM_REQUIRE(offsets != nullptr && (status != nullptr || counts != nullptr), "%s: offsets / status is NULL", what);
   CM_REQUIRE(nnodes == 0 || positions != nullptr, "%s: positions is NULL", what);
   CM_REQUIRE(cell != nullptr || !(pbc_x || pbc_y || pbc_z), "%s: a periodic axis needs a cell", what);
   const Workspace w = carve(workspace, nnodes, max_cells);
@@ -682,7 +694,7 @@ int search(const double *positions, const double *cell, int pbc_x, int pbc_y, in
   if (n > 0)
     hipLaunchKernelGGL(nl_scan_kernel<Scan::kCount>, dim3(static_cast<unsigned>(ceil_div(n, kScanWaves))), dim3(kScanWaves * kWave), 0, st,
                        w, cutoff, n, static_cast<const int32_t *>(nullptr), int64_t{0}, static_cast<int32_t *>(nullptr), GraphOut{}, 0);
-  hipLaunchKernelGGL(nl_offsets_kernel, dim3(1), dim3(kGridThreads), 0, st, w, n, offsets, status, max_degree);
+  hipLaunchKernelGGL(nl_offsets_kernel, dim3(1), dim3(kGridThreads), 0, st, w, n, offsets, status, max_degree, counts);
   return check_launch(what);
 }
 
@@ -693,7 +705,7 @@ extern "C" int cm_neighbour_list_count(const double *positions, const double *ce
                                        double cutoff, int64_t nnodes, int64_t max_cells, void *workspace,
                                        size_t workspace_bytes, int32_t *offsets, int32_t *status, cm_stream_t stream) {
   return cm::search(positions, cell, pbc_x, pbc_y, pbc_z, cutoff, nnodes, max_cells, workspace, workspace_bytes, offsets, status, nullptr,
-                    cm::as_stream(stream), "cm_neighbour_list_count");
+                    nullptr, cm::as_stream(stream), "cm_neighbour_list_count");
 }
 
 extern "C" int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnodes, int64_t max_cells,
@@ -722,7 +734,48 @@ extern "C" int cm_neighbour_list_search(const double *positions, const double *c
                                         cm_stream_t stream) {
   CM_REQUIRE(max_degree != nullptr, "cm_neighbour_list_search: max_degree is NULL");
   return cm::search(positions, cell, pbc_x, pbc_y, pbc_z, cutoff, nnodes, max_cells, workspace, workspace_bytes, offsets, status,
-                    max_degree, cm::as_stream(stream), "cm_neighbour_list_search");
+                    max_degree, nullptr, cm::as_stream(stream), "cm_neighbour_list_search");
+}
+
+// The host needs three numbers before it can ask for the list's memory.  The kernel writes them into host memory itself and
+// the host polls for them: the copy of three words and the wait for it took 12 us longer (2 000 atoms: search, list and step 393
+// -> 376 us with this and with what the host allocates before the wait in place of after it).  A search that has not ended after two
+// milliseconds sits behind other work of the stream, where that does not matter, and the host waits for the stream.  The call
+// returns once the device is done with `counts`, whatever it returns.
+extern "C" int cm_neighbour_list_search_counts(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z,
+                                               double cutoff, int64_t nnodes, int64_t max_cells, void *workspace,
+                                               size_t workspace_bytes, int32_t *offsets, int64_t *counts, int32_t *values,
+                                               cm_stream_t stream) {
+  static const char *what = "cm_neighbour_list_search_counts";
+  CM_REQUIRE(counts != nullptr && values != nullptr, "%s: counts / values is NULL", what);
+  hipStream_t st = cm::as_stream(stream);
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  CM_REQUIRE(hipStreamIsCapturing(st, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone,
+             "%s: the host has to read the number of pairs, which a stream under capture does not deliver", what);
+  uint64_t word[2];
+  const auto landed = [&] {
+    for (int k = 0; k < 2; ++k) word[k] = static_cast<uint64_t>(__atomic_load_n(counts + k, __ATOMIC_ACQUIRE));
+    return (word[0] & word[1] & 1) != 0;
+  };
+  for (int k = 0; k < 2; ++k) __atomic_store_n(counts + k, int64_t{0}, __ATOMIC_RELEASE);
+  int rc = cm::search(positions, cell, pbc_x, pbc_y, pbc_z, cutoff, nnodes, max_cells, workspace, workspace_bytes, offsets, nullptr, nullptr,
+                      reinterpret_cast<unsigned long long *>(counts), st, what);
+  if (rc == CM_EINVAL || rc == CM_ENOSPC) return rc;  // nothing was launched
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  while (rc == CM_OK && !landed() && std::chrono::steady_clock::now() < until) {
+  }
+  if (rc != CM_OK || !landed()) {
+    const hipError_t err = hipStreamSynchronize(st);
+    if (rc != CM_OK) return rc;
+    if (err != hipSuccess || !landed()) {
+      cm::set_error("%s: %s", what, hipGetErrorString(err));
+      return CM_ELAUNCH;
+    }
+  }
+  values[0] = static_cast<int32_t>(word[0] >> 32);
+  values[1] = static_cast<int32_t>(static_cast<uint32_t>(word[1]) >> 1);
+  values[2] = static_cast<int32_t>(word[1] >> 32);
+  return CM_OK;
 }
 
 // A wave keeps a segment's hits in LDS, 16 bytes each: four waves per workgroup up to 512 of them, then one.

@@ -76,6 +76,7 @@ SIGNATURES = {
     "cm_neighbour_list_count": (_i32, [_p, _p, _i32, _i32, _i32, _f64, _i64, _i64, _p, _sz, _p, _p, _p]),
     "cm_neighbour_list_fill": (_i32, [_p, _f64, _i64, _i64, _p, _p, _i64, _p, _p, _p, _p, _p]),
     "cm_neighbour_list_search": (_i32, [_p, _p, _i32, _i32, _i32, _f64, _i64, _i64, _p, _sz, _p, _p, _p, _p]),
+    "cm_neighbour_list_search_counts": (_i32, [_p, _p, _i32, _i32, _i32, _f64, _i64, _i64, _p, _sz, _p, _p, _p, _p]),
     "cm_neighbour_list_graph_max_degree": (_i32, []),
     "cm_neighbour_list_graph": (_i32, [_f64, _i64, _i64, _p, _p, _i64, _i32] + [_p] * 10),
     "cm_symmetric_sender_view": (_i32, [_p, _p, _p, _p, _i64, _i64, _p, _p]),
@@ -659,31 +660,35 @@ def neighbour_graph(positions, cell, pbc, cutoff: float, max_cells: int = 0):
     max_cells = int(max_cells) if max_cells else max(1, min(N, 1 << 22))
     ws_bytes = lib.cm_neighbour_list_workspace(N, max_cells)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    head = torch.empty(N + 3, dtype=I32, device=dev)  # offsets [N + 1], status, largest degree
-    offsets_ptr = head.data_ptr()
+    offsets = torch.empty(N + 1, dtype=I32, device=dev)
+    offsets_ptr = offsets.data_ptr()
+    # what does not depend on the numbers the host waits for is there before they come: from then to the next launch the
+    # device idles
+    first_occ = torch.empty(2 * N, dtype=I32, device=dev)
+    batch, ptr = torch.empty(N, dtype=I64, device=dev), torch.empty(2, dtype=I64, device=dev)
+    ptr32 = torch.empty(2, dtype=I32, device=dev)
+    counts = torch.empty(2, dtype=I64, pin_memory=True)  # host memory the device writes, of this call alone
+    values = (ctypes.c_int32 * 3)()
     px, py, pz = (int(bool(b)) for b in pbc)
     stream = _stream()
-    _check(lib.cm_neighbour_list_search(_dev(positions, F64, "positions"), _dev(cell, F64, "cell"), px, py, pz, float(cutoff), N, max_cells,
-                                        ws.data_ptr(), ws_bytes, offsets_ptr, offsets_ptr + 4 * (N + 1), offsets_ptr + 4 * (N + 2), stream))
-    E, status, most = head[N:].tolist()
+    at_search = (float(cutoff), N, max_cells, ws.data_ptr())
+    at_nodes = (first_occ.data_ptr(), batch.data_ptr(), ptr.data_ptr(), ptr32.data_ptr(), stream)
+    _check(lib.cm_neighbour_list_search_counts(_dev(positions, F64, "positions"), _dev(cell, F64, "cell"), px, py, pz, *at_search, ws_bytes,
+                                               offsets_ptr, counts.data_ptr(), ctypes.addressof(values), stream))
+    E, status, most = values
     _list_status(E, status)
     if most > _GRAPH_MAX_DEGREE:
         return None
     row_i, row_j = torch.empty(E, dtype=I32, device=dev), torch.empty(E, dtype=I32, device=dev)
     edge_index = torch.empty(2, E, dtype=I64, device=dev)
     unit_shifts, shifts = torch.empty(E, 3, dtype=F64, device=dev), torch.empty(E, 3, dtype=F64, device=dev)
-    first_occ = torch.empty(2 * N, dtype=I32, device=dev)
-    batch, ptr = torch.empty(N, dtype=I64, device=dev), torch.empty(2, dtype=I64, device=dev)
-    ptr32 = torch.empty(2, dtype=I32, device=dev)
     if N > 0:
-        at = lambda t: t.data_ptr() if E > 0 else None  # noqa: E731
-        _check(lib.cm_neighbour_list_graph(float(cutoff), N, max_cells, ws.data_ptr(), offsets_ptr, E, most, at(row_i), at(row_j),
-                                           at(edge_index), at(unit_shifts), at(shifts), first_occ.data_ptr(), batch.data_ptr(),
-                                           ptr.data_ptr(), ptr32.data_ptr(), stream))
+        _check(lib.cm_neighbour_list_graph(*at_search, offsets_ptr, E, most, row_i.data_ptr(), row_j.data_ptr(), edge_index.data_ptr(),
+                                           unit_shifts.data_ptr(), shifts.data_ptr(), *at_nodes))
     else:
         ptr.zero_(), ptr32.zero_()
     return {"row_i": row_i, "row_j": row_j, "edge_index": edge_index, "unit_shifts": unit_shifts, "shifts": shifts,
-            "first_occ": first_occ, "offsets": head[:N + 1], "batch": batch, "ptr": ptr, "ptr32": ptr32}
+            "first_occ": first_occ, "offsets": offsets, "batch": batch, "ptr": ptr, "ptr32": ptr32}
 
 
 def symmetric_sender_view(row_i, row_j, unit_shifts, first_occ, nnodes: int):

@@ -393,6 +393,9 @@ int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnode
 /* The same list with everything the model reads of it, in two calls that launch three kernels (up to 4 096 atoms,
  * seven beyond) and one:
  *   cm_neighbour_list_search: cm_neighbour_list_count, and max_degree int32 [1] = the most neighbours of one atom.
+ *   cm_neighbour_list_search_counts: the same for a host that needs the numbers at once: values int32 [3] (host) =
+ *     offsets[nnodes], status, max_degree on return.  counts int64 [2] is host memory that the device can write
+ *     (hipHostMalloc), of this call alone.  The one entry that waits for the device; refused while the stream is captured.
  *   cm_neighbour_list_graph: after the caller has read offsets[nnodes] = nedges and max_degree (at most
  *     cm_neighbour_list_graph_max_degree(); beyond that, cm_neighbour_list_fill), writes row_i, row_j int32 [nedges],
  *     edge_index int64 [2, nedges] (the same rows), unit_shifts fp64 [nedges, 3], shifts fp64 [nedges, 3] = S . cell (term by
@@ -405,6 +408,9 @@ int cm_neighbour_list_fill(const double *positions, double cutoff, int64_t nnode
 int cm_neighbour_list_search(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z, double cutoff,
                              int64_t nnodes, int64_t max_cells, void *workspace, size_t workspace_bytes, int32_t *offsets,
                              int32_t *status, int32_t *max_degree, cm_stream_t stream);
+int cm_neighbour_list_search_counts(const double *positions, const double *cell, int pbc_x, int pbc_y, int pbc_z, double cutoff,
+                                    int64_t nnodes, int64_t max_cells, void *workspace, size_t workspace_bytes, int32_t *offsets,
+                                    int64_t *counts, int32_t *values, cm_stream_t stream);
 int cm_neighbour_list_graph_max_degree(void);
 int cm_neighbour_list_graph(double cutoff, int64_t nnodes, int64_t max_cells, const void *workspace, const int32_t *offsets,
                             int64_t nedges, int max_degree, int32_t *row_i, int32_t *row_j, int64_t *edge_index,

@@ -136,6 +136,26 @@ def test_graph_of_a_list(cabi, name):
     assert torch.equal(cabi_mod.symmetric_sender_view(g["row_i"], g["row_j"], g["unit_shifts"], g["first_occ"], n), perm)
 
 
+@pytest.mark.parametrize("n", [0, 1, 300, 4097])
+@pytest.mark.parametrize("fills", [0, 60])
+def test_counts_reach_a_waiting_host(cabi, n, fills):
+    """The numbers the host polls for: with the stream idle, and with some ten milliseconds of fills of 1 GiB ahead of the
+    search (the host then gives up polling and waits for the stream), against the entry that leaves them on the device."""
+    from cuda_mace import _cabi as cabi_mod
+
+    rng = np.random.default_rng(n)
+    p = torch.tensor(rng.uniform(0.0, 1.0 + 3.0 * n ** (1.0 / 3.0), (n, 3)), dtype=torch.float64, device=DEV)
+    ri, rj, _ = cabi_mod.neighbour_list(p, None, (False,) * 3, 4.0)
+    ahead = torch.empty(1 << 28 if fills else 0, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(fills):
+        ahead.fill_(1.0)
+    g = cabi_mod.neighbour_graph(p, None, (False,) * 3, 4.0)
+    assert torch.equal(g["row_i"], ri) and torch.equal(g["row_j"], rj)
+    assert g["offsets"].shape == (n + 1,) and int(g["offsets"][-1]) == ri.numel()
+    assert g["ptr"].tolist() == [0, n]
+
+
 @pytest.mark.parametrize("satellites", [4097, 8191, 8192, 8300])
 def test_atom_with_thousands_of_neighbours(cabi, satellites):
     """One atom in the middle of a shell of others, all within its cutoff: up to 8 192 neighbours the last pass keeps them in
