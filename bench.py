@@ -106,18 +106,22 @@ def spline_backward_kernel_name(C, E):
 
 
 def linear_kernel_name(C, N):
-    """The library runs the [N,16,C] channel-mixing linear without tiles for few nodes, from 2 048 nodes on with the weights
-    resident (64, 96 and 128 columns: in LDS, 160 and more: in registers), else on the LDS-ring kernel for 64, 96, 128, 224
-    and 256 columns and on the plain one otherwise."""
+    """The library runs the [N,16,C] channel-mixing linear (one weight group) without tiles for few nodes, with a workgroup per 128
+    rows up to some thousand, and with the weights resident beyond (64, 96 and 128 columns: in LDS, 160 and more: in registers)."""
     nt = C // 32
     blocks = (N + 15) // 16 * C
     if blocks <= 3072:
         return "linear_few_rows_kernel<%d,false,%d>" % (C // 16, 1 if blocks <= 1024 else 2)
-    if nt in (2, 3, 4) and N >= 2048:
+    rows = (16 * N + 127) // 128
+    most = 0 if nt == 1 else 2 * nt if nt <= 6 else nt
+    one_round = 256 // (2 * nt // most) if most else 0
+    if 2 <= nt <= 4 and N * C <= 25000 * 64 or nt >= 5 and (N < 2048 or rows <= (2 if nt <= 6 else 1) * one_round):
+        return "linear_block_kernel<%d,%d,false>" % (nt, most // 2 if nt != 7 and 2 * rows <= one_round else most)
+    if nt in (2, 3, 4):
         return "linear_resident_kernel<%d,%d,false>" % (C, nt)
-    if nt >= 5 and N >= 2048:
+    if nt >= 5:
         return "linear_wide_kernel<%d,%d,16,false>" % (nt, 2 if nt == 8 else 1)
-    return ("linear_ring_kernel<%d,false>" if nt in (2, 3, 4, 7, 8) else "linear_kernel<%d,false>") % nt
+    return "linear_kernel<%d,false>" % nt
 
 
 def mp_algorithmic_bytes(N, E, C):
@@ -563,7 +567,7 @@ def main():
             tf = flops / (t_lin * 1e-3) / 1e12
             lin_bytes = 4 * (32 * N * C + 4 * C * C)
             # resident weights: two fp16 pieces per operand, three products; the others: three bf16 pieces, six
-            pieces = 3 if linear_kernel_name(C, N).startswith(("linear_resident", "linear_wide")) else 6
+            pieces = 3 if linear_kernel_name(C, N).startswith(("linear_resident", "linear_wide", "linear_block")) else 6
             others.append(entry(linear_kernel_name(C, N), lin_bytes, t_lin, launches_timed=launches("linear"),
                                 matrix_cores={"fp32_equivalent_TFLOP/s": round(tf, 1), "instruction_TFLOP/s_16_bit": round(pieces * tf, 1),
                                               "frac_of_16_bit_peak": round(pieces * tf / 2500.0, 4)},

@@ -484,9 +484,8 @@ def test_linear_few_rows(cabi, N, C, ncomp, ne):
 
 @pytest.mark.parametrize("N,C,ne,seed", [(2048, 128, 1, 0), (2500, 128, 10, 1), (4099, 96, 5, 2), (3000, 64, 3, 3), (6000, 128, 130, 4)])
 def test_linear_many_rows(cabi, N, C, ne, seed):
-    """16-component features with at least 2048 nodes and 64 / 96 / 128 square weights run on the kernel that keeps the
-    weight block in LDS (one workgroup per compute unit walking 32-row tiles); more than 128 weight groups stay on the
-    tiled kernels.  Groups of very different sizes, an empty group, a group of one node, tiles that end inside a group,
+    """16-component features with 64 / 96 / 128 square weights at some thousand nodes: a workgroup per 128 rows of one weight
+    block; more than 128 weight groups stay on the tiled kernels.  Groups of very different sizes, an empty group, a group of one node, tiles that end inside a group,
     rows of no group, with and without row_scale; twice, for the same bits."""
     _say("linear_many_rows", N, C, ne, seed)
     g = torch.Generator().manual_seed(seed)
@@ -533,6 +532,42 @@ def test_linear_many_rows_wide(cabi, N, C, ne, seed):
     """The same at 160 to 256 columns, where from 2 048 nodes on the weights stay in registers and the workgroup's waves share
     16-row tiles."""
     test_linear_many_rows(cabi, N, C, ne, seed)
+
+
+@pytest.mark.parametrize("N,C,ne,seed", [(12_500, 128, 4, 0), (12_501, 128, 10, 1), (25_001, 64, 3, 2), (16_667, 96, 1, 3), (5000, 64, 100, 4), (9, 224, 3, 5),
+                                         (130, 256, 63, 6), (129, 160, 64, 7), (1025, 192, 3, 8), (2047, 224, 2, 9), (4100, 160, 10, 10), (700, 128, 3, 11)])
+def test_linear_rows_of_a_weight_block(cabi, N, C, ne, seed):
+    """Both sides of the lines of the kernel with a workgroup per 128 rows: features that fit the last-level cache and those that do not
+    (the weights resident, 16-row tiles), 64 weight groups and more, one and two rounds of workgroups at 160 to 256 columns, half and all
+    columns per workgroup."""
+    test_linear_many_rows(cabi, N, C, ne, seed)
+
+
+@pytest.mark.parametrize("N,C,ne", [(1000, 160, 3), (3001, 192, 10), (9001, 256, 10), (8200, 224, 63), (8193, 160, 64), (33_000, 192, 2)])
+def test_scalar_linear_of_a_weight_block(cabi, N, C, ne):
+    """The same for [N, C] features with a weight block per group (rows of no group included) and with one for all, with a residual that is
+    the output itself."""
+    _say("scalar_linear_of_a_weight_block", N, C, ne)
+    g = torch.Generator().manual_seed(N + C)
+    X, R = torch.randn(N, C, generator=g), torch.randn(N, C, generator=g)
+    W = torch.randn(ne, C, C, generator=g)
+    elem = torch.randint(0, ne + 1, (N,), generator=g)
+    perm, off = cabi.stable_key_sort(elem.int().to(DEV), ne + 1)
+    d = lambda t: t.contiguous().to(DEV)  # noqa: E731
+    ref = torch.zeros(N, C, dtype=torch.float64)
+    for e in range(ne):
+        ref[elem == e] = X[elem == e].double() @ W[e].double()
+    WT = d(W.transpose(-1, -2))
+    out = cabi.linear(d(X), WT, perm, off, scale=1.0, zero_last_group=True)
+    close(out, ref, 1e-5, 2e-6)
+    shared = cabi.linear(d(X), WT[:1], scale=1.0)
+    close(shared, X.double() @ W[0].double(), 1e-5, 2e-6)
+    for want, weights, p, o, zero in ((out, WT, perm, off, 1), (shared, WT[:1], None, None, 0)):
+        inout, Xd = d(R), d(X)
+        cabi._check(cabi.lib.cm_linear(Xd.data_ptr(), weights.data_ptr(), p.data_ptr() if zero else None, o.data_ptr() if zero else None, N,
+                                       ne + 1 if zero else 1, zero, 1, C, C, 1.0, None, inout.data_ptr(), inout.data_ptr(),
+                                       torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(inout, want + d(R))
 
 
 @pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256)])
