@@ -113,9 +113,9 @@ def linear_kernel_name(C, N):
     if blocks <= 3072:
         return "linear_few_rows_kernel<%d,false,%d>" % (C // 16, 1 if blocks <= 1024 else 2)
     rows = (16 * N + 127) // 128
-    most = 0 if nt == 1 else 2 * nt if nt <= 6 else nt
-    one_round = 256 // (2 * nt // most) if most else 0
-    if 2 <= nt <= 4 and N * C <= 25000 * 64 or nt >= 5 and (N < 2048 or rows <= (2 if nt <= 6 else 1) * one_round):
+    most = 2 * nt if nt <= 6 else nt
+    one_round = 256 // (2 * nt // most)
+    if nt <= 4 and rows <= 4 * 256 or nt >= 5 and (N < 2048 or rows <= (2 if nt <= 6 else 1) * one_round):
         return "linear_block_kernel<%d,%d,false>" % (nt, most // 2 if nt != 7 and 2 * rows <= one_round else most)
     if nt in (2, 3, 4):
         return "linear_resident_kernel<%d,%d,false>" % (C, nt)

@@ -27,6 +27,7 @@
 
 #include "common.hpp"
 #include "mfma_f32.hpp"
+#include "mfma_rows.hpp"
 #include "mfma_split.hpp"
 
 namespace cm {
@@ -745,7 +746,7 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 constexpr int kResWaves = 8;
 constexpr int kResRows = 16;   // rows of a tile
 constexpr int kResSegRows = 2048;  // rows whose numbers a segment keeps in LDS
-typedef float v4f __attribute__((ext_vector_type(4)));
+using rows::v4f;
 constexpr int kResMaxGroups = 128;
 constexpr int kResMinNodes = 2048;
 constexpr int kOutLd = 36;            // floats per row of a wave's output staging block (32 columns + 16 bytes)
@@ -771,7 +772,7 @@ __device__ __forceinline__ void first_tiles(const int32_t *__restrict__ group_of
   }
 }
 
-__device__ __forceinline__ float largest4(f4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
+using rows::largest4;
 // largest value over eight neighbouring lanes, in all of them
 __device__ __forceinline__ float max_over_8(float v) {
   auto with = [&](auto ctrl) {
@@ -1347,8 +1348,7 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
 // ones walk K in phases.  Here a workgroup has one weight block and each of its eight waves one tile of 16 rows, so everything is asked
 // for at once: group offsets, then the weights and the row numbers, then the rows, one barrier, the products, the stores.  Rows of a
 // degree are counted node by node (row r of degree l is component l^2 + r % (2l + 1) of the block's node r / (2l + 1)): the rows of a wave lie
-// side by side in memory.  Arithmetic and operand layout as in linear_resident_kernel; a lane takes columns 32 s + 4 q + {0..3} and 32 s +
-// 16 + 4 q + {0..3} for its k step s (q: lane / 16), so that a load covers 64 bytes of a row, and the weight planes are written in that order.
+// side by side in memory.  Arithmetic as in linear_resident_kernel, operands as in mfma_rows.hpp (a load covers 64 bytes of a row).
 // Columns are split over COLS / 16 NB workgroups where the rows alone leave compute units idle, and where the planes of all would not fit LDS.
 // -----------------------------------------------------------------------------------------------
 constexpr int kBlockWaves = 8;
@@ -1366,34 +1366,37 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
   constexpr int K = 32 * KS;
   constexpr int NOUT = K;
   constexpr int COLS = 16 * NB;  // columns of this workgroup
-  constexpr int LD = K + 8;      // row stride of a plane in elements: an odd number of 16-byte units
-  __shared__ __attribute__((aligned(16))) _Float16 sW[2 * COLS * LD];
-  __shared__ __attribute__((aligned(16))) float sColumn[COLS];  // what takes a weight column's scale back
+  __shared__ __attribute__((aligned(16))) rows::Planes<KS, COLS> planes;
 
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int r16 = lane % 16, quarter = lane / 16;
   const int col0 = blockIdx.y * COLS;
 
   // weight group, its first place in the node order and its number of nodes; the block among the group's
   int g = 0, off0 = 0, n = nnodes, block = blockIdx.x;
-  if (group_offsets) {  // at most 64 groups, one per lane
-    const int lo = lane < ngroups ? group_offsets[lane] : 0, hi = lane < ngroups ? group_offsets[lane + 1] : 0;
-    const int blocks = row_blocks(max(hi - lo, 0), ncomp);
-    int upto = blocks;  // inclusive prefix sum over the lanes
-    for (int d = 1; d < ngroups; d <<= 1) {
-      const int v = __shfl_up(upto, d);
-      if (lane >= d) upto += v;
+  if (group_offsets) {  // 64 groups at a time, one per lane
+    for (int g0 = 0;; g0 += kWave) {
+      if (g0 >= ngroups) return;
+      const bool has = g0 + lane < ngroups;
+      const int lo = has ? group_offsets[g0 + lane] : 0, hi = has ? group_offsets[g0 + lane + 1] : 0;
+      const int blocks = row_blocks(max(hi - lo, 0), ncomp);
+      int upto = blocks;  // inclusive prefix sum over the lanes
+      for (int d = 1; d < min(ngroups - g0, kWave); d <<= 1) {
+        const int v = __shfl_up(upto, d);
+        if (lane >= d) upto += v;
+      }
+      const unsigned long long owners = __ballot(has && block < upto);
+      if (owners != 0) {
+        const int owner = __ffsll(static_cast<long long>(owners)) - 1;
+        g = g0 + owner;
+        block -= __builtin_amdgcn_readlane(upto - blocks, owner);
+        off0 = __builtin_amdgcn_readlane(lo, owner);
+        n = __builtin_amdgcn_readlane(hi, owner) - off0;
+        break;
+      }
+      block -= __builtin_amdgcn_readlane(upto, kWave - 1);
     }
-    const unsigned long long owners = __ballot(block < upto);
-    if (owners == 0) return;
-    g = __ffsll(static_cast<long long>(owners)) - 1;
-    block -= __builtin_amdgcn_readlane(upto - blocks, g);
-    off0 = __builtin_amdgcn_readlane(lo, g);
-    n = __builtin_amdgcn_readlane(hi, g) - off0;
-  } else if (block >= row_blocks(n, ncomp)) {
-    return;
   }
   int l = 0, nm = 1;
   if (ncomp != 1) {
@@ -1410,18 +1413,8 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
   int node = off0 + t;
   bool valid = t < n;
   if (node_perm) node = node_perm[valid ? node : off0];
-  constexpr int kLanes = 4;  // threads per weight column
-  constexpr int kPasses = (COLS * kLanes + kBlockWaves * kWave - 1) / (kBlockWaves * kWave);
-  f4 wv[kPasses][2 * KS];
-  if (!zero) {
-    const float *Wg = WT + ((static_cast<int64_t>(g) * (ncomp == 1 ? 1 : 4) + l) * NOUT + col0) * K + 4 * (tid % kLanes);
-#pragma unroll
-    for (int p = 0; p < kPasses; ++p) {
-      const int col = min(p * (kBlockWaves * kWave / kLanes) + tid / kLanes, COLS - 1);  // beyond the last: that one again
-#pragma unroll
-      for (int i = 0; i < 2 * KS; ++i) wv[p][i] = ld4(Wg + static_cast<int64_t>(col) * K + 16 * i);
-    }
-  }
+  rows::Fetched<KS, COLS, kBlockWaves * kWave> weights;
+  if (!zero) weights.request(WT + ((static_cast<int64_t>(g) * (ncomp == 1 ? 1 : 4) + l) * NOUT + col0) * K);
   valid = valid && static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
   if (!valid) node = 0;  // read, never stored
   const int64_t row = static_cast<int64_t>(node) * ncomp + (valid ? l * l + (r - t * nm) : 0);
@@ -1433,127 +1426,61 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
     for (int cb = 0; cb < NB; ++cb) st4(op + 16 * cb, rp ? ld4(rp + 16 * cb) : zero4());
     return;
   }
-  f4 xv[2 * KS];
-  {
-    const float *xp = X + row * K + 4 * quarter;
-#pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) xv[i] = ld4(xp + 16 * i);
-  }
-  f4 sv[SCALED ? 2 * KS : 1];
+  f4 x[2 * KS], factor[SCALED ? 2 * KS : 1];
+  rows::load(X + row * K, x);
+  if constexpr (SCALED) rows::load(row_scale + static_cast<int64_t>(node) * K, factor);
+  weights.store(planes, scale);
   if constexpr (SCALED) {
-    const float *sp = row_scale + static_cast<int64_t>(node) * K + 4 * quarter;
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) sv[i] = ld4(sp + 16 * i);
+    for (int i = 0; i < 2 * KS; ++i) x[i] *= factor[i];
   }
-
-#pragma unroll
-  for (int p = 0; p < kPasses; ++p) {
-    const int col = p * (kBlockWaves * kWave / kLanes) + tid / kLanes;
-    float big = 0.f;
-#pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) big = fmaxf(big, largest4(wv[p][i]));
-    big = fmaxf(big, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, big), 0xB1, 0xf, 0xf, false)));
-    big = fmaxf(big, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, big), 0x4E, 0xf, 0xf, false)));
-    const PieceScale of = piece_scale(big, kLeastColumnExponent);
-    if (col < COLS) {
-      _Float16 *to = sW + col * LD + 8 * (tid % kLanes);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        f16x4 h0, l0, h1, l1;
-        split2(wv[p][2 * s], of.s, h0, l0);
-        split2(wv[p][2 * s + 1], of.s, h1, l1);
-        *reinterpret_cast<f16x8 *>(to + 32 * s) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-        *reinterpret_cast<f16x8 *>(to + COLS * LD + 32 * s) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
-      if (tid % kLanes == 0) sColumn[col] = ldexpf(scale, of.exponent);
-    }
-  }
-
-  float big = 0.f;
-#pragma unroll
-  for (int i = 0; i < 2 * KS; ++i) {
-    if constexpr (SCALED) xv[i] *= sv[i];
-    big = fmaxf(big, largest4(xv[i]));
-  }
-  big = fmaxf(big, __shfl_xor(big, 16));
-  big = fmaxf(big, __shfl_xor(big, 32));  // the four lanes of a row
-  const PieceScale of_row = piece_scale(big, kLeastRowExponent);
-  f16x8 x[KS][2];
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    f16x4 h0, l0, h1, l1;
-    split2(xv[2 * s], of_row.s, h0, l0);
-    split2(xv[2 * s + 1], of_row.s, h1, l1);
-    x[s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-    x[s][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-  }
+  const rows::Operand<KS> operand(x);
   __syncthreads();
 
-  const _Float16 *wl = sW + r16 * LD + 8 * quarter;
-  constexpr int GB = NB % 4 == 0 ? 4 : (NB % 3 == 0 ? 3 : (NB % 2 == 0 ? 2 : 1));  // column blocks at a time
+  constexpr int GB = rows::blocks_at_a_time(NB);
 #pragma unroll
-  for (int t0 = 0; t0 < NB; t0 += GB) {
-    v4f acc[GB], small[GB];  // products of high pieces, and those with a low one
-    f4 res[GB];
+  for (int c0 = 0; c0 < NB; c0 += GB) {
+    f4 res[GB], v[GB];
 #pragma unroll
-    for (int c = 0; c < GB; ++c) {
-      acc[c] = small[c] = v4f{0.f, 0.f, 0.f, 0.f};
-      res[c] = rp ? ld4(rp + 16 * (t0 + c)) : zero4();
-    }
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      f16x8 wh[GB], wo[GB];
-#pragma unroll
-      for (int c = 0; c < GB; ++c) {
-        wh[c] = *reinterpret_cast<const f16x8 *>(wl + 16 * (t0 + c) * LD + 32 * s);
-        wo[c] = *reinterpret_cast<const f16x8 *>(wl + COLS * LD + 16 * (t0 + c) * LD + 32 * s);
-      }
-#pragma unroll
-      for (int c = 0; c < GB; ++c) small[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[c], x[s][1], small[c], 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < GB; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[c], x[s][0], acc[c], 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < GB; ++c) small[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wo[c], x[s][0], small[c], 0, 0, 0);
-    }
+    for (int c = 0; c < GB; ++c) res[c] = rp ? ld4(rp + 16 * (c0 + c)) : zero4();
+    rows::product(planes, operand, c0, v);
 #pragma unroll
     for (int c = 0; c < GB; ++c) {
-      f4 v = (acc[c] + small[c]) * ld4(sColumn + 16 * (t0 + c) + 4 * quarter);
       {
 #pragma clang fp contract(off)  // the product is rounded before the residual is added, as everywhere
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = __builtin_ldexpf(v[k], of_row.exponent);
-        if (rp) v = v + res[c];
+        if (rp) v[c] = v[c] + res[c];
       }
-      if (valid) st4(op + 16 * (t0 + c), v);
+      if (valid) st4(op + 16 * (c0 + c), v[c]);
     }
   }
 }
 
 // Column blocks (of 16) per workgroup of linear_block_kernel, or 0: another kernel.  Each line from both sides, us, shared weights /
 // ten weight groups / row_scale / both:
-//  - up to 128 columns, 16 components: as long as X and the result fit the last-level cache together (beyond it the kernel with resident
-//    weights, whose loads are always a tile ahead, streams better).  That kernel -> this one: 2 500 x 128 14.2 / 23.6 / 15.4 / 24.7
-//    -> 12.9 / 14.4 / 15.3 / 16.9, 5 000 x 96 16.1 / 23.3 / 17.9 / 25.8 -> 15.3 / 16.6 / 16.4 / 18.0, 10 000 x 128 37.6 / 43.1 / 39.6 /
-//    49.0 -> 35.0 / 37.3 / 37.0 / 39.0, 25 000 x 64 39 / 42 / 45 / 48 -> 37 / 41 / 42 / 45; 25 000 x 96 58 / 60 / 66 / 70 -> 72 / 76 / 76 / 81.
-//    Ring and tiled kernels, below 2 048 nodes: 700 x 128 9.3 / 11.3 / 10.3 / 12.4 -> 6.8 / 7.2 / 8.2 / 8.7, 2 000 x 128 12.7 / 17.2 / 13.6 /
-//    19.0 -> 9.6 / 13.6 / 11.1 / 16.1, 2 000 x 64 6.1 / 7.5 / 6.7 / 8.2 -> 5.8 / 7.2 / 6.6 / 8.9.
+//  - up to 128 columns, 16 components: up to four workgroups per compute unit (8 192 nodes).  Kernel with resident weights -> this one: 2 500
+//    x 128 16.4 / 20.9 / 18.5 / 22.3 -> 12.8 / 14.2 / 15.3 / 16.7, 5 000 x 96 20.6 / 25.5 / 21.4 / 27.2 -> 15.3 / 16.5 / 16.4 / 18.0.  It stays ahead
+//    on its own beyond that (10 000 x 128 43.6 / 51.3 / 48.1 / 58.2 -> 33.5 / 35.6 / 35.3 / 37.5), but not in a step, where X and the
+//    result share the last-level cache with everything else (step without -> with: 3 000 x 128 398 -> 378, 8 000 x 96 632 -> 616, 5 000 x 64
+//    312 -> 307; 10 000 x 64 504 -> 502, 10 752 x 64 in 512 graphs 285 -> 293, 10 000 x 128 927 -> 933): the other kernel has the loads of a
+//    tile under way while it works on the one before.  Ring and tiled kernels, below 2 048 nodes: 700 x 128 9.5 / 11.4 / 10.4 /
+//    12.4 -> 6.8 / 7.3 / 8.2 / 8.8, 2 000 x 128 12.8 / 17.0 / 13.5 / 19.1 -> 9.6 / 13.8 / 11.0 / 16.5, 2 000 x 64 6.1 / 7.6 / 6.6 / 8.2 -> 5.9 / 7.2 / 6.6 / 9.0.
 //    Half the columns each while that leaves one workgroup per compute unit (700 x 128 7.9 / 8.3 / 9.4 / 9.9 -> the figures above; 1 000
 //    x 128 with groups, two on some: 8.7 -> 10.8).
 //  - beyond 128 columns a compute unit holds one workgroup, and the kernel with weights in registers takes over after one round of them
-//    (two at 160 and 192 columns) where it runs: 1 000 x 192 16.4 / 20.9 / 18.3 / 22.8 -> 10.3 / 14.1 / 12.8 / 16.7, 3 500 x 192 28.6 /
-//    35.5 / 31.1 / 37.0 -> 28.0 / 31.5 / 29.7 / 34.2, 1 000 x 256 24.5 / 32.6 / 27.8 / 35.0 -> 15.1 / 25.6 / 19.0 / 29.4; 2 500 x 256
+//    (two at 160 and 192 columns) where it runs: 1 000 x 192 16.2 / 20.9 / 18.0 / 22.6 -> 10.4 / 14.2 / 12.9 / 16.5, 3 500 x 192 28.6 /
+//    35.5 / 31.1 / 37.0 -> 28.0 / 31.5 / 29.7 / 34.2, 1 000 x 256 24.4 / 32.5 / 27.6 / 34.9 -> 14.8 / 25.5 / 18.6 / 29.3; 2 500 x 256
 //    31.4 / 41.8 / 34.3 / 44.2 -> 37.0 / 43.6 / 42.1 / 49.0.
-//  - one component beyond 128 columns: the same round with one weight group (10 000 x 160 9.7 -> 8.1, 10 000 x 256 17.2 -> 12.5; 35 000 x 192
-//    21.6 -> 24.6); with several, where the other choice is the tiled kernel, always (10 000 x 256 21.5 -> 13.7, 100 000 x 192 61 -> 53),
+//  - one component, up to 128 columns, beyond the few rows of mfma_f32.hpp: always (3 200 x 128 7.5 / 8.0 -> 6.4 / 6.9, 25 000 x 128 12.3 / 13.2
+//    -> 9.4 / 10.0, 60 000 x 64 9.0 / 9.6 -> 8.2 / 8.9); it has the arithmetic of the chains of such products (node_glue.hip).
+//  - one component beyond 128 columns: one round with one weight group (10 000 x 160 9.8 -> 8.1, 10 000 x 256 17.7 -> 12.6; 35 000 x 192
+//    21.6 -> 24.6); with several, where the other choice is the tiled kernel, always (10 000 x 256 21.2 -> 13.7, 100 000 x 192 60 -> 52),
 //    but with row_scale for that round alone (50 000 x 224 55 -> 63).
 int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, bool scaled) {
-  if (K < 64 || ngroups > kWave || (ncomp == 1 && K <= 128)) return 0;
   // a workgroup per 128 rows, and on average half of the weight blocks end in one more
   const int64_t rows = ceil_div(nnodes * ncomp, kBlockRows) + (grouped ? static_cast<int64_t>(ngroups) * (ncomp == 1 ? 1 : 4) / 2 : 0);
   const int all = K / 16;
   if (K <= 128) {
-    constexpr int64_t kCached = 25000 * 64;  // nodes x columns: two times 102 MB
-    if (nnodes * K > kCached) return 0;
+    if (ncomp == 16 && rows > 4 * device_compute_units()) return 0;
     return 2 * rows <= device_compute_units() ? all / 2 : all;
   }
   const int most = K <= 192 ? all : all / 2;  // what fits LDS
@@ -1717,13 +1644,12 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
     switch (32 * K + cm::block_columns(nnodes, ncomp, K, ngroups, group_offsets != nullptr, row_scale != nullptr)) {
 #define CM_CASE(KS_, NB_) \
       case 32 * 32 * KS_ + NB_: return cm::launch_block<KS_, NB_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, ncomp, scale, row_scale, residual, OUT, st);
-      CM_CASE(2, 4) CM_CASE(2, 2) CM_CASE(3, 6) CM_CASE(3, 3) CM_CASE(4, 8) CM_CASE(4, 4) CM_CASE(5, 10) CM_CASE(5, 5)
+      CM_CASE(1, 2) CM_CASE(1, 1) CM_CASE(2, 4) CM_CASE(2, 2) CM_CASE(3, 6) CM_CASE(3, 3) CM_CASE(4, 8) CM_CASE(4, 4) CM_CASE(5, 10) CM_CASE(5, 5)
       CM_CASE(6, 12) CM_CASE(6, 6) CM_CASE(7, 7) CM_CASE(8, 8) CM_CASE(8, 4)
 #undef CM_CASE
     }
   }
-  // 16 components per node, square weights, and features beyond the last-level cache up to 128 columns: the kernel that keeps the
-  // weights in LDS (measured against the ring kernel at 25 000 nodes: 87 vs 102-112 us at 128 channels, 58 vs 67-71 at 96, 42 vs
+  // 16 components per node, square weights, beyond: up to 128 columns the kernel that keeps the weights in LDS (measured against the ring kernel at 25 000 nodes: 87 vs 102-112 us at 128 channels, 58 vs 67-71 at 96, 42 vs
   // 47 at 64; 360 vs 430 us at 100 000 x 128); at 160 to 256 columns the one that keeps them in registers
   if (ncomp == 16 && K == Nout && !residual && ngroups <= cm::kResMaxGroups && nnodes >= cm::kResMinNodes) {
     switch (K) {

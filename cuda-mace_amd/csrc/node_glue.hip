@@ -7,21 +7,21 @@
 //   forward    h1 = B1 . Wprod1          sc = skip_e(h1)   (weights of the node's element)      X2 = h1 . Wup
 //   backward   gh1 = gX2 . Wup^T + g1 + skip_e^T(g2)       gB1 = gh1 . Wprod1^T
 //
-// As separate launches of the linear kernel each of them keeps the device busy for a few microseconds and costs a
-// launch; in the first kernels below a workgroup takes a tile of 128 nodes of one element (32 where the node count leaves
-// most compute units without a tile of 128) through the whole chain.  The intermediate rows (h1, gh1) stay in LDS as fp32 and are the X operand of the next product.  Arithmetic, operand split and accumulation
-// order are those of the linear kernels (three bf16 pieces per fp32 operand, six piece products on
-// v_mfma_f32_32x32x16_bf16, K in chunks of 32), and every intermediate is rounded to fp32 where the separate launches
-// store it, so the chain returns the bits of the separate launches.
+// As separate launches of the linear kernel each of them keeps the device busy for a few microseconds and costs a launch; here a wave takes
+// 16 nodes of one element through the whole chain, the rows in its registers (Chain below), or, for few nodes, a workgroup does.
+// Arithmetic, operand split and accumulation order are those of the linear kernels (mfma_rows.hpp, mfma_f32.hpp), and every
+// intermediate is rounded to fp32 where the separate launches store it, so the chain returns the bits of the separate launches.
 //
 // A third launch has the product linear of the second layer, the readouts and the product of their derivative (node_head below).
 //
 // g1 and g2 are the gradients of minus the (weighted) sum of node energies with respect to the two layers' features:
 // g1[n, c] = -weight[n] scale w1[c] is formed here from the linear readout's weights; g2 = -dE/dh2 arrives as dE/dh2 and
 // its sign goes into the scale of the skip product.
+#include <type_traits>
+
 #include "common.hpp"
 #include "mfma_f32.hpp"
-#include "mfma_split.hpp"
+#include "mfma_rows.hpp"
 #include "node_glue.hpp"
 #include "readout_device.hpp"
 
@@ -32,204 +32,68 @@
 namespace cm {
 namespace {
 
-constexpr int kGlTile = 128;       // nodes per workgroup (ROWS below), or
-constexpr int kGlSmallTile = 32;   // where 128-node tiles would occupy less than half of the compute units
-constexpr int kGlKC = 32;          // K columns staged per step
-constexpr int kGlLdH = kGlKC + 8;  // padded row stride of a bf16 plane (elements)
-constexpr int kGlTPR = kGlKC / 4;  // threads that cover the 32 columns of a staged row, 16 bytes each
-
-// A workgroup has (ROWS / 32) * NT waves (C = 32 NT): wave w owns the 32 x 32 block of the tile's output at rows
-// 32 (w % (ROWS / 32)), columns 32 (w / (ROWS / 32)).  With one wave per block a product's matrix instructions, operand reads and staging
-// are spread over four waves per SIMD, which hide each other's latencies; with four waves and NT blocks each, a chain of
-// three products on one tile of 128 took twice as long (26 against 13 us at 128 channels).  A tile's three products keep
-// the matrix cores of one compute unit busy for 8 us at 128 rows and 128 channels, however few tiles there are: a system
-// of a few hundred atoms takes tiles of 32 rows, NT waves each, on four times as many compute units.
-template <int NT, int ROWS>
-struct GlueShared {
-  static constexpr int C = 32 * NT;
-  static constexpr int kRows = ROWS;
-  static constexpr int kRowWaves = ROWS / 32;
-  static constexpr int kThreads = kRowWaves * NT * kWave;
-  static constexpr int kLdT = C + 4;  // padded row stride of the fp32 tile (floats): rows 16 bytes apart in bank space
-  // pieces of 16 bytes per thread and K chunk: X (ROWS rows x 8 pieces over kThreads threads), weights (C rows x 8)
-  static constexpr int kAPieces = (ROWS * kGlTPR + kThreads - 1) / kThreads;
-  static constexpr int kBPieces = C * kGlTPR / kThreads;
-  static_assert(C * kGlTPR % kThreads == 0, "the weight pieces divide evenly among the threads");
-  __bf16 a[3 * ROWS * kGlLdH];
-  __bf16 b[3 * C * kGlLdH];
-  float tile[ROWS * kLdT];
-  int node[ROWS];
+// A workgroup of WAVES waves: a wave takes 16 nodes of one element through the whole chain.  The result of a product lies in the lanes
+// as the operand of the next one does (mfma_rows.hpp), so the rows never leave the registers, and the waves meet only where the
+// workgroup's weight planes change: all three blocks up to 96 columns, at 128 the third in the place of the first.  Before, tiles of 32 or
+// 128 nodes exchanged the rows through LDS and staged operands for each 32 columns of K between two barriers, three bf16 pieces
+// and six products (us, forward / backward): 5 000 x 96 13.7 / 12.8 -> 10.1 / 10.7, 10 752 x 64 12.4 / 11.1 -> 6.9 / 6.8, 5 000 x 128 15.2 / 13.9 ->
+// 14.1 / 14.3, 25 000 x 128 26.8 / 23.5 -> 20.7 / 20.9 (its 51 MB take 10), 60 000 x 96 40.7 / 36.3 -> 28.1 / 27.4.  What is left at
+// 128 columns: 7 us of matrix instructions and fragment reads for 128 rows, 3 us for the split of three weight blocks, 4 us until the
+// first operands are there.
+template <int NT, int WAVES>
+struct Chain {
+  static constexpr int C = 32 * NT, NB = 2 * NT;
+  static constexpr int kThreads = WAVES * kWave, kRows = 16 * WAVES;
+  static constexpr int kSlots = NT <= 3 ? 3 : 2;
+  using Planes = rows::Planes<NT, C>;
+  using Weights = rows::Fetched<NT, C, kThreads>;
+  using Operand = rows::Operand<NT>;
 };
-
-// Operands of a product on their way from memory: a thread's 16-byte pieces of every K chunk, requested all at once
-// and long before the product that consumes them.
-template <class S>
-struct WeightPieces {
-  f4 v[S::C / kGlKC][S::kBPieces];  // [chunk][i]: row (tid + i kThreads) / 8 of the transposed block, columns 32 chunk + 4 (tid % 8) ..
-};
-template <class S>
-struct RowPieces {
-  f4 v[S::C / kGlKC][S::kAPieces];
-};
-
-template <class S>
-__device__ __forceinline__ void fetch_weights(const float *__restrict__ Wg, WeightPieces<S> &w) {
-#pragma unroll
-  for (int i = 0; i < S::kBPieces; ++i) {
-    const int piece = threadIdx.x + i * S::kThreads;
-    const int srow = piece / kGlTPR, scol = (piece % kGlTPR) * 4;
-#pragma unroll
-    for (int k = 0; k < S::C / kGlKC; ++k) w.v[k][i] = ld4(Wg + static_cast<int64_t>(srow) * S::C + kGlKC * k + scol);
-  }
-}
-
-// rows of X [*, C] named by the tile's node list (zeros for rows beyond the tile)
-template <class S>
-__device__ __forceinline__ void fetch_rows(const S &s, const float *__restrict__ X, RowPieces<S> &a) {
-#pragma unroll
-  for (int i = 0; i < S::kAPieces; ++i) {
-    const int piece = threadIdx.x + i * S::kThreads;
-    const int row = piece / kGlTPR, scol = (piece % kGlTPR) * 4;
-    const int node = row < S::kRows ? s.node[row] : -1;
-#pragma unroll
-    for (int k = 0; k < S::C / kGlKC; ++k) a.v[k][i] = node >= 0 ? ld4(X + static_cast<int64_t>(node) * S::C + kGlKC * k + scol) : zero4();
-  }
-}
-
-// acc = the wave's 32 x 32 block of X . W over K = C.  X: the pieces fetched by fetch_rows, or (FROM_TILE) the fp32 tile in
-// LDS; W: the pieces fetched by fetch_weights from the transposed block [C out, C in].  All threads of the workgroup
-// take part; on return the operand planes may still be read by slower waves: whatever overwrites them next sits behind
-// a barrier.
-template <class S, bool FROM_TILE>
-__device__ __forceinline__ void product(S &s, const RowPieces<S> *rows, const WeightPieces<S> &w, v16f &acc) {
-  constexpr int C = S::C, ROWS = S::kRows;
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave, wave = tid / kWave;
-  const int wr = wave % S::kRowWaves, wc = wave / S::kRowWaves;
-  const int mrow = lane % 32, half = lane / 32;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-#pragma unroll
-  for (int k = 0; k < C / kGlKC; ++k) {
-    __syncthreads();  // previous chunk fully consumed (and, before the first, the tile complete)
-#pragma unroll
-    for (int i = 0; i < S::kAPieces; ++i) {
-      const int piece = tid + i * S::kThreads;
-      const int row = piece / kGlTPR, scol = (piece % kGlTPR) * 4;
-      if (S::kAPieces * S::kThreads != ROWS * kGlTPR && row >= ROWS) continue;
-      f4 x;
-      if constexpr (FROM_TILE)
-        x = *reinterpret_cast<const f4 *>(s.tile + row * S::kLdT + kGlKC * k + scol);
-      else
-        x = rows->v[k][i];
-      bf16x4 h, md, lw;
-      split3(x, h, md, lw);
-      const int at = row * kGlLdH + scol;
-      *reinterpret_cast<bf16x4 *>(s.a + at) = h;
-      *reinterpret_cast<bf16x4 *>(s.a + ROWS * kGlLdH + at) = md;
-      *reinterpret_cast<bf16x4 *>(s.a + 2 * ROWS * kGlLdH + at) = lw;
-    }
-#pragma unroll
-    for (int i = 0; i < S::kBPieces; ++i) {
-      const int piece = tid + i * S::kThreads;
-      bf16x4 h, md, lw;
-      split3(w.v[k][i], h, md, lw);
-      const int at = (piece / kGlTPR) * kGlLdH + (piece % kGlTPR) * 4;
-      *reinterpret_cast<bf16x4 *>(s.b + at) = h;
-      *reinterpret_cast<bf16x4 *>(s.b + C * kGlLdH + at) = md;
-      *reinterpret_cast<bf16x4 *>(s.b + 2 * C * kGlLdH + at) = lw;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < kGlKC; ks += 16) {
-      bf16x8 a[3], b[3];
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        a[p] = *reinterpret_cast<const bf16x8 *>(s.a + p * ROWS * kGlLdH + (32 * wr + mrow) * kGlLdH + ks + 8 * half);
-        b[p] = *reinterpret_cast<const bf16x8 *>(s.b + p * C * kGlLdH + (32 * wc + mrow) * kGlLdH + ks + 8 * half);
-      }
-      // piece products from small to large, as in the linear kernels
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
-    }
-  }
-}
-
-// Accumulator r of a lane is row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32 of the wave's block.
-template <class S, class F>
-__device__ __forceinline__ void for_each_output(const v16f &acc, F f) {
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int mrow = lane % 32, half = lane / 32;
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-    f(32 * (wave % S::kRowWaves) + 8 * (r / 4) + 4 * half + (r % 4), 32 * (wave / S::kRowWaves) + mrow, acc[r]);
-}
-
-template <class S>
-__device__ __forceinline__ void stage_nodes(S &s, const int32_t *__restrict__ node_perm, int pos0, int gend, int nnodes) {
-  const int tid = threadIdx.x;
-  if (tid < S::kRows) {
-    int node = -1;
-    if (tid < min(S::kRows, gend - pos0)) {
-      node = node_perm ? node_perm[pos0 + tid] : pos0 + tid;
-      if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) node = -1;
-    }
-    s.node[tid] = node;
-  }
-  __syncthreads();
-}
 
 // ---- forward: h1 = B1 . Wprod, sc = skip_scale h1 . Wskip[element], X2 = h1 . Wup ---------------------------------
-template <int NT, int ROWS>
-__global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_glue_forward_kernel(
+template <int NT, int WAVES>
+__global__ __launch_bounds__(WAVES *kWave) void node_glue_forward_kernel(
     const float *__restrict__ B1, const float *__restrict__ prod_WT, const float *__restrict__ skip_WT,
     const float *__restrict__ up_WT, const int32_t *__restrict__ node_perm, const int32_t *__restrict__ group_offsets, int nnodes,
     int ngroups, float skip_scale, float *__restrict__ h1, float *__restrict__ sc, float *__restrict__ X2) {
-  constexpr int C = 32 * NT;
-  using S = GlueShared<NT, ROWS>;
-  __shared__ __attribute__((aligned(16))) S s;
+  using S = Chain<NT, WAVES>;
+  constexpr int C = S::C;
+  __shared__ __attribute__((aligned(16))) typename S::Planes planes[S::kSlots];
+  typename S::Weights w_prod, w_up, w_skip;
+  w_prod.request(prod_WT);
   int g, pos0, gend;
-  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x, ROWS, g, pos0, gend)) return;
-  stage_nodes(s, node_perm, pos0, gend, nnodes);
-
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x, S::kRows, g, pos0, gend)) return;
+  const int pos = pos0 + threadIdx.x / kWave * 16 + threadIdx.x % 16;
+  const int node = node_perm[pos < gend ? pos : pos0];
+  const bool here = pos < gend && static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t at = static_cast<int64_t>(here ? node : 0) * C;
   const bool no_element = g == ngroups - 1;  // nodes of no element: the skip connection is defined as zero there
-  WeightPieces<S> wa, wb;
-  RowPieces<S> a0;
-  fetch_weights<S>(prod_WT, wa);
-  fetch_rows(s, B1, a0);
-  if (!no_element) fetch_weights<S>(skip_WT + static_cast<int64_t>(g) * C * C, wb);  // in flight during the first product
-
-  v16f acc;
-  product<S, false>(s, &a0, wa, acc);
-  fetch_weights<S>(up_WT, wa);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    const float out = v * 1.0f;
-    s.tile[row * S::kLdT + col] = out;
-    const int node = s.node[row];
-    if (node >= 0) h1[static_cast<int64_t>(node) * C + col] = out;
-  });
-  // (the tile is complete behind the barrier at the top of the next product)
+  f4 v[S::NB], h[S::NB];
+  rows::load(B1 + at, v);
+  w_up.request(up_WT);
+  if (!no_element) w_skip.request(skip_WT + static_cast<int64_t>(g) * C * C);
+  __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
+  w_prod.store(planes[0], 1.0f);
+  w_up.store(planes[1], 1.0f);
+  if (S::kSlots == 3 && !no_element) w_skip.store(planes[S::kSlots - 1], skip_scale);
+  __syncthreads();
+  rows::product_all(planes[0], typename S::Operand(v), h);
+  if (here) rows::store(h1 + at, h);
+  const typename S::Operand operand(h);
+  rows::product_all(planes[1], operand, v);
+  if (here) rows::store(X2 + at, v);
   if (no_element) {
-    for_each_output<S>(acc, [&](int row, int col, float) {
-      const int node = s.node[row];
-      if (node >= 0) sc[static_cast<int64_t>(node) * C + col] = 0.f;
-    });
+#pragma unroll
+    for (int i = 0; i < S::NB; ++i) v[i] = zero4();
   } else {
-    product<S, true>(s, nullptr, wb, acc);
-    for_each_output<S>(acc, [&](int row, int col, float v) {
-      const int node = s.node[row];
-      if (node >= 0) sc[static_cast<int64_t>(node) * C + col] = v * skip_scale;
-    });
+    if constexpr (S::kSlots == 2) {
+      __syncthreads();  // every wave is done with the first planes
+      w_skip.store(planes[0], skip_scale);
+      __syncthreads();
+    }
+    rows::product_all(planes[S::kSlots == 3 ? 2 : 0], operand, v);
   }
-  product<S, true>(s, nullptr, wa, acc);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    const int node = s.node[row];
-    if (node >= 0) X2[static_cast<int64_t>(node) * C + col] = v * 1.0f;
-  });
+  if (here) rows::store(sc + at, v);
 }
 
 // ---- few nodes (few::applies): tiles of 16, one wave per 16 output columns, products of mfma_f32.hpp ------------------
@@ -339,67 +203,66 @@ __device__ __forceinline__ void graph_energy(const EnergySums &q, int graph, dou
 }
 
 // ---- backward: gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip[element]^T, gB1 = gh1 . Wprod^T ------------------
-template <int NT, int ROWS>
-__global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_glue_backward_kernel(
+// gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip^T of four columns of a node from the two products (factor: what takes the
+// second one to -skip_scale dE/dh2 . Wskip^T)
+__device__ __forceinline__ f4 gh1_of(f4 up, f4 skip, const double *w1, double scale, double node_weight, float factor, bool no_element) {
+  const f4 g1{static_cast<float>(-1.0 * scale * w1[0] * node_weight), static_cast<float>(-1.0 * scale * w1[1] * node_weight),
+              static_cast<float>(-1.0 * scale * w1[2] * node_weight), static_cast<float>(-1.0 * scale * w1[3] * node_weight)};
+  const f4 sum = up + g1;
+  return no_element ? sum : sum + skip * factor;
+}
+
+template <int NT, int WAVES>
+__global__ __launch_bounds__(WAVES *kWave) void node_glue_backward_kernel(
     const float *__restrict__ gX2, const float *__restrict__ d_h2, const float *__restrict__ up_W, const float *__restrict__ skip_W,
     const float *__restrict__ prod_W, const double *__restrict__ w1, double scale, const double *__restrict__ node_weights,
     const int32_t *__restrict__ node_perm, const int32_t *__restrict__ group_offsets, int nnodes, int ngroups, float skip_scale,
     float *__restrict__ gB1, EnergySums sums, int first_tile) {
-  constexpr int C = 32 * NT;
-  using S = GlueShared<NT, ROWS>;
-  __shared__ __attribute__((aligned(16))) S s;
+  using S = Chain<NT, WAVES>;
+  constexpr int C = S::C;
+  __shared__ __attribute__((aligned(16))) typename S::Planes planes[S::kSlots];
   if (static_cast<int>(blockIdx.x) < first_tile) {
     // workgroups ahead of the tiles: the energy of one graph each, from node energies an earlier launch wrote
-    constexpr int kSum = S::kThreads >= 1024 ? 1024 : (S::kThreads >= 512 ? 512 : (S::kThreads >= 256 ? 256 : (S::kThreads >= 128 ? 128 : 64)));
-    static_assert(sizeof(s.tile) >= kSum * sizeof(double), "the tile holds the partial sums");
-    graph_energy<kSum>(sums, blockIdx.x, reinterpret_cast<double *>(s.tile));
+    static_assert(sizeof(planes) >= S::kThreads * sizeof(double), "the planes' place holds the partial sums");
+    graph_energy<S::kThreads>(sums, blockIdx.x, reinterpret_cast<double *>(planes));
     return;
   }
+  typename S::Weights w_up, w_skip, w_prod;
+  w_up.request(up_W);
   int g, pos0, gend;
-  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x - first_tile, ROWS, g, pos0, gend)) return;
-  stage_nodes(s, node_perm, pos0, gend, nnodes);
-
+  if (!locate_group_tile(group_offsets, ngroups, nnodes, blockIdx.x - first_tile, S::kRows, g, pos0, gend)) return;
+  const int pos = pos0 + threadIdx.x / kWave * 16 + threadIdx.x % 16;
+  const int node = node_perm[pos < gend ? pos : pos0];
+  const bool here = pos < gend && static_cast<unsigned>(node) < static_cast<unsigned>(nnodes);
+  const int64_t in = here ? node : 0, at = in * C;
   const bool no_element = g == ngroups - 1;
-  WeightPieces<S> wa, wb;
-  RowPieces<S> a0, a1;
-  fetch_weights<S>(up_W, wa);
-  fetch_rows(s, gX2, a0);
-  if (!no_element) {  // in flight during the first product
-    fetch_weights<S>(skip_W + static_cast<int64_t>(g) * C * C, wb);
-    fetch_rows(s, d_h2, a1);
-  }
-
-  v16f acc;
-  product<S, false>(s, &a0, wa, acc);
-  fetch_weights<S>(prod_W, wa);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    const int node = s.node[row];
-    const double nw = (node_weights && node >= 0) ? node_weights[node] : 1.0;
-    const float g1 = static_cast<float>(-1.0 * scale * w1[col] * nw);
-    const float part = v * 1.0f;
-    s.tile[row * S::kLdT + col] = part + g1;
-  });
+  f4 v[S::NB], d[S::NB], up[S::NB], skip[S::NB];
+  rows::load(gX2 + at, v);
+  if (!no_element) w_skip.request(skip_W + static_cast<int64_t>(g) * C * C);
+  rows::load(d_h2 + at, d);
+  w_prod.request(prod_W);
+  const double nw = node_weights ? node_weights[in] : 1.0;
+  __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
+  w_up.store(planes[0], 1.0f);
+  if (!no_element) w_skip.store(planes[1], -skip_scale);
+  if constexpr (S::kSlots == 3) w_prod.store(planes[S::kSlots - 1], 1.0f);
+  __syncthreads();
+  rows::product_all(planes[0], typename S::Operand(v), up);
   if (!no_element) {
-    product<S, false>(s, &a1, wb, acc);
-    // each element of the tile is read and written by the lane that wrote it above
-    for_each_output<S>(acc, [&](int row, int col, float v) {
-      const float part = v * -skip_scale;
-      s.tile[row * S::kLdT + col] += part;
-    });
+    rows::product_all(planes[1], typename S::Operand(d), skip);
+  } else {
+#pragma unroll
+    for (int i = 0; i < S::NB; ++i) skip[i] = zero4();
   }
-  product<S, true>(s, nullptr, wa, acc);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    const int node = s.node[row];
-    if (node >= 0) gB1[static_cast<int64_t>(node) * C + col] = v * 1.0f;
-  });
-}
-
-// gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip^T of four columns of a node from the two products
-__device__ __forceinline__ f4 few_gh1(f4 up, f4 skip, const double *w1, double scale, double node_weight, float skip_scale, bool no_element) {
-  const f4 g1{static_cast<float>(-1.0 * scale * w1[0] * node_weight), static_cast<float>(-1.0 * scale * w1[1] * node_weight),
-              static_cast<float>(-1.0 * scale * w1[2] * node_weight), static_cast<float>(-1.0 * scale * w1[3] * node_weight)};
-  const f4 sum = up + g1;
-  return no_element ? sum : sum + skip * -skip_scale;
+#pragma unroll
+  for (int i = 0; i < S::NB; ++i) v[i] = gh1_of(up[i], skip[i], w1 + 16 * i + 4 * (threadIdx.x % kWave / 16), scale, nw, 1.0f, no_element);
+  if constexpr (S::kSlots == 2) {
+    __syncthreads();  // every wave is done with the first planes
+    w_prod.store(planes[0], 1.0f);
+    __syncthreads();
+  }
+  rows::product_all(planes[S::kSlots == 3 ? 2 : 0], typename S::Operand(v), d);
+  if (here) rows::store(gB1 + at, d);
 }
 
 template <int NT>
@@ -435,7 +298,7 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_glue_backward_few_kernel(
   f4 v[1], u[1];
   few::product<KQ, 1>(x, wu, v);
   few::product<KQ, 1>(d, ws, u);
-  put(s, few_gh1(v[0], u[0], w1 + col0 + 4 * part, scale, nw, skip_scale, no_element));
+  put(s, gh1_of(v[0], u[0], w1 + col0 + 4 * part, scale, nw, -skip_scale, no_element));
   __syncthreads();
   few::product<KQ, 1>(get(s), wp, v);
   if (here) st4(gB1 + in * C + col0 + 4 * part, v[0]);
@@ -500,41 +363,41 @@ __global__ __launch_bounds__(4 * kWave) void node_glue_gh1_kernel(const float *_
   few::product<KQ, 1>(few::load_rows<KQ>(gX2 + in * C + 4 * part), wu, v);
   few::product<KQ, 1>(few::load_rows<KQ>(d_h2 + in * C + 4 * part), ws, u);
   if (!here) return;
-  st4(gh1 + in * C + col0 + 4 * part, few_gh1(v[0], u[0], w1 + col0 + 4 * part, scale, node_weights ? node_weights[in] : 1.0, skip_scale, no_element));
+  st4(gh1 + in * C + col0 + 4 * part, gh1_of(v[0], u[0], w1 + col0 + 4 * part, scale, node_weights ? node_weights[in] : 1.0, -skip_scale, no_element));
 }
 
 // ---- head: h2 = B2 . Wprod + sc, readouts of h1 and h2, gB2 = -w dE/dh2 . Wprod^T (w: the node's weight) --------------
 // Between the second layer's contraction and the backward chain every step is per node: a product with a residual, the
-// readouts (readout.hip has their arithmetic and the meaning of the operands), and the product of their derivative.  h2 stays
-// in LDS: of the [N, C] rows only dE/dh2 is written besides gB2, for the skip connection's gradient.  The readouts are
+// readouts (readout.hip has their arithmetic and the meaning of the operands), and the product of their derivative.  h2 stays on
+// chip: of the [N, C] rows only dE/dh2 is written besides gB2, for the skip connection's gradient.  The readouts are
 // bound by nothing but the fp64 matrix rate and the chain of a tile, 0.9 us each way at 128 x 128 on four matrix pipes.
 // Measured inside the step, three launches -> one (us): 21 x 64 9.0 -> 5.2, 216 x 128 14.8 -> 12.4, 2 000 x 128 15.4 -> 12.5 (tiles
-// of 16 nodes), 5 000 x 96 24.0 -> 15.6, 10 752 x 64 23.9 -> 13.5 (tiles of 32), 25 000 x 128 66.6 -> 40 (128; with tiles of 64, two
-// rounds of workgroups by their registers, 48; its 112 MB, half of them the fp64 feature rows, take 21).
+// of 16 nodes), 5 000 x 96 24.0 -> 15.6, 10 752 x 64 23.9 -> 13.5, 25 000 x 128 66.6 -> 40 (its 112 MB, half of them the fp64 feature
+// rows, take 21); with the rows of 16 nodes in a wave's registers, as in the chains above, 5 000 x 96 16.1 -> 14.6, 10 752 x 64 14.3 -> 11.2,
+// 25 000 x 128 41.6 -> 36.6.
 // Without d_h2 (energies alone) the kernel ends with the energies.  Bits of the separate launches, as above.
-// A wave takes tiles of 16 nodes, all classes of pieces of each (in the separate kernel four waves share the classes of a
-// tile; where there are two waves per tile they share them); the weights of the readouts wait in LDS.
-template <int NT, int ROWS>
-__global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_head_kernel(
+// A wave has all classes of pieces of its 16 nodes (in the separate kernel four waves share them); the weights of the readouts
+// wait in LDS.
+template <int NT, int WAVES>
+__global__ __launch_bounds__(WAVES *kWave) void node_head_kernel(
     const float *__restrict__ B2, const float *__restrict__ sc, const float *__restrict__ h1, const float *__restrict__ prod_WT,
     const float *__restrict__ prod_W, readout::Weights w, readout::Outputs out, const double *__restrict__ node_weights, int nnodes,
     float *__restrict__ d_h2, float *__restrict__ gB2) {
-  constexpr int C = 32 * NT, kPieces = C / 16, kHidden = readout::kHidden;
-  using S = GlueShared<NT, ROWS>;
-  constexpr int kWaves = S::kThreads / kWave, kTiles = ROWS / 16;
+  using S = Chain<NT, WAVES>;
+  constexpr int C = S::C, kHidden = readout::kHidden, kClasses = readout::kClasses;
   constexpr int kLdW = kHidden + 2;  // row stride of W2a in LDS (doubles): the four lane groups of a read start 64 bytes apart in bank space
-  __shared__ __attribute__((aligned(16))) S s;
+  __shared__ __attribute__((aligned(16))) typename S::Planes planes[2];
   __shared__ __attribute__((aligned(16))) double sW[C * kLdW], sw1[C];
-  const int tid = threadIdx.x;
-  const int node0 = blockIdx.x * ROWS, nrows = min(ROWS, nnodes - node0);  // consecutive nodes
-  sc += static_cast<int64_t>(node0) * C, h1 += static_cast<int64_t>(node0) * C;
-  if (d_h2) d_h2 += static_cast<int64_t>(node0) * C, gB2 += static_cast<int64_t>(node0) * C;
-  stage_nodes(s, nullptr, node0, nnodes, nnodes);
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int col = lane % 16, part = lane / 16;
+  const int node = blockIdx.x * S::kRows + tid / kWave * 16 + col;
+  const bool here = node < nnodes;
+  const int64_t at = static_cast<int64_t>(here ? node : 0) * C;
 
-  WeightPieces<S> wa;
-  RowPieces<S> a0;
-  fetch_weights<S>(prod_WT, wa);
-  fetch_rows(s, B2, a0);
+  typename S::Weights w_prod, w_back;
+  w_prod.request(prod_WT);
+  f4 x[S::NB], h2[S::NB], a[S::NB];
+  rows::load(B2 + at, x);
   constexpr int kWPer = (C * kHidden + S::kThreads - 1) / S::kThreads;
   double w2a[kWPer];
 #pragma unroll
@@ -543,125 +406,68 @@ __global__ __launch_bounds__(ROWS / 32 * NT *kWave) void node_head_kernel(
     w2a[i] = c < C && j < w.hidden ? w.W2a[c * w.hidden + j] : 0.0;
   }
   const double w1v = tid < C ? w.w1[tid] : 0.0;
-  // the residual rows go to the tile, as the readouts' weights go to LDS: during the product no registers are left for them
-  constexpr int kTilePer = ROWS * C / 4 / S::kThreads;
-  static_assert(kTilePer * S::kThreads == ROWS * C / 4, "the tile's pieces divide evenly among the threads");
-  f4 res[kTilePer];
-#pragma unroll
-  for (int i = 0; i < kTilePer; ++i) {
-    const int q = tid + i * S::kThreads;
-    res[i] = ld4(sc + min(4 * q / C, nrows - 1) * C + 4 * q % C);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < kTilePer; ++i) {
-    const int q = tid + i * S::kThreads;
-    *reinterpret_cast<f4 *>(s.tile + 4 * q / C * S::kLdT + 4 * q % C) = res[i];
-  }
+  const int row = here && out.rows ? out.rows[node] : node;
+  const bool row_ok = here && static_cast<unsigned>(row) < static_cast<unsigned>(nnodes);
+  if (d_h2) w_back.request(prod_W);
+  __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
+  w_prod.store(planes[0], 1.0f);
 #pragma unroll
   for (int i = 0; i < kWPer; ++i) {
     const int q = tid + i * S::kThreads;
     if (q < C * kHidden) sW[q / kHidden * kLdW + q % kHidden] = w2a[i];
   }
   if (tid < C) sw1[tid] = w1v;
-
-  v16f acc;
-  product<S, false>(s, &a0, wa, acc);
-  if (d_h2) fetch_weights<S>(prod_W, wa);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    float &h2 = s.tile[row * S::kLdT + col];
-    h2 = v * 1.0f + h2;
-  });
+  static_assert(S::kThreads >= C, "a thread per channel");
+  if (d_h2) w_back.store(planes[1], -1.0f);
+  rows::load(sc + at, a);  // the residual
+  const typename S::Operand operand(x);
   __syncthreads();
+  rows::product_all(planes[0], operand, h2);
+#pragma unroll
+  for (int p = 0; p < S::NB; ++p) h2[p] = h2[p] + a[p];
+  rows::load(h1 + at, a);
 
-  // a wave has half of the classes, of the hidden units and of the pieces of its tile where there are two per tile
-  constexpr int kShare = kWaves >= 2 * kTiles ? 2 : 1, kMine = readout::kClasses / kShare;
-  static_assert(kShare == 1 || kWaves == kShare * kTiles, "every wave has a tile: they all meet at the barriers");
-  static_assert(kShare == 1 || sizeof(s.a) >= kWaves * kWave * 3 * sizeof(double), "two values per lane and an energy to exchange");
-  double(*swap)[3][kWave] = reinterpret_cast<double(*)[3][kWave]>(s.a);
-  const int lane = tid % kWave, col = lane % 16, part = lane / 16;
-  const int half = tid / kWave % kShare, other = tid / kWave ^ (kShare - 1);
-  for (int t = tid / kWave / kShare; t < kTiles; t += kWaves / kShare) {
-    float *mine = s.tile + (16 * t + col) * S::kLdT + 4 * part;  // the lane's node of the tile, its channels of piece 0
-    const bool here = 16 * t + col < nrows;
-    const int node = node0 + 16 * t + col;
-    const int row = here && out.rows ? out.rows[node] : node;
-    const bool row_ok = here && static_cast<unsigned>(row) < static_cast<unsigned>(nnodes);
-    const int at = (here ? 16 * t + col : 0) * C + 4 * part;
-    // classes kMine half .. : piece u of the wave is class kMine half + u % kMine
-    constexpr int kOwn = kPieces / kShare;
-    static_assert(kShare == 1 || kPieces % readout::kClasses == 0, "the halves have the same number of pieces");
-    auto piece = [&](int u) { return readout::kClasses * (u / kMine) + kMine * half + u % kMine; };
-    readout::d4v z[kMine];
-    double e1[kMine];
+  readout::d4v z[kClasses];
+  double e1[kClasses];
 #pragma unroll
-    for (int k = 0; k < kMine; ++k) z[k] = readout::d4v{0.0, 0.0, 0.0, 0.0}, e1[k] = 0.0;
-    f4 a[kOwn];
+  for (int k = 0; k < kClasses; ++k) z[k] = readout::d4v{0.0, 0.0, 0.0, 0.0}, e1[k] = 0.0;
 #pragma unroll
-    for (int u = 0; u < kOwn; ++u) a[u] = ld4(h1 + at + 16 * piece(u));
+  for (int p = 0; p < S::NB; ++p) {
+    const int c = 16 * p + 4 * part;
+    double wz[4];
 #pragma unroll
-    for (int u = 0; u < kOwn; ++u) {
-      const f4 b = *reinterpret_cast<const f4 *>(mine + 16 * piece(u));
-      const int c = 16 * piece(u) + 4 * part;
-      double wz[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) wz[i] = sW[(c + i) * kLdW + readout::operand_row(col)];
-      readout::add_z(z[u % kMine], wz, b);
-      readout::add_linear(e1[u % kMine], *reinterpret_cast<const readout::d2v *>(sw1 + c), *reinterpret_cast<const readout::d2v *>(sw1 + c + 2), a[u]);
-      if (out.feats64 && row_ok) readout::store_feats(out.feats64 + static_cast<int64_t>(row) * (2 * C) + c, C, a[u], b);
-    }
-    // sums in pairs, (0 + 1) + (2 + 3), of classes and of hidden units, whoever has them
-    readout::d4v zsum = z[0] + z[1];
-    double esum = e1[0] + e1[1], e2[4], d[4];
-    auto gate = [&](int i) { return 4 * part + i < w.hidden ? w.w2b[4 * part + i] * w.act_cst : 0.0; };
-    if constexpr (kShare == 1) {
-      zsum = zsum + (z[2] + z[3]);
-      esum = esum + (e1[2] + e1[3]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) readout::activate(gate(i), zsum[i], e2[i], d[i]);
-      esum = esum + ((e2[0] + e2[1]) + (e2[2] + e2[3]));
-    } else {
-      // unit 2 half + j of the lane's four: from the other wave its share of z, to it (in the second exchange) the derivative
-      double(&out1)[3][kWave] = swap[tid / kWave], (&in1)[3][kWave] = swap[other];
-      out1[0][lane] = half == 0 ? zsum[2] : zsum[0];
-      out1[1][lane] = half == 0 ? zsum[3] : zsum[1];
-      out1[2][lane] = esum;
-      __syncthreads();
-      const double z0 = (half == 0 ? zsum[0] : zsum[2]) + in1[0][lane], z1 = (half == 0 ? zsum[1] : zsum[3]) + in1[1][lane];
-      esum = esum + in1[2][lane];
-      double d0, d1;
-      readout::activate(gate(2 * half), z0, e2[0], d0);
-      readout::activate(gate(2 * half + 1), z1, e2[1], d1);
-      __syncthreads();
-      out1[0][lane] = d0, out1[1][lane] = d1, out1[2][lane] = e2[0] + e2[1];
-      __syncthreads();
-      esum = esum + ((e2[0] + e2[1]) + in1[2][lane]);
-      const double d2 = in1[0][lane], d3 = in1[1][lane];
-      d[0] = half == 0 ? d0 : d2, d[1] = half == 0 ? d1 : d3, d[2] = half == 0 ? d2 : d0, d[3] = half == 0 ? d3 : d1;
-    }
-    const double en = readout::node_energy(esum, w.scale, w.shift);
-    if (here && part == 0 && half == 0) readout::store_energy(out, node, row, row_ok, en);
-    if (!d_h2) continue;
-#pragma unroll 2
-    for (int u = 0; u < kOwn; ++u) {
-      const int p = piece(u);
-      const double *wp = sW + (16 * p + readout::operand_row(col)) * kLdW + 4 * part;
-      const double wd[4] = {wp[0], wp[1], wp[2], wp[3]};
-      f4 g = readout::derivative(wd, d, w.scale);
-      if (node_weights) {
-        const double nw = here ? node_weights[node] : 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g[i] = static_cast<float>(static_cast<double>(g[i]) * nw);
-      }
-      if (here) st4(d_h2 + at + 16 * p, g);
-      *reinterpret_cast<f4 *>(mine + 16 * p) = g;  // read above by the lane itself
-    }
+    for (int i = 0; i < 4; ++i) wz[i] = sW[(c + i) * kLdW + readout::operand_row(col)];
+    readout::add_z(z[p % kClasses], wz, h2[p]);
+    readout::add_linear(e1[p % kClasses], *reinterpret_cast<const readout::d2v *>(sw1 + c), *reinterpret_cast<const readout::d2v *>(sw1 + c + 2), a[p]);
+    if (out.feats64 && row_ok) readout::store_feats(out.feats64 + static_cast<int64_t>(row) * (2 * C) + c, C, a[p], h2[p]);
   }
+  // sums in pairs, (0 + 1) + (2 + 3), of classes and of hidden units
+  const readout::d4v zsum = (z[0] + z[1]) + (z[2] + z[3]);
+  double esum = (e1[0] + e1[1]) + (e1[2] + e1[3]), e2[4], d[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const double gate = 4 * part + i < w.hidden ? w.w2b[4 * part + i] * w.act_cst : 0.0;
+    readout::activate(gate, zsum[i], e2[i], d[i]);
+  }
+  esum = esum + ((e2[0] + e2[1]) + (e2[2] + e2[3]));
+  const double en = readout::node_energy(esum, w.scale, w.shift);
+  if (here && part == 0) readout::store_energy(out, node, row, row_ok, en);
   if (!d_h2) return;
-  product<S, true>(s, nullptr, wa, acc);
-  for_each_output<S>(acc, [&](int row, int col, float v) {
-    if (row < nrows) gB2[row * C + col] = v * -1.0f;
-  });
+  const double nw = node_weights && here ? node_weights[node] : 1.0;
+#pragma unroll
+  for (int p = 0; p < S::NB; ++p) {
+    const double *wp = sW + (16 * p + readout::operand_row(col)) * kLdW + 4 * part;
+    const double wd[4] = {wp[0], wp[1], wp[2], wp[3]};
+    f4 g = readout::derivative(wd, d, w.scale);
+    if (node_weights) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) g[i] = static_cast<float>(static_cast<double>(g[i]) * nw);
+    }
+    x[p] = g;
+  }
+  if (here) rows::store(d_h2 + at, x);
+  rows::product_all(planes[1], typename S::Operand(x), h2);
+  if (here) rows::store(gB2 + at, h2);
 }
 
 // Few nodes: tiles of 16, a wave per 16 columns, the readouts' sums shared by the waves as in the separate kernel.
@@ -769,8 +575,10 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_head_few_kernel(
   if (here) st4(gB2 + at, v[0] * -1.0f);
 }
 
-// 128-node tiles where they give at least half of the compute units one each, 32-node tiles below that
-inline bool small_tiles(int64_t nnodes) { return ceil_div(nnodes, kGlTile) * 2 < device_compute_units(); }
+// Four waves per workgroup (64 nodes) while that is one round of workgroups, eight beyond.  us, four / eight waves, forward and backward:
+// 5 000 x 128 14.1 + 14.3 / 17.0 + 17.7, 10 752 x 64 6.9 + 6.8 / 8.4 + 8.4, 14 000 x 96 12.1 + 11.5 / 13.5 + 12.6; 25 000 x 96 20.5 + 21.2 /
+// 14.7 + 13.9, 25 000 x 128 28.9 + 29.1 / 20.7 + 20.9.
+inline bool four_waves(int64_t nnodes) { return ceil_div(nnodes, 128) * 2 < device_compute_units(); }
 
 template <int NT>
 int launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm,
@@ -790,15 +598,14 @@ int launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, 
     }
     return check_launch("cm_node_glue_forward");
   }
-  if (small_tiles(nnodes)) {
-    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
-    hipLaunchKernelGGL((node_glue_forward_kernel<NT, kGlSmallTile>), dim3(tiles), dim3(NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT,
-                       perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
-    return check_launch("cm_node_glue_forward");
-  }
-  const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlTile) + ngroups);
-  hipLaunchKernelGGL((node_glue_forward_kernel<NT, kGlTile>), dim3(tiles), dim3(4 * NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm,
-                     offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
+  const auto launch = [&](auto waves) {
+    constexpr int kW = decltype(waves)::value;
+    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, 16 * kW) + ngroups);
+    hipLaunchKernelGGL((node_glue_forward_kernel<NT, kW>), dim3(tiles), dim3(kW * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm, offs,
+                       static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
+  };
+  if (four_waves(nnodes)) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
   return check_launch("cm_node_glue_forward");
 }
 
@@ -823,17 +630,14 @@ int launch_backward(const float *gX2, const float *d_h2, const float *up_W, cons
                        static_cast<int>(extra));
     return check_launch("cm_node_glue_backward");
   }
-  if (small_tiles(nnodes)) {
-    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile) + ngroups);
-    hipLaunchKernelGGL((node_glue_backward_kernel<NT, kGlSmallTile>), dim3(tiles + extra), dim3(NT * kWave), 0, st, gX2, d_h2, up_W,
-                       skip_W, prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
-                       static_cast<int>(extra));
-    return check_launch("cm_node_glue_backward");
-  }
-  const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, kGlTile) + ngroups);
-  hipLaunchKernelGGL((node_glue_backward_kernel<NT, kGlTile>), dim3(tiles + extra), dim3(4 * NT * kWave), 0, st, gX2, d_h2, up_W, skip_W,
-                     prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
-                     static_cast<int>(extra));
+  const auto launch = [&](auto waves) {
+    constexpr int kW = decltype(waves)::value;
+    const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, 16 * kW) + ngroups);
+    hipLaunchKernelGGL((node_glue_backward_kernel<NT, kW>), dim3(tiles + extra), dim3(kW * kWave), 0, st, gX2, d_h2, up_W, skip_W, prod_W, w1, scale,
+                       node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums, static_cast<int>(extra));
+  };
+  if (four_waves(nnodes)) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
   return check_launch("cm_node_glue_backward");
 }
 
@@ -844,12 +648,12 @@ int launch_head(const float *B2, const float *sc, const float *h1, const float *
   if (few::applies(nnodes, 1, 32 * NT))
     hipLaunchKernelGGL((node_head_few_kernel<NT>), dim3(static_cast<unsigned>(ceil_div(nnodes, few::kRows))), dim3(2 * NT * kWave), 0, st, B2, sc, h1,
                        prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
-  else if (small_tiles(nnodes))
-    hipLaunchKernelGGL((node_head_kernel<NT, kGlSmallTile>), dim3(static_cast<unsigned>(ceil_div(nnodes, kGlSmallTile))), dim3(NT * kWave), 0, st, B2,
-                       sc, h1, prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
+  else if (four_waves(nnodes))
+    hipLaunchKernelGGL((node_head_kernel<NT, 4>), dim3(static_cast<unsigned>(ceil_div(nnodes, 64))), dim3(4 * kWave), 0, st, B2, sc, h1, prod_WT,
+                       prod_W, w, out, node_weights, n, d_h2, gB2);
   else
-    hipLaunchKernelGGL((node_head_kernel<NT, kGlTile>), dim3(static_cast<unsigned>(ceil_div(nnodes, kGlTile))), dim3(4 * NT * kWave), 0, st, B2, sc,
-                       h1, prod_WT, prod_W, w, out, node_weights, n, d_h2, gB2);
+    hipLaunchKernelGGL((node_head_kernel<NT, 8>), dim3(static_cast<unsigned>(ceil_div(nnodes, 128))), dim3(8 * kWave), 0, st, B2, sc, h1, prod_WT,
+                       prod_W, w, out, node_weights, n, d_h2, gB2);
   return check_launch("cm_mace_step");
 }
 

@@ -534,16 +534,16 @@ def test_linear_many_rows_wide(cabi, N, C, ne, seed):
     test_linear_many_rows(cabi, N, C, ne, seed)
 
 
-@pytest.mark.parametrize("N,C,ne,seed", [(12_500, 128, 4, 0), (12_501, 128, 10, 1), (25_001, 64, 3, 2), (16_667, 96, 1, 3), (5000, 64, 100, 4), (9, 224, 3, 5),
+@pytest.mark.parametrize("N,C,ne,seed", [(8000, 128, 4, 0), (8100, 128, 10, 1), (8192, 64, 3, 2), (8193, 96, 1, 3), (6000, 64, 100, 4), (9, 224, 3, 5), (300, 32, 3, 12),
                                          (130, 256, 63, 6), (129, 160, 64, 7), (1025, 192, 3, 8), (2047, 224, 2, 9), (4100, 160, 10, 10), (700, 128, 3, 11)])
 def test_linear_rows_of_a_weight_block(cabi, N, C, ne, seed):
-    """Both sides of the lines of the kernel with a workgroup per 128 rows: features that fit the last-level cache and those that do not
-    (the weights resident, 16-row tiles), 64 weight groups and more, one and two rounds of workgroups at 160 to 256 columns, half and all
-    columns per workgroup."""
+    """Both sides of the lines of the kernel with a workgroup per 128 rows: four workgroups per compute unit and more (the weights
+    resident, 16-row tiles), more than 64 weight groups, one and two rounds of workgroups at 160 to 256 columns, half and all columns per
+    workgroup."""
     test_linear_many_rows(cabi, N, C, ne, seed)
 
 
-@pytest.mark.parametrize("N,C,ne", [(1000, 160, 3), (3001, 192, 10), (9001, 256, 10), (8200, 224, 63), (8193, 160, 64), (33_000, 192, 2)])
+@pytest.mark.parametrize("N,C,ne", [(1000, 160, 3), (3001, 192, 10), (9001, 256, 10), (8200, 224, 63), (8193, 160, 70), (33_000, 192, 2), (5000, 32, 3), (3100, 128, 130)])
 def test_scalar_linear_of_a_weight_block(cabi, N, C, ne):
     """The same for [N, C] features with a weight block per group (rows of no group included) and with one for all, with a residual that is
     the output itself."""
