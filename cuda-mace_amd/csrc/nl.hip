@@ -149,62 +149,67 @@ __device__ __forceinline__ void make_grid(const double *__restrict__ pos, const 
     }
   }
   __syncthreads();
-  if (t == 0) {
-    const int per[3] = {px, py, pz};
+  if (t < kWave) {  // an axis per lane (square roots and divisions one after the other by one thread took 3 us)
     Grid &g = *out;
-    for (int k = 0; k < 9; ++k) {
-      g.inv[k] = inv[k];
-      g.cellv[k] = cell ? cell[k] : 0.0;
-    }
-    g.status = (singular && (px || py || pz)) ? 1 : 0;
-    double width[3];  // distance covered by the binned range of axis k, perpendicular to the other two axes
-    for (int k = 0; k < 3; ++k) {
+    const int k = min(t, 2);
+    const bool mine = t < 3, per = (k == 0 ? px : (k == 1 ? py : pz)) != 0;
+    const double height = 1.0 / sqrt(inv[k] * inv[k] + inv[3 + k] * inv[3 + k] + inv[6 + k] * inv[6 + k]);
+    double width, low = 0.0;  // distance covered by the binned range of the axis, perpendicular to the other two axes
+    if (per) {
+      width = height;
+    } else {
       double a = INFINITY, b = -INFINITY;
       for (int w = 0; w < kGridThreads / kWave; ++w) {
         a = fmin(a, lo[k][w]);
         b = fmax(b, hi[k][w]);
       }
-      const double height = 1.0 / sqrt(inv[k] * inv[k] + inv[3 + k] * inv[3 + k] + inv[6 + k] * inv[6 + k]);
-      g.periodic[k] = per[k] ? 1 : 0;
-      if (per[k]) {
-        g.fmin[k] = 0.0;
-        width[k] = height;
-        const double bins = floor(kBinsPerCutoff * height / (cutoff * kBinSlack));
-        g.nb[k] = bins >= 1.0 ? static_cast<int>(fmin(bins, 1.0e6)) : 1;
-      } else {
-        const double ext = (nnodes > 0 && b > a) ? (b - a) : 0.0;
-        g.fmin[k] = nnodes > 0 ? a : 0.0;
-        width[k] = ext * height;
-        const double bins = floor(kBinsPerCutoff * width[k] / (cutoff * kBinSlack));
-        g.nb[k] = bins >= 1.0 ? static_cast<int>(fmin(bins, 1.0e6)) : 1;
-      }
+      const double ext = (nnodes > 0 && b > a) ? (b - a) : 0.0;
+      low = nnodes > 0 ? a : 0.0;
+      width = ext * height;
+    }
+    const double bins = floor(kBinsPerCutoff * width / (cutoff * kBinSlack));
+    int nb = bins >= 1.0 ? static_cast<int>(fmin(bins, 1.0e6)) : 1;
+    if (t < 9) {
+      g.inv[t] = inv[t];
+      g.cellv[t] = cell ? cell[t] : 0.0;
     }
     // keep the number of bins within what the caller's workspace holds: halve the finest axis until it fits
-    while (static_cast<int64_t>(g.nb[0]) * g.nb[1] * g.nb[2] > max_cells) {
-      int k = 0;
-      if (g.nb[1] > g.nb[k]) k = 1;
-      if (g.nb[2] > g.nb[k]) k = 2;
-      g.nb[k] = (g.nb[k] + 1) / 2;
+    int n0 = __shfl(nb, 0), n1 = __shfl(nb, 1), n2 = __shfl(nb, 2);
+    while (static_cast<int64_t>(n0) * n1 * n2 > max_cells) {
+      int finest = 0;
+      if (n1 > n0) finest = 1;
+      if (n2 > (finest == 1 ? n1 : n0)) finest = 2;
+      if (finest == 0) n0 = (n0 + 1) / 2;
+      else if (finest == 1) n1 = (n1 + 1) / 2;
+      else n2 = (n2 + 1) / 2;
     }
-    for (int k = 0; k < 3; ++k) {
-      if (g.periodic[k]) {
-        g.fscale[k] = g.nb[k];
-        const double binw = width[k] / g.nb[k];
-        g.nscan[k] = static_cast<int>(ceil(cutoff * kBinSlack / binw));
-      } else {
-        const double ext = width[k] > 0.0 ? width[k] : 0.0;
-        // fscale maps (f - fmin) to a bin number; a zero extent puts every atom in bin 0
-        const double height = 1.0 / sqrt(inv[k] * inv[k] + inv[3 + k] * inv[3 + k] + inv[6 + k] * inv[6 + k]);
-        g.fscale[k] = ext > 0.0 ? g.nb[k] * height / ext : 0.0;
-        g.nscan[k] = g.nb[k] > 1 ? static_cast<int>(ceil(cutoff * kBinSlack / (ext / g.nb[k]))) : 0;
-      }
-      if (g.nscan[k] < 0) g.nscan[k] = 0;
-      if (g.nscan[k] > kMaxScan) {  // a cell far thinner than the cutoff: refuse rather than scan thousands of images
-        g.nscan[k] = 0;
-        g.status = 2;
-      }
+    nb = k == 0 ? n0 : (k == 1 ? n1 : n2);
+    double fscale;
+    int nscan;
+    if (per) {
+      fscale = nb;
+      const double binw = width / nb;
+      nscan = static_cast<int>(ceil(cutoff * kBinSlack / binw));
+    } else {
+      // fscale maps (f - fmin) to a bin number; a zero extent puts every atom in bin 0
+      const double ext = width > 0.0 ? width : 0.0;
+      fscale = ext > 0.0 ? nb * height / ext : 0.0;
+      nscan = nb > 1 ? static_cast<int>(ceil(cutoff * kBinSlack / (ext / nb))) : 0;
     }
-    *grid = g;
+    if (nscan < 0) nscan = 0;
+    const bool thin = nscan > kMaxScan;  // a cell far thinner than the cutoff: refuse rather than scan thousands of images
+    if (mine) {
+      g.fmin[k] = low;
+      g.fscale[k] = fscale;
+      g.nb[k] = nb;
+      g.nscan[k] = thin ? 0 : nscan;
+      g.periodic[k] = per ? 1 : 0;
+    }
+    const bool any_thin = __ballot(mine && thin) != 0;
+    if (t == 0) g.status = any_thin ? 2 : ((singular && (px || py || pz)) ? 1 : 0);
+    wave_lds_fence();
+    static_assert(sizeof(Grid) % 4 == 0, "copied word by word");
+    for (int q = t; q < static_cast<int>(sizeof(Grid) / 4); q += kWave) reinterpret_cast<int *>(grid)[q] = reinterpret_cast<const int *>(out)[q];
   }
   __syncthreads();
 }
@@ -236,7 +241,7 @@ __device__ __forceinline__ int bin_of(const Grid &g, double x, double y, double 
 
 // Up to kSmallAtoms atoms and bins: the whole cell list by one workgroup, with the bins counted and scanned in LDS, in place
 // of the five launches below.  Beyond that a thread's passes over its atoms cost more than the launches (12 000 atoms: 90
-// against 35 us; 2 000: 17 against 28).
+// against 35 us; 2 000: 17 against 28; with a thread's atoms in registers and the grid's axes side by side 2 000 17.5 -> 12.7, 216 10.2 -> 8.6).
 constexpr int kSmallAtoms = 4 * 1024;
 __global__ __launch_bounds__(kGridThreads) void nl_cells_small_kernel(const double *__restrict__ pos, const double *__restrict__ cell,
                                                                       int px, int py, int pz, double cutoff, int nnodes, int max_cells,
@@ -246,15 +251,23 @@ __global__ __launch_bounds__(kGridThreads) void nl_cells_small_kernel(const doub
   __shared__ int s_wave[kGridThreads / kWave];
   const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
   for (int c = t; c < max_cells; c += kGridThreads) s_count[c] = 0;
+  // a thread's atoms, t, t + 1024, ..., stay in its registers from here on
+  constexpr int kMine = kSmallAtoms / kGridThreads;
+  double r[kMine][3];
+  int key[kMine], slot[kMine], wrap[kMine][3];
+#pragma unroll
+  for (int u = 0; u < kMine; ++u) {
+    const int i = t + u * kGridThreads;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) r[u][k] = i < nnodes ? pos[3 * i + k] : 0.0;
+  }
   make_grid(pos, cell, px, py, pz, cutoff, nnodes, max_cells, w.grid, &g);  // ends with a barrier
   const int ncells = min(g.nb[0] * g.nb[1] * g.nb[2], max_cells);
-  for (int i = t; i < nnodes; i += kGridThreads) {
-    int wr[3];
-    const int key = bin_of(g, pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], wr);
-    w.keys[i] = key;
-    w.slot[i] = atomicAdd(&s_count[key], 1);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) w.wrap[3 * i + k] = wr[k];
+  for (int u = 0; u < kMine; ++u) {
+    if (t + u * kGridThreads >= nnodes) break;
+    key[u] = bin_of(g, r[u][0], r[u][1], r[u][2], wrap[u]);
+    slot[u] = atomicAdd(&s_count[key[u]], 1);
   }
   __syncthreads();
   // exclusive scan in place: a contiguous run of odd length per thread, then over the threads
@@ -280,13 +293,15 @@ __global__ __launch_bounds__(kGridThreads) void nl_cells_small_kernel(const doub
   __syncthreads();
   for (int c = t; c < ncells; c += kGridThreads) w.cell_offsets[c] = s_count[c];
   if (t == 0) w.cell_offsets[ncells] = nnodes;
-  for (int i = t; i < nnodes; i += kGridThreads) {  // a thread reads back what it wrote itself
-    const int key = w.keys[i];
-    const int at = s_count[key] + w.slot[i];
-    w.skey[at] = key;
-    w.smeta[at] = make_int4(i, w.wrap[3 * i], w.wrap[3 * i + 1], w.wrap[3 * i + 2]);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) w.spos[3 * static_cast<int64_t>(at) + k] = pos[3 * i + k];
+  for (int u = 0; u < kMine; ++u) {
+    const int i = t + u * kGridThreads;
+    if (i >= nnodes) break;
+    const int at = s_count[key[u]] + slot[u];
+    w.skey[at] = key[u];
+    w.smeta[at] = make_int4(i, wrap[u][0], wrap[u][1], wrap[u][2]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w.spos[3 * at + k] = r[u][k];
   }
 }
 
@@ -364,6 +379,16 @@ struct GraphOut {
   int32_t *ptr32;           // {0, N}; may be NULL
 };
 
+// A neighbour's place in the order of a segment: its index, then the image S.  The neighbours of one index j are scanned in images B of
+// the cell with S = B + (wrap of i) - (wrap of j), so B orders them as S does; |B| <= kMaxScan.
+__device__ __forceinline__ unsigned long long order_key(int j, int image) {
+  return static_cast<unsigned long long>(static_cast<unsigned>(j)) << 24 | static_cast<unsigned>(image);
+}
+__device__ __forceinline__ int pack_image(int b0, int b1, int b2) { return (b0 + 128) << 16 | (b1 + 128) << 8 | (b2 + 128); }
+__device__ __forceinline__ void unpack_image(int image, int (&b)[3]) {
+  b[0] = (image >> 16 & 255) - 128, b[1] = (image >> 8 & 255) - 128, b[2] = (image & 255) - 128;
+}
+
 __device__ __forceinline__ bool key_less(int ja, const int32_t *Sa, int jb, const int32_t *Sb) {
   if (ja != jb) return ja < jb;
   if (Sa[0] != Sb[0]) return Sa[0] < Sb[0];
@@ -375,14 +400,19 @@ __device__ __forceinline__ bool key_less(int ja, const int32_t *Sa, int jb, cons
 //   COUNT     degree[i] = number of neighbours
 //   SCRATCH   the neighbours (j, S) in scan order to scratch[offsets[i] ...] (j in scratch[0:E], S in scratch[E:4E])
 //   GRAPH     the neighbours collected in LDS (`cap` of them per wave), each written to its rank under the (j, S) order
+// Two times 64 candidates per trip, their look-ups and loads side by side: a trip is a chain of seven LDS reads and a load.  With that and
+// the rank from one 64-bit key per neighbour (the compare of index and image took 25 of 41 us at 123 neighbours, many of them images of one
+// atom) us, count / graph: 2 000 atoms with 52 neighbours 9.2 / 14.4 -> 7.7 / 10.8, 216 with 123 13.8 / 41 -> 12.9 / 16.7, 12 000
+// with 42 17.8 / 36.4 -> 18.3 / 32.6.
 enum class Scan { kCount, kScratch, kGraph };
 constexpr int kScanWaves = 4;
 template <Scan MODE>
 __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w, double cutoff, int nnodes,
                                                                      const int32_t *__restrict__ offsets, int64_t nedges,
                                                                      int32_t *__restrict__ scratch, GraphOut out, int cap) {
-  __shared__ int s_before[kScanWaves][kWave], s_first[kScanWaves][kWave], s_image[kScanWaves][kWave];
-  extern __shared__ int s_hits[];  // GRAPH: per wave cap neighbours, then cap images of three
+  constexpr int kBins = 2 * kWave;  // bins looked up at a time, two neighbouring ones per lane
+  __shared__ int s_before[kScanWaves][kBins], s_first[kScanWaves][kBins], s_image[kScanWaves][kBins];
+  extern __shared__ __attribute__((aligned(16))) unsigned char s_hits[];  // GRAPH: per wave cap keys, then cap places in bin order
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int at = blockIdx.x * (blockDim.x / kWave) + wave;
   if (at >= nnodes) return;
@@ -401,28 +431,42 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
 #pragma unroll
   for (int k = 0; k < 9; ++k) c[k] = grid->cellv[k];
   const int64_t seg = MODE == Scan::kCount ? 0 : offsets[i];
-  int *hj = s_hits + wave * 4 * cap, *hS = hj + cap;
+  unsigned long long *hkey = reinterpret_cast<unsigned long long *>(s_hits) + wave * cap;
+  int *hk = reinterpret_cast<int *>(s_hits + sizeof(*hkey) * (blockDim.x / kWave) * cap) + wave * cap;
   int count = 0;
   const int m1 = 2 * r1 + 1, m2 = 2 * r2 + 1;
   const int nscan = grid->status == 0 ? (2 * r0 + 1) * m1 * m2 : 0;
-  for (int first_bin = 0; first_bin < nscan; first_bin += kWave) {
-    // 64 bins side by side: where their atoms begin, how many there are, which image of the cell they belong to
-    const int q = first_bin + lane;
-    int first = 0, cnt = 0, image = 0;
-    if (q < nscan) {
-      int b0 = bi0 + q / (m1 * m2) - r0, b1 = bi1 + (q / m2) % m1 - r1, b2 = bi2 + q % m2 - r2;
-      int B0 = 0, B1 = 0, B2 = 0;
-      if (per0) B0 = floor_div(b0, nb0), b0 -= B0 * nb0;
-      if (per1) B1 = floor_div(b1, nb1), b1 -= B1 * nb1;
-      if (per2) B2 = floor_div(b2, nb2), b2 -= B2 * nb2;
-      if (b0 >= 0 && b0 < nb0 && b1 >= 0 && b1 < nb1 && b2 >= 0 && b2 < nb2) {
-        const int id = (b0 * nb1 + b1) * nb2 + b2;
-        first = w.cell_offsets[id];
-        cnt = w.cell_offsets[id + 1] - first;
-        image = (B0 + 128) | (B1 + 128) << 8 | (B2 + 128) << 16;  // |B| <= kMaxScan
+  const float per_plane = 1.0f / static_cast<float>(m1 * m2), per_row = 1.0f / static_cast<float>(m2);
+  // Exact: q + 1/2 over the divisor is half of its inverse away from an integer, and q < 65^3.
+  const auto quotient = [](int q, float inverse) { return static_cast<int>((static_cast<float>(q) + 0.5f) * inverse); };
+  // image of the cell that bin number b of an axis lies in, b then being its number in the cell
+  const auto wrap = [](int &b, int nb, int reach) {
+    const int B = reach <= nb ? (b < 0 ? -1 : (b >= nb ? 1 : 0)) : floor_div(b, nb);
+    b -= B * nb;
+    return B;
+  };
+  for (int first_bin = 0; first_bin < nscan; first_bin += kBins) {
+    // 128 bins side by side: where their atoms begin, how many there are, which image of the cell they belong to
+    int first[2] = {0, 0}, cnt[2] = {0, 0}, image[2] = {0, 0};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int q = first_bin + 2 * lane + u;
+      if (q < nscan) {
+        const int q0 = quotient(q, per_plane), in_plane = q - q0 * (m1 * m2), q1 = quotient(in_plane, per_row);
+        int b0 = bi0 + q0 - r0, b1 = bi1 + q1 - r1, b2 = bi2 + (in_plane - q1 * m2) - r2;
+        int B0 = 0, B1 = 0, B2 = 0;
+        if (per0) B0 = wrap(b0, nb0, r0);
+        if (per1) B1 = wrap(b1, nb1, r1);
+        if (per2) B2 = wrap(b2, nb2, r2);
+        if (b0 >= 0 && b0 < nb0 && b1 >= 0 && b1 < nb1 && b2 >= 0 && b2 < nb2) {
+          const int id = (b0 * nb1 + b1) * nb2 + b2;
+          first[u] = w.cell_offsets[id];
+          cnt[u] = w.cell_offsets[id + 1] - first[u];
+          image[u] = pack_image(B0, B1, B2);
+        }
       }
     }
-    int upto = cnt;
+    int upto = cnt[0] + cnt[1];
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       const int v = __shfl_up(upto, d);
@@ -430,47 +474,65 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
     }
     const int total = __shfl(upto, kWave - 1);
     wave_lds_fence();  // the previous bins' tables have been read
-    s_before[wave][lane] = upto - cnt;
-    s_first[wave][lane] = first;
-    s_image[wave][lane] = image;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      s_before[wave][2 * lane + u] = upto - cnt[1] - (u == 0 ? cnt[0] : 0);
+      s_first[wave][2 * lane + u] = first[u];
+      s_image[wave][2 * lane + u] = image[u];
+    }
     wave_lds_fence();
-    for (int base = 0; base < total; base += kWave) {
-      const int cand = base + lane;
-      bool hit = false;
-      int j = 0;
-      int S[3] = {0, 0, 0};
-      if (cand < total) {
-        int b = 0;  // the last bin whose atoms begin at or before cand: it is not empty, since cand < total
+    constexpr int kSets = 2;
+    for (int base = 0; base < total; base += kSets * kWave) {
+      int b[kSets], cand[kSets], image_of[kSets], S[kSets][3];
+      int64_t k_of[kSets];
+      int4 meta[kSets];
+      double pj[kSets][3];
 #pragma unroll
-        for (int step = kWave / 2; step > 0; step >>= 1)
-          if (s_before[wave][b + step] <= cand) b += step;
-        const int64_t k = s_first[wave][b] + (cand - s_before[wave][b]);
-        const int img = s_image[wave][b];
-        const int4 meta = w.smeta[k];
-        const double pj[3] = {w.spos[3 * k], w.spos[3 * k + 1], w.spos[3 * k + 2]};
-        j = meta.x;
-        S[0] = (img & 255) - 128 + wi[0] - meta.y;
-        S[1] = (img >> 8 & 255) - 128 + wi[1] - meta.z;
-        S[2] = (img >> 16 & 255) - 128 + wi[2] - meta.w;
-        hit = within(pi, pj, S, c, rc2) && !(j == i && S[0] == 0 && S[1] == 0 && S[2] == 0);
+      for (int u = 0; u < kSets; ++u) b[u] = 0, cand[u] = min(base + u * kWave + lane, total - 1);
+      // the last bin whose atoms begin at or before cand: it is not empty, since cand < total
+#pragma unroll
+      for (int step = kBins / 2; step > 0; step >>= 1) {
+        int before[kSets];
+#pragma unroll
+        for (int u = 0; u < kSets; ++u) before[u] = s_before[wave][b[u] + step];
+#pragma unroll
+        for (int u = 0; u < kSets; ++u) b[u] += before[u] <= cand[u] ? step : 0;
       }
-      const unsigned long long mask = __ballot(hit);
-      const int mine = count + __popcll(mask & ((1ull << lane) - 1ull));
-      if constexpr (MODE == Scan::kScratch) {
-        if (hit && seg + mine < nedges) {
-          scratch[seg + mine] = j;
 #pragma unroll
-          for (int k = 0; k < 3; ++k) scratch[nedges + 3 * (seg + mine) + k] = S[k];
+      for (int u = 0; u < kSets; ++u) {
+        k_of[u] = s_first[wave][b[u]] + (cand[u] - s_before[wave][b[u]]);
+        image_of[u] = s_image[wave][b[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < kSets; ++u) {
+        meta[u] = w.smeta[k_of[u]];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) pj[u][k] = w.spos[3 * k_of[u] + k];
+      }
+#pragma unroll
+      for (int u = 0; u < kSets; ++u) {
+        unpack_image(image_of[u], S[u]);
+        S[u][0] += wi[0] - meta[u].y, S[u][1] += wi[1] - meta[u].z, S[u][2] += wi[2] - meta[u].w;
+        const int j = meta[u].x;
+        const bool hit = base + u * kWave + lane < total && within(pi, pj[u], S[u], c, rc2) &&
+                         !(j == i && S[u][0] == 0 && S[u][1] == 0 && S[u][2] == 0);
+        const unsigned long long mask = __ballot(hit);
+        const int mine = count + __popcll(mask & ((1ull << lane) - 1ull));
+        if constexpr (MODE == Scan::kScratch) {
+          if (hit && seg + mine < nedges) {
+            scratch[seg + mine] = j;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) scratch[nedges + 3 * (seg + mine) + k] = S[u][k];
+          }
         }
-      }
-      if constexpr (MODE == Scan::kGraph) {
-        if (hit && mine < cap) {
-          hj[mine] = j;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) hS[3 * mine + k] = S[k];
+        if constexpr (MODE == Scan::kGraph) {
+          if (hit && mine < cap) {
+            hkey[mine] = order_key(j, image_of[u]);
+            hk[mine] = static_cast<int>(k_of[u]);
+          }
         }
+        count += __popcll(mask);
       }
-      count += __popcll(mask);
     }
   }
   if constexpr (MODE == Scan::kCount) {
@@ -479,24 +541,53 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
   if constexpr (MODE == Scan::kGraph) {
     wave_lds_fence();
     const int d = min(min(count, cap), static_cast<int>(min(static_cast<int64_t>(offsets[i + 1]), nedges) - seg));
-    for (int e = lane; e < d; e += kWave) {
-      const int j = hj[e];
-      const int S[3] = {hS[3 * e], hS[3 * e + 1], hS[3 * e + 2]};
-      int rank = 0;
-      for (int q = 0; q < d; ++q) {
-        const int jq = hj[q];
-        rank += jq < j ? 1 : 0;
-        if (jq == j && q != e) rank += key_less(jq, hS + 3 * q, j, S) ? 1 : 0;
-      }
-      const int64_t to = seg + rank;
+    // up to the next multiple of four (cap is one): keys above all others
+    if (lane < (-d & 3)) hkey[d + lane] = ~0ull;
+    wave_lds_fence();
+    auto emit = [&](int64_t to, unsigned long long key, int k) {
+      const int j = static_cast<int>(key >> 24);
+      const int4 meta = w.smeta[k];
+      int S[3];
+      unpack_image(static_cast<int>(key & 0xffffffu), S);
+      S[0] += wi[0] - meta.y, S[1] += wi[1] - meta.z, S[2] += wi[2] - meta.w;
       out.row_i[to] = i;
       out.row_j[to] = j;
       out.edge_index[to] = i;
       out.edge_index[nedges + to] = j;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        out.unit_shifts[3 * to + k] = S[k];
-        out.shifts[3 * to + k] = image_shift(S, c, k);
+      for (int q = 0; q < 3; ++q) {
+        out.unit_shifts[3 * to + q] = S[q];
+        out.shifts[3 * to + q] = image_shift(S, c, q);
+      }
+    };
+    // two neighbours per lane and pass over the keys
+    for (int e0 = 0; e0 < d; e0 += 2 * kWave) {
+      unsigned long long key[2];
+      int k[2], rank[2] = {0, 0};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int e = min(e0 + u * kWave + lane, d - 1);
+        key[u] = hkey[e], k[u] = hk[e];
+      }
+#pragma unroll 2
+      for (int q = 0; q < d; q += 4) {
+        unsigned long long other[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) other[v] = hkey[q + v];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rank[0] += other[v] < key[0] ? 1 : 0, rank[1] += other[v] < key[1] ? 1 : 0;
+      }
+      if (d <= 2 * kWave) {  // all of them are in registers: into their order in LDS first, then out in that order, lane by lane
+        wave_lds_fence();
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (u * kWave + lane < d) hkey[rank[u]] = key[u], hk[rank[u]] = k[u];
+        wave_lds_fence();
+        for (int e = lane; e < d; e += kWave) emit(seg + e, hkey[e], hk[e]);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (e0 + u * kWave + lane < d) emit(seg + rank[u], key[u], k[u]);
       }
     }
     if (lane == 0) {
@@ -778,7 +869,7 @@ extern "C" int cm_neighbour_list_search_counts(const double *positions, const do
   return CM_OK;
 }
 
-// A wave keeps a segment's hits in LDS, 16 bytes each: four waves per workgroup up to 512 of them, then one.
+// A wave keeps a segment's hits in LDS, 12 bytes each: four waves per workgroup up to 512 of them, then one.
 static constexpr int kGraphMaxDegree = 8192;
 
 extern "C" int cm_neighbour_list_graph_max_degree(void) { return kGraphMaxDegree; }
@@ -801,7 +892,7 @@ extern "C" int cm_neighbour_list_graph(double cutoff, int64_t nnodes, int64_t ma
   const int cap = std::max(kGraphMaxDegree > max_degree ? (max_degree + 63) / 64 * 64 : max_degree, 64);
   const int waves = cap <= 512 ? cm::kScanWaves : 1;
   hipLaunchKernelGGL(cm::nl_scan_kernel<cm::Scan::kGraph>, dim3(static_cast<unsigned>(cm::ceil_div(n, waves))), dim3(waves * cm::kWave),
-                     static_cast<unsigned>(waves * cap * 16), cm::as_stream(stream), w, cutoff, n, offsets, nedges,
+                     static_cast<unsigned>(waves * cap * 12), cm::as_stream(stream), w, cutoff, n, offsets, nedges,
                      static_cast<int32_t *>(nullptr), cm::GraphOut{row_i, row_j, edge_index, unit_shifts, shifts, first_occ, batch, ptr, ptr32},
                      cap);
   return cm::check_launch("cm_neighbour_list_graph");

@@ -99,6 +99,8 @@ GRAPH_CASES = {
     "box": (1000, 21.5, (1, 1, 1), 5.0),
     "dense": (900, 9.0, (1, 1, 1), 5.5),          # more than 512 neighbours: one wave per workgroup
     "denser": (400, 3.0, (0, 0, 0), 6.0),
+    "about_two_per_lane": (260, 8.6, (1, 1, 1), 4.4),  # 128 neighbours and a few less or more: in order through LDS, or by rank
+    "thinner_than_the_reach": (3, 1.3, (1, 1, 1), 6.0),
     "one_workgroup_most": (4096, 34.5, (1, 1, 1), 4.0),
     "several_launches": (4097, 34.5, (1, 1, 0), 4.0),
     "many_32768": (32768, 69.0, (1, 1, 1), 4.0),
@@ -120,7 +122,7 @@ def test_graph_of_a_list(cabi, name):
     cell = None if box is None else np.eye(3) * box + np.array([[0, 0, 0], [0.3, 0, 0], [0.1, -0.2, 0]])
     p = torch.tensor(pos, dtype=torch.float64, device=DEV)
     c = None if cell is None else torch.tensor(cell, dtype=torch.float64, device=DEV)
-    if name in ("one_atom_images", "few_atoms_many_images", "wave_edges"):
+    if name in ("one_atom_images", "few_atoms_many_images", "wave_edges", "thinner_than_the_reach"):
         _check(pos, cell, pbc, cutoff)
     ri, rj, S = cabi_mod.neighbour_list(p, c, pbc, cutoff)
     g = cabi_mod.neighbour_graph(p, c, pbc, cutoff)
