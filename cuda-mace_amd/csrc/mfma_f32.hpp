@@ -60,7 +60,8 @@ __device__ __forceinline__ void product(const Rows<KQ> &x, const Rows<KQ> (&wt)[
 // after the other waits for the fp32 matrix rate.  Measured (us, the tiled kernels -> this one):
 //   [N, C]      216 x 64 5.0 -> 2.7, 216 x 128 6.7 -> 3.6, 2 000 x 128 6.9 -> 3.7, 2 000 x 256 10.8 -> 7.7, 10 000 x 64 5.5 -> 4.7;
 //               even at 5 000 x 128 and 192 (2 500 and 3 750 blocks).  At 96 and 128 columns the products between the layers
-//               run as chains on shared tiles (node_glue.hip), which are the faster ones from 1 536 blocks on
+//               run as chains on shared tiles (node_glue.hip), which are the faster ones from 1 536 blocks on; at 224 and 256 the
+//               kernel with a workgroup per 128 rows is from 2 048 on (2 500 x 256 12.4 -> 9.2)
 //   [N, 16, C]  216 x 64 5.3 -> 2.9, 216 x 128 7.2 -> 5.0, 500 x 96 6.9 -> 5.5, 216 x 192 9.9 -> 8.6 (2 688 blocks); even at 500 x 128
 //               and 1 000 x 64 (4 000 blocks), slower beyond
 // From 1 024 blocks (a wave on every SIMD) a wave takes two neighbouring blocks of columns and reads its rows once for
@@ -68,7 +69,7 @@ __device__ __forceinline__ void product(const Rows<KQ> &x, const Rows<KQ> (&wt)[
 inline int64_t blocks(int64_t nnodes, int ncomp, int columns) { return ceil_div(nnodes, kRows) * ncomp * (columns / kRows); }
 constexpr int64_t kOneColumnBlock = 1024;
 inline bool applies(int64_t nnodes, int ncomp, int columns) {
-  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 || columns == 128 ? 1536 : 2560);
+  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 || columns == 128 ? 1536 : (columns >= 224 ? 2048 : 2560));
   return blocks(nnodes, ncomp, columns) <= limit;
 }
 

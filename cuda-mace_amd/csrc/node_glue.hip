@@ -308,6 +308,8 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_glue_backward_few_kernel(
 // pipes: 3 x 0.9 us at 128 channels, and 3 x 64 KB of weights on their way to it), so the chain is cut at h1 / gh1 and each
 // part spreads its 16-column blocks over the device like any linear.  Measured in the step of 216 nodes and 128 channels
 // (32-row tiles -> both launches): forward 15.4 -> 9.3 us, backward 16.3 -> 11.4 (one launch of the chain above: 10.8, 13.1).
+// Beyond 128 channels the same two cuts serve the step of few nodes (node_chains_cut), three launches fewer: 216 x 192 181 -> 172 us per
+// step, 500 x 224 255 -> 248, 216 x 256 209 -> 202, 60 x 192 160 -> 154, 1 000 x 256 349 -> 343.
 template <int KQ>
 __global__ __launch_bounds__(4 * kWave) void node_glue_skip_up_kernel(const float *__restrict__ h1, const float *__restrict__ skip_WT,
                                                                       const float *__restrict__ up_WT, const int32_t *__restrict__ node_perm,
@@ -580,6 +582,34 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_head_few_kernel(
 // 14.7 + 13.9, 25 000 x 128 28.9 + 29.1 / 20.7 + 20.9.
 inline bool four_waves(int64_t nnodes) { return ceil_div(nnodes, 128) * 2 < device_compute_units(); }
 
+// The chains cut at h1 / gh1 (few nodes): product and skip + up, or gh1 and product.
+template <int NT>
+int launch_forward_cut(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm, const int32_t *offs,
+                       int64_t nnodes, int ngroups, float skip_scale, float *h1, float *sc, float *X2, hipStream_t st) {
+  constexpr int kBlocks = 4 * NT, kPerGroup = NT == 3 ? 3 : 4;
+  static_assert(kBlocks % kPerGroup == 0, "the blocks divide evenly among the workgroups");
+  const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
+  const int rc = cm_linear(B1, prod_WT, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, h1, st);
+  if (rc != CM_OK) return rc;
+  hipLaunchKernelGGL((node_glue_skip_up_kernel<2 * NT>), dim3(tiles, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, h1, skip_WT, up_WT, perm,
+                     offs, static_cast<int>(nnodes), ngroups, skip_scale, sc, X2);
+  return check_launch("cm_node_glue_forward");
+}
+template <int NT>
+int launch_backward_cut(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W, const double *w1,
+                        double scale, const double *node_weights, const int32_t *perm, const int32_t *offs, int64_t nnodes, int ngroups,
+                        float skip_scale, float *gh1, float *gB1, const EnergySums &sums, hipStream_t st) {
+  constexpr int kBlocks = 2 * NT, kPerGroup = NT % 2 == 0 ? 4 : (NT % 3 == 0 ? 3 : 2);
+  static_assert(kBlocks % kPerGroup == 0, "the blocks divide evenly among the workgroups");
+  const unsigned extra = sums.out ? static_cast<unsigned>(sums.ngraphs) : 0u;
+  const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
+  hipLaunchKernelGGL((node_glue_gh1_kernel<2 * NT>), dim3(tiles + extra, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, gX2, d_h2, up_W, skip_W,
+                     w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gh1, sums, static_cast<int>(extra));
+  const int rc = check_launch("cm_node_glue_backward");
+  if (rc != CM_OK) return rc;
+  return cm_linear(gh1, prod_W, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, gB1, st);
+}
+
 template <int NT>
 int launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *perm,
                    const int32_t *offs, int64_t nnodes, int ngroups, float skip_scale, float *h1, float *sc, float *X2,
@@ -587,11 +617,7 @@ int launch_forward(const float *B1, const float *prod_WT, const float *skip_WT, 
   if (few::applies(nnodes, 1, 32 * NT)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
     if constexpr (NT >= 3) {
-      constexpr int kBlocks = 4 * NT, kPerGroup = NT == 3 ? 3 : 4;
-      const int rc = cm_linear(B1, prod_WT, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, h1, st);
-      if (rc != CM_OK) return rc;
-      hipLaunchKernelGGL((node_glue_skip_up_kernel<2 * NT>), dim3(tiles, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, h1, skip_WT,
-                         up_WT, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, sc, X2);
+      return launch_forward_cut<NT>(B1, prod_WT, skip_WT, up_WT, perm, offs, nnodes, ngroups, skip_scale, h1, sc, X2, st);
     } else {
       hipLaunchKernelGGL((node_glue_forward_few_kernel<NT>), dim3(tiles), dim3(2 * NT * kWave), 0, st, B1, prod_WT, skip_WT, up_WT, perm,
                          offs, static_cast<int>(nnodes), ngroups, skip_scale, h1, sc, X2);
@@ -616,15 +642,8 @@ int launch_backward(const float *gX2, const float *d_h2, const float *up_W, cons
   const unsigned extra = sums.out ? static_cast<unsigned>(sums.ngraphs) : 0u;
   if (few::applies(nnodes, 1, 32 * NT)) {
     const unsigned tiles = static_cast<unsigned>(ceil_div(nnodes, few::kRows) + ngroups);
-    if (NT >= 3 && gh1) {
-      constexpr int kBlocks = 2 * NT, kPerGroup = NT % 2 == 0 ? 4 : (NT % 3 == 0 ? 3 : 2);
-      hipLaunchKernelGGL((node_glue_gh1_kernel<2 * NT>), dim3(tiles + extra, kBlocks / kPerGroup), dim3(kPerGroup * kWave), 0, st, gX2, d_h2,
-                         up_W, skip_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gh1, sums,
-                         static_cast<int>(extra));
-      const int rc = check_launch("cm_node_glue_backward");
-      if (rc != CM_OK) return rc;
-      return cm_linear(gh1, prod_W, nullptr, nullptr, nnodes, 1, 0, 1, 32 * NT, 32 * NT, 1.0f, nullptr, nullptr, gB1, st);
-    }
+    if (NT >= 3 && gh1)
+      return launch_backward_cut<NT>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, perm, offs, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     hipLaunchKernelGGL((node_glue_backward_few_kernel<NT>), dim3(tiles + extra), dim3(2 * NT * kWave), 0, st, gX2, d_h2, up_W, skip_W,
                        prod_W, w1, scale, node_weights, perm, offs, static_cast<int>(nnodes), ngroups, skip_scale, gB1, sums,
                        static_cast<int>(extra));
@@ -682,6 +701,23 @@ extern "C" int cm_node_glue_forward(const float *B1, const float *prod_WT, const
 
 namespace cm {
 
+// Up to 1 536 blocks: beyond, a product is faster on tiles of 128 rows that share its operands (2 500 x 256 as three launches 28 us, cut 33).
+bool node_chains_cut(int64_t nnodes, int channels) {
+  return channels > 128 && few::blocks(nnodes, 1, channels) <= 1536 && few::applies(nnodes, 1, channels);
+}
+
+int node_glue_forward_cut(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *node_perm,
+                          const int32_t *group_offsets, int64_t nnodes, int ngroups, int channels, float skip_scale, float *h1, float *sc, float *X2,
+                          hipStream_t st) {
+  switch (channels / 32) {
+#define CM_CASE(NT_) \
+    case NT_: return launch_forward_cut<NT_>(B1, prod_WT, skip_WT, up_WT, node_perm, group_offsets, nnodes, ngroups, skip_scale, h1, sc, X2, st);
+    CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8)
+#undef CM_CASE
+    default: set_error("node glue: channels=%d not supported", channels); return CM_EINVAL;
+  }
+}
+
 // cm_node_glue_backward whose launch also sums the node energies per graph (operands checked by the caller, cm_mace_step)
 int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, const float *up_W, const float *skip_W, const float *prod_W,
                                         const double *w1, double scale, const double *node_weights, const int32_t *node_perm,
@@ -694,6 +730,10 @@ int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, con
     case 2: return launch_backward<2>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     case 3: return launch_backward<3>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
     case 4: return launch_backward<4>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
+#define CM_CASE(NT_) \
+    case NT_: return launch_backward_cut<NT_>(gX2, d_h2, up_W, skip_W, prod_W, w1, scale, node_weights, node_perm, group_offsets, nnodes, ngroups, skip_scale, gh1, gB1, sums, st);
+    CM_CASE(5) CM_CASE(6) CM_CASE(7) CM_CASE(8)
+#undef CM_CASE
     default: set_error("node glue: channels=%d not supported", channels); return CM_EINVAL;
   }
 }

@@ -16,6 +16,13 @@ int node_glue_backward_with_energy_sums(const float *gX2, const float *d_h2, con
                                         float *gB1, const double *node_es, const int32_t *graph_ptr, int ngraphs, double *energies,
                                         const double *graph_e0, double *total_energies, hipStream_t st);
 
+// Beyond 128 channels, few nodes: whether node_glue_forward_cut and node_glue_backward_with_energy_sums take the step's products between
+// the layers, two launches per direction (the same products as three or four launches of the linear kernel).
+bool node_chains_cut(int64_t nnodes, int channels);
+int node_glue_forward_cut(const float *B1, const float *prod_WT, const float *skip_WT, const float *up_WT, const int32_t *node_perm,
+                          const int32_t *group_offsets, int64_t nnodes, int ngroups, int channels, float skip_scale, float *h1, float *sc, float *X2,
+                          hipStream_t st);
+
 // h2 = B2 . Wprod + sc (kept on chip), the readouts of h1 and h2 with everything cm_readout_forward writes, and, with d_h2
 // given, d_h2 = weight dE/dh2 (node_weights NULL: one) and gB2 = -d_h2 . Wprod^T.  32 to 128 channels (cm_node_glue_supported).
 int node_head(const float *B2, const float *sc, const float *h1, const float *prod_WT, const float *prod_W, const readout::Weights &w,

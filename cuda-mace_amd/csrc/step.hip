@@ -519,8 +519,11 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   const char *glue_env = getenv("CM_STEP_GLUE");  // development switch: smallest node count that takes the chained kernels; -1: none
   const int glue_min = glue_env ? atoi(glue_env) : 0;
   const bool glue = cm_node_glue_supported(C) != 0 && glue_min >= 0 && N >= glue_min;
+  // beyond 128 channels and for few nodes the same in two launches; the head stays three, and weights of the nodes need their pass over dE/dh2
+  const bool cut = !glue && glue_min >= 0 && cm::node_chains_cut(N, C);
+  const bool cut_backward = cut && !g->node_weights;
   for (int t = 0; t < 2; ++t) {
-    if (t == 1 && !glue) {
+    if (t == 1 && !glue && !cut) {
       // residual skip connection per element and linear_up, both of the first layer's output
       CM_STAGE(5, cm_linear(L.h1, w->skip_WT, oh_perm, oh_off, N, ne + 1, 1, 1, C, C, w->skip_scale, none, none, L.sc, stream));
       CM_STAGE(6, cm_linear(L.h1, w->up_WT, nullptr, nullptr, N, 1, 0, 1, C, C, 1.0f, none, none, L.X2, stream));
@@ -542,6 +545,9 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
     if (t == 0 && glue)
       CM_STAGE(4, cm_node_glue_forward(L.B1, w->prod_WT[0], w->skip_WT, w->up_WT, oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.h1, L.sc,
                                        L.X2, stream));
+    else if (t == 0 && cut)
+      CM_STAGE(4, cm::node_glue_forward_cut(L.B1, w->prod_WT[0], w->skip_WT, w->up_WT, oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.h1, L.sc, L.X2,
+                                            st));
     else if (t == 0 || !glue)
       CM_STAGE(t == 0 ? 4 : 10, cm_linear(B[t], w->prod_WT[t], nullptr, nullptr, N, 1, 0, 1, C, C, 1.0f, none, t == 1 ? L.sc : none, h[t], stream));
   }
@@ -566,7 +572,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // own: the gradient with respect to the second layer's features is -d_h2 (the sign goes into the scale of the two
   // linears that consume it, which is exact; node weights scale its rows first), the one with respect to the first
   // layer's is a constant row (times the node's weight).
-  if (!glue) {  // the chained kernels form the constant rows themselves, weight the others, and take the energy sums along
+  if (!glue && !cut_backward) {  // the chained kernels form the constant rows themselves, weight the others, and take the energy sums along
     cm::StageTimer timer_(st, 13, timing_mask);
     const unsigned rows = static_cast<unsigned>(std::min<int64_t>(cm::ceil_div(N, cm::kSumThreads / cm::kWave), 1024));
     hipLaunchKernelGGL(cm::energies_and_seeds_kernel, dim3(g->ngraphs + rows), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights, g->graph_ptr,
@@ -579,7 +585,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   CM_STAGE(16, cm_mp_edge_backward(L.X2, L.vec, w->r_knots, w->spline[1], w->nknots, w->r_width, w->r_max, L.bufA, g->sender,
                               fo_live, g->sender_perm, g->sender_offsets, N, E, C, L.gX2, L.gv2, L.edge_scratch, stream));
   // layer 0 (first interaction): its input features depend on the species alone, so no gradient with respect to them
-  if (glue) {
+  if (glue || cut_backward) {
     CM_STAGE(17, cm::node_glue_backward_with_energy_sums(L.gX2, L.d_h2, w->up_W, w->skip_W, w->prod_W[0], w->w1, w->scale, g->node_weights,
                                                          oh_perm, oh_off, N, ne + 1, C, w->skip_scale, L.gh1, L.gB, node_energy, g->graph_ptr,
                                                          g->ngraphs, interaction_energy, g->graph_e0, total_energy, st));

@@ -547,7 +547,7 @@ def test_native_step_on_a_list_with_a_skin(cabi, relabel):
 @pytest.mark.parametrize("natoms,channels", [(60, 64), (700, 128), (3000, 96)])
 def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
     """Up to 128 channels the one-call step runs the three [N,C] products between the layers, and their transposes, as one
-    chained launch per direction (on 32-node tiles for few nodes, 128-node tiles otherwise) and sums the energies in that
+    chained launch per direction (two for a few hundred nodes of 96 or 128 channels) and sums the energies in that
     launch; the library's switch for the separate launches (CM_STEP_GLUE=-1, read per call) gives the same step as the
     same kernels beyond 128 channels run it.  Same operand split, piece order and rounding points: node energies, node
     features and forces agree bit for bit; the graph energy is a sum in another (fixed) order."""
@@ -568,11 +568,13 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
     torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
-@pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32)])
+@pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32),
+                                             (60, 192), (400, 160), (300, 224), (1536, 256), (1537, 256)])
 def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
     """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 32
     and 128 nodes with a partly filled last one, against the separate launches: bit for bit, for forces and for energies alone,
-    with weights on the node energies and without."""
+    with weights on the node energies and without.  Beyond 128 channels the products between the layers in two launches per direction,
+    for few nodes."""
     data = make_system(natoms, 4, seed=7, density=None, cluster_box=12.0) if natoms < 130 else make_system(natoms, 4, seed=7, density=0.015)
     _, model = _build(channels, (1, 6, 7, 8), data, seed=8)
     dev = to_device(data, "cuda")
