@@ -17,6 +17,8 @@
 // straight into the gradient with respect to its vector (harmonics Jacobian + radial part), so Y[16, E], grad_Y and
 // grad_r never exist either.  Beyond a thousand or two of receiver nodes the forward from edge vectors runs on the kernel of
 // mp_sliced.hip, which keeps a workgroup's part of the table in LDS (same arithmetic per edge, sums in list order).
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "mp_common.hpp"
@@ -183,7 +185,7 @@ struct MRange {
 // -----------------------------------------------------------------------------------------------
 // forward
 // -----------------------------------------------------------------------------------------------
-// MULTI: a workgroup of up to eight waves per node, each on a part of the node's edge range (launched for few nodes)
+// MULTI: a workgroup of up to six waves per node, each on a part of the node's edge range (launched for few nodes)
 template <int C, bool FROM_VEC, bool MULTI>
 __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::V > 5 ? 2 : CM_FUSED_FWD_WAVES)) void mp_spline_forward_kernel(const float *__restrict__ X,
                                                                  const float *__restrict__ Y, Spline sp,
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::
                                                                  int64_t nedges, float *__restrict__ out) {
   using K = Cfg<C, true>;
   using vec = typename K::vec;
-  // A workgroup is one wave per part of the node's edge range (MULTI; otherwise one wave and one part: see parts_for).
+  // A workgroup is one wave per part of the node's edge range (MULTI; otherwise one wave and one part: see forward_parts).
   // Every wave stages its own edges in its own piece of LDS; the waves meet once, at the end.
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn_lds[];
   const int wave = MULTI ? threadIdx.x / kWave : 0;
@@ -471,7 +473,7 @@ __global__ __launch_bounds__(kWave, (kOneOperandSet<C, FROM_VEC> ? 3 : CM_FUSED_
   // waited for behind everything the wave has in flight (the gradient rows from HBM first of all).
   __shared__ float sKnots[kKnotsInLds];
 
-  // one wave per node, or (few nodes: parts_for) per part of a node's edge range: every output of this pass belongs to
+  // one wave per node, or (backward_parts) per part of a node's edge range: every output of this pass belongs to
   // one edge, so the parts share nothing but the node's gradient rows, which each of them reads
   const int node = parts == 1 ? blockIdx.x : blockIdx.x / parts;
   const int lane = threadIdx.x;
@@ -846,10 +848,49 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
   while (cursor < e1) chunk(std::false_type{});
 }
 
+// Parts of a receiver's edges in the forward pass, a wave each, all of one node in a workgroup.  A part is worth its place in the sum of the
+// parts from four edges per slot on (three at eight slots), and a compute unit holds eight such waves: more nodes than one round of
+// workgroups of p waves take fewer parts.  us at p = 1 2 3 4 5 6 8, the rule's p in brackets: 128 channels 216 x 52 18.9 12.1 11.2 10.8
+// 10.6 [10.6] 11.7, 400 x 52 19.4 14.5 13.9 [14.2] 18.4 19.0 20.1, 60 x 30 11.0 8.3 [8.2] 8.4 8.3 8.7 9.8; 64 216 x 52 11.8 8.8 [8.5] 9.0 9.2 9.7
+// 10.7, 1 000 x 30 [10.2] 11.6 15.7 17.5 28 30 34; 256 21 x 12 14.0 8.2 [7.5] 7.7 7.6 7.8 8.0, 300 x 9 12.8 [8.6] 8.6 8.9 11.9 12.1 12.9, 216 x 52
+// 43.5 20.5 17.2 16.1 15.1 [15.1] 15.7; 192 672 x 9 14.7 [10.7] 11.6 12.2 15.7 15.9 17.4.
+template <int C>
+int forward_parts(int64_t nnodes, int64_t nedges) {
+  constexpr int kSlots = Cfg<C, true>::EPW, kLeast = kSlots >= 8 ? 24 : 4 * kSlots;
+  if (nnodes <= 0) return 1;
+  int parts = static_cast<int>(std::min<int64_t>(6, std::max<int64_t>(1, nedges / (kLeast * nnodes))));
+  while (parts > 1 && nnodes > static_cast<int64_t>(device_compute_units()) * (8 / parts)) --parts;
+  return parts;
+}
+
+// Parts of a receiver's edges in the backward edge pass, waves that share nothing: the number that takes the least time if a wave costs its
+// edges and eight more (the gradient rows, the staging), waves run in rounds of what the chip holds, and a round that is
+// filled by a share f takes 0.55 + 0.45 f of a full one.  us without / with gX at p = 1 2 3 4 6 8, the rule's p in brackets: 128 channels 216 x
+// 52 26.1 / 40 16.2 / 24 12.3 / 19 10.4 / 17 9.3 / 15.6 [9.3 / 15.7], 700 x 52 28.7 / 43 [20.2 / 31] 22.3 / 33 21.8 / 33 23.8 / 36 25.2 / 37, 1 200 x 52
+// 33.4 / 49 31.5 / 47 [28.5 / 43], 2 200 x 52 58 / 81 [53.5 / 75] 55.3 / 79, 3 300 x 52 [68.9 / 98.7] 67.5 / 98.5 72 / 106, 5 000 x 52 [105.6 / 149]
+// 107 / 150 116 / 162, 2 500 x 12 [20.3 / 29.9] 22.1 / 32.4; 64 21 x 9 6.2 / 9.7 5.3 / 8.7 4.8 / 8.1 4.6 / 8.3 (five: [4.3 / 7.8]) 4.3 / 7.9 4.3 / 8.1,
+// 1 200 x 52 19.7 / 29.9 [16.5 / 25.5] 18.3 / 28.2; 256 21 x 12 16.2 / 24 10.1 / 15.6 7.7 / 12.7 7.1 / 11.5 5.8 / 9.9 [5.3 / 9.5], 1 200 x 52 64 / 98 59 / 85
+// [55 / 78]; 160 2 200 x 52 76 / 109 [67 / 98] 68 / 101.
+template <int C, bool FROM_VEC>
+int backward_parts(int64_t nnodes, int64_t nedges) {
+  if (nnodes <= 0) return 1;
+  constexpr int kMost = C <= 64 ? 5 : 8;  // (narrow rows: 400 x 52 x 64 five 8.1 us, eight 10.9)
+  const double slots = device_compute_units() * (kOneOperandSet<C, FROM_VEC> ? 12.0 : 8.0);
+  const double edges = static_cast<double>(nedges) / static_cast<double>(nnodes);
+  int best = 1;
+  double least = 0.0;
+  for (int p = 1; p <= kMost && (p == 1 || edges >= p); ++p) {
+    const double rounds = static_cast<double>(nnodes) * p / slots, full = std::floor(rounds);
+    const double time = (full + (rounds > full ? 0.55 + 0.45 * (rounds - full) : 0.0)) * (edges / p + 8.0);
+    if (p == 1 || time < least) best = p, least = time;
+  }
+  return best;
+}
+
 template <int C, bool FROM_VEC>
 int launch_forward(const float *X, const float *Y, const Spline &sp, const int32_t *sender, const int32_t *first_occ,
                    int64_t nnodes, int64_t nedges, float *out, hipStream_t st) {
-  const int parts = parts_for(nnodes, nedges);
+  const int parts = forward_parts<C>(nnodes, nedges);
   const size_t lds = static_cast<size_t>(parts) * kStageBytes + static_cast<size_t>(parts - 1) * 16 * C * sizeof(float);
   if (parts > 1)
     hipLaunchKernelGGL((mp_spline_forward_kernel<C, FROM_VEC, true>), dim3(static_cast<unsigned>(nnodes)), dim3(kWave * parts), lds, st,
@@ -887,7 +928,7 @@ template <int C, bool FROM_VEC, bool GY, bool GR, bool GX>
 void launch_edge(const float *X, const float *Y, const Spline &sp, const float *G, const int32_t *sender,
                  const int32_t *first_occ, int64_t nnodes, int64_t nedges, float *gY, float *g_r, float *gXe,
                  hipStream_t st) {
-  const int parts = parts_for(nnodes, nedges);
+  const int parts = backward_parts<C, FROM_VEC>(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
   if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {
     if (steps_of_four_edges<C>(nnodes, nedges, parts)) {
@@ -993,7 +1034,7 @@ extern "C" int cm_mp_edge_forward_kernel(int64_t nnodes, int64_t nedges, int cha
 extern "C" int cm_mp_edge_backward_kernel(int64_t nnodes, int64_t nedges, int channels) {
   if (nnodes <= 0) return 0;
   bool steps = false;
-  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, cm::mp::parts_for(nnodes, nedges)));
+  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, (cm::backward_parts<C_, true>(nnodes, nedges))));
   return steps ? 1 : 0;
 }
 
