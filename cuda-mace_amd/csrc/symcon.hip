@@ -11,6 +11,7 @@
 // Every kernel is a template over the scalar type: fp32 is the model's precision, fp64 is built because the reference
 // dispatches the contraction on float and double (jit_wrappers/src/symmetric_contraction_wrapper.cpp:68).
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "symcon_lmax3.inc"
@@ -144,12 +145,28 @@ __global__ void symcon_forward_kernel(const S *__restrict__ X, const int32_t *__
 
 // Specialised forward for the l_max = 3 structure known at build time: the monomial lists are unrolled, so a
 // thread (= one channel) keeps its 77 + 16 + 1 coefficients, the node's 16 inputs and 16 gradient accumulators in
-// registers and streams over `npb` nodes of one element.  No LDS; loads and stores are coalesced rows.  npb is 16 where
-// that still gives every SIMD two waves (the coefficient loads are then a fifth of a wave's loads), fewer for fewer
-// nodes, down to 1: at 5 000 nodes x 96 channels 16 nodes per wave leave the device at 0.6 waves per SIMD (29 us per
-// launch, the time of one wave's 16 nodes), and a wave's second node costs what its first does (21 nodes x 64 channels
-// 5.9 -> 4.7 us, 216 x 128 6.3 -> 5.2, with the search for the wave's element done by all lanes at once).
+// registers and streams over `npb` nodes of one element (nodes_per_wave).  No LDS; loads and stores are coalesced rows.
 constexpr int kMaxNodesPerBlock = 16;
+
+// Nodes per wave: a wave's coefficients are a third of a node's time, three waves fit a SIMD, and waves that run in rounds should fill
+// them: the number with the least time if a round takes its nodes and 0.3 more, and one filled by a share f 0.45 + 0.55 f of that.  us at
+// 1 2 3 4 6 8 12 16 nodes, the rule's or the nearest one in brackets: 25 000 x 128 84.7 71.0 68.6 68.5 68.6 [73.0 75.7] 84.9 (nine 68: 6 TB/s of
+// its bytes; sixteen are one round and two waves more), 25 000 x 96 80.8 66.7 62.8 62.8 62.0 [66.4 68.6] 77.7, 2 000 x 128 11.0 [9.0] 10.1 11.1 13.2 15.7
+// 21.7 26.8, 5 000 x 96 21.3 17.3 19.1 [16.3] 17.1 19.9 24.4 30.1, 10 752 x 128 39.7 34.3 34.0 33.4 37.2 [32.7] 32.1 36.0, 10 752 x 64 22.5 20.1 21.4 [19.2] 19.5 21.9 26.0 30.8, 216 x 128 [4.8] 6.1 7.4 8.8.
+// In fp64 one wave fills a SIMD: 16 nodes where that still gives every SIMD two waves, fewer for fewer nodes.
+template <typename S>
+int nodes_per_wave(int64_t nnodes, int nelements, int64_t column_blocks) {
+  const double simds = 4.0 * device_compute_units(), n = static_cast<double>(nnodes), columns = static_cast<double>(column_blocks);
+  if (sizeof(S) == 8) return std::max(1, static_cast<int>(std::min<double>(kMaxNodesPerBlock, n * columns / (2.0 * simds))));
+  int best = 1;
+  double least = 0.0;
+  for (int p = 1; p <= kMaxNodesPerBlock; ++p) {
+    const double rounds = columns * (n / p + 0.5 * nelements) / (3.0 * simds), full = std::floor(rounds);  // (half a wave lost per element)
+    const double time = (full + (rounds > full ? 0.45 + 0.55 * (rounds - full) : 0.0)) * (p + 0.3);
+    if (p == 1 || time < least) best = p, least = time;
+  }
+  return best;
+}
 
 template <typename S, bool GRAD>
 __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict__ X,
@@ -290,8 +307,7 @@ int forward(const char *what, const S *X, const int32_t *node_perm, const int32_
                CM_SYMCON_N2, n3, n2);
     CM_REQUIRE(T3 && T2, "%s: NULL table", what);
     const int64_t column_blocks = ceil_div(channels, kWave);
-    const int64_t two_waves_per_simd = static_cast<int64_t>(device_compute_units()) * 4 * 2;
-    const int npb = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMaxNodesPerBlock, nnodes * column_blocks / two_waves_per_simd)));
+    const int npb = nodes_per_wave<S>(nnodes, nelements, column_blocks);
     const dim3 grid(static_cast<unsigned>(ceil_div(nnodes, npb) + nelements), static_cast<unsigned>(column_blocks));
     if (grad)
       hipLaunchKernelGGL((symcon_lmax3_kernel<S, true>), grid, dim3(kWave), 0, st, X, node_perm, group_offsets, T3, T2, T1,
