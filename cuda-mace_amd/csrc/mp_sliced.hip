@@ -97,7 +97,21 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 //   224  35 000 x 6 3 000 -> 3 012, x 8.2 3 206 -> 3 164, 60 000 x 6 5 115 -> 5 130, x 8.3 5 454 -> 5 368
 //   256  6 000 x 8.4 765 -> 778, x 16 882 -> 880, 12 000 x 8.2 1 279 -> 1 318, x 13 1 408 -> 1 393, 20 000 x 8.3 2 055 -> 2 076, x 13 2 272 -> 2 249, 60 000 x 10.5 6 442 ->
 //        6 559, x 16 7 247 -> 7 153, 80 000 x 13 9 053 -> 9 270, x 19 10 491 -> 10 346
-inline int64_t min_nodes_per_workgroup(int channels) { return channels == 32 ? 60 : (channels == 160 ? 64 : 76); }
+// The lines as they were redrawn when the other kernel's nodes came to be cut into up to six parts, steps with forces, one wave per node (or
+// part) -> this one, us: 160 540 x 52 214.9 -> 205.6, x 26 178.4 -> 173.7, 420 x 52 192.6 -> 194.8; 192 560 x 52 224.8 -> 221.8, x 26 185.0 ->
+// 186.5; 224 400 x 52 234.7 -> 224.0, x 26 201.1 -> 197.1, 60 molecules of 21 (8.8 neighbours) 277.5 -> 271.8; 256 560 x 52 273.3 -> 266.4, x 26
+// 226.1 -> 227.0, 500 x 52 247.4 -> 250.2, molecules of 21: 96 398.9 -> 389.4, 190 (7.3) 513.3 -> 499.1, 240 617 -> 597; 96 190 molecules 216.1 ->
+// 211.2, (7.3) 206.9 -> 206.7; 192 190 molecules (7.3) 394.6 -> 385.5.
+inline int64_t min_nodes_per_workgroup(int channels) {
+  switch (channels) {
+    case 32: return 60;
+    case 160: return 44;
+    case 192: return 58;
+    case 224: return 43;
+    case 256: return 69;
+    default: return 76;
+  }
+}
 inline int64_t min_edges(int64_t nnodes, int channels) {
   struct Line {
     int64_t cached;             // edges, while the output fits the last-level cache
@@ -107,12 +121,12 @@ inline int64_t min_edges(int64_t nnodes, int channels) {
     switch (channels) {
       case 32: return {0, 0.0, 0.0};
       case 64: return {26000, 0.0, 0.0};
-      case 96: return {std::max(34000 + 6 * nnodes / 5, 5 * nnodes), 5.5, 2.0};
+      case 96: return {std::max(28000 + 6 * nnodes / 5, 5 * nnodes), 5.5, 2.0};
       case 128: return {std::max(24000 + 2 * nnodes, 9 * nnodes / 2), 7.0, 3.2};
       case 160: return {std::max(3500 + 7 * nnodes / 2, 21 * nnodes / 5), 6.5, 2.5};
-      case 192: return {std::max(4000 + 11 * nnodes / 2, 15 * nnodes / 2), 9.0, 1.9};
-      case 224: return {std::max(8000 + 3 * nnodes, 9 * nnodes / 2), 6.0, 1.5};
-      default: return {std::max(5000 + 23 * nnodes / 4, 21 * nnodes / 2), 11.0, 2.0};
+      case 192: return {std::max(4000 + 11 * nnodes / 2, 7 * nnodes), 9.0, 1.9};
+      case 224: return {std::max(7000 + 3 * nnodes, 9 * nnodes / 2), 6.0, 1.5};
+      default: return {nnodes <= 5000 ? 5000 + 23 * nnodes / 4 : 21 * nnodes / 2, 11.0, 2.0};  // (82 MB of output)
     }
   }();
   const double caches = 64.0 * static_cast<double>(nnodes) * channels / (1 << 28);  // 16 components of 4 bytes in 256 MB
