@@ -9,6 +9,8 @@
 // 64 edges are staged through LDS with coalesced row reads.  No atomics anywhere: partial sums
 // of the slots are combined with cross-lane moves in a fixed order, so results are reproducible
 // bit for bit.
+#include <algorithm>
+
 #include "mp_common.hpp"
 
 namespace cm {
@@ -318,7 +320,7 @@ __device__ __forceinline__ void arrived(T &v) {
 }
 
 //
-// MULTI (few senders, see parts_for): a workgroup of up to eight waves per sender, each on a part of the sender's range;
+// MULTI (few senders, see sender_parts): a workgroup of up to eight waves per sender, each on a part of the sender's range;
 // the parts' sums are added by the first wave in the order of the parts.
 template <int C, int LIVE, bool MULTI>
 __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave) void mp_backward_sender_kernel(
@@ -513,10 +515,20 @@ int launch_backward(const float *X, const float *Y, const float *R, const float 
   return rc;
 }
 
+// Waves per sender: four rows each while they fit three rounds of half a chip's waves (a row is one load, and what a wave waits for is
+// its list and its first rows).  us of edge and sender pass at 1 2 3 4 6 8, the rule's in brackets: 128 channels 216 x 52 21.2 17.9 16.7 16.4
+// 15.7 [15.8], 700 x 52 34.8 31.2 30.4 [30.5] 31.3 30.9, 1 500 x 52 53.6 [52.4] 52.3 52.2 53.9 53.4, 672 x 9 14.5 [13.8] 13.9 14.3 15.1 15.4;
+// 256 60 x 30 20.1 15.9 14.4 13.6 [12.8] 13.0, 216 x 52 36.8 30.5 27.7 26.9 25.1 [25.0], 300 x 9 15.7 [14.5] 14.0 14.1 14.9 15.2; 64 21 x 19 8.6
+// 8.1 8.3 [8.4] 8.6 8.8.
+inline int sender_parts(int64_t nnodes, int64_t nedges) {
+  if (nnodes <= 0) return 1;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(8, std::min(3072 / nnodes, nedges / (4 * nnodes)))));
+}
+
 template <int C>
 int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes, int64_t nedges,
                   float *gX, hipStream_t st, const float *live_vec, const float *live_r, float r_max) {
-  const int parts = parts_for(nnodes, nedges);
+  const int parts = sender_parts(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes)), block(parts * kWave);
 #define CM_SENDER(LIVE_, by_, rmax_)                                                                                                   \
   do {                                                                                                                                 \

@@ -332,10 +332,20 @@ __global__ __launch_bounds__(kWave) void mp_backward_sender_f64_kernel(const dou
   }
 }
 
+// Parts a node's edge range is cut into where one wave per node would leave most of the device idle (a 216-atom cell is
+// 216 waves for 1 024 SIMDs, each walking its ~90 edges one after the other): as many as fill about 2 048 wave slots
+// and leave a part a dozen edges on average, at most 8.
+inline int parts_for(int64_t nnodes, int64_t nedges) {
+  if (nnodes <= 0) return 1;
+  const int64_t by_slots = 2048 / nnodes, by_edges = nedges / (12 * nnodes);
+  const int64_t parts = by_slots < by_edges ? by_slots : by_edges;
+  return parts < 1 ? 1 : (parts > 8 ? 8 : static_cast<int>(parts));
+}
+
 template <int SW>
 void launch_forward(const double *X, const double *Y, const double *R, const int32_t *sender, const int32_t *first_occ, int64_t nnodes,
                     int64_t nedges, int C, double *out, hipStream_t st) {
-  const int parts = std::min(mp::parts_for(nnodes, nedges), 4);  // a wave's 16 x 4 fp64 sums leave room for four waves per workgroup
+  const int parts = std::min(parts_for(nnodes, nedges), 4);  // a wave's 16 x 4 fp64 sums leave room for four waves per workgroup
   hipLaunchKernelGGL(mp_forward_f64_kernel<SW>, dim3(static_cast<unsigned>(nnodes)), dim3(parts * kWave),
                      static_cast<unsigned>(parts * kForwardLdsPerWave), st, X, Y, R, sender, first_occ, static_cast<int>(nnodes), nedges,
                      C, out);
@@ -345,7 +355,7 @@ template <int SW, bool GY, bool GR, bool GX>
 void launch_edge(const double *X, const double *Y, const double *R, const double *G, const int32_t *sender,
                  const int32_t *first_occ, int64_t nnodes, int64_t nedges, int C, double *gY, double *gR, double *gXe,
                  hipStream_t st) {
-  const int parts = mp::parts_for(nnodes, nedges);
+  const int parts = parts_for(nnodes, nedges);
   hipLaunchKernelGGL((mp_backward_edge_f64_kernel<SW, GY, GR, GX>), dim3(static_cast<unsigned>(nnodes), parts), dim3(kWave), 0, st,
                      X, Y, R, G, sender, first_occ, static_cast<int>(nnodes), nedges, C, gY, gR, gXe);
 }
