@@ -14,7 +14,8 @@
 // a single launch; per-element weights are selected through a node permutation that lists the nodes group
 // by group, without any host synchronisation.
 //
-// Arithmetic (the two kernels with resident weights at the end of this file have their own): every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
+// Arithmetic (the kernels with resident weights and the one with a workgroup per 128 rows, at the end of this file, have their own, the one for
+// few rows multiplies fp32 values): every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
 // in all), and the product is accumulated in fp32 from the six piece products that matter (hi.hi, hi.mid, mid.hi, hi.lo,
 // lo.hi, mid.mid; the dropped ones are below 2^-24 of the product) on v_mfma_f32_32x32x16_bf16, whose rate is 16x that of
 // the fp32 matrix instruction.  The result matches an fp32 GEMM to rounding (measured rms error 1.7e-7 against fp64 on

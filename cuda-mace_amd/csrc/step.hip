@@ -112,25 +112,15 @@ __global__ void copy_or_zero_f64_kernel(double *p, const double *src, int64_t n)
 __device__ __forceinline__ int walk_back_to_live_edge(const double *__restrict__ pos, const int32_t *__restrict__ a,
                                                       const int32_t *__restrict__ b, const double *__restrict__ shifts,
                                                       const int32_t *__restrict__ rows, int nnodes, float r_max, int e0, int e) {
-  constexpr int kAhead = 4;  // edges per trip, their operands requested together
-  bool found = false;
-  while (e > e0 && !found) {
-    float len[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int64_t q = max(e - 1 - u, e0);  // below the range: the first edge again, never looked at
-      double w[3];
-      edge_vector_f64(pos, a, b, shifts, rows, q, nnodes, w);
-      len[u] = mp::edge_length(static_cast<float>(w[0]), static_cast<float>(w[1]), static_cast<float>(w[2]));
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      if (found || e <= e0) continue;
-      if (len[u] <= r_max)
-        found = true;
-      else
-        --e;
-    }
+  // by the whole wave, 64 edges per trip, with the same arguments in every lane: one past the last live edge of e0 .. e - 1, or e0
+  while (e > e0) {
+    const int q = e - 1 - static_cast<int>(threadIdx.x % kWave);
+    double w[3];
+    edge_vector_f64(pos, a, b, shifts, rows, max(q, e0), nnodes, w);
+    const bool live = q >= e0 && mp::edge_length(static_cast<float>(w[0]), static_cast<float>(w[1]), static_cast<float>(w[2])) <= r_max;
+    const unsigned long long lives = __ballot(live);
+    if (lives != 0) return e - (__ffsll(static_cast<long long>(lives)) - 1);
+    e = max(e - kWave, e0);
   }
   return e;
 }
@@ -169,13 +159,15 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
   const unsigned long long inside_mask = __ballot(inside);
   if (lane == 0) s_inside[wave] = inside_mask;
   __syncthreads();
-  if (i < nedges && recv != next_recv && static_cast<unsigned>(recv) < static_cast<unsigned>(nnodes)) {
-    int e0 = first_occ[recv], e1 = first_occ[nnodes + recv];
+  const bool closes = i < nedges && recv != next_recv && static_cast<unsigned>(recv) < static_cast<unsigned>(nnodes);
+  int e0 = 0, e = -1, from = 0;  // from: where the walk begins if the ballots do not settle it
+  if (closes) {
+    int e1 = first_occ[nnodes + recv];
+    e0 = first_occ[recv];
     clamp_edge_range(e0, e1, nedges);
-    int e;
+    from = e1;
     if (e1 == i + 1) {  // this is the last edge of the receiver's range, as in every sorted list
       const int64_t group_first = i - threadIdx.x;  // first edge of the workgroup
-      e = -1;
       // the node's edges in this workgroup, from this wave down: the highest one inside the cutoff
       for (int w = wave; w >= 0 && e < 0; --w) {
         const int64_t wave_first = group_first + w * kWave;
@@ -186,12 +178,17 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
         const unsigned long long mine = s_inside[w] & upto & ~((1ull << lo) - 1ull);
         if (mine != 0) e = static_cast<int>(wave_first) + (63 - __clzll(static_cast<long long>(mine))) + 1;
       }
-      if (e < 0)
-        e = e0 >= group_first ? e0
-                              : walk_back_to_live_edge(pos, a, b, shifts, rows, nnodes, r_max, e0, static_cast<int>(group_first));
-    } else {
-      e = walk_back_to_live_edge(pos, a, b, shifts, rows, nnodes, r_max, e0, e1);
+      if (e < 0 && e0 >= group_first) e = e0;
+      from = static_cast<int>(group_first);
     }
+  }
+  // what is left, a node at a time, by all lanes (every lane of the wave arrives here)
+  for (unsigned long long left = __ballot(closes && e < 0); left != 0; left &= left - 1) {
+    const int of = __ffsll(static_cast<long long>(left)) - 1;
+    const int found = walk_back_to_live_edge(pos, a, b, shifts, rows, nnodes, r_max, __builtin_amdgcn_readlane(e0, of), __builtin_amdgcn_readlane(from, of));
+    if (lane == of) e = found;
+  }
+  if (closes) {
     live[recv] = e0;
     live[nnodes + recv] = e;
   }

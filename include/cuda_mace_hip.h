@@ -480,7 +480,7 @@ int cm_graph_prepare(const double *positions, const int32_t *row_i, const int32_
  * The three [nnodes, C] x [C, C] linears between the two interaction layers as one launch per direction: the product's
  * linear and linear_up (the reference's linear_matmul, models/InvariantMACE.py:41-53) and the per-element skip
  * connection between them (element_linear_to_cuda, :56-74; called at :145-150 and :330).  A workgroup takes a tile of nodes
- * of one element through the chain with the intermediate rows in LDS (few nodes at 96 and 128 channels: two launches); same
+ * of one element through the chain with the intermediate rows on chip (few nodes at 96 and 128 channels: two launches); same
  * arithmetic, rounding points and results as the three cm_linear calls it stands for.  channels = 32, 64, 96 or 128 (cm_node_glue_supported).
  *   node_perm / group_offsets: nodes grouped by element, ngroups = nelements + 1 with the last group holding the nodes
  *   without an element (their skip connection is zero), as cm_linear takes them with zero_last_group.
@@ -505,7 +505,7 @@ int cm_node_glue_backward(const float *gX2, const float *d_h2, const float *up_W
  * Python forward over its TorchScript classes followed by an autograd backward (models/InvariantMACE.py:246-379:
  * interactions :76-160, products :330, readouts :336, scale/shift :344, forces through get_outputs :354): same kernels,
  * same order, same numbers as that sequence, without a Python interpreter or an autograd engine between the launches
- * (16 launches up to 128 channels, 18 with few nodes at 96 and 128, 23 beyond; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
+ * (16 launches up to 128 channels, 18 with few nodes at 96 and 128, 23 beyond, 20 with few nodes; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
  *
  * cm_mace_weights: the model's frozen weights in the layouts the op modules hold them (device pointers).
  *   spline[t]      [nknots - 1, 4, 4C]   radial spline table of layer t (cm_spline_forward's coeffs)
@@ -603,7 +603,7 @@ int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double
  * per graph may differ from its in the last bits (up to 128 channels the full step forms them in another launch, with
  * another number of partial sums).  No backward chain runs, nothing that only it reads is written, and the workspace,
  * cm_mace_energy_workspace(nnodes, nedges, channels) bytes, has no room for it (a workspace of cm_mace_step will do as well).
- * 10 launches up to 128 channels (11 with few nodes at 96 and 128), 13 beyond.  For callers that compare energies: Monte Carlo moves, screening. */
+ * 10 launches up to 128 channels (11 with few nodes at 96 and 128), 13 beyond (12 with few nodes).  For callers that compare energies: Monte Carlo moves, screening. */
 size_t cm_mace_energy_workspace(int64_t nnodes, int64_t nedges, int channels);
 int cm_mace_energy(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
                    void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy, double *node_feats,

@@ -529,8 +529,8 @@ def test_linear_many_rows(cabi, N, C, ne, seed):
 @pytest.mark.parametrize("N,C,ne,seed", [(2048, 160, 1, 0), (2500, 192, 10, 1), (2063, 224, 5, 2), (3001, 256, 3, 3), (4100, 192, 40, 4),
                                          (9000, 160, 2, 5), (2049, 256, 130, 6)])
 def test_linear_many_rows_wide(cabi, N, C, ne, seed):
-    """The same at 160 to 256 columns, where from 2 048 nodes on the weights stay in registers and the workgroup's waves share
-    16-row tiles."""
+    """The same at 160 to 256 columns, where beyond one or two rounds of workgroups the weights stay in registers and the workgroup's waves
+    share 16-row tiles."""
     test_linear_many_rows(cabi, N, C, ne, seed)
 
 
