@@ -282,7 +282,10 @@ __global__ __launch_bounds__(kWave) void mp_backward_edge_kernel(
 // backward, sender pass: gX[n, :] = sum over the edges sent by n of the per-edge contributions
 // -----------------------------------------------------------------------------------------------
 // LIVE: 0 = every row of gXe is read; 1 / 2 = only rows of edges within r_max, by the edge vector / the edge length
-// (the spline-fused edge pass writes no others).
+// (the spline-fused edge pass writes no others); 3 = the same by a bit per edge, which the step's geometry launch leaves: a random 12 bytes
+// per edge were 64 from memory, a tenth of what the pass fetches, the bits (160 KB at 25 000 x 52) stay in L2
+// (vectors -> bits, us: 25 000 x 52 x 128 126 -> 112, with a quarter of the list beyond the cutoff 148 -> 130, 100 000 x 192 847 -> 734, 5 000 x 96
+// 24.9 -> 20.5).
 //
 // A slot (the lanes that carry one row) takes four edges per iteration.  Three loads depend on each other per edge --
 // its index from the sender-sorted view, its vector or length (LIVE), its row -- so the loop is pipelined over
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave) void mp_backward_sender_
     const int emax = static_cast<int>(nedges - 1);
     int e_cur[B], e_nxt[B], e_aft[B];   // indices of batches i, i + 1 (arrived) and i + 2 (being loaded)
     f3 lv_cur[B], lv_nxt[B];    // LIVE 1: vectors of batch i (arrived) and i + 1 (being loaded)
-    float lr_cur[B], lr_nxt[B];  // LIVE 2: lengths of the same
+    float lr_cur[B], lr_nxt[B];  // LIVE 2: lengths of the same; LIVE 3: words of the bit array they have their bit in
     f4 rows4[B];                        // rows of the previous batch (four channels per lane: one 16-byte load)
     float rowsf[B][K::V];               // the same for the other channel counts per lane (dword loads)
     bool take[B];
@@ -367,7 +370,7 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave) void mp_backward_sender_
         for (int j = 0; j < B; ++j) {
           const int ec = min(max(e[j], 0), emax);
           if constexpr (LIVE == 1) issue_load(lv_nxt[j], live_by + 3 * static_cast<int64_t>(ec));
-          else issue_load(lr_nxt[j], live_by + ec);
+          else issue_load(lr_nxt[j], live_by + (LIVE == 3 ? ec >> 5 : ec));
         }
       }
     };
@@ -418,7 +421,7 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave) void mp_backward_sender_
       for (int j = 0; j < B; ++j) {
         arrived(e_aft[j]);
         if constexpr (LIVE == 1) arrived(lv_nxt[j]);
-        if constexpr (LIVE == 2) arrived(lr_nxt[j]);
+        if constexpr (LIVE >= 2) arrived(lr_nxt[j]);
       }
     };
 
@@ -446,13 +449,14 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave) void mp_backward_sender_
         e_cur[j] = e_nxt[j];
         e_nxt[j] = e_aft[j];
         if constexpr (LIVE == 1) lv_cur[j] = lv_nxt[j];
-        if constexpr (LIVE == 2) lr_cur[j] = lr_nxt[j];
+        if constexpr (LIVE >= 2) lr_cur[j] = lr_nxt[j];
       }
 #pragma unroll
       for (int j = 0; j < B; ++j) {
         bool ok = (k + j * K::EPW < k1) & (static_cast<unsigned>(e_cur[j]) <= static_cast<unsigned>(emax));
         if constexpr (LIVE == 1) ok = ok & (edge_length(lv_cur[j].x, lv_cur[j].y, lv_cur[j].z) <= r_max);
         if constexpr (LIVE == 2) ok = ok & (lr_cur[j] <= r_max);
+        if constexpr (LIVE == 3) ok = ok & ((__float_as_uint(lr_cur[j]) >> (e_cur[j] & 31) & 1u) != 0);
         take[j] = ok;
         good = ok ? e_cur[j] : good;
         e_cur[j] = ok ? e_cur[j] : good;
@@ -527,7 +531,7 @@ inline int sender_parts(int64_t nnodes, int64_t nedges) {
 
 template <int C>
 int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes, int64_t nedges,
-                  float *gX, hipStream_t st, const float *live_vec, const float *live_r, float r_max) {
+                  float *gX, hipStream_t st, const float *live_vec, const float *live_r, float r_max, const uint32_t *live_bits) {
   const int parts = sender_parts(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes)), block(parts * kWave);
 #define CM_SENDER(LIVE_, by_, rmax_)                                                                                                   \
@@ -539,7 +543,9 @@ int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets,
       hipLaunchKernelGGL((mp_backward_sender_kernel<C, LIVE_, false>), grid, block, 0, st, gXe, perm, offsets,                         \
                          static_cast<int>(nnodes), nedges, by_, rmax_, gX);                                                            \
   } while (0)
-  if (live_vec)
+  if (live_bits)
+    CM_SENDER(3, reinterpret_cast<const float *>(live_bits), 0.f);
+  else if (live_vec)
     CM_SENDER(1, live_vec, r_max);
   else if (live_r)
     CM_SENDER(2, live_r, r_max);
@@ -553,9 +559,9 @@ int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets,
 
 int mp::launch_sender_pass(int channels, const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes,
                            int64_t nedges, float *gX, hipStream_t st, const float *live_vec, const float *live_r,
-                           float r_max) {
+                           float r_max, const uint32_t *live_bits) {
   int rc = CM_EINVAL;
-  CM_DISPATCH_C(channels, rc = launch_sender<C_>(gXe, perm, offsets, nnodes, nedges, gX, st, live_vec, live_r, r_max));
+  CM_DISPATCH_C(channels, rc = launch_sender<C_>(gXe, perm, offsets, nnodes, nedges, gX, st, live_vec, live_r, r_max, live_bits));
   return rc;
 }
 

@@ -269,10 +269,10 @@ __device__ __forceinline__ float edge_length(float v0, float v1, float v2) {
 
 // Sender pass of the backward, shared by both variants (defined in mp.hip).  With live_vec (edge vectors [E, 3]) or
 // live_r (edge lengths [E]) given, only the rows of edges within r_max are read: the spline-fused edge pass writes no
-// others.
+// others.  live_bits (bit e % 32 of word e / 32: edge e is within r_max) in place of either.
 int launch_sender_pass(int channels, const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes,
                        int64_t nedges, float *gX, hipStream_t st, const float *live_vec = nullptr,
-                       const float *live_r = nullptr, float r_max = 0.f);
+                       const float *live_r = nullptr, float r_max = 0.f, const uint32_t *live_bits = nullptr);
 
 // Forward from edge vectors with the radial table in LDS, two degrees and one 16-channel slice per workgroup (defined in
 // mp_sliced.hip): whether it takes a launch of this shape, and the launch.  records: NULL, or per edge 16 bytes, the vector and
@@ -286,6 +286,13 @@ int launch_sliced_forward(const float *X, const float *vec, const void *records,
 // cm_mp_edge_forward of a caller that has written records (defined in mp_spline.hip; operands already checked by the caller).
 int edge_forward_from_records(const float *X, const void *records, const float *r_knots, const float *coeffs, int nknots, float r_width,
                               float r_max, const int32_t *first_occ, int64_t nnodes, int64_t nedges, int channels, float *out, hipStream_t st);
+
+// cm_mp_edge_backward with gX of a caller that has a bit per edge within r_max (or NULL), for the sender pass (defined in mp_spline.hip;
+// operands already checked by the caller).
+int edge_backward_with_live_bits(const float *X, const float *vectors, const float *r_knots, const float *coeffs, int nknots, float r_width,
+                                 float r_max, const float *grad_out, const int32_t *sender, const int32_t *first_occ, const int32_t *sender_perm,
+                                 const int32_t *sender_offsets, int64_t nnodes, int64_t nedges, int channels, float *gX, float *grad_vectors,
+                                 float *edge_scratch, const uint32_t *live_bits, hipStream_t st);
 
 // The spline-fused backward edge pass from edge vectors without gX, writing (this layer's vector gradient + addend[e])
 // (defined in mp_spline.hip; operands as cm_mp_edge_backward, already checked by the caller).

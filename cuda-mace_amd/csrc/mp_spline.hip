@@ -46,6 +46,7 @@ struct Spline {
   int nknots;
   float r_width;
   float r_max;
+  const uint32_t *live_bits = nullptr;  // backward with gX: a bit per edge within r_max, or NULL (the sender pass then looks at vec or r)
 };
 
 // Knot interval (or -1 beyond the cutoff) and offset inside it for one edge length.  lds_knots: a copy of the knots in LDS,
@@ -969,7 +970,7 @@ int launch_backward(const float *X, const float *Y, const Spline &sp, const floa
   int rc = check_launch(FROM_VEC ? "cm_mp_edge_backward (edge pass)" : "cm_mp_spline_backward (edge pass)");
   if (rc != CM_OK) return rc;
   if (gX) rc = mp::launch_sender_pass(C, gXe, perm, offsets, nnodes, nedges, gX, st, FROM_VEC ? sp.vec : nullptr,
-                                      FROM_VEC ? nullptr : sp.r, sp.r_max);
+                                      FROM_VEC ? nullptr : sp.r, sp.r_max, sp.live_bits);
   return rc;
 }
 
@@ -1066,6 +1067,20 @@ int edge_forward_from_records(const float *X, const void *records, const float *
   const int rc = check_spline("cm_mace_step", static_cast<const float *>(records), r_knots, coeffs, nknots, r_width, nedges, nnodes, channels);
   if (rc != CM_OK) return rc;
   return launch_sliced_forward(X, nullptr, records, r_knots, coeffs, nknots, r_width, r_max, nullptr, first_occ, nnodes, nedges, channels, out, st);
+}
+
+int edge_backward_with_live_bits(const float *X, const float *vectors, const float *r_knots, const float *coeffs, int nknots, float r_width,
+                                 float r_max, const float *grad_out, const int32_t *sender, const int32_t *first_occ, const int32_t *sender_perm,
+                                 const int32_t *sender_offsets, int64_t nnodes, int64_t nedges, int channels, float *gX, float *grad_vectors,
+                                 float *edge_scratch, const uint32_t *live_bits, hipStream_t st) {
+  if (nnodes == 0) return CM_OK;
+  int rc = check_spline("cm_mace_step", vectors, r_knots, coeffs, nknots, r_width, nedges, nnodes, channels);
+  if (rc != CM_OK) return rc;
+  const Spline sp{vectors, nullptr, r_knots, coeffs, nknots, r_width, r_max, live_bits};
+  rc = CM_EINVAL;
+  CM_DISPATCH_C(channels, rc = (launch_backward<C_, true>(X, nullptr, sp, grad_out, sender, first_occ, sender_perm, sender_offsets, nnodes, nedges,
+                                                          gX, grad_vectors, nullptr, edge_scratch, st)));
+  return rc;
 }
 
 // cm_mp_edge_backward without gX whose vector gradient is written as (this layer's gradient + addend[e]): saves the pass

@@ -100,7 +100,7 @@ __global__ void copy_or_zero_f64_kernel(double *p, const double *src, int64_t n)
 // arithmetic of cm_edge_geometry_forward), writes it as the row of `vec` the backward chain reads and, for the forward kernel with
 // the table in LDS, as a record of 16 bytes with the sender (either may be NULL), and, where a backward chain follows (gv1 and gv2 given), clears the vector
 // gradients of an edge beyond the cutoff (the backward edge passes skip the edges behind a node's mark, and write the same
-// zeros for those before it).  The thread of a receiver's
+// zeros for those before it), and leaves a bit per edge inside the cutoff for the sender pass (live_bits, may be NULL).  The thread of a receiver's
 // last edge closes the receiver's range: live[n] = first_occ[n], live[nnodes + n] = one past the last edge e of the node
 // with |vec[e]| <= r_max (the node's first edge if there is none).  The message-passing kernels, forward and backward,
 // skip the edges behind that mark, which contribute exact zeros.  A Verlet list holds a third more pairs than the cutoff
@@ -130,7 +130,8 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
                                                                   const int32_t *__restrict__ rows, const int32_t *__restrict__ first_occ,
                                                                   float r_max, int nnodes, int64_t nedges, float *__restrict__ vec,
                                                                   float4 *__restrict__ records, int32_t *__restrict__ live,
-                                                                  float *__restrict__ gv1, float *__restrict__ gv2) {
+                                                                  float *__restrict__ gv1, float *__restrict__ gv2,
+                                                                  unsigned long long *__restrict__ live_bits) {
   const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   const int lane = threadIdx.x % kWave;
   bool inside = false;
@@ -157,7 +158,10 @@ __global__ __launch_bounds__(256) void geometry_live_range_kernel(const double *
   __shared__ unsigned long long s_inside[4];
   const int wave = threadIdx.x / kWave;
   const unsigned long long inside_mask = __ballot(inside);
-  if (lane == 0) s_inside[wave] = inside_mask;
+  if (lane == 0) {
+    s_inside[wave] = inside_mask;
+    if (live_bits && i < nedges) live_bits[i / kWave] = inside_mask;
+  }
   __syncthreads();
   const bool closes = i < nedges && recv != next_recv && static_cast<unsigned>(recv) < static_cast<unsigned>(nnodes);
   int e0 = 0, e = -1, from = 0;  // from: where the walk begins if the ballots do not settle it
@@ -345,6 +349,7 @@ struct Layout {
   float *B1, *h1, *sc, *X2, *B2, *h2, *d_h2, *g1, *gB, *gX2, *gh1a, *gh1;
   int32_t *live;         // [2 N] edge ranges cut back to the last edge inside the cutoff
   double *node_virial;   // [N, 6]
+  uint32_t *live_bits;   // a bit per edge inside the cutoff, until the virials are written to the same place; NULL where they do not fit it
   size_t bytes;
 
   Layout(void *base, int64_t N, int64_t E, int C, bool forces) {
@@ -371,6 +376,7 @@ struct Layout {
     g1 = backward(NC), gB = backward(NC), gX2 = backward(NC), gh1a = backward(NC), gh1 = backward(NC);
     live = reinterpret_cast<int32_t *>(take(static_cast<size_t>(2 * N) * sizeof(int32_t)));
     node_virial = forces ? reinterpret_cast<double *>(take(static_cast<size_t>(6 * N) * sizeof(double))) : nullptr;
+    live_bits = forces && E > 0 && (E + kWave - 1) / kWave <= 6 * N ? reinterpret_cast<uint32_t *>(node_virial) : nullptr;
     bytes = at;
   }
 };
@@ -505,7 +511,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
     hipLaunchKernelGGL(cm::geometry_live_range_kernel, dim3(static_cast<unsigned>(cm::ceil_div(std::max(N, E), 256))), dim3(256), 0, st,
                        positions, g->receiver, g->sender, shifts, g->node_rows, g->first_occ, w->r_max, static_cast<int>(N), E,
                        want_forces || !records ? L.vec : nullptr, records ? reinterpret_cast<float4 *>(L.records) : nullptr, L.live, L.gv1,
-                       L.gv2);
+                       L.gv2, reinterpret_cast<unsigned long long *>(L.live_bits));
   }
   const int32_t *fo_live = E > 0 ? L.live : g->first_occ;
   const float *X[2] = {g->X1, L.X2};
@@ -579,8 +585,9 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   if (!glue)
     CM_STAGE(14, cm_linear(L.d_h2, w->prod_W[1], nullptr, nullptr, N, 1, 0, 1, C, C, -1.0f, none, none, L.gB, stream));
   CM_STAGE(15, cm_linear(L.bufM2, w->mix_W[1], nullptr, nullptr, N, 1, 0, 16, C, C, w->mix_scale[1], L.gB, none, L.bufA, stream));
-  CM_STAGE(16, cm_mp_edge_backward(L.X2, L.vec, w->r_knots, w->spline[1], w->nknots, w->r_width, w->r_max, L.bufA, g->sender,
-                              fo_live, g->sender_perm, g->sender_offsets, N, E, C, L.gX2, L.gv2, L.edge_scratch, stream));
+  CM_REQUIRE(E < INT32_MAX / 3, "cm_mace_step: number of edges out of range");
+  CM_STAGE(16, cm::mp::edge_backward_with_live_bits(L.X2, L.vec, w->r_knots, w->spline[1], w->nknots, w->r_width, w->r_max, L.bufA, g->sender, fo_live,
+                                                    g->sender_perm, g->sender_offsets, N, E, C, L.gX2, L.gv2, L.edge_scratch, L.live_bits, st));
   // layer 0 (first interaction): its input features depend on the species alone, so no gradient with respect to them
   if (glue || cut_backward) {
     CM_STAGE(17, cm::node_glue_backward_with_energy_sums(L.gX2, L.d_h2, w->up_W, w->skip_W, w->prod_W[0], w->w1, w->scale, g->node_weights,
