@@ -773,6 +773,47 @@ __device__ __forceinline__ void first_tiles(const int32_t *__restrict__ group_of
   }
 }
 
+// A workgroup's piece of the list of all tiles, tiles [first, last).  With row_scale (SCALED) the 2 l + 1 tiles of a node tile share its
+// row_scale rows: a node tile of l = 0 fetches and multiplies them for one tile, of l = 3 for seven, and with pieces of as many tiles each the
+// launch waited for those of l = 0.  A node tile counts 2 l + 1 + 1/2 there (a quarter: the same within 2 %).  us, shared weights / ten
+// weight groups, equal pieces -> these: 12 000 x 64 23.8 / 25.3 -> 22.5 / 25.2, 60 000 x 64 97.5 / 99.8 -> 91.0 / 93.5, 12 000 x 128 46.2 / 51.2 ->
+// 42.6 / 46.1, 25 000 x 128 91.2 / 94.7 -> 84.1 / 85.8 (73 / 82 without row_scale), 60 000 x 128 226 / 238 -> 211 / 216, 12 000 x 192 77.3 /
+// 88.0 -> 72.6 / 80.7, 100 000 x 192 653 / 657 -> 594 / 603, 100 000 x 256 800 / 877 -> 787 / 814.  With one weight block per l an l
+// gets whole workgroups, so that none of them stages two blocks; with more, where pieces cross blocks anyway, the workgroups of
+// an XCD take neighbouring pieces, whose rows of row_scale meet in its L2 (25 000 x 128 94.7 -> 92.7 of the above).  An XCD for an eighth of the
+// nodes with shared weights: 88.1 with the nearest whole workgroups, 3 : 6 : 10 : 13 of 32.
+// Steps: 25 000 x 128 2 180 -> 2 159, dynamics of it 55.6 -> 55.1 ms, 100 000 x 192 13.74 -> 13.69.
+struct Share {
+  int first, last;
+};
+constexpr int kXcds = 8;
+template <bool SCALED, int COMP>
+__device__ __forceinline__ Share own_share(const int *cum, int ngroups) {
+  const auto whole = [](int64_t n, int index, int of) { return static_cast<int>(n * index / of); };
+  const int of = gridDim.x, index = blockIdx.x, ntiles = cum[ngroups];
+  if constexpr (!SCALED || COMP != 16) return {whole(ntiles, index, of), whole(ntiles, index + 1, of)};
+  const auto cost_before = [](int l) { return 2 * l * l + l; };  // of the l blocks before l, per node tile, in half tiles
+  constexpr int kCost = 36;                                      // = cost_before(4)
+  if (ngroups == 1 && of >= kCost) {
+    int l = 0, first = 0, end = (of * cost_before(1) + kCost / 2) / kCost;  // workgroups [first, end) have l
+    while (index >= end) ++l, first = end, end = (of * cost_before(l + 1) + kCost / 2) / kCost;
+    const int before = ntiles / 16 * l * l, tiles = ntiles / 16 * (2 * l + 1);
+    return {before + whole(tiles, index - first, end - first), before + whole(tiles, index + 1 - first, end - first)};
+  }
+  const auto tile_at = [&](int piece) {
+    int64_t cost = static_cast<int64_t>(ntiles / 16) * kCost * piece / of;
+    int g = 0, l = 0;
+    while (g < ngroups - 1 && static_cast<int64_t>(cum[g + 1] / 16) * kCost <= cost) ++g;
+    cost -= static_cast<int64_t>(cum[g] / 16) * kCost;
+    const int64_t tiles = (cum[g + 1] - cum[g]) / 16;
+    while (l < 3 && tiles * cost_before(l + 1) <= cost) ++l;
+    const int64_t in_l = (cost - tiles * cost_before(l)) * (2 * l + 1) / (cost_before(l + 1) - cost_before(l));
+    return static_cast<int>(cum[g] + min(tiles * (l * l) + in_l, tiles * 16));
+  };
+  const int piece = of % kXcds == 0 ? index % kXcds * (of / kXcds) + index / kXcds : index;
+  return {tile_at(piece), tile_at(piece + 1)};
+}
+
 using rows::largest4;
 // largest value over eight neighbouring lanes, in all of them
 __device__ __forceinline__ float max_over_8(float v) {
@@ -825,9 +866,9 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
   }
   __syncthreads();
 
-  const int ntiles = sCum[ngw];
-  const int i1 = static_cast<int>(static_cast<int64_t>(ntiles) * (blockIdx.x + 1) / gridDim.x);
-  int i = static_cast<int>(static_cast<int64_t>(ntiles) * blockIdx.x / gridDim.x);
+  const Share share = own_share<SCALED, 16>(sCum, ngw);
+  const int i1 = share.last;
+  int i = share.first;
   int g = 0, staged_g = -1, staged_l = -1;
 
   while (i < i1) {
@@ -1151,9 +1192,9 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
   const unsigned raw_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sRaw)) + wave * (kWave * 16);
   const unsigned scale_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sScale)) + wave * (kWave * 16);
 
-  const int ntiles = sCum[ngw];
-  const int i1 = static_cast<int>(static_cast<int64_t>(ntiles) * (blockIdx.x + 1) / gridDim.x);
-  int i = static_cast<int>(static_cast<int64_t>(ntiles) * blockIdx.x / gridDim.x);
+  const Share share = own_share<SCALED, COMP>(sCum, ngw);
+  const int i1 = share.last;
+  int i = share.first;
   int g = 0, held_g = -1, held_l = -1;
   f16x8 w[CB][KS][2];  // weight pieces: column block, k step, piece
   f4 column[CB];       // what takes the weight columns' scales back, of the four columns whose sums a lane gets

@@ -570,6 +570,30 @@ def test_scalar_linear_of_a_weight_block(cabi, N, C, ne):
         assert torch.equal(inout, want + d(R))
 
 
+@pytest.mark.parametrize("N,C,sizes", [(8300, 128, None), (12_345, 64, None), (9001, 192, None), (20_000, 256, None),
+                                       (8300, 128, (0, 0, 1, 8000, 0, 17, 282, 0)), (9001, 192, (9001,)), (12_345, 64, (0, 12_300, 0)),
+                                       (9001, 256, (1,) * 100 + (8000, 0, 16)), (10_000, 96, (4000, 0, 0, 6000))])
+def test_linear_pieces_of_the_tile_list_with_row_scale(cabi, N, C, sizes):
+    """With row_scale the kernels with resident weights cut the list of tiles by cost, not by number: shared weights, and weight groups that
+    are empty, tiny or nearly everything, with and without rows of no group.  The scaled rows are X * row_scale in fp32: the same
+    bits as the launch without row_scale gives for that product."""
+    _say("linear_pieces", N, C, sizes)
+    g = torch.Generator().manual_seed(N + C)
+    d = lambda t: t.contiguous().to(DEV)  # noqa: E731
+    X, S = d(torch.randn(N, 16, C, generator=g)), d(torch.randn(N, C, generator=g))
+    if sizes is None:
+        W = d(torch.randn(4, C, C, generator=g))
+        assert torch.equal(cabi.linear(X, W, row_scale=S), cabi.linear(X * S[:, None], W))
+        return
+    W = d(torch.randn(len(sizes), 4, C, C, generator=g))
+    sizes = torch.tensor(sizes + (N - sum(sizes),))
+    elem = torch.arange(len(sizes)).repeat_interleave(sizes)[torch.randperm(N, generator=g)]
+    perm, off = cabi.stable_key_sort(elem.int().to(DEV), len(sizes))
+    out = cabi.linear(X, W, perm, off, zero_last_group=True, row_scale=S)
+    assert torch.equal(out, cabi.linear(X * S[:, None], W, perm, off, zero_last_group=True))
+    assert float(out[(elem == len(sizes) - 1).to(DEV)].abs().sum()) == 0.0
+
+
 @pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256)])
 def test_linear_scales_of_rows_and_columns(cabi, N, C):
     """The kernels with resident weights scale rows of X and columns of W by powers of two: rows and columns multiplied by powers of
