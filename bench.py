@@ -107,21 +107,22 @@ def spline_backward_kernel_name(C, E):
 
 def linear_kernel_name(C, N):
     """The library runs the [N,16,C] channel-mixing linear (one weight group) without tiles for few nodes, with a workgroup per 128
-    rows up to some thousand, and with the weights resident beyond (64, 96 and 128 columns: in LDS, 160 and more: in registers)."""
-    nt = C // 32
+    rows up to some thousand (beyond 128 columns: for one round of workgroups), and with the weights resident beyond (64, 96 and
+    128 columns: in LDS, 160 and more: in registers)."""
+    nt, cus = C // 32, 256
     blocks = (N + 15) // 16 * C
     if blocks <= 3072:
         return "linear_few_rows_kernel<%d,false,%d>" % (C // 16, 1 if blocks <= 1024 else 2)
-    rows = (16 * N + 127) // 128
-    most = 2 * nt if nt <= 6 else nt
-    one_round = 256 // (2 * nt // most)
-    if nt <= 4 and rows <= 4 * 256 or nt >= 5 and (N < 2048 or rows <= (2 if nt <= 6 else 1) * one_round):
-        return "linear_block_kernel<%d,%d,false>" % (nt, most // 2 if nt != 7 and 2 * rows <= one_round else most)
-    if nt in (2, 3, 4):
-        return "linear_resident_kernel<%d,%d,false>" % (C, nt)
-    if nt >= 5:
-        return "linear_wide_kernel<%d,%d,16,false>" % (nt, 2 if nt == 8 else 1)
-    return "linear_kernel<%d,false>" % nt
+    rows, parts = (16 * N + 127) // 128, 1 if nt <= 5 else (4 if nt == 8 else 2)
+    most, per_round = 2 * nt // parts, cus // parts
+    if 2 * rows <= per_round and nt != 7:
+        most //= 2
+    resident = nt > 1 and N >= 2048
+    if rows <= per_round or nt == 1 or resident and (nt < 4 and rows <= 4 * cus or nt == 4 and 3 * cus < 2 * rows <= 4 * cus):
+        return "linear_block_kernel<%d,%d,false>" % (nt, most)
+    if not resident:
+        return ("linear_ring_kernel<%d,false>" if nt >= 7 else "linear_kernel<%d,false>") % nt
+    return "linear_resident_kernel<%d,%d,false>" % (C, nt) if nt <= 4 else "linear_wide_kernel<%d,%d,16,false>" % (nt, 2 if nt == 8 else 1)
 
 
 def mp_algorithmic_bytes(N, E, C):
@@ -566,13 +567,11 @@ def main():
             flops = 32 * N * C * C
             tf = flops / (t_lin * 1e-3) / 1e12
             lin_bytes = 4 * (32 * N * C + 4 * C * C)
-            # resident weights: two fp16 pieces per operand, three products; the others: three bf16 pieces, six
-            pieces = 3 if linear_kernel_name(C, N).startswith(("linear_resident", "linear_wide", "linear_block")) else 6
             others.append(entry(linear_kernel_name(C, N), lin_bytes, t_lin, launches_timed=launches("linear"),
-                                matrix_cores={"fp32_equivalent_TFLOP/s": round(tf, 1), "instruction_TFLOP/s_16_bit": round(pieces * tf, 1),
-                                              "frac_of_16_bit_peak": round(pieces * tf / 2500.0, 4)},
-                                note="[N,16,C] x [C,C] channel mixing: bound by its memory traffic, not by the matrix cores "
-                                     "(every fp32 product is %d products of 16-bit pieces on the matrix cores)" % pieces))
+                                matrix_cores={"fp32_equivalent_TFLOP/s": round(tf, 1), "instruction_TFLOP/s_bf16": round(6 * tf, 1),
+                                              "frac_of_bf16_peak": round(6 * tf / 2500.0, 4)},
+                                note="[N,16,C] x [C,C] channel mixing: every fp32 product is six bf16 piece products on the matrix cores, "
+                                     "whose rate and the memory traffic bound it together"))
             others[-1]["traffic"] = traffic_of(traffic["standalone"], linear_kernel_name(C, N)) if default_workload else None
     else:
         # The model drives the tabulated ops through the TorchScript classes, which the Python-side brackets above do not

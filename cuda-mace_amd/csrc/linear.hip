@@ -14,8 +14,7 @@
 // a single launch; per-element weights are selected through a node permutation that lists the nodes group
 // by group, without any host synchronisation.
 //
-// Arithmetic (the kernels with resident weights and the one with a workgroup per 128 rows, at the end of this file, have their own, the one for
-// few rows multiplies fp32 values): every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
+// Arithmetic (the kernel for few rows multiplies fp32 values): every fp32 operand is split into three bf16 pieces when it is staged (a = hi + mid + lo, 24 mantissa bits
 // in all), and the product is accumulated in fp32 from the six piece products that matter (hi.hi, hi.mid, mid.hi, hi.lo,
 // lo.hi, mid.mid; the dropped ones are below 2^-24 of the product) on v_mfma_f32_32x32x16_bf16, whose rate is 16x that of
 // the fp32 matrix instruction.  The result matches an fp32 GEMM to rounding (measured rms error 1.7e-7 against fp64 on
@@ -705,29 +704,27 @@ __global__ __launch_bounds__(kWaves *kWave, (NT <= 4 ? 2 : 1)) void linear_ring_
 // The kernels above stage the K x Nout weight block again for every tile of 128 rows (as many bytes from L2 as the tile
 // has from HBM) and walk K in barrier-separated phases.  Here a launch has one workgroup per compute unit, and a
 // workgroup takes a contiguous piece of the list of all 16-row tiles, ordered by (weight group, l, node tile, m within
-// l), so that it needs one or two weight blocks in its whole life: it splits a block once into two fp16 planes that
-// cover all of K (70 KB at 128 x 128) and then its eight waves run independently of each other, one 16-row tile at a
+// l), so that it needs one or two weight blocks in its whole life: it splits a block once into three bf16 planes that
+// cover all of K (102 KB at 128 x 128) and then its eight waves run independently of each other, one 16-row tile at a
 // time, with no barrier until the weight block changes.
 //
-// Two fp16 pieces per operand and three piece products on v_mfma_f32_16x16x32_f16 (mfma_split.hpp), rows of X and columns of W
-// scaled by powers of two that the output takes back: half the matrix instructions of three bf16 pieces and six products,
-// four vector instructions per value instead of five and a half, two thirds of the fragment reads.  The products with a low piece
-// have an accumulator of their own, so a sum of K terms is rounded K / 32 times.  us and rms error against fp64 (normal
-// values), bf16 -> fp16: 25 000 x 128 90.4 -> 80.3, 1.65e-7 -> 1.13e-7, with a weight block per element 93.4 -> 85.0, with row_scale 97.9 ->
-// 90.9, 1.68e-7 -> 1.15e-7; 96 columns 1.41e-7 -> 1.07e-7, 64 1.12e-7 -> 1.02e-7, equal times at 5 000 and 10 752 nodes (one
-// accumulator: 1.45e-7 at 128, 1.32e-7 at 96, 1.16e-7 at 64).
+// Two accumulators: the products of the high pieces have one, the five others, below 2^-8 of them, another (mfma_rows.hpp), so a
+// sum of K terms is rounded K / 32 times at its own size.  rms error against fp64 (normal values), one accumulator -> two: 64 columns
+// 1.12e-7 -> 5.0e-8, 96 1.41e-7 -> 5.8e-8, 128 1.65e-7 -> 6.5e-8 (with row_scale 7.4e-8).  Two fp16 pieces of rows and columns scaled to their
+// largest values and three products are faster at 128 columns (25 000 nodes 90 -> 75 us; equal at 64 and 96) but hold an operand to
+// 2^-23 and drop products of 2^-22 (a row of one value: 7.5 2^-24 off), and a value 2^-20 of its row's largest has 19 bits left: not fp32.
 //
-// Two waves per SIMD on 16-row tiles: four waves on 32-row tiles (32x32x16 instructions, half the weight fragments per row, what the
-// figures above were taken with) spent 6 500 cycles on a tile of 96 columns whose matrix instructions take 1 700, because a
-// wave alone on its SIMD issues an instruction every six cycles.  Now 25 000 x 128 80 -> 72, with a weight block per element 82 -> 78, with
-// row_scale 96 (the row_scale rows come again for each l); 10 752 x 64 24.9 -> 21.3, 5 000 x 96 x 10 elements 24.9 -> 20.8, 2 500 x 128 x
-// 10 with row_scale 27.3 -> 21.3, 50 000 x 64 74 -> 70.  Twelve waves are equal at 64 and 96 columns and spill at 128.
+// Two waves per SIMD on 16-row tiles: a wave alone on its SIMD, on 32-row tiles (32x32x16 instructions, half the weight
+// fragments per row), issues an instruction every six cycles.  us, four waves -> eight, shared weights / a weight block per element / row_scale /
+// both: 10 752 x 64 21.3 / 25.5 / 23.8 / 27.9 -> 20.1 / 22.2 / 21.7 / 26.2, 25 000 x 96 64 / 70 / 70 / 76 -> 58 / 64 / 64 / 68, 25 000 x 128 91 / 101 / 102 /
+// 108 -> 90 / 96 / 92 / 98, where matrix instructions and fragment reads take 31 us each of the 62 that its bytes need.  Twelve waves are
+// equal at 64 and 96 columns and spill at 128.
 //
 // What a wave has in flight lives in registers, not in LDS: the loads of tile i + 1 (8 x 16 bytes per lane at 128
 // columns, whole 128-byte lines of 8 rows per instruction) are issued before tile i is multiplied and land in
 // accumulator-file registers; 64 KB per compute unit are on their way at any time.  When its turn comes a tile changes
 // from that row-major layout to the operand layout of the matrix instruction (a lane holds 8 values of one row per
-// 32-wide k step) through the wave's own corner of LDS, up to 96 columns at a time; the rows' largest values are found on the way.
+// 32-wide k step) through the wave's own corner of LDS, up to 96 columns at a time.
 // The operands are swapped with respect to the kernels above (weights as the row operand, X rows as the column operand): a lane's
 // accumulators are then 4 consecutive output columns of one row; a block of 32 columns goes back through the same corner of LDS
 // and leaves as whole lines.
@@ -776,22 +773,20 @@ __device__ __forceinline__ void first_tiles(const int32_t *__restrict__ group_of
 // A workgroup's piece of the list of all tiles, tiles [first, last).  With row_scale (SCALED) the 2 l + 1 tiles of a node tile share its
 // row_scale rows: a node tile of l = 0 fetches and multiplies them for one tile, of l = 3 for seven, and with pieces of as many tiles each the
 // launch waited for those of l = 0.  A node tile counts 2 l + 1 + 1/2 there (a quarter: the same within 2 %).  us, shared weights / ten
-// weight groups, equal pieces -> these: 12 000 x 64 23.8 / 25.3 -> 22.5 / 25.2, 60 000 x 64 97.5 / 99.8 -> 91.0 / 93.5, 12 000 x 128 46.2 / 51.2 ->
-// 42.6 / 46.1, 25 000 x 128 91.2 / 94.7 -> 84.1 / 85.8 (73 / 82 without row_scale), 60 000 x 128 226 / 238 -> 211 / 216, 12 000 x 192 77.3 /
-// 88.0 -> 72.6 / 80.7, 100 000 x 192 653 / 657 -> 594 / 603, 100 000 x 256 800 / 877 -> 787 / 814.  With one weight block per l an l
+// weight groups, equal pieces -> these: 12 000 x 64 24.5 / 26.4 -> 24.1 / 27.9, 60 000 x 64 101 / 102 -> 94 / 94, 25 000 x 96 68.7 / 70.6 -> 65.1 /
+// 68.0, 25 000 x 128 94.8 / 101 -> 91.6 / 98.1 (89 / 96 without row_scale), 60 000 x 128 236 / 252 -> 219 / 228.  With one weight block per l an l
 // gets whole workgroups, so that none of them stages two blocks; with more, where pieces cross blocks anyway, the workgroups of
-// an XCD take neighbouring pieces, whose rows of row_scale meet in its L2 (25 000 x 128 94.7 -> 92.7 of the above).  An XCD for an eighth of the
-// nodes with shared weights: 88.1 with the nearest whole workgroups, 3 : 6 : 10 : 13 of 32.
-// Steps: 25 000 x 128 2 180 -> 2 159, dynamics of it 55.6 -> 55.1 ms, 100 000 x 192 13.74 -> 13.69.
+// an XCD take neighbouring pieces, whose rows of row_scale meet in its L2.  (The kernel with weights in registers waits for its matrix
+// instructions: equal pieces there, 12 000 x 192 86.7 / 97.8 -> 85.1 / 90.2.)
 struct Share {
   int first, last;
 };
 constexpr int kXcds = 8;
-template <bool SCALED, int COMP>
+template <bool SCALED>
 __device__ __forceinline__ Share own_share(const int *cum, int ngroups) {
   const auto whole = [](int64_t n, int index, int of) { return static_cast<int>(n * index / of); };
   const int of = gridDim.x, index = blockIdx.x, ntiles = cum[ngroups];
-  if constexpr (!SCALED || COMP != 16) return {whole(ntiles, index, of), whole(ntiles, index + 1, of)};
+  if constexpr (!SCALED) return {whole(ntiles, index, of), whole(ntiles, index + 1, of)};
   const auto cost_before = [](int l) { return 2 * l * l + l; };  // of the l blocks before l, per node tile, in half tiles
   constexpr int kCost = 36;                                      // = cost_before(4)
   if (ngroups == 1 && of >= kCost) {
@@ -814,18 +809,6 @@ __device__ __forceinline__ Share own_share(const int *cum, int ngroups) {
   return {tile_at(piece), tile_at(piece + 1)};
 }
 
-using rows::largest4;
-// largest value over eight neighbouring lanes, in all of them
-__device__ __forceinline__ float max_over_8(float v) {
-  auto with = [&](auto ctrl) {
-    constexpr int kCtrl = decltype(ctrl)::value;
-    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false)));
-  };
-  v = with(std::integral_constant<int, 0xB1>{});   // lane ^ 1
-  v = with(std::integral_constant<int, 0x4E>{});   // lane ^ 2
-  return with(std::integral_constant<int, 0x141>{});  // the eight lanes in reverse
-}
-
 template <int K, int NT, bool SCALED>
 __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_resident_kernel(
     const float *__restrict__ X, const float *__restrict__ WT, const int32_t *__restrict__ node_perm,
@@ -835,9 +818,7 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
   static_assert(K == NOUT, "square weights");
   constexpr int LD = K + 8;      // row stride of a plane in elements: an odd number of 16-byte units
   constexpr int KS = K / 32;
-  __shared__ __attribute__((aligned(16))) _Float16 sW[2 * NOUT * LD];
-  __shared__ __attribute__((aligned(16))) float sColumn[NOUT];  // largest magnitude of a weight column, then what takes its scale back
-  __shared__ float sRowMax[kResWaves * kResRows];
+  __shared__ __attribute__((aligned(16))) __bf16 sW[3 * NOUT * LD];
   __shared__ int sId[kResSegRows];
   constexpr int kChunk = K <= 96 ? K : 64;  // columns of X per trip through LDS
   constexpr int kTLd = kChunk + 4;          // floats per row of the transposition block: an odd number of 16-byte units
@@ -866,7 +847,7 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
   }
   __syncthreads();
 
-  const Share share = own_share<SCALED, 16>(sCum, ngw);
+  const Share share = own_share<SCALED>(sCum, ngw);
   const int i1 = share.last;
   int i = share.first;
   int g = 0, staged_g = -1, staged_l = -1;
@@ -883,10 +864,13 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
     const int off0 = sOff[g], off1 = sOff[g + 1];
     const bool new_weights = g != staged_g || l != staged_l;
 
-    // W^T[j, :] of block (g, l) -> two planes.  All loads of a thread first, ahead of the row numbers: one trip through L2.
+    // W^T[j, :] of block (g, l) -> three planes.  All loads of a thread first, ahead of the row numbers: one trip through L2.
     const float *Wg = WT + (static_cast<int64_t>(g) * 4 + l) * NOUT * K;
     constexpr int kPieces = (NOUT * (K / 4) + kResWaves * kWave - 1) / (kResWaves * kWave);
-    const auto piece_of = [&](int it) { return min(it * (kResWaves * kWave) + tid, NOUT * (K / 4) - 1); };  // beyond the block: its last piece once more
+    const auto piece_of = [&](int it) {  // beyond the block: its last piece once more
+      const int q = it * (kResWaves * kWave) + tid;
+      return NOUT * (K / 4) % (kResWaves * kWave) == 0 ? q : min(q, NOUT * (K / 4) - 1);
+    };
     f4 wv[kPieces];
     if (new_weights) {
 #pragma unroll
@@ -908,26 +892,16 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
       sId[r] = node;
     }
     if (new_weights) {
-      if (tid < NOUT) sColumn[tid] = 0.f;
-      __syncthreads();
-      // eight neighbouring threads hold pieces of one column (K / 4 is a multiple of eight)
-#pragma unroll
-      for (int it = 0; it < kPieces; ++it) {
-        const float big = max_over_8(largest4(wv[it]));
-        if (tid % 8 == 0) atomicMax(reinterpret_cast<unsigned *>(sColumn) + piece_of(it) / (K / 4), __float_as_uint(big));
-      }
-      __syncthreads();
 #pragma unroll
       for (int it = 0; it < kPieces; ++it) {
         const int q = piece_of(it);
-        const int j = q / (K / 4), kq = q % (K / 4);
-        f16x4 h, lw;
-        split2(wv[it], piece_scale(sColumn[j], kLeastColumnExponent).s, h, lw);
-        *reinterpret_cast<f16x4 *>(sW + j * LD + 4 * kq) = h;
-        *reinterpret_cast<f16x4 *>(sW + NOUT * LD + j * LD + 4 * kq) = lw;
+        const int at = q / (K / 4) * LD + 4 * (q % (K / 4));
+        bf16x4 h, md, lw;
+        split3(wv[it], h, md, lw);
+        *reinterpret_cast<bf16x4 *>(sW + at) = h;
+        *reinterpret_cast<bf16x4 *>(sW + NOUT * LD + at) = md;
+        *reinterpret_cast<bf16x4 *>(sW + 2 * NOUT * LD + at) = lw;
       }
-      __syncthreads();
-      if (tid < NOUT) sColumn[tid] = ldexpf(scale, piece_scale(sColumn[tid], kLeastColumnExponent).exponent);
       staged_g = g;
       staged_l = l;
     }
@@ -989,22 +963,26 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
         }
       }
     };
-    const _Float16 *wl = sW + r16 * LD + 8 * quarter;
+    // a base per plane: the third lies beyond the offset an LDS read can hold, and an address per fragment would take 32 registers
+    const __bf16 *wl[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      unsigned at = (q * NOUT + r16) * LD + 8 * quarter;
+      asm("" : "+v"(at));
+      wl[q] = sW + at;
+    }
     int m_next, tb_next;
     issue(wb, m_next, tb_next);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     for (int idx = wb; idx < we; ++idx) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRg * NT) : "memory");
       const int m_cur = m_next, tb_cur = tb_next;
-      float big[kRg];
-#pragma unroll
-      for (int rg = 0; rg < kRg; ++rg) big[rg] = 0.f;
-      f4 cur[2 * KS];
+      bf16x8 x[KS][3];
 #pragma unroll
       for (int c = 0; c < kChunks; ++c) {
         wave_lds_fence();
 #pragma unroll
-        for (int rg = 0; rg < kRg; ++rg) {
+        for (int rg = 0; rg < kRg; ++rg)
 #pragma unroll
           for (int ln = 0; ln < kLines; ++ln) {
             const int j = (c * kRg + rg) * kLines + ln;
@@ -1014,33 +992,16 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
               asm volatile("; landed %0" : "+a"(sland[j]));
               v *= sland[j];
             }
-            big[rg] = fmaxf(big[rg], largest4(v));
             *reinterpret_cast<f4 *>(stg + (8 * rg + orow) * kTLd + 32 * ln + 4 * opiece) = v;
           }
-          if (c == kChunks - 1) {  // the eight lanes of a row have all of it
-            const float row = max_over_8(big[rg]);
-            if (opiece == 0) sRowMax[kResRows * wave + 8 * rg + orow] = row;
-          }
-        }
         wave_lds_fence();
         // k step s of the chunk: the lane's values are columns 32 s + 8 quarter + {0..7}
+        f4 cur[kChunk / 16];
 #pragma unroll
-        for (int sc = 0; sc < kChunk / 32; ++sc) {
-          const int s = c * (kChunk / 32) + sc;
-          cur[2 * s] = *reinterpret_cast<const f4 *>(stg + r16 * kTLd + 32 * sc + 8 * quarter);
-          cur[2 * s + 1] = *reinterpret_cast<const f4 *>(stg + r16 * kTLd + 32 * sc + 8 * quarter + 4);
-        }
-      }
-      const PieceScale row = piece_scale(sRowMax[kResRows * wave + r16], kLeastRowExponent);
-      if (idx + 1 < we) issue(idx + 1, m_next, tb_next);
-      f16x8 x[KS][2];
+        for (int i = 0; i < kChunk / 16; ++i) cur[i] = ld4(stg + r16 * kTLd + 32 * (i / 2) + 8 * quarter + 4 * (i % 2));
+        if (c == kChunks - 1 && idx + 1 < we) issue(idx + 1, m_next, tb_next);
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        f16x4 h0, l0, h1, l1;
-        split2(cur[2 * s], row.s, h0, l0);
-        split2(cur[2 * s + 1], row.s, h1, l1);
-        x[s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-        x[s][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        for (int sc = 0; sc < kChunk / 32; ++sc) split3(cur[2 * sc], cur[2 * sc + 1], x[c * (kChunk / 32) + sc]);
       }
       __builtin_amdgcn_sched_barrier(0);
       float *orows[kRg];
@@ -1051,23 +1012,17 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
       constexpr int GB = NT % 2 == 0 ? 4 : 2;  // column blocks of 16 at a time
 #pragma unroll
       for (int t0 = 0; t0 < 2 * NT; t0 += GB) {
-        v4f acc[GB], small[GB];  // products of high pieces, and those with a low one
+        v4f acc[GB], small[GB];
 #pragma unroll
         for (int t = 0; t < GB; ++t) acc[t] = small[t] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          f16x8 wh[GB], wo[GB];
+          bf16x8 w[GB][3];
 #pragma unroll
-          for (int t = 0; t < GB; ++t) {
-            wh[t] = *reinterpret_cast<const f16x8 *>(wl + 16 * (t0 + t) * LD + 32 * s);
-            wo[t] = *reinterpret_cast<const f16x8 *>(wl + NOUT * LD + 16 * (t0 + t) * LD + 32 * s);
-          }
+          for (int t = 0; t < GB; ++t)
 #pragma unroll
-          for (int t = 0; t < GB; ++t) small[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[t], x[s][1], small[t], 0, 0, 0);
-#pragma unroll
-          for (int t = 0; t < GB; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[t], x[s][0], acc[t], 0, 0, 0);
-#pragma unroll
-          for (int t = 0; t < GB; ++t) small[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wo[t], x[s][0], small[t], 0, 0, 0);
+            for (int q = 0; q < 3; ++q) w[t][q] = *reinterpret_cast<const bf16x8 *>(wl[q] + 16 * (t0 + t) * LD + 32 * s);
+          rows::add_products(w, x[s], acc, small);
           if (K == 128) __builtin_amdgcn_sched_barrier(0);  // fragment reads of later steps hoisted further would not fit the register file
         }
         // accumulator r of a lane: output column 16 t + 4 quarter + r of row r16 of the tile.  A block of 32 columns goes
@@ -1077,12 +1032,7 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
         for (int t = 0; t < GB; t += 2) {
           wave_lds_fence();
 #pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            f4 v = (acc[t + q] + small[t + q]) * ld4(sColumn + 16 * (t0 + t + q) + 4 * quarter);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = __builtin_ldexpf(v[k], row.exponent);
-            st4(stg + r16 * kOutLd + 16 * q + 4 * quarter, v);
-          }
+          for (int q = 0; q < 2; ++q) st4(stg + r16 * kOutLd + 16 * q + 4 * quarter, f4((acc[t + q] + small[t + q]) * scale));
           wave_lds_fence();
 #pragma unroll
           for (int r = 0; r < kRg; ++r) {
@@ -1106,19 +1056,17 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
 // again for every 128 rows in barrier-separated phases that one or two waves per SIMD cannot overlap: 192 columns ran at
 // 2.8-3.0 TB/s of their bytes, 256 at 2.2.  The register file of a compute unit holds 512 KB: here a workgroup takes a
 // contiguous piece of the list of all 16-row tiles (as the kernel above does), wave w keeps the pieces of its 16 CB weight
-// columns for all of K in its registers (CB K / 4 of them) until the weight block changes, and all waves multiply the
+// columns for all of K in its registers (6 CB K / 16 of them) until the weight block changes, and all waves multiply the
 // same tile of X rows, whose piece planes they share through LDS, double-buffered with one barrier per tile.  X goes
 // global -> LDS as raw fp32 by direct loads; a wave splits exactly the pieces it fetched itself, so only the planes are
 // shared.  The waves of a SIMD take turns in the order of their phases: every other one multiplies the current tile before
 // it splits the next.
 //
 // Operands as in the kernel above (weights as the row operand): a lane's accumulators are four consecutive output columns of
-// one row, stored as 16 bytes.  Two fp16 pieces per operand as above, v_mfma_f32_16x16x32_f16: K steps of 32.  A row is
-// fetched by several waves, and its scale needs its largest value: a wave takes its pieces of tile k + 2 from LDS into registers
-// and adds them to the maxima of the rows (LDS atomics) while tile k is multiplied, and splits them a barrier later.
+// one row, stored as 16 bytes.  v_mfma_f32_16x16x32_bf16: K steps of 32, pieces, products and accumulators as above.
 //
-// Vector-memory operations of the tile loop are issued from assembly: the loads of tile k + 3 right after tile k + 2 has been
-// taken, then the stores of a tile; the wait before a tile is taken lets exactly those stores stay out.
+// Vector-memory operations of the tile loop are issued from assembly: the loads of tile k + 2 right after the split of tile
+// k + 1, then the stores of a tile; the wait before a split lets exactly those stores stay out.
 //
 // CB: 16 columns per wave give 10, 12 and 14 waves, three or four per SIMD (32 columns per wave: 5, 6 and 7 waves, two on
 // some SIMDs and one on others; 5-8 % slower at 160 and 192); at 256 columns 32 per wave (8 waves) are equal up to 20 000
@@ -1127,9 +1075,10 @@ __global__ __launch_bounds__(kResWaves *kWave, kResWaves / 4) void linear_reside
 //
 // Measured against the tiled kernels (plain / row_scale): 100 000 x 192 810 / 860 -> 655 / 675 us, 50 000 x 160 326 / 345 ->
 // 285 / 290, 20 000 x 224 255 / 272 -> 180 / 190, 40 000 x 256 595 / 643 -> 415 / 445, 12 000 x 256 183 / 198 -> 122 / 145,
-// equal at 2 048 nodes.  That was with three bf16 pieces and six products, whose matrix instructions alone took 514 of the 655
-// us at 192 columns; with two fp16 pieces, us and rms error against fp64: 100 000 x 192 647 -> 557, 1.96e-7 -> 1.24e-7, 20 000 x 224
-// 184 -> 134, 2.14e-7 -> 1.29e-7, 12 000 x 256 137 -> 110, 2.31e-7 -> 1.34e-7, 10 007 x 160 64.8 -> 61.1, 1.77e-7 -> 1.18e-7.
+// equal at 2 048 nodes.  Without its matrix instructions 192 columns take 520 us (4.7 TB/s, the rate of a copy), without
+// loads, stores and split 514 us: what is left is their overlap.  All that with one accumulator; with two, us and rms error against fp64:
+// 100 000 x 192 672 -> 685, 1.96e-7 -> 7.8e-8, 20 000 x 192 129 -> 133, 10 007 x 224 92 -> 93, 2.14e-7 -> 8.4e-8, 12 000 x 256 130 -> 130, 2.31e-7 -> 8.9e-8,
+// 10 007 x 160 57 -> 57, 1.77e-7 -> 7.2e-8.  (Two fp16 pieces of scaled rows and columns and three products, not fp32 any more: 584, -, -, 98 and 53.)
 // -----------------------------------------------------------------------------------------------
 constexpr int kWideMinScalarNodes = 8192;
 constexpr int kWideSegRows = 2048;  // rows whose node numbers a segment keeps in LDS
@@ -1149,9 +1098,7 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
   constexpr int PIECES = TR * K / 4 / (WAVES * kWave);  // 16-byte pieces of a tile per thread
   constexpr int STORES = CB * RB;             // per wave and tile
   constexpr int kSegTiles = kWideSegRows / TR;
-  __shared__ __attribute__((aligned(16))) _Float16 sP[2][2][TR * LD];
-  __shared__ unsigned sRowMax[4][TR];  // largest magnitude of a row (its bits): of the tile multiplied, the next two, and one being cleared
-  __shared__ __attribute__((aligned(16))) float sColumn[K];
+  __shared__ __attribute__((aligned(16))) __bf16 sP[2][3][TR * LD];
   __shared__ __attribute__((aligned(16))) float sRaw[TR * K];
   __shared__ __attribute__((aligned(16))) float sScale[SCALED ? TR * K : 4];
   __shared__ int sId[kWideSegRows];
@@ -1192,12 +1139,11 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
   const unsigned raw_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sRaw)) + wave * (kWave * 16);
   const unsigned scale_lds = static_cast<unsigned>(reinterpret_cast<uintptr_t>(sScale)) + wave * (kWave * 16);
 
-  const Share share = own_share<SCALED, COMP>(sCum, ngw);
+  const Share share = own_share<false>(sCum, ngw);
   const int i1 = share.last;
   int i = share.first;
   int g = 0, held_g = -1, held_l = -1;
-  f16x8 w[CB][KS][2];  // weight pieces: column block, k step, piece
-  f4 column[CB];       // what takes the weight columns' scales back, of the four columns whose sums a lane gets
+  bf16x8 w[KS][CB][3];  // weight pieces: k step, column block, piece
 
   while (i < i1) {
     while (sCum[g + 1] <= i) ++g;
@@ -1223,36 +1169,16 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
     }
     if (g != held_g || l != held_l) {
       // a lane feeds 8 consecutive k of one weight column per step
-      const float *Wg = WT + ((static_cast<int64_t>(g) * (COMP == 1 ? 1 : 4) + l) * K + 16 * CB * wave + r16) * K + 8 * quarter;
+      int at = (16 * CB * wave + r16) * K + 8 * quarter;
+      asm volatile("" : "+v"(at));  // computed here: ahead of the loops it would be registers that 224 columns do not have
+      const float *Wg = WT + (static_cast<int64_t>(g) * (COMP == 1 ? 1 : 4) + l) * K * K + at;
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) {
-        f4 v[2 * KS];
-        float big = 0.f;
+      for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          v[2 * s] = ld4(Wg + 16 * cb * K + 32 * s), v[2 * s + 1] = ld4(Wg + 16 * cb * K + 32 * s + 4);
-          big = fmaxf(big, fmaxf(largest4(v[2 * s]), largest4(v[2 * s + 1])));
-        }
-        big = fmaxf(big, __shfl_xor(big, 16));
-        big = fmaxf(big, __shfl_xor(big, 32));  // the four lanes of a column
-        const PieceScale of = piece_scale(big, kLeastColumnExponent);
-        if (quarter == 0) sColumn[16 * CB * wave + 16 * cb + r16] = ldexpf(scale, of.exponent);
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          f16x4 h0, l0, h1, l1;
-          split2(v[2 * s], of.s, h0, l0);
-          split2(v[2 * s + 1], of.s, h1, l1);
-          w[cb][s][0] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-          w[cb][s][1] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-      }
-      wave_lds_fence();  // a wave reads back its own columns
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb) column[cb] = ld4(sColumn + 16 * CB * wave + 16 * cb + 4 * quarter);
+        for (int s = 0; s < KS; ++s) split3(ld4(Wg + 16 * cb * K + 32 * s), ld4(Wg + 16 * cb * K + 32 * s + 4), w[s][cb]);
       held_g = g;
       held_l = l;
     }
-    for (int r = tid; r < 4 * TR; r += WAVES * kWave) sRowMax[r / TR][r % TR] = 0;
     __syncthreads();
 
     const int n = seg_end - i;
@@ -1279,49 +1205,35 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
         }
       }
     };
-    // This wave's pieces of tile k, once they are there, from LDS into registers, and their part in the rows' largest magnitudes.
-    f4 piece[PIECES];
-    auto take = [&](int k) {
+    auto split = [&](int k) {
+      __bf16 *plane = &sP[k & 1][0][0];
 #pragma unroll
       for (int j = 0; j < PIECES; ++j) {
         const int p = (j * WAVES + wave) * kWave + lane;
-        piece[j] = *reinterpret_cast<const f4 *>(sRaw + 4 * p);
-        if constexpr (SCALED) piece[j] *= *reinterpret_cast<const f4 *>(sScale + 4 * p);
-        const float big = max_over_8(largest4(piece[j]));  // eight neighbouring lanes hold pieces of one row
-        if (lane % 8 == 0) atomicMax(&sRowMax[k & 3][prow[j]], __float_as_uint(big));
-      }
-    };
-    auto split = [&](int k) {
-      _Float16 *plane = &sP[k & 1][0][0];
-#pragma unroll
-      for (int j = 0; j < PIECES; ++j) {
-        f16x4 h, lw;
-        split2(piece[j], piece_scale(__uint_as_float(sRowMax[k & 3][prow[j]]), kLeastRowExponent).s, h, lw);
+        f4 v = *reinterpret_cast<const f4 *>(sRaw + 4 * p);
+        if constexpr (SCALED) v *= *reinterpret_cast<const f4 *>(sScale + 4 * p);
+        bf16x4 h, md, lw;
+        split3(v, h, md, lw);
         const int at = prow[j] * LD + pcol[j];
-        *reinterpret_cast<f16x4 *>(plane + at) = h;
-        *reinterpret_cast<f16x4 *>(plane + TR * LD + at) = lw;
+        *reinterpret_cast<bf16x4 *>(plane + at) = h;
+        *reinterpret_cast<bf16x4 *>(plane + TR * LD + at) = md;
+        *reinterpret_cast<bf16x4 *>(plane + 2 * TR * LD + at) = lw;
       }
     };
     auto multiply = [&](int k) {
       int m, tb;
       where(k, m, tb);
-      const _Float16 *plane = &sP[k & 1][0][0] + r16 * LD + 8 * quarter;
+      const __bf16 *plane = &sP[k & 1][0][0] + r16 * LD + 8 * quarter;
       static_assert(RB == 1, "a lane's sums belong to one row");
-      const int exponent = piece_scale(__uint_as_float(sRowMax[k & 3][r16]), kLeastRowExponent).exponent;
-      v4f acc[CB], small[CB];  // products of high pieces, and those with a low one
+      v4f acc[CB], small[CB];
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) acc[cb] = small[cb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        f16x8 x[2];
+        bf16x8 x[3];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) x[q] = *reinterpret_cast<const f16x8 *>(plane + q * (TR * LD) + 32 * s);
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) small[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][0], x[1], small[cb], 0, 0, 0);
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][0], x[0], acc[cb], 0, 0, 0);
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) small[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[cb][s][1], x[0], small[cb], 0, 0, 0);
+        for (int q = 0; q < 3; ++q) x[q] = *reinterpret_cast<const bf16x8 *>(plane + q * (TR * LD) + 32 * s);
+        rows::add_products(w[s], x, acc, small);
       }
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
@@ -1341,9 +1253,7 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
           v4f v;
           {
 #pragma clang fp contract(off)  // the product is rounded before the residual is added, as everywhere
-            v = (acc[cb] + small[cb]) * column[cb];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = __builtin_ldexpf(v[i], exponent);
+            v = (acc[cb] + small[cb]) * scale;
             if (COMP == 1 && residual) v = v + res[cb];
           }
           // (the two idle issue slots: see the stores of the kernel above)
@@ -1354,26 +1264,17 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
 
     issue(0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    take(0);
-    if (n > 1) issue(1);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // largest magnitudes of tile 0 complete
     split(0);
-    if (n > 1) take(1);
-    if (n > 2) issue(2);
-    // before the first wait of the loop only loads are out; it is exact from the second tile on
+    if (n > 1) issue(1);
+    // before the first split of the loop only loads are out; the wait below is exact from the second tile on
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     for (int k = 0; k < n; ++k) {
-      // planes of tile k and largest magnitudes of tile k + 1 complete, the planes of tile k - 1 free
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // planes of tile k complete, those of tile k - 1 free
       if (late) multiply(k);
       if (k + 1 < n) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");  // the loads of tile k + 1; the stores after them may stay out
         split(k + 1);
-        if (tid < TR) sRowMax[(k + 3) & 3][tid] = 0;  // last read when tile k - 1 was multiplied
-        if (k + 2 < n) {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");  // the loads of tile k + 2; the stores after them may stay out
-          take(k + 2);
-          if (k + 3 < n) issue(k + 3);
-        }
+        if (k + 2 < n) issue(k + 2);
       }
       if (!late) multiply(k);
     }
@@ -1390,7 +1291,7 @@ __global__ __launch_bounds__(2 * NT / CB * kWave, (2 * NT / CB + 3) / 4) void li
 // ones walk K in phases.  Here a workgroup has one weight block and each of its eight waves one tile of 16 rows, so everything is asked
 // for at once: group offsets, then the weights and the row numbers, then the rows, one barrier, the products, the stores.  Rows of a
 // degree are counted node by node (row r of degree l is component l^2 + r % (2l + 1) of the block's node r / (2l + 1)): the rows of a wave lie
-// side by side in memory.  Arithmetic as in linear_resident_kernel, operands as in mfma_rows.hpp (a load covers 64 bytes of a row).
+// side by side in memory.  Operands and arithmetic: mfma_rows.hpp (a load covers 64 bytes of a row).
 // Columns are split over COLS / 16 NB workgroups where the rows alone leave compute units idle, and where the planes of all would not fit LDS.
 // -----------------------------------------------------------------------------------------------
 constexpr int kBlockWaves = 8;
@@ -1402,7 +1303,7 @@ __host__ __device__ __forceinline__ int row_blocks(int nodes, int ncomp) {
 }
 
 template <int KS, int NB, bool SCALED>
-__global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 && !SCALED) ? 4 : 2) void linear_block_kernel(
+__global__ __launch_bounds__(kBlockWaves *kWave, KS <= 3 || (KS == 4 && NB == 4 && !SCALED) || (KS == 5 && NB == 5 && !SCALED) ? 4 : 2) void linear_block_kernel(
     const float *__restrict__ X, const float *__restrict__ WT, const int32_t *__restrict__ node_perm, const int32_t *__restrict__ group_offsets,
     int nnodes, int ngroups, int zero_last_group, int ncomp, float scale, const float *__restrict__ row_scale, const float *residual, float *OUT) {
   constexpr int K = 32 * KS;
@@ -1471,7 +1372,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
   f4 x[2 * KS], factor[SCALED ? 2 * KS : 1];
   rows::load(X + row * K, x);
   if constexpr (SCALED) rows::load(row_scale + static_cast<int64_t>(node) * K, factor);
-  weights.store(planes, scale);
+  weights.store(planes);
   if constexpr (SCALED) {
 #pragma unroll
     for (int i = 0; i < 2 * KS; ++i) x[i] *= factor[i];
@@ -1485,7 +1386,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
     f4 res[GB], v[GB];
 #pragma unroll
     for (int c = 0; c < GB; ++c) res[c] = rp ? ld4(rp + 16 * (c0 + c)) : zero4();
-    rows::product(planes, operand, c0, v);
+    rows::product(planes, operand, c0, scale, v);
 #pragma unroll
     for (int c = 0; c < GB; ++c) {
       {
@@ -1497,39 +1398,46 @@ __global__ __launch_bounds__(kBlockWaves *kWave, KS <= 4 || (KS == 5 && NB == 5 
   }
 }
 
-// Column blocks (of 16) per workgroup of linear_block_kernel, or 0: another kernel.  Each line from both sides, us, shared weights /
-// ten weight groups / row_scale / both:
-//  - up to 128 columns, 16 components: up to four workgroups per compute unit (8 192 nodes).  Kernel with resident weights -> this one: 2 500
-//    x 128 16.4 / 20.9 / 18.5 / 22.3 -> 12.8 / 14.2 / 15.3 / 16.7, 5 000 x 96 20.6 / 25.5 / 21.4 / 27.2 -> 15.3 / 16.5 / 16.4 / 18.0.  It stays ahead
-//    on its own beyond that (10 000 x 128 43.6 / 51.3 / 48.1 / 58.2 -> 33.5 / 35.6 / 35.3 / 37.5), but not in a step, where X and the
-//    result share the last-level cache with everything else (step without -> with: 3 000 x 128 398 -> 378, 8 000 x 96 632 -> 616, 5 000 x 64
-//    312 -> 307; 10 000 x 64 504 -> 502, 10 752 x 64 in 512 graphs 285 -> 293, 10 000 x 128 927 -> 933): the other kernel has the loads of a
-//    tile under way while it works on the one before.  Ring and tiled kernels, below 2 048 nodes: 700 x 128 9.5 / 11.4 / 10.4 /
-//    12.4 -> 6.8 / 7.3 / 8.2 / 8.8, 2 000 x 128 12.8 / 17.0 / 13.5 / 19.1 -> 9.6 / 13.8 / 11.0 / 16.5, 2 000 x 64 6.1 / 7.6 / 6.6 / 8.2 -> 5.9 / 7.2 / 6.6 / 9.0.
-//    Half the columns each while that leaves one workgroup per compute unit (700 x 128 7.9 / 8.3 / 9.4 / 9.9 -> the figures above; 1 000
-//    x 128 with groups, two on some: 8.7 -> 10.8).
-//  - beyond 128 columns a compute unit holds one workgroup, and the kernel with weights in registers takes over after one round of them
-//    (two at 160 and 192 columns) where it runs: 1 000 x 192 16.2 / 20.9 / 18.0 / 22.6 -> 10.4 / 14.2 / 12.9 / 16.5, 3 500 x 192 28.6 /
-//    35.5 / 31.1 / 37.0 -> 28.0 / 31.5 / 29.7 / 34.2, 1 000 x 256 24.4 / 32.5 / 27.6 / 34.9 -> 14.8 / 25.5 / 18.6 / 29.3; 2 500 x 256
-//    31.4 / 41.8 / 34.3 / 44.2 -> 37.0 / 43.6 / 42.1 / 49.0.
-//  - one component, up to 128 columns, beyond the few rows of mfma_f32.hpp: always (3 200 x 128 7.5 / 8.0 -> 6.4 / 6.9, 25 000 x 128 12.3 / 13.2
-//    -> 9.4 / 10.0, 60 000 x 64 9.0 / 9.6 -> 8.2 / 8.9); it has the arithmetic of the chains of such products (node_glue.hip).
-//  - one component beyond 128 columns: one round with one weight group (10 000 x 160 9.8 -> 8.1, 10 000 x 256 17.7 -> 12.6; 35 000 x 192
-//    21.6 -> 24.6); with several, where the other choice is the tiled kernel, always (10 000 x 256 21.2 -> 13.7, 100 000 x 192 60 -> 52),
-//    but with row_scale for that round alone (50 000 x 224 55 -> 63).
-int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, bool scaled) {
+// Whether the kernels that keep square weights in LDS (64 to 128 columns) or in registers (160 and more) take a call.
+bool resident_weights(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, bool residual) {
+  if (ncomp == 16) return K >= 64 && !residual && ngroups <= kResMaxGroups && nnodes >= kResMinNodes;
+  return K >= 160 && !grouped && nnodes >= kWideMinScalarNodes;
+}
+
+// Column blocks (of 16) per workgroup of linear_block_kernel, or 0: another kernel.  Each line from both sides, us, shared weights / ten weight
+// groups / row_scale / both, the kernel that would run otherwise -> this one:
+//  - half of the columns where that leaves no more than one workgroup per compute unit (all -> half: 700 x 128 9.2 / 10.2 / 10.6 / 11.2 ->
+//    6.9 / 7.7 / 8.4 / 8.9, 1 000 x 128 with groups, two on some: 10.4 -> 11.0).
+//  - up to one round of workgroups always: 2 000 x 64 6.2 / 7.9 / 6.9 / 8.5 -> 5.5 / 7.6 / 6.0 / 8.9, 1 500 x 128 11.9 / 16.8 / 13.0 / 18.5 -> 10.2 /
+//    11.3 / 11.8 / 12.9, 1 500 x 160 17.3 / 21.5 / 18.5 / 23.4 -> 14.3 / 15.9 / 16.3 / 17.9, 700 x 192 15.3 / 20.7 / 16.9 / 22.5 -> 11.6 / 12.9 / 14.0 / 15.3,
+//    700 x 224 18.1 / 27.7 / 19.4 / 29.5 -> 14.2 / 16.5 / 17.4 / 19.0, 300 x 256 15.3 / 33 / 16.7 / 33 -> 10.6 / 13.1 / 13.6 / 14.8; one component 12 000 x 160
+//    10.6 / 14.9 / 11.3 / 21.4 -> 9.3 / 10.0 / 11.9 / 12.4, 12 000 x 192 12.5 / 17.5 / 13.4 / 27.1 -> 11.2 / 11.9 / 14.3 / 15.0, 6 000 x 256 17.7 / 16.9 / 21.6 / 21.4 ->
+//    10.8 / 12.5 / 14.8 / 16.7.  (One component, 224 columns, up to 4 096 nodes: the tiled kernel cuts its tiles to 32 columns there, 10.9 -> 12.5.)
+//  - beyond it against resident weights at 64 and 96 columns, two workgroups per compute unit: up to four (8 192 nodes; 5 000 x 64 12.2 / 17.2 / 13.3 / 17.6 ->
+//    11.0 / 12.3 / 12.5 / 13.4, 8 000 x 96 27.8 / 31.7 / 29.0 / 31.5 -> 22.8 / 24.8 / 25.1 / 27.0).  It stays ahead on its own beyond that, but not in a step, where X and the
+//    result share the last-level cache with everything else (10 752 x 64 in 512 graphs 285 -> 293): the other kernel has the loads
+//    of a tile under way while it works on the one before.  At 128 columns one workgroup fits a compute unit, and a second round pays
+//    where at least half of it is filled: 2 500 16.7 / 20.1 / 18.0 / 22.5 -> 17.9 / 19.7 / 19.3 / 21.4, 3 500 23.3 / 26.1 / 22.1 / 27.3 -> 20.2 / 23.8 / 21.8 / 25.8,
+//    5 000 27.1 / 31.5 / 27.7 / 34.2 -> 27.5 / 30.7 / 29.5 / 33.1.  Beyond 128 columns it does not: 2 500 x 160 21.2 / 26.6 / 22.7 / 29.8 -> 25.4 / 27.3 / 27.1 / 29.5, 2 500 x
+//    224 32 / 40 / 34 / 43 -> 40 / 45 / 44 / 50, 16 000 and 24 000 x 192 of one component 14.7 / 20.7 -> 12.3 / 19.9 and 18.2 / 21.6 -> 20.0 / 22.6.
+//  - beyond it against the tiled kernels: one component up to 128 columns always (100 000 x 96 26.7 -> 20.2, 33 000 x 128 16.2 -> 16.8: it has the
+//    arithmetic of the chains of such products, node_glue.hip), at 224 with groups (33 000 50 -> 40; with row_scale 50 000 56 -> 70; at 192 24 000 21.6 -> 22.6); 16
+//    components with groups below 2 048 nodes at 224 columns (1 500 49 -> 31, 2 000 49 -> 42) and, unless the tiled kernel's workgroups are one
+//    round, at 256 (700 32 -> 24, 1 000 34 -> 33, 1 500 in two rounds 59 -> 44, 2 000 60 -> 53), not at 160 and 192 (2 000 22.4 -> 27.3, 28.4 -> 33.3).
+int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, bool scaled, bool residual) {
   // a workgroup per 128 rows, and on average half of the weight blocks end in one more
   const int64_t rows = ceil_div(nnodes * ncomp, kBlockRows) + (grouped ? static_cast<int64_t>(ngroups) * (ncomp == 1 ? 1 : 4) / 2 : 0);
-  const int all = K / 16;
-  if (K <= 128) {
-    if (ncomp == 16 && rows > 4 * device_compute_units()) return 0;
-    return 2 * rows <= device_compute_units() ? all / 2 : all;
-  }
-  const int most = K <= 192 ? all : all / 2;  // what fits LDS
-  const int64_t round = device_compute_units() / (all / most);
-  if (K != 224 && 2 * rows <= round) return most / 2;
-  const bool elsewhere = ncomp == 16 ? nnodes >= kResMinNodes : nnodes >= kWideMinScalarNodes && (!grouped || scaled);
-  return !elsewhere || rows <= (ncomp == 16 && K <= 192 ? 2 * round : round) ? most : 0;
+  const int64_t units = device_compute_units();
+  const int all = K / 16, most = K <= 160 ? all : (K == 256 ? all / 4 : all / 2);  // what fits LDS
+  const int64_t round = units / (all / most);
+  const bool resident = resident_weights(nnodes, ncomp, K, ngroups, grouped, residual);
+  if (2 * rows <= round && K != 224) return most / 2;
+  if (rows <= round) return K == 224 && ncomp == 1 && !grouped && nnodes <= 4096 ? 0 : most;
+  if (resident) return (K < 128 && rows <= 4 * units) || (K == 128 && 2 * rows > 3 * units && rows <= 2 * units) ? most : 0;
+  if (K <= 128) return ncomp == 1 || rows <= 4 * units ? most : 0;
+  if (ncomp == 1) return K == 224 && grouped && !scaled ? most : 0;
+  if (!grouped || K <= 192 || nnodes >= kResMinNodes) return 0;
+  return K == 224 || rows <= 2 * round || 4 * 16 * (ceil_div(nnodes, 128) + ngroups / 2) > 5 * units ? most : 0;
 }
 
 template <int KS, int NB>
@@ -1683,17 +1591,18 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
   }
   // up to some thousand nodes (cm::block_columns): a workgroup per 128 rows of one weight block
   if (K == Nout) {
-    switch (32 * K + cm::block_columns(nnodes, ncomp, K, ngroups, group_offsets != nullptr, row_scale != nullptr)) {
+    switch (32 * K + cm::block_columns(nnodes, ncomp, K, ngroups, group_offsets != nullptr, row_scale != nullptr, residual != nullptr)) {
 #define CM_CASE(KS_, NB_) \
       case 32 * 32 * KS_ + NB_: return cm::launch_block<KS_, NB_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, ncomp, scale, row_scale, residual, OUT, st);
       CM_CASE(1, 2) CM_CASE(1, 1) CM_CASE(2, 4) CM_CASE(2, 2) CM_CASE(3, 6) CM_CASE(3, 3) CM_CASE(4, 8) CM_CASE(4, 4) CM_CASE(5, 10) CM_CASE(5, 5)
-      CM_CASE(6, 12) CM_CASE(6, 6) CM_CASE(7, 7) CM_CASE(8, 8) CM_CASE(8, 4)
+      CM_CASE(6, 6) CM_CASE(6, 3) CM_CASE(7, 7) CM_CASE(8, 4) CM_CASE(8, 2)
 #undef CM_CASE
     }
   }
   // 16 components per node, square weights, beyond: up to 128 columns the kernel that keeps the weights in LDS (measured against the ring kernel at 25 000 nodes: 87 vs 102-112 us at 128 channels, 58 vs 67-71 at 96, 42 vs
   // 47 at 64; 360 vs 430 us at 100 000 x 128); at 160 to 256 columns the one that keeps them in registers
-  if (ncomp == 16 && K == Nout && !residual && ngroups <= cm::kResMaxGroups && nnodes >= cm::kResMinNodes) {
+  const bool resident = K == Nout && cm::resident_weights(nnodes, ncomp, K, ngroups, group_offsets != nullptr, residual != nullptr);
+  if (resident && ncomp == 16) {
     switch (K) {
 #define CM_CASE(K_, NT_) \
       case K_: return cm::launch_resident<K_, NT_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, scale, row_scale, OUT, st);
@@ -1707,7 +1616,7 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
   }
   // One component per node, one weight group, 160 columns and more, beyond one round of the kernel above: the same kernel (100 000 x
   // 192 65.7 -> 51.3 us against the tiled one)
-  if (ncomp == 1 && K == Nout && !group_offsets && nnodes >= cm::kWideMinScalarNodes) {
+  if (resident && ncomp == 1) {
     switch (K) {
 #define CM_CASE(NT_, CB_) \
       case 32 * NT_: return cm::launch_wide<NT_, CB_, 1>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, scale, row_scale, residual, OUT, st);

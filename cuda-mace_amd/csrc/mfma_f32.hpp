@@ -69,7 +69,7 @@ __device__ __forceinline__ void product(const Rows<KQ> &x, const Rows<KQ> (&wt)[
 inline int64_t blocks(int64_t nnodes, int ncomp, int columns) { return ceil_div(nnodes, kRows) * ncomp * (columns / kRows); }
 constexpr int64_t kOneColumnBlock = 1024;
 inline bool applies(int64_t nnodes, int ncomp, int columns) {
-  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 || columns == 128 ? 1536 : (columns >= 224 ? 2048 : 2560));
+  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 || columns == 128 ? 1536 : (columns >= 256 ? 2048 : 2560));
   return blocks(nnodes, ncomp, columns) <= limit;
 }
 

@@ -34,20 +34,26 @@ namespace {
 
 // A workgroup of WAVES waves: a wave takes 16 nodes of one element through the whole chain.  The result of a product lies in the lanes
 // as the operand of the next one does (mfma_rows.hpp), so the rows never leave the registers, and the waves meet only where the
-// workgroup's weight planes change: all three blocks up to 96 columns, at 128 the third in the place of the first.  Before, tiles of 32 or
-// 128 nodes exchanged the rows through LDS and staged operands for each 32 columns of K between two barriers, three bf16 pieces
-// and six products (us, forward / backward): 5 000 x 96 13.7 / 12.8 -> 10.1 / 10.7, 10 752 x 64 12.4 / 11.1 -> 6.9 / 6.8, 5 000 x 128 15.2 / 13.9 ->
-// 14.1 / 14.3, 25 000 x 128 26.8 / 23.5 -> 20.7 / 20.9 (its 51 MB take 10), 60 000 x 96 40.7 / 36.3 -> 28.1 / 27.4.  What is left at
-// 128 columns: 7 us of matrix instructions and fragment reads for 128 rows, 3 us for the split of three weight blocks, 4 us until the
-// first operands are there.
+// workgroup's weight planes change: all three blocks fit LDS together up to 64 columns, two at 96, one at 128.  Before, tiles of 32 or
+// 128 nodes exchanged the rows through LDS and staged operands for each 32 columns of K between two barriers (us, forward / backward):
+// 10 752 x 64 12.5 / 11.1 -> 7.4 / 7.3, 60 000 x 64 21.5 / 18.4 -> 19.5 / 19.8, 5 000 x 96 13.7 / 12.9 -> 12.0 / 12.2, 25 000 x 96 19.7 / 17.0 -> 16.8 / 16.8,
+// 5 000 x 128 15.3 / 14.0 -> 17.4 / 17.1, 14 000 x 128 21.1 / 19.0 -> 19.5 / 18.2, 25 000 x 128 26.9 / 23.4 -> 25.3 / 25.0 (its 51 MB take 10), 60 000 x 128 52.6 / 48.4 ->
+// 48.1 / 49.2.  What is left at 128 columns: matrix instructions and fragment reads of 128 rows, and the split of three weight
+// blocks, each between two barriers.
 template <int NT, int WAVES>
 struct Chain {
   static constexpr int C = 32 * NT, NB = 2 * NT;
   static constexpr int kThreads = WAVES * kWave, kRows = 16 * WAVES;
-  static constexpr int kSlots = NT <= 3 ? 3 : 2;
+  static constexpr int kSlots = NT <= 2 ? 3 : (NT == 3 ? 2 : 1);  // weight blocks whose planes fit LDS together
   using Planes = rows::Planes<NT, C>;
   using Weights = rows::Fetched<NT, C, kThreads>;
   using Operand = rows::Operand<NT>;
+  // another block in the place of one that every wave has multiplied
+  __device__ static void replace(Planes &planes, const Weights &w) {
+    __syncthreads();
+    w.store(planes);
+    __syncthreads();
+  }
 };
 
 // ---- forward: h1 = B1 . Wprod, sc = skip_scale h1 . Wskip[element], X2 = h1 . Wup ---------------------------------
@@ -73,25 +79,22 @@ __global__ __launch_bounds__(WAVES *kWave) void node_glue_forward_kernel(
   w_up.request(up_WT);
   if (!no_element) w_skip.request(skip_WT + static_cast<int64_t>(g) * C * C);
   __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
-  w_prod.store(planes[0], 1.0f);
-  w_up.store(planes[1], 1.0f);
-  if (S::kSlots == 3 && !no_element) w_skip.store(planes[S::kSlots - 1], skip_scale);
+  w_prod.store(planes[0]);
+  if constexpr (S::kSlots >= 2) w_up.store(planes[1 % S::kSlots]);
+  if (S::kSlots == 3 && !no_element) w_skip.store(planes[2 % S::kSlots]);
   __syncthreads();
-  rows::product_all(planes[0], typename S::Operand(v), h);
+  rows::product_all(planes[0], typename S::Operand(v), 1.0f, h);
   if (here) rows::store(h1 + at, h);
   const typename S::Operand operand(h);
-  rows::product_all(planes[1], operand, v);
+  if constexpr (S::kSlots == 1) S::replace(planes[0], w_up);
+  rows::product_all(planes[1 % S::kSlots], operand, 1.0f, v);
   if (here) rows::store(X2 + at, v);
   if (no_element) {
 #pragma unroll
     for (int i = 0; i < S::NB; ++i) v[i] = zero4();
   } else {
-    if constexpr (S::kSlots == 2) {
-      __syncthreads();  // every wave is done with the first planes
-      w_skip.store(planes[0], skip_scale);
-      __syncthreads();
-    }
-    rows::product_all(planes[S::kSlots == 3 ? 2 : 0], operand, v);
+    if constexpr (S::kSlots < 3) S::replace(planes[2 % S::kSlots], w_skip);
+    rows::product_all(planes[2 % S::kSlots], operand, skip_scale, v);
   }
   if (here) rows::store(sc + at, v);
 }
@@ -243,25 +246,22 @@ __global__ __launch_bounds__(WAVES *kWave) void node_glue_backward_kernel(
   w_prod.request(prod_W);
   const double nw = node_weights ? node_weights[in] : 1.0;
   __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
-  w_up.store(planes[0], 1.0f);
-  if (!no_element) w_skip.store(planes[1], -skip_scale);
-  if constexpr (S::kSlots == 3) w_prod.store(planes[S::kSlots - 1], 1.0f);
+  w_up.store(planes[0]);
+  if (S::kSlots >= 2 && !no_element) w_skip.store(planes[1 % S::kSlots]);
+  if constexpr (S::kSlots == 3) w_prod.store(planes[2 % S::kSlots]);
   __syncthreads();
-  rows::product_all(planes[0], typename S::Operand(v), up);
+  rows::product_all(planes[0], typename S::Operand(v), 1.0f, up);
   if (!no_element) {
-    rows::product_all(planes[1], typename S::Operand(d), skip);
+    if constexpr (S::kSlots == 1) S::replace(planes[0], w_skip);
+    rows::product_all(planes[1 % S::kSlots], typename S::Operand(d), -skip_scale, skip);
   } else {
 #pragma unroll
     for (int i = 0; i < S::NB; ++i) skip[i] = zero4();
   }
 #pragma unroll
   for (int i = 0; i < S::NB; ++i) v[i] = gh1_of(up[i], skip[i], w1 + 16 * i + 4 * (threadIdx.x % kWave / 16), scale, nw, 1.0f, no_element);
-  if constexpr (S::kSlots == 2) {
-    __syncthreads();  // every wave is done with the first planes
-    w_prod.store(planes[0], 1.0f);
-    __syncthreads();
-  }
-  rows::product_all(planes[S::kSlots == 3 ? 2 : 0], typename S::Operand(v), d);
+  if constexpr (S::kSlots < 3) S::replace(planes[2 % S::kSlots], w_prod);
+  rows::product_all(planes[2 % S::kSlots], typename S::Operand(v), 1.0f, d);
   if (here) rows::store(gB1 + at, d);
 }
 
@@ -388,7 +388,8 @@ __global__ __launch_bounds__(WAVES *kWave) void node_head_kernel(
   using S = Chain<NT, WAVES>;
   constexpr int C = S::C, kHidden = readout::kHidden, kClasses = readout::kClasses;
   constexpr int kLdW = kHidden + 2;  // row stride of W2a in LDS (doubles): the four lane groups of a read start 64 bytes apart in bank space
-  __shared__ __attribute__((aligned(16))) typename S::Planes planes[2];
+  constexpr int kSlots = NT <= 3 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) typename S::Planes planes[kSlots];
   __shared__ __attribute__((aligned(16))) double sW[C * kLdW], sw1[C];
   const int tid = threadIdx.x, lane = tid % kWave;
   const int col = lane % 16, part = lane / 16;
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(WAVES *kWave) void node_head_kernel(
   const bool row_ok = here && static_cast<unsigned>(row) < static_cast<unsigned>(nnodes);
   if (d_h2) w_back.request(prod_W);
   __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is waited for
-  w_prod.store(planes[0], 1.0f);
+  w_prod.store(planes[0]);
 #pragma unroll
   for (int i = 0; i < kWPer; ++i) {
     const int q = tid + i * S::kThreads;
@@ -420,11 +421,11 @@ __global__ __launch_bounds__(WAVES *kWave) void node_head_kernel(
   }
   if (tid < C) sw1[tid] = w1v;
   static_assert(S::kThreads >= C, "a thread per channel");
-  if (d_h2) w_back.store(planes[1], -1.0f);
+  if (kSlots == 2 && d_h2) w_back.store(planes[1 % kSlots]);
   rows::load(sc + at, a);  // the residual
   const typename S::Operand operand(x);
   __syncthreads();
-  rows::product_all(planes[0], operand, h2);
+  rows::product_all(planes[0], operand, 1.0f, h2);
 #pragma unroll
   for (int p = 0; p < S::NB; ++p) h2[p] = h2[p] + a[p];
   rows::load(h1 + at, a);
@@ -468,7 +469,8 @@ __global__ __launch_bounds__(WAVES *kWave) void node_head_kernel(
     x[p] = g;
   }
   if (here) rows::store(d_h2 + at, x);
-  rows::product_all(planes[1], typename S::Operand(x), h2);
+  if constexpr (kSlots == 1) S::replace(planes[0], w_back);
+  rows::product_all(planes[1 % kSlots], typename S::Operand(x), -1.0f, h2);
   if (here) rows::store(gB2 + at, h2);
 }
 
@@ -578,8 +580,8 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_head_few_kernel(
 }
 
 // Four waves per workgroup (64 nodes) while that is one round of workgroups, eight beyond.  us, four / eight waves, forward and backward:
-// 5 000 x 128 14.1 + 14.3 / 17.0 + 17.7, 10 752 x 64 6.9 + 6.8 / 8.4 + 8.4, 14 000 x 96 12.1 + 11.5 / 13.5 + 12.6; 25 000 x 96 20.5 + 21.2 /
-// 14.7 + 13.9, 25 000 x 128 28.9 + 29.1 / 20.7 + 20.9.
+// 5 000 x 128 17.5 + 17.0 / 21.7 + 22.1, 10 752 x 64 7.4 + 7.3 / 8.8 + 9.5, 16 000 x 96 14.4 + 13.6 / 15.9 + 15.9; 18 000 x 64 12.6 + 12.8 /
+// 9.8 + 9.9, 18 000 x 128 33.1 + 32.8 / 23.9 + 23.3, 25 000 x 96 23.5 + 23.6 / 16.8 + 17.0.
 inline bool four_waves(int64_t nnodes) { return ceil_div(nnodes, 128) * 2 < device_compute_units(); }
 
 // The chains cut at h1 / gh1 (few nodes): product and skip + up, or gh1 and product.

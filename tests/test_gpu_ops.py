@@ -594,13 +594,89 @@ def test_linear_pieces_of_the_tile_list_with_row_scale(cabi, N, C, sizes):
     assert float(out[(elem == len(sizes) - 1).to(DEV)].abs().sum()) == 0.0
 
 
-@pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256)])
+# Sizes on every kernel of the linears with 16-bit pieces: a workgroup per 128 rows of one weight block (all columns, half of them), the weights
+# resident in LDS, in registers (16 components per node and one).  (21 and 300 nodes of 64: fp32 products, to the same bounds.)
+PIECE_CASES = [(21, 64, 16), (2050, 32, 16), (2048, 64, 16), (700, 96, 16), (2049, 96, 16), (700, 128, 16), (2050, 128, 16), (1500, 160, 16),
+               (700, 192, 16), (2048, 192, 16), (1000, 224, 16), (500, 256, 16),
+               (8300, 64, 16), (8301, 96, 16), (8303, 128, 16), (9001, 160, 16), (9001, 192, 16), (9003, 224, 16), (9007, 256, 16),
+               (300, 64, 1), (9001, 32, 1), (9001, 64, 1), (9002, 96, 1), (9003, 128, 1), (9001, 160, 1), (9007, 192, 1), (9001, 224, 1), (9005, 256, 1),
+               (33_000, 160, 1), (33_003, 192, 1), (33_001, 224, 1), (33_007, 256, 1)]
+
+
+def _piece_case(N, C, ncomp, seed):
+    """Inputs on the GPU, and X . W in fp64 for any operands of their shapes."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    nl = 4 if ncomp == 16 else 1
+    X, W = torch.randn(N, ncomp, C, generator=g, device=DEV), torch.randn(nl, C, C, generator=g, device=DEV)  # W[l, j, k]: as the library takes it
+
+    def exact(x, w):
+        x, w = x.double(), w.double()
+        return torch.stack([x[:, m] @ w[math.isqrt(m) if ncomp == 16 else 0].T.contiguous() for m in range(ncomp)], 1)
+
+    return g, X, W, exact
+
+
+def _linear_of(cabi, X, W, **more):
+    if X.shape[1] == 16:
+        return cabi.linear(X, W, scale=1.0, **more)
+    return cabi.linear(X[:, 0].contiguous(), W, scale=1.0, **more)[:, None]
+
+
+@pytest.mark.parametrize("N,C,ncomp", PIECE_CASES)
+def test_linear_holds_its_operands_in_fp32(cabi, N, C, ncomp):
+    """An fp32 value is three bf16 pieces, exactly (8 bits each), and of a product only mid . lo, lo . mid and lo . lo are dropped: with
+    |mid| <= 2^-8, |lo| <= 2^-17 of a value in [1, 2) at most 2^-24 (1 + 2^-10) of it.  Rows of one value show that without a sum: 2^-24 for the
+    dropped products, 2^-24 for the rounding of the result, and 5 . 2^-31 for those of the small products' sum.  Sums of K products:
+    K roundings more, of the sum of magnitudes, whatever else lies in the row or the column: values 2^30 times the others that meet
+    zeros, and rows whose values spread over 30 powers of two."""
+    _say("linear_fp32_operands", N, C, ncomp)
+    g, X, W, exact = _piece_case(N, C, ncomp, N + C)
+    at = torch.randint(0, C, (N, ncomp, 1), generator=g, device=DEV)
+    alone = torch.zeros_like(X).scatter_(2, at, X.gather(2, at))
+    for x, w in ((alone, W), (X, torch.zeros_like(W).scatter_(2, torch.randint(0, C, W.shape[:2] + (1,), generator=g, device=DEV), torch.randn(W.shape[:2] + (1,), generator=g, device=DEV)))):
+        ref = exact(x, w)
+        err = (_linear_of(cabi, x, w).double() - ref).abs()
+        assert bool((err <= 2.1 * 2.0 ** -24 * ref.abs()).all()), float((err / ref.abs().clamp_min(1e-300)).max()) * 2 ** 24
+    k = C // 3
+    big, none = X.clone(), W.clone()
+    big[:, :, k] *= 2.0 ** 30
+    none[:, :, k] = 0.0
+    spread = torch.ldexp(X, torch.randint(-30, 1, X.shape, generator=g, device=DEV))
+    without, wide = X.clone(), W.clone()
+    without[:, :, k] = 0.0
+    wide[:, :, k] *= 2.0 ** 30
+    for x, w in ((big, none), (without, wide), (spread, W), (X, torch.ldexp(W, torch.randint(-30, 1, W.shape, generator=g, device=DEV)))):
+        err = (_linear_of(cabi, x, w).double() - exact(x, w)).abs()
+        assert bool((err <= (2.1 + C) * 2.0 ** -24 * exact(x.abs(), w.abs())).all())
+
+
+@pytest.mark.parametrize("N,C,ncomp", PIECE_CASES)
+def test_linear_keeps_infinities_in_their_row_or_column(cabi, N, C, ncomp):
+    """A row with an infinity or a NaN, a column of weights with one: nothing finite comes of them, and every other row and column has the
+    bits it has without them (the rows share tiles, the columns fragments)."""
+    _say("linear_infinities", N, C, ncomp)
+    _, X, W, _ = _piece_case(N, C, ncomp, N + C)
+    want = _linear_of(cabi, X, W)
+    rows = torch.tensor([0, 3, 17 % N, N // 2, N - 1], device=DEV).unique()
+    for value in (float("inf"), float("-inf"), float("nan")):
+        x, w = X.clone(), W.clone()
+        x[rows, -1, C - 1] = value
+        out = _linear_of(cabi, x, W)
+        assert not bool(torch.isfinite(out[rows, -1]).any())
+        out[rows, -1] = want[rows, -1]
+        assert torch.equal(out, want)
+        w[:, 5, 7] = value
+        out = _linear_of(cabi, X, w)
+        assert not bool(torch.isfinite(out[:, :, 5]).any())
+        out[:, :, 5] = want[:, :, 5]
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256),
+                                 (8300, 64), (8301, 96), (8303, 128), (9001, 160), (9001, 192), (9003, 224), (9007, 256)])
 def test_linear_scales_of_rows_and_columns(cabi, N, C):
-    """The kernels with resident weights scale rows of X and columns of W by powers of two: rows and columns multiplied by powers of
-    two give the same bits, multiplied alike (as long as nothing leaves the normal range), also next to rows of zeros, in one tile
-    with huge ones.  Errors stay within the bound of the split, element by element: |x w| times 3 * 2^-24 for the two roundings and
-    the dropped product, 2^-39 of the row's and the column's largest values for what falls below the pieces' range, and K fp32 sums
-    (at most K 2^-24 of the sum of magnitudes), on rows whose values spread over 30 powers of two."""
+    """Rows of X and columns of W multiplied by powers of two give the same bits, multiplied alike (as long as nothing leaves the normal
+    range), also next to rows of zeros, in one tile with huge ones, with a workgroup per 128 rows and with resident weights."""
     _say("linear_scales", N, C)
     g = torch.Generator().manual_seed(C)
     X, W = torch.randn(N, 16, C, generator=g), torch.randn(4, C, C, generator=g)
@@ -618,13 +694,6 @@ def test_linear_scales_of_rows_and_columns(cabi, N, C):
         base = cabi.linear(d(X), d(W), scale=0.7, **more)
         out = cabi.linear(d(grown), d(torch.ldexp(W, columns)), scale=0.7, **more)
         assert torch.equal(out, base * d(factor))
-    spread = torch.ldexp(X, torch.randint(-30, 1, X.shape, generator=g))
-    out = cabi.linear(d(spread), d(W), scale=1.0).double().cpu()
-    xd, wd = spread.double(), W.double()[lm]                      # [16, C, C], W^T rows are output columns
-    ref = torch.einsum("nmk,mjk->nmj", xd, wd)
-    size = torch.einsum("nmk,mjk->nmj", xd.abs(), wd.abs())
-    floor = 2.0 ** -39 * (xd.abs().amax(-1, keepdim=True) * wd.abs().sum(-1) + xd.abs().sum(-1, keepdim=True) * wd.abs().amax(-1))
-    assert bool(((out - ref).abs() <= (3.0 + C) * 2.0 ** -24 * size + floor).all())
 
 
 @pytest.mark.parametrize("N,C", [(8192, 160), (8193, 192), (9007, 224), (12345, 256)])
