@@ -1420,10 +1420,14 @@ bool resident_weights(int64_t nnodes, int ncomp, int K, int ngroups, bool groupe
 //    where at least half of it is filled: 2 500 16.7 / 20.1 / 18.0 / 22.5 -> 17.9 / 19.7 / 19.3 / 21.4, 3 500 23.3 / 26.1 / 22.1 / 27.3 -> 20.2 / 23.8 / 21.8 / 25.8,
 //    5 000 27.1 / 31.5 / 27.7 / 34.2 -> 27.5 / 30.7 / 29.5 / 33.1.  Beyond 128 columns it does not: 2 500 x 160 21.2 / 26.6 / 22.7 / 29.8 -> 25.4 / 27.3 / 27.1 / 29.5, 2 500 x
 //    224 32 / 40 / 34 / 43 -> 40 / 45 / 44 / 50, 16 000 and 24 000 x 192 of one component 14.7 / 20.7 -> 12.3 / 19.9 and 18.2 / 21.6 -> 20.0 / 22.6.
-//  - beyond it against the tiled kernels: one component up to 128 columns always (100 000 x 96 26.7 -> 20.2, 33 000 x 128 16.2 -> 16.8: it has the
-//    arithmetic of the chains of such products, node_glue.hip), at 224 with groups (33 000 50 -> 40; with row_scale 50 000 56 -> 70; at 192 24 000 21.6 -> 22.6); 16
-//    components with groups below 2 048 nodes at 224 columns (1 500 49 -> 31, 2 000 49 -> 42) and, unless the tiled kernel's workgroups are one
-//    round, at 256 (700 32 -> 24, 1 000 34 -> 33, 1 500 in two rounds 59 -> 44, 2 000 60 -> 53), not at 160 and 192 (2 000 22.4 -> 27.3, 28.4 -> 33.3).
+//  - beyond it where resident weights are not to be had, against the tiled kernels.  Up to 128 columns always (16 components with a residual / 130 groups: 9 000 x 32
+//    22 / 42 -> 12 / 12, 15 000 x 64 39 / 82 -> 32 / 33, 30 000 x 96 149 / 164 -> 127 / 99, 30 000 x 128 202 / 191 -> 160 / 171; 32 columns, plain, 30 000 28.2 -> 21.2, 100 000
+//    80.0 -> 81.9; one component 100 000 x 96 26.7 -> 20.2, 33 000 x 128 16.2 -> 16.8: it has the arithmetic of the chains of such products, node_glue.hip).  With many
+//    weight groups, each of which costs the others sixteen part-filled tiles and this one four, always (130: 1 000 x 160 94 -> 42, 20 000 x 160 208 -> 179, 20 000
+//    x 192 271 -> 258, 2 500 x 256 288 -> 100).  With a residual on 16 components up to 6 000 nodes (5 000 x 192 66 -> 56, 5 000 x 256 114 -> 103; 9 000 101 -> 102, 188 ->
+//    192), at 160 columns always (20 000 160 -> 155).  With few groups below 2 048 nodes at 224 columns (1 500 49 -> 31, 2 000 49 -> 42) and, unless the tiled kernel's
+//    workgroups are one round, at 256 (700 32 -> 24, 1 000 34 -> 33, 1 500 in two rounds 59 -> 44, 2 000 60 -> 53), not at 160 and 192 (2 000 22.4 ->
+//    27.3, 28.4 -> 33.3); one component at 224 (33 000 50 -> 40; with row_scale 50 000 56 -> 70), at 192 24 000 21.6 -> 22.6.
 int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, bool scaled, bool residual) {
   // a workgroup per 128 rows, and on average half of the weight blocks end in one more
   const int64_t rows = ceil_div(nnodes * ncomp, kBlockRows) + (grouped ? static_cast<int64_t>(ngroups) * (ncomp == 1 ? 1 : 4) / 2 : 0);
@@ -1434,9 +1438,11 @@ int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, b
   if (2 * rows <= round && K != 224) return most / 2;
   if (rows <= round) return K == 224 && ncomp == 1 && !grouped && nnodes <= 4096 ? 0 : most;
   if (resident) return (K < 128 && rows <= 4 * units) || (K == 128 && 2 * rows > 3 * units && rows <= 2 * units) ? most : 0;
-  if (K <= 128) return ncomp == 1 || rows <= 4 * units ? most : 0;
+  if (K <= 128) return most;
   if (ncomp == 1) return K == 224 && grouped && !scaled ? most : 0;
-  if (!grouped || K <= 192 || nnodes >= kResMinNodes) return 0;
+  if (ngroups > 16) return most;
+  if (nnodes >= kResMinNodes) return K == 160 || nnodes <= 6000 ? most : 0;
+  if (!grouped || K <= 192) return 0;
   return K == 224 || rows <= 2 * round || 4 * 16 * (ceil_div(nnodes, 128) + ngroups / 2) > 5 * units ? most : 0;
 }
 

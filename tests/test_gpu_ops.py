@@ -484,8 +484,8 @@ def test_linear_few_rows(cabi, N, C, ncomp, ne):
 
 @pytest.mark.parametrize("N,C,ne,seed", [(2048, 128, 1, 0), (2500, 128, 10, 1), (4099, 96, 5, 2), (3000, 64, 3, 3), (6000, 128, 130, 4)])
 def test_linear_many_rows(cabi, N, C, ne, seed):
-    """16-component features with 64 / 96 / 128 square weights at some thousand nodes: a workgroup per 128 rows of one weight
-    block; more than 128 weight groups stay on the tiled kernels.  Groups of very different sizes, an empty group, a group of one node, tiles that end inside a group,
+    """16-component features with square weights at some thousand nodes: up to 128 columns a workgroup per 128 rows of one weight
+    block.  Groups of very different sizes, an empty group, a group of one node, tiles that end inside a group,
     rows of no group, with and without row_scale; twice, for the same bits."""
     _say("linear_many_rows", N, C, ne, seed)
     g = torch.Generator().manual_seed(seed)
@@ -541,6 +541,36 @@ def test_linear_rows_of_a_weight_block(cabi, N, C, ne, seed):
     resident, 16-row tiles), more than 64 weight groups, one and two rounds of workgroups at 160 to 256 columns, half and all columns per
     workgroup."""
     test_linear_many_rows(cabi, N, C, ne, seed)
+
+
+@pytest.mark.parametrize("N,C,ne,seed", [(10_000, 64, 130, 0), (10_001, 96, 131, 1), (10_003, 128, 130, 2), (8300, 32, 1, 3), (33_000, 32, 3, 4), (3001, 160, 129, 5),
+                                         (2100, 192, 130, 6), (2500, 224, 130, 7), (2100, 256, 140, 8), (1000, 192, 16, 9), (1000, 192, 17, 10)])
+def test_linear_where_no_weights_are_resident(cabi, N, C, ne, seed):
+    """More weight groups than the kernels with resident weights take, and 32 columns, for which there is none: a workgroup per 128 rows of one
+    weight block at any number of nodes (with few groups and beyond 128 columns the tiled kernels)."""
+    test_linear_many_rows(cabi, N, C, ne, seed)
+
+
+@pytest.mark.parametrize("N,C", [(9000, 32), (9001, 64), (8300, 96), (8301, 128), (9003, 160), (6000, 192), (6001, 192), (2500, 224), (2050, 256), (6001, 256)])
+def test_linear_with_a_residual_on_many_rows(cabi, N, C):
+    """A residual on 16 components, which the kernels with resident weights do not take: both sides of the line (6 000 nodes beyond 160
+    columns), with row_scale and with a residual that is the output itself."""
+    _say("linear_with_a_residual_on_many_rows", N, C)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    X, R = (torch.randn(N, 16, C, generator=g, device=DEV) for _ in range(2))
+    S, WT = torch.randn(N, C, generator=g, device=DEV), torch.randn(4, C, C, generator=g, device=DEV)
+    rows = torch.randperm(N, device=DEV, generator=g)[:700]
+    rows[:2] = torch.tensor([0, N - 1], device=DEV)
+    x, w, r = X[rows].double().cpu(), WT.transpose(-1, -2).double().cpu(), R[rows].double().cpu()
+    for scale in (None, S):
+        more = {} if scale is None else {"row_scale": scale}
+        xs = x if scale is None else x * scale[rows].double().cpu()[:, None]
+        out = cabi.linear(X, WT, residual=R, **more)
+        close(out[rows], O.linear(xs, w) + r, 1e-5, 2e-6)
+        inout = R.clone()
+        cabi._check(cabi.lib.cm_linear(X.data_ptr(), WT.data_ptr(), None, None, N, 1, 0, 16, C, C, 1.0 / math.sqrt(C), scale.data_ptr() if more else None,
+                                       inout.data_ptr(), inout.data_ptr(), cabi._stream()))
+        assert torch.equal(inout, out)
 
 
 @pytest.mark.parametrize("N,C,ne", [(1000, 160, 3), (3001, 192, 10), (9001, 256, 10), (8200, 224, 63), (8193, 160, 70), (33_000, 192, 2), (5000, 32, 3), (3100, 128, 130)])
