@@ -869,14 +869,25 @@ int forward_parts(int64_t nnodes, int64_t nedges) {
 // filled by a share f takes 0.55 + 0.45 f of a full one.  us without / with gX at p = 1 2 3 4 6 8, the rule's p in brackets: 128 channels 216 x
 // 52 26.1 / 40 16.2 / 24 12.3 / 19 10.4 / 17 9.3 / 15.6 [9.3 / 15.7], 700 x 52 28.7 / 43 [20.2 / 31] 22.3 / 33 21.8 / 33 23.8 / 36 25.2 / 37, 1 200 x 52
 // 33.4 / 49 31.5 / 47 [28.5 / 43], 2 200 x 52 58 / 81 [53.5 / 75] 55.3 / 79, 3 300 x 52 [68.9 / 98.7] 67.5 / 98.5 72 / 106, 5 000 x 52 [105.6 / 149]
-// 107 / 150 116 / 162, 2 500 x 12 [20.3 / 29.9] 22.1 / 32.4; 64 21 x 9 6.2 / 9.7 5.3 / 8.7 4.8 / 8.1 4.6 / 8.3 (five: [4.3 / 7.8]) 4.3 / 7.9 4.3 / 8.1,
-// 1 200 x 52 19.7 / 29.9 [16.5 / 25.5] 18.3 / 28.2; 256 21 x 12 16.2 / 24 10.1 / 15.6 7.7 / 12.7 7.1 / 11.5 5.8 / 9.9 [5.3 / 9.5], 1 200 x 52 64 / 98 59 / 85
+// 107 / 150 116 / 162, 2 500 x 12 [20.3 / 29.9] 22.1 / 32.4; 256 21 x 12 16.2 / 24 10.1 / 15.6 7.7 / 12.7 7.1 / 11.5 5.8 / 9.9 [5.3 / 9.5], 1 200 x 52 64 / 98 59 / 85
 // [55 / 78]; 160 2 200 x 52 76 / 109 [67 / 98] 68 / 101.
-template <int C, bool FROM_VEC>
+// Up to 64 channels a wave's loads are a quarter or half of that, its start-up is not, and more than a round of waves never pays: eight
+// waves per compute unit, five parts at most (400 x 52 x 64 five 8.1, eight 10.9), of two edges each, beyond two nodes per unit of 256 / C;
+// two parts of 16 edges while they fit twelve waves.  us without gX at p = 1 2 3 4 5: 64 channels 21 x 9 6.2 5.3 4.8 4.6 [4.3], 120 x 52
+// 17.1 10.1 8.4 7.4 [7.0], 500 x 52 17.3 10.7 9.8 [9.4] 10.4, 1 000 x 52 17.9 [13.4] 14.3 16.6 17.2, 1 500 x 52 21.9 [18.9] 20.9, 1 800 x 52 [23.3] 23.9
+// 24.7, 2 000 x 52 [25.3] 26.6 26.4, 800 x 20 10.5 [8.6] 9.1, 1 200 x 20 [10.6] 10.5, 300 x 9 6.9 6.2 6.0 5.6 [5.8], 500 x 9 7.0 6.5 6.2 [6.4], 1 000 x
+// 9 7.5 [7.4]; 32 channels 500 x 52 11.5 7.8 7.5 [7.4], 1 500 x 52 14.1 [12.2] 14.1, 2 000 x 52 [15.4] 16.8 17.6, 800 x 20 7.2 [6.8], 1 500 x 20 [8.2] 9.0,
+// 1 000 x 9 [6.0] 6.6 7.6.
+template <int C>
 int backward_parts(int64_t nnodes, int64_t nedges) {
   if (nnodes <= 0) return 1;
-  constexpr int kMost = C <= 64 ? 5 : 8;  // (narrow rows: 400 x 52 x 64 five 8.1 us, eight 10.9)
-  const double slots = device_compute_units() * (kOneOperandSet<C, FROM_VEC> ? 12.0 : 8.0);
+  if constexpr (C <= 64) {
+    const int64_t units = device_compute_units(), each = nedges / nnodes, least = nnodes > 2 * units ? 256 / C : 2;
+    const int64_t parts = std::min<int64_t>(5, std::min(8 * units / nnodes, (each + 1) / least));
+    return static_cast<int>(parts < 2 && nnodes <= 6 * units && each >= 32 ? 2 : std::max<int64_t>(1, parts));
+  }
+  constexpr int kMost = 8;
+  const double slots = device_compute_units() * 8.0;
   const double edges = static_cast<double>(nedges) / static_cast<double>(nnodes);
   int best = 1;
   double least = 0.0;
@@ -929,7 +940,7 @@ template <int C, bool FROM_VEC, bool GY, bool GR, bool GX>
 void launch_edge(const float *X, const float *Y, const Spline &sp, const float *G, const int32_t *sender,
                  const int32_t *first_occ, int64_t nnodes, int64_t nedges, float *gY, float *g_r, float *gXe,
                  hipStream_t st) {
-  const int parts = backward_parts<C, FROM_VEC>(nnodes, nedges);
+  const int parts = backward_parts<C>(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
   if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {
     if (steps_of_four_edges<C>(nnodes, nedges, parts)) {
@@ -1035,7 +1046,7 @@ extern "C" int cm_mp_edge_forward_kernel(int64_t nnodes, int64_t nedges, int cha
 extern "C" int cm_mp_edge_backward_kernel(int64_t nnodes, int64_t nedges, int channels) {
   if (nnodes <= 0) return 0;
   bool steps = false;
-  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, (cm::backward_parts<C_, true>(nnodes, nedges))));
+  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, cm::backward_parts<C_>(nnodes, nedges)));
   return steps ? 1 : 0;
 }
 

@@ -307,7 +307,8 @@ def test_mp_edge_backward_of_four_edges_per_step(cabi, case):
     assert torch.equal(cabi.mp_edge_backward(*args, need_gX=False)[1], gvec)
 
 
-@pytest.mark.parametrize("case", [(40, 9, 160, 0.0, 31, 3, 0), (90, 21, 192, 0.0, 32, 257, 150), (300, 19, 224, 0.1, 33, 600, 150),
+@pytest.mark.parametrize("case", [(120, 9, 64, 0.1, 51, 256, 0), (409, 20, 32, 0.0, 52, 256, 0), (513, 16, 32, 0.1, 53, 256, 0), (1024, 9, 64, 0.0, 54, 256, 0), (1025, 33, 64, 0.0, 55, 256, 0),
+                                  (1536, 33, 32, 0.2, 56, 256, 0), (1537, 33, 32, 0.0, 57, 256, 150), (40, 9, 160, 0.0, 31, 3, 0), (90, 21, 192, 0.0, 32, 257, 150), (300, 19, 224, 0.1, 33, 600, 150),
                                   (1100, 13, 224, 0.0, 34, 256, 129), (40, 7, 64, 0.0, 35, 4, 0), (300, 13, 64, 0.1, 36, 512, 150),
                                   (1100, 9, 32, 0.1, 37, 5, 150), (2100, 6, 128, 0.1, 38, 513, 70), (300, 17, 96, 0.0, 39, 256, 130)],
                          ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
