@@ -520,19 +520,24 @@ int launch_backward(const float *X, const float *Y, const float *R, const float 
 }
 
 // Waves per sender: four rows each while they fit three rounds of half a chip's waves (a row is one load, and what a wave waits for is
-// its list and its first rows).  us of edge and sender pass at 1 2 3 4 6 8, the rule's in brackets: 128 channels 216 x 52 21.2 17.9 16.7 16.4
+// its list and its first rows); at 64 and 32 channels, where a load covers four rows and eight, up to eight rows, and twelve.  us of edge and
+// sender pass at 1 2 3 4 6 8, the rule's in brackets: 128 channels 216 x 52 21.2 17.9 16.7 16.4
 // 15.7 [15.8], 700 x 52 34.8 31.2 30.4 [30.5] 31.3 30.9, 1 500 x 52 53.6 [52.4] 52.3 52.2 53.9 53.4, 672 x 9 14.5 [13.8] 13.9 14.3 15.1 15.4;
-// 256 60 x 30 20.1 15.9 14.4 13.6 [12.8] 13.0, 216 x 52 36.8 30.5 27.7 26.9 25.1 [25.0], 300 x 9 15.7 [14.5] 14.0 14.1 14.9 15.2; 64 21 x 19 8.6
-// 8.1 8.3 [8.4] 8.6 8.8.
-inline int sender_parts(int64_t nnodes, int64_t nedges) {
+// 256 60 x 30 20.1 15.9 14.4 13.6 [12.8] 13.0, 216 x 52 36.8 30.5 27.7 26.9 25.1 [25.0], 300 x 9 15.7 [14.5] 14.0 14.1 14.9 15.2; 64
+// 21 x 9 8.0 [7.9] 8.2 (the sender pass in the step 4.1 [3.9] 4.0, of four such molecules 4.3 [3.8] 3.9, one with 216 x 10 3.4 [4.1]), 21 x 19 8.5 8.0
+// [8.2] 8.4 8.5, 60 x 30 10.1 9.7 8.9 [9.1] 9.2, 300 x 20 10.8 10.5 [10.2] 10.4 11.7, 216 x 52 14.2 13.2 12.6 12.5 [11.9] 12.0; 32 21 x 9 [7.0] 7.5 7.6 (in the
+// step [3.4] 3.8 3.9), 60 x 30 8.3 [7.9] 8.0 8.2, 672 x 9 [9.1] 9.6 10.4, 216 x 52 10.9 10.4 9.7 [9.8] 10.1.
+template <int C>
+int sender_parts(int64_t nnodes, int64_t nedges) {
   if (nnodes <= 0) return 1;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(8, std::min(3072 / nnodes, nedges / (4 * nnodes)))));
+  const int64_t by_rows = C == 32 ? nedges / (12 * nnodes) : (C == 64 ? ceil_div(nedges, 8 * nnodes) : nedges / (4 * nnodes));
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(8, std::min(3072 / nnodes, by_rows))));
 }
 
 template <int C>
 int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes, int64_t nedges,
                   float *gX, hipStream_t st, const float *live_vec, const float *live_r, float r_max, const uint32_t *live_bits) {
-  const int parts = sender_parts(nnodes, nedges);
+  const int parts = sender_parts<C>(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes)), block(parts * kWave);
 #define CM_SENDER(LIVE_, by_, rmax_)                                                                                                   \
   do {                                                                                                                                 \
