@@ -61,7 +61,7 @@ constexpr unsigned kSlRowBytes = 576;  // of a knot interval: 512 and a quarter 
 constexpr int kSlMaxIntervals = 272;   // 153 KB of table (one row of it is the row of zeros)
 constexpr int kSlSub = 2816;          // nodes sorted at a time: what LDS holds next to the largest table
 constexpr int kSlBins = 64;           // edge blocks per node that the sort tells apart
-// From nearly five rounds of 16 nodes per workgroup on (2 432 nodes at 64 channels, 1 216 at 128; 3 840 and 768 at 32 and 160); below
+// From nearly five rounds of 16 nodes per workgroup on (2 432 nodes at 64 channels, 1 216 at 128; three to four at 160 to 256, see the numbers below); below
 // that most of its waves have none.  From there on the edges decide: a workgroup spends 3 us on its slice of the table, and
 // nodes with few edges leave it with the fixed part of a round, while the kernel with one wave per node pays per edge.
 // Measured, the launch alone, one wave per node -> this one (us), nodes x neighbours:
@@ -102,6 +102,14 @@ constexpr int kSlBins = 64;           // edge blocks per node that the sort tell
 // 186.5; 224 400 x 52 234.7 -> 224.0, x 26 201.1 -> 197.1, 60 molecules of 21 (8.8 neighbours) 277.5 -> 271.8; 256 560 x 52 273.3 -> 266.4, x 26
 // 226.1 -> 227.0, 500 x 52 247.4 -> 250.2, molecules of 21: 96 398.9 -> 389.4, 190 (7.3) 513.3 -> 499.1, 240 617 -> 597; 96 190 molecules 216.1 ->
 // 211.2, (7.3) 206.9 -> 206.7; 192 190 molecules (7.3) 394.6 -> 385.5.
+//
+// 256 channels around 5 000 nodes, steps with forces: batches of molecules of 21 with 8.8 neighbours gain at every size (3 150 nodes 528 -> 502, 5 040
+// 716 -> 680, 6 006 805 -> 768, 9 996 1 279 -> 1 233), periodic ones from eight to nine neighbours on (3 000 x 7 442 -> 445, 4 000 x 7 493 -> 499, x 8.4
+// 556 -> 547, 5 100 x 7 608 -> 615, x 8.4 688 -> 684, 6 000 x 7 692 -> 708, x 8.4 780 -> 787, 8 000 x 7 873 -> 891, x 8.4 984 -> 986): the line rises
+// from 6.75 neighbours at 5 000 nodes to 8.25 at 8 000 and 9 at 12 000.
+//
+// Nodes of a (pair of degrees, slice) that a workgroup has at least.  There are share_of(channels) workgroups for each, so the lines are 3 840
+// nodes at 32 channels, 2 432, 1 596 and 1 216 at 64, 96 and 128, and 528, 580, 387 and 552 at 160 to 256; both sides of them are above.
 inline int64_t min_nodes_per_workgroup(int channels) {
   switch (channels) {
     case 32: return 60;
@@ -126,7 +134,7 @@ inline int64_t min_edges(int64_t nnodes, int channels) {
       case 160: return {std::max(3500 + 7 * nnodes / 2, 21 * nnodes / 5), 6.5, 2.5};
       case 192: return {std::max(4000 + 11 * nnodes / 2, 7 * nnodes), 9.0, 1.9};
       case 224: return {std::max(7000 + 3 * nnodes, 9 * nnodes / 2), 6.0, 1.5};
-      default: return {nnodes <= 5000 ? 5000 + 23 * nnodes / 4 : 21 * nnodes / 2, 11.0, 2.0};  // (82 MB of output)
+      default: return {std::max(5000 + 23 * nnodes / 4, 43 * nnodes / 4 - 20000), 11.0, 2.0};
     }
   }();
   const double caches = 64.0 * static_cast<double>(nnodes) * channels / (1 << 28);  // 16 components of 4 bytes in 256 MB

@@ -54,6 +54,11 @@ def test_the_library_names_the_kernels_it_takes():
     assert forward(25000, 1301200, 128, 300) == 0  # the table does not fit LDS
     assert forward(500, 50000, 128) == 0 and forward(25000, 0, 128) == 0 and forward(0, 0, 128) == 0 and forward(25000, 1301200, 48) == 0
     assert forward(20000, 89999, 128) == 0 and forward(20000, 90000, 128) == 1
+    # at 256 channels one line without a step, which 240 molecules of 21 with 8.8 neighbours are above
+    assert forward(5040, 44352, 256) == 1 and [forward(5000, e, 256) for e in (33749, 33750)] == [0, 1]
+    assert [forward(5001, e, 256) for e in (33759, 33760)] == [0, 1] and [forward(8000, e, 256) for e in (65999, 66000)] == [0, 1]
+    # and the nodes below which its workgroups have too few: 8 of them per pair of degrees and slice at 256 channels
+    assert [forward(n, 52 * n, 256) for n in (552, 553)] == [0, 1] and [forward(n, 52 * n, 160) for n in (528, 529)] == [0, 1]
     # output of twice the last-level cache and more: 11 neighbours, and two more for every doubling
     n = 1 << 15
     assert forward(n, 13 * n - 1, 256) == 0 and forward(n, 13 * n, 256) == 1 and forward(2 * n, 15 * 2 * n - 1, 256) == 0
