@@ -540,7 +540,8 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
   }
   if constexpr (MODE == Scan::kGraph) {
     wave_lds_fence();
-    const int d = min(min(count, cap), static_cast<int>(min(static_cast<int64_t>(offsets[i + 1]), nedges) - seg));
+    // never below zero: where the caller's `nedges` ends before the segment begins, nothing of it is written, here neither
+    const int d = max(0, min(min(count, cap), static_cast<int>(min(static_cast<int64_t>(offsets[i + 1]), nedges) - seg)));
     // up to the next multiple of four (cap is one): keys above all others
     if (lane < (-d & 3)) hkey[d + lane] = ~0ull;
     wave_lds_fence();

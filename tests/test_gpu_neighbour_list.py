@@ -138,6 +138,48 @@ def test_graph_of_a_list(cabi, name):
     assert torch.equal(cabi_mod.symmetric_sender_view(g["row_i"], g["row_j"], g["unit_shifts"], g["first_occ"], n), perm)
 
 
+def _search(cabi_mod, p, c, pbc, cutoff):
+    """cm_neighbour_list_search as the header has it: the workspace, offsets [N + 1], status [1] and max_degree [1], left on the device."""
+    n = p.shape[0]
+    max_cells = max(1, n)
+    size = cabi_mod.lib.cm_neighbour_list_workspace(n, max_cells)
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+    offsets, numbers = torch.full((n + 1,), -7, dtype=torch.int32, device=DEV), torch.full((2,), -7, dtype=torch.int32, device=DEV)
+    cabi_mod._check(cabi_mod.lib.cm_neighbour_list_search(p.data_ptr(), c.data_ptr() if c is not None else None, *(int(b) for b in pbc), cutoff, n, max_cells,
+                                                          ws.data_ptr(), size, offsets.data_ptr(), numbers.data_ptr(), numbers.data_ptr() + 4,
+                                                          cabi_mod._stream()))
+    return ws, max_cells, offsets, numbers
+
+
+@pytest.mark.parametrize("n,box,cutoff", [(300, 12.0, 4.0), (700, 9.0, 5.5), (4097, 34.5, 4.0)])
+def test_graph_into_fewer_places_than_pairs(cabi, n, box, cutoff):
+    """cm_neighbour_list_graph with `nedges` below the number of pairs: the segments that end before it come out whole, nothing is written
+    behind it, and segments that begin behind it (their room is negative) touch nothing."""
+    from cuda_mace import _cabi as cabi_mod
+
+    p = torch.tensor(np.random.default_rng(n).uniform(0.0, box, (n, 3)), dtype=torch.float64, device=DEV)
+    c = torch.eye(3, dtype=torch.float64, device=DEV) * box
+    whole = cabi_mod.neighbour_graph(p, c, (True,) * 3, cutoff)
+    ws, max_cells, offsets, numbers = _search(cabi_mod, p, c, (True,) * 3, cutoff)
+    pairs = whole["row_i"].numel()
+    for nedges in (pairs - 1, pairs // 2 + 1, 3):
+        guard = 64
+        ri, rj = (torch.full((nedges + guard,), -5, dtype=torch.int32, device=DEV) for _ in range(2))
+        index = torch.full((2 * nedges + guard,), -5, dtype=torch.int64, device=DEV)
+        S, shifts = (torch.full((nedges + guard, 3), -5.0, dtype=torch.float64, device=DEV) for _ in range(2))
+        fo = torch.empty(2 * n, dtype=torch.int32, device=DEV)
+        cabi_mod._check(cabi_mod.lib.cm_neighbour_list_graph(cutoff, n, max_cells, ws.data_ptr(), offsets.data_ptr(), nedges, int(numbers[1]), ri.data_ptr(),
+                                                             rj.data_ptr(), index.data_ptr(), S.data_ptr(), shifts.data_ptr(), fo.data_ptr(), None, None, None,
+                                                             cabi_mod._stream()))
+        inside = int(offsets[offsets <= nedges].max())  # pairs of segments that fit
+        assert torch.equal(ri[:inside], whole["row_i"][:inside]) and torch.equal(rj[:inside], whole["row_j"][:inside])
+        assert torch.equal(index[:inside], whole["edge_index"][0, :inside]) and torch.equal(index[nedges:nedges + inside], whole["edge_index"][1, :inside])
+        assert torch.equal(S[:inside], whole["unit_shifts"][:inside]) and torch.equal(shifts[:inside], whole["shifts"][:inside])
+        assert bool((ri[nedges:] == -5).all()) and bool((rj[nedges:] == -5).all()) and bool((index[2 * nedges:] == -5).all())
+        assert bool((S[nedges:] == -5).all()) and bool((shifts[nedges:] == -5).all())
+        assert torch.equal(fo, whole["first_occ"])
+
+
 @pytest.mark.parametrize("n", [0, 1, 300, 4097])
 @pytest.mark.parametrize("fills", [0, 60])
 def test_counts_reach_a_waiting_host(cabi, n, fills):
