@@ -1435,7 +1435,7 @@ int block_columns(int64_t nnodes, int ncomp, int K, int ngroups, bool grouped, b
   const int all = K / 16, most = K <= 160 ? all : (K == 256 ? all / 4 : all / 2);  // what fits LDS
   const int64_t round = units / (all / most);
   const bool resident = resident_weights(nnodes, ncomp, K, ngroups, grouped, residual);
-  if (2 * rows <= round && K != 224) return most / 2;
+  if (2 * rows <= round && K != 224 && K != 32) return most / 2;  // (so few rows of 32 columns are the few-rows kernel's)
   if (rows <= round) return K == 224 && ncomp == 1 && !grouped && nnodes <= 4096 ? 0 : most;
   if (resident) return (K < 128 && rows <= 4 * units) || (K == 128 && 2 * rows > 3 * units && rows <= 2 * units) ? most : 0;
   if (K <= 128) return most;
@@ -1600,7 +1600,7 @@ extern "C" int cm_linear(const float *X, const float *W_T, const int32_t *node_p
     switch (32 * K + cm::block_columns(nnodes, ncomp, K, ngroups, group_offsets != nullptr, row_scale != nullptr, residual != nullptr)) {
 #define CM_CASE(KS_, NB_) \
       case 32 * 32 * KS_ + NB_: return cm::launch_block<KS_, NB_>(X, W_T, node_perm, group_offsets, nnodes, ngroups, zero_last_group, ncomp, scale, row_scale, residual, OUT, st);
-      CM_CASE(1, 2) CM_CASE(1, 1) CM_CASE(2, 4) CM_CASE(2, 2) CM_CASE(3, 6) CM_CASE(3, 3) CM_CASE(4, 8) CM_CASE(4, 4) CM_CASE(5, 10) CM_CASE(5, 5)
+      CM_CASE(1, 2) CM_CASE(2, 4) CM_CASE(2, 2) CM_CASE(3, 6) CM_CASE(3, 3) CM_CASE(4, 8) CM_CASE(4, 4) CM_CASE(5, 10) CM_CASE(5, 5)
       CM_CASE(6, 6) CM_CASE(6, 3) CM_CASE(7, 7) CM_CASE(8, 4) CM_CASE(8, 2)
 #undef CM_CASE
     }

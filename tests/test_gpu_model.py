@@ -571,7 +571,7 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
 @pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32),
                                              (60, 192), (400, 160), (300, 224), (1536, 256), (1537, 256)])
 def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
-    """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 32
+    """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 64
     and 128 nodes with a partly filled last one, against the separate launches: bit for bit, for forces and for energies alone,
     with weights on the node energies and without.  Beyond 128 channels the products between the layers in two launches per direction,
     for few nodes."""

@@ -108,11 +108,24 @@ GRAPH_CASES = {
 }
 
 
+def _search(cabi_mod, p, c, pbc, cutoff):
+    """cm_neighbour_list_search as the header has it: the workspace, offsets [N + 1], status [1] and max_degree [1], left on the device."""
+    n = p.shape[0]
+    max_cells = max(1, n)
+    size = cabi_mod.lib.cm_neighbour_list_workspace(n, max_cells)
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+    offsets, numbers = torch.full((n + 1,), -7, dtype=torch.int32, device=DEV), torch.full((2,), -7, dtype=torch.int32, device=DEV)
+    cabi_mod._check(cabi_mod.lib.cm_neighbour_list_search(p.data_ptr(), c.data_ptr() if c is not None else None, *(int(b) for b in pbc), cutoff, n, max_cells,
+                                                          ws.data_ptr(), size, offsets.data_ptr(), numbers.data_ptr(), numbers.data_ptr() + 4,
+                                                          cabi_mod._stream()))
+    return ws, max_cells, offsets, numbers
+
+
 @pytest.mark.parametrize("name", list(GRAPH_CASES))
 def test_graph_of_a_list(cabi, name):
-    """cm_neighbour_list_search / _graph: the pairs of cm_neighbour_list_count / _fill (held against the oracle above; against
-    the oracle here too where it is quick), the same in int64 and fp64, shifts, CSR offsets, batch and ptr; and
-    cm_symmetric_sender_view against the stable sort by sender."""
+    """cm_neighbour_list_search_counts / _graph: the pairs of cm_neighbour_list_count / _fill (held against the oracle above; against
+    the oracle here too where it is quick), the same in int64 and fp64, shifts, CSR offsets, batch and ptr;
+    cm_neighbour_list_search, which leaves the same numbers on the device; and cm_symmetric_sender_view against the stable sort by sender."""
     from cuda_mace import _cabi as cabi_mod
     from cuda_mace.utils.neighbour_list import shifts_from_unit_shifts
 
@@ -135,20 +148,9 @@ def test_graph_of_a_list(cabi, name):
     assert g["batch"].tolist() == [0] * n and g["ptr"].tolist() == [0, n] and g["ptr32"].tolist() == [0, n]
     perm, off = cabi_mod.stable_key_sort(rj, n)
     assert torch.equal(g["offsets"], off)
+    _, _, offsets, numbers = _search(cabi_mod, p, c, pbc, cutoff)
+    assert torch.equal(offsets, off) and numbers.tolist() == [0, int((off[1:] - off[:-1]).max())]
     assert torch.equal(cabi_mod.symmetric_sender_view(g["row_i"], g["row_j"], g["unit_shifts"], g["first_occ"], n), perm)
-
-
-def _search(cabi_mod, p, c, pbc, cutoff):
-    """cm_neighbour_list_search as the header has it: the workspace, offsets [N + 1], status [1] and max_degree [1], left on the device."""
-    n = p.shape[0]
-    max_cells = max(1, n)
-    size = cabi_mod.lib.cm_neighbour_list_workspace(n, max_cells)
-    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
-    offsets, numbers = torch.full((n + 1,), -7, dtype=torch.int32, device=DEV), torch.full((2,), -7, dtype=torch.int32, device=DEV)
-    cabi_mod._check(cabi_mod.lib.cm_neighbour_list_search(p.data_ptr(), c.data_ptr() if c is not None else None, *(int(b) for b in pbc), cutoff, n, max_cells,
-                                                          ws.data_ptr(), size, offsets.data_ptr(), numbers.data_ptr(), numbers.data_ptr() + 4,
-                                                          cabi_mod._stream()))
-    return ws, max_cells, offsets, numbers
 
 
 @pytest.mark.parametrize("n,box,cutoff", [(300, 12.0, 4.0), (700, 9.0, 5.5), (4097, 34.5, 4.0)])

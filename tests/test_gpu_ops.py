@@ -403,7 +403,7 @@ def test_scalar_elemental_linear_and_zero_group(cabi, N, K, Nout, ne, seed):
     close(out16, ref16, 1e-5, 2e-6)
 
 
-@pytest.mark.parametrize("N,C,ne,seed", [(1, 32, 1, 0), (21, 64, 4, 1), (700, 128, 10, 2), (5000, 96, 10, 3), (25000, 128, 10, 4)])
+@pytest.mark.parametrize("N,C,ne,seed", [(1, 32, 1, 0), (21, 64, 4, 1), (700, 128, 10, 2), (5000, 96, 10, 3), (25000, 128, 10, 4), (22_000, 32, 3, 5), (40_000, 32, 3, 6), (11_000, 64, 5, 7), (20_000, 64, 5, 8), (20_000, 96, 5, 9)])
 def test_node_glue_chains(cabi, N, C, ne, seed):
     """The three [N, C] linears between the layers as one launch per direction: against the fp64 definition, and bit for
     bit against the three separate launches of the linear kernel they stand for (rows without an element included)."""
@@ -629,7 +629,7 @@ def test_linear_pieces_of_the_tile_list_with_row_scale(cabi, N, C, sizes):
 PIECE_CASES = [(21, 64, 16), (2050, 32, 16), (2048, 64, 16), (700, 96, 16), (2049, 96, 16), (700, 128, 16), (2050, 128, 16), (1500, 160, 16),
                (700, 192, 16), (2048, 192, 16), (1000, 224, 16), (500, 256, 16),
                (8300, 64, 16), (8301, 96, 16), (8303, 128, 16), (9001, 160, 16), (9001, 192, 16), (9003, 224, 16), (9007, 256, 16),
-               (300, 64, 1), (9001, 32, 1), (9001, 64, 1), (9002, 96, 1), (9003, 128, 1), (9001, 160, 1), (9007, 192, 1), (9001, 224, 1), (9005, 256, 1),
+               (300, 64, 1), (9001, 32, 1), (12_000, 64, 1), (20_600, 32, 1), (40_001, 64, 1), (3000, 256, 1), (9002, 96, 1), (9003, 128, 1), (9001, 160, 1), (9007, 192, 1), (9001, 224, 1), (9005, 256, 1),
                (33_000, 160, 1), (33_003, 192, 1), (33_001, 224, 1), (33_007, 256, 1)]
 
 
@@ -702,7 +702,7 @@ def test_linear_keeps_infinities_in_their_row_or_column(cabi, N, C, ncomp):
         assert torch.equal(out, want)
 
 
-@pytest.mark.parametrize("N,C", [(2048, 64), (2049, 96), (2050, 128), (2063, 160), (2048, 192), (2049, 224), (2081, 256),
+@pytest.mark.parametrize("N,C", [(2048, 64), (700, 96), (2049, 96), (2050, 128), (1100, 160), (2063, 160), (2048, 192), (2049, 224), (2081, 256),
                                  (8300, 64), (8301, 96), (8303, 128), (9001, 160), (9001, 192), (9003, 224), (9007, 256)])
 def test_linear_scales_of_rows_and_columns(cabi, N, C):
     """Rows of X and columns of W multiplied by powers of two give the same bits, multiplied alike (as long as nothing leaves the normal
@@ -726,7 +726,7 @@ def test_linear_scales_of_rows_and_columns(cabi, N, C):
         assert torch.equal(out, base * d(factor))
 
 
-@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 192), (9007, 224), (12345, 256)])
+@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 192), (9007, 224), (12345, 256), (33_001, 160), (17_003, 192), (17_001, 224), (8200, 256)])
 def test_scalar_linear_many_rows_wide(cabi, N, C):
     """One component per node at 160 to 256 columns and 8 192 nodes and more: plain, with row_scale, with a residual that is a
     tensor of its own, twice for the same bits."""
@@ -743,7 +743,7 @@ def test_scalar_linear_many_rows_wide(cabi, N, C):
     assert torch.equal(cabi.linear(d(X), WT, scale=1.0), out)
 
 
-@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 160), (8195, 192), (9007, 224), (12345, 256), (100007, 192)])
+@pytest.mark.parametrize("N,C", [(8192, 160), (8193, 160), (8195, 192), (9007, 224), (12345, 256), (100007, 192), (33_003, 160), (17_005, 224)])
 def test_scalar_linear_many_rows_wide_in_place(cabi, N, C):
     """The residual is the output itself, at node counts that leave the last tile of 16 rows short: the places behind its
     rows stand in for its first row, which must receive its residual once."""
@@ -956,10 +956,54 @@ def test_linear_row_scale(cabi):
     close(got, ref, 1e-5, 2e-6)
 
 
+# K, Nout, nodes: weights that are not square.  The tiled kernels: few tiles, cut to 32 columns each (K of one to four chunks, and more);
+# a tile of all columns, with K walked through a ring of chunks in LDS or chunk by chunk.
+TILED_CASES = [(32, 256, 333), (64, 256, 333), (96, 256, 333), (128, 256, 300), (128, 160, 333), (160, 256, 333), (256, 224, 300),
+               (64, 32, 3000), (128, 32, 9000), (32, 64, 1500), (128, 64, 2500), (32, 96, 1500), (64, 96, 1501), (32, 128, 1500), (96, 128, 1503), (256, 128, 1100),
+               (128, 160, 1300), (96, 192, 1201), (32, 224, 1200), (192, 224, 1207), (128, 256, 1250), (224, 256, 1100), (32, 256, 1200)]
+
+
+@pytest.mark.parametrize("K,Nout,N", TILED_CASES)
+@pytest.mark.parametrize("ncomp", [16, 1])
+def test_linear_of_weights_that_are_not_square(cabi, K, Nout, N, ncomp):
+    """Every width of the tiled kernels, with 16 components and with one (sixteen times the nodes): shared weights and weights per group
+    with rows of no group and a group of one node, with row_scale and without, with a residual that is the output itself (which adds to the
+    bits without it); the last tile of each group is short."""
+    _say("linear_not_square", K, Nout, N, ncomp)
+    N = N if ncomp == 16 else 16 * N + 5
+    g = torch.Generator(device=DEV).manual_seed(K + Nout + N)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    X, S, R = rand(N, ncomp, K), rand(N, K), rand(N, ncomp, Nout)
+    W = rand(3, 4 if ncomp == 16 else 1, Nout, K)
+    elem = torch.randint(0, 4, (N,), generator=g, device=DEV)  # value 3: no group
+    elem[elem == 1] = 0
+    elem[N // 3] = 1
+    perm, off = cabi.stable_key_sort(elem.int(), 4)
+    rows = torch.randperm(N, generator=g, device=DEV)[:400]
+    rows[:3] = torch.tensor([0, N // 3, N - 1], device=DEV)
+    for scale in (None, S):
+        x = (X if scale is None else X * scale[:, None])[rows].double()
+        for groups in (False, True):
+            ref = torch.zeros(rows.numel(), ncomp, Nout, dtype=torch.float64, device=DEV)
+            for e in range(3 if groups else 1):
+                mine = elem[rows] == e if groups else torch.ones_like(rows, dtype=torch.bool)
+                for m in range(ncomp):
+                    ref[mine, m] = x[mine, m] @ W[e, math.isqrt(m) if ncomp == 16 else 0].double().T.contiguous()
+
+            def call(residual, out):
+                cabi._check(cabi.lib.cm_linear(X.data_ptr(), W.data_ptr(), perm.data_ptr() if groups else None, off.data_ptr() if groups else None, N,
+                                               4 if groups else 1, 1 if groups else 0, ncomp, K, Nout, 0.5, scale.data_ptr() if scale is not None else None,
+                                               residual.data_ptr() if residual is not None else None, out.data_ptr(), cabi._stream()))
+                return out
+            out = call(None, torch.empty(N, ncomp, Nout, device=DEV))
+            close(out[rows], 0.5 * ref.cpu(), 1e-5, 2e-6)
+            inout = R.clone()
+            assert torch.equal(call(inout, inout), out + R)
+
+
 @pytest.mark.parametrize("K,Nout", [(128, 128), (64, 160), (32, 96)])
 def test_linear_residual(cabi, K, Nout):
-    """residual is added to the written rows, for 16-component and scalar features (both kernel variants: 128 and 96
-    columns run on the LDS-ring kernel when K has more than one chunk, 160 columns and K = 32 on the plain one)."""
+    """residual is added to the written rows, for 16-component and scalar features, square and not, at some hundred nodes."""
     g = torch.Generator().manual_seed(5)
     N = 333
     X = torch.randn(N, 16, K, generator=g, dtype=torch.float64).float().double()
