@@ -59,9 +59,11 @@ __device__ __forceinline__ void product(const Rows<KQ> &x, const Rows<KQ> (&wt)[
 // the traffic between L2 and the compute units grows with the blocks where a tile of 128 rows shares it, and one block
 // after the other waits for the fp32 matrix rate.  Measured (us, the tiled kernels -> this one):
 //   [N, C]      216 x 64 5.0 -> 2.7, 216 x 128 6.7 -> 3.6, 2 000 x 128 6.9 -> 3.7, 2 000 x 256 10.8 -> 7.7, 10 000 x 64 5.5 -> 4.7;
-//               even at 5 000 x 128 and 192 (2 500 and 3 750 blocks).  At 96 and 128 columns the products between the layers
-//               run as chains on shared tiles (node_glue.hip), which are the faster ones from 1 536 blocks on; at 224 and 256 the
-//               kernel with a workgroup per 128 rows is from 2 048 on (2 500 x 256 12.4 -> 9.2)
+//               even at 5 000 x 128 and 192 (2 500 and 3 750 blocks).  At 96 and 128 columns the line is one tile of 16 rows
+//               per compute unit (1 536 and 2 048 blocks), where the chains of these products (node_glue.hip) change with it: steps of
+//               3 500 x 128 421 -> 412 us, 4 000 454 -> 444, 4 500 513 -> 523 (chains forward / backward 17.1 / 17.1 -> 16.9 / 12.6, 17.6 / 17.0 -> 23.6 /
+//               23.2 at 5 000).  At 256 columns the kernel with a workgroup per 128 rows is faster from 2 048 on (2 500 x 256 13.6 -> 8.3, 2 500 x
+//               224 equal)
 //   [N, 16, C]  216 x 64 5.3 -> 2.9, 216 x 128 7.2 -> 5.0, 500 x 96 6.9 -> 5.5, 216 x 192 9.9 -> 8.6 (2 688 blocks); even at 500 x 128
 //               and 1 000 x 64 (4 000 blocks), slower beyond
 // From 1 024 blocks (a wave on every SIMD) a wave takes two neighbouring blocks of columns and reads its rows once for
@@ -69,7 +71,7 @@ __device__ __forceinline__ void product(const Rows<KQ> &x, const Rows<KQ> (&wt)[
 inline int64_t blocks(int64_t nnodes, int ncomp, int columns) { return ceil_div(nnodes, kRows) * ncomp * (columns / kRows); }
 constexpr int64_t kOneColumnBlock = 1024;
 inline bool applies(int64_t nnodes, int ncomp, int columns) {
-  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 || columns == 128 ? 1536 : (columns >= 256 ? 2048 : 2560));
+  const int64_t limit = ncomp > 1 ? 3072 : (columns == 96 ? 1536 : (columns == 128 || columns == 256 ? 2048 : 2560));
   return blocks(nnodes, ncomp, columns) <= limit;
 }
 

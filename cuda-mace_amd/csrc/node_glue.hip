@@ -375,8 +375,8 @@ __global__ __launch_bounds__(4 * kWave) void node_glue_gh1_kernel(const float *_
 // bound by nothing but the fp64 matrix rate and the chain of a tile, 0.9 us each way at 128 x 128 on four matrix pipes.
 // Measured inside the step, three launches -> one (us): 21 x 64 9.0 -> 5.2, 216 x 128 14.8 -> 12.4, 2 000 x 128 15.4 -> 12.5 (tiles
 // of 16 nodes), 5 000 x 96 24.0 -> 15.6, 10 752 x 64 23.9 -> 13.5, 25 000 x 128 66.6 -> 40 (its 112 MB, half of them the fp64 feature
-// rows, take 21); with the rows of 16 nodes in a wave's registers, as in the chains above, 5 000 x 96 16.1 -> 14.6, 10 752 x 64 14.3 -> 11.2,
-// 25 000 x 128 41.6 -> 36.6.
+// rows, take 21); with the rows of 16 nodes in a wave's registers, as in the chains above, 5 000 x 96 16.1 -> 15.4, 10 752 x 64 14.3 -> 11.5,
+// 25 000 x 128 41.7 -> 39.4, and 5 000 x 128 16.8 -> 21.5, whose weight blocks take turns in LDS.
 // Without d_h2 (energies alone) the kernel ends with the energies.  Bits of the separate launches, as above.
 // A wave has all classes of pieces of its 16 nodes (in the separate kernel four waves share them); the weights of the readouts
 // wait in LDS.

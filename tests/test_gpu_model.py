@@ -568,7 +568,7 @@ def test_step_with_chained_node_kernels_equals_the_separate_launches(cabi, natom
     torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
-@pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32),
+@pytest.mark.parametrize("natoms,channels", [(17, 32), (65, 128), (3105, 128), (4110, 128), (4150, 96), (10260, 64), (16290, 96), (16290, 128), (20500, 32),
                                              (60, 192), (400, 160), (300, 224), (1536, 256), (1537, 256)])
 def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, channels, monkeypatch):
     """The product linear before the readouts, the readouts, and the product of their derivative as one launch, on tiles of 16, 64

@@ -451,7 +451,7 @@ def test_node_glue_chains(cabi, N, C, ne, seed):
 
 
 @pytest.mark.parametrize("N,C,ncomp,ne", [(15, 32, 1, 1), (17, 160, 16, 3), (256, 64, 16, 2), (257, 64, 16, 2), (768, 64, 16, 1), (769, 64, 16, 1),
-                                          (2048, 128, 1, 3), (2049, 128, 1, 3), (3073, 128, 1, 2), (2560, 256, 1, 1), (2561, 256, 1, 70), (193, 96, 16, 1)])
+                                          (2048, 128, 1, 3), (2049, 128, 1, 3), (3073, 128, 1, 2), (4096, 128, 1, 2), (4097, 128, 1, 2), (2560, 256, 1, 1), (2561, 256, 1, 70), (193, 96, 16, 1)])
 def test_linear_few_rows(cabi, N, C, ncomp, ne):
     """Both sides of the lines between one and two column blocks per wave and between this kernel and the tiled ones, with
     per-element weights, a group without weights, row_scale and (one component) a residual; twice for the same bits."""
