@@ -1415,7 +1415,7 @@ bool resident_weights(int64_t nnodes, int ncomp, int K, int ngroups, bool groupe
 //    10.8 / 12.5 / 14.8 / 16.7.  (One component, 224 columns, up to 4 096 nodes: the tiled kernel cuts its tiles to 32 columns there, 10.9 -> 12.5.)
 //  - beyond it against resident weights at 64 and 96 columns, two workgroups per compute unit: up to four (8 192 nodes; 5 000 x 64 12.2 / 17.2 / 13.3 / 17.6 ->
 //    11.0 / 12.3 / 12.5 / 13.4, 8 000 x 96 27.8 / 31.7 / 29.0 / 31.5 -> 22.8 / 24.8 / 25.1 / 27.0).  It stays ahead on its own beyond that, but not in a step, where X and the
-//    result share the last-level cache with everything else (10 752 x 64 in 512 graphs 285 -> 293): the other kernel has the loads
+//    result share the last-level cache with everything else (12 000 x 96 881 -> 900, 10 752 x 64 in 512 graphs 318 -> 320): the other kernel has the loads
 //    of a tile under way while it works on the one before.  At 128 columns one workgroup fits a compute unit, and a second round pays
 //    where at least half of it is filled: 2 500 16.7 / 20.1 / 18.0 / 22.5 -> 17.9 / 19.7 / 19.3 / 21.4, 3 500 23.3 / 26.1 / 22.1 / 27.3 -> 20.2 / 23.8 / 21.8 / 25.8,
 //    5 000 27.1 / 31.5 / 27.7 / 34.2 -> 27.5 / 30.7 / 29.5 / 33.1.  Beyond 128 columns it does not: 2 500 x 160 21.2 / 26.6 / 22.7 / 29.8 -> 25.4 / 27.3 / 27.1 / 29.5, 2 500 x
