@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -403,7 +404,8 @@ __device__ __forceinline__ bool key_less(int ja, const int32_t *Sa, int jb, cons
 // Two times 64 candidates per trip, their look-ups and loads side by side: a trip is a chain of seven LDS reads and a load.  With that and
 // the rank from one 64-bit key per neighbour (the compare of index and image took 25 of 41 us at 123 neighbours, many of them images of one
 // atom) us, count / graph: 2 000 atoms with 52 neighbours 9.2 / 14.4 -> 7.7 / 10.8, 216 with 123 13.8 / 41 -> 12.9 / 16.7, 12 000
-// with 42 17.8 / 36.4 -> 18.3 / 32.6.
+// with 42 17.8 / 36.4 -> 18.3 / 32.6.  64 bins where no more are in reach (large cells, whose bins are halved to fit the workspace) and 64 candidates where no
+// more are left: 40 000 with 10, 45 bins and 58 candidates, 29.8 / 49.2 -> 35.8 / 58.7 with 128 of each always, 28.7 / 52.2 with this.
 enum class Scan { kCount, kScratch, kGraph };
 constexpr int kScanWaves = 4;
 template <Scan MODE>
@@ -445,12 +447,14 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
     b -= B * nb;
     return B;
   };
-  for (int first_bin = 0; first_bin < nscan; first_bin += kBins) {
-    // 128 bins side by side: where their atoms begin, how many there are, which image of the cell they belong to
-    int first[2] = {0, 0}, cnt[2] = {0, 0}, image[2] = {0, 0};
+  const auto look_at = [&](int first_bin, auto per_lane) {
+    // 64 or 128 bins side by side: where their atoms begin, how many there are, which image of the cell they belong to
+    constexpr int U = decltype(per_lane)::value;
+    int first[U], cnt[U], image[U];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int q = first_bin + 2 * lane + u;
+    for (int u = 0; u < U; ++u) {
+      first[u] = cnt[u] = image[u] = 0;
+      const int q = first_bin + U * lane + u;
       if (q < nscan) {
         const int q0 = quotient(q, per_plane), in_plane = q - q0 * (m1 * m2), q1 = quotient(in_plane, per_row);
         int b0 = bi0 + q0 - r0, b1 = bi1 + q1 - r1, b2 = bi2 + (in_plane - q1 * m2) - r2;
@@ -466,7 +470,7 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
         }
       }
     }
-    int upto = cnt[0] + cnt[1];
+    int upto = cnt[0] + (U == 2 ? cnt[U - 1] : 0);
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       const int v = __shfl_up(upto, d);
@@ -475,14 +479,14 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
     const int total = __shfl(upto, kWave - 1);
     wave_lds_fence();  // the previous bins' tables have been read
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      s_before[wave][2 * lane + u] = upto - cnt[1] - (u == 0 ? cnt[0] : 0);
-      s_first[wave][2 * lane + u] = first[u];
-      s_image[wave][2 * lane + u] = image[u];
+    for (int u = 0; u < U; ++u) {
+      s_before[wave][U * lane + u] = upto - cnt[U - 1] - (u == U - 2 ? cnt[0] : 0);
+      s_first[wave][U * lane + u] = first[u];
+      s_image[wave][U * lane + u] = image[u];
     }
     wave_lds_fence();
-    constexpr int kSets = 2;
-    for (int base = 0; base < total; base += kSets * kWave) {
+    const auto trip = [&](int base, auto sets) {
+      constexpr int kSets = decltype(sets)::value;
       int b[kSets], cand[kSets], image_of[kSets], S[kSets][3];
       int64_t k_of[kSets];
       int4 meta[kSets];
@@ -491,7 +495,7 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
       for (int u = 0; u < kSets; ++u) b[u] = 0, cand[u] = min(base + u * kWave + lane, total - 1);
       // the last bin whose atoms begin at or before cand: it is not empty, since cand < total
 #pragma unroll
-      for (int step = kBins / 2; step > 0; step >>= 1) {
+      for (int step = U * kWave / 2; step > 0; step >>= 1) {
         int before[kSets];
 #pragma unroll
         for (int u = 0; u < kSets; ++u) before[u] = s_before[wave][b[u] + step];
@@ -533,8 +537,17 @@ __global__ __launch_bounds__(kScanWaves * kWave) void nl_scan_kernel(Workspace w
         }
         count += __popcll(mask);
       }
+    };
+    // the last 64 or fewer by themselves: with few candidates in all of the bins the second set would be all of the work again
+    for (int base = 0; base < total; base += 2 * kWave) {
+      if (total - base > kWave) trip(base, std::integral_constant<int, 2>{});
+      else trip(base, std::integral_constant<int, 1>{});
     }
-  }
+  };
+  // a reach of one or two bins (large cells, whose bins are halved to fit the workspace): 64 at a time
+  if (nscan <= kWave) look_at(0, std::integral_constant<int, 1>{});
+  else
+    for (int first_bin = 0; first_bin < nscan; first_bin += kBins) look_at(first_bin, std::integral_constant<int, 2>{});
   if constexpr (MODE == Scan::kCount) {
     if (lane == 0) w.degree[i] = count;
   }

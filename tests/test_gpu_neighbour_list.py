@@ -105,6 +105,8 @@ GRAPH_CASES = {
     "several_launches": (4097, 34.5, (1, 1, 0), 4.0),
     "many_32768": (32768, 69.0, (1, 1, 1), 4.0),
     "many_32769": (32769, 69.0, (1, 1, 0), 4.0),
+    "bins_halved": (40000, 126.0, (1, 1, 1), 5.0),  # 45 bins in reach, about 58 candidates: one set of 64 of each
+    "bins_halved_dense": (3000, 60.0, (1, 1, 1), 10.0),
 }
 
 
