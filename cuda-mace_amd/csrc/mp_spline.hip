@@ -855,11 +855,14 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
 // 10.6 [10.6] 11.7, 400 x 52 19.4 14.5 13.9 [14.2] 18.4 19.0 20.1, 60 x 30 11.0 8.3 [8.2] 8.4 8.3 8.7 9.8; 64 216 x 52 11.8 8.8 [8.5] 9.0 9.2 9.7
 // 10.7, 1 000 x 30 [10.2] 11.6 15.7 17.5 28 30 34; 256 21 x 12 14.0 8.2 [7.5] 7.7 7.6 7.8 8.0, 300 x 9 12.8 [8.6] 8.6 8.9 11.9 12.1 12.9, 216 x 52
 // 43.5 20.5 17.2 16.1 15.1 [15.1] 15.7; 192 672 x 9 14.7 [10.7] 11.6 12.2 15.7 15.9 17.4.
-template <int C>
+// With lengths and harmonics given a wave has less to wait for, and beyond two nodes per unit a part takes twelve edges (128 channels 1 000 x 20
+// 13.3 in one, 14.5 in two).
+template <int C, bool FROM_VEC>
 int forward_parts(int64_t nnodes, int64_t nedges) {
   constexpr int kSlots = Cfg<C, true>::EPW, kLeast = kSlots >= 8 ? 24 : 4 * kSlots;
   if (nnodes <= 0) return 1;
-  int parts = static_cast<int>(std::min<int64_t>(6, std::max<int64_t>(1, nedges / (kLeast * nnodes))));
+  const int64_t least = !FROM_VEC && nnodes > 2 * device_compute_units() ? std::max(12, kLeast) : kLeast;
+  int parts = static_cast<int>(std::min<int64_t>(6, std::max<int64_t>(1, nedges / (least * nnodes))));
   while (parts > 1 && nnodes > static_cast<int64_t>(device_compute_units()) * (8 / parts)) --parts;
   return parts;
 }
@@ -873,18 +876,19 @@ int forward_parts(int64_t nnodes, int64_t nedges) {
 // [55 / 78]; 160 2 200 x 52 76 / 109 [67 / 98] 68 / 101.
 // Up to 64 channels a wave's loads are a quarter or half of that, its start-up is not, and more than a round of waves never pays: eight
 // waves per compute unit, five parts at most (400 x 52 x 64 five 8.1, eight 10.9), of two edges each, beyond two nodes per unit of 256 / C;
-// two parts of 16 edges while they fit twelve waves.  us without gX at p = 1 2 3 4 5: 64 channels 21 x 9 6.2 5.3 4.8 4.6 [4.3], 120 x 52
+// two parts of 16 edges while they fit twelve waves.  (From lengths, two sets of operands and eight waves: no such two parts, 1 500 x 52 x 32 23.5
+// in one, 26.0 in two, and twelve edges per part beyond two nodes per unit.)  us without gX at p = 1 2 3 4 5: 64 channels 21 x 9 6.2 5.3 4.8 4.6 [4.3], 120 x 52
 // 17.1 10.1 8.4 7.4 [7.0], 500 x 52 17.3 10.7 9.8 [9.4] 10.4, 1 000 x 52 17.9 [13.4] 14.3 16.6 17.2, 1 500 x 52 21.9 [18.9] 20.9, 1 800 x 52 [23.3] 23.9
 // 24.7, 2 000 x 52 [25.3] 26.6 26.4, 800 x 20 10.5 [8.6] 9.1, 1 200 x 20 [10.6] 10.5, 300 x 9 6.9 6.2 6.0 5.6 [5.8], 500 x 9 7.0 6.5 6.2 [6.4], 1 000 x
 // 9 7.5 [7.4]; 32 channels 500 x 52 11.5 7.8 7.5 [7.4], 1 500 x 52 14.1 [12.2] 14.1, 2 000 x 52 [15.4] 16.8 17.6, 800 x 20 7.2 [6.8], 1 500 x 20 [8.2] 9.0,
 // 1 000 x 9 [6.0] 6.6 7.6.
-template <int C>
+template <int C, bool FROM_VEC>
 int backward_parts(int64_t nnodes, int64_t nedges) {
   if (nnodes <= 0) return 1;
   if constexpr (C <= 64) {
-    const int64_t units = device_compute_units(), each = nedges / nnodes, least = nnodes > 2 * units ? 256 / C : 2;
+    const int64_t units = device_compute_units(), each = nedges / nnodes, least = nnodes <= 2 * units ? 2 : (FROM_VEC ? 256 / C : 12);
     const int64_t parts = std::min<int64_t>(5, std::min(8 * units / nnodes, (each + 1) / least));
-    return static_cast<int>(parts < 2 && nnodes <= 6 * units && each >= 32 ? 2 : std::max<int64_t>(1, parts));
+    return static_cast<int>(FROM_VEC && parts < 2 && nnodes <= 6 * units && each >= 32 ? 2 : std::max<int64_t>(1, parts));
   }
   constexpr int kMost = 8;
   const double slots = device_compute_units() * 8.0;
@@ -902,7 +906,7 @@ int backward_parts(int64_t nnodes, int64_t nedges) {
 template <int C, bool FROM_VEC>
 int launch_forward(const float *X, const float *Y, const Spline &sp, const int32_t *sender, const int32_t *first_occ,
                    int64_t nnodes, int64_t nedges, float *out, hipStream_t st) {
-  const int parts = forward_parts<C>(nnodes, nedges);
+  const int parts = forward_parts<C, FROM_VEC>(nnodes, nedges);
   const size_t lds = static_cast<size_t>(parts) * kStageBytes + static_cast<size_t>(parts - 1) * 16 * C * sizeof(float);
   if (parts > 1)
     hipLaunchKernelGGL((mp_spline_forward_kernel<C, FROM_VEC, true>), dim3(static_cast<unsigned>(nnodes)), dim3(kWave * parts), lds, st,
@@ -940,7 +944,7 @@ template <int C, bool FROM_VEC, bool GY, bool GR, bool GX>
 void launch_edge(const float *X, const float *Y, const Spline &sp, const float *G, const int32_t *sender,
                  const int32_t *first_occ, int64_t nnodes, int64_t nedges, float *gY, float *g_r, float *gXe,
                  hipStream_t st) {
-  const int parts = backward_parts<C>(nnodes, nedges);
+  const int parts = backward_parts<C, FROM_VEC>(nnodes, nedges);
   const dim3 grid(static_cast<unsigned>(nnodes * parts));
   if constexpr (FROM_VEC && (C == 160 || C == 192 || C == 224)) {
     if (steps_of_four_edges<C>(nnodes, nedges, parts)) {
@@ -1046,7 +1050,7 @@ extern "C" int cm_mp_edge_forward_kernel(int64_t nnodes, int64_t nedges, int cha
 extern "C" int cm_mp_edge_backward_kernel(int64_t nnodes, int64_t nedges, int channels) {
   if (nnodes <= 0) return 0;
   bool steps = false;
-  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, cm::backward_parts<C_>(nnodes, nedges)));
+  CM_DISPATCH_C(channels, steps = cm::steps_of_four_edges<C_>(nnodes, nedges, (cm::backward_parts<C_, true>(nnodes, nedges))));
   return steps ? 1 : 0;
 }
 
