@@ -1,0 +1,746 @@
+// The step of few nodes: a workgroup takes one node through everything between two exchanges with its neighbours, so that a step is
+// three launches and the forces instead of fifteen.
+//
+// A step of some ten to some hundred atoms spends its time on the chain of its launches: each is over in 3 to 6 us, next to nothing of
+// which is arithmetic or traffic, and waits for what the one before has written (21 atoms x 64 channels: 16 launches, 71 us).  All that
+// crosses from one node to another is the gather of the sender rows in the two message passes and of the per-edge gradients on the way
+// back; between those a node's rows [16, C] fit a workgroup's LDS, the weights (4 C^2 per mixing, C^2 per product) come from L2 in as many
+// bytes as the node's table rows do, and every product of one row is K multiply-adds per column, which the vector ALU does in less time
+// than 16 rows of a matrix instruction, fifteen of them empty, would take.
+//
+//   first_layer    vectors, live edge range, M1, A, B1 and grad1, h1, sc, X2                    (stages of step.hip in its notation)
+//   second_layer   M2, A, B2, h2, the readouts, gB2, gA, gv2 and the per-edge rows of gX2
+//   back_to_edges  gX2 (sender pass), gh1, gB1, gA, gv1; extra workgroups: the graph energies
+//
+// Every sum is formed in the order of the launch it stands for: v_mfma_f32_16x16x4_f32 and v_mfma_f64_16x16x4_f64 add their four products one
+// after the other, fused, k ascending (checked bit for bit against fma chains), so the chains of mfma_f32.hpp and readout_device.hpp are
+// chains of fmaf and fma here, and the step returns the bits of the separate launches.
+#include "common.hpp"
+#include "few_nodes.hpp"
+#include "mfma_f32.hpp"
+#include "mp_spline_device.hpp"
+#include "node_glue.hpp"
+#include "symcon_device.hpp"
+
+namespace cm {
+namespace fewnodes {
+namespace {
+
+using namespace mp;
+
+constexpr int kThreads = 512;
+constexpr int kWaves = kThreads / kWave;
+constexpr int kMostParts = 6;  // of the forward (forward_parts)
+
+// Workgroup barrier that orders LDS alone: loads of weights that a thread has requested stay in flight across it.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// ---- products of one row ------------------------------------------------------------------------------------------------
+// The chain of channel k in mfma_f32.hpp's product is (k / 16 + k % 4) % 4, its place there 4 (k / 16) + k % 16 / 4.  A row that is about to be
+// multiplied lies in LDS chain by chain, so that a thread reads its chain's values 16 bytes at a time.
+template <int C>
+__device__ __forceinline__ int place(int k) {
+  return ((k / 16 + k % 4) & 3) * (C / 4) + 4 * (k / 16) + k % 16 / 4;
+}
+// channel at place j of chain ch
+__device__ __forceinline__ int channel_at(int ch, int j) { return 16 * (j / 4) + 4 * (j % 4) + ((ch - j / 4) & 3); }
+
+// A thread's share of NMAT products of a row and a [C, C] matrix W[k][column]: one chain of one column, C / 4 multiply-adds.
+template <int C, int NMAT>
+struct Products {
+  static constexpr int kUnits = 4 * C * NMAT, kPer = (kUnits + kThreads - 1) / kThreads;
+  float w[kPer][C / 4];
+  __device__ __forceinline__ void request(const float *W0, const float *W1 = nullptr) {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int u = threadIdx.x + p * kThreads;
+      if (kUnits % kThreads != 0 && u >= kUnits) break;
+      const int unit = NMAT == 1 ? u : u % (4 * C), ch = unit / C;
+      const float *W = (NMAT == 1 || u < 4 * C ? W0 : W1) + unit % C;
+#pragma unroll
+      for (int j = 0; j < C / 4; ++j) w[p][j] = W[channel_at(ch, j) * C];
+    }
+  }
+  // x0, x1: the rows, by place; partial sums to part[matrix][chain][column]
+  __device__ __forceinline__ void run(const float *x0, const float *x1, float *part) const {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int u = threadIdx.x + p * kThreads;
+      if (kUnits % kThreads != 0 && u >= kUnits) break;
+      const int unit = NMAT == 1 ? u : u % (4 * C), ch = unit / C;
+      const float *x = (NMAT == 1 || u < 4 * C ? x0 : x1) + ch * (C / 4);
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < C / 4; j += 4) {
+        const f4 v = ld4(x + j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum = fmaf(w[p][j + i], v[i], sum);
+      }
+      part[u] = sum;
+    }
+  }
+};
+// the four chains of a column
+template <int C>
+__device__ __forceinline__ float column(const float *part, int c) {
+  return (part[c] + part[C + c]) + (part[2 * C + c] + part[3 * C + c]);
+}
+
+// The channel mixing of a node's 16 rows, a [C, C] block per degree: a thread has one chain of one column for the degrees of its set.
+template <int C>
+struct Mixing {
+  static constexpr int kSets = kThreads / (4 * C) >= 4 ? 4 : (kThreads / (4 * C) >= 2 ? 2 : 1);
+  float w[4][C / 4];
+  __device__ __forceinline__ static bool mine(int l) {  // equal work: 7 + 1 and 5 + 3 rows
+    const int set = threadIdx.x / (4 * C);
+    return set < kSets && (kSets == 1 || (kSets == 2 ? (l == 0 || l == 3) == (set == 0) : l == set));
+  }
+  __device__ __forceinline__ void request(const float *W) {
+    const int unit = threadIdx.x % (4 * C), ch = unit / C;
+#pragma unroll
+    for (int l = 3; l >= 0; --l) {
+      if (!mine(l)) continue;
+#pragma unroll
+      for (int j = 0; j < C / 4; ++j) w[l][j] = W[(l * C + channel_at(ch, j)) * C + unit % C];
+    }
+  }
+  // x: [16][C] by place; partial sums to part[chain][16][C]
+  __device__ __forceinline__ void run(const float *x, float *part) const {
+    const int unit = threadIdx.x % (4 * C), ch = unit / C, col = unit % C;
+    const float *xc = x + ch * (C / 4);
+    float *to = part + ch * (16 * C) + col;
+    auto degree = [&](auto lc) {
+      constexpr int L = decltype(lc)::value;
+      if (!mine(L)) return;
+      float sum[2 * L + 1];
+#pragma unroll
+      for (int m = 0; m < 2 * L + 1; ++m) sum[m] = 0.f;
+#pragma unroll
+      for (int j = 0; j < C / 4; j += 4)
+#pragma unroll
+        for (int m = 0; m < 2 * L + 1; ++m) {
+          const f4 v = ld4(xc + (L * L + m) * C + j);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum[m] = fmaf(w[L][j + i], v[i], sum[m]);
+        }
+#pragma unroll
+      for (int m = 0; m < 2 * L + 1; ++m) to[(L * L + m) * C] = sum[m];
+    };
+    degree(std::integral_constant<int, 3>{});
+    degree(std::integral_constant<int, 2>{});
+    degree(std::integral_constant<int, 1>{});
+    degree(std::integral_constant<int, 0>{});
+  }
+};
+template <int C>
+__device__ __forceinline__ float mixed(const float *part, int at, float scale) {  // at: m C + column
+#pragma clang fp contract(off)
+  const float v = (part[at] + part[16 * C + at]) + (part[32 * C + at] + part[48 * C + at]);
+  return v * scale;
+}
+
+// ---- LDS of a workgroup -----------------------------------------------------------------------------------------------
+template <int C, bool FORWARD, bool BACKWARD>
+struct Shared {
+  static constexpr int kForward = FORWARD ? kMostParts * kStageBytes + kMostParts * 16 * C * 4 : 0;
+  static constexpr int kBackward = BACKWARD ? kWaves * (kStageBytes + 16 * kChunk * 4) : 0;
+  static constexpr int kMixing = 64 * C * 4;
+  static constexpr int kMost = kForward > kBackward ? kForward : kBackward;
+  // staged edges and the parts' sums; partial sums of products; staged edges and the edges' sums, one after the other
+  __attribute__((aligned(16))) unsigned char work[kMost > kMixing ? kMost : kMixing];
+  __attribute__((aligned(16))) float rows[16 * C];  // operand rows, by place
+  __attribute__((aligned(16))) float grad[16 * C];  // gradient rows, by channel
+  __attribute__((aligned(16))) float row[3][C];     // operand rows of the products, by place
+  float h2[C];
+  double z[4][16], e1[4][4], e2[16], d[16];
+  float knots[kKnotsInLds];
+  int mark;
+  __device__ float *part() { return reinterpret_cast<float *>(work); }
+  __device__ float *sums(int p) { return reinterpret_cast<float *>(work + kMostParts * kStageBytes) + p * (16 * C); }
+};
+
+// the waves that contract: the last ones, which have no part of the forward
+template <int C>
+struct Contraction {
+  static constexpr int kFirst = kWaves - (C + kWave - 1) / kWave;
+  static_assert(kFirst >= kMostParts, "no part of the forward falls to a wave that contracts");
+  float t3[CM_SYMCON_N3], t2[CM_SYMCON_N2], t1;
+  __device__ __forceinline__ static int channel() { return static_cast<int>(threadIdx.x) - kFirst * kWave; }
+  __device__ __forceinline__ static bool here() { return channel() >= 0 && channel() < C; }
+  // by whole waves (a lane beyond the last channel reads the last one's)
+  __device__ __forceinline__ void request(const float *T3, const float *T2, const float *T1, int element) {
+    const int c = min(channel(), C - 1);
+#pragma unroll
+    for (int t = 0; t < CM_SYMCON_N3; ++t) t3[t] = T3[(static_cast<int64_t>(element) * CM_SYMCON_N3 + t) * C + c];
+#pragma unroll
+    for (int t = 0; t < CM_SYMCON_N2; ++t) t2[t] = T2[(static_cast<int64_t>(element) * CM_SYMCON_N2 + t) * C + c];
+    t1 = T1[static_cast<int64_t>(element) * C + c];
+  }
+  template <bool GRAD>
+  __device__ __forceinline__ float run(const float *part, float scale, float (&g)[16]) const {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = mixed<C>(part, i * C + channel(), scale);
+    return symcon::contract<float, GRAD>(x, t3, t2, t1, g);
+  }
+};
+
+// the wave's number in a scalar register: a branch on it is the wave's, and what one side holds takes no registers of the other
+__device__ __forceinline__ int wave_number() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
+
+// Message of the node over its edges e0 .. e1 - 1 into s.rows, the parts by waves as in mp_spline_forward_kernel.  `others` is called by the
+// waves that have no part and contract later, `meanwhile` by every thread between its part and the barrier behind which the parts are added.
+template <int C, class S, class Fn0, class Fn>
+__device__ __forceinline__ void message(S &s, const float *__restrict__ X, const Spline &sp, const int32_t *__restrict__ sender, int nnodes, int64_t nedges,
+                                        int e0, int e1, int parts, Fn0 others, Fn meanwhile) {
+  using K = Cfg<C, true>;
+  const int wave = wave_number(), lane = threadIdx.x % kWave;
+  if (wave < parts) {
+    const int64_t len = e1 - e0;
+    const int lo = e0 + static_cast<int>(len * wave / parts), hi = e0 + static_cast<int>(len * (wave + 1) / parts);
+    typename K::vec acc[16];
+    forward_wave<C, true, K::V <= 4>(X, nullptr, sp, sender, nnodes, nedges, lo, hi, Staged(s.work + wave * kStageBytes), acc);
+    if (lane < K::LPE) {
+      float *to = s.sums(wave) + K::off(lane);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) K::st(to + m * C, acc[m]);
+    }
+  } else if (wave >= Contraction<C>::kFirst) {
+    others();
+  }
+  meanwhile();
+  lds_barrier();
+  for (int i = threadIdx.x; i < 16 * C; i += kThreads) {
+    float v = s.sums(0)[i];
+    for (int p = 1; p < parts; ++p) v += s.sums(p)[i];
+    s.rows[i / C * C + place<C>(i % C)] = v;
+  }
+  lds_barrier();
+}
+
+// Gradients of the edges e0 .. e1 - 1 of a node from its gradient rows s.grad, as mp_spline_backward_edge_kernel forms them: every edge on its
+// own, so the split over the waves is free; a wave takes as many edges as it has slots before another is given some.
+template <int C, bool WANT_GX, class S>
+__device__ __forceinline__ void edge_gradients(S &s, const float *__restrict__ X, const Spline &sp, const int32_t *__restrict__ sender, int nnodes,
+                                               int64_t nedges, int e0, int e1, float *gvec, const float *addend, float *__restrict__ gXe) {
+  using K = Cfg<C>;
+  using vec = typename K::vec;
+  const int wave = wave_number(), lane = threadIdx.x % kWave;
+  const int slot = lane / K::SW, cl = lane % K::SW;
+  const bool active = cl < K::LPE;
+  const unsigned cla = active ? cl : 0;
+  const int64_t len = e1 - e0;
+  const int parts = static_cast<int>(min(static_cast<int64_t>(kWaves), (len + K::EPW - 1) / K::EPW));
+  if (wave >= parts) return;
+  const int lo = e0 + static_cast<int>(len * wave / parts), hi = e0 + static_cast<int>(len * (wave + 1) / parts);
+  unsigned char *mine = s.work + wave * (kStageBytes + 16 * kChunk * 4);
+  const Staged st(mine);
+  float *sGY = reinterpret_cast<float *>(mine + kStageBytes);
+  vec g[16];
+#pragma unroll
+  for (int m = 0; m < 16; ++m) g[m] = active ? K::ld(s.grad + m * C + K::off(cl)) : zerov<vec>();
+  for (int cursor = lo; cursor < hi;) {
+    const int base = cursor;
+    wave_lds_fence();
+    auto dead = [&](int pass_base, int, unsigned long long, bool lane_is_dead) {
+      if (lane_is_dead) {
+        const int64_t e = pass_base + lane;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gvec[3 * e + k] = addend ? addend[3 * e + k] : 0.f;
+      }
+    };
+    const int nlive = stage_edges<true>(nullptr, sender, sp, nnodes, nedges, cursor, hi, lane, st.sY, st.sS, st.sIdx, st.sXr, st.sOrig, dead,
+                                        RawEdge{-1, 0.f, 0.f, 0.f}, s.knots, KnotCopy<>::applies(sp));
+    wave_lds_fence();
+    Operands<K> o;
+    if (slot < nlive) fetch_operands<C>(o, X, sp.coeffs, st.sS[slot], st.sIdx[slot], st.sXr[slot], cla);
+#pragma unroll 1
+    for (int j = slot; j < nlive; j += K::EPW) {
+      float y[16], p[16];
+      staged_harmonics(st.sY, j, y);
+      vec gxe = zerov<vec>(), grq = zerov<vec>();
+      edge_products<K, true, true, true, WANT_GX>(o, y, g, p, gxe, grq);
+      p[0] = dotv(o.x, grq);
+      if constexpr (WANT_GX) {
+        if (active) K::st(gXe + static_cast<int64_t>(base + st.sOrig[j]) * C + K::off(cl), gxe);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const int next = j + K::EPW < nlive ? j + K::EPW : j;
+      fetch_operands<C>(o, X, sp.coeffs, st.sS[next], st.sIdx[next], st.sXr[next], cla);
+      slot_reduce16<K::SW>(p, cl);
+      store_reduced16<K::SW>(p, cl, j, sGY);
+    }
+    wave_lds_fence();
+    if (lane < nlive) {
+      float sums[16];
+#pragma unroll
+      for (int m = 0; m < 16; ++m) sums[m] = sGY[m * kChunk + lane];
+      finish_vector_gradient(sp.vec, base + st.sOrig[lane], sums, addend, gvec);
+    }
+  }
+}
+
+// copy of the knots for edge_gradients; a barrier follows before they are read
+__device__ __forceinline__ void copy_knots(const Spline &sp, float *to) {
+  if (KnotCopy<>::applies(sp))
+    for (int i = threadIdx.x; i < sp.nknots; i += kThreads) to[i] = sp.knots[i];
+}
+
+// Position of `node` in a permutation of the nodes (-1: not there), by the calling wave, and the group of a position.
+__device__ __forceinline__ int position_of(const int32_t *__restrict__ perm, int nnodes, int node, int guess) {
+  if (perm[guess] == node) return guess;
+  for (int base = 0; base < nnodes; base += kWave) {
+    const int i = base + threadIdx.x % kWave;
+    const unsigned long long found = __ballot(i < nnodes && perm[min(i, nnodes - 1)] == node);
+    if (found != 0) return base + __ffsll(static_cast<long long>(found)) - 1;
+  }
+  return -1;
+}
+__device__ __forceinline__ int group_of(const int32_t *__restrict__ offsets, int ngroups, int pos) {
+  for (int base = 0; base < ngroups; base += kWave) {
+    const int i = base + threadIdx.x % kWave;
+    const bool here = i < ngroups && offsets[min(i, ngroups - 1)] <= pos && pos < offsets[min(i, ngroups - 1) + 1];
+    const unsigned long long found = __ballot(here);
+    if (found != 0) return base + __ffsll(static_cast<long long>(found)) - 1;
+  }
+  return -1;
+}
+
+// A permutation that does not name a node leaves its row of the scratch arrays as it was: what is read from them is clamped.
+struct Graph {
+  int nnodes, ngroups, nelements;
+  int64_t nedges;
+  const int32_t *receiver, *sender, *first_occ, *sender_perm, *sender_offsets, *elem_perm, *elem_offsets, *onehot_perm, *onehot_offsets, *rows;
+};
+
+// ---- first layer ----------------------------------------------------------------------------------------------------------
+struct FirstLayer {
+  const double *positions, *shifts;
+  const float *X1, *mix, *T3, *T2, *T1, *prod, *up, *skip;  // matrices as [k][column]
+  float mix_scale, skip_scale;
+  int parts;
+  float *vec;
+  Scratch s;
+};
+
+template <int C, bool FORCES>
+__global__ __launch_bounds__(kThreads, 2) void first_layer_kernel(Graph q, Spline sp, FirstLayer a) {
+  using S = Shared<C, true, false>;
+  __shared__ S s;
+  const int tid = threadIdx.x;
+  int g, pos, gend;
+  if (!locate_group_tile(q.onehot_offsets, q.ngroups, q.nnodes, blockIdx.x, 1, g, pos, gend)) return;
+  const int node = q.onehot_perm[pos];
+  if (static_cast<unsigned>(node) >= static_cast<unsigned>(q.nnodes)) return;
+  const bool no_element = g == q.ngroups - 1;
+
+  // edge vectors, and the end of the range of edges inside the cutoff
+  int e0 = q.first_occ[node], e1 = q.first_occ[q.nnodes + node];
+  clamp_edge_range(e0, e1, q.nedges);
+  if (tid == 0) s.mark = e0;
+  lds_barrier();
+  for (int e = e0 + tid; e < e1; e += kThreads) {
+    double v[3];
+    edge_vector_f64(a.positions, q.receiver, q.sender, a.shifts, q.rows, e, q.nnodes, v);
+    const float v0 = static_cast<float>(v[0]), v1 = static_cast<float>(v[1]), v2 = static_cast<float>(v[2]);
+    a.vec[3 * static_cast<int64_t>(e) + 0] = v0;
+    a.vec[3 * static_cast<int64_t>(e) + 1] = v1;
+    a.vec[3 * static_cast<int64_t>(e) + 2] = v2;
+    if (edge_length(v0, v1, v2) <= sp.r_max) {
+      atomicMax(&s.mark, e + 1);
+    } else if (FORCES) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) a.s.gv1[3 * static_cast<int64_t>(e) + k] = a.s.gv2[3 * static_cast<int64_t>(e) + k] = 0.f;
+    }
+  }
+  __syncthreads();  // the vectors are in memory
+  e1 = s.mark;
+
+  Contraction<C> contraction;
+  Mixing<C> mixing;
+  message<C>(
+      s, a.X1, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.parts,
+      [&]() {
+        const int in_elements = position_of(q.elem_perm, q.nnodes, node, pos);
+        const int element = in_elements < 0 ? -1 : group_of(q.elem_offsets, q.nelements, in_elements);
+        if (tid == kThreads - 1) {
+          a.s.live[node] = e0;
+          a.s.live[q.nnodes + node] = e1;
+          a.s.groups[node] = g;
+          a.s.groups[q.nnodes + node] = element;
+        }
+        contraction.request(a.T3, a.T2, a.T1, max(element, 0));
+      },
+      [&]() {
+        if (!no_element) mixing.request(a.mix + static_cast<int64_t>(g) * (4 * C * C));
+      });
+  if (no_element) {
+    for (int i = tid; i < 64 * C; i += kThreads) s.part()[i] = 0.f;
+  } else {
+    mixing.run(s.rows, s.part());
+  }
+  Products<C, 1> prod;
+  prod.request(a.prod);
+  lds_barrier();
+  if (Contraction<C>::here()) {
+    const int c = Contraction<C>::channel();
+    float grad[16];
+    float b = contraction.template run<FORCES>(s.part(), a.mix_scale, grad);
+    s.row[0][place<C>(c)] = b;
+    if constexpr (FORCES) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a.s.grad1[(static_cast<int64_t>(node) * 16 + i) * C + c] = grad[i];
+    }
+  }
+  lds_barrier();
+  prod.run(s.row[0], nullptr, s.part());
+  Products<C, 2> both;
+  both.request(a.up, a.skip + static_cast<int64_t>(no_element ? 0 : g) * C * C);
+  lds_barrier();
+  const int64_t at = static_cast<int64_t>(node) * C;
+  if (tid < C) {
+    const float h1 = column<C>(s.part(), tid);
+    a.s.h1[at + tid] = h1;
+    s.row[1][place<C>(tid)] = h1;
+  }
+  lds_barrier();
+  both.run(s.row[1], s.row[1], s.part());
+  lds_barrier();
+  if (tid < C) {
+    a.s.X2[at + tid] = column<C>(s.part(), tid);
+  } else if (tid < 2 * C) {
+#pragma clang fp contract(off)
+    const float v = column<C>(s.part() + 4 * C, tid - C) * a.skip_scale;
+    a.s.sc[at + tid - C] = no_element ? 0.f : v;
+  }
+}
+
+// ---- second layer, forward and back to its edges ----------------------------------------------------------------------------
+struct SecondLayer {
+  const float *mix, *mix_T, *T3, *T2, *T1, *prod, *prod_T;
+  float mix_scale;
+  int parts;
+  readout::Weights w;
+  readout::Outputs out;
+  const double *node_weights;
+  Scratch s;
+};
+
+template <int C, bool FORCES>
+__global__ __launch_bounds__(kThreads, 2) void second_layer_kernel(Graph q, Spline sp, SecondLayer a) {
+  using S = Shared<C, true, FORCES>;
+  constexpr int kHidden = readout::kHidden, kClasses = readout::kClasses, kPieces = C / 16, kPer = (kPieces + kClasses - 1) / kClasses;
+  __shared__ S s;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_number();
+  const int node = blockIdx.x;
+  int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
+  clamp_edge_range(e0, e1, q.nedges);
+  const int element = a.s.groups[q.nnodes + node];
+  const int64_t at = static_cast<int64_t>(node) * C;
+  if (FORCES) copy_knots(sp, s.knots);
+
+  Contraction<C> contraction;
+  Mixing<C> mixing;
+  message<C>(
+      s, a.s.X2, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.parts,
+      [&]() { contraction.request(a.T3, a.T2, a.T1, static_cast<unsigned>(element) < static_cast<unsigned>(q.nelements) ? element : 0); },
+      [&]() { mixing.request(a.mix); });
+  mixing.run(s.rows, s.part());
+  Products<C, 1> prod;
+  prod.request(a.prod);
+  // the readouts' weights: the first wave has the hidden units (unit by lane % 16, class by lane / 16), the second the linear readout
+  double wz[kPer][16];
+  f4 h1v[kPer];
+  readout::d2v wl[kPer][2];
+  const int unit = lane % 16, cls = lane / 16, lin_cls = lane % 4, lin_part = lane / 16;
+  if (wave == 0) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int c = 16 * (cls + kClasses * u) + k;
+        wz[u][k] = c < C && unit < a.w.hidden ? a.w.W2a[c * a.w.hidden + unit] : 0.0;
+      }
+  } else if (wave == 1) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int c = 16 * (lin_cls + kClasses * u) + 4 * lin_part;
+      const bool in = c < C;
+      h1v[u] = in ? ld4(a.s.h1 + at + c) : zero4();
+      wl[u][0] = in ? readout::d2v{a.w.w1[c], a.w.w1[c + 1]} : readout::d2v{0.0, 0.0};
+      wl[u][1] = in ? readout::d2v{a.w.w1[c + 2], a.w.w1[c + 3]} : readout::d2v{0.0, 0.0};
+    }
+  }
+  const float residual = tid < C ? a.s.sc[at + tid] : 0.f;
+  const int to = a.out.rows ? a.out.rows[node] : node;
+  const bool to_ok = static_cast<unsigned>(to) < static_cast<unsigned>(q.nnodes);
+  lds_barrier();
+  if (Contraction<C>::here()) {
+    const int c = Contraction<C>::channel();
+    float grad[16];
+    s.row[0][place<C>(c)] = contraction.template run<FORCES>(s.part(), a.mix_scale, grad);
+    if constexpr (FORCES) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s.grad[i * C + c] = grad[i];
+    }
+  }
+  lds_barrier();
+  prod.run(s.row[0], nullptr, s.part());
+  lds_barrier();
+  if (tid < C) {
+    const float h2 = column<C>(s.part(), tid) + residual;
+    s.h2[tid] = h2;
+    if (a.out.feats64 && to_ok) {
+      double *f = a.out.feats64 + static_cast<int64_t>(to) * (2 * C) + tid;
+      f[0] = a.s.h1[at + tid];
+      f[C] = h2;
+    }
+  }
+  Products<C, 1> back;
+  if (FORCES) back.request(a.prod_T);
+  lds_barrier();
+  // hidden units and linear readout in the classes and orders of readout_device.hpp
+  if (wave == 0) {
+    double z = 0.0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int c0 = 16 * (cls + kClasses * u);
+      if (c0 >= C) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) z = fma(wz[u][4 * p + i], static_cast<double>(s.h2[c0 + 4 * p + i]), z);
+    }
+    s.z[cls][unit] = z;
+  } else if (wave == 1 && unit < 4) {
+    double e1sum = 0.0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+      if (lin_cls + kClasses * u < kPieces) readout::add_linear(e1sum, wl[u][0], wl[u][1], h1v[u]);
+    s.e1[lin_cls][lin_part] = e1sum;
+  }
+  double wd[kHidden];
+  if (FORCES && tid < C) {
+#pragma unroll
+    for (int k = 0; k < kHidden; ++k) wd[k] = k < a.w.hidden ? a.w.W2a[tid * a.w.hidden + k] : 0.0;
+  }
+  lds_barrier();
+  if (wave == 0) {
+    const double gate = unit < a.w.hidden ? a.w.w2b[unit] * a.w.act_cst : 0.0;
+    double e2, d;
+    readout::activate(gate, (s.z[0][unit] + s.z[1][unit]) + (s.z[2][unit] + s.z[3][unit]), e2, d);
+    if (lane < 16) s.e2[unit] = e2, s.d[unit] = d;
+    wave_lds_fence();
+    const int p = lane / 16;
+    const double e = ((s.e1[0][p] + s.e1[1][p]) + (s.e1[2][p] + s.e1[3][p])) + ((s.e2[4 * p] + s.e2[4 * p + 1]) + (s.e2[4 * p + 2] + s.e2[4 * p + 3]));
+    const double en = readout::node_energy(e, a.w.scale, a.w.shift);
+    if (lane == 0) readout::store_energy(a.out, node, to, to_ok, en);
+  }
+  if constexpr (FORCES) {
+    lds_barrier();
+    if (tid < C) {
+      double g = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) g = fma(wd[4 * p + i], s.d[4 * p + i], g);
+      float d_h2 = static_cast<float>(a.w.scale * g);
+      if (a.node_weights) d_h2 = static_cast<float>(static_cast<double>(d_h2) * a.node_weights[node]);
+      a.s.d_h2[at + tid] = d_h2;
+      s.row[1][place<C>(tid)] = d_h2;
+    }
+    Mixing<C> mixing_back;
+    mixing_back.request(a.mix_T);
+    lds_barrier();
+    back.run(s.row[1], nullptr, s.part());
+    lds_barrier();
+    if (tid < C) s.h2[tid] = column<C>(s.part(), tid) * -1.0f;
+    lds_barrier();
+    for (int i = tid; i < 16 * C; i += kThreads) s.rows[i / C * C + place<C>(i % C)] = s.grad[i] * s.h2[i % C];
+    lds_barrier();
+    mixing_back.run(s.rows, s.part());
+    lds_barrier();
+    for (int i = tid; i < 16 * C; i += kThreads) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
+    lds_barrier();
+    edge_gradients<C, true>(s, a.s.X2, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.s.gv2, nullptr, a.s.gXe);
+  }
+}
+
+// ---- backward between the layers and through the first one ----------------------------------------------------------------
+struct BackToEdges {
+  const float *X1, *mix_T, *up_T, *skip_T, *prod_T;
+  float mix_scale, skip_scale;
+  const double *w1, *node_weights;
+  double scale;
+  int sender_parts, first_node;
+  EnergySums sums;
+  Scratch s;
+};
+
+// A wave's part of a sender's row sum, in the lanes of its first slot: mp_backward_sender_kernel's batches of four rows per slot.
+template <int C>
+__device__ __forceinline__ f4 sender_rows(const Spline &sp, const float *__restrict__ gXe, const int32_t *__restrict__ perm, int64_t nedges, int k0, int k1) {
+  using K = Cfg<C, false, true>;
+  const int lane = threadIdx.x % kWave, slot = lane / K::SW, cl = lane % K::SW;
+  f4 acc = zero4();
+  if (cl < K::LPE) {
+    for (int k = k0 + slot; k < k1; k += 4 * K::EPW) {
+      int e[4];
+      f4 row[4];
+      bool take[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[j] = perm[min(k + j * K::EPW, k1 - 1)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        take[j] = k + j * K::EPW < k1 && static_cast<unsigned>(e[j]) < static_cast<uint64_t>(nedges);
+        const int64_t ec = take[j] ? e[j] : 0;
+        row[j] = ld4(gXe + ec * C + 4 * cl);
+        take[j] = take[j] & (edge_length(sp.vec[3 * ec], sp.vec[3 * ec + 1], sp.vec[3 * ec + 2]) <= sp.r_max);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[j] = take[j] ? row[j] : zero4();
+      acc += (row[0] + row[1]) + (row[2] + row[3]);
+    }
+  }
+#pragma unroll
+  for (int off = kWave / 2; off >= K::SW; off >>= 1) acc += shfl_down4(acc, off);
+  return acc;
+}
+
+template <int C>
+__global__ __launch_bounds__(kThreads, 2) void back_to_edges_kernel(Graph q, Spline sp, BackToEdges a) {
+  using S = Shared<C, false, true>;
+  __shared__ S s;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_number();
+  if (static_cast<int>(blockIdx.x) < a.first_node) {
+    static_assert(sizeof(s.work) >= kThreads * sizeof(double), "the sums' place");
+    graph_energy<kThreads>(a.sums, blockIdx.x, reinterpret_cast<double *>(s.work));
+    return;
+  }
+  const int node = blockIdx.x - a.first_node;
+  const int g = min(max(a.s.groups[node], 0), q.ngroups - 1);
+  const bool no_element = g == q.ngroups - 1;
+  int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
+  clamp_edge_range(e0, e1, q.nedges);
+  const int64_t at = static_cast<int64_t>(node) * C;
+  Products<C, 2> both;
+  both.request(a.up_T, a.skip_T + static_cast<int64_t>(no_element ? 0 : g) * C * C);
+  copy_knots(sp, s.knots);
+  {
+    using K = Cfg<C, false, true>;
+    const int k0 = q.sender_offsets[node], k1 = q.sender_offsets[node + 1];
+    const int64_t len = k1 - k0;
+    if (wave < a.sender_parts) {
+      const int lo = k0 + static_cast<int>(len * wave / a.sender_parts), hi = k0 + static_cast<int>(len * (wave + 1) / a.sender_parts);
+      const f4 acc = q.nedges > 0 ? sender_rows<C>(sp, a.s.gXe, q.sender_perm, q.nedges, lo, hi) : zero4();
+      if (lane < K::LPE) st4(s.part() + wave * C + 4 * lane, acc);
+    }
+  }
+  const float d_h2 = tid < C ? a.s.d_h2[at + tid] : 0.f;
+  lds_barrier();
+  if (tid < C) {
+    float v = s.part()[tid];
+    for (int p = 1; p < a.sender_parts; ++p) v += s.part()[p * C + tid];
+    s.row[0][place<C>(tid)] = v;
+    s.row[1][place<C>(tid)] = d_h2;
+  }
+  lds_barrier();
+  both.run(s.row[0], s.row[1], s.part());
+  Products<C, 1> prod;
+  prod.request(a.prod_T);
+  lds_barrier();
+  if (tid < C)
+    s.row[2][place<C>(tid)] = gh1_of(column<C>(s.part(), tid), column<C>(s.part() + 4 * C, tid), a.w1[tid], a.scale,
+                                     a.node_weights ? a.node_weights[node] : 1.0, -a.skip_scale, no_element);
+  lds_barrier();
+  float grad1[(16 * C + kThreads - 1) / kThreads];
+#pragma unroll
+  for (int i = 0; i < 16 * C / kThreads; ++i) grad1[i] = a.s.grad1[16 * at + tid + i * kThreads];
+  Mixing<C> mixing;
+  if (!no_element) mixing.request(a.mix_T + static_cast<int64_t>(g) * (4 * C * C));
+  prod.run(s.row[2], nullptr, s.part());
+  lds_barrier();
+  if (tid < C) s.h2[tid] = column<C>(s.part(), tid);
+  lds_barrier();
+#pragma unroll
+  for (int p = 0; p < 16 * C / kThreads; ++p) {
+    const int i = tid + p * kThreads;
+    s.rows[i / C * C + place<C>(i % C)] = grad1[p] * s.h2[i % C];
+  }
+  lds_barrier();
+  if (no_element) {
+    for (int i = tid; i < 64 * C; i += kThreads) s.part()[i] = 0.f;
+  } else {
+    mixing.run(s.rows, s.part());
+  }
+  lds_barrier();
+  for (int i = tid; i < 16 * C; i += kThreads) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
+  lds_barrier();
+  edge_gradients<C, false>(s, a.X1, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.s.gv1, a.s.gv2, nullptr);
+}
+
+Graph graph_of(const cm_mace_weights &w, const cm_mace_graph &g) {
+  return Graph{static_cast<int>(g.nnodes), w.nelements + 1, w.nelements, g.nedges, g.receiver, g.sender, g.first_occ, g.sender_perm, g.sender_offsets,
+               g.elem_perm, g.elem_offsets, g.onehot_perm, g.onehot_offsets, g.node_rows};
+}
+Spline spline_of(const cm_mace_weights &w, int layer, const Scratch &s) {
+  return Spline{s.vec, nullptr, w.r_knots, w.spline[layer], w.nknots, w.r_width, w.r_max};
+}
+
+}  // namespace
+
+#define CM_FEW_NODES_C(channels, CALL)                \
+  switch (channels) {                                 \
+    case 32: { constexpr int C_ = 32; CALL; } break;   \
+    case 64: { constexpr int C_ = 64; CALL; } break;   \
+    case 96: { constexpr int C_ = 96; CALL; } break;   \
+    case 128: { constexpr int C_ = 128; CALL; } break; \
+    default: set_error("cm_mace_step: channels=%d not supported", channels); return CM_EINVAL; \
+  }
+
+// One round of workgroups, one to a compute unit (its registers and most of its LDS).  Step in us, the separate launches -> these: 21 x 64 channels
+// 77 -> 40, 256 x 52 x 32 79 -> 47, x 64 94 -> 55, x 96 121 -> 74, x 128 138 -> 88, 252 x 9 x 128 122 -> 75, 216 x 92 x 128 144 -> 101; a second round costs as
+// much again: 300 x 52 x 64 102 -> 93, x 128 149 -> 154, 1 000 x 52 x 32 102 -> 148.
+bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges) {
+  const int C = w.channels;
+  return C <= 128 && nnodes <= device_compute_units() && !w.mono3[0] && !w.mono2[0] && !w.mono3[1] && !w.mono2[1] && w.n3[0] == CM_SYMCON_N3 && w.n2[0] == CM_SYMCON_N2 &&
+         w.n3[1] == CM_SYMCON_N3 && w.n2[1] == CM_SYMCON_N2 && few::applies(nnodes, 16, C) && few::applies(nnodes, 1, C) &&
+         !sliced_forward_applies(nnodes, nedges, C, w.nknots);
+}
+
+int first_layer(const cm_mace_weights &w, const cm_mace_graph &g, const double *positions, const double *shifts, const Scratch &s, hipStream_t st) {
+  const FirstLayer a{positions, shifts, g.X1, w.mix_W[0], w.T3[0], w.T2[0], w.T1[0], w.prod_W[0], w.up_W, w.skip_W,
+                     w.mix_scale[0], w.skip_scale, edge_forward_parts(w.channels, g.nnodes, g.nedges), s.vec, s};
+  const Spline sp = spline_of(w, 0, s);
+  const dim3 grid(static_cast<unsigned>(g.nnodes));
+  CM_FEW_NODES_C(w.channels, {
+    if (s.grad1) hipLaunchKernelGGL((first_layer_kernel<C_, true>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+    else hipLaunchKernelGGL((first_layer_kernel<C_, false>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+  });
+  return check_launch("cm_mace_step (first layer)");
+}
+
+int second_layer(const cm_mace_weights &w, const cm_mace_graph &g, const readout::Outputs &out, const Scratch &s, hipStream_t st) {
+  const SecondLayer a{w.mix_W[1], w.mix_WT[1], w.T3[1], w.T2[1], w.T1[1], w.prod_W[1], w.prod_WT[1], w.mix_scale[1],
+                      edge_forward_parts(w.channels, g.nnodes, g.nedges),
+                      readout::Weights{w.w1, w.W2a, w.w2b, w.act_cst, w.scale, w.shift, w.hidden}, out, g.node_weights, s};
+  const Spline sp = spline_of(w, 1, s);
+  const dim3 grid(static_cast<unsigned>(g.nnodes));
+  CM_FEW_NODES_C(w.channels, {
+    if (s.grad1) hipLaunchKernelGGL((second_layer_kernel<C_, true>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+    else hipLaunchKernelGGL((second_layer_kernel<C_, false>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+  });
+  return check_launch("cm_mace_step (second layer)");
+}
+
+int back_to_edges(const cm_mace_weights &w, const cm_mace_graph &g, const EnergySums &sums, const Scratch &s, hipStream_t st) {
+  const BackToEdges a{g.X1, w.mix_WT[0], w.up_WT, w.skip_WT, w.prod_WT[0], w.mix_scale[0], w.skip_scale, w.w1, g.node_weights, w.scale,
+                      sender_parts_of(w.channels, g.nnodes, g.nedges), g.ngraphs, sums, s};
+  const Spline sp = spline_of(w, 0, s);
+  const dim3 grid(static_cast<unsigned>(g.nnodes + g.ngraphs));
+  CM_FEW_NODES_C(w.channels, hipLaunchKernelGGL((back_to_edges_kernel<C_>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a));
+  return check_launch("cm_mace_step (back to the edges)");
+}
+
+}  // namespace fewnodes
+}  // namespace cm

@@ -562,6 +562,12 @@ int launch_sender(const float *gXe, const int32_t *perm, const int32_t *offsets,
 
 }  // namespace
 
+int mp::sender_parts_of(int channels, int64_t nnodes, int64_t nedges) {
+  int parts = 1;
+  CM_DISPATCH_C(channels, parts = sender_parts<C_>(nnodes, nedges));
+  return parts;
+}
+
 int mp::launch_sender_pass(int channels, const float *gXe, const int32_t *perm, const int32_t *offsets, int64_t nnodes,
                            int64_t nedges, float *gX, hipStream_t st, const float *live_vec, const float *live_r,
                            float r_max, const uint32_t *live_bits) {

@@ -274,6 +274,10 @@ int launch_sender_pass(int channels, const float *gXe, const int32_t *perm, cons
                        int64_t nedges, float *gX, hipStream_t st, const float *live_vec = nullptr,
                        const float *live_r = nullptr, float r_max = 0.f, const uint32_t *live_bits = nullptr);
 
+// Parts that the forward from edge vectors with one wave per node (mp_spline.hip) and the sender pass (mp.hip) cut a node's edges into.
+int edge_forward_parts(int channels, int64_t nnodes, int64_t nedges);
+int sender_parts_of(int channels, int64_t nnodes, int64_t nedges);
+
 // Forward from edge vectors with the radial table in LDS, two degrees and one 16-channel slice per workgroup (defined in
 // mp_sliced.hip): whether it takes a launch of this shape, and the launch.  records: NULL, or per edge 16 bytes, the vector and
 // the sender (at most kMaxRecords edges), from which it reads instead of from vec and sender.

@@ -23,6 +23,7 @@
 #include "mfma_f32.hpp"
 #include "mfma_rows.hpp"
 #include "node_glue.hpp"
+#include "node_glue_device.hpp"
 #include "readout_device.hpp"
 
 // Products and the additions that follow them stay separate roundings, as they are where separate launches store the
@@ -159,60 +160,13 @@ __global__ __launch_bounds__(2 * NT *kWave) void node_glue_forward_few_kernel(
   if (here) st4(sc + at, no_element ? zero4() : v[0] * skip_scale);
 }
 
-// Energies per graph, riding in the backward launch (its tiles do not depend on them): out[g] = sum over the graph's nodes
-// of weight[n] * node_es[n], strided partial sums of the workgroup's threads (the largest power of two of them) and a tree
-// over them: a fixed order.
-struct EnergySums {
-  const double *node_es, *node_weights;
-  const int32_t *graph_ptr;
-  double *out;
-  int ngraphs;
-  const double *graph_e0;  // a constant per graph added into `total` (NULL: zero)
-  double *total;           // NULL: not asked for
-};
-template <int THREADS, int PARTS = 4>  // THREADS: a power of two, at most the workgroup's size
-__device__ __forceinline__ void graph_energy(const EnergySums &q, int graph, double *part) {
-  const int tid = threadIdx.x;
-  if (tid < THREADS) {
-    const int lo = q.graph_ptr[graph], hi = q.graph_ptr[graph + 1];
-    auto term = [&](int i) { return q.node_weights ? q.node_weights[i] * q.node_es[i] : q.node_es[i]; };
-    // PARTS strided partial sums per thread, their loads requested together: one sum after the other waits for memory
-    // once per node, and this workgroup would outlast the tiles of the launch
-    double sum[PARTS];
-#pragma unroll
-    for (int k = 0; k < PARTS; ++k) sum[k] = 0.0;
-    for (int i = lo + tid; i < hi; i += PARTS * THREADS) {
-      double t[PARTS];
-#pragma unroll
-      for (int k = 0; k < PARTS; ++k) t[k] = i + k * THREADS < hi ? term(i + k * THREADS) : 0.0;
-#pragma unroll
-      for (int k = 0; k < PARTS; ++k) sum[k] += t[k];
-    }
-#pragma unroll
-    for (int d = PARTS / 2; d > 0; d /= 2)
-#pragma unroll
-      for (int k = 0; k < d; ++k) sum[k] += sum[k + d];
-    part[tid] = sum[0];
-  }
-  __syncthreads();
-  for (int d = THREADS / 2; d > 0; d >>= 1) {
-    if (tid < d) part[tid] += part[tid + d];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    q.out[graph] = part[0];
-    if (q.total) q.total[graph] = part[0] + (q.graph_e0 ? q.graph_e0[graph] : 0.0);
-  }
-}
-
 // ---- backward: gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip[element]^T, gB1 = gh1 . Wprod^T ------------------
-// gh1 = gX2 . Wup^T + g1 - skip_scale dE/dh2 . Wskip^T of four columns of a node from the two products (factor: what takes the
-// second one to -skip_scale dE/dh2 . Wskip^T)
+// four columns of it
 __device__ __forceinline__ f4 gh1_of(f4 up, f4 skip, const double *w1, double scale, double node_weight, float factor, bool no_element) {
-  const f4 g1{static_cast<float>(-1.0 * scale * w1[0] * node_weight), static_cast<float>(-1.0 * scale * w1[1] * node_weight),
-              static_cast<float>(-1.0 * scale * w1[2] * node_weight), static_cast<float>(-1.0 * scale * w1[3] * node_weight)};
-  const f4 sum = up + g1;
-  return no_element ? sum : sum + skip * factor;
+  f4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = cm::gh1_of(up[i], skip[i], w1[i], scale, node_weight, factor, no_element);
+  return r;
 }
 
 template <int NT, int WAVES>

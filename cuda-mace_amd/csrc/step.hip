@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "few_nodes.hpp"
 #include "geometry.hpp"
 #include "mp_common.hpp"
 #include "node_glue.hpp"
@@ -448,6 +449,22 @@ extern "C" int cm_mace_step_timing_read(double *total_ms, int64_t *launches, int
 
 namespace {
 
+// The end of the step: forces, and virials on request, from the edge gradients of both layers.
+int forces_of_step(const cm::Layout &L, const cm_mace_graph *g, const double *positions, const double *shifts, double *forces, double *virials,
+                   unsigned timing_mask, cm_stream_t stream) {
+  const int64_t N = g->nnodes, E = g->nedges;
+  hipStream_t st = cm::as_stream(stream);
+  if (virials) {
+    CM_STAGE(23, cm::forces_and_node_virials(L.gv1, L.vec, g->node_rows, g->first_occ, g->sender_perm, g->sender_offsets, N, E, forces, L.node_virial, st));
+    cm::StageTimer timer_(st, 24, timing_mask);
+    hipLaunchKernelGGL(cm::graph_virial_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, L.node_virial, g->graph_ptr, virials);
+  } else {
+    CM_STAGE(23, cm_edge_geometry_backward(positions, g->receiver, g->sender, shifts, g->node_rows, g->first_occ, g->sender_perm,
+                                           g->sender_offsets, L.gv1, nullptr, N, E, forces, nullptr, stream));
+  }
+  return cm::check_launch("cm_mace_step");
+}
+
 // The step of cm_mace_step, or, with want_forces false, its forward half alone: no backward chain, and none of what only
 // that chain reads (the contractions' gradient tables, the readouts' derivative, cleared edge gradients) is formed, written or
 // given room.
@@ -501,6 +518,27 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   const int32_t *el_perm = g->elem_perm, *el_off = g->elem_offsets;
   const float *none = nullptr;
 
+  const char *glue_env = getenv("CM_STEP_GLUE");  // development switch: smallest node count that takes the chained kernels; -1: none
+  const int glue_min = glue_env ? atoi(glue_env) : 0;
+  // Few nodes: a workgroup takes a node through a whole layer (few_nodes.hip), three launches and the forces.
+  if (glue_min >= 0 && N >= glue_min && cm::fewnodes::applies(*w, N, E)) {
+    const cm::fewnodes::Scratch s{L.vec, L.X2, L.h1, L.sc, L.live, reinterpret_cast<int32_t *>(L.bufA), want_forces ? L.bufM1 : nullptr, L.d_h2,
+                                  L.edge_scratch, L.gv1, L.gv2};
+    CM_REQUIRE(w->hidden >= 1 && w->hidden <= cm::readout::kHidden, "cm_mace_step: hidden=%d must be in [1, %d]", w->hidden, cm::readout::kHidden);
+    CM_REQUIRE(E < INT32_MAX / 3, "cm_mace_step: number of edges out of range");
+    CM_STAGE(1, cm::fewnodes::first_layer(*w, *g, positions, shifts, s, st));
+    CM_STAGE(7, cm::fewnodes::second_layer(*w, *g, cm::readout::Outputs{node_energy, node_feats, g->node_rows, g->node_e0, total_node_energy}, s, st));
+    if (!want_forces) {
+      cm::StageTimer timer_(st, 12, timing_mask);
+      hipLaunchKernelGGL(cm::segment_sum_f64_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, node_energy, g->node_weights,
+                         g->graph_ptr, interaction_energy, g->graph_e0, total_energy);
+      return cm::check_launch("cm_mace_energy");
+    }
+    CM_STAGE(21, cm::fewnodes::back_to_edges(*w, *g, cm::EnergySums{node_energy, g->node_weights, g->graph_ptr, interaction_energy, g->ngraphs,
+                                                                    g->graph_e0, total_energy}, s, st));
+    return forces_of_step(L, g, positions, shifts, forces, virials, timing_mask, stream);
+  }
+
   // ---- forward ----
   // The forward kernel with the table in LDS reads an edge's vector and sender once per pair of degrees and 16 channels: one load
   // of 16 bytes from one place instead of two loads from two arrays (forward pass alone, 25 000 x 128 238 -> 229 us, 12 000 x 256
@@ -519,8 +557,6 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   float *B[2] = {L.B1, L.B2};
   float *h[2] = {L.h1, L.h2};
   // the three [N, C] products between the layers (and their three transposes in the backward) as one launch each
-  const char *glue_env = getenv("CM_STEP_GLUE");  // development switch: smallest node count that takes the chained kernels; -1: none
-  const int glue_min = glue_env ? atoi(glue_env) : 0;
   const bool glue = cm_node_glue_supported(C) != 0 && glue_min >= 0 && N >= glue_min;
   // beyond 128 channels and for few nodes the same in two launches; the head stays three, and weights of the nodes need their pass over dE/dh2
   const bool cut = !glue && glue_min >= 0 && cm::node_chains_cut(N, C);
@@ -602,15 +638,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   // its vector gradient is written onto the second layer's: gv1 = (this layer's) + gv2
   CM_STAGE(21, cm::mp::edge_backward_onto(g->X1, L.vec, w->r_knots, w->spline[0], w->nknots, w->r_width, w->r_max, L.bufA, g->sender,
                                          fo_live, N, E, C, L.gv1, L.gv2, st));
-  if (virials) {
-    CM_STAGE(23, cm::forces_and_node_virials(L.gv1, L.vec, g->node_rows, g->first_occ, g->sender_perm, g->sender_offsets, N, E, forces, L.node_virial, st));
-    cm::StageTimer timer_(st, 24, timing_mask);
-    hipLaunchKernelGGL(cm::graph_virial_kernel, dim3(g->ngraphs), dim3(cm::kSumThreads), 0, st, L.node_virial, g->graph_ptr, virials);
-  } else {
-    CM_STAGE(23, cm_edge_geometry_backward(positions, g->receiver, g->sender, shifts, g->node_rows, g->first_occ, g->sender_perm,
-                                           g->sender_offsets, L.gv1, nullptr, N, E, forces, nullptr, stream));
-  }
-  return cm::check_launch("cm_mace_step");
+  return forces_of_step(L, g, positions, shifts, forces, virials, timing_mask, stream);
 }
 
 }  // namespace

@@ -14,13 +14,12 @@
 #include <cmath>
 
 #include "common.hpp"
-#include "symcon_lmax3.inc"
+#include "symcon_device.hpp"
 
 namespace cm {
 namespace {
 
-__device__ __forceinline__ float fmad(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ __forceinline__ double fmad(double a, double b, double c) { return fma(a, b, c); }
+using symcon::fmad;
 
 // T[e, t, c] = sum over the CSR row t of val * W[e, path, c]
 template <typename S>
@@ -193,36 +192,8 @@ __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict
     const S *xp = X + static_cast<int64_t>(node) * 16 * C + c;
     S x[16], g[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      x[i] = xp[i * C];
-      g[i] = S(0);
-    }
-    S acc = t1 * x[0];
-    g[0] = t1;
-#define CM_TERM3(t, i, j, k)                    \
-  {                                             \
-    const S w = t3[t];                      \
-    const S wjk = w * (x[j] * x[k]);        \
-    acc = fmad(wjk, x[i], acc);                 \
-    if (GRAD) {                                 \
-      g[i] += wjk;                              \
-      g[j] = fmad(w * x[i], x[k], g[j]);        \
-      g[k] = fmad(w * x[i], x[j], g[k]);        \
-    }                                           \
-  }
-    CM_SYMCON_MONO3(CM_TERM3)
-#undef CM_TERM3
-#define CM_TERM2(t, i, j)                       \
-  {                                             \
-    const S w = t2[t];                      \
-    acc = fmad(w * x[i], x[j], acc);            \
-    if (GRAD) {                                 \
-      g[i] = fmad(w, x[j], g[i]);               \
-      g[j] = fmad(w, x[i], g[j]);               \
-    }                                           \
-  }
-    CM_SYMCON_MONO2(CM_TERM2)
-#undef CM_TERM2
+    for (int i = 0; i < 16; ++i) x[i] = xp[i * C];
+    const S acc = symcon::contract<S, GRAD>(x, t3, t2, t1, g);
     out[static_cast<int64_t>(node) * C + c] = acc;
     if (GRAD) {
       S *gp = grad + static_cast<int64_t>(node) * 16 * C + c;

@@ -592,6 +592,51 @@ def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, c
         torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
+@pytest.mark.parametrize("case,channels", [("alone", 32), ("molecule", 64), ("molecule", 128), ("molecules", 96), ("crowded", 32), ("crowded", 96),
+                                           ("skin", 64), ("skin", 128), ("one round", 64), ("one round", 128), ("beyond", 32), ("beyond", 128)])
+def test_step_of_few_nodes_equals_the_separate_launches(cabi, case, channels, monkeypatch):
+    """Up to a node per compute unit a workgroup takes a node through a whole layer, three launches and the forces; CM_STEP_GLUE=-1 runs the
+    launches it stands for.  Bit for bit (graph energies up to the order of their sum): no edge at all; one structure and several; more
+    edges per node than a workgroup has threads, and ranges that take several chunks; pairs beyond the cutoff, at the end of a node's range
+    and inside it; atoms of no element; weights on the node energies; energies alone; virials; the last size of the rule and the first beyond."""
+    from cuda_mace.utils.neighbour_list import neighbour_data
+    from cuda_mace.utils.synthetic import collate
+
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    if case == "crowded":
+        g = torch.Generator().manual_seed(1)
+        attrs = torch.nn.functional.one_hot(torch.randint(0, 4, (34,), generator=g), 4).double().cuda()
+        data = neighbour_data((torch.rand(34, 3, generator=g, dtype=torch.float64) * 3.0).cuda(), attrs, 5.0, (True, True, True),
+                              torch.eye(3, dtype=torch.float64, device="cuda") * 3.0)
+        assert data["edge_index"].shape[1] > 512 * 34
+    else:
+        n = {"alone": 1, "molecule": 21, "molecules": 19, "skin": 150, "one round": units, "beyond": units + 1}[case]
+        box = {"alone": 4.0, "molecule": 8.0, "molecules": 8.0}.get(case)
+        parts = [make_system(n, 4, seed=31 + k, density=None if box else 0.05, cluster_box=box) for k in range(3 if case == "molecules" else 1)]
+        data = to_device(collate(parts) if len(parts) > 1 else parts[0], "cuda")
+    if case == "skin":
+        data = neighbour_data(data["positions"], data["node_attrs"], 5.7, (True, True, True), data["cell"])
+    n = data["positions"].shape[0]
+    if n > 1:
+        data["node_attrs"] = data["node_attrs"].clone()
+        data["node_attrs"][n // 2] = 0.0  # an atom of no element
+    host = {"edge_index": data["edge_index"], "positions": data["positions"]}
+    _, model = _build(channels, (1, 6, 7, 8), host if host["edge_index"].shape[1] else {"edge_index": torch.zeros(2, 9), "positions": host["positions"]}, seed=8)
+    weighted = dict(data, node_weights=torch.rand(n, generator=torch.Generator().manual_seed(9), dtype=torch.float64).cuda())
+    for inputs, keys in ((data, {}), (weighted, {}), (data, {"compute_virials": True}), (data, {"compute_force": False})):
+        monkeypatch.delenv("CM_STEP_GLUE", raising=False)
+        with torch.set_grad_enabled("compute_force" not in keys):
+            a, again = model(dict(inputs), **keys), model(dict(inputs), **keys)
+            monkeypatch.setenv("CM_STEP_GLUE", "-1")
+            b = model(dict(inputs), **keys)
+        monkeypatch.delenv("CM_STEP_GLUE")
+        assert model._native not in (None, False)
+        for key in ("node_energy", "node_feats") + (() if "compute_force" in keys else ("forces",)) + (("virials",) if "compute_virials" in keys else ()):
+            assert torch.isfinite(a[key]).all(), key
+            assert torch.equal(a[key], b[key]) and torch.equal(a[key], again[key]), key
+        torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
+
+
 @pytest.mark.parametrize("channels", [32, 64, 96, 128, 160, 192, 224, 256])
 def test_repeated_evaluations_agree_bit_for_bit_at_every_width(cabi, channels):
     """Every kernel sums in a fixed order and reads nothing it (or an earlier kernel of the same step) has not written:
