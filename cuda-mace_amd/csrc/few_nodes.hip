@@ -28,12 +28,16 @@ namespace {
 
 using namespace mp;
 
-constexpr int kThreads = 512;
-constexpr int kWaves = kThreads / kWave;
-constexpr int kMostParts = 6;  // of the forward (forward_parts)
+// Threads of a workgroup: 512 while every node has a compute unit to itself, 256 and two nodes to a unit beyond.
+constexpr int kAlone = 512, kShared = 256;
+template <int T>
+constexpr int kMostParts = T == kAlone ? 6 : 4;  // of the forward (forward_parts; with more than a node per unit it gives no more than four)
 
 // Workgroup barrier that orders LDS alone: loads of weights that a thread has requested stay in flight across it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// the wave's number in a scalar register: a branch on it is the wave's, and what one side holds takes no registers of the other
+__device__ __forceinline__ int wave_number() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
 
 // ---- products of one row ------------------------------------------------------------------------------------------------
 // The chain of channel k in mfma_f32.hpp's product is (k / 16 + k % 4) % 4, its place there 4 (k / 16) + k % 16 / 4.  A row that is about to be
@@ -45,39 +49,36 @@ __device__ __forceinline__ int place(int k) {
 // channel at place j of chain ch
 __device__ __forceinline__ int channel_at(int ch, int j) { return 16 * (j / 4) + 4 * (j % 4) + ((ch - j / 4) & 3); }
 
-// A thread's share of NMAT products of a row and a [C, C] matrix W[k][column]: one chain of one column, C / 4 multiply-adds.
+// A thread's share of NMAT products of a row and a [C, C] matrix W[k][column]: one chain of four neighbouring columns, 16 bytes per load (a
+// load costs the path from L1 about as much with 4 bytes per lane).
 template <int C, int NMAT>
 struct Products {
-  static constexpr int kUnits = 4 * C * NMAT, kPer = (kUnits + kThreads - 1) / kThreads;
-  float w[kPer][C / 4];
+  f4 w[C / 4];
+  // whole waves: a lane beyond the last unit repeats that one
+  __device__ __forceinline__ static bool here() { return wave_number() * kWave < C * NMAT; }
+  __device__ __forceinline__ static int thread() { return min(static_cast<int>(threadIdx.x), C * NMAT - 1); }
   __device__ __forceinline__ void request(const float *W0, const float *W1 = nullptr) {
+    if (!here()) return;
+    const int unit = thread() % C, ch = unit / (C / 4);
+    const float *W = (thread() < C ? W0 : W1) + 4 * (unit % (C / 4));
 #pragma unroll
-    for (int p = 0; p < kPer; ++p) {
-      const int u = threadIdx.x + p * kThreads;
-      if (kUnits % kThreads != 0 && u >= kUnits) break;
-      const int unit = NMAT == 1 ? u : u % (4 * C), ch = unit / C;
-      const float *W = (NMAT == 1 || u < 4 * C ? W0 : W1) + unit % C;
-#pragma unroll
-      for (int j = 0; j < C / 4; ++j) w[p][j] = W[channel_at(ch, j) * C];
-    }
+    for (int j = 0; j < C / 4; ++j) w[j] = ld4(W + channel_at(ch, j) * C);
   }
   // x0, x1: the rows, by place; partial sums to part[matrix][chain][column]
   __device__ __forceinline__ void run(const float *x0, const float *x1, float *part) const {
+    if (!here()) return;
+    const int unit = thread() % C, ch = unit / (C / 4);
+    const float *x = (thread() < C ? x0 : x1) + ch * (C / 4);
+    f4 sum = zero4();
 #pragma unroll
-    for (int p = 0; p < kPer; ++p) {
-      const int u = threadIdx.x + p * kThreads;
-      if (kUnits % kThreads != 0 && u >= kUnits) break;
-      const int unit = NMAT == 1 ? u : u % (4 * C), ch = unit / C;
-      const float *x = (NMAT == 1 || u < 4 * C ? x0 : x1) + ch * (C / 4);
-      float sum = 0.f;
+    for (int j = 0; j < C / 4; j += 4) {
+      const f4 v = ld4(x + j);
 #pragma unroll
-      for (int j = 0; j < C / 4; j += 4) {
-        const f4 v = ld4(x + j);
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sum = fmaf(w[p][j + i], v[i], sum);
-      }
-      part[u] = sum;
+        for (int q = 0; q < 4; ++q) sum[q] = fmaf(w[j + i][q], v[i], sum[q]);
     }
+    st4(part + 4 * thread(), sum);
   }
 };
 // the four chains of a column
@@ -86,50 +87,85 @@ __device__ __forceinline__ float column(const float *part, int c) {
   return (part[c] + part[C + c]) + (part[2 * C + c] + part[3 * C + c]);
 }
 
-// The channel mixing of a node's 16 rows, a [C, C] block per degree: a thread has one chain of one column for the degrees of its set.
-template <int C>
+// The channel mixing of a node's 16 rows, a [C, C] block per degree: a thread has one chain of four neighbouring columns for the rows of
+// its set, all of one degree.  Sets are as many as the threads allow, in an order that gives the four SIMDs equal work (wave w is SIMD w % 4's).
+template <int C, int T>
 struct Mixing {
-  static constexpr int kSets = kThreads / (4 * C) >= 4 ? 4 : (kThreads / (4 * C) >= 2 ? 2 : 1);
-  float w[4][C / 4];
-  __device__ __forceinline__ static bool mine(int l) {  // equal work: 7 + 1 and 5 + 3 rows
-    const int set = threadIdx.x / (4 * C);
-    return set < kSets && (kSets == 1 || (kSets == 2 ? (l == 0 || l == 3) == (set == 0) : l == set));
+  static constexpr int kSpan = C <= 64 ? C : 128;  // threads of a set: whole waves from 64 columns on, the last one partly idle at 96
+  static constexpr int kSets = T / kSpan;
+  static_assert(kSets == 2 || kSets == 4 || kSets == 8 || kSets == 16, "sets");
+  f4 w[C / 4];
+  __device__ __forceinline__ static int set() {
+    const int s = threadIdx.x / kSpan;
+    return kSpan >= kWave ? __builtin_amdgcn_readfirstlane(s) : s;
   }
-  __device__ __forceinline__ void request(const float *W) {
-    const int unit = threadIdx.x % (4 * C), ch = unit / C;
+  __device__ __forceinline__ static int unit() { return threadIdx.x % kSpan; }
+  // degree of a set (4: none)
+  __device__ __forceinline__ static int degree_of(int set) {
+    if constexpr (kSets == 16) return l_of_m(set & 15);
+    if constexpr (kSets == 8) return (0x14102233 >> (4 * set)) & 7;  // as in run
+    return set == 0 ? 3 : (set == 1 ? 2 : (set == 2 ? 0 : 1));  // (of two sets the first degree)
+  }
+  __device__ __forceinline__ static bool here() { return degree_of(set()) < 4 && unit() < C; }
+  __device__ __forceinline__ void request(const float *W) { request_degree(W, degree_of(set())); }
+  __device__ __forceinline__ void request_degree(const float *W, int l) {
+    if (!here()) return;
+    const int ch = unit() / (C / 4);
+    const float *at = W + static_cast<int64_t>(l) * (C * C) + 4 * (unit() % (C / 4));
 #pragma unroll
-    for (int l = 3; l >= 0; --l) {
-      if (!mine(l)) continue;
+    for (int j = 0; j < C / 4; ++j) w[j] = ld4(at + channel_at(ch, j) * C);
+  }
+  template <int M0, int N>
+  __device__ __forceinline__ void rows(const float *x, float *part) const {
+    if (unit() >= C) return;
+    const int ch = unit() / (C / 4);
+    const float *xc = x + M0 * C + ch * (C / 4);
+    f4 sum[N];
 #pragma unroll
-      for (int j = 0; j < C / 4; ++j) w[l][j] = W[(l * C + channel_at(ch, j)) * C + unit % C];
+    for (int m = 0; m < N; ++m) sum[m] = zero4();
+#pragma unroll
+    for (int j = 0; j < C / 4; j += 4)
+#pragma unroll
+      for (int m = 0; m < N; ++m) {
+        const f4 v = ld4(xc + m * C + j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[m][q] = fmaf(w[j + i][q], v[i], sum[m][q]);
+      }
+    float *to = part + ch * (16 * C) + M0 * C + 4 * (unit() % (C / 4));
+#pragma unroll
+    for (int m = 0; m < N; ++m) st4(to + m * C, sum[m]);
+  }
+  // x: [16][C] by place; partial sums to part[chain][16][C].  W: the weights once more, for sets of two degrees.
+  __device__ __forceinline__ void run(const float *x, float *part, const float *W) {
+    const int s = set();
+    if constexpr (kSets == 16) {
+      rows<0, 1>(x + s * C, part + s * C);
+    } else if constexpr (kSets == 8) {
+      switch (s) {
+        case 0: rows<9, 4>(x, part); break;
+        case 1: rows<13, 3>(x, part); break;
+        case 2: rows<4, 3>(x, part); break;
+        case 3: rows<7, 2>(x, part); break;
+        case 4: rows<0, 1>(x, part); break;
+        case 5: rows<1, 1>(x, part); break;
+        case 7: rows<2, 2>(x, part); break;
+      }
+    } else if constexpr (kSets == 2) {
+      if (s == 0) rows<9, 7>(x, part);
+      else rows<4, 5>(x, part);
+      request_degree(W, s);
+      if (s == 0) rows<0, 1>(x, part);
+      else rows<1, 3>(x, part);
+    } else {
+      switch (s) {
+        case 0: rows<9, 7>(x, part); break;
+        case 1: rows<4, 5>(x, part); break;
+        case 2: rows<0, 1>(x, part); break;
+        case 3: rows<1, 3>(x, part); break;
+      }
     }
-  }
-  // x: [16][C] by place; partial sums to part[chain][16][C]
-  __device__ __forceinline__ void run(const float *x, float *part) const {
-    const int unit = threadIdx.x % (4 * C), ch = unit / C, col = unit % C;
-    const float *xc = x + ch * (C / 4);
-    float *to = part + ch * (16 * C) + col;
-    auto degree = [&](auto lc) {
-      constexpr int L = decltype(lc)::value;
-      if (!mine(L)) return;
-      float sum[2 * L + 1];
-#pragma unroll
-      for (int m = 0; m < 2 * L + 1; ++m) sum[m] = 0.f;
-#pragma unroll
-      for (int j = 0; j < C / 4; j += 4)
-#pragma unroll
-        for (int m = 0; m < 2 * L + 1; ++m) {
-          const f4 v = ld4(xc + (L * L + m) * C + j);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sum[m] = fmaf(w[L][j + i], v[i], sum[m]);
-        }
-#pragma unroll
-      for (int m = 0; m < 2 * L + 1; ++m) to[(L * L + m) * C] = sum[m];
-    };
-    degree(std::integral_constant<int, 3>{});
-    degree(std::integral_constant<int, 2>{});
-    degree(std::integral_constant<int, 1>{});
-    degree(std::integral_constant<int, 0>{});
   }
 };
 template <int C>
@@ -140,30 +176,33 @@ __device__ __forceinline__ float mixed(const float *part, int at, float scale) {
 }
 
 // ---- LDS of a workgroup -----------------------------------------------------------------------------------------------
-template <int C, bool FORWARD, bool BACKWARD>
+template <int C, int T, bool FORWARD, bool BACKWARD>
 struct Shared {
-  static constexpr int kForward = FORWARD ? kMostParts * kStageBytes + kMostParts * 16 * C * 4 : 0;
-  static constexpr int kBackward = BACKWARD ? kWaves * (kStageBytes + 16 * kChunk * 4) : 0;
-  static constexpr int kMixing = 64 * C * 4;
-  static constexpr int kMost = kForward > kBackward ? kForward : kBackward;
-  // staged edges and the parts' sums; partial sums of products; staged edges and the edges' sums, one after the other
-  __attribute__((aligned(16))) unsigned char work[kMost > kMixing ? kMost : kMixing];
+  static constexpr int kWaves = T / kWave, kStaged = kMostParts<T> * kStageBytes;
+  static constexpr int kForward = FORWARD ? kStaged + kMostParts<T> * 16 * C * 4 : 0;
+  static constexpr int kMixing = 64 * C * 4, kEdgeSums = BACKWARD ? kWaves * 16 * kChunk * 4 : 0;
+  static constexpr int kEdges = kMixing > kEdgeSums ? kMixing : kEdgeSums;  // where the edges staged for the backward pass lie
+  static constexpr int kBackward = kEdges + (BACKWARD ? kWaves * kStageBytes : 0);
+  // edges staged for the forward and the parts' sums; then partial sums of products or the edges' sums, and behind them, some time before they are
+  // needed, the edges staged for the backward pass
+  __attribute__((aligned(16))) unsigned char work[kForward > kBackward ? kForward : kBackward];
   __attribute__((aligned(16))) float rows[16 * C];  // operand rows, by place
   __attribute__((aligned(16))) float grad[16 * C];  // gradient rows, by channel
   __attribute__((aligned(16))) float row[3][C];     // operand rows of the products, by place
   float h2[C];
   double z[4][16], e1[4][4], e2[16], d[16];
   float knots[kKnotsInLds];
-  int mark;
+  int mark, group, element;
   __device__ float *part() { return reinterpret_cast<float *>(work); }
-  __device__ float *sums(int p) { return reinterpret_cast<float *>(work + kMostParts * kStageBytes) + p * (16 * C); }
+  __device__ float *sums(int p) { return reinterpret_cast<float *>(work + kStaged) + p * (16 * C); }
+  __device__ Staged edges() { return Staged(work + kEdges + wave_number() * kStageBytes); }
 };
 
-// the waves that contract: the last ones, which have no part of the forward
-template <int C>
+// the waves that contract: the last ones, which come last for parts of the forward too
+template <int C, int T>
 struct Contraction {
-  static constexpr int kFirst = kWaves - (C + kWave - 1) / kWave;
-  static_assert(kFirst >= kMostParts, "no part of the forward falls to a wave that contracts");
+  static constexpr int kFirst = T / kWave - (C + kWave - 1) / kWave;
+  static_assert(C <= kFirst * kWave, "the next product's threads are others");
   float t3[CM_SYMCON_N3], t2[CM_SYMCON_N2], t1;
   __device__ __forceinline__ static int channel() { return static_cast<int>(threadIdx.x) - kFirst * kWave; }
   __device__ __forceinline__ static bool here() { return channel() >= 0 && channel() < C; }
@@ -185,12 +224,9 @@ struct Contraction {
   }
 };
 
-// the wave's number in a scalar register: a branch on it is the wave's, and what one side holds takes no registers of the other
-__device__ __forceinline__ int wave_number() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
-
 // Message of the node over its edges e0 .. e1 - 1 into s.rows, the parts by waves as in mp_spline_forward_kernel.  `others` is called by the
-// waves that have no part and contract later, `meanwhile` by every thread between its part and the barrier behind which the parts are added.
-template <int C, class S, class Fn0, class Fn>
+// waves that contract later, `meanwhile` by every thread between its part and the barrier behind which the parts are added.
+template <int C, int T, class S, class Fn0, class Fn>
 __device__ __forceinline__ void message(S &s, const float *__restrict__ X, const Spline &sp, const int32_t *__restrict__ sender, int nnodes, int64_t nedges,
                                         int e0, int e1, int parts, Fn0 others, Fn meanwhile) {
   using K = Cfg<C, true>;
@@ -199,18 +235,20 @@ __device__ __forceinline__ void message(S &s, const float *__restrict__ X, const
     const int64_t len = e1 - e0;
     const int lo = e0 + static_cast<int>(len * wave / parts), hi = e0 + static_cast<int>(len * (wave + 1) / parts);
     typename K::vec acc[16];
-    forward_wave<C, true, K::V <= 4>(X, nullptr, sp, sender, nnodes, nedges, lo, hi, Staged(s.work + wave * kStageBytes), acc);
-    if (lane < K::LPE) {
-      float *to = s.sums(wave) + K::off(lane);
+    forward_wave<C>(X, sp, sender, nnodes, nedges, lo, hi, Staged(s.work + wave * kStageBytes), acc,
+                                      KnotCopy<>::applies(sp) ? s.knots : nullptr);
+    using Sums = SlotSums<K>;
+    Sums::total(acc);
+    if (Sums::holds(lane)) {
+      float *to = s.sums(wave) + Sums::first_row(lane) * C + K::off(lane % K::SW);
 #pragma unroll
-      for (int m = 0; m < 16; ++m) K::st(to + m * C, acc[m]);
+      for (int m = 0; m < Sums::kRows; ++m) K::st(to + m * C, acc[m]);
     }
-  } else if (wave >= Contraction<C>::kFirst) {
-    others();
   }
+  if (wave >= Contraction<C, T>::kFirst) others();
   meanwhile();
   lds_barrier();
-  for (int i = threadIdx.x; i < 16 * C; i += kThreads) {
+  for (int i = threadIdx.x; i < 16 * C; i += T) {
     float v = s.sums(0)[i];
     for (int p = 1; p < parts; ++p) v += s.sums(p)[i];
     s.rows[i / C * C + place<C>(i % C)] = v;
@@ -218,30 +256,51 @@ __device__ __forceinline__ void message(S &s, const float *__restrict__ X, const
   lds_barrier();
 }
 
+struct Graph {
+  int nnodes, ngroups, nelements;
+  int64_t nedges;
+  const int32_t *receiver, *sender, *first_occ, *sender_perm, *sender_offsets, *elem_perm, *elem_offsets, *onehot_perm, *onehot_offsets, *rows;
+};
+
 // Gradients of the edges e0 .. e1 - 1 of a node from its gradient rows s.grad, as mp_spline_backward_edge_kernel forms them: every edge on its
-// own, so the split over the waves is free; a wave takes as many edges as it has slots before another is given some.
-template <int C, bool WANT_GX, class S>
-__device__ __forceinline__ void edge_gradients(S &s, const float *__restrict__ X, const Spline &sp, const int32_t *__restrict__ sender, int nnodes,
-                                               int64_t nedges, int e0, int e1, float *gvec, const float *addend, float *__restrict__ gXe) {
+// own, so the split over the waves is free; a wave takes as many edges as it has slots before another is given some.  The wave's first
+// chunk is staged (stage) some time before the gradient rows are there, behind other waits.
+template <int C, int T, bool WANT_GX, class S>
+struct EdgeGradients {
   using K = Cfg<C>;
   using vec = typename K::vec;
-  const int wave = wave_number(), lane = threadIdx.x % kWave;
-  const int slot = lane / K::SW, cl = lane % K::SW;
-  const bool active = cl < K::LPE;
-  const unsigned cla = active ? cl : 0;
-  const int64_t len = e1 - e0;
-  const int parts = static_cast<int>(min(static_cast<int64_t>(kWaves), (len + K::EPW - 1) / K::EPW));
-  if (wave >= parts) return;
-  const int lo = e0 + static_cast<int>(len * wave / parts), hi = e0 + static_cast<int>(len * (wave + 1) / parts);
-  unsigned char *mine = s.work + wave * (kStageBytes + 16 * kChunk * 4);
-  const Staged st(mine);
-  float *sGY = reinterpret_cast<float *>(mine + kStageBytes);
-  vec g[16];
-#pragma unroll
-  for (int m = 0; m < 16; ++m) g[m] = active ? K::ld(s.grad + m * C + K::off(cl)) : zerov<vec>();
-  for (int cursor = lo; cursor < hi;) {
-    const int base = cursor;
-    wave_lds_fence();
+  S &s;
+  const Spline &sp;
+  const int32_t *sender;
+  int nnodes;
+  int64_t nedges;
+  float *gvec;
+  const float *addend;
+  int cursor, hi, nlive, base;
+
+  __device__ __forceinline__ Staged staged() const { return s.edges(); }
+  __device__ __forceinline__ EdgeGradients(S &s_, const Spline &sp_, const Graph &q, float *gvec_, const float *addend_, int e0, int e1)
+      : s(s_), sp(sp_), sender(q.sender), nnodes(q.nnodes), nedges(q.nedges), gvec(gvec_), addend(addend_) {
+    const int64_t len = e1 - e0, wave = wave_number();
+    const int parts = static_cast<int>(min(static_cast<int64_t>(T / kWave), (len + K::EPW - 1) / K::EPW));
+    cursor = wave < parts ? e0 + static_cast<int>(len * wave / parts) : e1;
+    hi = wave < parts ? e0 + static_cast<int>(len * (wave + 1) / parts) : e1;
+    nlive = 0, base = cursor;
+  }
+  // the raw edges of the first chunk, and their staging; the knots are in LDS
+  __device__ __forceinline__ RawEdge request() const {
+    RawEdge r{-1, 0.f, 0.f, 0.f};
+    if (cursor >= hi) return r;
+    const int64_t e = min(cursor + static_cast<int>(threadIdx.x % kWave), hi - 1);
+    r.s = sender[e];
+    r.v0 = sp.vec[3 * e + 0], r.v1 = sp.vec[3 * e + 1], r.v2 = sp.vec[3 * e + 2];
+    return r;
+  }
+  template <bool AHEAD>
+  __device__ __forceinline__ void stage(RawEdge ahead) {
+    if (cursor >= hi) return;
+    const int lane = threadIdx.x % kWave;
+    base = cursor;
     auto dead = [&](int pass_base, int, unsigned long long, bool lane_is_dead) {
       if (lane_is_dead) {
         const int64_t e = pass_base + lane;
@@ -249,69 +308,87 @@ __device__ __forceinline__ void edge_gradients(S &s, const float *__restrict__ X
         for (int k = 0; k < 3; ++k) gvec[3 * e + k] = addend ? addend[3 * e + k] : 0.f;
       }
     };
-    const int nlive = stage_edges<true>(nullptr, sender, sp, nnodes, nedges, cursor, hi, lane, st.sY, st.sS, st.sIdx, st.sXr, st.sOrig, dead,
-                                        RawEdge{-1, 0.f, 0.f, 0.f}, s.knots, KnotCopy<>::applies(sp));
+    const Staged st = staged();
     wave_lds_fence();
-    Operands<K> o;
-    if (slot < nlive) fetch_operands<C>(o, X, sp.coeffs, st.sS[slot], st.sIdx[slot], st.sXr[slot], cla);
-#pragma unroll 1
-    for (int j = slot; j < nlive; j += K::EPW) {
-      float y[16], p[16];
-      staged_harmonics(st.sY, j, y);
-      vec gxe = zerov<vec>(), grq = zerov<vec>();
-      edge_products<K, true, true, true, WANT_GX>(o, y, g, p, gxe, grq);
-      p[0] = dotv(o.x, grq);
-      if constexpr (WANT_GX) {
-        if (active) K::st(gXe + static_cast<int64_t>(base + st.sOrig[j]) * C + K::off(cl), gxe);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      const int next = j + K::EPW < nlive ? j + K::EPW : j;
-      fetch_operands<C>(o, X, sp.coeffs, st.sS[next], st.sIdx[next], st.sXr[next], cla);
-      slot_reduce16<K::SW>(p, cl);
-      store_reduced16<K::SW>(p, cl, j, sGY);
-    }
+    nlive = stage_edges<true, AHEAD>(nullptr, sender, sp, nnodes, nedges, cursor, hi, lane, st.sY, st.sS, st.sIdx, st.sXr, st.sOrig, dead, ahead, s.knots,
+                                     KnotCopy<>::applies(sp));
     wave_lds_fence();
-    if (lane < nlive) {
-      float sums[16];
+  }
+  // the operands of the slots' first edges
+  __device__ __forceinline__ void fetch(Operands<K> &o, const float *__restrict__ X, int j) const {
+    const int cl = threadIdx.x % K::SW;
+    const Staged st = staged();
+    fetch_operands<C>(o, X, sp.coeffs, st.sS[j], st.sIdx[j], st.sXr[j], cl < K::LPE ? cl : 0);
+  }
+  __device__ __forceinline__ void run(const float *__restrict__ X, float *__restrict__ gXe) {
+    const int lane = threadIdx.x % kWave, slot = lane / K::SW, cl = lane % K::SW;
+    const bool active = cl < K::LPE;
+    if (base >= hi) return;
+    const Staged st = staged();
+    float *const sGY = s.part() + wave_number() * (16 * kChunk);
+    vec g[16];
 #pragma unroll
-      for (int m = 0; m < 16; ++m) sums[m] = sGY[m * kChunk + lane];
-      finish_vector_gradient(sp.vec, base + st.sOrig[lane], sums, addend, gvec);
+    for (int m = 0; m < 16; ++m) g[m] = active ? K::ld(s.grad + m * C + K::off(cl)) : zerov<vec>();
+    for (;;) {
+      Operands<K> o;
+      if (slot < nlive) fetch(o, X, slot);
+#pragma unroll 1
+      for (int j = slot; j < nlive; j += K::EPW) {
+        float y[16], p[16];
+        staged_harmonics(st.sY, j, y);
+        vec gxe = zerov<vec>(), grq = zerov<vec>();
+        edge_products<K, true, true, true, WANT_GX>(o, y, g, p, gxe, grq);
+        p[0] = dotv(o.x, grq);
+        if constexpr (WANT_GX) {
+          if (active) K::st(gXe + static_cast<int64_t>(base + st.sOrig[j]) * C + K::off(cl), gxe);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(o, X, j + K::EPW < nlive ? j + K::EPW : j);
+        slot_reduce16<K::SW>(p, cl);
+        store_reduced16<K::SW>(p, cl, j, sGY);
+      }
+      wave_lds_fence();
+      if (lane < nlive) {
+        float sums[16];
+#pragma unroll
+        for (int m = 0; m < 16; ++m) sums[m] = sGY[m * kChunk + lane];
+        finish_vector_gradient(sp.vec, base + st.sOrig[lane], sums, addend, gvec);
+      }
+      if (cursor >= hi) break;
+      stage<false>(RawEdge{-1, 0.f, 0.f, 0.f});
     }
   }
-}
+};
 
-// copy of the knots for edge_gradients; a barrier follows before they are read
+// copy of the knots; a barrier follows before they are read
+template <int T>
 __device__ __forceinline__ void copy_knots(const Spline &sp, float *to) {
   if (KnotCopy<>::applies(sp))
-    for (int i = threadIdx.x; i < sp.nknots; i += kThreads) to[i] = sp.knots[i];
+    for (int i = threadIdx.x; i < sp.nknots; i += T) to[i] = sp.knots[i];
 }
 
-// Position of `node` in a permutation of the nodes (-1: not there), by the calling wave, and the group of a position.
-__device__ __forceinline__ int position_of(const int32_t *__restrict__ perm, int nnodes, int node, int guess) {
-  if (perm[guess] == node) return guess;
-  for (int base = 0; base < nnodes; base += kWave) {
-    const int i = base + threadIdx.x % kWave;
-    const unsigned long long found = __ballot(i < nnodes && perm[min(i, nnodes - 1)] == node);
-    if (found != 0) return base + __ffsll(static_cast<long long>(found)) - 1;
+// The group of a node in a grouped order of the nodes (-1: the order does not name it), by the calling wave.
+__device__ __forceinline__ int group_of(const int32_t *__restrict__ perm, const int32_t *__restrict__ offsets, int nnodes, int ngroups, int node) {
+  const int lane = threadIdx.x % kWave;
+  int pos = -1;
+  for (int base = 0; base < nnodes && pos < 0; base += 4 * kWave) {
+    int at[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) at[k] = perm[min(base + k * kWave + lane, nnodes - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const unsigned long long found = __ballot(base + k * kWave + lane < nnodes && at[k] == node);
+      if (found != 0 && pos < 0) pos = base + k * kWave + __ffsll(static_cast<long long>(found)) - 1;
+    }
   }
-  return -1;
-}
-__device__ __forceinline__ int group_of(const int32_t *__restrict__ offsets, int ngroups, int pos) {
+  if (pos < 0) return -1;
   for (int base = 0; base < ngroups; base += kWave) {
-    const int i = base + threadIdx.x % kWave;
-    const bool here = i < ngroups && offsets[min(i, ngroups - 1)] <= pos && pos < offsets[min(i, ngroups - 1) + 1];
-    const unsigned long long found = __ballot(here);
+    const int i = min(base + lane, ngroups - 1);
+    const unsigned long long found = __ballot(base + lane < ngroups && offsets[i] <= pos && pos < offsets[i + 1]);
     if (found != 0) return base + __ffsll(static_cast<long long>(found)) - 1;
   }
   return -1;
 }
-
-// A permutation that does not name a node leaves its row of the scratch arrays as it was: what is read from them is clamped.
-struct Graph {
-  int nnodes, ngroups, nelements;
-  int64_t nedges;
-  const int32_t *receiver, *sender, *first_occ, *sender_perm, *sender_offsets, *elem_perm, *elem_offsets, *onehot_perm, *onehot_offsets, *rows;
-};
 
 // ---- first layer ----------------------------------------------------------------------------------------------------------
 struct FirstLayer {
@@ -323,23 +400,26 @@ struct FirstLayer {
   Scratch s;
 };
 
-template <int C, bool FORCES>
-__global__ __launch_bounds__(kThreads, 2) void first_layer_kernel(Graph q, Spline sp, FirstLayer a) {
-  using S = Shared<C, true, false>;
+template <int C, int T, bool FORCES>
+__global__ __launch_bounds__(T, 2) void first_layer_kernel(Graph q, Spline sp, FirstLayer a) {
+  using S = Shared<C, T, true, false>;
   __shared__ S s;
   const int tid = threadIdx.x;
-  int g, pos, gend;
-  if (!locate_group_tile(q.onehot_offsets, q.ngroups, q.nnodes, blockIdx.x, 1, g, pos, gend)) return;
-  const int node = q.onehot_perm[pos];
-  if (static_cast<unsigned>(node) >= static_cast<unsigned>(q.nnodes)) return;
-  const bool no_element = g == q.ngroups - 1;
-
-  // edge vectors, and the end of the range of edges inside the cutoff
+  const int node = blockIdx.x, wave = wave_number();
+  // edge vectors, and the end of the range of edges inside the cutoff; the last two waves look the node's groups up meanwhile
   int e0 = q.first_occ[node], e1 = q.first_occ[q.nnodes + node];
   clamp_edge_range(e0, e1, q.nedges);
+  copy_knots<T>(sp, s.knots);
   if (tid == 0) s.mark = e0;
   lds_barrier();
-  for (int e = e0 + tid; e < e1; e += kThreads) {
+  if (wave == S::kWaves - 1) {
+    const int element = group_of(q.elem_perm, q.elem_offsets, q.nnodes, q.nelements, node);
+    if (tid % kWave == 0) s.element = element;
+  } else if (wave == S::kWaves - 2) {
+    const int g = group_of(q.onehot_perm, q.onehot_offsets, q.nnodes, q.ngroups, node);
+    if (tid % kWave == 0) s.group = g < 0 ? q.ngroups - 1 : g;
+  }
+  for (int e = e0 + tid; e < e1; e += T) {
     double v[3];
     edge_vector_f64(a.positions, q.receiver, q.sender, a.shifts, q.rows, e, q.nnodes, v);
     const float v0 = static_cast<float>(v[0]), v1 = static_cast<float>(v[1]), v2 = static_cast<float>(v[2]);
@@ -355,35 +435,34 @@ __global__ __launch_bounds__(kThreads, 2) void first_layer_kernel(Graph q, Splin
   }
   __syncthreads();  // the vectors are in memory
   e1 = s.mark;
+  const int g = s.group, element = s.element;
+  const bool no_element = g == q.ngroups - 1;
+  if (tid == T - 1) {
+    a.s.live[node] = e0;
+    a.s.live[q.nnodes + node] = e1;
+    a.s.groups[node] = g;
+    a.s.groups[q.nnodes + node] = element;
+  }
 
-  Contraction<C> contraction;
-  Mixing<C> mixing;
-  message<C>(
-      s, a.X1, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.parts,
+  const float *mix = a.mix + static_cast<int64_t>(no_element ? 0 : g) * (4 * C * C);
+  Contraction<C, T> contraction;
+  Mixing<C, T> mixing;
+  message<C, T>(
+      s, a.X1, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.parts, [&]() { contraction.request(a.T3, a.T2, a.T1, max(element, 0)); },
       [&]() {
-        const int in_elements = position_of(q.elem_perm, q.nnodes, node, pos);
-        const int element = in_elements < 0 ? -1 : group_of(q.elem_offsets, q.nelements, in_elements);
-        if (tid == kThreads - 1) {
-          a.s.live[node] = e0;
-          a.s.live[q.nnodes + node] = e1;
-          a.s.groups[node] = g;
-          a.s.groups[q.nnodes + node] = element;
-        }
-        contraction.request(a.T3, a.T2, a.T1, max(element, 0));
-      },
-      [&]() {
-        if (!no_element) mixing.request(a.mix + static_cast<int64_t>(g) * (4 * C * C));
+        if (!no_element) mixing.request(mix);
       });
   if (no_element) {
-    for (int i = tid; i < 64 * C; i += kThreads) s.part()[i] = 0.f;
+    for (int i = tid; i < 64 * C; i += T) s.part()[i] = 0.f;
   } else {
-    mixing.run(s.rows, s.part());
+    mixing.run(s.rows, s.part(), mix);
   }
   Products<C, 1> prod;
-  prod.request(a.prod);
   lds_barrier();
-  if (Contraction<C>::here()) {
-    const int c = Contraction<C>::channel();
+  if (wave < Contraction<C, T>::kFirst) {
+    prod.request(a.prod);
+  } else if (Contraction<C, T>::here()) {
+    const int c = Contraction<C, T>::channel();
     float grad[16];
     float b = contraction.template run<FORCES>(s.part(), a.mix_scale, grad);
     s.row[0][place<C>(c)] = b;
@@ -426,57 +505,60 @@ struct SecondLayer {
   Scratch s;
 };
 
-template <int C, bool FORCES>
-__global__ __launch_bounds__(kThreads, 2) void second_layer_kernel(Graph q, Spline sp, SecondLayer a) {
-  using S = Shared<C, true, FORCES>;
+template <int C, int T, bool FORCES>
+__global__ __launch_bounds__(T, 2) void second_layer_kernel(Graph q, Spline sp, SecondLayer a) {
+  using S = Shared<C, T, true, FORCES>;
   constexpr int kHidden = readout::kHidden, kClasses = readout::kClasses, kPieces = C / 16, kPer = (kPieces + kClasses - 1) / kClasses;
   __shared__ S s;
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_number();
   const int node = blockIdx.x;
-  int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
-  clamp_edge_range(e0, e1, q.nedges);
+  const int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
   const int element = a.s.groups[q.nnodes + node];
   const int64_t at = static_cast<int64_t>(node) * C;
-  if (FORCES) copy_knots(sp, s.knots);
+  copy_knots<T>(sp, s.knots);
+  EdgeGradients<C, T, true, S> gradients(s, sp, q, a.s.gv2, nullptr, e0, e1);
+  lds_barrier();
 
-  Contraction<C> contraction;
-  Mixing<C> mixing;
-  message<C>(
+  Contraction<C, T> contraction;
+  Mixing<C, T> mixing;
+  message<C, T>(
       s, a.s.X2, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.parts,
-      [&]() { contraction.request(a.T3, a.T2, a.T1, static_cast<unsigned>(element) < static_cast<unsigned>(q.nelements) ? element : 0); },
+      [&]() { contraction.request(a.T3, a.T2, a.T1, max(element, 0)); },
       [&]() { mixing.request(a.mix); });
-  mixing.run(s.rows, s.part());
+  mixing.run(s.rows, s.part(), a.mix);
   Products<C, 1> prod;
-  prod.request(a.prod);
   // the readouts' weights: the first wave has the hidden units (unit by lane % 16, class by lane / 16), the second the linear readout
   double wz[kPer][16];
   f4 h1v[kPer];
   readout::d2v wl[kPer][2];
   const int unit = lane % 16, cls = lane / 16, lin_cls = lane % 4, lin_part = lane / 16;
-  if (wave == 0) {
-#pragma unroll
-    for (int u = 0; u < kPer; ++u)
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int c = 16 * (cls + kClasses * u) + k;
-        wz[u][k] = c < C && unit < a.w.hidden ? a.w.W2a[c * a.w.hidden + unit] : 0.0;
-      }
-  } else if (wave == 1) {
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int c = 16 * (lin_cls + kClasses * u) + 4 * lin_part;
-      const bool in = c < C;
-      h1v[u] = in ? ld4(a.s.h1 + at + c) : zero4();
-      wl[u][0] = in ? readout::d2v{a.w.w1[c], a.w.w1[c + 1]} : readout::d2v{0.0, 0.0};
-      wl[u][1] = in ? readout::d2v{a.w.w1[c + 2], a.w.w1[c + 3]} : readout::d2v{0.0, 0.0};
-    }
-  }
   const float residual = tid < C ? a.s.sc[at + tid] : 0.f;
   const int to = a.out.rows ? a.out.rows[node] : node;
   const bool to_ok = static_cast<unsigned>(to) < static_cast<unsigned>(q.nnodes);
   lds_barrier();
-  if (Contraction<C>::here()) {
-    const int c = Contraction<C>::channel();
+  if (wave < Contraction<C, T>::kFirst) {
+    prod.request(a.prod);
+    if (wave == 0) {
+#pragma unroll
+      for (int u = 0; u < kPer; ++u)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          const int c = 16 * (cls + kClasses * u) + k;
+          wz[u][k] = c < C && unit < a.w.hidden ? a.w.W2a[c * a.w.hidden + unit] : 0.0;
+        }
+    } else if (wave == 1) {
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int c = 16 * (lin_cls + kClasses * u) + 4 * lin_part;
+        const bool in = c < C;
+        h1v[u] = in ? ld4(a.s.h1 + at + c) : zero4();
+        wl[u][0] = in ? readout::d2v{a.w.w1[c], a.w.w1[c + 1]} : readout::d2v{0.0, 0.0};
+        wl[u][1] = in ? readout::d2v{a.w.w1[c + 2], a.w.w1[c + 3]} : readout::d2v{0.0, 0.0};
+      }
+    }
+    if (FORCES) gradients.template stage<false>(RawEdge{-1, 0.f, 0.f, 0.f});
+  } else if (Contraction<C, T>::here()) {
+    const int c = Contraction<C, T>::channel();
     float grad[16];
     s.row[0][place<C>(c)] = contraction.template run<FORCES>(s.part(), a.mix_scale, grad);
     if constexpr (FORCES) {
@@ -487,6 +569,7 @@ __global__ __launch_bounds__(kThreads, 2) void second_layer_kernel(Graph q, Spli
   lds_barrier();
   prod.run(s.row[0], nullptr, s.part());
   lds_barrier();
+  if (FORCES && wave >= Contraction<C, T>::kFirst) gradients.template stage<false>(RawEdge{-1, 0.f, 0.f, 0.f});
   if (tid < C) {
     const float h2 = column<C>(s.part(), tid) + residual;
     s.h2[tid] = h2;
@@ -549,20 +632,20 @@ __global__ __launch_bounds__(kThreads, 2) void second_layer_kernel(Graph q, Spli
       a.s.d_h2[at + tid] = d_h2;
       s.row[1][place<C>(tid)] = d_h2;
     }
-    Mixing<C> mixing_back;
-    mixing_back.request(a.mix_T);
     lds_barrier();
     back.run(s.row[1], nullptr, s.part());
+    Mixing<C, T> mixing_back;
+    mixing_back.request(a.mix_T);
     lds_barrier();
     if (tid < C) s.h2[tid] = column<C>(s.part(), tid) * -1.0f;
     lds_barrier();
-    for (int i = tid; i < 16 * C; i += kThreads) s.rows[i / C * C + place<C>(i % C)] = s.grad[i] * s.h2[i % C];
+    for (int i = tid; i < 16 * C; i += T) s.rows[i / C * C + place<C>(i % C)] = s.grad[i] * s.h2[i % C];
     lds_barrier();
-    mixing_back.run(s.rows, s.part());
+    mixing_back.run(s.rows, s.part(), a.mix_T);
     lds_barrier();
-    for (int i = tid; i < 16 * C; i += kThreads) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
+    for (int i = tid; i < 16 * C; i += T) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
     lds_barrier();
-    edge_gradients<C, true>(s, a.s.X2, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.s.gv2, nullptr, a.s.gXe);
+    gradients.run(a.s.X2, a.s.gXe);
   }
 }
 
@@ -607,35 +690,40 @@ __device__ __forceinline__ f4 sender_rows(const Spline &sp, const float *__restr
   return acc;
 }
 
-template <int C>
-__global__ __launch_bounds__(kThreads, 2) void back_to_edges_kernel(Graph q, Spline sp, BackToEdges a) {
-  using S = Shared<C, false, true>;
+template <int C, int T>
+__global__ __launch_bounds__(T, 2) void back_to_edges_kernel(Graph q, Spline sp, BackToEdges a) {
+  using S = Shared<C, T, false, true>;
   __shared__ S s;
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_number();
   if (static_cast<int>(blockIdx.x) < a.first_node) {
-    static_assert(sizeof(s.work) >= kThreads * sizeof(double), "the sums' place");
-    graph_energy<kThreads>(a.sums, blockIdx.x, reinterpret_cast<double *>(s.work));
+    static_assert(sizeof(s.work) >= T * sizeof(double), "the sums' place");
+    graph_energy<T>(a.sums, blockIdx.x, reinterpret_cast<double *>(s.work));
     return;
   }
   const int node = blockIdx.x - a.first_node;
-  const int g = min(max(a.s.groups[node], 0), q.ngroups - 1);
+  const int g = a.s.groups[node];
   const bool no_element = g == q.ngroups - 1;
-  int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
-  clamp_edge_range(e0, e1, q.nedges);
+  const int e0 = a.s.live[node], e1 = a.s.live[q.nnodes + node];
   const int64_t at = static_cast<int64_t>(node) * C;
+  copy_knots<T>(sp, s.knots);
+  EdgeGradients<C, T, false, S> gradients(s, sp, q, a.s.gv1, a.s.gv2, e0, e1);
+  const RawEdge raw = gradients.request();
+  lds_barrier();
+  const float *skip_T = a.skip_T + static_cast<int64_t>(no_element ? 0 : g) * C * C;
   Products<C, 2> both;
-  both.request(a.up_T, a.skip_T + static_cast<int64_t>(no_element ? 0 : g) * C * C);
-  copy_knots(sp, s.knots);
+  if constexpr (C <= 96) both.request(a.up_T, skip_T);  // (no registers for them here beyond)
   {
     using K = Cfg<C, false, true>;
     const int k0 = q.sender_offsets[node], k1 = q.sender_offsets[node + 1];
     const int64_t len = k1 - k0;
-    if (wave < a.sender_parts) {
-      const int lo = k0 + static_cast<int>(len * wave / a.sender_parts), hi = k0 + static_cast<int>(len * (wave + 1) / a.sender_parts);
-      const f4 acc = q.nedges > 0 ? sender_rows<C>(sp, a.s.gXe, q.sender_perm, q.nedges, lo, hi) : zero4();
-      if (lane < K::LPE) st4(s.part() + wave * C + 4 * lane, acc);
+    for (int p = wave; p < a.sender_parts; p += S::kWaves) {
+      const int lo = k0 + static_cast<int>(len * p / a.sender_parts), hi = k0 + static_cast<int>(len * (p + 1) / a.sender_parts);
+      const f4 acc = sender_rows<C>(sp, a.s.gXe, q.sender_perm, q.nedges, lo, hi);
+      if (lane < K::LPE) st4(s.part() + p * C + 4 * lane, acc);
     }
   }
+  gradients.template stage<true>(raw);
+  if constexpr (C > 96) both.request(a.up_T, skip_T);
   const float d_h2 = tid < C ? a.s.d_h2[at + tid] : 0.f;
   lds_barrier();
   if (tid < C) {
@@ -653,30 +741,31 @@ __global__ __launch_bounds__(kThreads, 2) void back_to_edges_kernel(Graph q, Spl
     s.row[2][place<C>(tid)] = gh1_of(column<C>(s.part(), tid), column<C>(s.part() + 4 * C, tid), a.w1[tid], a.scale,
                                      a.node_weights ? a.node_weights[node] : 1.0, -a.skip_scale, no_element);
   lds_barrier();
-  float grad1[(16 * C + kThreads - 1) / kThreads];
+  float grad1[(16 * C + T - 1) / T];
 #pragma unroll
-  for (int i = 0; i < 16 * C / kThreads; ++i) grad1[i] = a.s.grad1[16 * at + tid + i * kThreads];
-  Mixing<C> mixing;
-  if (!no_element) mixing.request(a.mix_T + static_cast<int64_t>(g) * (4 * C * C));
+  for (int i = 0; i < 16 * C / T; ++i) grad1[i] = a.s.grad1[16 * at + tid + i * T];
   prod.run(s.row[2], nullptr, s.part());
+  Mixing<C, T> mixing;
+  const float *mix_T = a.mix_T + static_cast<int64_t>(no_element ? 0 : g) * (4 * C * C);
+  if (!no_element) mixing.request(mix_T);
   lds_barrier();
   if (tid < C) s.h2[tid] = column<C>(s.part(), tid);
   lds_barrier();
 #pragma unroll
-  for (int p = 0; p < 16 * C / kThreads; ++p) {
-    const int i = tid + p * kThreads;
+  for (int p = 0; p < 16 * C / T; ++p) {
+    const int i = tid + p * T;
     s.rows[i / C * C + place<C>(i % C)] = grad1[p] * s.h2[i % C];
   }
   lds_barrier();
   if (no_element) {
-    for (int i = tid; i < 64 * C; i += kThreads) s.part()[i] = 0.f;
+    for (int i = tid; i < 64 * C; i += T) s.part()[i] = 0.f;
   } else {
-    mixing.run(s.rows, s.part());
+    mixing.run(s.rows, s.part(), mix_T);
   }
   lds_barrier();
-  for (int i = tid; i < 16 * C; i += kThreads) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
+  for (int i = tid; i < 16 * C; i += T) s.grad[i] = mixed<C>(s.part(), i, a.mix_scale);
   lds_barrier();
-  edge_gradients<C, false>(s, a.X1, sp, q.sender, q.nnodes, q.nedges, e0, e1, a.s.gv1, a.s.gv2, nullptr);
+  gradients.run(a.X1, nullptr);
 }
 
 Graph graph_of(const cm_mace_weights &w, const cm_mace_graph &g) {
@@ -687,23 +776,36 @@ Spline spline_of(const cm_mace_weights &w, int layer, const Scratch &s) {
   return Spline{s.vec, nullptr, w.r_knots, w.spline[layer], w.nknots, w.r_width, w.r_max};
 }
 
+// call(std::integral_constant channels, std::integral_constant threads)
+template <class Call>
+int dispatch(int channels, int64_t nnodes, Call call) {
+  const auto threads = [&](auto c) {
+    if (nnodes <= device_compute_units()) call(c, std::integral_constant<int, kAlone>{});
+    else call(c, std::integral_constant<int, kShared>{});
+    return CM_OK;
+  };
+  switch (channels) {
+    case 32: return threads(std::integral_constant<int, 32>{});
+    case 64: return threads(std::integral_constant<int, 64>{});
+    case 96: return threads(std::integral_constant<int, 96>{});
+    case 128: return threads(std::integral_constant<int, 128>{});
+    default: set_error("cm_mace_step: channels=%d not supported", channels); return CM_EINVAL;
+  }
+}
+
 }  // namespace
 
-#define CM_FEW_NODES_C(channels, CALL)                \
-  switch (channels) {                                 \
-    case 32: { constexpr int C_ = 32; CALL; } break;   \
-    case 64: { constexpr int C_ = 64; CALL; } break;   \
-    case 96: { constexpr int C_ = 96; CALL; } break;   \
-    case 128: { constexpr int C_ = 128; CALL; } break; \
-    default: set_error("cm_mace_step: channels=%d not supported", channels); return CM_EINVAL; \
-  }
-
-// One round of workgroups, one to a compute unit (its registers and most of its LDS).  Step in us, the separate launches -> these: 21 x 64 channels
-// 77 -> 40, 256 x 52 x 32 79 -> 47, x 64 94 -> 55, x 96 121 -> 74, x 128 138 -> 88, 252 x 9 x 128 122 -> 75, 216 x 92 x 128 144 -> 101; a second round costs as
-// much again: 300 x 52 x 64 102 -> 93, x 128 149 -> 154, 1 000 x 52 x 32 102 -> 148.
+// Up to a node per compute unit a workgroup of eight waves has a unit to itself, up to two it has four waves and half of one; a second round of
+// those pays at 32 and 64 channels, whose weights are small.  Beyond, the launches that share weights between nodes are faster (and round
+// otherwise beyond few::applies: 384 nodes at 128 channels, 512 at 96, 768 at 64).  Step in us, the separate launches -> these:
+//   32   21 x 9 71 -> 36, 256 x 52 75 -> 42, 512 x 52 85 -> 51, 756 x 9 77 -> 65, 1 000 x 52 99 -> 90, 1 500 x 52 113 -> 131
+//   64   21 x 9 71 -> 39, 100 x 52 85 -> 49, 256 x 52 91 -> 53, 500 x 52 111 -> 70, 504 x 9 95 -> 48, 600 x 52 117 -> 113, 756 x 9 102 -> 82
+//   96   21 x 9 82 -> 53, 256 x 52 116 -> 72, 500 x 52 138 -> 95, 504 x 9 115 -> 71
+//   128  21 x 9 92 -> 62, 216 x 92 141 -> 99, 256 x 52 136 -> 86, 384 x 52 155 -> 115, 378 x 9 132 -> 85
+// (eight waves to half of the nodes: 64 channels, 216 x 52, 51 against 55 with four.)
 bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges) {
   const int C = w.channels;
-  return C <= 128 && nnodes <= device_compute_units() && !w.mono3[0] && !w.mono2[0] && !w.mono3[1] && !w.mono2[1] && w.n3[0] == CM_SYMCON_N3 && w.n2[0] == CM_SYMCON_N2 &&
+  return C <= 128 && nnodes <= (C == 32 ? 4 : 3) * device_compute_units() && !w.mono3[0] && !w.mono2[0] && !w.mono3[1] && !w.mono2[1] && w.n3[0] == CM_SYMCON_N3 && w.n2[0] == CM_SYMCON_N2 &&
          w.n3[1] == CM_SYMCON_N3 && w.n2[1] == CM_SYMCON_N2 && few::applies(nnodes, 16, C) && few::applies(nnodes, 1, C) &&
          !sliced_forward_applies(nnodes, nedges, C, w.nknots);
 }
@@ -713,10 +815,12 @@ int first_layer(const cm_mace_weights &w, const cm_mace_graph &g, const double *
                      w.mix_scale[0], w.skip_scale, edge_forward_parts(w.channels, g.nnodes, g.nedges), s.vec, s};
   const Spline sp = spline_of(w, 0, s);
   const dim3 grid(static_cast<unsigned>(g.nnodes));
-  CM_FEW_NODES_C(w.channels, {
-    if (s.grad1) hipLaunchKernelGGL((first_layer_kernel<C_, true>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
-    else hipLaunchKernelGGL((first_layer_kernel<C_, false>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+  const int rc = dispatch(w.channels, g.nnodes, [&](auto c, auto t) {
+    constexpr int kC = decltype(c)::value, kT = decltype(t)::value;
+    if (s.grad1) hipLaunchKernelGGL((first_layer_kernel<kC, kT, true>), grid, dim3(kT), 0, st, graph_of(w, g), sp, a);
+    else hipLaunchKernelGGL((first_layer_kernel<kC, kT, false>), grid, dim3(kT), 0, st, graph_of(w, g), sp, a);
   });
+  if (rc != CM_OK) return rc;
   return check_launch("cm_mace_step (first layer)");
 }
 
@@ -726,10 +830,12 @@ int second_layer(const cm_mace_weights &w, const cm_mace_graph &g, const readout
                       readout::Weights{w.w1, w.W2a, w.w2b, w.act_cst, w.scale, w.shift, w.hidden}, out, g.node_weights, s};
   const Spline sp = spline_of(w, 1, s);
   const dim3 grid(static_cast<unsigned>(g.nnodes));
-  CM_FEW_NODES_C(w.channels, {
-    if (s.grad1) hipLaunchKernelGGL((second_layer_kernel<C_, true>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
-    else hipLaunchKernelGGL((second_layer_kernel<C_, false>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a);
+  const int rc = dispatch(w.channels, g.nnodes, [&](auto c, auto t) {
+    constexpr int kC = decltype(c)::value, kT = decltype(t)::value;
+    if (s.grad1) hipLaunchKernelGGL((second_layer_kernel<kC, kT, true>), grid, dim3(kT), 0, st, graph_of(w, g), sp, a);
+    else hipLaunchKernelGGL((second_layer_kernel<kC, kT, false>), grid, dim3(kT), 0, st, graph_of(w, g), sp, a);
   });
+  if (rc != CM_OK) return rc;
   return check_launch("cm_mace_step (second layer)");
 }
 
@@ -738,7 +844,11 @@ int back_to_edges(const cm_mace_weights &w, const cm_mace_graph &g, const Energy
                       sender_parts_of(w.channels, g.nnodes, g.nedges), g.ngraphs, sums, s};
   const Spline sp = spline_of(w, 0, s);
   const dim3 grid(static_cast<unsigned>(g.nnodes + g.ngraphs));
-  CM_FEW_NODES_C(w.channels, hipLaunchKernelGGL((back_to_edges_kernel<C_>), grid, dim3(kThreads), 0, st, graph_of(w, g), sp, a));
+  const int rc = dispatch(w.channels, g.nnodes, [&](auto c, auto t) {
+    constexpr int kC = decltype(c)::value, kT = decltype(t)::value;
+    hipLaunchKernelGGL((back_to_edges_kernel<kC, kT>), grid, dim3(kT), 0, st, graph_of(w, g), sp, a);
+  });
+  if (rc != CM_OK) return rc;
   return check_launch("cm_mace_step (back to the edges)");
 }
 

@@ -54,6 +54,11 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::
   const int wave = MULTI ? threadIdx.x / kWave : 0;
   const int parts = MULTI ? blockDim.x / kWave : 1;
   unsigned char *mine = dyn_lds + wave * kStageBytes;
+  float *sY = reinterpret_cast<float *>(mine);
+  int *sS = reinterpret_cast<int *>(mine + kChunk * 64);
+  int *sIdx = sS + kChunk;
+  float *sXr = reinterpret_cast<float *>(sIdx + kChunk);
+  int *sOrig = reinterpret_cast<int *>(sXr + kChunk);
 
   const int node = blockIdx.x;
   const int lane = threadIdx.x % kWave;
@@ -71,7 +76,105 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::
   }
 
   vec acc[16];
-  forward_wave<C, FROM_VEC, MULTI && K::V <= 4>(X, Y, sp, sender, nnodes, nedges, e0, e1, Staged(mine), acc);
+#pragma unroll
+  for (int m = 0; m < 16; ++m) acc[m] = zerov<vec>();
+
+  for (int base = e0; base < e1;) {
+    wave_lds_fence();  // the staged edges belong to this wave alone
+    const int nlive = stage_edges<FROM_VEC>(Y, sender, sp, nnodes, nedges, base, e1, lane, sY, sS, sIdx, sXr, sOrig,
+                                            [](int, int, unsigned long long, bool) {});
+    wave_lds_fence();
+    if (active) {
+      // what one edge brings in: the sender's row piece, the 16 coefficient pieces of its knot interval, its harmonics
+      struct Edge {
+        vec x, coef[16];
+        float y[16], xr;
+      };
+      auto fetch = [&](int j, Edge &e) {
+        const int s = sS[j];
+        const int idx = sIdx[j];
+        e.xr = sXr[j];
+        e.x = K::ld(X + (static_cast<unsigned>(s) * C + unsigned(K::off(cl))));
+        const f4 *yp = reinterpret_cast<const f4 *>(sY + j * 16);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f4 v = yp[q];
+          e.y[4 * q] = v.x, e.y[4 * q + 1] = v.y, e.y[4 * q + 2] = v.z, e.y[4 * q + 3] = v.w;
+        }
+        const unsigned co = static_cast<unsigned>(idx) * (16u * C) + unsigned(K::off(cl));  // 32-bit offset from the uniform table base
+        // addressed from the middle of the interval's 16C-float row: all 16 pieces lie within +-8C floats of it, which
+        // up to C = 128 fits the signed immediate offset of a load, so one address serves them all
+        const float *mid = sp.coeffs + (co + 8 * C);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) e.coef[q] = K::ld(mid + (q * C - 8 * C));  // piece q: coefficient q / 4 of degree q % 4
+      };
+      auto accumulate = [&](const Edge &e) {
+        auto per_l = [&](auto lc) {
+          constexpr int L = decltype(lc)::value;
+          const vec t = e.x * (e.coef[L] + e.xr * (e.coef[4 + L] + e.xr * (e.coef[8 + L] + e.xr * e.coef[12 + L])));
+#pragma unroll
+          for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) acc[m] += e.y[m] * t;
+        };
+        per_l(std::integral_constant<int, 0>{});
+        per_l(std::integral_constant<int, 1>{});
+        per_l(std::integral_constant<int, 2>{});
+        per_l(std::integral_constant<int, 3>{});
+      };
+      if constexpr (MULTI && K::V <= 4) {
+        // few nodes: a wave's part is a dozen edges, and what it waits for is one memory round trip per trip of this
+        // loop, so two edges per slot are requested per trip (same order of the sums; registers for it up to four
+        // channels per lane)
+        for (int j = slot; j < nlive; j += 2 * K::EPW) {
+          Edge e0, e1;
+          const bool two = j + K::EPW < nlive;
+          fetch(j, e0);
+          fetch(two ? j + K::EPW : j, e1);
+          __builtin_amdgcn_sched_barrier(0);  // both edges' loads stay ahead of the first edge's arithmetic
+          accumulate(e0);
+          if (two) accumulate(e1);
+        }
+      } else {
+        // one edge per trip; per degree the four coefficient pieces are loaded, used and dropped (16 registers of
+        // radial data live at a time)
+        for (int j = slot; j < nlive; j += K::EPW) {
+          const int s = sS[j];
+          const int idx = sIdx[j];
+          const float xr = sXr[j];
+          const vec x = K::ld(X + (static_cast<unsigned>(s) * C + unsigned(K::off(cl))));
+          float y[16];
+          {
+            const f4 *yp = reinterpret_cast<const f4 *>(sY + j * 16);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f4 v = yp[q];
+              y[4 * q] = v.x, y[4 * q + 1] = v.y, y[4 * q + 2] = v.z, y[4 * q + 3] = v.w;
+            }
+          }
+          const unsigned co = static_cast<unsigned>(idx) * (16u * C) + unsigned(K::off(cl));
+          const float *__restrict__ tab = sp.coeffs;
+          auto per_l = [&](auto lc) {
+            constexpr int L = decltype(lc)::value;
+            const float *mid = tab + (co + 8 * C);
+            const vec a = K::ld(mid + (L * C - 8 * C)), b = K::ld(mid + (L * C - 4 * C)), c = K::ld(mid + L * C),
+                      d = K::ld(mid + (L * C + 4 * C));
+            const vec t = x * (a + xr * (b + xr * (c + xr * d)));
+#pragma unroll
+            for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) acc[m] += y[m] * t;
+          };
+          per_l(std::integral_constant<int, 0>{});
+          per_l(std::integral_constant<int, 1>{});
+          per_l(std::integral_constant<int, 2>{});
+          per_l(std::integral_constant<int, 3>{});
+        }
+      }
+    }
+  }
+
+#pragma unroll
+  for (int off = kWave / 2; off >= K::SW; off >>= 1) {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) acc[m] += shfl_downv(acc[m], off);
+  }
   if (parts > 1) {
     // sums of the parts, added up by the first wave in the order of the parts (the same on every run)
     float *comb = reinterpret_cast<float *>(dyn_lds + parts * kStageBytes);

@@ -165,12 +165,45 @@ struct Staged {
         sXr(reinterpret_cast<float *>(sIdx + kChunk)), sOrig(reinterpret_cast<int *>(sXr + kChunk)) {}
 };
 
-// A wave's sums over the edges e0 .. e1 - 1 of a node, in the lanes of its first slot: acc[m] for the lane's channels.
-// TWO: two edges per slot are requested per trip.
-template <int C, bool FROM_VEC, bool TWO>
-__device__ __forceinline__ void forward_wave(const float *__restrict__ X, const float *__restrict__ Y, const Spline &sp,
+// The slots of a wave have sums of their own (a vector per row m and lane); total() adds them up, (s0 + s2) + (s1 + s3) for four slots, and
+// leaves every lane with kRows of the node's 16 rows, from first_row on: a stage swaps half of the rows against the other half of the
+// lanes, so that it adds where a plain exchange of all 16 rows through LDS (ds_bpermute, one per value) took as many again.
+template <class K>
+struct SlotSums {
+  using vec = typename K::vec;
+  static constexpr int kRows = K::SW >= 64 ? 16 : (K::SW == 32 ? 8 : 4);
+  __device__ static __forceinline__ int first_row(int lane) { return K::SW >= 64 ? 0 : (K::SW == 32 ? 8 * (lane / 32) : 4 * (2 * (lane / 32) + lane / 16 % 2)); }
+  // the lane has a share of the result (each share is held once)
+  __device__ static __forceinline__ bool holds(int lane) { return lane % K::SW < K::LPE && (K::SW > 8 || (lane & 8) == 0); }
+  template <int N, class Swap>
+  __device__ static __forceinline__ void halve(vec (&acc)[16], Swap swap) {
+#pragma unroll
+    for (int m = 0; m < N; ++m)
+#pragma unroll
+      for (int i = 0; i < K::V; ++i) {
+        const auto both = swap(__float_as_uint(acc[m][i]), __float_as_uint(acc[N + m][i]));
+        const unsigned first = both[0], second = both[1];  // element-wise copies, as in slot_reduce16
+        acc[m][i] = __uint_as_float(first) + __uint_as_float(second);
+      }
+  }
+  __device__ static __forceinline__ void total(vec (&acc)[16]) {
+    if constexpr (K::SW <= 32) halve<8>(acc, [](unsigned p, unsigned q) { return __builtin_amdgcn_permlane32_swap(p, q, false, false); });
+    if constexpr (K::SW <= 16) halve<4>(acc, [](unsigned p, unsigned q) { return __builtin_amdgcn_permlane16_swap(p, q, false, false); });
+    if constexpr (K::SW == 8) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int i = 0; i < K::V; ++i) acc[m][i] += dpp_move<0x128>(acc[m][i]);
+    }
+  }
+};
+
+// A wave's sums over the edges e0 .. e1 - 1 of a node, in each slot: acc[m] for the lane's channels.  The loop of mp_spline_forward_kernel's
+// several waves per node (up to four channels per lane).  lds_knots: a copy of the knots in LDS, or NULL.
+template <int C>
+__device__ __forceinline__ void forward_wave(const float *__restrict__ X, const Spline &sp,
                                              const int32_t *__restrict__ sender, int nnodes, int64_t nedges, int e0, int e1, const Staged &st,
-                                             typename Cfg<C, true>::vec (&acc)[16]) {
+                                             typename Cfg<C, true>::vec (&acc)[16], const float *lds_knots = nullptr) {
   using K = Cfg<C, true>;
   using vec = typename K::vec;
   const int lane = threadIdx.x % kWave;
@@ -186,8 +219,9 @@ __device__ __forceinline__ void forward_wave(const float *__restrict__ X, const 
 
   for (int base = e0; base < e1;) {
     wave_lds_fence();  // the staged edges belong to this wave alone
-    const int nlive = stage_edges<FROM_VEC>(Y, sender, sp, nnodes, nedges, base, e1, lane, sY, sS, sIdx, sXr, sOrig,
-                                            [](int, int, unsigned long long, bool) {});
+    const int nlive = stage_edges<true>(nullptr, sender, sp, nnodes, nedges, base, e1, lane, sY, sS, sIdx, sXr, sOrig,
+                                            [](int, int, unsigned long long, bool) {}, RawEdge{-1, 0.f, 0.f, 0.f}, lds_knots,
+                                            lds_knots != nullptr);
     wave_lds_fence();
     if (active) {
       // what one edge brings in: the sender's row piece, the 16 coefficient pieces of its knot interval, its harmonics
@@ -225,60 +259,19 @@ __device__ __forceinline__ void forward_wave(const float *__restrict__ X, const 
         per_l(std::integral_constant<int, 2>{});
         per_l(std::integral_constant<int, 3>{});
       };
-      if constexpr (TWO) {
-        // few nodes: a wave's part is a dozen edges, and what it waits for is one memory round trip per trip of this
-        // loop, so two edges per slot are requested per trip (same order of the sums; registers for it up to four
-        // channels per lane)
-        for (int j = slot; j < nlive; j += 2 * K::EPW) {
-          Edge e0, e1;
-          const bool two = j + K::EPW < nlive;
-          fetch(j, e0);
-          fetch(two ? j + K::EPW : j, e1);
-          __builtin_amdgcn_sched_barrier(0);  // both edges' loads stay ahead of the first edge's arithmetic
-          accumulate(e0);
-          if (two) accumulate(e1);
-        }
-      } else {
-        // one edge per trip; per degree the four coefficient pieces are loaded, used and dropped (16 registers of
-        // radial data live at a time)
-        for (int j = slot; j < nlive; j += K::EPW) {
-          const int s = sS[j];
-          const int idx = sIdx[j];
-          const float xr = sXr[j];
-          const vec x = K::ld(X + (static_cast<unsigned>(s) * C + unsigned(K::off(cl))));
-          float y[16];
-          {
-            const f4 *yp = reinterpret_cast<const f4 *>(sY + j * 16);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const f4 v = yp[q];
-              y[4 * q] = v.x, y[4 * q + 1] = v.y, y[4 * q + 2] = v.z, y[4 * q + 3] = v.w;
-            }
-          }
-          const unsigned co = static_cast<unsigned>(idx) * (16u * C) + unsigned(K::off(cl));
-          const float *__restrict__ tab = sp.coeffs;
-          auto per_l = [&](auto lc) {
-            constexpr int L = decltype(lc)::value;
-            const float *mid = tab + (co + 8 * C);
-            const vec a = K::ld(mid + (L * C - 8 * C)), b = K::ld(mid + (L * C - 4 * C)), c = K::ld(mid + L * C),
-                      d = K::ld(mid + (L * C + 4 * C));
-            const vec t = x * (a + xr * (b + xr * (c + xr * d)));
-#pragma unroll
-            for (int m = MRange<L>::lo; m < MRange<L>::hi; ++m) acc[m] += y[m] * t;
-          };
-          per_l(std::integral_constant<int, 0>{});
-          per_l(std::integral_constant<int, 1>{});
-          per_l(std::integral_constant<int, 2>{});
-          per_l(std::integral_constant<int, 3>{});
-        }
+      // few nodes: a wave's part is a dozen edges, and what it waits for is one memory round trip per trip of this
+      // loop, so two edges per slot are requested per trip (same order of the sums; registers for it up to four
+      // channels per lane)
+      for (int j = slot; j < nlive; j += 2 * K::EPW) {
+        Edge e0, e1;
+        const bool two = j + K::EPW < nlive;
+        fetch(j, e0);
+        fetch(two ? j + K::EPW : j, e1);
+        __builtin_amdgcn_sched_barrier(0);  // both edges' loads stay ahead of the first edge's arithmetic
+        accumulate(e0);
+        if (two) accumulate(e1);
       }
     }
-  }
-
-#pragma unroll
-  for (int off = kWave / 2; off >= K::SW; off >>= 1) {
-#pragma unroll
-    for (int m = 0; m < 16; ++m) acc[m] += shfl_downv(acc[m], off);
   }
 }
 

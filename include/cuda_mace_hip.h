@@ -585,8 +585,8 @@ typedef struct cm_mace_graph {
  * 13 seeds of the backward chain, with 12 in their launch; 14 / 19 linear after the contraction, backward; 15 / 20 channel mixing backward (contraction
  * backward folded in); 16 message passing backward of layer 1 (edge pass + sender pass); 21 of layer 0 (edge pass
  * only); 17 linear_up backward; 18 skip backward; 22 sum of the two layers' per-edge gradients; 23 edge geometry backward
- * (forces); 24 virials.  Up to a node per compute unit and 128 channels a launch takes a node through a whole layer: 0 to 6 count as 1,
- * 7 to 16 as 7, 17 to 21 as 21. */
+ * (forces); 24 virials.  With few nodes (up to 1 024 at 32 channels, 384 at 128; few_nodes.hip) a launch takes a node through a whole layer: 0 to 6 count as
+ * 1, 7 to 16 as 7, 17 to 21 as 21. */
 int cm_mace_step_timing(unsigned stage_mask);
 /* A control launch for benchmarks (no counterpart in the reference): `workgroups` workgroups of 256 lanes, each lane
  * 8 * iters independent fp32 multiply-adds and nothing else (2 * 8 * iters * 256 * workgroups flop); out: one float the
@@ -604,7 +604,7 @@ int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double
  * per graph may differ from its in the last bits (up to 128 channels the full step forms them in another launch, with
  * another number of partial sums).  No backward chain runs, nothing that only it reads is written, and the workspace,
  * cm_mace_energy_workspace(nnodes, nedges, channels) bytes, has no room for it (a workspace of cm_mace_step will do as well).
- * 3 launches up to a node per compute unit and 128 channels, 10 for more nodes (11 with few at 96 and 128), 13 beyond (12 with few nodes).  For callers that compare energies: Monte Carlo moves, screening. */
+ * 3 launches with few nodes up to 128 channels (few_nodes.hip), 10 with more (11 up to some thousand at 96 and 128), 13 beyond (12 with few nodes).  For callers that compare energies: Monte Carlo moves, screening. */
 size_t cm_mace_energy_workspace(int64_t nnodes, int64_t nedges, int channels);
 int cm_mace_energy(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
                    void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy, double *node_feats,

@@ -593,12 +593,14 @@ def test_step_with_chained_readouts_equals_the_separate_launches(cabi, natoms, c
 
 
 @pytest.mark.parametrize("case,channels", [("alone", 32), ("molecule", 64), ("molecule", 128), ("molecules", 96), ("crowded", 32), ("crowded", 96),
-                                           ("skin", 64), ("skin", 128), ("one round", 64), ("one round", 128), ("beyond", 32), ("beyond", 128)])
+                                           ("skin", 64), ("skin", 128), ("one round", 64), ("one round", 128), ("two to a unit", 32), ("two to a unit", 128),
+                                           ("last", 32), ("last", 64), ("last", 96), ("last", 128), ("beyond", 32), ("beyond", 128)])
 def test_step_of_few_nodes_equals_the_separate_launches(cabi, case, channels, monkeypatch):
-    """Up to a node per compute unit a workgroup takes a node through a whole layer, three launches and the forces; CM_STEP_GLUE=-1 runs the
+    """With few nodes a workgroup takes a node through a whole layer, three launches and the forces; CM_STEP_GLUE=-1 runs the
     launches it stands for.  Bit for bit (graph energies up to the order of their sum): no edge at all; one structure and several; more
     edges per node than a workgroup has threads, and ranges that take several chunks; pairs beyond the cutoff, at the end of a node's range
-    and inside it; atoms of no element; weights on the node energies; energies alone; virials; the last size of the rule and the first beyond."""
+    and inside it; atoms of no element; weights on the node energies; energies alone; virials; a node per compute unit and the first size beyond it; the last size of the rule
+    at every width and the first beyond."""
     from cuda_mace.utils.neighbour_list import neighbour_data
     from cuda_mace.utils.synthetic import collate
 
@@ -610,7 +612,8 @@ def test_step_of_few_nodes_equals_the_separate_launches(cabi, case, channels, mo
                               torch.eye(3, dtype=torch.float64, device="cuda") * 3.0)
         assert data["edge_index"].shape[1] > 512 * 34
     else:
-        n = {"alone": 1, "molecule": 21, "molecules": 19, "skin": 150, "one round": units, "beyond": units + 1}[case]
+        last = {32: 4 * units, 64: min(3 * units, 768), 96: min(3 * units, 512), 128: min(3 * units, 384)}[channels]
+        n = {"alone": 1, "molecule": 21, "molecules": 19, "skin": 150, "one round": units, "two to a unit": units + 1, "last": last, "beyond": last + 1}[case]
         box = {"alone": 4.0, "molecule": 8.0, "molecules": 8.0}.get(case)
         parts = [make_system(n, 4, seed=31 + k, density=None if box else 0.05, cluster_box=box) for k in range(3 if case == "molecules" else 1)]
         data = to_device(collate(parts) if len(parts) > 1 else parts[0], "cuda")
