@@ -12,6 +12,7 @@
 // dispatches the contraction on float and double (jit_wrappers/src/symmetric_contraction_wrapper.cpp:68).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 #include "symcon_device.hpp"
@@ -153,28 +154,38 @@ constexpr int kMaxNodesPerBlock = 16;
 // its bytes; sixteen are one round and two waves more), 25 000 x 96 80.8 66.7 62.8 62.8 62.0 [66.4 68.6] 77.7, 2 000 x 128 11.0 [9.0] 10.1 11.1 13.2 15.7
 // 21.7 26.8, 5 000 x 96 21.3 17.3 19.1 [16.3] 17.1 19.9 24.4 30.1, 10 752 x 128 39.7 34.3 34.0 33.4 37.2 [32.7] 32.1 36.0, 10 752 x 64 22.5 20.1 21.4 [19.2] 19.5 21.9 26.0 30.8, 216 x 128 [4.8] 6.1 7.4 8.8.
 // In fp64 one wave fills a SIMD: 16 nodes where that still gives every SIMD two waves, fewer for fewer nodes.
+// PAIRED kernels (below) have two nodes at a time: p / 2 of a node's time.
 template <typename S>
-int nodes_per_wave(int64_t nnodes, int nelements, int64_t column_blocks) {
+int nodes_per_wave(int64_t nnodes, int nelements, int64_t column_blocks, bool paired) {
   const double simds = 4.0 * device_compute_units(), n = static_cast<double>(nnodes), columns = static_cast<double>(column_blocks);
   if (sizeof(S) == 8) return std::max(1, static_cast<int>(std::min<double>(kMaxNodesPerBlock, n * columns / (2.0 * simds))));
-  int best = 1;
+  const int each = paired ? 2 : 1;
+  int best = each;
   double least = 0.0;
-  for (int p = 1; p <= kMaxNodesPerBlock; ++p) {
+  for (int p = each; p <= kMaxNodesPerBlock * each; p += each) {
     const double rounds = columns * (n / p + 0.5 * nelements) / (3.0 * simds), full = std::floor(rounds);  // (half a wave lost per element)
-    const double time = (full + (rounds > full ? 0.45 + 0.55 * (rounds - full) : 0.0)) * (p + 0.3);
-    if (p == 1 || time < least) best = p, least = time;
+    const double time = (full + (rounds > full ? 0.45 + 0.55 * (rounds - full) : 0.0)) * (p / each + 0.3);
+    if (p == each || time < least) best = p, least = time;
   }
   return best;
 }
 
-template <typename S, bool GRAD>
+// PAIRED: 32 channels of two nodes per wave, for channel counts that are an odd multiple of 32, where 64 channels of one leave half of the
+// last wave idle.  us with the gradient, 64 channels -> two nodes: 32 channels 5 000 9.0 -> 6.5, 25 000 29 -> 21 (32 without the gradient 17 -> 12); 96
+// 600 5.0 -> 5.3, 1 200 6.8 -> 7.2, 2 000 7.9 -> 7.4, 3 500 12.1 -> 10.0, 25 000 63 -> 55, 60 000 175 -> 160; 160 600 5.8 -> 5.5, 2 000 10.9 -> 9.8, 25 000
+// 108 -> 101; 224, where an eighth of the lanes is all there is to gain, 2 000 13.5 -> 13.1, 3 500 20.7 -> 22.6, 25 000 159 -> 156.
+inline bool two_nodes_per_wave(int channels, int64_t nnodes) {
+  return channels == 32 || channels == 160 || (channels == 96 && nnodes > 6 * device_compute_units());
+}
+template <typename S, bool GRAD, bool PAIRED>
 __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict__ X,
                                                             const int32_t *__restrict__ node_perm,
                                                             const int32_t *__restrict__ group_offsets,
                                                             const S *__restrict__ T3, const S *__restrict__ T2,
                                                             const S *__restrict__ T1, int nnodes, int ne, int C,
                                                             int npb, S *__restrict__ out, S *__restrict__ grad) {
-  const int c = blockIdx.y * kWave + threadIdx.x;
+  constexpr int kChannels = PAIRED ? kWave / 2 : kWave, kNodes = kWave / kChannels;
+  const int c = blockIdx.y * kChannels + threadIdx.x % kChannels;
   int e, pos0, gend;
   if (!locate_group_tile(group_offsets, ne, nnodes, blockIdx.x, npb, e, pos0, gend) || c >= C) return;
   const int nb = min(npb, gend - pos0);
@@ -186,7 +197,7 @@ __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict
   for (int t = 0; t < CM_SYMCON_N2; ++t) t2[t] = T2[(static_cast<int64_t>(e) * CM_SYMCON_N2 + t) * C + c];
   const S t1 = T1[static_cast<int64_t>(e) * C + c];
 
-  for (int b = 0; b < nb; ++b) {
+  for (int b = threadIdx.x / kChannels; b < nb; b += kNodes) {
     const int node = node_perm[pos0 + b];
     if (static_cast<unsigned>(node) >= static_cast<unsigned>(nnodes)) continue;
     const S *xp = X + static_cast<int64_t>(node) * 16 * C + c;
@@ -277,15 +288,23 @@ int forward(const char *what, const S *X, const int32_t *node_perm, const int32_
                "%s: built-in structure has %d cubic and %d quadratic monomials, got %d and %d", what, CM_SYMCON_N3,
                CM_SYMCON_N2, n3, n2);
     CM_REQUIRE(T3 && T2, "%s: NULL table", what);
-    const int64_t column_blocks = ceil_div(channels, kWave);
-    const int npb = nodes_per_wave<S>(nnodes, nelements, column_blocks);
+    const bool paired = sizeof(S) == 4 && two_nodes_per_wave(channels, nnodes);
+    const int64_t column_blocks = ceil_div(channels, paired ? kWave / 2 : kWave);
+    const int npb = nodes_per_wave<S>(nnodes, nelements, column_blocks, paired);
     const dim3 grid(static_cast<unsigned>(ceil_div(nnodes, npb) + nelements), static_cast<unsigned>(column_blocks));
-    if (grad)
-      hipLaunchKernelGGL((symcon_lmax3_kernel<S, true>), grid, dim3(kWave), 0, st, X, node_perm, group_offsets, T3, T2, T1,
-                         static_cast<int>(nnodes), nelements, channels, npb, out, grad);
-    else
-      hipLaunchKernelGGL((symcon_lmax3_kernel<S, false>), grid, dim3(kWave), 0, st, X, node_perm, group_offsets, T3, T2, T1,
-                         static_cast<int>(nnodes), nelements, channels, npb, out, grad);
+    const auto launch = [&](auto with_grad, auto two) {
+      hipLaunchKernelGGL((symcon_lmax3_kernel<S, decltype(with_grad)::value, decltype(two)::value>), grid, dim3(kWave), 0, st, X, node_perm,
+                         group_offsets, T3, T2, T1, static_cast<int>(nnodes), nelements, channels, npb, out, grad);
+    };
+    if constexpr (sizeof(S) == 4) {
+      if (paired) {
+        if (grad) launch(std::true_type{}, std::true_type{});
+        else launch(std::false_type{}, std::true_type{});
+        return check_launch(what);
+      }
+    }
+    if (grad) launch(std::true_type{}, std::false_type{});
+    else launch(std::false_type{}, std::false_type{});
     return check_launch(what);
   }
   // LDS per workgroup is held to 32 KB in fp32, 64 KB in fp64 (two [NB][16][C] arrays) so that several fit a CU

@@ -60,3 +60,31 @@ def test_symmetric_contraction_module(cabi, N, C, ne, seed):
     close(grad_b, grad_t.double().cpu(), 1e-5, 1e-6)
     out_ng, none = cabi.symcon_forward(xa, perm, off, t(m3), t(m2), T3, T2, T1, want_grad=False, builtin=True)
     assert none is None and torch.equal(out_ng, out_b)
+
+
+@pytest.mark.parametrize("N,C,ne", [(1, 32, 1), (2, 160, 2), (3, 32, 3), (35, 160, 3), (1001, 32, 10), (1700, 96, 4), (1700, 160, 4), (5003, 96, 10)])
+def test_two_nodes_per_wave(cabi, N, C, ne):
+    """Channel counts that are an odd multiple of 32 have 32 channels of two nodes in a wave (at 96 beyond some nodes): groups of odd size, of one
+    node and without any; with and without the gradient.  A node's numbers are those it has in a call of a few nodes, and the oracle's."""
+    up, mod = _module(ne, C, N)
+    con = up.contractions[0]
+    g = torch.Generator().manual_seed(N)
+    X = torch.randn(N, 16, C, generator=g, dtype=torch.float32)
+    types = torch.randint(0, max(ne - 1, 1), (N,), generator=g).int()  # the last element has no node where there are several
+    types[N // 2] = 0
+    Xg = X.cuda().requires_grad_(True)
+    out = mod(Xg, types.cuda()).squeeze(1)
+    (grad,) = torch.autograd.grad(out.sum(), Xg)
+    assert torch.equal(mod(X.cuda(), types.cuda()).squeeze(1), out)
+    pick = torch.unique(torch.cat([torch.arange(min(N, 5)), torch.arange(max(N - 5, 0), N), torch.randint(0, N, (20,), generator=g)]))
+    Xp = X[pick].cuda().requires_grad_(True)
+    out_p = mod(Xp, types[pick].cuda()).squeeze(1)
+    (grad_p,) = torch.autograd.grad(out_p.sum(), Xp)
+    assert torch.equal(out[pick.cuda()], out_p) and torch.equal(grad[pick.cuda()], grad_p)
+    U1, U2, U3 = (torch.from_numpy(u) for u in u_tensors())
+    W3, W2, W1 = (w.detach().float().double() for w in (con.weights_max, con.weights[0], con.weights[1]))
+    Xa = X[pick].double().requires_grad_(True)
+    ref = O.symmetric_contraction(Xa, types[pick], U3, U2, W3, W2, W1)
+    ref.sum().backward()
+    close(out_p.detach(), ref.detach(), 3e-5, 3e-6)
+    close(grad_p, Xa.grad, 3e-5, 3e-6)
