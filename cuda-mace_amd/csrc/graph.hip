@@ -13,6 +13,7 @@
 //            within the cutoff come first, by the new label of atom j (ties in the list's order), then the others by
 //            length (ties in the list's order).  No global sort of the edges: a wave ranks the pairs of one atom.
 //   derived  CSR offsets of the new row i, the view of the new list sorted by row j.
+#include <algorithm>
 #include <cfloat>
 
 #include "common.hpp"
@@ -24,121 +25,200 @@
 namespace cm {
 namespace {
 
-constexpr int kBoxThreads = 1024;
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / kWave;
+constexpr int kMaxBoxes = 64;  // partial bounding boxes; a wave reduces them
 constexpr int kScanThreads = 1024;
 constexpr int kScanStage = 32 * 1024;  // values staged in LDS at a time (128 KB)
-constexpr int kSegLds = 1024;  // keys of a segment that a wave keeps in LDS
+constexpr int kSegLds = 512;   // keys of a segment that a wave keeps in LDS
+constexpr int kBucketLds = 256;  // pairs of one sender that a wave keeps in LDS
 
-// box[0..2] = smallest coordinate per axis, box[3] = largest extent over the axes (one workgroup; a fixed order)
-__global__ __launch_bounds__(kBoxThreads) void bounding_box_kernel(const double *__restrict__ pos, int64_t n, double *__restrict__ box) {
-  __shared__ double lo[3][kBoxThreads], hi[3][kBoxThreads];
-  const int t = threadIdx.x;
-  double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  for (int64_t i = t; i < n; i += kBoxThreads) {
+// What bounds the whole call is the launches: each holds microseconds of work that waits for the one before.  There are eight
+// of them, where one kernel per step (box, keys, clear, histogram, scan, fill, rank, ...) took seventeen: every counter is
+// cleared by the first, the old CSR and the pairs per sender are taken while the atoms are binned, and the offsets of the view
+// by sender are known before the pairs are placed, so the pairs drop into their buckets there.
+// A list that holds the reverse of each of its pairs and comes with its CSR (what the neighbour search of this library
+// delivers) needs neither: an atom sends as many pairs as it receives, and 470 000 atomic additions in the old labels, which lie
+// anywhere in space, are 23 of the 100 us that the eight launches take at 12 000 atoms (153 as seventeen).
+
+struct Box {
+  double lo[3], hi[3];
+};
+
+__device__ __forceinline__ void include(Box &box, const Box &other) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const double v = pos[3 * i + k];
-      mn[k] = v < mn[k] ? v : mn[k];
-      mx[k] = v > mx[k] ? v : mx[k];
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) lo[k][t] = mn[k], hi[k][t] = mx[k];
-  __syncthreads();
-  for (int d = kBoxThreads / 2; d > 0; d >>= 1) {
-    if (t < d) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        lo[k][t] = lo[k][t + d] < lo[k][t] ? lo[k][t + d] : lo[k][t];
-        hi[k][t] = hi[k][t + d] > hi[k][t] ? hi[k][t + d] : hi[k][t];
-      }
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    double extent = 0.0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      box[k] = n > 0 ? lo[k][0] : 0.0;
-      const double e = n > 0 ? hi[k][0] - lo[k][0] : 0.0;
-      extent = e > extent ? e : extent;
-    }
-    box[3] = extent;
+  for (int k = 0; k < 3; ++k) {
+    box.lo[k] = other.lo[k] < box.lo[k] ? other.lo[k] : box.lo[k];
+    box.hi[k] = other.hi[k] > box.hi[k] ? other.hi[k] : box.hi[k];
   }
 }
 
-// key = ((graph * bins + bx) * bins + by) * bins + bz
-__global__ void atom_key_kernel(const double *__restrict__ pos, const int32_t *__restrict__ graph_of_node, int64_t n,
-                                const double *__restrict__ box, double min_width, int bins, int ngraphs, int32_t *__restrict__ keys) {
-  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (i >= n) return;
-  double width = box[3] / bins * (1.0 + 1e-12);
+// The box of a wave's boxes, in every lane (smallest and largest values: the order does not matter; a NaN is never taken).
+__device__ __forceinline__ Box box_of_wave(Box box) {
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    Box other;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) other.lo[k] = __shfl_xor(box.lo[k], d), other.hi[k] = __shfl_xor(box.hi[k], d);
+    include(box, other);
+  }
+  return box;
+}
+
+__device__ __forceinline__ Box empty_box() { return Box{{DBL_MAX, DBL_MAX, DBL_MAX}, {-DBL_MAX, -DBL_MAX, -DBL_MAX}}; }
+
+// Workgroups [0, nboxes): the bounding box of a share of the positions each; the others clear `counters`.
+__global__ __launch_bounds__(kThreads) void box_and_clear_kernel(const double *__restrict__ pos, int64_t n, int nboxes, Box *__restrict__ boxes,
+                                                                 int32_t *__restrict__ counters, int64_t ncounters) {
+  __shared__ Box part[kWaves];
+  const int t = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) >= nboxes) {
+    const int64_t step = static_cast<int64_t>(gridDim.x - nboxes) * kThreads;
+    for (int64_t k = static_cast<int64_t>(blockIdx.x - nboxes) * kThreads + t; k < ncounters; k += step) counters[k] = 0;
+    return;
+  }
+  Box box = empty_box();
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + t; i < n; i += static_cast<int64_t>(nboxes) * kThreads) {
+    Box at;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) at.lo[k] = at.hi[k] = pos[3 * i + k];
+    include(box, at);
+  }
+  box = box_of_wave(box);
+  if (t % kWave == 0) part[t / kWave] = box;
+  __syncthreads();
+  if (t == 0) {
+    for (int w = 1; w < kWaves; ++w) include(box, part[w]);
+    boxes[blockIdx.x] = box;
+  }
+}
+
+// Workgroups [0, node_blocks), a thread per atom: key = ((graph * bins + bx) * bins + by) * bins + bz, and the atoms per key.
+// The others, a thread per pair: the old CSR (a change of the value of row_i closes every atom before it and opens every
+// atom up to it, values out of range counting as the nearest atom) and the pairs per atom j.
+__global__ __launch_bounds__(kThreads) void count_kernel(const double *__restrict__ pos, const int32_t *__restrict__ graph_of_node, int nnodes,
+                                                         int node_blocks, const Box *__restrict__ boxes, int nboxes, double min_width, int bins,
+                                                         int ngraphs, int32_t *__restrict__ keys, int32_t *__restrict__ atoms_of_key,
+                                                         const int32_t *__restrict__ row_i, const int32_t *__restrict__ row_j, int64_t nedges,
+                                                         int32_t *__restrict__ first_occ, int32_t *__restrict__ pairs_of_sender) {
+  __shared__ double s_box[4];
+  const int t = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) >= node_blocks) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x - node_blocks) * kThreads + t;
+    if (e >= nedges) return;
+    const auto clamped = [&](int i) { return i < 0 ? 0 : (i >= nnodes ? nnodes - 1 : i); };
+    const int cur = clamped(row_i[e]), prev = e > 0 ? clamped(row_i[e - 1]) : -1, j = row_j[e];
+    for (int i = prev + 1; i <= cur; ++i) first_occ[i] = static_cast<int32_t>(e);
+    for (int i = prev < 0 ? 0 : prev; i < cur; ++i) first_occ[nnodes + i] = static_cast<int32_t>(e);
+    if (e == nedges - 1) {
+      first_occ[nnodes + cur] = static_cast<int32_t>(nedges);
+      for (int i = cur + 1; i < nnodes; ++i) first_occ[i] = first_occ[nnodes + i] = static_cast<int32_t>(nedges);
+    }
+    if (static_cast<unsigned>(j) < static_cast<unsigned>(nnodes)) atomicAdd(&pairs_of_sender[j], 1);
+    return;
+  }
+  if (t < kWave) {
+    const Box box = box_of_wave(t < nboxes ? boxes[t] : empty_box());
+    if (t == 0) {
+      double extent = 0.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        s_box[k] = box.lo[k];
+        const double e = box.hi[k] - box.lo[k];
+        extent = e > extent ? e : extent;
+      }
+      s_box[3] = extent;
+    }
+  }
+  __syncthreads();
+  const int i = blockIdx.x * kThreads + t;
+  if (i >= nnodes) return;
+  double width = s_box[3] / bins * (1.0 + 1e-12);
   width = width > min_width ? width : min_width;
   int b[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const double f = floor((pos[3 * i + k] - box[k]) / width);
+    const double f = floor((pos[3 * static_cast<int64_t>(i) + k] - s_box[k]) / width);
     b[k] = f < 0.0 ? 0 : (f >= bins ? bins - 1 : static_cast<int>(f));  // NaN positions land in bin 0
   }
   int g = graph_of_node ? graph_of_node[i] : 0;
   g = g < 0 ? 0 : (g >= ngraphs ? ngraphs - 1 : g);
-  keys[i] = ((g * bins + b[0]) * bins + b[1]) * bins + b[2];
+  const int key = ((g * bins + b[0]) * bins + b[1]) * bins + b[2];
+  keys[i] = key;
+  atomicAdd(&atoms_of_key[key], 1);
 }
 
-// inverse[perm[a]] = a; degree of the new atom a = length of the segment of its old atom
-__global__ void relabel_nodes_kernel(const int32_t *__restrict__ perm, const int32_t *__restrict__ old_first_occ, int nnodes,
-                                     int64_t nedges, int32_t *__restrict__ inverse, int32_t *__restrict__ degree) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= nnodes) return;
-  const int o = perm[a];
+// One workgroup: offsets of the bins, and a copy of them that counts up while the bins are filled.
+__global__ __launch_bounds__(kScanThreads) void bin_offsets_kernel(const int32_t *__restrict__ atoms_of_key, int nkeys,
+                                                                   int32_t *__restrict__ offsets, int32_t *__restrict__ cursor) {
+  __shared__ int part[kScanThreads];
+  __shared__ int stage[kScanStage];
+  const int total = workgroup_exclusive_scan<kScanThreads, kScanStage, int>(
+      nkeys, stage, part, [&](int k) { return atoms_of_key[k]; },
+      [&](int k, int before, int) { offsets[k] = cursor[k] = before; });
+  if (threadIdx.x == 0) offsets[nkeys] = total;
+}
+
+__global__ void bin_atoms_kernel(const int32_t *__restrict__ keys, int nnodes, int32_t *__restrict__ cursor, int32_t *__restrict__ binned) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nnodes) binned[atomicAdd(&cursor[keys[i]], 1)] = i;
+}
+
+// The atoms of a bin in the order of their indices: perm and its inverse; under the new label, the length of the atom's
+// segment and the pairs it sends (pairs_of_sender NULL: as many as it receives).
+__global__ void relabel_nodes_kernel(const int32_t *__restrict__ keys, const int32_t *__restrict__ binned, const int32_t *__restrict__ offsets,
+                                     const int32_t *__restrict__ old_first_occ, const int32_t *__restrict__ pairs_of_sender, int nnodes,
+                                     int64_t nedges, int32_t *__restrict__ perm, int32_t *__restrict__ inverse, int32_t *__restrict__ degree,
+                                     int32_t *__restrict__ sent) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnodes) return;
+  const int o = binned[p], key = keys[o];
+  const int lo = offsets[key], hi = offsets[key + 1];
+  int rank = 0;
+  for (int q = lo; q < hi; ++q) rank += binned[q] < o ? 1 : 0;
+  const int a = lo + rank;
+  perm[a] = o;
   inverse[o] = a;
   int e0 = old_first_occ[o], e1 = old_first_occ[nnodes + o];
   clamp_edge_range(e0, e1, nedges);
   degree[a] = e1 - e0;
+  sent[a] = pairs_of_sender ? pairs_of_sender[o] : e1 - e0;
 }
 
-// One workgroup: first_occ[a] = exclusive scan of degree, first_occ[n + a] = inclusive scan (the CSR layout the
-// message-passing kernels take: starts, then ends).
-__global__ __launch_bounds__(kScanThreads) void degree_scan_kernel(const int32_t *__restrict__ degree, int n,
-                                                                   int32_t *__restrict__ first_occ) {
+// Two workgroups.  The first: first_occ[a] = exclusive scan of degree, first_occ[n + a] = inclusive scan (the CSR layout the
+// message-passing kernels take: starts, then ends).  The second: the offsets of the view by sender, and a copy to fill by.
+__global__ __launch_bounds__(kScanThreads) void edge_offsets_kernel(const int32_t *__restrict__ degree, const int32_t *__restrict__ sent, int n,
+                                                                    int32_t *__restrict__ first_occ, int32_t *__restrict__ sender_offsets,
+                                                                    int32_t *__restrict__ cursor) {
   __shared__ int part[kScanThreads];
   __shared__ int stage[kScanStage];
-  workgroup_exclusive_scan<kScanThreads, kScanStage, int>(
-      n, stage, part, [&](int k) { return degree[k]; },
+  const bool by_sender = blockIdx.x == 1;
+  const int32_t *__restrict__ counts = by_sender ? sent : degree;
+  const int total = workgroup_exclusive_scan<kScanThreads, kScanStage, int>(
+      n, stage, part, [&](int k) { return counts[k]; },
       [&](int k, int before, int value) {
-        first_occ[k] = before;
-        first_occ[n + k] = before + value;
+        if (by_sender) {
+          sender_offsets[k] = cursor[k] = before;
+        } else {
+          first_occ[k] = before;
+          first_occ[n + k] = before + value;
+        }
       });
+  if (by_sender && threadIdx.x == 0) sender_offsets[n] = total;
 }
 
-// Sort key of an edge inside its segment: pairs within the cutoff by the new label of atom j, the others behind them
-// by length (the bit pattern of a non-negative double orders like its value).
-__global__ void edge_key_kernel(const double *__restrict__ pos, const int32_t *__restrict__ row_i, const int32_t *__restrict__ row_j,
-                                const double *__restrict__ shifts, const int32_t *__restrict__ inverse, int64_t nedges, int nnodes,
-                                double r_max, unsigned long long *__restrict__ key) {
-  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (e >= nedges) return;
-  const int i = row_i[e], j = row_j[e];
-  unsigned long long k = 0x7fffffffull;  // a pair that names no atom: behind the pairs within the cutoff
-  if (static_cast<unsigned>(i) < static_cast<unsigned>(nnodes) && static_cast<unsigned>(j) < static_cast<unsigned>(nnodes)) {
-    double v[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) v[c] = (pos[3 * static_cast<int64_t>(j) + c] - pos[3 * static_cast<int64_t>(i) + c]) + shifts[3 * e + c];
-    const double len = sqrt((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]);
-    k = len > r_max ? (1ull << 63) | static_cast<unsigned long long>(__double_as_longlong(len))
-                    : static_cast<unsigned long long>(static_cast<unsigned>(inverse[j]));
-  }
-  key[e] = k;
-}
-
-// One wave per new atom: ranks the pairs of its segment by (key, position in the list) and writes them to their places.
-__global__ __launch_bounds__(kWave) void place_edges_kernel(const int32_t *__restrict__ perm, const int32_t *__restrict__ inverse,
-                                                            const int32_t *__restrict__ old_first_occ,
-                                                            const int32_t *__restrict__ new_first_occ,
-                                                            const int32_t *__restrict__ row_j, const double *__restrict__ shifts,
-                                                            const unsigned long long *__restrict__ key, int nnodes, int64_t nedges,
+// One wave per new atom: keys of the pairs of its segment (pairs within the cutoff by the new label of atom j, the others
+// behind them by length: the bit pattern of a non-negative double orders like its value), their ranks by (key, position in
+// the list), the pairs at their places, and each into its sender's bucket in any order.  Keys of more pairs than LDS holds
+// go through `key`.  Of a list that is not sorted by row i, pairs may stay without a place: none is written out of range.
+__global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__restrict__ pos, const int32_t *__restrict__ perm,
+                                                            const int32_t *__restrict__ inverse, const int32_t *__restrict__ old_first_occ,
+                                                            const int32_t *__restrict__ new_first_occ, const int32_t *__restrict__ row_i,
+                                                            const int32_t *__restrict__ row_j, const double *__restrict__ shifts, double r_max,
+                                                            unsigned long long *__restrict__ key, int nnodes, int64_t nedges,
                                                             int32_t *__restrict__ receiver, int32_t *__restrict__ sender,
-                                                            int32_t *__restrict__ edge_perm, double *__restrict__ shifts_out) {
+                                                            int32_t *__restrict__ edge_perm, double *__restrict__ shifts_out,
+                                                            const int32_t *__restrict__ sender_offsets, int32_t *__restrict__ cursor,
+                                                            int32_t *__restrict__ bucketed) {
   __shared__ unsigned long long sk[kSegLds];
   const int a = blockIdx.x, lane = threadIdx.x;
   const int o = perm[a];
@@ -147,36 +227,130 @@ __global__ __launch_bounds__(kWave) void place_edges_kernel(const int32_t *__res
   const int d = s1 - s0;
   const int base = new_first_occ[a];
   const bool in_lds = d <= kSegLds;
-  if (in_lds) {
-    for (int t = lane; t < d; t += kWave) sk[t] = key[s0 + t];
-    __syncthreads();
-  }
-  for (int k = lane; k < d; k += kWave) {
-    const unsigned long long mine = in_lds ? sk[k] : key[s0 + k];
-    int rank = 0;
-    for (int t = 0; t < d; ++t) {
-      const unsigned long long other = in_lds ? sk[t] : key[s0 + t];
-      rank += (other < mine || (other == mine && t < k)) ? 1 : 0;
+  for (int t = lane; t < d; t += kWave) {
+    const int64_t e = s0 + t;
+    const int i = row_i[e], j = row_j[e];
+    unsigned long long k = 0x7fffffffull;  // a pair that names no atom: behind the pairs within the cutoff
+    if (static_cast<unsigned>(i) < static_cast<unsigned>(nnodes) && static_cast<unsigned>(j) < static_cast<unsigned>(nnodes)) {
+      double v[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c] = (pos[3 * static_cast<int64_t>(j) + c] - pos[3 * static_cast<int64_t>(i) + c]) + shifts[3 * e + c];
+      const double len = sqrt((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]);
+      k = len > r_max ? (1ull << 63) | static_cast<unsigned long long>(__double_as_longlong(len))
+                      : static_cast<unsigned long long>(static_cast<unsigned>(inverse[j]));
     }
-    const int64_t e = s0 + k, at = base + rank;
+    if (in_lds)
+      sk[t] = k;
+    else
+      key[e] = k;
+  }
+  __syncthreads();
+  for (int k = lane; k < d; k += kWave) {
+    const int64_t e = s0 + k;
+    const unsigned long long mine = in_lds ? sk[k] : key[e];
     const int j = row_j[e];
+    const double s[3] = {shifts[3 * e + 0], shifts[3 * e + 1], shifts[3 * e + 2]};
+    int rank = 0;
+    if (in_lds) {
+#pragma unroll 4
+      for (int t = 0; t < d; ++t) rank += (sk[t] < mine || (sk[t] == mine && t < k)) ? 1 : 0;
+    } else {
+      for (int t = 0; t < d; ++t) {
+        const unsigned long long other = key[s0 + t];
+        rank += (other < mine || (other == mine && t < k)) ? 1 : 0;
+      }
+    }
+    const int64_t at = static_cast<int64_t>(base) + rank;
+    if (at >= nedges) continue;
+    const bool named = static_cast<unsigned>(j) < static_cast<unsigned>(nnodes);
+    const int s_new = named ? inverse[j] : j;
     receiver[at] = a;
-    sender[at] = static_cast<unsigned>(j) < static_cast<unsigned>(nnodes) ? inverse[j] : j;
+    sender[at] = s_new;
     edge_perm[at] = static_cast<int32_t>(e);
-    shifts_out[3 * at + 0] = shifts[3 * e + 0];
-    shifts_out[3 * at + 1] = shifts[3 * e + 1];
-    shifts_out[3 * at + 2] = shifts[3 * e + 2];
+    shifts_out[3 * at + 0] = s[0];
+    shifts_out[3 * at + 1] = s[1];
+    shifts_out[3 * at + 2] = s[2];
+    if (named) {
+      const int to = atomicAdd(&cursor[s_new], 1);
+      if (to < sender_offsets[s_new + 1]) bucketed[to] = static_cast<int32_t>(at);
+    }
+  }
+}
+
+// One wave per sender: its pairs in the order of the new list.  Slots that no pair took (a list that is not sorted by row
+// i) name pair 0.
+__global__ __launch_bounds__(kThreads) void rank_senders_kernel(const int32_t *__restrict__ sender_offsets, const int32_t *__restrict__ cursor,
+                                                                const int32_t *__restrict__ bucketed, int nnodes, int32_t *__restrict__ perm) {
+  __shared__ int stage[kWaves][kBucketLds];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int a = blockIdx.x * kWaves + w;
+  const int lo = a < nnodes ? sender_offsets[a] : 0, end = a < nnodes ? sender_offsets[a + 1] : 0;
+  const int hi = a < nnodes ? min(cursor[a], end) : 0;
+  const bool in_lds = hi - lo <= kBucketLds;
+  if (in_lds)
+    for (int p = lo + lane; p < hi; p += kWave) stage[w][p - lo] = bucketed[p];
+  __syncthreads();
+  for (int p = lo + lane; p < hi; p += kWave) {
+    const int mine = bucketed[p];
+    int rank = 0;
+    if (in_lds) {
+#pragma unroll 4
+      for (int q = 0; q < hi - lo; ++q) rank += stage[w][q] < mine ? 1 : 0;
+    } else {
+      for (int q = lo; q < hi; ++q) rank += bucketed[q] < mine ? 1 : 0;
+    }
+    perm[lo + rank] = mine;
+  }
+  for (int p = hi + lane; p < end; p += kWave) perm[p] = 0;
+}
+
+// Rows `perm` of several arrays in one launch.  A workgroup copies a few rows of one array, in the widest units that the
+// length of its rows and both addresses allow.
+constexpr int kMaxRowArrays = 8;
+
+struct RowArrays {
+  const char *src[kMaxRowArrays];
+  char *dst[kMaxRowArrays];
+  int units[kMaxRowArrays], width[kMaxRowArrays], rows[kMaxRowArrays];  // units per row, bytes per unit, rows per workgroup
+  unsigned first[kMaxRowArrays + 1];                                    // first workgroup
+  int count;
+};
+
+template <typename Unit>
+__device__ __forceinline__ void copy_rows(const char *src, char *dst, const int32_t *__restrict__ perm, int units, int64_t r0, int rows, int64_t n) {
+  const Unit *from = reinterpret_cast<const Unit *>(src);
+  Unit *to = reinterpret_cast<Unit *>(dst);
+  const unsigned total = static_cast<unsigned>(rows) * static_cast<unsigned>(units);
+  for (unsigned k = threadIdx.x; k < total; k += kThreads) {
+    const unsigned r = k / static_cast<unsigned>(units);
+    const int o = perm[r0 + r];
+    if (static_cast<uint64_t>(static_cast<int64_t>(o)) < static_cast<uint64_t>(n))
+      to[r0 * units + k] = from[static_cast<int64_t>(o) * units + (k - r * units)];
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void gather_rows_kernel(RowArrays a, const int32_t *__restrict__ perm, int64_t n) {
+  int k = 0;
+  while (k + 1 < a.count && blockIdx.x >= a.first[k + 1]) ++k;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x - a.first[k]) * a.rows[k];
+  const int rows = static_cast<int>(n - r0 < a.rows[k] ? n - r0 : a.rows[k]);
+  switch (a.width[k]) {
+    case 16: return copy_rows<int4>(a.src[k], a.dst[k], perm, a.units[k], r0, rows, n);
+    case 8: return copy_rows<int2>(a.src[k], a.dst[k], perm, a.units[k], r0, rows, n);
+    case 4: return copy_rows<int>(a.src[k], a.dst[k], perm, a.units[k], r0, rows, n);
+    default: return copy_rows<char>(a.src[k], a.dst[k], perm, a.units[k], r0, rows, n);
   }
 }
 
 inline size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
 struct PrepareLayout {
-  double *box;
-  int32_t *atom_keys, *bin_offsets, *old_first_occ, *degree;
+  Box *boxes;
+  int32_t *counters, *atoms_of_key, *old_first_occ, *pairs_of_sender;  // the last three are cleared together
+  int64_t ncounters;
+  int32_t *atom_keys, *bin_offsets, *bin_cursor, *binned, *degree, *sent, *sender_cursor, *bucketed;
   unsigned long long *edge_key;
-  void *sort_ws;
-  size_t sort_bytes, bytes;
+  size_t bytes;
   PrepareLayout(void *base, int64_t N, int64_t E, int64_t nkeys) {
     size_t at = 0;
     auto take = [&](size_t n) {
@@ -184,15 +358,22 @@ struct PrepareLayout {
       at += align256(n);
       return p;
     };
-    box = reinterpret_cast<double *>(take(4 * sizeof(double)));
-    atom_keys = reinterpret_cast<int32_t *>(take(static_cast<size_t>(N) * 4));
-    bin_offsets = reinterpret_cast<int32_t *>(take(static_cast<size_t>(nkeys + 1) * 4));
-    old_first_occ = reinterpret_cast<int32_t *>(take(static_cast<size_t>(2 * N) * 4));
-    degree = reinterpret_cast<int32_t *>(take(static_cast<size_t>(N) * 4));
+    auto ints = [&](int64_t n) { return reinterpret_cast<int32_t *>(take(static_cast<size_t>(n) * 4)); };
+    boxes = reinterpret_cast<Box *>(take(kMaxBoxes * sizeof(Box)));
+    ncounters = nkeys + 3 * N;
+    counters = ints(ncounters);
+    atoms_of_key = counters;
+    old_first_occ = counters + nkeys;
+    pairs_of_sender = old_first_occ + 2 * N;
+    atom_keys = ints(N);
+    bin_offsets = ints(nkeys + 1);
+    bin_cursor = ints(nkeys);
+    binned = ints(N);
+    degree = ints(N);
+    sent = ints(N);
+    sender_cursor = ints(N);
+    bucketed = ints(E);
     edge_key = reinterpret_cast<unsigned long long *>(take(static_cast<size_t>(E) * 8));
-    const size_t a = cm_stable_key_sort_workspace(N, nkeys), b = cm_stable_key_sort_workspace(E, N);
-    sort_bytes = a > b ? a : b;
-    sort_ws = take(sort_bytes);
     bytes = at;
   }
 };
@@ -205,51 +386,106 @@ extern "C" size_t cm_graph_prepare_workspace(int64_t nnodes, int64_t nedges, int
   return cm::PrepareLayout(nullptr, nnodes, nedges, static_cast<int64_t>(ngraphs) * bins * bins * bins).bytes;
 }
 
+namespace cm {
+namespace {
+
+int prepare(const double *positions, const int32_t *row_i, const int32_t *row_j, const double *shifts,
+                                const int32_t *known_first_occ, const int32_t *graph_of_node, int64_t nnodes, int64_t nedges, int ngraphs, double r_max, int bins,
+                                int32_t *node_perm, int32_t *node_inverse, int32_t *receiver, int32_t *sender, int32_t *edge_perm,
+                                double *shifts_out, int32_t *first_occ, int32_t *sender_perm, int32_t *sender_offsets,
+                                void *workspace, size_t workspace_bytes, cm_stream_t stream, const char *what) {
+  CM_REQUIRE(nnodes >= 0 && nedges >= 0 && nnodes < INT32_MAX / 4 && nedges < INT32_MAX / 3, "%s: sizes out of range", what);
+  CM_REQUIRE(ngraphs >= 1 && bins >= 1 && bins <= 64, "%s: need at least one graph and 1 to 64 bins per axis", what);
+  const int64_t nkeys = static_cast<int64_t>(ngraphs) * bins * bins * bins;
+  CM_REQUIRE(nkeys < (int64_t{1} << 24), "%s: ngraphs * bins^3 = %lld keys, at most 2^24 - 1", what, static_cast<long long>(nkeys));
+  CM_REQUIRE(r_max > 0.0, "%s: r_max must be positive", what);
+  CM_REQUIRE(sender_offsets && (nnodes == 0 || first_occ), "%s: NULL output", what);
+  CM_REQUIRE(nnodes == 0 || (positions && node_perm && node_inverse), "%s: NULL node operand", what);
+  CM_REQUIRE(nedges == 0 || (row_i && row_j && shifts && receiver && sender && edge_perm && shifts_out && sender_perm),
+             "%s: NULL edge operand", what);
+  const PrepareLayout L(workspace, nnodes, nedges, nkeys);
+  if (workspace == nullptr || workspace_bytes < L.bytes) {
+    set_error("%s: workspace of %zu bytes, need %zu", what, workspace_bytes, L.bytes);
+    return CM_ENOSPC;
+  }
+  CM_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "%s: workspace must be 256-byte aligned", what);
+  CM_REQUIRE(nnodes > 0 || nedges == 0, "%s: pairs without atoms", what);
+  hipStream_t st = as_stream(stream);
+  const int N = static_cast<int>(nnodes);
+  const int32_t *old_first_occ = known_first_occ ? known_first_occ : L.old_first_occ;
+  const dim3 block(kThreads);
+  const unsigned gn = static_cast<unsigned>(ceil_div(nnodes, kThreads)), ge = static_cast<unsigned>(ceil_div(nedges, kThreads));
+  if (nnodes > 0) {
+    // atoms by bin; old CSR and pairs per sender
+    const int64_t ncounters = known_first_occ ? nkeys : L.ncounters;
+    const int nboxes = static_cast<int>(std::min<int64_t>(ceil_div(nnodes, 4 * kThreads), kMaxBoxes));
+    const unsigned clears = static_cast<unsigned>(std::min<int64_t>(ceil_div(ncounters, 4 * kThreads), 1024));
+    hipLaunchKernelGGL(box_and_clear_kernel, dim3(nboxes + clears), block, 0, st, positions, nnodes, nboxes, L.boxes, L.counters, ncounters);
+    hipLaunchKernelGGL(count_kernel, dim3(gn + (known_first_occ ? 0 : ge)), block, 0, st, positions, graph_of_node, N, static_cast<int>(gn), L.boxes, nboxes,
+                       0.5 * r_max, bins, ngraphs, L.atom_keys, L.atoms_of_key, row_i, row_j, nedges, L.old_first_occ, L.pairs_of_sender);
+    hipLaunchKernelGGL(bin_offsets_kernel, dim3(1), dim3(kScanThreads), 0, st, L.atoms_of_key, static_cast<int>(nkeys), L.bin_offsets,
+                       L.bin_cursor);
+    hipLaunchKernelGGL(bin_atoms_kernel, dim3(gn), block, 0, st, L.atom_keys, N, L.bin_cursor, L.binned);
+    hipLaunchKernelGGL(relabel_nodes_kernel, dim3(gn), block, 0, st, L.atom_keys, L.binned, L.bin_offsets, old_first_occ,
+                       known_first_occ ? static_cast<const int32_t *>(nullptr) : L.pairs_of_sender, N, nedges, node_perm, node_inverse, L.degree, L.sent);
+  }
+  hipLaunchKernelGGL(edge_offsets_kernel, dim3(2), dim3(kScanThreads), 0, st, L.degree, L.sent, N, first_occ, sender_offsets,
+                     L.sender_cursor);
+  if (nedges > 0) {
+    hipLaunchKernelGGL(place_edges_kernel, dim3(static_cast<unsigned>(nnodes)), dim3(kWave), 0, st, positions, node_perm, node_inverse,
+                       old_first_occ, first_occ, row_i, row_j, shifts, r_max, L.edge_key, N, nedges, receiver, sender, edge_perm, shifts_out,
+                       sender_offsets, L.sender_cursor, L.bucketed);
+    hipLaunchKernelGGL(rank_senders_kernel, dim3(static_cast<unsigned>(ceil_div(nnodes, kWaves))), block, 0, st, sender_offsets,
+                       L.sender_cursor, L.bucketed, N, sender_perm);
+  }
+  return check_launch(what);
+}
+
+}  // namespace
+}  // namespace cm
+
 extern "C" int cm_graph_prepare(const double *positions, const int32_t *row_i, const int32_t *row_j, const double *shifts,
                                 const int32_t *graph_of_node, int64_t nnodes, int64_t nedges, int ngraphs, double r_max, int bins,
                                 int32_t *node_perm, int32_t *node_inverse, int32_t *receiver, int32_t *sender, int32_t *edge_perm,
                                 double *shifts_out, int32_t *first_occ, int32_t *sender_perm, int32_t *sender_offsets,
                                 void *workspace, size_t workspace_bytes, cm_stream_t stream) {
-  CM_REQUIRE(nnodes >= 0 && nedges >= 0 && nnodes < INT32_MAX / 4 && nedges < INT32_MAX / 3, "cm_graph_prepare: sizes out of range");
-  CM_REQUIRE(ngraphs >= 1 && bins >= 1 && bins <= 64, "cm_graph_prepare: need at least one graph and 1 to 64 bins per axis");
-  const int64_t nkeys = static_cast<int64_t>(ngraphs) * bins * bins * bins;
-  CM_REQUIRE(nkeys < (int64_t{1} << 24), "cm_graph_prepare: ngraphs * bins^3 = %lld keys, at most 2^24 - 1", static_cast<long long>(nkeys));
-  CM_REQUIRE(r_max > 0.0, "cm_graph_prepare: r_max must be positive");
-  CM_REQUIRE(sender_offsets && (nnodes == 0 || first_occ), "cm_graph_prepare: NULL output");
-  CM_REQUIRE(nnodes == 0 || (positions && node_perm && node_inverse), "cm_graph_prepare: NULL node operand");
-  CM_REQUIRE(nedges == 0 || (row_i && row_j && shifts && receiver && sender && edge_perm && shifts_out && sender_perm),
-             "cm_graph_prepare: NULL edge operand");
-  const cm::PrepareLayout L(workspace, nnodes, nedges, nkeys);
-  if (workspace == nullptr || workspace_bytes < L.bytes) {
-    cm::set_error("cm_graph_prepare: workspace of %zu bytes, need %zu", workspace_bytes, L.bytes);
-    return CM_ENOSPC;
+  return cm::prepare(positions, row_i, row_j, shifts, nullptr, graph_of_node, nnodes, nedges, ngraphs, r_max, bins, node_perm, node_inverse, receiver, sender,
+                     edge_perm, shifts_out, first_occ, sender_perm, sender_offsets, workspace, workspace_bytes, stream, "cm_graph_prepare");
+}
+
+extern "C" int cm_graph_prepare_symmetric(const double *positions, const int32_t *row_i, const int32_t *row_j, const double *shifts,
+                                const int32_t *old_first_occ, const int32_t *graph_of_node, int64_t nnodes, int64_t nedges, int ngraphs, double r_max, int bins,
+                                int32_t *node_perm, int32_t *node_inverse, int32_t *receiver, int32_t *sender, int32_t *edge_perm,
+                                double *shifts_out, int32_t *first_occ, int32_t *sender_perm, int32_t *sender_offsets,
+                                void *workspace, size_t workspace_bytes, cm_stream_t stream) {
+  CM_REQUIRE(nnodes == 0 || old_first_occ != nullptr, "cm_graph_prepare_symmetric: old_first_occ is NULL");
+  return cm::prepare(positions, row_i, row_j, shifts, old_first_occ, graph_of_node, nnodes, nedges, ngraphs, r_max, bins, node_perm, node_inverse, receiver, sender,
+                     edge_perm, shifts_out, first_occ, sender_perm, sender_offsets, workspace, workspace_bytes, stream, "cm_graph_prepare_symmetric");
+}
+
+extern "C" int cm_gather_rows(const int32_t *perm, int64_t nrows, int narrays, const void *const *src, void *const *dst, const int64_t *row_bytes,
+                              cm_stream_t stream) {
+  static const char *what = "cm_gather_rows";
+  CM_REQUIRE(nrows >= 0 && nrows < INT32_MAX, "%s: nrows out of range", what);
+  CM_REQUIRE(narrays >= 0 && narrays <= cm::kMaxRowArrays, "%s: %d arrays, at most %d", what, narrays, cm::kMaxRowArrays);
+  CM_REQUIRE(narrays == 0 || (src && dst && row_bytes), "%s: NULL pointer", what);
+  CM_REQUIRE(nrows == 0 || narrays == 0 || perm, "%s: perm is NULL", what);
+  cm::RowArrays a{};
+  uint64_t blocks = 0;
+  for (int k = 0; k < narrays; ++k) {
+    CM_REQUIRE(row_bytes[k] >= 0 && row_bytes[k] <= (1 << 20), "%s: rows of 0 to 2^20 bytes", what);
+    if (row_bytes[k] == 0 || nrows == 0) continue;
+    CM_REQUIRE(src[k] && dst[k], "%s: NULL array", what);
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(src[k]) | reinterpret_cast<uintptr_t>(dst[k]) | static_cast<uintptr_t>(row_bytes[k]);
+    const int at = a.count++, width = bits % 16 == 0 ? 16 : bits % 8 == 0 ? 8 : bits % 4 == 0 ? 4 : 1;
+    a.src[at] = static_cast<const char *>(src[k]), a.dst[at] = static_cast<char *>(dst[k]);
+    a.width[at] = width, a.units[at] = static_cast<int>(row_bytes[k] / width);
+    a.rows[at] = std::max(1, 4 * cm::kThreads / a.units[at]);
+    a.first[at] = static_cast<unsigned>(blocks);
+    blocks += static_cast<uint64_t>(cm::ceil_div(nrows, a.rows[at]));
   }
-  CM_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "cm_graph_prepare: workspace must be 256-byte aligned");
-  hipStream_t st = cm::as_stream(stream);
-  const int N = static_cast<int>(nnodes);
-  const unsigned gn = static_cast<unsigned>(cm::ceil_div(nnodes > 0 ? nnodes : 1, 256));
-  const unsigned ge = static_cast<unsigned>(cm::ceil_div(nedges > 0 ? nedges : 1, 256));
-  int rc;
-  // atoms: bounding box -> grid keys -> stable counting sort
-  hipLaunchKernelGGL(cm::bounding_box_kernel, dim3(1), dim3(cm::kBoxThreads), 0, st, positions, nnodes, L.box);
-  if (nnodes > 0)
-    hipLaunchKernelGGL(cm::atom_key_kernel, dim3(gn), dim3(256), 0, st, positions, graph_of_node, nnodes, L.box, 0.5 * r_max, bins,
-                       ngraphs, L.atom_keys);
-  if ((rc = cm::check_launch("cm_graph_prepare")) != CM_OK) return rc;
-  if ((rc = cm_stable_key_sort(L.atom_keys, nnodes, nkeys, node_perm, L.bin_offsets, L.sort_ws, L.sort_bytes, stream)) != CM_OK) return rc;
-  // old CSR, inverse, degrees in the new order, new CSR
-  if ((rc = cm_first_occurences(row_i, nedges, nnodes, L.old_first_occ, stream)) != CM_OK) return rc;
-  if (nnodes > 0)
-    hipLaunchKernelGGL(cm::relabel_nodes_kernel, dim3(gn), dim3(256), 0, st, node_perm, L.old_first_occ, N, nedges, node_inverse, L.degree);
-  hipLaunchKernelGGL(cm::degree_scan_kernel, dim3(1), dim3(cm::kScanThreads), 0, st, L.degree, N, first_occ);
-  // edges: key inside the segment, then every segment ranked and written by one wave
-  if (nedges > 0) {
-    hipLaunchKernelGGL(cm::edge_key_kernel, dim3(ge), dim3(256), 0, st, positions, row_i, row_j, shifts, node_inverse, nedges, N, r_max,
-                       L.edge_key);
-    hipLaunchKernelGGL(cm::place_edges_kernel, dim3(static_cast<unsigned>(nnodes)), dim3(cm::kWave), 0, st, node_perm, node_inverse,
-                       L.old_first_occ, first_occ, row_j, shifts, L.edge_key, N, nedges, receiver, sender, edge_perm, shifts_out);
-  }
-  if ((rc = cm::check_launch("cm_graph_prepare")) != CM_OK) return rc;
-  // the new list sorted by row j
-  return cm_stable_key_sort(sender, nedges, nnodes, sender_perm, sender_offsets, L.sort_ws, L.sort_bytes, stream);
+  CM_REQUIRE(blocks < (1ull << 31), "%s: too many rows", what);
+  if (blocks == 0) return CM_OK;
+  hipLaunchKernelGGL(cm::gather_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(cm::kThreads), 0, cm::as_stream(stream), a, perm, nrows);
+  return cm::check_launch(what);
 }

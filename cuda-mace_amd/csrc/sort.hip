@@ -116,6 +116,84 @@ __global__ __launch_bounds__(kFewBlock) void block_place_kernel(const int32_t *_
   if (blockIdx.x == 0 && t <= nkeys) offsets[t] = base[static_cast<int64_t>(t) * nblocks];
 }
 
+// ---- the nodes by element, by two definitions at once -----------------------------------------------------------------
+// The model groups its nodes by element index and by the column of the one-hot matrix that holds a one (rows without one come
+// last), which are two sorts of the few-keys kind over keys that a compare, two reductions and a select over [n, nelements]
+// make.  As torch operations and two sorts they were 20 launches of 3 to 7 us each at 12 000 nodes, behind a host that takes
+// 8 us for each; here three.  Table 0 counts the element indices (nelements keys), table 1 the columns (one key more).
+struct ElementTables {
+  int nelements, nblocks;
+  __host__ __device__ int keys(int table) const { return nelements + table; }
+  __host__ __device__ int64_t entries(int table) const { return static_cast<int64_t>(keys(table)) * nblocks; }
+};
+
+__global__ __launch_bounds__(kFewBlock) void element_histogram_kernel(const int32_t *__restrict__ types, const float *__restrict__ one_hot, int64_t n,
+                                                                      ElementTables tables, int32_t *__restrict__ column,
+                                                                      int32_t *__restrict__ counts) {
+  __shared__ int hist[2][kFewKeys];
+  const int t = threadIdx.x, ne = tables.nelements;
+  if (t < 2 * kFewKeys) hist[t / kFewKeys][t % kFewKeys] = 0;
+  __syncthreads();
+  const int64_t i = blockIdx.x * static_cast<int64_t>(kFewBlock) + t;
+  if (i < n) {
+    const int type = types[i];
+    const float *__restrict__ row = one_hot + i * ne;
+    int c = ne;
+    for (int k = ne - 1; k >= 0; --k) c = row[k] == 1.0f ? k : c;
+    column[i] = c;
+    if (static_cast<unsigned>(type) < static_cast<unsigned>(ne)) atomicAdd(&hist[0][type], 1);
+    atomicAdd(&hist[1][c], 1);
+  }
+  __syncthreads();
+  for (int table = 0; table < 2; ++table)
+    if (t < tables.keys(table)) counts[table * tables.entries(0) + static_cast<int64_t>(t) * tables.nblocks + blockIdx.x] = hist[table][t];
+}
+
+// A workgroup per table; base: entries + 1 values per table.
+__global__ __launch_bounds__(kScanThreads) void element_scan_kernel(ElementTables tables, const int32_t *__restrict__ counts,
+                                                                    int32_t *__restrict__ base) {
+  __shared__ int part[kScanThreads];
+  __shared__ int stage[kScanStage];
+  const int table = blockIdx.x, entries = static_cast<int>(tables.entries(table));
+  counts += table * tables.entries(0);
+  base += table * (tables.entries(0) + 1);
+  const int total = workgroup_exclusive_scan<kScanThreads, kScanStage, int>(
+      entries, stage, part, [&](int k) { return counts[k]; }, [&](int k, int before, int) { base[k] = before; });
+  if (threadIdx.x == 0) base[entries] = total;
+}
+
+struct ElementGroups {
+  int32_t *perm[2], *offsets[2];
+};
+
+__global__ __launch_bounds__(kFewBlock) void element_place_kernel(const int32_t *__restrict__ types, const int32_t *__restrict__ column, int64_t n,
+                                                                  ElementTables tables, const int32_t *__restrict__ base, ElementGroups out) {
+  __shared__ int skey[2][kFewBlock];
+  const int t = threadIdx.x;
+  const int64_t i = blockIdx.x * static_cast<int64_t>(kFewBlock) + t;
+  int key[2] = {-1, -1};
+  if (i < n) {
+    key[0] = types[i], key[1] = column[i];
+    if (static_cast<unsigned>(key[0]) >= static_cast<unsigned>(tables.nelements)) key[0] = -1;
+  }
+  skey[0][t] = key[0], skey[1][t] = key[1];
+  __syncthreads();
+  int rank[2] = {0, 0};
+#pragma unroll 4
+  for (int j = 0; j < t; ++j) rank[0] += skey[0][j] == key[0] ? 1 : 0, rank[1] += skey[1][j] == key[1] ? 1 : 0;
+  for (int table = 0; table < 2; ++table) {
+    const int32_t *at = base + table * (tables.entries(0) + 1);
+    if (key[table] >= 0) out.perm[table][at[static_cast<int64_t>(key[table]) * tables.nblocks + blockIdx.x] + rank[table]] = static_cast<int32_t>(i);
+    if (blockIdx.x == 0 && t <= tables.keys(table)) out.offsets[table][t] = at[static_cast<int64_t>(t) * tables.nblocks];
+  }
+}
+
+// column, counts, base
+inline size_t element_groups_ints(int64_t n, int nelements) {
+  const ElementTables tables{nelements, static_cast<int>(ceil_div(n, kFewBlock))};
+  return static_cast<size_t>(n + 2 * (tables.entries(0) + tables.entries(1)) + 2);
+}
+
 }  // namespace
 }  // namespace cm
 
@@ -187,6 +265,36 @@ extern "C" int cm_stable_key_sort(const int32_t *keys, int64_t n, int64_t nkeys,
     return CM_ENOSPC;
   }
   return cm::sort_enqueue(keys, n, nkeys, perm, offsets, workspace, cm::as_stream(stream), "cm_stable_key_sort");
+}
+
+extern "C" int cm_element_groups_max_elements(void) { return cm::kFewKeys - 1; }
+
+extern "C" size_t cm_element_groups_workspace(int64_t nnodes, int nelements) {
+  if (nnodes < 0 || nnodes >= INT32_MAX / 4 || nelements < 1 || nelements >= cm::kFewKeys) return 0;
+  return (cm::element_groups_ints(nnodes, nelements) * sizeof(int32_t) + 255) & ~static_cast<size_t>(255);
+}
+
+extern "C" int cm_element_groups(const int32_t *types, const float *one_hot, int64_t nnodes, int nelements, int32_t *type_perm,
+                                 int32_t *type_offsets, int32_t *column_perm, int32_t *column_offsets, void *workspace,
+                                 size_t workspace_bytes, cm_stream_t stream) {
+  static const char *what = "cm_element_groups";
+  CM_REQUIRE(nnodes >= 0 && nnodes < INT32_MAX / 4, "%s: nnodes out of range", what);
+  CM_REQUIRE(nelements >= 1 && nelements < cm::kFewKeys, "%s: %d elements, 1 to %d", what, nelements, cm::kFewKeys - 1);
+  CM_REQUIRE(type_offsets && column_offsets && (nnodes == 0 || (types && one_hot && type_perm && column_perm)), "%s: NULL pointer", what);
+  if (workspace == nullptr || workspace_bytes < cm_element_groups_workspace(nnodes, nelements)) {
+    cm::set_error("%s: workspace of %zu bytes, need %zu", what, workspace_bytes, cm_element_groups_workspace(nnodes, nelements));
+    return CM_ENOSPC;
+  }
+  hipStream_t st = cm::as_stream(stream);
+  const cm::ElementTables tables{nelements, static_cast<int>(cm::ceil_div(nnodes, cm::kFewBlock))};
+  int32_t *column = static_cast<int32_t *>(workspace), *counts = column + nnodes, *base = counts + tables.entries(0) + tables.entries(1);
+  const dim3 grid(static_cast<unsigned>(std::max(tables.nblocks, 1))), block(cm::kFewBlock);
+  if (nnodes > 0)
+    hipLaunchKernelGGL(cm::element_histogram_kernel, grid, block, 0, st, types, one_hot, nnodes, tables, column, counts);
+  hipLaunchKernelGGL(cm::element_scan_kernel, dim3(2), dim3(cm::kScanThreads), 0, st, tables, counts, base);
+  hipLaunchKernelGGL(cm::element_place_kernel, grid, block, 0, st, types, column, nnodes, tables, base,
+                     cm::ElementGroups{{type_perm, column_perm}, {type_offsets, column_offsets}});
+  return cm::check_launch(what);
 }
 
 // ---- the same sort without a caller's workspace ---------------------------------------------------------------

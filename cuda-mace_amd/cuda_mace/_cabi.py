@@ -69,6 +69,11 @@ SIGNATURES = {
     "cm_readout_backward": (_i32, [_p, _p, _p, _f64, _i64, _i32, _p, _p, _p]),
     "cm_graph_prepare_workspace": (_sz, [_i64, _i64, _i32, _i32]),
     "cm_graph_prepare": (_i32, [_p] * 5 + [_i64, _i64, _i32, _f64, _i32] + [_p] * 10 + [_sz, _p]),
+    "cm_graph_prepare_symmetric": (_i32, [_p] * 6 + [_i64, _i64, _i32, _f64, _i32] + [_p] * 10 + [_sz, _p]),
+    "cm_gather_rows": (_i32, [_p, _i64, _i32, _p, _p, _p, _p]),
+    "cm_element_groups_max_elements": (_i32, []),
+    "cm_element_groups_workspace": (_sz, [_i64, _i32]),
+    "cm_element_groups": (_i32, [_p, _p, _i64, _i32] + [_p] * 5 + [_sz, _p]),
     "cm_node_glue_supported": (_i32, [_i32]),
     "cm_node_glue_forward": (_i32, [_p] * 6 + [_i64, _i32, _i32, _f32, _p, _p, _p, _p]),
     "cm_node_glue_backward": (_i32, [_p] * 6 + [_f64, _p, _p, _p, _i64, _i32, _i32, _f32, _p, _p]),
@@ -214,20 +219,23 @@ def stable_key_sort_static(keys: torch.Tensor, nkeys: int, perm: torch.Tensor, o
 
 
 def graph_prepare(positions: torch.Tensor, row_i: torch.Tensor, row_j: torch.Tensor, shifts: torch.Tensor,
-                  graph_of_node: Optional[torch.Tensor], ngraphs: int, r_max: float, bins: int) -> dict:
+                  graph_of_node: Optional[torch.Tensor], ngraphs: int, r_max: float, bins: int, symmetric_first_occ=None) -> dict:
     """cm_graph_prepare: the spatially ordered, shell-last copy of a neighbour list with its CSR offsets and its view sorted
     by sender, in one call without a host synchronisation.  Returns a dict of int32 tensors (node_perm, node_inverse,
-    receiver, sender, edge_perm, first_occ, sender_perm, sender_offsets) and shifts (fp64 [E, 3], reordered)."""
+    edges [2, E] and its rows receiver and sender, edge_perm, first_occ, sender_perm, sender_offsets) and shifts (fp64 [E, 3],
+    reordered).  symmetric_first_occ int32 [2 N]: the CSR of row0, for a list that holds the reverse of each of its pairs."""
     N, E = positions.shape[0], row_i.numel()
     dev = positions.device
     i32 = lambda n: torch.empty(n, dtype=I32, device=dev)  # noqa: E731
-    out = {"node_perm": i32(N), "node_inverse": i32(N), "receiver": i32(E), "sender": i32(E), "edge_perm": i32(E),
+    edges = torch.empty(2, -(-E // 64) * 64, dtype=I32, device=dev)[:, :E]  # both rows as aligned as an allocation
+    out = {"node_perm": i32(N), "node_inverse": i32(N), "edges": edges, "receiver": edges[0], "sender": edges[1], "edge_perm": i32(E),
            "shifts": torch.empty(E, 3, dtype=F64, device=dev), "first_occ": i32(2 * N), "sender_perm": i32(E),
            "sender_offsets": i32(N + 1)}
     need = lib.cm_graph_prepare_workspace(N, E, int(ngraphs), int(bins))
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
-    _check(lib.cm_graph_prepare(
-        _dev(positions, F64, "positions"), _dev(row_i, I32, "row_i"), _dev(row_j, I32, "row_j"), _dev(shifts, F64, "shifts"),
+    known = () if symmetric_first_occ is None else (_dev(symmetric_first_occ, I32, "symmetric_first_occ"),)
+    _check((lib.cm_graph_prepare_symmetric if known else lib.cm_graph_prepare)(
+        _dev(positions, F64, "positions"), _dev(row_i, I32, "row_i"), _dev(row_j, I32, "row_j"), _dev(shifts, F64, "shifts"), *known,
         _dev(graph_of_node, I32, "graph_of_node"), N, E, int(ngraphs), float(r_max), int(bins),
         _dev(out["node_perm"], I32, "node_perm"), _dev(out["node_inverse"], I32, "node_inverse"),
         _dev(out["receiver"], I32, "receiver"), _dev(out["sender"], I32, "sender"), _dev(out["edge_perm"], I32, "edge_perm"),
@@ -235,6 +243,42 @@ def graph_prepare(positions: torch.Tensor, row_i: torch.Tensor, row_j: torch.Ten
         _dev(out["sender_perm"], I32, "sender_perm"), _dev(out["sender_offsets"], I32, "sender_offsets"),
         ws.data_ptr(), ws.numel(), _stream()))
     return out
+
+
+def gather_rows(perm: torch.Tensor, *tensors: torch.Tensor):
+    """Rows `perm` (a permutation, int32 [N]) of each tensor, all with N rows, in one launch; no graph is recorded.  Tensors in
+    host memory are gathered there."""
+    n = perm.numel()
+    if not perm.is_cuda:
+        return [t.detach().index_select(0, perm) for t in tensors]
+    src = [t.detach().contiguous() for t in tensors]
+    for t in src:
+        if not t.is_cuda or t.dim() == 0 or t.shape[0] != n:
+            raise CudaMaceError("gather_rows: %s must live on the GPU with %d rows" % (tuple(t.shape), n))
+    out = [torch.empty_like(t) for t in src]
+    addresses = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])  # noqa: E731
+    sizes = (ctypes.c_int64 * len(src))(*[t.numel() // max(n, 1) * t.element_size() for t in src])
+    _check(lib.cm_gather_rows(_dev(perm, I32, "perm"), n, len(src), addresses(src), addresses(out), sizes, _stream()))
+    return out
+
+
+MAX_GROUPED_ELEMENTS = lib.cm_element_groups_max_elements()
+
+
+def element_groups(types: torch.Tensor, one_hot: torch.Tensor):
+    """((perm, offsets) by element index, (perm, offsets) by the first column of one_hot that is one, rows without one last)."""
+    n, ne = one_hot.shape
+    if types.shape != (n,):
+        raise CudaMaceError("element_groups: types must be [%d]" % n)
+    perms = torch.empty(2, -(-n // 64) * 64, dtype=I32, device=types.device)[:, :n]
+    by_type = perms[0], torch.empty(ne + 1, dtype=I32, device=types.device)
+    by_column = perms[1], torch.empty(ne + 2, dtype=I32, device=types.device)
+    nbytes = lib.cm_element_groups_workspace(n, ne)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=types.device)
+    _check(lib.cm_element_groups(_dev(types, I32, "types"), _dev(one_hot, F32, "one_hot"), n, ne, _dev(by_type[0], I32, "perm"),
+                                 _dev(by_type[1], I32, "offsets"), _dev(by_column[0], I32, "perm"), _dev(by_column[1], I32, "offsets"),
+                                 ws.data_ptr(), nbytes, _stream()))
+    return by_type, by_column
 
 
 # ---- message passing --------------------------------------------------------------------------

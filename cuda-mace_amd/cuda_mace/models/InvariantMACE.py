@@ -23,8 +23,8 @@ from cuda_mace.ops.spherical_harmonics import SphericalHarmonics
 from cuda_mace.ops.symmetric_contraction import SymmetricContraction as CUDAContraction
 from cuda_mace import _cabi as cabi
 from cuda_mace.ops._autograd import (EdgeGeometryAutograd, LinearContractionAutograd, ReadoutEnergyAutograd, ScalarLinearAutograd,
-                                     _cached, _cached_for, _cached_per, _found, _here, _leave, _leave_for, groups_of, groups_of_one_hot,
-                                     monomials_from_packed)
+                                     _cached, _cached_for, _cached_per, _found, _here, _leave, _leave_for, csr_of, groups_of, groups_of_one_hot,
+                                     monomials_from_packed, symmetric_list_of)
 from cuda_mace.utils.irreps import Instruction
 
 
@@ -498,13 +498,14 @@ class OptimizedInvariantMACE(torch.nn.Module):
                              lambda: (edge_index[0].int().contiguous(), edge_index[1].int().contiguous()))
         shifts = data["shifts"].detach().double().contiguous()
         # cells per axis from the size alone (a host constant): enough for cells of half a cutoff at 0.05 atoms / A^3
-        bins = int(min(64, max(1, np.ceil((n / max(ngraphs, 1) / 0.05) ** (1.0 / 3.0) / (0.5 * float(self.r_max))))))
+        r_max = self.edge_splines[0]._rmax  # on the host; reading the buffer would wait for the device, which has a list to build
+        bins = int(min(64, max(1, np.ceil((n / max(ngraphs, 1) / 0.05) ** (1.0 / 3.0) / (0.5 * r_max)))))
         while ngraphs * bins ** 3 >= 2 ** 24:
             bins -= 1
-        g = cabi.graph_prepare(pos, row0, row1, shifts, None if ngraphs == 1 else batch.int().contiguous(), ngraphs,
-                               float(self.r_max), bins)
-        receiver, sender = g["receiver"], g["sender"]
-        new_edges = torch.stack((receiver, sender))
+        known = symmetric_list_of(row1, n)
+        g = cabi.graph_prepare(pos, row0, row1, shifts, None if ngraphs == 1 else batch.int().contiguous(), ngraphs, r_max, bins,
+                               csr_of(row0, n) if known is not None and known[0] is row0 else None)
+        receiver, sender, new_edges = g["receiver"], g["sender"], g["edges"]
         # what the ops derive from a list is already there: leave it where they look it up
         _leave(new_edges, "_cm_int32_rows", None, (receiver, sender))
         _leave(receiver, "_cm_csr", n, g["first_occ"])
@@ -543,14 +544,15 @@ class OptimizedInvariantMACE(torch.nn.Module):
             hit = owner.__dict__.get("_cm_species_only")
             return hit is not None and hit[0] is self._weights_token and hit[1] == (owner._version, owner.data_ptr(), 0)
 
-        out = node_attrs.detach().index_select(0, perm)
         tag, before, streams = node_attrs.__dict__.pop("_cm_species_first_list", (None, None, None))
         if not knows(node_attrs) and tag == (node_attrs._version, node_attrs.data_ptr()) and knows(before[0]):
             first, its_inverse = _found(node_attrs, before, streams)
-            put(node_attrs, tuple(t.index_select(0, its_inverse) for t in self._species_of(first)))
+            put(node_attrs, tuple(cabi.gather_rows(its_inverse, *self._species_of(first))))
         if knows(node_attrs):
-            put(out, tuple(t.index_select(0, perm) for t in self._species_of(node_attrs)))
+            out, *known = cabi.gather_rows(perm, node_attrs, *self._species_of(node_attrs))
+            put(out, tuple(known))
         else:
+            out = node_attrs.detach().index_select(0, perm)
             node_attrs.__dict__["_cm_species_first_list"] = ((node_attrs._version, node_attrs.data_ptr()), (out, inverse), [_here(out)])
         return out
 

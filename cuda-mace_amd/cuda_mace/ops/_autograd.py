@@ -167,14 +167,23 @@ def csr_of(receiver: torch.Tensor, nnodes: int) -> torch.Tensor:
     return _cached(receiver, "_cm_csr", nnodes, lambda: cabi.first_occurences(receiver, nnodes))
 
 
+def symmetric_list_of(sender: torch.Tensor, nnodes: int):
+    """(receiver, unit_shifts, first_occ, offsets) of a list of the device search, which knows that it holds the reverse of each
+    of its pairs, while its tensors are unchanged; else None."""
+    known = sender.__dict__.get("_cm_symmetric_list")
+    if known is not None:
+        row_i, unit_shifts, first_occ, offsets, versions = known
+        if versions == (sender._version, row_i._version, unit_shifts._version) and offsets.numel() == nnodes + 1:
+            return row_i, unit_shifts, first_occ, offsets
+    return None
+
+
 def sender_view_of(sender: torch.Tensor, nnodes: int):
     def build():
-        # a list of the device search knows that it holds the reverse of each of its pairs: no sort is needed
-        known = sender.__dict__.get("_cm_symmetric_list")
-        if known is not None:
-            row_i, unit_shifts, first_occ, offsets, versions = known
-            if versions == (sender._version, row_i._version, unit_shifts._version) and offsets.numel() == nnodes + 1:
-                return cabi.symmetric_sender_view(row_i, sender, unit_shifts, first_occ, nnodes), offsets
+        known = symmetric_list_of(sender, nnodes)
+        if known is not None:  # no sort is needed
+            row_i, unit_shifts, first_occ, offsets = known
+            return cabi.symmetric_sender_view(row_i, sender, unit_shifts, first_occ, nnodes), offsets
         return cabi.stable_key_sort(sender, nnodes)
 
     return _cached(sender, "_cm_sender_view", nnodes, build)
@@ -196,6 +205,17 @@ def groups_of_one_hot(one_hot: torch.Tensor):
         return cabi.stable_key_sort(elem.contiguous(), ne + 1)  # group ne collects the rows without an element
 
     return _cached(one_hot, "_cm_groups", None, build)
+
+
+def groups_of_species(atom_types: torch.Tensor, one_hot: torch.Tensor, nelements: int):
+    """(groups_of(atom_types, nelements), groups_of_one_hot(one_hot)), both by one call where neither is there yet."""
+    if (one_hot.is_cuda and one_hot.dtype is F32 and one_hot.is_contiguous() and 0 < one_hot.shape[1] == nelements <= cabi.MAX_GROUPED_ELEMENTS
+            and "_cm_groups" not in atom_types.__dict__ and "_cm_groups" not in one_hot.__dict__):
+        by_type, by_column = cabi.element_groups(atom_types, one_hot)
+        _leave(atom_types, "_cm_groups", nelements, by_type)
+        _leave(one_hot, "_cm_groups", None, by_column)
+        return by_type, by_column
+    return groups_of(atom_types, nelements), groups_of_one_hot(one_hot)
 
 
 # ------------------------------------------------------------------------------------------------

@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from .. import _cabi as cabi
-from ._autograd import _cached, _found, _here, csr_of, groups_of, groups_of_one_hot, sender_view_of
+from ._autograd import _cached, _found, _here, csr_of, groups_of_species, sender_view_of
 
 _fp = ctypes.c_void_p
 
@@ -109,8 +109,7 @@ class NativeStep:
         I32 = torch.int32
         first_occ = csr_of(receiver, N)
         sperm, soff = sender_view_of(sender, N)
-        eperm, eoff = groups_of(atom_types, self.nelements)
-        operm, ooff = groups_of_one_hot(node_attrs32)
+        (eperm, eoff), (operm, ooff) = groups_of_species(atom_types, node_attrs32, self.nelements)
         ptr32 = _cached(ptr, "_cm_ptr32", None, lambda: ptr.int().contiguous())
         X1 = X1.contiguous()
         g.nnodes, g.nedges, g.ngraphs = N, int(receiver.numel()), int(ptr.numel()) - 1

@@ -476,6 +476,32 @@ int cm_graph_prepare(const double *positions, const int32_t *row_i, const int32_
                      double *shifts_out, int32_t *first_occ, int32_t *sender_perm, int32_t *sender_offsets, void *workspace,
                      size_t workspace_bytes, cm_stream_t stream);
 
+/* The same for a list that holds the reverse (j, i, -shift) of each of its pairs, as cm_neighbour_list_graph's do, and comes
+ * with old_first_occ [2 nnodes] = cm_first_occurences(row_i): the pairs need not be counted.  (Of any other list the view by
+ * sender is wrong, though every index in it lies in range.) */
+int cm_graph_prepare_symmetric(const double *positions, const int32_t *row_i, const int32_t *row_j, const double *shifts,
+                               const int32_t *old_first_occ, const int32_t *graph_of_node, int64_t nnodes, int64_t nedges,
+                               int ngraphs, double r_max, int bins, int32_t *node_perm, int32_t *node_inverse, int32_t *receiver,
+                               int32_t *sender, int32_t *edge_perm, double *shifts_out, int32_t *first_occ,
+                               int32_t *sender_perm, int32_t *sender_offsets, void *workspace, size_t workspace_bytes,
+                               cm_stream_t stream);
+
+/* Rows `perm` (int32 [nrows], a permutation; entries outside [0, nrows) leave their row unwritten) of narrays <= 8 arrays
+ * in one launch: row r of dst[k] = row perm[r] of src[k], row_bytes[k] <= 2^20 bytes each.  src, dst and row_bytes are host
+ * arrays; what moves with the atoms of a relabelled list goes through it. */
+int cm_gather_rows(const int32_t *perm, int64_t nrows, int narrays, const void *const *src, void *const *dst,
+                   const int64_t *row_bytes, cm_stream_t stream);
+
+/* Nodes grouped by element in both senses the model uses, three launches: type_perm [nnodes], type_offsets [nelements + 1] =
+ * cm_stable_key_sort(types, nnodes, nelements); column_perm [nnodes], column_offsets [nelements + 2] the same for the first
+ * column of one_hot fp32 [nnodes, nelements] that equals one, nodes without such a column last.
+ * nelements <= cm_element_groups_max_elements() = 63; workspace: cm_element_groups_workspace(nnodes, nelements) bytes. */
+int cm_element_groups_max_elements(void);
+size_t cm_element_groups_workspace(int64_t nnodes, int nelements);
+int cm_element_groups(const int32_t *types, const float *one_hot, int64_t nnodes, int nelements, int32_t *type_perm,
+                      int32_t *type_offsets, int32_t *column_perm, int32_t *column_offsets, void *workspace,
+                      size_t workspace_bytes, cm_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * The three [nnodes, C] x [C, C] linears between the two interaction layers as one launch per direction: the product's
  * linear and linear_up (the reference's linear_matmul, models/InvariantMACE.py:41-53) and the per-element skip

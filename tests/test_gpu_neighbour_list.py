@@ -323,3 +323,71 @@ def test_graph_prepare_matches_the_host_restatement(cabi, case):
         for n in (0, N // 2, N - 1):
             seg = beyond[fo[n]:fo[N + n]]
             assert bool((seg[1:] >= seg[:-1]).all())
+
+
+@pytest.mark.parametrize("degrees", [(512, 513, 0, 64, 65, 1), (1500, 2)])
+def test_graph_prepare_long_segments(cabi, degrees):
+    """cm_graph_prepare where a segment or a sender's bucket is longer than what a wave keeps on chip (512 keys, 256 pairs), on a
+    list in which a pair has no reverse and names of atoms out of range occur, against the numpy restatement."""
+    from oracle import ops as O
+    from tests.util import spatial_order_reference
+
+    g = torch.Generator().manual_seed(len(degrees))
+    N = len(degrees) + 3  # the last three atoms receive nothing
+    pos = 4.0 * torch.rand(N, 3, generator=g, dtype=torch.float64)
+    rcv = torch.repeat_interleave(torch.arange(len(degrees)), torch.tensor(degrees))
+    E = rcv.numel()
+    snd = torch.where(torch.rand(E, generator=g) < 0.7, torch.tensor(N - 1), torch.randint(0, N, (E,), generator=g))
+    shifts = 2.0 * torch.randint(-2, 3, (E, 3), generator=g).double()
+    got = cabi.graph_prepare(pos.cuda(), rcv.int().cuda(), snd.int().cuda(), shifts.cuda(), None, 1, 5.0, 8)
+    perm, inverse, new_rcv, new_snd, order = spatial_order_reference(pos, torch.zeros(N, dtype=torch.int64), torch.stack([rcv, snd]), shifts, 5.0, 8)
+    for name, want in (("node_perm", perm), ("node_inverse", inverse), ("receiver", new_rcv), ("sender", new_snd), ("edge_perm", order)):
+        np.testing.assert_array_equal(got[name].cpu().numpy(), want, err_msg=name)
+    sperm, soff = O.stable_key_sort(torch.from_numpy(new_snd).int(), N)
+    assert torch.equal(got["sender_perm"].cpu(), sperm) and torch.equal(got["sender_offsets"].cpu(), soff)
+    # names out of range: of atom j a pair counts for no sender; the views stay a function of the pairs that count
+    snd[::7] = N + 5
+    got = cabi.graph_prepare(pos.cuda(), rcv.int().cuda(), snd.int().cuda(), shifts.cuda(), None, 1, 5.0, 8)
+    new_snd = got["sender"].cpu()
+    counted = int(((snd >= 0) & (snd < N)).sum())
+    want = torch.sort(new_snd, stable=True).indices[:counted]
+    assert int(got["sender_offsets"][-1]) == counted and torch.equal(got["sender_perm"].cpu()[:counted].long(), want)
+
+
+@pytest.mark.parametrize("n,ne", [(0, 3), (1, 1), (255, 2), (256, 63), (257, 10), (5000, 4)])
+def test_element_groups_and_gathered_rows(cabi, n, ne):
+    """Both groupings against the sorts they stand for, with rows that hold no one, two ones or other values and with types out
+    of range; rows of 1 to 40 bytes gathered by a permutation against torch, all equal to the bit."""
+    g = torch.Generator().manual_seed(n + ne)
+    types = torch.randint(-1, ne + 1, (n,), generator=g).int().cuda()
+    one_hot = torch.randint(0, 3, (n, ne), generator=g).float().cuda()
+    by_type, by_column = cabi.element_groups(types, one_hot)
+    mask = one_hot == 1
+    column = torch.where(mask.any(dim=1), mask.to(torch.int8).argmax(dim=1), ne).int() if n else types
+    for got, keys, nkeys in ((by_type, types, ne), (by_column, column, ne + 1)):
+        perm, offsets = cabi.stable_key_sort(keys, nkeys)
+        count = int(offsets[-1])
+        assert torch.equal(got[1], offsets) and torch.equal(got[0][:count], perm[:count])
+    perm = torch.randperm(n, generator=g).int().cuda()
+    arrays = [torch.randint(0, 127, (n, w), generator=g, dtype=torch.int8).cuda() for w in (1, 4, 8, 16, 31, 40)] + [types, one_hot.double().T.contiguous().T]
+    for got, want in zip(cabi.gather_rows(perm, *arrays), arrays):
+        assert torch.equal(got, want.index_select(0, perm))
+
+
+@pytest.mark.parametrize("n,pbc", [(1, False), (40, True), (700, True), (9000, False)])
+def test_symmetric_list_is_prepared_alike(cabi, n, pbc):
+    """What cm_graph_prepare_symmetric makes of a list of the device search, whose pairs it does not count, is to the bit what
+    cm_graph_prepare makes of it."""
+    from cuda_mace.utils.neighbour_list import neighbour_data
+
+    g = torch.Generator().manual_seed(n)
+    box = (n / 0.08) ** (1.0 / 3.0) + 2.0
+    pos = (box * torch.rand(n, 3, generator=g, dtype=torch.float64)).cuda()
+    cell = torch.eye(3, dtype=torch.float64, device="cuda") * box if pbc else None
+    data = neighbour_data(pos, torch.ones(n, 1, dtype=torch.float64, device="cuda"), 5.5, (pbc,) * 3, cell)
+    row_i, row_j = (r.contiguous() for r in data["edge_index"].int())
+    first_occ = cabi.first_occurences(row_i, n)
+    args = (pos, row_i, row_j, data["shifts"], None, 1, 5.0, 20)
+    plain, known = cabi.graph_prepare(*args), cabi.graph_prepare(*args, symmetric_first_occ=first_occ)
+    for name in plain:
+        assert torch.equal(plain[name], known[name]), name
