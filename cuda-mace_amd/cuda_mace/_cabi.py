@@ -92,6 +92,9 @@ SIGNATURES = {
     "cm_mace_step_timing_read": (_i32, [_p, _p, _i32]),
     "cm_mace_step_workspace": (_sz, [_i64, _i64, _i32]),
     "cm_mace_energy_workspace": (_sz, [_i64, _i64, _i32]),
+    "cm_mace_step_stress": (_i32, [_p] * 6 + [_sz] + [_p] * 9),
+    "cm_report": (_i32, [_i32, _p, _p, _p, _p]),
+    "cm_host_max_displacement": (_f64, [_p, _p, _i64]),
     "cm_stress": (_i32, [_p, _p, _i64, _p, _p]),
     "cm_mace_energy": (_i32, [_p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p]),
     "cm_mace_step": (_i32, [_p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p, _p, _p]),
@@ -764,6 +767,23 @@ def stress_of(virials, cell):
     out = torch.empty_like(virials)
     _check(lib.cm_stress(_dev(virials, F64, "virials"), _dev(cell, F64, "cell"), virials.shape[0], _dev(out, F64, "stress"), _stream()))
     return out
+
+
+def report(tensors, host: torch.Tensor) -> None:
+    """The values of fp64 tensors on the GPU (at most four), one after the other, into `host` (pinned fp64 memory); returns when
+    they are there."""
+    total = sum(t.numel() for t in tensors)
+    if not (host.is_pinned() and host.dtype is F64 and host.is_contiguous() and host.numel() >= total):
+        raise CudaMaceError("report: needs contiguous pinned fp64 memory for %d values" % total)
+    n = len(tensors)
+    src = (ctypes.c_void_p * n)(*[_dev(t, F64, "result") for t in tensors])
+    counts = (ctypes.c_int64 * n)(*[t.numel() for t in tensors])
+    _check(lib.cm_report(n, src, counts, host.data_ptr(), _stream()))
+
+
+def host_max_displacement(positions, reference) -> float:
+    """Squared, for two contiguous fp64 numpy arrays [N, 3]."""
+    return lib.cm_host_max_displacement(positions.ctypes.data, reference.ctypes.data, positions.shape[0])
 
 
 # ---- readouts -------------------------------------------------------------------------------------

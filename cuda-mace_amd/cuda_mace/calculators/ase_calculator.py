@@ -19,7 +19,15 @@ from typing import Dict, Optional, Sequence
 import numpy as np
 import torch
 
+from cuda_mace import _cabi
+
 from .device_calculator import DeviceCalculator
+
+
+def _three(pbc) -> tuple:
+    """Three booleans from one or three."""
+    flags = np.asarray(pbc)
+    return tuple(map(bool, (flags if flags.shape == (3,) else np.broadcast_to(flags, (3,))).tolist()))
 
 
 class MACECalculator:
@@ -52,7 +60,7 @@ class MACECalculator:
     def _prepare(self, atoms, want_stress: bool) -> DeviceCalculator:
         numbers = np.asarray(atoms.get_atomic_numbers(), dtype=np.int64)
         cell = np.asarray(atoms.get_cell(), dtype=np.float64).reshape(3, 3)
-        pbc = tuple(bool(b) for b in np.broadcast_to(np.asarray(atoms.get_pbc()), (3,)))
+        pbc = _three(atoms.get_pbc())
         key = (numbers.tobytes(), cell.tobytes(), pbc, want_stress)
         if key != self._key:
             if want_stress and not all(pbc):
@@ -84,10 +92,10 @@ class MACECalculator:
         sent, received = self._staged
         sent.numpy()[...] = positions
         out = calc.compute(sent.to(self.device, non_blocking=True), host_positions=positions)
-        parts = [out["forces"].reshape(-1), out["energy"].reshape(-1)[:1]] + ([out["stress"].reshape(-1)] if calc.compute_stress else [])
-        packed = torch.cat([p.double() for p in parts])  # one copy and one wait instead of three
-        received[:packed.numel()].copy_(packed, non_blocking=True)
-        torch.cuda.current_stream(self.device).synchronize()
+        parts = [_cabi.as_f64(out["forces"]), _cabi.as_f64(out["energy"].reshape(-1)[:1])]
+        if calc.compute_stress:
+            parts.append(_cabi.as_f64(out["stress"]))
+        _cabi.report(parts, received)
         got = received.numpy()
         energy = float(got[3 * n])
         self.results = {"energy": energy, "free_energy": energy, "forces": got[:3 * n].reshape(n, 3).copy()}
@@ -102,7 +110,7 @@ class MACECalculator:
             return False
         numbers = np.asarray(atoms.get_atomic_numbers(), dtype=np.int64)
         cell = np.asarray(atoms.get_cell(), dtype=np.float64).reshape(3, 3)
-        pbc = tuple(bool(b) for b in np.broadcast_to(np.asarray(atoms.get_pbc()), (3,)))
+        pbc = _three(atoms.get_pbc())
         return (self._last[1][:3] == (numbers.tobytes(), cell.tobytes(), pbc)
                 and np.array_equal(self._last[0], np.asarray(atoms.get_positions(), dtype=np.float64)))
 

@@ -69,9 +69,10 @@ class DeviceCalculator:
         self._growth = math.inf     # largest growth of that between two tests (decays slowly); unknown at first
 
     # -- Verlet list ---------------------------------------------------------------------------------------
-    def _rebuild(self, positions: torch.Tensor) -> None:
-        pos = positions.detach().double().contiguous()
-        self._ref_positions = pos.clone()
+    def _rebuild(self, positions: torch.Tensor, host_positions: Optional[np.ndarray]) -> None:
+        # the reference of the displacement test: the caller may write to its own tensor (it is on the host where the test is)
+        self._ref_positions = positions if host_positions is not None else positions.clone()
+        self._ref_host = None if host_positions is None else host_positions.copy()
         self._data = neighbour_data(self._ref_positions, self.node_attrs, self.cutoff + self.skin, self.pbc, self.cell)
         self._graph = None
         if self.use_graph:
@@ -96,17 +97,18 @@ class DeviceCalculator:
         less than the round trip)."""
         positions = positions.detach().double().contiguous()
         self.steps += 1
-        if host_positions is not None and host_positions.shape[0] > 4096:
-            host_positions = None
+        if host_positions is not None:
+            host_positions = np.ascontiguousarray(host_positions, dtype=np.float64) if host_positions.shape[0] <= 4096 else None
         if self._ref_positions is None or self._ref_positions.shape != positions.shape:
             return self._on_fresh_list(positions, host_positions)
         limit = 0.5 * self.skin
         if host_positions is not None and self._ref_host is not None:
-            d = host_positions - self._ref_host
-            moved = math.sqrt(float(np.einsum("ij,ij->i", d, d).max(initial=0.0)))
+            moved = math.sqrt(_cabi.host_max_displacement(host_positions, self._ref_host))
             if not moved <= limit:
                 return self._on_fresh_list(positions, host_positions)
             return self._run(positions)
+        if self._ref_host is not None:  # the reference on the device was the caller's own tensor
+            self._ref_positions, self._ref_host = torch.from_numpy(self._ref_host).to(positions.device), None
         _cabi.max_displacement(positions, self._ref_positions, out=self._moved_sq)
         self._moved_sq_host.copy_(self._moved_sq, non_blocking=True)
         self._arrived.record()
@@ -122,6 +124,5 @@ class DeviceCalculator:
         return out if ahead else self._run(positions)
 
     def _on_fresh_list(self, positions: torch.Tensor, host_positions: Optional[np.ndarray]) -> Dict[str, torch.Tensor]:
-        self._rebuild(positions)
-        self._ref_host = None if host_positions is None else host_positions.copy()
+        self._rebuild(positions, host_positions)
         return self._run(positions)

@@ -160,6 +160,19 @@ def _select_head(per_head: torch.Tensor, heads_of_nodes) -> torch.Tensor:
     return torch.gather(per_head, 1, heads_of_nodes().view(-1, 1)).squeeze(1)
 
 
+def _weights_of_nodes(data):
+    """data["node_weights"] [N] (optional): every node energy enters the graph's energy, and hence the quantity the forces, virials
+    and stress derive from, with this weight (1 for a rank's own atoms, 0 for ghost copies in a domain-decomposed MD code);
+    node_energy itself stays unweighted."""
+    weights = data.get("node_weights")
+    return None if weights is None else weights.detach().to(torch.float64)
+
+
+def _rows_of(edge_index: torch.Tensor):
+    """(receiver, sender) of a list as int32 rows."""
+    return _cached(edge_index, "_cm_int32_rows", None, lambda: (edge_index[0].int().contiguous(), edge_index[1].int().contiguous()))
+
+
 def fused_readout_parameters(readouts, scale_shift):
     """Weights of the readout pair in the form the fused readout kernel takes, or None when the modules are not the
     standard pair of a two-layer invariant model (a linear readout to one scalar, then linear -> normalised silu gate ->
@@ -494,8 +507,7 @@ class OptimizedInvariantMACE(torch.nn.Module):
         pos = data["positions"].detach().double().contiguous()
         batch, edge_index = data["batch"], data["edge_index"]
         n, ngraphs = pos.shape[0], int(data["ptr"].numel()) - 1
-        row0, row1 = _cached(edge_index, "_cm_int32_rows", None,
-                             lambda: (edge_index[0].int().contiguous(), edge_index[1].int().contiguous()))
+        row0, row1 = _rows_of(edge_index)
         shifts = data["shifts"].detach().double().contiguous()
         # cells per axis from the size alone (a host constant): enough for cells of half a cutoff at 0.05 atoms / A^3
         r_max = self.edge_splines[0]._rmax  # on the host; reading the buffer would wait for the device, which has a list to build
@@ -599,6 +611,59 @@ class OptimizedInvariantMACE(torch.nn.Module):
         return self._forward_ordered(inner, training, compute_force, compute_virials, compute_stress, compute_displacement,
                                      node_rows=(perm, inverse), positions_in_caller_order=direct, compute_node_feats=compute_node_feats)
 
+    def _graph_e0(self, data, node_e0: torch.Tensor, weights, one_head: bool) -> torch.Tensor:
+        """(Weighted) sum of the atomic reference energies per graph.  The one-call step evaluates it once per list (it rides
+        in the step's graph handle); the autograd path evaluates it per call."""
+        num_graphs = data["ptr"].numel() - 1
+        if weights is None and num_graphs == 1 and one_head:
+            # one graph: the sum of the atomic reference energies is a function of the species tensor alone, too
+            return _cached_for(data["node_attrs"], "_cm_e0_sum", self._weights_token, lambda: node_e0.sum(dim=0, keepdim=True))
+        return scatter_sum(src=node_e0 if weights is None else node_e0 * weights, index=data["batch"], dim=0, dim_size=num_graphs,
+                           ptr=data["ptr"])
+
+    def _forward_native(self, native, data, num_graphs: int, compute_force: bool, compute_virials: bool, compute_stress: bool, node_rows,
+                        compute_node_feats: bool) -> Dict[str, Optional[torch.Tensor]]:
+        """`_forward_ordered` by the library's one call.  What the list and the species decide is looked up as a whole (the
+        handle), so a call on a known list touches nothing else of theirs."""
+        positions, edge_index, node_attrs = data["positions"], data["edge_index"], data["node_attrs"]
+
+        def build():
+            e0_per_head, node_feats_up, node_attrs32, atom_types = self._species_of(node_attrs)
+            receiver, sender = _rows_of(edge_index)
+            node_e0 = self._node_e0(data, e0_per_head)
+            return native.graph(edge_index, receiver, sender, node_attrs32, atom_types, data["ptr"], node_feats_up,
+                                None if node_rows is None else node_rows[0], node_e0, self._graph_e0(data, node_e0, None, True))
+
+        # one entry per model on the list's tensor, keyed on this model's weights token itself (the handle holds X1, which
+        # depends on this model's weights)
+        handle = _cached_per(edge_index, "_cm_native_graphs", self._weights_token, node_attrs, build)
+        if data.get("node_weights") is not None:
+            plain = handle
+
+            def weighted():
+                weights = _weights_of_nodes(data)
+                node_e0 = self._node_e0(data, self._species_of(node_attrs)[0])
+                return plain.with_node_weights(weights, self._graph_e0(data, node_e0, weights, True))
+
+            handle = _cached_per(data["node_weights"], "_cm_native_graphs_weighted", self._weights_token, plain, weighted)
+        want_virials = compute_virials or compute_stress
+        cell = data.get("cell") if compute_stress else None
+        res = native(handle, positions, data["shifts"], want_feats=compute_node_feats, want_virials=want_virials, want_forces=compute_force,
+                     cell=cell)
+        # energy = e0 + interaction energy and node_energy = node_e0 + its interaction part (already in the caller's
+        # order) are written by the step's own kernels: the atomic reference energies ride in the handle
+        dtype = positions.dtype
+        return {
+            "energy": res["energy"], "node_energy": res["node_energy"], "interaction_energy": res["interaction_energy"],
+            "forces": res["forces"].to(dtype) if compute_force else None, "virials": res["virials"].to(dtype) if want_virials else None,
+            "stress": None if cell is None else res["stress"].to(dtype), "hessian": None,
+            "displacement": _constant(0.0, (num_graphs, 3, 3), dtype, positions.device), "node_feats": res["node_feats"], "edge_forces": None,
+        }
+
+    def _node_e0(self, data, e0_per_head: torch.Tensor) -> torch.Tensor:
+        """Atomic reference energy of every node where all read head 0."""
+        return _select_head(e0_per_head, lambda: _cached(data["batch"], "_cm_zero_heads", None, lambda: torch.zeros_like(data["batch"])))
+
     def _forward_ordered(self, data: Dict[str, torch.Tensor], training: bool = False, compute_force: bool = True,
                          compute_virials: bool = False, compute_stress: bool = False, compute_displacement: bool = False,
                          node_rows=None, positions_in_caller_order: bool = False,
@@ -608,77 +673,35 @@ class OptimizedInvariantMACE(torch.nn.Module):
         positions_in_caller_order: data["positions"] (and hence the forces) are rows of the caller, read through rows."""
         data["positions"].requires_grad_(True)
         positions = data["positions"]
+        num_graphs = data["ptr"].numel() - 1
+        native = None
+        if node_rows is None or positions_in_caller_order:
+            native = self._native_step_for(data, training, compute_force, compute_displacement, compute_virials or compute_stress)
+        if native is not None:
+            return self._forward_native(native, data, num_graphs, compute_force, compute_virials, compute_stress, node_rows, compute_node_feats)
+
         node_attrs = data["node_attrs"]
         batch = data["batch"]
         node_heads = data["head"][batch] if "head" in data else None  # None: every node reads head 0
         heads_of_nodes = lambda: (node_heads if node_heads is not None  # noqa: E731
                                   else _cached(batch, "_cm_zero_heads", None, lambda: torch.zeros_like(batch)))
-        num_graphs = data["ptr"].numel() - 1
         shifts = data["shifts"]
         cell = data.get("cell")
 
-        native = None
-        if node_rows is None or positions_in_caller_order:
-            native = self._native_step_for(data, training, compute_force, compute_displacement, compute_virials or compute_stress)
         displacement = _constant(0.0, (num_graphs, 3, 3), positions.dtype, positions.device)  # replaced below when strained
-        if native is None and (compute_virials or compute_stress or compute_displacement):
+        if compute_virials or compute_stress or compute_displacement:
             positions, shifts, displacement, cell = get_symmetric_displacement(
                 positions=positions, unit_shifts=data["unit_shifts"], cell=cell, edge_index=data["edge_index"],
                 num_graphs=num_graphs, batch=batch)
 
         e0_per_head, node_feats_up, node_attrs32, atom_types = self._species_of(node_attrs)
         node_e0 = _select_head(e0_per_head, heads_of_nodes)
-        # data["node_weights"] [N] (optional): every node energy enters the graph's energy, and hence the quantity the
-        # forces, virials and stress derive from, with this weight (1 for a rank's own atoms, 0 for ghost copies in a
-        # domain-decomposed MD code); node_energy itself stays unweighted.
-        node_weights = data.get("node_weights")
-        if node_weights is not None:
-            node_weights = node_weights.detach().to(torch.float64)
-
-        def graph_e0(weights=node_weights):
-            """(Weighted) sum of the atomic reference energies per graph.  The one-call step evaluates it once per
-            list (it rides in the step's graph handle); the autograd path evaluates it per call."""
-            if weights is not None:
-                return scatter_sum(src=node_e0 * weights, index=batch, dim=0, dim_size=num_graphs, ptr=data["ptr"])
-            if num_graphs == 1 and node_heads is None:
-                # one graph: the sum of the atomic reference energies is a function of the species tensor alone, too
-                return _cached_for(node_attrs, "_cm_e0_sum", self._weights_token, lambda: node_e0.sum(dim=0, keepdim=True))
-            return scatter_sum(src=node_e0, index=batch, dim=0, dim_size=num_graphs, ptr=data["ptr"])
-
+        node_weights = _weights_of_nodes(data)
         node_feats = None
 
         # index structures shared by both layers, cached on the caller's tensors so that they are rebuilt only when
         # the neighbour list changes: int32 edge lists (their CSR offsets and sender-sorted view are in turn cached on these)
-        edge_index = data["edge_index"]
-        receiver, sender = _cached(edge_index, "_cm_int32_rows", None,
-                                   lambda: (edge_index[0].int().contiguous(), edge_index[1].int().contiguous()))
-
-        if native is not None:
-            rows32 = None if node_rows is None else node_rows[0]
-            # one entry per model on the list's tensor, keyed on this model's weights token itself (the handle holds
-            # X1, which depends on this model's weights)
-            handle = _cached_per(edge_index, "_cm_native_graphs", self._weights_token, node_attrs,
-                                 lambda: native.graph(edge_index, receiver, sender, node_attrs32, atom_types, data["ptr"],
-                                                      node_feats_up, rows32, node_e0, graph_e0(None)))
-            if node_weights is not None:
-                plain = handle
-                handle = _cached_per(data["node_weights"], "_cm_native_graphs_weighted", self._weights_token, plain,
-                                     lambda: plain.with_node_weights(node_weights, graph_e0()))
-            want_virials = compute_virials or compute_stress
-            res = native(handle, positions, shifts, want_feats=compute_node_feats, want_virials=want_virials, want_forces=compute_force)
-            inter_e = res["interaction_energy"]
-            virials = res["virials"].to(positions.dtype) if want_virials else None
-            stress = None
-            if compute_stress and cell is not None:
-                c3 = cell.detach().double().reshape(-1, 3, 3).expand_as(res["virials"]).contiguous()
-                stress = cabi.stress_of(res["virials"], c3).to(virials.dtype)
-            # energy = e0 + interaction energy and node_energy = node_e0 + its interaction part (already in the caller's
-            # order) are written by the step's own kernels: the atomic reference energies ride in the handle
-            return {
-                "energy": res["energy"], "node_energy": res["node_energy"], "interaction_energy": inter_e,
-                "forces": res["forces"].to(data["positions"].dtype) if compute_force else None, "virials": virials, "stress": stress, "hessian": None,
-                "displacement": displacement, "node_feats": res["node_feats"], "edge_forces": None,
-            }
+        receiver, sender = _rows_of(data["edge_index"])
 
         # vectors = positions[edge_index[1]] - positions[edge_index[0]] + shifts in fp64, rounded once to fp32
         vectors32, lengths32 = EdgeGeometryAutograd.apply(positions, shifts, receiver, sender,
@@ -727,7 +750,7 @@ class OptimizedInvariantMACE(torch.nn.Module):
         weighted_es = node_inter_es.double() if node_weights is None else node_inter_es.double() * node_weights
         inter_e = scatter_sum(src=weighted_es, index=batch, dim=-1, dim_size=num_graphs, ptr=data["ptr"])
 
-        total_energy = graph_e0() + inter_e
+        total_energy = self._graph_e0(data, node_e0, node_weights, node_heads is None) + inter_e
         node_energy = node_e0 + node_inter_es
         if node_rows is not None:  # node_feats is already written in the caller's order
             node_energy = node_energy.index_select(0, node_rows[1])

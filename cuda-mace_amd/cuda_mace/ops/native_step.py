@@ -113,10 +113,11 @@ class NativeStep:
         ptr32 = _cached(ptr, "_cm_ptr32", None, lambda: ptr.int().contiguous())
         X1 = X1.contiguous()
         g.nnodes, g.nedges, g.ngraphs = N, int(receiver.numel()), int(ptr.numel()) - 1
-        g.receiver, g.sender, g.first_occ = _ptr(receiver, I32, "receiver"), _ptr(sender, I32, "sender"), _ptr(first_occ, I32, "first_occ")
-        g.sender_perm, g.sender_offsets = _ptr(sperm, I32, "sender_perm"), _ptr(soff, I32, "sender_offsets")
-        g.elem_perm, g.elem_offsets = _ptr(eperm, I32, "elem_perm"), _ptr(eoff, I32, "elem_offsets")
-        g.onehot_perm, g.onehot_offsets = _ptr(operm, I32, "onehot_perm"), _ptr(ooff, I32, "onehot_offsets")
+        g.receiver, g.sender = _ptr(receiver, I32, "receiver"), _ptr(sender, I32, "sender")
+        # what this package derived itself needs no check
+        g.first_occ, g.sender_perm, g.sender_offsets = first_occ.data_ptr(), sperm.data_ptr(), soff.data_ptr()
+        g.elem_perm, g.elem_offsets = eperm.data_ptr(), eoff.data_ptr()
+        g.onehot_perm, g.onehot_offsets = operm.data_ptr(), ooff.data_ptr()
         g.node_rows = _ptr(node_rows, I32, "node_rows") if node_rows is not None else None
         g.graph_ptr, g.X1 = _ptr(ptr32, I32, "graph_ptr"), _ptr(X1, torch.float32, "X1")
         g.node_weights = None
@@ -135,11 +136,12 @@ class NativeStep:
                                 graph_e0))
 
     def __call__(self, handle: "_GraphHandle", positions: torch.Tensor, shifts: torch.Tensor, want_feats: bool = True,
-                 want_virials: bool = False, want_forces: bool = True) -> Dict[str, torch.Tensor]:
-        """want_forces=False: the forward half alone (cm_mace_energy), "forces" and "virials" are None."""
+                 want_virials: bool = False, want_forces: bool = True, cell: Optional[torch.Tensor] = None) -> Dict[str, torch.Tensor]:
+        """want_forces=False: the forward half alone (cm_mace_energy), "forces" and "virials" are None.  cell (one for all
+        graphs or one per graph): "stress" as well, which needs the virials."""
         _found(positions, self, self._streams)
-        g = handle.struct
-        N, E, C = int(g.nnodes), int(g.nedges), self.channels
+        N, E, ngraphs = handle.sizes
+        C = self.channels
         dev = positions.device
         F64 = torch.float64
         pos64, sh64 = cabi.as_f64(positions), cabi.as_f64(shifts)
@@ -149,37 +151,45 @@ class NativeStep:
         # stream, so calls on other streams or from other threads (ctypes lets go of the interpreter lock) have theirs, and a
         # captured step has its own for as long as its graph lives.  A steady caller gets the same block every time.
         ws = torch.empty(handle.workspace(want_forces, C), dtype=torch.uint8, device=dev)
-        energy = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
+        energy = torch.empty(ngraphs, dtype=F64, device=dev)
         node_energy = torch.empty(N, dtype=F64, device=dev)
         forces = torch.empty(N, 3, dtype=F64, device=dev) if want_forces else None
         feats = torch.empty(N, 2 * C, dtype=F64, device=dev) if want_feats else None
-        virials = torch.empty(int(g.ngraphs), 3, 3, dtype=F64, device=dev) if want_virials else None
-        total = torch.empty(int(g.ngraphs), dtype=F64, device=dev)
+        virials = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if want_virials else None
+        stress = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if cell is not None else None
+        total = torch.empty(ngraphs, dtype=F64, device=dev)
         node_total = torch.empty(N, dtype=F64, device=dev)
-        feats_at, virials_at = (None if t is None else t.data_ptr() for t in (feats, virials))
-        head = (ctypes.addressof(self.weights), ctypes.addressof(g), _ptr(pos64, F64, "positions"), _ptr(sh64, F64, "shifts"),
-                ws.data_ptr(), ws.numel(), energy.data_ptr(), node_energy.data_ptr())
+        feats_at, virials_at = None if feats is None else feats.data_ptr(), None if virials is None else virials.data_ptr()
+        where = (ctypes.addressof(self.weights), handle.address, _ptr(pos64, F64, "positions"), _ptr(sh64, F64, "shifts"))
+        head = (ws.data_ptr(), ws.numel(), energy.data_ptr(), node_energy.data_ptr())
         tail = (total.data_ptr(), node_total.data_ptr(), cabi._stream())
-        if want_forces:
-            cabi._check(cabi.lib.cm_mace_step(*head, forces.data_ptr(), feats_at, virials_at, *tail))
+        if not want_forces:
+            cabi._check(cabi.lib.cm_mace_energy(*where, *head, feats_at, *tail))
+        elif cell is None:
+            cabi._check(cabi.lib.cm_mace_step(*where, *head, forces.data_ptr(), feats_at, virials_at, *tail))
         else:
-            cabi._check(cabi.lib.cm_mace_energy(*head, feats_at, *tail))
+            cell64 = cabi.as_f64(cell)
+            if cell64.numel() != 9 * ngraphs:
+                cell64 = cell64.reshape(-1, 3, 3).expand(ngraphs, 3, 3).contiguous()
+            cabi._check(cabi.lib.cm_mace_step_stress(*where, _ptr(cell64, F64, "cell"), *head, forces.data_ptr(), feats_at, virials_at,
+                                                     stress.data_ptr(), *tail))
         # energy / node_energy: the interaction part plus the handle's graph_e0 / node_e0, node_energy in the caller's
         # order (rows node_rows of the handle); interaction_node_energy: the interaction part alone, in list order
         return {"interaction_energy": energy, "interaction_node_energy": node_energy, "energy": total, "node_energy": node_total,
-                "forces": forces, "node_feats": feats, "virials": virials}
+                "forces": forces, "node_feats": feats, "virials": virials, "stress": stress}
 
 
 class _GraphHandle:
     def __init__(self, struct, keep):
         self.struct, self._keep, self._bytes = struct, keep, {}
+        self.address, self.sizes = ctypes.addressof(struct), (int(struct.nnodes), int(struct.nedges), int(struct.ngraphs))
 
     def workspace(self, forces: bool, channels: int) -> int:
         """Bytes of scratch memory of a call on this handle."""
         nbytes = self._bytes.get((forces, channels))
         if nbytes is None:
             size = cabi.lib.cm_mace_step_workspace if forces else cabi.lib.cm_mace_energy_workspace
-            nbytes = self._bytes[forces, channels] = size(int(self.struct.nnodes), int(self.struct.nedges), channels)
+            nbytes = self._bytes[forces, channels] = size(*self.sizes[:2], channels)
         return nbytes
 
     def with_node_weights(self, weights: torch.Tensor, graph_e0: Optional[torch.Tensor] = None) -> "_GraphHandle":

@@ -626,6 +626,18 @@ int cm_mace_step(const cm_mace_weights *weights, const cm_mace_graph *graph, con
 /* stress fp64 [ngraphs, 3, 3] = -virials / |det cell|, cell fp64 [ngraphs, 3, 3] row vectors (the reference's get_outputs,
  * models/InvariantMACE.py:354, in one launch). */
 int cm_stress(const double *virials, const double *cell, int64_t ngraphs, double *stress, cm_stream_t stream);
+/* cm_mace_step that also writes stress fp64 [ngraphs, 3, 3] (NULL: not asked for) for cell fp64 [ngraphs, 3, 3], without the
+ * launch of cm_stress; virials may not be NULL then. */
+int cm_mace_step_stress(const cm_mace_weights *weights, const cm_mace_graph *graph, const double *positions, const double *shifts,
+                        const double *cell, void *workspace, size_t workspace_bytes, double *interaction_energy, double *node_energy,
+                        double *forces, double *node_feats, double *virials, double *stress, double *total_energy,
+                        double *total_node_energy, cm_stream_t stream);
+/* Results for a caller on the host: narrays <= 4 arrays of counts[k] doubles one after the other into `host`, memory of the host that
+ * the device can write (hipHostMalloc, torch's pin_memory), room for their sum; src and counts are host arrays.  The call returns
+ * when the values are there, whatever else it returns; refused on a stream under capture. */
+int cm_report(int narrays, const double *const *src, const int64_t *counts, double *host, cm_stream_t stream);
+/* cm_max_displacement for positions in host memory; nothing is enqueued.  Returns the largest squared distance. */
+double cm_host_max_displacement(const double *positions, const double *reference, int64_t nnodes);
 /* The forward half of cm_mace_step without forces: node energies and features bit for bit those of the full step; the sums
  * per graph may differ from its in the last bits (up to 128 channels the full step forms them in another launch, with
  * another number of partial sums).  No backward chain runs, nothing that only it reads is written, and the workspace,

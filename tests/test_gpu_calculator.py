@@ -262,3 +262,55 @@ def test_ase_protocol_calculator(cabi):
     atoms.numbers[0] = 79
     with pytest.raises(ValueError, match="not covered"):
         calc.get_forces(atoms)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (255, 0, 1), (256, 9, 257), (40_000, 1, 9, 3)])
+def test_results_reported_to_the_host(cabi, sizes):
+    """cm_report brings every word as it is: infinities, NaNs of any payload, the value it waits with, before and after other
+    work on the stream, on a stream that is not the default one."""
+    g = torch.Generator().manual_seed(sum(sizes))
+    arrays = [torch.randn(n, generator=g, dtype=torch.float64) for n in sizes]
+    bits = [0x7FF0000000000000, -0x10000000000000, 0x7FF4C0DEC0DEC0DE, 0x7FF8000000000001]
+    odd = torch.tensor(bits, dtype=torch.int64).view(torch.float64)
+    host = torch.empty(sum(sizes) + 3, dtype=torch.float64, pin_memory=True)
+    side = torch.cuda.Stream()
+    for round_ in range(3):
+        arrays[0][: min(4, sizes[0])] = odd[: min(4, sizes[0])].roll(round_)
+        on_device = [a.cuda() for a in arrays]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            doubled = [a.view(torch.int64) * 1 for a in on_device]  # made by the stream right before
+            cabi.report([d.view(torch.float64) for d in doubled], host)
+        got = host[: sum(sizes)].clone().view(torch.int64)
+        assert torch.equal(got, torch.cat(arrays).view(torch.int64))
+    with pytest.raises(cabi.CudaMaceError):
+        cabi.report([torch.zeros(host.numel() + 1, dtype=torch.float64, device="cuda")], host)
+
+
+@pytest.mark.parametrize("n", [0, 1, 1000])
+def test_displacement_on_the_host(cabi, n):
+    """cm_host_max_displacement is cm_max_displacement to the bit."""
+    g = torch.Generator().manual_seed(n)
+    a, b = torch.randn(n, 3, generator=g, dtype=torch.float64), torch.randn(n, 3, generator=g, dtype=torch.float64)
+    assert cabi.host_max_displacement(a.numpy(), b.numpy()) == float(cabi.max_displacement(a.cuda(), b.cuda())[0])
+    if n:
+        a[n // 2, 2] = float("nan")
+        assert cabi.host_max_displacement(a.numpy(), b.numpy()) == float("inf")
+
+
+def test_stress_of_the_step_is_that_of_its_virials(cabi):
+    """Stress written with the virials against cm_stress of them, for one cell per graph and one cell for all, at node counts of
+    both routes of the step (a workgroup per node, launches over all nodes)."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.synthetic import collate, make_system
+
+    up = SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=20.0, seed=2)
+    model = OptimizedInvariantMACE(up, device="cuda")
+    for sizes in ((100,), (110, 150), (700, 800)):
+        data = {k: v.cuda() for k, v in collate([make_system(n, 4, seed=n, density=0.08) for n in sizes]).items()}
+        out = model(dict(data), compute_stress=True)
+        cells = data["cell"].double().reshape(-1, 3, 3)
+        assert torch.equal(out["stress"], cabi.stress_of(out["virials"], cells.contiguous()))
+        one = dict(data, cell=cells[0])
+        shared = model(one, compute_stress=True)
+        assert torch.equal(shared["stress"], cabi.stress_of(shared["virials"], cells[:1].expand_as(shared["virials"]).contiguous()))
