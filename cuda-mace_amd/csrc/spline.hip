@@ -35,7 +35,7 @@ __global__ void spline_forward_kernel(const float *__restrict__ r, const float *
     val = a + x * (b + x * (c + x * d));
     if (DERIV) der = b + x * (2.f * c + (3.f * x) * d);
   }
-  st4_stream(R_out + e * J + j, val);
+  st4(R_out + e * J + j, val);
   if (DERIV) st4_stream(R_deriv + e * J + j, der);
 }
 
@@ -49,6 +49,8 @@ __global__ void spline_forward_kernel(const float *__restrict__ r, const float *
 // store writes eight whole lines (4.0 -> 5.2 TB/s at 1.3 million edges x 512 outputs; stores that scatter whole lines
 // over rows do not reach what a contiguous stream does).  The workgroups of one
 // output slice sit `nslices` apart in the grid, so at any time all slices, hence all parts of a row, are being written.
+// The rows are written through the caches: message passing reads them next, from the Infinity Cache as far as they fit there (122 880
+// edges x 384 outputs, 189 MB: this kernel 42 -> 37.5 us, the message passing after it 43 -> 39; at 1.6 GB no difference).
 constexpr int kSpThreads = 512;
 constexpr int kSpSlice = 32;            // outputs per workgroup
 constexpr int kSpMaxIntervals = 272;    // rows of the slice, the row of zeros included: 272 * 4 * 32 * 4 B = 139 264 B of LDS
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(kSpThreads) void spline_forward_sliced_kernel(
       const f4 a = *reinterpret_cast<const f4 *>(row), b = *reinterpret_cast<const f4 *>(row + 128),
                c = *reinterpret_cast<const f4 *>(row + 256), d = *reinterpret_cast<const f4 *>(row + 384);
       const int64_t e = round * kWave + src;
-      if (inside && e <= last) st4_stream(R_out + e * J + j, a + xs * (b + xs * (c + xs * d)));
+      if (inside && e <= last) st4(R_out + e * J + j, a + xs * (b + xs * (c + xs * d)));
     }
     re = re_next;
   }
@@ -439,12 +441,20 @@ template <int VEC>
 __device__ __forceinline__ typename Doubles<VEC>::type ldd(const double *p) {
   return *reinterpret_cast<const typename Doubles<VEC>::type *>(p);
 }
-template <int VEC>
-__device__ __forceinline__ void std_stream(double *p, typename Doubles<VEC>::type v) {
-  __builtin_nontemporal_store(v, reinterpret_cast<typename Doubles<VEC>::type *>(p));
+// KEEP: through the caches, for rows that the next kernel finds in the Infinity Cache (kKeepBytes); else past them
+template <int VEC, bool KEEP>
+__device__ __forceinline__ void std_out(double *p, typename Doubles<VEC>::type v) {
+  typedef typename Doubles<VEC>::type dv;
+  if constexpr (KEEP)
+    *reinterpret_cast<dv *>(p) = v;
+  else
+    __builtin_nontemporal_store(v, reinterpret_cast<dv *>(p));
 }
+// us for a layer of the op modules, past the caches -> through them: 61 MB of rows 219 -> 217, 307 MB 469 -> 464, 328 MB 533 -> 527, 369 MB 570 -> 571, 410 MB
+// 715 -> 738, 460 MB 721 -> 734
+constexpr int64_t kKeepBytes = int64_t{320} << 20;
 
-template <int VEC>
+template <int VEC, bool KEEP>
 __global__ __launch_bounds__(256) void spline_forward_f64_wave_kernel(const double *__restrict__ r, const double *__restrict__ r_knots,
                                                                       const double *__restrict__ coeffs, int64_t nedges, int nknots, int J,
                                                                       double r_width, double r_max, double *__restrict__ R_out,
@@ -458,8 +468,8 @@ __global__ __launch_bounds__(256) void spline_forward_f64_wave_kernel(const doub
   if (!(re <= r_max)) {  // beyond the cutoff (or no number): zeros, and no row of the table is read
 #pragma unroll 1
     for (int j = VEC * lane; j < J; j += VEC * kWave) {
-      std_stream<VEC>(R_out + e * J + j, dv{});
-      if (R_deriv) std_stream<VEC>(R_deriv + e * J + j, dv{});
+      std_out<VEC, KEEP>(R_out + e * J + j, dv{});
+      if (R_deriv) std_out<VEC, false>(R_deriv + e * J + j, dv{});
     }
     return;
   }
@@ -469,8 +479,8 @@ __global__ __launch_bounds__(256) void spline_forward_f64_wave_kernel(const doub
 #pragma unroll 1
   for (int j = VEC * lane; j < J; j += VEC * kWave) {
     const dv a = ldd<VEC>(cp + j), b = ldd<VEC>(cp + J + j), c = ldd<VEC>(cp + 2 * J + j), d = ldd<VEC>(cp + 3 * J + j);
-    std_stream<VEC>(R_out + e * J + j, a + x * (b + x * (c + x * d)));
-    if (R_deriv) std_stream<VEC>(R_deriv + e * J + j, b + x * (2.0 * c + (3.0 * x) * d));
+    std_out<VEC, KEEP>(R_out + e * J + j, a + x * (b + x * (c + x * d)));
+    if (R_deriv) std_out<VEC, false>(R_deriv + e * J + j, b + x * (2.0 * c + (3.0 * x) * d));
   }
 }
 
@@ -601,11 +611,13 @@ extern "C" int cm_spline_forward_f64(const double *r, const double *r_knots, con
   const bool pairs = cm::pairs_of_doubles(nedges, noutputs, {coeffs, R_out, R_deriv});
   const bool waves = cm::wave_per_edge_f64(nedges, noutputs, pairs);
   const dim3 grid(static_cast<unsigned>(cm::ceil_div(waves ? nedges * cm::kWave : threads, block)));
+  const bool keep = threads * 8 <= cm::kKeepBytes;
 #define CM_FORWARD_F64(KERNEL)                                                                                               \
   hipLaunchKernelGGL(KERNEL, grid, dim3(block), 0, cm::as_stream(stream), r, r_knots, coeffs, nedges, nknots, noutputs, r_width, \
                      r_max, R_out, R_deriv)
-  if (waves && pairs) CM_FORWARD_F64(cm::spline_forward_f64_wave_kernel<2>);
-  else if (waves) CM_FORWARD_F64(cm::spline_forward_f64_wave_kernel<1>);
+  if (waves && pairs && keep) CM_FORWARD_F64((cm::spline_forward_f64_wave_kernel<2, true>));
+  else if (waves && pairs) CM_FORWARD_F64((cm::spline_forward_f64_wave_kernel<2, false>));
+  else if (waves) CM_FORWARD_F64((cm::spline_forward_f64_wave_kernel<1, false>));
   else if (R_deriv) CM_FORWARD_F64(cm::spline_forward_f64_kernel<true>);
   else CM_FORWARD_F64(cm::spline_forward_f64_kernel<false>);
 #undef CM_FORWARD_F64

@@ -177,7 +177,19 @@ int nodes_per_wave(int64_t nnodes, int nelements, int64_t column_blocks, bool pa
 inline bool two_nodes_per_wave(int channels, int64_t nnodes) {
   return channels == 32 || channels == 160 || (channels == 96 && nnodes > 6 * device_compute_units());
 }
-template <typename S, bool GRAD, bool PAIRED>
+// The gradient is read again in the backward pass only.  Written past the caches it leaves room for everything in between (25 %
+// faster at 25 000 x 128); where the whole of it is about as large as the L2s (32 MB) or somewhat more, the Infinity Cache still has most of it then,
+// and the backward linear reads it from there.  A step of forces at 25 neighbours upward, us, past the caches -> through them: 5 000 x 64 (20 MB)
+// 313 -> 304, 8 000 x 64 (33) 421 -> 409, 6 500 x 96 (40) 560 -> 546, 4 000 x 128 (33) 459 -> 451, 5 000 x 128 (41) 578 -> 563; below and above that
+// the other way: 2 000 x 96 (12) 241 -> 242, 1 000 x 128 (8) 202 -> 206, 12 000 x 64 (49) 579 -> 577, 900 molecules x 64 (77) 437 -> 444, 8 000 x 128
+// (66) 787 -> 795; beyond 128 channels at all sizes: 4 000 x 160 (41) 611 -> 616, 3 000 x 192 (37) 578 -> 589.
+inline bool gradient_stays_near(int64_t nnodes, int channels) {
+  const int64_t bytes = nnodes * 16 * channels * 4;
+  return channels <= 128 && bytes >= (int64_t{18} << 20) && bytes <= (int64_t{48} << 20);
+}
+
+// KEEP is no argument of the kernel: of two branches that store the same value the compiler makes one plain store.
+template <typename S, bool GRAD, bool PAIRED, bool KEEP>
 __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict__ X,
                                                             const int32_t *__restrict__ node_perm,
                                                             const int32_t *__restrict__ group_offsets,
@@ -209,8 +221,10 @@ __global__ __launch_bounds__(kWave) void symcon_lmax3_kernel(const S *__restrict
     if (GRAD) {
       S *gp = grad + static_cast<int64_t>(node) * 16 * C + c;
 #pragma unroll
-      // streamed out: the gradient is read again only in the backward pass (measured 25 % faster at 128 channels)
-      for (int i = 0; i < 16; ++i) __builtin_nontemporal_store(g[i], gp + i * C);
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (KEEP) gp[i * C] = g[i];
+        else __builtin_nontemporal_store(g[i], gp + i * C);
+      }
     }
   }
 }
@@ -292,19 +306,25 @@ int forward(const char *what, const S *X, const int32_t *node_perm, const int32_
     const int64_t column_blocks = ceil_div(channels, paired ? kWave / 2 : kWave);
     const int npb = nodes_per_wave<S>(nnodes, nelements, column_blocks, paired);
     const dim3 grid(static_cast<unsigned>(ceil_div(nnodes, npb) + nelements), static_cast<unsigned>(column_blocks));
-    const auto launch = [&](auto with_grad, auto two) {
-      hipLaunchKernelGGL((symcon_lmax3_kernel<S, decltype(with_grad)::value, decltype(two)::value>), grid, dim3(kWave), 0, st, X, node_perm,
+    const auto launch = [&](auto with_grad, auto two, auto keep) {
+      hipLaunchKernelGGL((symcon_lmax3_kernel<S, decltype(with_grad)::value, decltype(two)::value, decltype(keep)::value>), grid, dim3(kWave), 0, st, X, node_perm,
                          group_offsets, T3, T2, T1, static_cast<int>(nnodes), nelements, channels, npb, out, grad);
     };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
     if constexpr (sizeof(S) == 4) {
-      if (paired) {
-        if (grad) launch(std::true_type{}, std::true_type{});
-        else launch(std::false_type{}, std::true_type{});
-        return check_launch(what);
-      }
+      const bool keep = gradient_stays_near(nnodes, channels);
+      if (grad && paired && keep) launch(yes, yes, yes);
+      else if (grad && paired) launch(yes, yes, no);
+      else if (grad && keep) launch(yes, no, yes);
+      else if (grad) launch(yes, no, no);
+      else if (paired) launch(no, yes, no);
+      else launch(no, no, no);
+    } else if (grad) {
+      launch(yes, no, no);
+    } else {
+      launch(no, no, no);
     }
-    if (grad) launch(std::true_type{}, std::false_type{});
-    else launch(std::false_type{}, std::false_type{});
     return check_launch(what);
   }
   // LDS per workgroup is held to 32 KB in fp32, 64 KB in fp64 (two [NB][16][C] arrays) so that several fit a CU

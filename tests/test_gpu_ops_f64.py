@@ -194,6 +194,18 @@ def test_spline_f64_more_edges_than_waves_in_a_launch(cabi):
     assert float(out[(r > 5.0)].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("E", [40_960, 40_961])
+def test_spline_f64_rows_through_and_past_the_caches(cabi, E):
+    """On both sides of the rule on the size of the rows (320 MB): the values are those of a call on some of the edges."""
+    g = torch.Generator().manual_seed(E)
+    knots = torch.linspace(0.0, 6.0, 64, dtype=F64, device=DEV)
+    coeffs = torch.randn(63, 4, 1024, generator=g, dtype=F64).to(DEV)
+    r = (torch.rand(E, generator=g, dtype=F64) * 5.6).to(DEV)
+    out = cabi.spline_forward(r, knots, coeffs, float(knots[1]), 5.0)
+    for part in (slice(0, 3000), slice(E - 3000, E)):
+        assert torch.equal(out[part], cabi.spline_forward(r[part].contiguous(), knots, coeffs, float(knots[1]), 5.0))
+
+
 @pytest.mark.parametrize("E,J", [(300, 4), (3001, 33), (20_000, 64), (20_000, 65), (2049, 640)])
 def test_spline_f64_reads_nothing_of_the_table_beyond_the_cutoff(cabi, E, J):
     """Lengths beyond the cutoff and lengths that are no numbers give zeros, value and derivative, in every kernel of the forward,

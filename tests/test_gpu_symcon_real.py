@@ -88,3 +88,9 @@ def test_two_nodes_per_wave(cabi, N, C, ne):
     ref.sum().backward()
     close(out_p.detach(), ref.detach(), 3e-5, 3e-6)
     close(grad_p, Xa.grad, 3e-5, 3e-6)
+
+
+@pytest.mark.parametrize("N,C", [(2303, 128), (2304, 128), (6144, 128), (6145, 128), (9215, 32), (9216, 32), (8193, 96)])
+def test_gradient_through_and_past_the_caches(cabi, N, C):
+    """Both sides of the rules on the size of the gradient (18 and 48 MB), one and two nodes per wave."""
+    test_two_nodes_per_wave(cabi, N, C, 4)
