@@ -133,6 +133,14 @@ __global__ __launch_bounds__(MULTI ? 8 * kWave : kWave, (MULTI || Cfg<C, true>::
           accumulate(e0);
           if (two) accumulate(e1);
         }
+      } else if constexpr (MULTI && K::V == 5) {
+        // five channels per lane: one edge's 85 registers (degree by degree, as below, an edge is four round trips)
+        for (int j = slot; j < nlive; j += K::EPW) {
+          Edge e0;
+          fetch(j, e0);
+          __builtin_amdgcn_sched_barrier(0);
+          accumulate(e0);
+        }
       } else {
         // one edge per trip; per degree the four coefficient pieces are loaded, used and dropped (16 registers of
         // radial data live at a time)
@@ -620,11 +628,15 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
 // 10.6 [10.6] 11.7, 400 x 52 19.4 14.5 13.9 [14.2] 18.4 19.0 20.1, 60 x 30 11.0 8.3 [8.2] 8.4 8.3 8.7 9.8; 64 216 x 52 11.8 8.8 [8.5] 9.0 9.2 9.7
 // 10.7, 1 000 x 30 [10.2] 11.6 15.7 17.5 28 30 34; 256 21 x 12 14.0 8.2 [7.5] 7.7 7.6 7.8 8.0, 300 x 9 12.8 [8.6] 8.6 8.9 11.9 12.1 12.9, 216 x 52
 // 43.5 20.5 17.2 16.1 15.1 [15.1] 15.7; 192 672 x 9 14.7 [10.7] 11.6 12.2 15.7 15.9 17.4.
+// At 160 channels a part is worth it from two edges per slot on, and up to one round of waves the kernel with parts also where there is one: a whole
+// step, us, with parts from four edges per slot on and degree by degree -> as it is: 20 x 8 120 -> 108, 50 x 11 134 -> 119, 200 x 15 145 -> 135, 420 x 9 156 ->
+// 150, 200 x 52 161 -> 156, 700 x 52 the same; at 224 channels, where 17 pieces of seven do not fit, no gain, and where two edges per slot are fetched at
+// once one part is better off alone (1 260 x 9 x 32 channels 84 -> 86, 1 500 x 128 154 -> 156).
 // With lengths and harmonics given a wave has less to wait for, and beyond two nodes per unit a part takes twelve edges (128 channels 1 000 x 20
 // 13.3 in one, 14.5 in two).
 template <int C, bool FROM_VEC>
 int forward_parts(int64_t nnodes, int64_t nedges) {
-  constexpr int kSlots = Cfg<C, true>::EPW, kLeast = kSlots >= 8 ? 24 : 4 * kSlots;
+  constexpr int kSlots = Cfg<C, true>::EPW, kLeast = kSlots >= 8 ? 24 : (Cfg<C, true>::V == 5 ? 2 : 4) * kSlots;
   if (nnodes <= 0) return 1;
   const int64_t least = !FROM_VEC && nnodes > 2 * device_compute_units() ? std::max(12, kLeast) : kLeast;
   int parts = static_cast<int>(std::min<int64_t>(6, std::max<int64_t>(1, nedges / (least * nnodes))));
@@ -673,7 +685,8 @@ int launch_forward(const float *X, const float *Y, const Spline &sp, const int32
                    int64_t nnodes, int64_t nedges, float *out, hipStream_t st) {
   const int parts = forward_parts<C, FROM_VEC>(nnodes, nedges);
   const size_t lds = static_cast<size_t>(parts) * kStageBytes + static_cast<size_t>(parts - 1) * 16 * C * sizeof(float);
-  if (parts > 1)
+  const int64_t one_round = 8 * device_compute_units();
+  if (parts > 1 || (Cfg<C, true>::V == 5 && nnodes <= one_round))
     hipLaunchKernelGGL((mp_spline_forward_kernel<C, FROM_VEC, true>), dim3(static_cast<unsigned>(nnodes)), dim3(kWave * parts), lds, st,
                        X, Y, sp, sender, first_occ, static_cast<int>(nnodes), nedges, out);
   else

@@ -354,3 +354,13 @@ def test_forward_from_vectors_is_no_less_precise_than_from_harmonics_and_lengths
     error_a, error_b = (float((t.double().cpu() - ref).norm() / ref.norm()) for t in (a, b))
     print("C=%d from vectors %.3e, from harmonics and lengths %.3e" % (C, error_a, error_b), flush=True)
     assert error_a <= 1.02 * error_b
+
+
+@pytest.mark.parametrize("case", [(1, 3, 160, 0.0, 61, 256, 0), (40, 1, 160, 0.3, 62, 200, 0), (60, 3, 160, 0.0, 63, 256, 70), (60, 4, 160, 0.0, 64, 256, 0), (200, 13, 160, 0.1, 65, 600, 130),
+                                  (1024, 6, 160, 0.0, 66, 256, 0), (2048, 2, 160, 0.2, 67, 256, 0), (2049, 2, 160, 0.2, 68, 256, 0)],
+                         ids=lambda c: "N%d_d%d_k%d" % (c[0], c[1], c[5]))
+def test_mp_forward_of_five_channels_per_lane(cabi, case):
+    """160 channels with few nodes: one part and several, parts without an edge, one round of waves and one node more; from vectors and from
+    lengths and harmonics."""
+    test_mp_edge_forward_many_nodes(cabi, case)
+    test_mp_spline_forward_backward(cabi, case[:5])
