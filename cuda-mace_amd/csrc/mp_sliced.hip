@@ -382,23 +382,20 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
 
   const int tid = threadIdx.x;
   // Which (pair, slice) and which piece j of the node range.  Consecutive workgroups go to consecutive XCDs (eight of
-  // them, each with its own L2): all workgroups of a piece sit on one XCD, so that the edge data and the X rows of the
-  // piece are fetched into one L2 only, for as many pieces as divide evenly among the XCDs (all of them at 64, 128 and
-  // 256 channels).
+  // them, each with its own L2).  The pieces in order, each with all its types, are cut into eight runs, one per XCD: the edge data
+  // and the X rows of neighbouring nodes are fetched into one L2, or two where a piece is cut (share / 8 is no whole number at 96, 160, 192
+  // and 224 channels).  With pieces 8 apart on an XCD and the rest of share / 8 spread over all of them every L2 fetched up to a third of
+  // the nodes.  Energies alone, us, that -> this: 96 channels 10 000 265 -> 261, 40 000 979 -> 931; 128 25 000 773 -> 765, 30 000 938 -> 933;
+  // 160 10 007 450 -> 444, 25 000 1 088 -> 1 055; 192 10 000 540.5 -> 540.2, 40 000 2 055 -> 2 028; 224 30 000 1 848 -> 1 839; 32 12 000 143 -> 139; 64
+  // and 256 the same.  Sixteen workgroups more at 160 and 192 channels, each with its share of the nodes of one or two types, gave
+  // 0 to 0.8 % in place of that (the second slice of the table, the rounds at the end of both parts).
   int type, j;
   {
     const int types = 2 * p.nslices;
-    const int aligned = (p.share / 8) * 8;  // pieces that go to one XCD each; the others are spread over all of them
-    const int b = blockIdx.x;
-    if (b < aligned * types) {
-      const int xcd = b % 8, q = b / 8;
-      type = q % types;
-      j = xcd + 8 * (q / types);
-    } else {
-      const int rest = b - aligned * types;
-      type = rest % types;
-      j = aligned + rest / types;
-    }
+    const int total = types * p.share, xcd = blockIdx.x % 8;
+    const int rank = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+    type = rank % types;
+    j = rank / types;
   }
   const int slice = type >> 1;
   const int pair = type & 1;
