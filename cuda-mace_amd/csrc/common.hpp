@@ -118,6 +118,15 @@ __device__ __forceinline__ void edge_vector_f64(const double *__restrict__ pos, 
   }
 }
 
+// Which piece of work workgroup b of `total` takes so that RUN neighbouring pieces are on one XCD: workgroups go to the eight XCDs in
+// turn, each with an L2 of its own.  Runs and not an eighth of the work each, so that dense and empty regions meet on every
+// XCD; the pieces behind the last 8 RUN stay in turn.
+template <int RUN>
+__device__ __forceinline__ int place_on_xcd(int b, int total) {
+  constexpr int kRuns = 8 * RUN;
+  return b < total / kRuns * kRuns ? b / kRuns * kRuns + b % 8 * RUN + b / 8 % RUN : b;
+}
+
 // Edge range [e0, e1) of a node as read from caller-provided CSR offsets, forced into [0, nedges] with e0 <= e1: offsets
 // derived from an unsorted or out-of-range receiver list then name a wrong but addressable range instead of memory
 // outside the edge arrays.

@@ -77,6 +77,7 @@ __global__ void edge_grad_kernel(const double *__restrict__ pos, const double *_
 // VIRIAL: the atom's share of the virial from the edges that start at it, as the comment on virials in step.hip has it, instead of
 // in a launch of its own: 216 x 90 edges 5.7 + 5.5 -> 6.0 (16 lanes 11.0), 1 000 x 52 5.3 (16 lanes 7.7), 5 000 x 52 9.1 + 5.0 -> 12.1,
 // 12 000 x 24 14.1 + 5.8 -> 13.5; alone, 5 000 x 52 with 64 lanes 9.6 and with 16 lanes 6.4.
+// Runs of 128 neighbouring atoms on an XCD: gradients of edges that end at neighbours share lines (25 000 x 52 20.0 -> 17.2, 100 000 x 52 65.7 -> 62.3).
 constexpr int64_t kFewAtoms = 2048;
 template <int LANES, bool HAS_GLEN, bool VIRIAL>
 __global__ __launch_bounds__(256) void edge_geometry_backward_kernel(
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(256) void edge_geometry_backward_kernel(
     double *__restrict__ node_virial) {
   constexpr int kEdgesAhead = kWave / LANES;
   const int lane = threadIdx.x % LANES;
-  const int node = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES;
+  const int node = place_on_xcd<LANES / 2>(blockIdx.x, gridDim.x) * (blockDim.x / LANES) + threadIdx.x / LANES;
   const bool here = node < nnodes;
   double acc[3] = {0.0, 0.0, 0.0}, vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   int kb0 = 0, kb1 = 0, ea0 = 0, ea1 = 0, row = 0;

@@ -452,7 +452,12 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
   constexpr int kKnots = C == 224 ? 256 : kKnotsInLds;
   __shared__ float sKnots[kKnots];
 
-  const int node = parts == 1 ? blockIdx.x : blockIdx.x / parts;
+  // Runs of 128 neighbouring nodes on an XCD: where the X rows are more than one L2 holds, a neighbour's rows come from there more
+  // often (step, us, with the forces' runs: 40 000 x 160 4 810 -> 4 776, 100 000 x 192 by the card 13 987 -> 13 849 or 13 985 -> 13 968; runs of 32
+  // and 512 the same; 10 007 x 160 and 20 000 x 224 equal).  The kernel above gains nothing from it (25 000 x 128, 40 000 x 96,
+  // 12 000 x 256; 25 000 x 128 without gX 448 -> 459 alone).
+  const int place = place_on_xcd<128>(blockIdx.x, nnodes * parts);
+  const int node = parts == 1 ? place : place / parts;
   const int lane = threadIdx.x;
   const int row = lane / 16;  // which edge of a group
   const int cl = lane % 16;
@@ -469,7 +474,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
   int e1 = first_occ[nnodes + node];
   clamp_edge_range(e0, e1, nedges);
   if (parts > 1) {
-    const int part = blockIdx.x % parts;
+    const int part = place % parts;
     const int64_t len = e1 - e0;
     const int lo = e0 + static_cast<int>(len * part / parts);
     e1 = e0 + static_cast<int>(len * (part + 1) / parts);

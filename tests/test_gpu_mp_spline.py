@@ -318,6 +318,13 @@ def test_mp_edge_backward_few_and_many_nodes(cabi, case):
     test_mp_edge_backward_of_four_edges_per_step(cabi, case)
 
 
+@pytest.mark.parametrize("case", [(1023, 9, 160, 0.1, 71, 256, 0), (1025, 9, 192, 0.0, 72, 256, 0), (2049, 7, 224, 0.1, 73, 256, 70)],
+                         ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
+def test_mp_edge_backward_of_nodes_beyond_whole_runs(cabi, case):
+    """Nodes are dealt to the eight XCDs in runs of 128, those behind the last 1 024 one at a time."""
+    test_mp_edge_backward_of_four_edges_per_step(cabi, case)
+
+
 @pytest.mark.parametrize("case", [(600, 4, 192, 0.0, 41, 256, 70), (600, 6, 192, 0.0, 42, 256, 70), (700, 2, 224, 0.0, 43, 256, 66),
                                   (700, 4, 224, 0.0, 44, 300, 66), (1537, 9, 224, 0.0, 45, 256, 0), (1536, 9, 224, 0.0, 46, 256, 0),
                                   (2048, 6, 224, 0.1, 47, 512, 130), (2049, 4, 224, 0.0, 48, 256, 0), (2049, 6, 224, 0.0, 49, 256, 0),

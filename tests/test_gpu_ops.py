@@ -914,6 +914,12 @@ def test_edge_geometry_with_a_wave_or_a_quarter_per_atom(cabi, nnodes, avg, iso,
     test_edge_geometry(cabi, nnodes, avg, iso, seed)
 
 
+@pytest.mark.parametrize("nnodes,avg,iso,seed", [(1021, 9, 0.1, 8), (1024, 9, 0.0, 9), (1027, 9, 0.1, 10), (3071, 9, 0.0, 11), (3089, 9, 0.1, 12)])
+def test_edge_geometry_of_atoms_beyond_whole_runs(cabi, nnodes, avg, iso, seed):
+    """Atoms are dealt to the eight XCDs in runs of 128, those behind the last 1 024 one workgroup at a time."""
+    test_edge_geometry(cabi, nnodes, avg, iso, seed)
+
+
 # ---- readouts ---------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("N,C,H,seed", [(1, 32, 16, 0), (1000, 128, 16, 1), (37, 96, 5, 2), (515, 256, 1, 3), (16, 64, 16, 4), (50, 30, 7, 5), (20000, 128, 16, 6)])
 def test_readout_forward_backward(cabi, N, C, H, seed):
