@@ -348,6 +348,25 @@ def test_spline_backward_on_both_sides_of_the_line_of_its_row(cabi, E, J, nknots
     test_spline_backward_in_the_order_of_the_intervals(cabi, E, J, nknots)
 
 
+@pytest.mark.parametrize("E,J,share", [(32_768, 256, 0.0), (32_768, 132, 0.01), (32_771, 384, 0.25), (40_003, 260, 0.5), (33_333, 388, 0.3), (32_769, 512, 0.26),
+                                       (40_960, 512, 1.0), (70_000, 384, 1.0)])
+def test_spline_backward_with_few_edges_of_a_chunk_inside_the_cutoff(cabi, E, J, share):
+    """No edge, a few, one for each of a workgroup's 32 half-waves and some more, or all: the next row is requested ahead, and the
+    last one again behind it.  Against the kernel with a wave per edge, which takes shorter lists; a sum of up to 512 terms differs
+    by its order, at most 18 roundings of each side, 2^-24 each: 5e-6 of the terms' magnitudes as above."""
+    _say("spline backward sorted", E, J, share)
+    g = torch.Generator().manual_seed(E + J)
+    knots, coeffs = torch.linspace(0.0, 6.0, 256).to(DEV), torch.randn(255, 4, J, generator=g).to(DEV)
+    r = torch.where(torch.rand(E, generator=g) < share, torch.rand(E, generator=g) * 4.9, torch.full((E,), 5.5)).to(DEV)
+    gR = torch.randn(E, J, generator=g).to(DEV)
+    gr = cabi.spline_backward(r, knots, coeffs, gR, 6.0 / 255, 5.0)
+    ref = torch.cat([cabi.spline_backward(r[k:k + 20_000], knots, coeffs, gR[k:k + 20_000], 6.0 / 255, 5.0) for k in range(0, E, 20_000)])
+    x = 6.0 / 255
+    bound = 5e-6 * (gR.abs() * (1 + 2 * x + 3 * x * x)).sum(-1) * coeffs.abs().max()
+    assert bool(((gr - ref).abs() <= bound).all()) and float(gr[r > 5.0].abs().sum()) == 0.0
+    assert share < 0.2 or float(gr.abs().max()) > 1.0
+
+
 # ------------------------------------------------------------------------------------------------
 # linears (fp32 MFMA)
 # ------------------------------------------------------------------------------------------------
