@@ -186,30 +186,34 @@ __global__ void relabel_nodes_kernel(const int32_t *__restrict__ keys, const int
 
 // Two workgroups.  The first: first_occ[a] = exclusive scan of degree, first_occ[n + a] = inclusive scan (the CSR layout the
 // message-passing kernels take: starts, then ends).  The second: the offsets of the view by sender, and a copy to fill by.
+// Ranges of the old CSR overlap where the list is not sorted by row i, and then add up to more than nedges, or more than 32 bits hold:
+// the sums have 64, and no offset lies beyond the list.
 __global__ __launch_bounds__(kScanThreads) void edge_offsets_kernel(const int32_t *__restrict__ degree, const int32_t *__restrict__ sent, int n,
-                                                                    int32_t *__restrict__ first_occ, int32_t *__restrict__ sender_offsets,
-                                                                    int32_t *__restrict__ cursor) {
-  __shared__ int part[kScanThreads];
-  __shared__ int stage[kScanStage];
+                                                                    int64_t nedges, int32_t *__restrict__ first_occ,
+                                                                    int32_t *__restrict__ sender_offsets, int32_t *__restrict__ cursor) {
+  __shared__ int64_t part[kScanThreads];
+  __shared__ int64_t stage[kScanStage / 2];
   const bool by_sender = blockIdx.x == 1;
   const int32_t *__restrict__ counts = by_sender ? sent : degree;
-  const int total = workgroup_exclusive_scan<kScanThreads, kScanStage, int>(
+  const auto within = [&](int64_t offset) { return static_cast<int32_t>(offset < nedges ? offset : nedges); };
+  const int64_t total = workgroup_exclusive_scan<kScanThreads, kScanStage / 2, int64_t>(
       n, stage, part, [&](int k) { return counts[k]; },
-      [&](int k, int before, int value) {
+      [&](int k, int64_t before, int64_t value) {
         if (by_sender) {
-          sender_offsets[k] = cursor[k] = before;
+          sender_offsets[k] = cursor[k] = within(before);
         } else {
-          first_occ[k] = before;
-          first_occ[n + k] = before + value;
+          first_occ[k] = within(before);
+          first_occ[n + k] = within(before + value);
         }
       });
-  if (by_sender && threadIdx.x == 0) sender_offsets[n] = total;
+  if (by_sender && threadIdx.x == 0) sender_offsets[n] = within(total);
 }
 
 // One wave per new atom: keys of the pairs of its segment (pairs within the cutoff by the new label of atom j, the others
 // behind them by length: the bit pattern of a non-negative double orders like its value), their ranks by (key, position in
 // the list), the pairs at their places, and each into its sender's bucket in any order.  Keys of more pairs than LDS holds
-// go through `key`.  Of a list that is not sorted by row i, pairs may stay without a place: none is written out of range.
+// go through `key`.  Of a list that is not sorted by row i, an atom has the pairs that find a place, and others stay without: none is
+// written out of range.
 __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__restrict__ pos, const int32_t *__restrict__ perm,
                                                             const int32_t *__restrict__ inverse, const int32_t *__restrict__ old_first_occ,
                                                             const int32_t *__restrict__ new_first_occ, const int32_t *__restrict__ row_i,
@@ -224,8 +228,7 @@ __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__rest
   const int o = perm[a];
   int s0 = old_first_occ[o], s1 = old_first_occ[nnodes + o];
   clamp_edge_range(s0, s1, nedges);
-  const int d = s1 - s0;
-  const int base = new_first_occ[a];
+  const int base = new_first_occ[a], d = min(s1 - s0, new_first_occ[nnodes + a] - base);
   const bool in_lds = d <= kSegLds;
   for (int t = lane; t < d; t += kWave) {
     const int64_t e = s0 + t;
@@ -260,8 +263,7 @@ __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__rest
         rank += (other < mine || (other == mine && t < k)) ? 1 : 0;
       }
     }
-    const int64_t at = static_cast<int64_t>(base) + rank;
-    if (at >= nedges) continue;
+    const int64_t at = base + rank;
     const bool named = static_cast<unsigned>(j) < static_cast<unsigned>(nnodes);
     const int s_new = named ? inverse[j] : j;
     receiver[at] = a;
@@ -429,7 +431,7 @@ int prepare(const double *positions, const int32_t *row_i, const int32_t *row_j,
     hipLaunchKernelGGL(relabel_nodes_kernel, dim3(gn), block, 0, st, L.atom_keys, L.binned, L.bin_offsets, old_first_occ,
                        known_first_occ ? static_cast<const int32_t *>(nullptr) : L.pairs_of_sender, N, nedges, node_perm, node_inverse, L.degree, L.sent);
   }
-  hipLaunchKernelGGL(edge_offsets_kernel, dim3(2), dim3(kScanThreads), 0, st, L.degree, L.sent, N, first_occ, sender_offsets,
+  hipLaunchKernelGGL(edge_offsets_kernel, dim3(2), dim3(kScanThreads), 0, st, L.degree, L.sent, N, nedges, first_occ, sender_offsets,
                      L.sender_cursor);
   if (nedges > 0) {
     hipLaunchKernelGGL(place_edges_kernel, dim3(static_cast<unsigned>(nnodes)), dim3(kWave), 0, st, positions, node_perm, node_inverse,

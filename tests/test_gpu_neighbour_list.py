@@ -391,3 +391,39 @@ def test_symmetric_list_is_prepared_alike(cabi, n, pbc):
     plain, known = cabi.graph_prepare(*args), cabi.graph_prepare(*args, symmetric_first_occ=first_occ)
     for name in plain:
         assert torch.equal(plain[name], known[name]), name
+
+
+@pytest.mark.parametrize("case", ["rows_in_turn", "all_ranges_whole", "sums_beyond_32_bits"])
+@pytest.mark.parametrize("known", [True, False])
+def test_graph_prepare_of_unsorted_rows_stays_within_the_list(cabi, case, known):
+    """Rows that are not sorted, or a CSR whose ranges overlap, give a view that means nothing, every index of which lies within
+    the list: offsets ascend to at most the number of pairs, and nothing is written behind an output."""
+    N, E = {"rows_in_turn": (2, 400), "all_ranges_whole": (70, 300), "sums_beyond_32_bits": (600_000, 4096)}[case]
+    print("graph_prepare", case, known, flush=True)
+    if not known and case != "rows_in_turn":
+        pytest.skip("the CSR is given only where the list is known")
+    g = torch.Generator().manual_seed(N)
+    pos = (30.0 * torch.rand(N, 3, generator=g, dtype=torch.float64)).cuda()
+    row_i = (torch.arange(E) % N).int().cuda()
+    row_j = torch.randint(0, N, (E,), generator=g).int().cuda()
+    shifts = torch.zeros(E, 3, dtype=torch.float64, device="cuda")
+    if case == "rows_in_turn":  # what the two writers of one entry can leave: both ranges all but whole
+        csr = torch.tensor([0, 1, E - 1, E], dtype=torch.int32, device="cuda")
+    else:
+        csr = torch.cat([torch.zeros(N), torch.full((N,), E)]).int().cuda()
+    guard, word = 4096, 0x5A5A5A5A
+    sizes = {"node_perm": N, "node_inverse": N, "receiver": E, "sender": E, "edge_perm": E, "shifts": 6 * E, "first_occ": 2 * N,
+             "sender_perm": E, "sender_offsets": N + 1}
+    out = {k: torch.full((n + guard,), word, dtype=torch.int32, device="cuda") for k, n in sizes.items()}
+    ws = torch.empty(cabi.lib.cm_graph_prepare_workspace(N, E, 1, 8), dtype=torch.uint8, device="cuda")
+    prepare = cabi.lib.cm_graph_prepare_symmetric if known else cabi.lib.cm_graph_prepare
+    cabi._check(prepare(pos.data_ptr(), row_i.data_ptr(), row_j.data_ptr(), shifts.data_ptr(), *([csr.data_ptr()] if known else []), None, N, E, 1, 5.0, 8,
+                        *[out[k].data_ptr() for k in sizes], ws.data_ptr(), ws.numel(), cabi._stream()))
+    torch.cuda.synchronize()
+    for k, n in sizes.items():
+        assert bool((out[k][n:] == word).all()), "%s: written behind its end" % k
+    offsets, first_occ = out["sender_offsets"][:N + 1].cpu(), out["first_occ"][:2 * N].cpu()
+    assert int(offsets[0]) == 0 and int(offsets[-1]) <= E and bool((offsets[1:] >= offsets[:-1]).all())
+    assert bool(((first_occ >= 0) & (first_occ <= E)).all()) and bool((first_occ[N:] >= first_occ[:N]).all())
+    view = out["sender_perm"][:int(offsets[-1])].cpu()
+    assert bool(((view >= 0) & (view < E)).all())
