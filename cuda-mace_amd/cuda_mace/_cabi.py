@@ -10,6 +10,7 @@ import ctypes
 import os
 from typing import Optional
 
+import numpy as np
 import torch
 
 _HERE = os.path.realpath(os.path.dirname(__file__))
@@ -782,7 +783,12 @@ def report(tensors, host: torch.Tensor) -> None:
 
 
 def host_max_displacement(positions, reference) -> float:
-    """Squared, for two contiguous fp64 numpy arrays [N, 3]."""
+    """Squared, for two contiguous fp64 numpy arrays [N, 3] (the library reads as many rows of both as the first has)."""
+    for name, a in (("positions", positions), ("reference", reference)):
+        if a.ndim != 2 or a.shape[1] != 3 or a.dtype != np.float64 or not a.flags.c_contiguous:
+            raise CudaMaceError("host_max_displacement: %s must be a contiguous fp64 array [N, 3] (got %s %s)" % (name, a.dtype, a.shape))
+    if positions.shape != reference.shape:
+        raise CudaMaceError("host_max_displacement: positions and reference differ in shape")
     return lib.cm_host_max_displacement(positions.ctypes.data, reference.ctypes.data, positions.shape[0])
 
 

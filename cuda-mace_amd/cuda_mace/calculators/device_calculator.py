@@ -96,9 +96,14 @@ class DeviceCalculator:
         anyway; the displacement test is then made there and nothing waits for the GPU (up to 4 096 atoms, where it costs
         less than the round trip)."""
         positions = positions.detach().double().contiguous()
-        self.steps += 1
         if host_positions is not None:
-            host_positions = np.ascontiguousarray(host_positions, dtype=np.float64) if host_positions.shape[0] <= 4096 else None
+            if host_positions.shape[0] > 4096:
+                host_positions = None
+            elif host_positions.shape != tuple(positions.shape):
+                raise ValueError("host_positions %s must have the shape of the positions, %s" % (host_positions.shape, tuple(positions.shape)))
+            else:
+                host_positions = np.ascontiguousarray(host_positions, dtype=np.float64)
+        self.steps += 1
         if self._ref_positions is None or self._ref_positions.shape != positions.shape:
             return self._on_fresh_list(positions, host_positions)
         limit = 0.5 * self.skin

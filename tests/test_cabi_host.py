@@ -244,3 +244,20 @@ def test_header_is_valid_c_and_cpp(tmp_path):
         res = subprocess.run([exe, std, "-pedantic", "-Wall", "-Werror", "-fsyntax-only", "-I" + os.path.join(ROOT, "include"),
                               str(src)], capture_output=True, text=True, timeout=120)
         assert res.returncode == 0, res.stderr
+
+
+def test_displacement_on_the_host_refuses_arrays_it_would_misread():
+    """The library is handed two addresses and one number of rows: what is no contiguous fp64 [N, 3] of the same N in both is
+    refused before that."""
+    import numpy as np
+    import pytest
+    from cuda_mace import _cabi
+
+    four, six = np.zeros((4, 3)), np.zeros((6, 3))
+    six[5, 0] = 2.0
+    assert _cabi.host_max_displacement(six, np.zeros((6, 3))) == 4.0
+    for positions, reference in ((six, four), (four, six), (four.reshape(-1), four), (four, four.reshape(-1)), (four.reshape(-1), four.reshape(-1)),
+                                 (np.zeros((4, 6))[:, ::2], four), (four, np.zeros((8, 3))[::2]), (four, np.asfortranarray(six[:4])),
+                                 (four.astype(np.float32), four), (four, four.astype(">f8")), (four, four.reshape(3, 4))):
+        with pytest.raises(_cabi.CudaMaceError):
+            _cabi.host_max_displacement(positions, reference)

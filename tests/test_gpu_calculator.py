@@ -314,3 +314,28 @@ def test_stress_of_the_step_is_that_of_its_virials(cabi):
         one = dict(data, cell=cells[0])
         shared = model(one, compute_stress=True)
         assert torch.equal(shared["stress"], cabi.stress_of(shared["virials"], cells[:1].expand_as(shared["virials"]).contiguous()))
+
+
+def test_host_positions_of_another_shape_are_refused(cabi):
+    """At the call that builds the list and at a later one; the calculator goes on with the list that it has."""
+    from cuda_mace.calculators import DeviceCalculator
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.synthetic import make_system, to_device
+
+    n = 40
+    data = to_device(make_system(n, 2, seed=3, density=None, cluster_box=9.0), "cuda")
+    upstream = SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6), avg_num_neighbors=20.0, seed=4)
+    calc = DeviceCalculator(OptimizedInvariantMACE(upstream, device="cuda"), data["node_attrs"], skin=0.5)
+    pos = data["positions"].double()
+    host = pos.cpu().numpy()
+    wrong = (host.reshape(-1), host[:-1], host.repeat(2, axis=0), host[:, :2], host[None])
+    for bad in wrong:
+        with pytest.raises(ValueError):
+            calc.compute(pos, host_positions=bad)
+    assert calc.steps == 0 and calc.builds == 0
+    first = calc.compute(pos, host_positions=host)
+    for bad in wrong:
+        with pytest.raises(ValueError):
+            calc.compute(pos, host_positions=bad)
+    again = calc.compute(pos, host_positions=host.T.copy().T)  # another layout of the same values
+    assert calc.steps == 2 and calc.builds == 1 and torch.equal(first["forces"], again["forces"])
