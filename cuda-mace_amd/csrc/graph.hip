@@ -190,7 +190,8 @@ __global__ void relabel_nodes_kernel(const int32_t *__restrict__ keys, const int
 // the sums have 64, and no offset lies beyond the list.
 __global__ __launch_bounds__(kScanThreads) void edge_offsets_kernel(const int32_t *__restrict__ degree, const int32_t *__restrict__ sent, int n,
                                                                     int64_t nedges, int32_t *__restrict__ first_occ,
-                                                                    int32_t *__restrict__ sender_offsets, int32_t *__restrict__ cursor) {
+                                                                    int32_t *__restrict__ sender_offsets, int32_t *__restrict__ cursor,
+                                                                    int32_t *__restrict__ long_bucket) {
   __shared__ int64_t part[kScanThreads];
   __shared__ int64_t stage[kScanStage / 2];
   const bool by_sender = blockIdx.x == 1;
@@ -201,6 +202,7 @@ __global__ __launch_bounds__(kScanThreads) void edge_offsets_kernel(const int32_
       [&](int k, int64_t before, int64_t value) {
         if (by_sender) {
           sender_offsets[k] = cursor[k] = within(before);
+          if (value > kBucketLds) *long_bucket = 1;
         } else {
           first_occ[k] = within(before);
           first_occ[n + k] = within(before + value);
@@ -279,30 +281,49 @@ __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__rest
   }
 }
 
-// One wave per sender: its pairs in the order of the new list.  Slots that no pair took (a list that is not sorted by row
-// i) name pair 0.
+// Workgroups [0, sender_blocks), a wave per sender: its pairs in the order of the new list.  Slots that no pair took (a list that
+// is not sorted by row i) name pair 0.  A bucket that does not fit a wave's LDS is left to the other workgroups, a thread per slot, which
+// leave at once where there is none (long_bucket): one wave would take the square of its pairs, in a row.  The whole call, us, a list of 160 000
+// pairs in which one of 20 000 atoms sends 1 000 / 5 000 / 20 000 of them: by waves alone 1 201 / 27 400 / 438 000, so 111 / 282 / 946; every atom
+// sends about 400, 200 atoms 413 -> 207; none that many, 12 000 atoms x 40 105.0 -> 105.2, 25 000 x 85 301.3 -> 300.8.
 __global__ __launch_bounds__(kThreads) void rank_senders_kernel(const int32_t *__restrict__ sender_offsets, const int32_t *__restrict__ cursor,
-                                                                const int32_t *__restrict__ bucketed, int nnodes, int32_t *__restrict__ perm) {
+                                                                const int32_t *__restrict__ bucketed, const int32_t *__restrict__ sender,
+                                                                const int32_t *__restrict__ long_bucket, int sender_blocks, int nnodes,
+                                                                int64_t nedges, int32_t *__restrict__ perm) {
+  if (static_cast<int>(blockIdx.x) >= sender_blocks) {
+    if (*long_bucket == 0) return;
+    const int64_t step = static_cast<int64_t>(gridDim.x - sender_blocks) * kThreads;
+    for (int64_t p = static_cast<int64_t>(blockIdx.x - sender_blocks) * kThreads + threadIdx.x; p < nedges; p += step) {
+      const int mine = bucketed[p];  // anything where no pair took the slot, which then lies in no sender's range
+      if (static_cast<uint64_t>(static_cast<int64_t>(mine)) >= static_cast<uint64_t>(nedges)) continue;
+      const int a = sender[mine];
+      if (static_cast<unsigned>(a) >= static_cast<unsigned>(nnodes)) continue;
+      const int lo = sender_offsets[a], end = sender_offsets[a + 1], hi = min(cursor[a], end);
+      if (p < lo || p >= hi || end - lo <= kBucketLds) continue;
+      int rank = 0;
+#pragma unroll 8
+      for (int q = lo; q < hi; ++q) rank += bucketed[q] < mine ? 1 : 0;
+      perm[lo + rank] = mine;
+    }
+    return;
+  }
   __shared__ int stage[kWaves][kBucketLds];
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int a = blockIdx.x * kWaves + w;
   const int lo = a < nnodes ? sender_offsets[a] : 0, end = a < nnodes ? sender_offsets[a + 1] : 0;
   const int hi = a < nnodes ? min(cursor[a], end) : 0;
-  const bool in_lds = hi - lo <= kBucketLds;
-  if (in_lds)
+  const bool here = end - lo <= kBucketLds;
+  if (here)
     for (int p = lo + lane; p < hi; p += kWave) stage[w][p - lo] = bucketed[p];
   __syncthreads();
-  for (int p = lo + lane; p < hi; p += kWave) {
-    const int mine = bucketed[p];
-    int rank = 0;
-    if (in_lds) {
+  if (here)
+    for (int p = lo + lane; p < hi; p += kWave) {
+      const int mine = stage[w][p - lo];
+      int rank = 0;
 #pragma unroll 4
       for (int q = 0; q < hi - lo; ++q) rank += stage[w][q] < mine ? 1 : 0;
-    } else {
-      for (int q = lo; q < hi; ++q) rank += bucketed[q] < mine ? 1 : 0;
+      perm[lo + rank] = mine;
     }
-    perm[lo + rank] = mine;
-  }
   for (int p = hi + lane; p < end; p += kWave) perm[p] = 0;
 }
 
@@ -348,7 +369,7 @@ inline size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255);
 
 struct PrepareLayout {
   Box *boxes;
-  int32_t *counters, *atoms_of_key, *old_first_occ, *pairs_of_sender;  // the last three are cleared together
+  int32_t *counters, *long_bucket, *atoms_of_key, *old_first_occ, *pairs_of_sender;  // the last four are cleared together
   int64_t ncounters;
   int32_t *atom_keys, *bin_offsets, *bin_cursor, *binned, *degree, *sent, *sender_cursor, *bucketed;
   unsigned long long *edge_key;
@@ -362,10 +383,11 @@ struct PrepareLayout {
     };
     auto ints = [&](int64_t n) { return reinterpret_cast<int32_t *>(take(static_cast<size_t>(n) * 4)); };
     boxes = reinterpret_cast<Box *>(take(kMaxBoxes * sizeof(Box)));
-    ncounters = nkeys + 3 * N;
+    ncounters = 1 + nkeys + 3 * N;
     counters = ints(ncounters);
-    atoms_of_key = counters;
-    old_first_occ = counters + nkeys;
+    long_bucket = counters;
+    atoms_of_key = long_bucket + 1;
+    old_first_occ = atoms_of_key + nkeys;
     pairs_of_sender = old_first_occ + 2 * N;
     atom_keys = ints(N);
     bin_offsets = ints(nkeys + 1);
@@ -419,7 +441,7 @@ int prepare(const double *positions, const int32_t *row_i, const int32_t *row_j,
   const unsigned gn = static_cast<unsigned>(ceil_div(nnodes, kThreads)), ge = static_cast<unsigned>(ceil_div(nedges, kThreads));
   if (nnodes > 0) {
     // atoms by bin; old CSR and pairs per sender
-    const int64_t ncounters = known_first_occ ? nkeys : L.ncounters;
+    const int64_t ncounters = known_first_occ ? 1 + nkeys : L.ncounters;
     const int nboxes = static_cast<int>(std::min<int64_t>(ceil_div(nnodes, 4 * kThreads), kMaxBoxes));
     const unsigned clears = static_cast<unsigned>(std::min<int64_t>(ceil_div(ncounters, 4 * kThreads), 1024));
     hipLaunchKernelGGL(box_and_clear_kernel, dim3(nboxes + clears), block, 0, st, positions, nnodes, nboxes, L.boxes, L.counters, ncounters);
@@ -432,13 +454,14 @@ int prepare(const double *positions, const int32_t *row_i, const int32_t *row_j,
                        known_first_occ ? static_cast<const int32_t *>(nullptr) : L.pairs_of_sender, N, nedges, node_perm, node_inverse, L.degree, L.sent);
   }
   hipLaunchKernelGGL(edge_offsets_kernel, dim3(2), dim3(kScanThreads), 0, st, L.degree, L.sent, N, nedges, first_occ, sender_offsets,
-                     L.sender_cursor);
+                     L.sender_cursor, L.long_bucket);
   if (nedges > 0) {
     hipLaunchKernelGGL(place_edges_kernel, dim3(static_cast<unsigned>(nnodes)), dim3(kWave), 0, st, positions, node_perm, node_inverse,
                        old_first_occ, first_occ, row_i, row_j, shifts, r_max, L.edge_key, N, nedges, receiver, sender, edge_perm, shifts_out,
                        sender_offsets, L.sender_cursor, L.bucketed);
-    hipLaunchKernelGGL(rank_senders_kernel, dim3(static_cast<unsigned>(ceil_div(nnodes, kWaves))), block, 0, st, sender_offsets,
-                       L.sender_cursor, L.bucketed, N, sender_perm);
+    const unsigned sender_blocks = static_cast<unsigned>(ceil_div(nnodes, kWaves));
+    hipLaunchKernelGGL(rank_senders_kernel, dim3(sender_blocks + std::min(ge, 1024u)), block, 0, st, sender_offsets, L.sender_cursor, L.bucketed, sender,
+                       L.long_bucket, static_cast<int>(sender_blocks), N, nedges, sender_perm);
   }
   return check_launch(what);
 }

@@ -354,6 +354,33 @@ def test_graph_prepare_long_segments(cabi, degrees):
     assert int(got["sender_offsets"][-1]) == counted and torch.equal(got["sender_perm"].cpu()[:counted].long(), want)
 
 
+@pytest.mark.parametrize("sent,N,degree", [(256, 40, 20), (257, 40, 20), (20000, 3000, 100)])
+def test_graph_prepare_long_buckets(cabi, sent, N, degree):
+    """Some atoms send exactly `sent` pairs: as many as a wave ranks on chip, one more, and more than the slots that one round of
+    threads takes, against the numpy restatement; and with names out of range, whose slots no pair takes."""
+    from oracle import ops as O
+    from tests.util import spatial_order_reference
+
+    g = torch.Generator().manual_seed(sent)
+    pos = 15.0 * torch.rand(N, 3, generator=g, dtype=torch.float64)
+    E = N * degree
+    rcv = torch.arange(N).repeat_interleave(degree)
+    snd = torch.randint(3, N, (E,), generator=g)
+    snd[torch.randperm(E, generator=g)[:2 * sent]] = torch.tensor([0, 2]).repeat(sent)
+    shifts = torch.zeros(E, 3, dtype=torch.float64)
+    got = cabi.graph_prepare(pos.cuda(), rcv.int().cuda(), snd.int().cuda(), shifts.cuda(), None, 1, 5.0, 6)
+    _, inverse, new_rcv, new_snd, order = spatial_order_reference(pos, torch.zeros(N, dtype=torch.int64), torch.stack([rcv, snd]), shifts, 5.0, 6)
+    for name, want in (("receiver", new_rcv), ("sender", new_snd), ("edge_perm", order)):
+        np.testing.assert_array_equal(got[name].cpu().numpy(), want, err_msg=name)
+    sperm, soff = O.stable_key_sort(torch.from_numpy(new_snd).int(), N)
+    assert torch.equal(got["sender_perm"].cpu(), sperm) and torch.equal(got["sender_offsets"].cpu(), soff)
+    lost = torch.randperm(E, generator=g)[:50]
+    snd[lost] = N + 1
+    got = cabi.graph_prepare(pos.cuda(), rcv.int().cuda(), snd.int().cuda(), shifts.cuda(), None, 1, 5.0, 6)
+    want = torch.sort(got["sender"].cpu(), stable=True).indices[:E - 50]
+    assert int(got["sender_offsets"][-1]) == E - 50 and torch.equal(got["sender_perm"].cpu()[:E - 50].long(), want)
+
+
 @pytest.mark.parametrize("n,ne", [(0, 3), (1, 1), (255, 2), (256, 63), (257, 10), (5000, 4)])
 def test_element_groups_and_gathered_rows(cabi, n, ne):
     """Both groupings against the sorts they stand for, with rows that hold no one, two ones or other values and with types out
