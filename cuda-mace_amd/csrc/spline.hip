@@ -500,9 +500,12 @@ __device__ __forceinline__ void std_out(double *p, typename Doubles<VEC>::type v
   else
     __builtin_nontemporal_store(v, reinterpret_cast<dv *>(p));
 }
-// us for a layer of the op modules, past the caches -> through them: 61 MB of rows 219 -> 217, 307 MB 469 -> 464, 328 MB 533 -> 527, 369 MB 570 -> 571, 410 MB
-// 715 -> 738, 460 MB 721 -> 734
-constexpr int64_t kKeepBytes = int64_t{320} << 20;
+// This kernel and the message passing after it, us, past the caches -> through them, 12 and 40 edges per node: 60 MB of rows, 32 channels 48.2 -> 48.2 and 36.1 -> 36.1,
+// 64 37.2 -> 36.9 and 36.6 -> 36.2, 128 34.8 -> 34.1 and 37.3 -> 36.1, 192 40.4 -> 38.3 and 40.6 -> 40.0, 256 43.9 -> 40.5 and 43.3 -> 42.6; 20 MB the same to
+// 3 less.  The wider the row the more this kernel itself loses (75 MB, 256 channels 21.9 -> 27.1), and from there on it is more than the next one gains: 75 MB, 64 channels
+// 44.1 -> 43.4, 160 42.0 -> 45.3, 256 49.3 -> 54.3; 90 MB, 64 43.9 -> 45.5, 128 48.4 -> 50.2, 256 56.2 -> 64.3; 120 MB, 64 62.1 -> 66.4, 256 64.4 -> 75.2; 200 MB,
+// 64 84.0 -> 82.3, 128 87.3 -> 90.8, 192 90.7 -> 104.9; 300 MB, 64 127 -> 122, 192 130 -> 145, 256 142 -> 165.
+constexpr int64_t kKeepBytes = int64_t{64} << 20;
 
 template <int VEC, bool KEEP>
 __global__ __launch_bounds__(256) void spline_forward_f64_wave_kernel(const double *__restrict__ r, const double *__restrict__ r_knots,

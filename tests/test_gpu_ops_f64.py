@@ -194,9 +194,9 @@ def test_spline_f64_more_edges_than_waves_in_a_launch(cabi):
     assert float(out[(r > 5.0)].abs().max()) == 0.0
 
 
-@pytest.mark.parametrize("E", [40_960, 40_961])
+@pytest.mark.parametrize("E", [8_192, 8_193, 40_960, 40_961])
 def test_spline_f64_rows_through_and_past_the_caches(cabi, E):
-    """On both sides of the rule on the size of the rows (320 MB): the values are those of a call on some of the edges."""
+    """On both sides of the rule on the size of the rows (64 MiB), and far beyond: the values are those of a call on some of the edges."""
     g = torch.Generator().manual_seed(E)
     knots = torch.linspace(0.0, 6.0, 64, dtype=F64, device=DEV)
     coeffs = torch.randn(63, 4, 1024, generator=g, dtype=F64).to(DEV)
