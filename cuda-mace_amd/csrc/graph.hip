@@ -31,6 +31,7 @@ constexpr int kMaxBoxes = 64;  // partial bounding boxes; a wave reduces them
 constexpr int kScanThreads = 1024;
 constexpr int kScanStage = 32 * 1024;  // values staged in LDS at a time (128 KB)
 constexpr int kSegLds = 512;   // keys of a segment that a wave keeps in LDS
+constexpr int kSegKeys = 4;    // keys of a longer one that a lane ranks at a time
 constexpr int kBucketLds = 256;  // pairs of one sender that a wave keeps in LDS
 
 // What bounds the whole call is the launches: each holds microseconds of work that waits for the one before.  There are eight
@@ -213,9 +214,12 @@ __global__ __launch_bounds__(kScanThreads) void edge_offsets_kernel(const int32_
 
 // One wave per new atom: keys of the pairs of its segment (pairs within the cutoff by the new label of atom j, the others
 // behind them by length: the bit pattern of a non-negative double orders like its value), their ranks by (key, position in
-// the list), the pairs at their places, and each into its sender's bucket in any order.  Keys of more pairs than LDS holds
-// go through `key`.  Of a list that is not sorted by row i, an atom has the pairs that find a place, and others stay without: none is
-// written out of range.
+// the list), the pairs at their places, and each into its sender's bucket in any order.  Of a list that is not sorted by row i, an atom
+// has the pairs that find a place, and others stay without: none is written out of range.
+// Keys of more pairs than LDS holds go through `key`, and from there through LDS piece by piece, each read by a lane for several of its
+// keys.  The whole call, us, every key read from memory for every pair -> that: 200 atoms x 600 pairs 718 -> 423, 1 000 x 900 1 852 -> 990, 5 000 x
+// 900 4 359 -> 2 055.  (1 024 keys in LDS are faster up to that number, 342, 862 and 2 050, and make every other list slower: half as many waves to a
+// unit, 12 000 x 40 105 -> 106.4, 100 000 x 4 413 -> 438.)
 __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__restrict__ pos, const int32_t *__restrict__ perm,
                                                             const int32_t *__restrict__ inverse, const int32_t *__restrict__ old_first_occ,
                                                             const int32_t *__restrict__ new_first_occ, const int32_t *__restrict__ row_i,
@@ -250,34 +254,59 @@ __global__ __launch_bounds__(kWave) void place_edges_kernel(const double *__rest
       key[e] = k;
   }
   __syncthreads();
-  for (int k = lane; k < d; k += kWave) {
+  struct Pair {
+    int j;
+    double shift[3];
+  };
+  const auto pair_of = [&](int k) {
     const int64_t e = s0 + k;
-    const unsigned long long mine = in_lds ? sk[k] : key[e];
-    const int j = row_j[e];
-    const double s[3] = {shifts[3 * e + 0], shifts[3 * e + 1], shifts[3 * e + 2]};
-    int rank = 0;
-    if (in_lds) {
-#pragma unroll 4
-      for (int t = 0; t < d; ++t) rank += (sk[t] < mine || (sk[t] == mine && t < k)) ? 1 : 0;
-    } else {
-      for (int t = 0; t < d; ++t) {
-        const unsigned long long other = key[s0 + t];
-        rank += (other < mine || (other == mine && t < k)) ? 1 : 0;
-      }
-    }
+    return Pair{row_j[e], {shifts[3 * e + 0], shifts[3 * e + 1], shifts[3 * e + 2]}};
+  };
+  const auto place = [&](int k, int rank, const Pair &pair) {
     const int64_t at = base + rank;
+    const int j = pair.j;
     const bool named = static_cast<unsigned>(j) < static_cast<unsigned>(nnodes);
     const int s_new = named ? inverse[j] : j;
     receiver[at] = a;
     sender[at] = s_new;
-    edge_perm[at] = static_cast<int32_t>(e);
-    shifts_out[3 * at + 0] = s[0];
-    shifts_out[3 * at + 1] = s[1];
-    shifts_out[3 * at + 2] = s[2];
+    edge_perm[at] = s0 + k;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) shifts_out[3 * at + c] = pair.shift[c];
     if (named) {
       const int to = atomicAdd(&cursor[s_new], 1);
       if (to < sender_offsets[s_new + 1]) bucketed[to] = static_cast<int32_t>(at);
     }
+  };
+  if (in_lds) {
+    for (int k = lane; k < d; k += kWave) {
+      const unsigned long long mine = sk[k];
+      const Pair pair = pair_of(k);  // on its way meanwhile
+      int rank = 0;
+#pragma unroll 4
+      for (int t = 0; t < d; ++t) rank += (sk[t] < mine || (sk[t] == mine && t < k)) ? 1 : 0;
+      place(k, rank, pair);
+    }
+    return;
+  }
+  for (int first = 0; first < d; first += kSegKeys * kWave) {
+    unsigned long long mine[kSegKeys];
+    int rank[kSegKeys];
+#pragma unroll
+    for (int u = 0; u < kSegKeys; ++u) mine[u] = key[s0 + min(first + u * kWave + lane, d - 1)], rank[u] = 0;
+    for (int from = 0; from < d; from += kSegLds) {
+      const int cnt = min(kSegLds, d - from);
+      __syncthreads();  // the piece before has been read
+      for (int t = lane; t < cnt; t += kWave) sk[t] = key[s0 + from + t];
+      __syncthreads();
+      for (int t = 0; t < cnt; ++t) {
+        const unsigned long long other = sk[t];
+#pragma unroll
+        for (int u = 0; u < kSegKeys; ++u) rank[u] += (other < mine[u] || (other == mine[u] && from + t < first + u * kWave + lane)) ? 1 : 0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSegKeys; ++u)
+      if (const int k = first + u * kWave + lane; k < d) place(k, rank[u], pair_of(k));
   }
 }
 

@@ -325,7 +325,7 @@ def test_graph_prepare_matches_the_host_restatement(cabi, case):
             assert bool((seg[1:] >= seg[:-1]).all())
 
 
-@pytest.mark.parametrize("degrees", [(512, 513, 0, 64, 65, 1), (1500, 2)])
+@pytest.mark.parametrize("degrees", [(512, 513, 0, 64, 65, 1), (1500, 2), (1024, 768, 1025)])
 def test_graph_prepare_long_segments(cabi, degrees):
     """cm_graph_prepare where a segment or a sender's bucket is longer than what a wave keeps on chip (512 keys, 256 pairs), on a
     list in which a pair has no reverse and names of atoms out of range occur, against the numpy restatement."""
