@@ -93,7 +93,8 @@ __global__ __launch_bounds__(kThreads) void box_and_clear_kernel(const double *_
   }
 }
 
-// Workgroups [0, node_blocks), a thread per atom: key = ((graph * bins + bx) * bins + by) * bins + bz, and the atoms per key.
+// Workgroups [0, node_blocks), a thread per atom: key = ((graph * bins + bx) * bins + by) * bins + bz, and the atoms per key
+// (atoms_of_key NULL: not asked for).
 // The others, a thread per pair: the old CSR (a change of the value of row_i closes every atom before it and opens every
 // atom up to it, values out of range counting as the nearest atom) and the pairs per atom j.
 __global__ __launch_bounds__(kThreads) void count_kernel(const double *__restrict__ pos, const int32_t *__restrict__ graph_of_node, int nnodes,
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(kThreads) void count_kernel(const double *__restric
   g = g < 0 ? 0 : (g >= ngraphs ? ngraphs - 1 : g);
   const int key = ((g * bins + b[0]) * bins + b[1]) * bins + b[2];
   keys[i] = key;
-  atomicAdd(&atoms_of_key[key], 1);
+  if (atoms_of_key) atomicAdd(&atoms_of_key[key], 1);
 }
 
 // One workgroup: offsets of the bins, and a copy of them that counts up while the bins are filled.
@@ -165,18 +166,22 @@ __global__ void bin_atoms_kernel(const int32_t *__restrict__ keys, int nnodes, i
 }
 
 // The atoms of a bin in the order of their indices: perm and its inverse; under the new label, the length of the atom's
-// segment and the pairs it sends (pairs_of_sender NULL: as many as it receives).
+// segment and the pairs it sends (pairs_of_sender NULL: as many as it receives).  binned NULL: perm is there.
 __global__ void relabel_nodes_kernel(const int32_t *__restrict__ keys, const int32_t *__restrict__ binned, const int32_t *__restrict__ offsets,
                                      const int32_t *__restrict__ old_first_occ, const int32_t *__restrict__ pairs_of_sender, int nnodes,
                                      int64_t nedges, int32_t *__restrict__ perm, int32_t *__restrict__ inverse, int32_t *__restrict__ degree,
                                      int32_t *__restrict__ sent) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nnodes) return;
-  const int o = binned[p], key = keys[o];
-  const int lo = offsets[key], hi = offsets[key + 1];
-  int rank = 0;
-  for (int q = lo; q < hi; ++q) rank += binned[q] < o ? 1 : 0;
-  const int a = lo + rank;
+  int a = p, o;
+  if (binned) {
+    o = binned[p];
+    const int key = keys[o], lo = offsets[key], hi = offsets[key + 1];
+    a = lo;
+    for (int q = lo; q < hi; ++q) a += binned[q] < o ? 1 : 0;
+  } else {
+    o = perm[p];
+  }
   perm[a] = o;
   inverse[o] = a;
   int e0 = old_first_occ[o], e1 = old_first_occ[nnodes + o];
@@ -396,13 +401,20 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(RowArrays a, cons
 
 inline size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
+// Few bins of many atoms: an atom's rank in its bin takes as many reads as the bin has atoms, and all atoms count in a few places.  The sort
+// for few keys (sort.hip), which it takes where this holds, ranks within 256 atoms instead.  The whole call, us, that -> this: 4 096 atoms in one bin 436 -> 49,
+// in 27 65 -> 47, in 64 53 -> 49; 8 191 in 64 78 -> 49, 20 000 in one 2 005 -> 64, in 64 148 -> 67, 100 000 in one 9 940 -> 181, in 64 620 -> 192.
+inline bool many_atoms_per_key(int64_t nnodes, int64_t nkeys) { return nkeys <= 64 && nnodes >= 4096; }
+
 struct PrepareLayout {
   Box *boxes;
   int32_t *counters, *long_bucket, *atoms_of_key, *old_first_occ, *pairs_of_sender;  // the last four are cleared together
   int64_t ncounters;
   int32_t *atom_keys, *bin_offsets, *bin_cursor, *binned, *degree, *sent, *sender_cursor, *bucketed;
   unsigned long long *edge_key;
-  size_t bytes;
+  bool many_per_key;
+  void *sort;  // many_per_key alone
+  size_t sort_bytes, bytes;
   PrepareLayout(void *base, int64_t N, int64_t E, int64_t nkeys) {
     size_t at = 0;
     auto take = [&](size_t n) {
@@ -427,6 +439,9 @@ struct PrepareLayout {
     sender_cursor = ints(N);
     bucketed = ints(E);
     edge_key = reinterpret_cast<unsigned long long *>(take(static_cast<size_t>(E) * 8));
+    many_per_key = many_atoms_per_key(N, nkeys);
+    sort_bytes = many_per_key ? cm_stable_key_sort_workspace(N, nkeys) : 0;
+    sort = take(sort_bytes);
     bytes = at;
   }
 };
@@ -475,11 +490,17 @@ int prepare(const double *positions, const int32_t *row_i, const int32_t *row_j,
     const unsigned clears = static_cast<unsigned>(std::min<int64_t>(ceil_div(ncounters, 4 * kThreads), 1024));
     hipLaunchKernelGGL(box_and_clear_kernel, dim3(nboxes + clears), block, 0, st, positions, nnodes, nboxes, L.boxes, L.counters, ncounters);
     hipLaunchKernelGGL(count_kernel, dim3(gn + (known_first_occ ? 0 : ge)), block, 0, st, positions, graph_of_node, N, static_cast<int>(gn), L.boxes, nboxes,
-                       0.5 * r_max, bins, ngraphs, L.atom_keys, L.atoms_of_key, row_i, row_j, nedges, L.old_first_occ, L.pairs_of_sender);
-    hipLaunchKernelGGL(bin_offsets_kernel, dim3(1), dim3(kScanThreads), 0, st, L.atoms_of_key, static_cast<int>(nkeys), L.bin_offsets,
-                       L.bin_cursor);
-    hipLaunchKernelGGL(bin_atoms_kernel, dim3(gn), block, 0, st, L.atom_keys, N, L.bin_cursor, L.binned);
-    hipLaunchKernelGGL(relabel_nodes_kernel, dim3(gn), block, 0, st, L.atom_keys, L.binned, L.bin_offsets, old_first_occ,
+                       0.5 * r_max, bins, ngraphs, L.atom_keys, L.many_per_key ? static_cast<int32_t *>(nullptr) : L.atoms_of_key, row_i, row_j, nedges,
+                       L.old_first_occ, L.pairs_of_sender);
+    if (L.many_per_key) {
+      if (const int rc = cm_stable_key_sort(L.atom_keys, nnodes, nkeys, node_perm, L.bin_offsets, L.sort, L.sort_bytes, stream); rc != CM_OK) return rc;
+    } else {
+      hipLaunchKernelGGL(bin_offsets_kernel, dim3(1), dim3(kScanThreads), 0, st, L.atoms_of_key, static_cast<int>(nkeys), L.bin_offsets,
+                         L.bin_cursor);
+      hipLaunchKernelGGL(bin_atoms_kernel, dim3(gn), block, 0, st, L.atom_keys, N, L.bin_cursor, L.binned);
+    }
+    hipLaunchKernelGGL(relabel_nodes_kernel, dim3(gn), block, 0, st, L.atom_keys, L.many_per_key ? static_cast<const int32_t *>(nullptr) : L.binned,
+                       L.bin_offsets, old_first_occ,
                        known_first_occ ? static_cast<const int32_t *>(nullptr) : L.pairs_of_sender, N, nedges, node_perm, node_inverse, L.degree, L.sent);
   }
   hipLaunchKernelGGL(edge_offsets_kernel, dim3(2), dim3(kScanThreads), 0, st, L.degree, L.sent, N, nedges, first_occ, sender_offsets,
