@@ -250,18 +250,18 @@ def graph_prepare(positions: torch.Tensor, row_i: torch.Tensor, row_j: torch.Ten
 
 
 def gather_rows(perm: torch.Tensor, *tensors: torch.Tensor):
-    """Rows `perm` (a permutation, int32 [N]) of each tensor, all with N rows, in one launch; no graph is recorded.  Tensors in
-    host memory are gathered there."""
+    """Rows `perm` (a permutation, int32 [N]) of each tensor in one launch; no graph is recorded.  Rows behind the first N are left
+    out, as index_select leaves them.  Tensors in host memory are gathered there."""
     n = perm.numel()
     if not perm.is_cuda:
         return [t.detach().index_select(0, perm) for t in tensors]
     src = [t.detach().contiguous() for t in tensors]
     for t in src:
-        if not t.is_cuda or t.dim() == 0 or t.shape[0] != n:
+        if not t.is_cuda or t.dim() == 0 or t.shape[0] < n:
             raise CudaMaceError("gather_rows: %s must live on the GPU with %d rows" % (tuple(t.shape), n))
-    out = [torch.empty_like(t) for t in src]
+    out = [torch.empty_like(t[:n]) for t in src]
     addresses = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])  # noqa: E731
-    sizes = (ctypes.c_int64 * len(src))(*[t.numel() // max(n, 1) * t.element_size() for t in src])
+    sizes = (ctypes.c_int64 * len(src))(*[t.numel() // max(n, 1) * t.element_size() for t in out])
     _check(lib.cm_gather_rows(_dev(perm, I32, "perm"), n, len(src), addresses(src), addresses(out), sizes, _stream()))
     return out
 

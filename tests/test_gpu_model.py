@@ -875,3 +875,21 @@ def test_a_list_first_seen_on_another_stream(cabi, atoms, relabel, native):
         torch.cuda.synchronize()
         for k in want[0]:
             assert torch.equal(a[k].detach(), want[0][k]) and torch.equal(b[k].detach(), want[0][k]) and torch.equal(c[k].detach(), want[1][k]), k
+
+
+def test_species_of_more_rows_than_atoms_over_many_lists(cabi):
+    """A one-hot matrix with rows behind those of the atoms is accepted where the atoms are relabelled, at the first list and at
+    every later one, and its further rows count for nothing."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.synthetic import make_system, to_device
+
+    n = 300
+    data = to_device(make_system(n, 4, seed=8, density=0.1), "cuda")
+    model = OptimizedInvariantMACE(SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=50.0, seed=9), device="cuda",
+                                   spatial_order_min_atoms=0)
+    want = model(dict(data))
+    longer = torch.cat([data["node_attrs"], data["node_attrs"][:7]])
+    for _ in range(4):
+        got = model(dict(data, edge_index=data["edge_index"].clone(), node_attrs=longer))
+        for name in ("energy", "node_energy", "forces", "node_feats"):
+            assert torch.equal(got[name], want[name]), name

@@ -424,6 +424,12 @@ def test_element_groups_and_gathered_rows(cabi, n, ne):
     arrays = [torch.randint(0, 127, (n, w), generator=g, dtype=torch.int8).cuda() for w in (1, 4, 8, 16, 31, 40)] + [types, one_hot.double().T.contiguous().T]
     for got, want in zip(cabi.gather_rows(perm, *arrays), arrays):
         assert torch.equal(got, want.index_select(0, perm))
+    more = [torch.cat([a, a[:1], a]) for a in arrays]  # rows behind the first n
+    for got, want in zip(cabi.gather_rows(perm, *more), arrays):
+        assert torch.equal(got, want.index_select(0, perm))
+    if n:
+        with pytest.raises(cabi.CudaMaceError):
+            cabi.gather_rows(perm, types[:-1])
 
 
 @pytest.mark.parametrize("n,pbc", [(1, False), (40, True), (700, True), (9000, False)])
