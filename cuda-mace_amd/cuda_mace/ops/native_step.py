@@ -137,8 +137,8 @@ class NativeStep:
 
     def __call__(self, handle: "_GraphHandle", positions: torch.Tensor, shifts: torch.Tensor, want_feats: bool = True,
                  want_virials: bool = False, want_forces: bool = True, cell: Optional[torch.Tensor] = None) -> Dict[str, torch.Tensor]:
-        """want_forces=False: the forward half alone (cm_mace_energy), "forces" and "virials" are None.  cell (one for all
-        graphs or one per graph): "stress" as well, which needs the virials."""
+        """want_forces=False: the forward half alone (cm_mace_energy), "forces", "virials" and "stress" are None.  cell (one for
+        all graphs or one per graph): "stress" as well, which needs the virials."""
         _found(positions, self, self._streams)
         N, E, ngraphs = handle.sizes
         C = self.channels
@@ -155,8 +155,8 @@ class NativeStep:
         node_energy = torch.empty(N, dtype=F64, device=dev)
         forces = torch.empty(N, 3, dtype=F64, device=dev) if want_forces else None
         feats = torch.empty(N, 2 * C, dtype=F64, device=dev) if want_feats else None
-        virials = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if want_virials else None
-        stress = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if cell is not None else None
+        virials = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if want_virials and want_forces else None
+        stress = torch.empty(ngraphs, 3, 3, dtype=F64, device=dev) if cell is not None and want_forces else None
         total = torch.empty(ngraphs, dtype=F64, device=dev)
         node_total = torch.empty(N, dtype=F64, device=dev)
         feats_at, virials_at = None if feats is None else feats.data_ptr(), None if virials is None else virials.data_ptr()

@@ -893,3 +893,16 @@ def test_species_of_more_rows_than_atoms_over_many_lists(cabi):
         got = model(dict(data, edge_index=data["edge_index"].clone(), node_attrs=longer))
         for name in ("energy", "node_energy", "forces", "node_feats"):
             assert torch.equal(got[name], want[name]), name
+
+
+def test_energies_alone_hold_no_gradient_that_was_not_formed(cabi):
+    """The step asked for energies alone returns None for virials and stress, whatever else it was asked for."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+
+    data = to_device(make_system(120, 4, seed=2, density=0.1), "cuda")
+    model = OptimizedInvariantMACE(SyntheticInvariantMACE(channels=32, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=50.0, seed=3), device="cuda")
+    full = model(dict(data), compute_stress=True)
+    handle, = (entry[2] for entry in data["edge_index"].__dict__["_cm_native_graphs"].values())
+    out = model._native(handle, data["positions"], data["shifts"], want_virials=True, want_forces=False, cell=data["cell"])
+    assert out["forces"] is None and out["virials"] is None and out["stress"] is None
+    assert torch.equal(out["node_energy"], full["node_energy"])
