@@ -1,6 +1,8 @@
-// Device code shared by the spline-fused message-passing kernels (mp_spline.hip, whose head has the formulas) and the kernels that
-// take a node through a whole layer (few_nodes.hip): the staging of a node's edges, a wave's part of the forward sum, and the
-// products of one edge of the backward pass.  Both sum in the same order and return the same bits.
+// Device code of the spline-fused message passing (mp_spline.hip, whose head has the formulas) and of the kernels that take a node
+// through a whole layer (few_nodes.hip).  Both use the staging of a node's edges, the operands and products of one edge of the backward pass and
+// the end of its vector gradient.  Staged, SlotSums and forward_wave are few_nodes.hip's alone: a second writing of the loop of
+// mp_spline_forward_kernel, which reads its knots and lays out its LDS otherwise and has variants that this one does not need.  Both sum in
+// the same order and must stay alike: the step of few nodes is compared with the separate launches bit for bit in the tests.
 #pragma once
 
 #include <type_traits>

@@ -179,10 +179,13 @@ inline bool two_nodes_per_wave(int channels, int64_t nnodes) {
 }
 // The gradient is read again in the backward pass only.  Written past the caches it leaves room for everything in between (25 %
 // faster at 25 000 x 128); where the whole of it is about as large as the L2s (32 MB) or somewhat more, the Infinity Cache still has most of it then,
-// and the backward linear reads it from there.  A step of forces at 25 neighbours upward, us, past the caches -> through them: 5 000 x 64 (20 MB)
-// 313 -> 304, 8 000 x 64 (33) 421 -> 409, 6 500 x 96 (40) 560 -> 546, 4 000 x 128 (33) 459 -> 451, 5 000 x 128 (41) 578 -> 563; below and above that
-// the other way: 2 000 x 96 (12) 241 -> 242, 1 000 x 128 (8) 202 -> 206, 12 000 x 64 (49) 579 -> 577, 900 molecules x 64 (77) 437 -> 444, 8 000 x 128
-// (66) 787 -> 795; beyond 128 channels at all sizes: 4 000 x 160 (41) 611 -> 616, 3 000 x 192 (37) 578 -> 589.
+// and the backward linear reads it from there.  A step of forces, us, past the caches -> through them, by the size of the gradient in MiB:
+//   32 channels   18 275.6 -> 274.4, 22 318.3 -> 317.5, 36 468.9 -> 463.6, 48 602.5 -> 601.5, 52 656.8 -> 658.2, 60 748 -> 762, 70 884 -> 923
+//   64            12 213.0 -> 212.8, 15 248.1 -> 247.9, 18 295.0 -> 290.3, 22 327.6 -> 321.7, 36 466.7 -> 456.6, 48 585.1 -> 578.2, 52 619.8 -> 616.0, 60 699.6 -> 698.9, 70 813.5 -> 818.7
+//   96            12 241.7 -> 243.3, 15 290.6 -> 293.6, 18 322.2 -> 322.5, 21 357.1 -> 354.4, 36 513.2 -> 502.4, 48 648.2 -> 634.5, 51 685.7 -> 677.8, 60 762.2 -> 767.7, 69 872.1 -> 886.4
+//   128           12 238.5 -> 240.6, 15 261.8 -> 262.3, 18 343.3 -> 338.1, 22 389.8 -> 378.8, 36 537.0 -> 527.3, 48 642.3 -> 632.0, 52 700.8 -> 691.4, 60 759.7 -> 768.9, 70 847.0 -> 862.8
+// (the upper line could lie at 52 for what it is worth at 64 to 128 channels); beyond 128 channels the other way at all sizes: 4 000 x 160 (41 MB) 611 -> 616,
+// 3 000 x 192 (37) 578 -> 589.
 inline bool gradient_stays_near(int64_t nnodes, int channels) {
   const int64_t bytes = nnodes * 16 * channels * 4;
   return channels <= 128 && bytes >= (int64_t{18} << 20) && bytes <= (int64_t{48} << 20);

@@ -640,6 +640,28 @@ def test_step_of_few_nodes_equals_the_separate_launches(cabi, case, channels, mo
         torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
+@pytest.mark.parametrize("knots,channels,nodes", [(2, 64, 130), (3, 128, 130), (4, 32, 130), (512, 96, 300), (513, 64, 130), (513, 128, 300), (800, 32, 600)])
+def test_step_of_few_nodes_with_any_number_of_knots(cabi, knots, channels, nodes, monkeypatch):
+    """The same where the knots do not lie in LDS (fewer than four, more than 512) and where they just do, with eight and with four waves
+    per node: forces, virials and energies alone are those of the separate launches to the bit, edges beyond the cutoff included."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.neighbour_list import neighbour_data
+
+    base = to_device(make_system(nodes, 4, seed=51, density=0.06), "cuda")
+    data = neighbour_data(base["positions"], base["node_attrs"], 5.6, (True, True, True), base["cell"])
+    up = SyntheticInvariantMACE(channels=channels, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=30.0, seed=52)
+    model = OptimizedInvariantMACE(up, device="cuda", num_spline_knots=knots)
+    for keys in ({"compute_virials": True}, {"compute_force": False}):
+        with torch.set_grad_enabled("compute_force" not in keys):
+            monkeypatch.delenv("CM_STEP_GLUE", raising=False)
+            a = model(dict(data), **keys)
+            monkeypatch.setenv("CM_STEP_GLUE", "-1")
+            b = model(dict(data), **keys)
+        for key in ("node_energy", "node_feats") + (("forces", "virials") if "compute_virials" in keys else ()):
+            assert torch.isfinite(a[key]).all() and torch.equal(a[key], b[key]), key
+    assert model._native not in (None, False)
+
+
 @pytest.mark.parametrize("channels", [32, 64, 96, 128, 160, 192, 224, 256])
 def test_repeated_evaluations_agree_bit_for_bit_at_every_width(cabi, channels):
     """Every kernel sums in a fixed order and reads nothing it (or an earlier kernel of the same step) has not written:

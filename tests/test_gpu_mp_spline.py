@@ -318,10 +318,14 @@ def test_mp_edge_backward_few_and_many_nodes(cabi, case):
     test_mp_edge_backward_of_four_edges_per_step(cabi, case)
 
 
-@pytest.mark.parametrize("case", [(1023, 9, 160, 0.1, 71, 256, 0), (1025, 9, 192, 0.0, 72, 256, 0), (2049, 7, 224, 0.1, 73, 256, 70)],
+@pytest.mark.parametrize("case", [(1023, 9, 160, 0.1, 71, 256, 0), (1025, 9, 192, 0.0, 72, 256, 0), (2049, 7, 224, 0.1, 73, 256, 70), (2047, 1, 160, 0.0, 74, 256, 0),
+                                  (511, 9, 160, 0.1, 75, 256, 0), (512, 9, 160, 0.0, 76, 256, 0), (513, 9, 160, 0.1, 77, 256, 0), (341, 9, 160, 0.0, 78, 256, 0),
+                                  (343, 9, 160, 0.1, 79, 256, 0)],
                          ids=lambda c: "N%d_d%d_C%d_k%d" % (c[0], c[1], c[2], c[5]))
 def test_mp_edge_backward_of_nodes_beyond_whole_runs(cabi, case):
-    """Nodes are dealt to the eight XCDs in runs of 128, those behind the last 1 024 one at a time."""
+    """Workgroups, a node's parts in order, are dealt to the eight XCDs in runs of 128, those behind the last 1 024 one at a time.
+    Just below and above a multiple of 1 024 workgroups with one part per node (1 025, 2 047, 2 049 nodes), with two (1 022, 1 024, 1 026 and
+    2 046 workgroups) and with three (1 023 and 1 029), where a run begins and ends inside a node."""
     test_mp_edge_backward_of_four_edges_per_step(cabi, case)
 
 
