@@ -795,6 +795,24 @@ int dispatch(int channels, int64_t nnodes, Call call) {
 
 }  // namespace
 
+// Edges per node up to which the step of few nodes is no slower than the separate launches.  A node has eight waves, or four, whatever its edges;
+// the separate launches cut them into as many parts as the chip has room for, and the fewer nodes share a round the more of it they leave
+// idle here.  Step in us, the separate launches -> these, edges per node:
+//   up to a node per unit   64   20 x 1 571 325 -> 305; 96 20 x 262 174 -> 169, x 524 197 -> 197, x 785 250 -> 269, 60 x 785 262 -> 272, 100 x 785 276 -> 273, x 1 152 362 -> 376,
+//                           150 x 1 571 490 -> 494, 256 x 1 571 543 -> 503; 128 20 x 524 228 -> 226, x 785 291 -> 303, 60 x 785 304 -> 303, 100 x 1 152 419 -> 416
+//   up to two               32   300 x 1 152 257 -> 253, x 1 571 321 -> 330; 64 300 x 785 305 -> 299, x 1 152 401 -> 410, 384 x 1 152 444 -> 415; 96 257 x 262 202 -> 199, x 367 238 -> 245,
+//                           320 x 367 262 -> 257, x 524 330 -> 338, 384 x 524 351 -> 342, x 785 472 -> 479; 128 257 x 262 240 -> 234, x 367 285 -> 292, 384 x 785 554 -> 551
+//   a second round          32   513 x 157 111 -> 110, x 209 127 -> 130, x 524 205 -> 243, 768 x 209 141 -> 138, x 262 161 -> 169, 1 024 x 262 175 -> 177; 64 513 x 79 123 -> 120, x 157
+//                           153 -> 164, x 524 317 -> 383, 640 x 105 140 -> 138, x 131 155 -> 158, 768 x 157 183 -> 181, x 209 207 -> 209; energies alone 32 768 x 209 67.0 ->
+//                           70.0, 1 024 x 209 75.0 -> 74.0, x 262 83.8 -> 85.5; 64 513 x 79 65.7 -> 56.0, 768 x 157 88.1 -> 88.2, x 209 98.3 -> 103.5
+static double most_edges_per_node(int channels, int64_t nnodes, bool forces) {
+  const double u = static_cast<double>(nnodes) / device_compute_units();
+  if (u <= 1.0) return channels <= 64 ? 2000.0 : 430.0 + 1100.0 * u;
+  if (u <= 2.0) return channels == 32 ? 1000.0 + 1400.0 * (u - 1.0) : (channels == 64 ? 700.0 + 1600.0 * (u - 1.0) : 290.0 + 600.0 * (u - 1.0));
+  const double v = u - 2.0;
+  return channels == 32 ? 155.0 + (forces ? 53.0 : 30.0) * v : 85.0 + (forces ? (40.0 + 70.0 * v) * v : 70.0 * v);
+}
+
 // Up to a node per compute unit a workgroup of eight waves has a unit to itself, up to two it has four waves and half of one; a second round of
 // those pays at 32 and 64 channels, whose weights are small.  Beyond, the launches that share weights between nodes are faster (and round
 // otherwise beyond few::applies: 384 nodes at 128 channels, 512 at 96, 768 at 64).  Step in us, the separate launches -> these:
@@ -803,9 +821,10 @@ int dispatch(int channels, int64_t nnodes, Call call) {
 //   96   21 x 9 82 -> 53, 256 x 52 116 -> 72, 500 x 52 138 -> 95, 504 x 9 115 -> 71
 //   128  21 x 9 92 -> 62, 216 x 92 141 -> 99, 256 x 52 136 -> 86, 384 x 52 155 -> 115, 378 x 9 132 -> 85
 // (eight waves to half of the nodes: 64 channels, 216 x 52, 51 against 55 with four.)
-bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges) {
+bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges, bool forces) {
   const int C = w.channels;
-  return C <= 128 && nnodes <= (C == 32 ? 4 : 3) * device_compute_units() && !w.mono3[0] && !w.mono2[0] && !w.mono3[1] && !w.mono2[1] && w.n3[0] == CM_SYMCON_N3 && w.n2[0] == CM_SYMCON_N2 &&
+  return C <= 128 && nnodes <= (C == 32 ? 4 : 3) * device_compute_units() && static_cast<double>(nedges) <= most_edges_per_node(C, nnodes, forces) * static_cast<double>(nnodes) &&
+         !w.mono3[0] && !w.mono2[0] && !w.mono3[1] && !w.mono2[1] && w.n3[0] == CM_SYMCON_N3 && w.n2[0] == CM_SYMCON_N2 &&
          w.n3[1] == CM_SYMCON_N3 && w.n2[1] == CM_SYMCON_N2 && few::applies(nnodes, 16, C) && few::applies(nnodes, 1, C) &&
          !sliced_forward_applies(nnodes, nedges, C, w.nknots);
 }

@@ -8,8 +8,8 @@
 namespace cm {
 namespace fewnodes {
 
-// Whether the step of this size takes a node through a whole layer per launch.
-bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges);
+// Whether the step of this size (forces, or energies alone) takes a node through a whole layer per launch.
+bool applies(const cm_mace_weights &w, int64_t nnodes, int64_t nedges, bool forces);
 
 // Where the step keeps what one launch leaves for the next (rows of the workspace; energies alone: the second line NULL).
 struct Scratch {

@@ -597,7 +597,7 @@ int run_step(const cm_mace_weights *w, const cm_mace_graph *g, const double *pos
   const char *glue_env = getenv("CM_STEP_GLUE");  // development switch: smallest node count that takes the chained kernels; -1: none
   const int glue_min = glue_env ? atoi(glue_env) : 0;
   // Few nodes: a workgroup takes a node through a whole layer (few_nodes.hip), three launches and the forces.
-  if (glue_min >= 0 && N >= glue_min && cm::fewnodes::applies(*w, N, E)) {
+  if (glue_min >= 0 && N >= glue_min && cm::fewnodes::applies(*w, N, E, want_forces)) {
     const cm::fewnodes::Scratch s{L.vec, L.X2, L.h1, L.sc, L.live, reinterpret_cast<int32_t *>(L.bufA), want_forces ? L.bufM1 : nullptr, L.d_h2,
                                   L.edge_scratch, L.gv1, L.gv2};
     CM_REQUIRE(w->hidden >= 1 && w->hidden <= cm::readout::kHidden, "cm_mace_step: hidden=%d must be in [1, %d]", w->hidden, cm::readout::kHidden);

@@ -640,6 +640,33 @@ def test_step_of_few_nodes_equals_the_separate_launches(cabi, case, channels, mo
         torch.testing.assert_close(a["energy"], b["energy"], rtol=1e-13, atol=1e-13)
 
 
+@pytest.mark.parametrize("channels,nodes,edges", [(96, 40, 560), (96, 40, 650), (128, 256, 1400), (96, 320, 400), (128, 320, 480), (64, 300, 850), (64, 300, 1100),
+                                                  (32, 520, 140), (32, 520, 175), (64, 520, 80), (64, 520, 105)])
+def test_step_of_few_nodes_on_both_sides_of_its_number_of_edges(cabi, channels, nodes, edges, monkeypatch):
+    """Just below and above the number of edges per node up to which a step of few nodes takes a workgroup per node, in each range of
+    node counts (430 + 1100 u, 290 + 600 (u - 1), 700 + 1600 (u - 1), 155 + 53 (u - 2), 85 + 40 (u - 2) + 70 (u - 2)^2 for u nodes per compute unit): what
+    comes back is the same to the bit, with many chunks of edges to a wave below it."""
+    from cuda_mace.models import OptimizedInvariantMACE, SyntheticInvariantMACE
+    from cuda_mace.utils.neighbour_list import neighbour_data
+
+    g = torch.Generator().manual_seed(nodes + edges)
+    box = (nodes * 4.0 / 3.0 * np.pi * 125.0 / edges) ** (1.0 / 3.0)
+    attrs = torch.nn.functional.one_hot(torch.randint(0, 4, (nodes,), generator=g), 4).double().cuda()
+    data = neighbour_data((torch.rand(nodes, 3, generator=g, dtype=torch.float64) * box).cuda(), attrs, 5.0, (True, True, True),
+                          torch.eye(3, dtype=torch.float64, device="cuda") * box)
+    assert abs(data["edge_index"].shape[1] / nodes - edges) < 0.03 * edges
+    model = OptimizedInvariantMACE(SyntheticInvariantMACE(channels=channels, atomic_numbers=(1, 6, 7, 8), avg_num_neighbors=float(edges), seed=53), device="cuda")
+    for keys in ({"compute_virials": True}, {"compute_force": False}):
+        with torch.set_grad_enabled("compute_force" not in keys):
+            monkeypatch.delenv("CM_STEP_GLUE", raising=False)
+            a = model(dict(data), **keys)
+            monkeypatch.setenv("CM_STEP_GLUE", "-1")
+            b = model(dict(data), **keys)
+        for key in ("node_energy", "node_feats") + (("forces", "virials") if "compute_virials" in keys else ()):
+            assert torch.isfinite(a[key]).all() and torch.equal(a[key], b[key]), key
+    assert model._native not in (None, False)
+
+
 @pytest.mark.parametrize("knots,channels,nodes", [(2, 64, 130), (3, 128, 130), (4, 32, 130), (512, 96, 300), (513, 64, 130), (513, 128, 300), (800, 32, 600)])
 def test_step_of_few_nodes_with_any_number_of_knots(cabi, knots, channels, nodes, monkeypatch):
     """The same where the knots do not lie in LDS (fewer than four, more than 512) and where they just do, with eight and with four waves
