@@ -10,7 +10,6 @@ import ctypes
 import os
 from typing import Optional
 
-import numpy as np
 import torch
 
 _HERE = os.path.realpath(os.path.dirname(__file__))
@@ -784,12 +783,13 @@ def report(tensors, host: torch.Tensor) -> None:
 
 def host_max_displacement(positions, reference) -> float:
     """Squared, for two contiguous fp64 numpy arrays [N, 3] (the library reads as many rows of both as the first has)."""
-    for name, a in (("positions", positions), ("reference", reference)):
-        if a.ndim != 2 or a.shape[1] != 3 or a.dtype != np.float64 or not a.flags.c_contiguous:
-            raise CudaMaceError("host_max_displacement: %s must be a contiguous fp64 array [N, 3] (got %s %s)" % (name, a.dtype, a.shape))
-    if positions.shape != reference.shape:
-        raise CudaMaceError("host_max_displacement: positions and reference differ in shape")
-    return lib.cm_host_max_displacement(positions.ctypes.data, reference.ctypes.data, positions.shape[0])
+    p, r = positions.__array_interface__, reference.__array_interface__  # one look at each: this runs at every step of an MD driver
+    shape = p["shape"]
+    if (len(shape) != 2 or shape[1] != 3 or r["shape"] != shape or p["typestr"] != "<f8" or r["typestr"] != "<f8"
+            or p["strides"] is not None or r["strides"] is not None):
+        raise CudaMaceError("host_max_displacement: positions %s %s and reference %s %s must be contiguous fp64 arrays [N, 3] of one shape"
+                            % (shape, p["typestr"], r["shape"], r["typestr"]))
+    return lib.cm_host_max_displacement(p["data"][0], r["data"][0], shape[0])
 
 
 # ---- readouts -------------------------------------------------------------------------------------

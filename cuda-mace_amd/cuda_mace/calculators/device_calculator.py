@@ -99,7 +99,7 @@ class DeviceCalculator:
         if host_positions is not None:
             if host_positions.shape[0] > 4096:
                 host_positions = None
-            elif host_positions.shape != tuple(positions.shape):
+            elif positions.shape != host_positions.shape:
                 raise ValueError("host_positions %s must have the shape of the positions, %s" % (host_positions.shape, tuple(positions.shape)))
             else:
                 host_positions = np.ascontiguousarray(host_positions, dtype=np.float64)
