@@ -35,7 +35,7 @@ constexpr int kSegKeys = 4;    // keys of a longer one that a lane ranks at a ti
 constexpr int kBucketLds = 256;  // pairs of one sender that a wave keeps in LDS
 
 // What bounds the whole call is the launches: each holds microseconds of work that waits for the one before.  There are eight
-// of them, where one kernel per step (box, keys, clear, histogram, scan, fill, rank, ...) took seventeen: every counter is
+// of them (nine where few bins hold many atoms), where one kernel per step (box, keys, clear, histogram, scan, fill, rank, ...) took seventeen: every counter is
 // cleared by the first, the old CSR and the pairs per sender are taken while the atoms are binned, and the offsets of the view
 // by sender are known before the pairs are placed, so the pairs drop into their buckets there.
 // A list that holds the reverse of each of its pairs and comes with its CSR (what the neighbour search of this library

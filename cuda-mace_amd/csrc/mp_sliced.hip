@@ -385,9 +385,10 @@ __global__ __launch_bounds__(kSlThreads) void mp_edge_forward_sliced_kernel(cons
   // them, each with its own L2).  The pieces in order, each with all its types, are cut into eight runs, one per XCD: the edge data
   // and the X rows of neighbouring nodes are fetched into one L2, or two where a piece is cut (share / 8 is no whole number at 96, 160, 192
   // and 224 channels).  With pieces 8 apart on an XCD and the rest of share / 8 spread over all of them every L2 fetched up to a third of
-  // the nodes.  Energies alone, us, that -> this: 96 channels 10 000 265 -> 261, 40 000 979 -> 931; 128 25 000 773 -> 765, 30 000 938 -> 933;
-  // 160 10 007 450 -> 444, 25 000 1 088 -> 1 055; 192 10 000 540.5 -> 540.2, 40 000 2 055 -> 2 028; 224 30 000 1 848 -> 1 839; 32 12 000 143 -> 139; 64
-  // and 256 the same.  Sixteen workgroups more at 160 and 192 channels, each with its share of the nodes of one or two types, gave
+  // the nodes.  Energies alone, us, that -> this in turn on one card (best of three runs): 96 channels 40 000 955.7 -> 941.2; 128 25 000 778.4 ->
+  // 773.8; 160 10 007 455.1 -> 449.0; 192 40 000 2 075 -> 2 060; 224 30 000 1 870 -> 1 864; within the runs' spread 32 12 000 134.2 -> 133.8, 96 10 000 259.2 -> 259.4, 128 30 000
+  // 934.8 -> 932.8, 192 10 000 538.2 -> 537.2, 160 25 000 1 085 -> 1 091; 64 and 256 the same (the gain differs by the card: 979 -> 931 and 1 088 -> 1 055 have been
+  // seen for 96 x 40 000 and 160 x 25 000).  Sixteen workgroups more at 160 and 192 channels, each with its share of the nodes of one or two types, gave
   // 0 to 0.8 % in place of that (the second slice of the table, the rounds at the end of both parts).
   int type, j;
   {

@@ -453,7 +453,7 @@ __global__ __launch_bounds__(kWave, CM_FUSED_BWD_WAVES) void mp_edge_backward_st
   __shared__ float sKnots[kKnots];
 
   // Runs of 128 workgroups, a node's parts in order, on an XCD: where the X rows are more than one L2 holds, a neighbour's rows come from there more
-  // often (step, us, with the forces' runs: 40 000 x 160 4 810 -> 4 776, 100 000 x 192 by the card 13 987 -> 13 849 or 13 985 -> 13 968; runs of 32
+  // often (step, us, with the forces' runs: 40 000 x 160 4 810 -> 4 776 and 4 736 -> 4 720 by the card, 100 000 x 192 by the card 13 987 -> 13 849 or 13 985 -> 13 968; runs of 32
   // and 512 the same; 10 007 x 160 and 20 000 x 224 equal).  The kernel above gains nothing from it (25 000 x 128, 40 000 x 96,
   // 12 000 x 256; 25 000 x 128 without gX 448 -> 459 alone).
   const int place = place_on_xcd<128>(blockIdx.x, nnodes * parts);

@@ -531,7 +531,8 @@ int cm_node_glue_backward(const float *gX2, const float *d_h2, const float *up_W
  * Python forward over its TorchScript classes followed by an autograd backward (models/InvariantMACE.py:246-379:
  * interactions :76-160, products :330, readouts :336, scale/shift :344, forces through get_outputs :354): same kernels,
  * same order, same numbers as that sequence, without a Python interpreter or an autograd engine between the launches
- * (16 launches up to 128 channels, 18 with few nodes at 96 and 128, 23 beyond, 20 with few nodes; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
+ * (up to 128 channels 16 launches, 18 up to some 4 000 nodes at 96 and 128 channels, four with few nodes and not too many edges each (few_nodes.hip);
+ * 23 beyond, 20 with few nodes; host cost of a step drops from ~0.4 ms to well under 0.1 ms).
  *
  * cm_mace_weights: the model's frozen weights in the layouts the op modules hold them (device pointers).
  *   spline[t]      [nknots - 1, 4, 4C]   radial spline table of layer t (cm_spline_forward's coeffs)
@@ -611,7 +612,7 @@ typedef struct cm_mace_graph {
  * 13 seeds of the backward chain, with 12 in their launch; 14 / 19 linear after the contraction, backward; 15 / 20 channel mixing backward (contraction
  * backward folded in); 16 message passing backward of layer 1 (edge pass + sender pass); 21 of layer 0 (edge pass
  * only); 17 linear_up backward; 18 skip backward; 22 sum of the two layers' per-edge gradients; 23 edge geometry backward
- * (forces); 24 virials.  With few nodes (up to 1 024 at 32 channels, 384 at 128; few_nodes.hip) a launch takes a node through a whole layer: 0 to 6 count as
+ * (forces); 24 virials.  With few nodes (up to 1 024 at 32 channels, 384 at 128, and not too many edges each; few_nodes.hip) a launch takes a node through a whole layer: 0 to 6 count as
  * 1, 7 to 16 as 7, 17 to 21 as 21. */
 int cm_mace_step_timing(unsigned stage_mask);
 /* A control launch for benchmarks (no counterpart in the reference): `workgroups` workgroups of 256 lanes, each lane
